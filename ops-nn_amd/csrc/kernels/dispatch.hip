@@ -29,6 +29,9 @@ int launch_kg_mfma(const OpsnnQmmArgs& a, hipStream_t st);   // qmm_i4_kg.hip
 uint64_t kg_workspace_bytes(const OpsnnQmmArgs& a);
 int launch_mx_mfma(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk = {});
 int launch_wqmm_mfma(const OpsnnWqmmArgs& a, hipStream_t st);
+bool wq_dense_wanted(const OpsnnWqmmArgs& a);   // wq_dense.hip
+uint64_t wq_dense_workspace(const OpsnnWqmmArgs& a);
+int launch_wq_dense(const OpsnnWqmmArgs& a, hipStream_t st);
 uint64_t mx_workspace_bytes(const OpsnnQmmArgs& a);
 }  // namespace opsnn
 
@@ -442,7 +445,9 @@ extern "C" int opsnnWqmm(const OpsnnWqmmArgs* a, void* stream)
     WeightCacheScope cache_scope;
     if (!a || !a->x || !a->w.ptr || !a->scale.ptr || !a->y || a->M <= 0 || a->N <= 0 || a->K <= 0) return -1;
     if (a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain()) {
-        int rc = launch_wqmm_mfma(*a, (hipStream_t)stream);
+        int rc = launch_wq_dense(*a, (hipStream_t)stream);
+        if (rc != OPSNN_NOT_TAKEN) return rc;
+        rc = launch_wqmm_mfma(*a, (hipStream_t)stream);
         if (rc != OPSNN_NOT_TAKEN) return rc;
         if (a->force_variant != 0) return -4;
     }
@@ -490,6 +495,7 @@ static uint64_t qmm_workspace_base(const OpsnnQmmArgs* a, int mode)
 extern "C" uint64_t opsnnWqmmWorkspace(const OpsnnWqmmArgs* a)
 {
     if (!a || a->M <= 0 || a->N <= 0 || a->K <= 0) return 0;
+    if (wq_dense_wanted(*a)) return wq_dense_workspace(*a);   // many rows: the dequantised weight (and partial sums)
     const uint64_t bits = (a->w_dtype == DT_I4 || a->w_dtype == DT_E2M1) ? 4 : 8;
     // up to 16 rows against a long K: fp32 partial sums of the x-in-registers kernel's K split, in front of everything else
     // (from 17 rows against a narrow N and a long K: those of the many-rows kernel's K split)

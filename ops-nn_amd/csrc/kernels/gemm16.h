@@ -1,0 +1,24 @@
+// 16-bit operand GEMM (gemm16.hip): the dense step behind a pass that has widened quantized operands to fp16 / bf16.
+#pragma once
+#include "launch.h"
+#include "qgemm_core.hip.h"
+
+namespace opsnn {
+
+// How a [M, K] x [N, K] product of 16-bit operands is tiled.  cfg: 8 .. 11 the four-wave kernel with 256 x 32*cfg tiles
+// (qmm_int8_wide.hip); 2: 128 x 128 tiles, two workgroups per CU.  splits > 1 (cfg 2): K split over workgroups, fp32 partial
+// sums [splits][batch][M][N].  us: the estimate that the choice rests on.
+struct Gemm16Plan {
+    int cfg = 2, splits = 1;
+    double us = 0;
+};
+Gemm16Plan gemm16_plan(int64_t M, int64_t N, int64_t K, int64_t batch);
+inline uint64_t gemm16_part_bytes(const Gemm16Plan& pl, int64_t M, int64_t N, int64_t batch)
+{
+    return pl.splits > 1 ? ((uint64_t)pl.splits * (uint64_t)batch * (uint64_t)M * (uint64_t)N * 4 + 255) / 256 * 256 : 0;
+}
+// p: a / b with strides in bytes, KB = 2 K, K % 64 == 0, out [batch, M, N] with ldc = N; x1s / x2s / bias as in QgemmParams
+// (each may be null).  `part`: gemm16_part_bytes of the plan.
+int launch_gemm16(QgemmParams p, const Gemm16Plan& pl, bool bf16_operands, int64_t batch, int out_dt, float* part, hipStream_t st);
+
+}  // namespace opsnn

@@ -1,0 +1,132 @@
+// Dense product of two 16-bit operands (fp16 or bf16, both K-contiguous) with fp32 sums and a row scale, column scale and bias
+// in the epilogue: the step behind the passes that widen quantized operands once per call (wq_dense.hip).  The kernels
+// are the tile kernels of the quantized modes with another matrix instruction: everything in them is addressed in bytes
+// of K, and a lane's 16 bytes feed one 16-bit instruction where they feed one int8 instruction.
+#include "gemm16.h"
+#include "launch.h"
+
+namespace opsnn {
+
+int launch_16_wide(const QgemmParams& p, int fn, bool bf16_operands, int64_t batch, int out_dt, hipStream_t st);   // qmm_int8_wide.hip
+
+// out[b, m, n] = rounded(sum over the splits, in split order, * x2s[n] * x1s[m] + bias[n]).  One row per blockIdx.y, four
+// columns per thread: no divisions (the row and column come from the block index), 16-byte loads where N % 4 == 0.
+template <int OUT_DT>
+__global__ __launch_bounds__(256) void gemm16_splitk_reduce_kernel(QgemmParams p, int64_t total)
+{
+    const int64_t n0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (n0 >= p.N) return;
+    const float* part = (const float*)p.part;
+    const bool vec = (p.N % 4) == 0;
+    for (int64_t row = blockIdx.y; row < total / p.N; row += gridDim.y) {
+        const int64_t bz = row / p.M, m = row - bz * p.M, at = row * p.N + n0;
+        const int cols = p.N - n0 < 4 ? (int)(p.N - n0) : 4;
+        v4f v = {0, 0, 0, 0};
+        auto load = [&](int s) -> v4f {
+            const float* q = part + (int64_t)s * total + at;
+            if (vec) return *(const v4f*)q;
+            v4f r = {0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (e < cols) r[e] = q[e];
+            return r;
+        };
+        v = load(0);
+        int s = 1;
+        for (; s + 3 < p.splits; s += 4) {
+            const v4f a = load(s), b = load(s + 1), c = load(s + 2), d = load(s + 3);
+            v = v + a; v = v + b; v = v + c; v = v + d;
+        }
+        for (; s < p.splits; s++) v = v + load(s);
+        const float s1 = p.x1s ? p.x1s[p.x1s_one ? 0 : m] : 1.0f;
+        uint16_t o[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int64_t n = n0 + (e < cols ? e : cols - 1);
+            float t = v[e];
+            if (p.x2s) t = t * load_scalar_as_f32(p.x2s, p.x2s_dt, p.x2s_len == 1 ? 0 : n);
+            t = t * s1;
+            if (p.bias) t = t + load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + n);
+            o[e] = to_b16<OUT_DT>(t);
+        }
+        uint16_t* out = (uint16_t*)p.out + row * p.ldc + n0;
+        if (vec && ((uintptr_t)p.out % 8) == 0) *(v4us*)out = (v4us){o[0], o[1], o[2], o[3]};
+        else {
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (e < cols) out[e] = o[e];
+        }
+    }
+}
+
+template <int MODE, int BM, int BN, int WGM, int WGN>
+static int launch_split16(const QgemmParams& p, int64_t batch, int out_dt, hipStream_t st)
+{
+    constexpr int BK = 128, STAGES = 2;
+    if (!p.part || p.splits < 2 || (p.KB % BK) != 0 || p.splits > p.KB / BK / 2 || p.ldc != p.N) return -1;
+    const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
+    const size_t lds = (size_t)STAGES * (BM + BN) * BK;
+    auto k = qgemm_kernel<MODE, BM, BN, BK, WGM, WGN, STAGES, 1, false, DT_BF16, true>;
+    static std::atomic<uint64_t> attr_set{0};
+    if (!device_flag_test(attr_set)) {
+        hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return (int)e;
+        device_flag_set(attr_set);
+    }
+    hipLaunchKernelGGL(k, dim3((unsigned)(tiles_m * tiles_n), (unsigned)batch, (unsigned)p.splits), dim3(WGM * WGN * 64), lds, st, p, tiles_m, tiles_n);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return (int)e;
+    const int64_t rows = batch * p.M;
+    const dim3 grid((unsigned)((p.N + 1023) / 1024), (unsigned)(rows < 65535 ? rows : 65535));
+    if (out_dt == DT_BF16) hipLaunchKernelGGL(gemm16_splitk_reduce_kernel<DT_BF16>, grid, dim3(256), 0, st, p, rows * p.N);
+    else hipLaunchKernelGGL(gemm16_splitk_reduce_kernel<DT_F16>, grid, dim3(256), 0, st, p, rows * p.N);
+    return (int)hipGetLastError();
+}
+
+template <int MODE>
+static int launch16(const QgemmParams& p, const Gemm16Plan& pl, int64_t batch, int out_dt, hipStream_t st)
+{
+    if (pl.cfg >= 8) return launch_16_wide(p, pl.cfg, MODE == MODE_BF16, batch, out_dt, st);
+    if (pl.splits > 1) return launch_split16<MODE, 128, 128, 2, 2>(p, batch, out_dt, st);
+    return qgemm_launch<MODE, 128, 128, 128, 2, 2, 2, 1>(p, batch, out_dt, st);
+}
+
+// The estimate, in microseconds, for each tiling; fitted to one box (random operands, K = 4096 .. 18432):
+//   four-wave kernel: 0.185 us per 32 columns of tile width and 64-element K tile, 8 us a round beside (4096^3: 99 us in one
+//   round of 256 x 256 tiles = 1.39 Pflop/s; 2048 x 4096 x 11008: 134 us in one round of 256 x 352);
+//   128 x 128 tiles: 0.65 us per K tile alone on a CU, 1.0 us for two that share one, 6 us beside;
+//   K split: the partial sums written and read back at 4 TB/s, and 5 us for the second kernel.
+Gemm16Plan gemm16_plan(int64_t M, int64_t N, int64_t K, int64_t batch)
+{
+    const int64_t cus = 256, kt = K / 64;
+    Gemm16Plan best;
+    best.us = 1e30;
+    const int64_t tm = (M + 255) / 256;
+    for (int fn = 8; fn <= 11; fn++) {
+        const int64_t tiles = tm * ((N + 32 * fn - 1) / (32 * fn)) * batch;
+        const double us = (double)((tiles + cus - 1) / cus) * (0.185 * fn * (double)kt + 8.0);
+        if (us < best.us) { best.cfg = fn; best.splits = 1; best.us = us; }
+    }
+    const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128) * batch;
+    for (int s = 1; s <= 16; s++) {
+        if (s > 1 && (t128 * s > 2 * cus || kt / s < 4)) break;
+        const int64_t per_cu = (t128 * s + cus - 1) / cus;
+        const double steps = (double)(kt + s - 1) / s;
+        double us = steps * ((double)(per_cu / 2) * 1.0 + (double)(per_cu % 2) * 0.65) + 6.0;
+        if (s > 1) us += 5.0 + 8.0 * s * (double)M * (double)N * (double)batch / 4.0e6;
+        if (us < best.us) { best.cfg = 2; best.splits = s; best.us = us; }
+    }
+    return best;
+}
+
+int launch_gemm16(QgemmParams p, const Gemm16Plan& pl, bool bf16_operands, int64_t batch, int out_dt, float* part, hipStream_t st)
+{
+    if (p.KB % 128 != 0 || p.KB < 128 || (out_dt != DT_BF16 && out_dt != DT_F16)) return OPSNN_NOT_TAKEN;
+    if (((uintptr_t)p.a | (uintptr_t)p.b | (uint64_t)p.lda | (uint64_t)p.ldb | (uint64_t)p.a_bs | (uint64_t)p.b_bs) % 16) return OPSNN_NOT_TAKEN;
+    if (256 * p.lda >= (1ll << 31) || 352 * p.ldb >= (1ll << 31)) return OPSNN_NOT_TAKEN;   // 32-bit offsets inside a tile
+    p.splits = pl.splits;
+    p.part = (int32_t*)part;
+    return bf16_operands ? launch16<MODE_BF16>(p, pl, batch, out_dt, st) : launch16<MODE_F16>(p, pl, batch, out_dt, st);
+}
+
+}  // namespace opsnn

@@ -1,4 +1,4 @@
-// int8 x int8 (and fp8 e4m3 x e4m3) tile kernel with one wave per SIMD and a 256 x (32*FN) output tile, FN = 8..11.
+// int8 x int8 (and fp8 e4m3 x e4m3, fp16 x fp16, bf16 x bf16) tile kernel with one wave per SIMD and a 256 x (32*FN) output tile, FN = 8..11.
 //
 // Why a second int8 tile kernel: a GEMM runs in rounds of one tile per CU, and with a fixed 256 x 256 tile a shape
 // such as 2048 x 11008 needs 1.34 rounds -- the last third of a round costs a whole one (or a second launch of small
@@ -28,11 +28,15 @@
 // launch of 128 x 128 tiles on the remaining 2816; at 256 x 256 (FN = 8) it is level with the 8-wave kernel
 // (62-64 against 65 us on 2048 x 4096 x 8192, 540 against 560 us on 8192^3).
 //
-// F8 = true: the same kernel on fp8 e4m3 operands for the modes with one scale per row and per column (K-C, K-T,
+// EL = EL_F8: the same kernel on fp8 e4m3 operands for the modes with one scale per row and per column (K-C, K-T,
 // separately multiplied double scale): one v_mfma_f32_16x16x128_f8f6f4 per fragment pair and K tile instead of two
 // int8 instructions, float sums, and the same epilogue without the integer bias.
 //
-// MXS = true (with F8): MXFP8.  A K tile needs four e8m0 bytes per row; one 16-byte copy per row brings the scales of
+// EL = EL_F16 / EL_BF16: the same kernel on 16-bit floating operands (launch_16_wide).  Everything is addressed in bytes of K: a
+// lane's 16 bytes are 8 elements of v_mfma_f32_16x16x32_{f16,bf16} where they are 16 of v_mfma_i32_16x16x64_i8, the
+// instruction takes the same 16 clocks, and so the loop is the int8 loop with another opcode: a K tile is 64 elements.
+//
+// MXS = true (with EL_F8): MXFP8.  A K tile needs four e8m0 bytes per row; one 16-byte copy per row brings the scales of
 // FOUR tiles into one of two slots behind the operand stages (a 4-byte copy per row and tile costs a cache-line request
 // for four useful bytes -- as many requests as the operands themselves, and the kernel ran no faster than the 8-wave
 // one).  Each lane reads the dword of its row with its fragment and shifts its own block's byte down (lane group q
@@ -94,9 +98,25 @@ __device__ __forceinline__ void dma_copy16v(const void* g, uint32_t lds_base)
     asm volatile("s_add_u32 m0, %0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_base), "v"(g), "n"(LDS_IMM) : "memory", "m0", "scc");
 }
 
-template <int FN, int OUT_DT, bool F8 = false, bool MXS = false>
+// acc += a (16 x 32) x b (32 x 16), 16-bit floating operands, fp32 sums
+template <bool AG, bool BF>
+__device__ __forceinline__ void mfma_16_16x16x32(v4f& c, const v4i a, const v4i b)
+{
+    if constexpr (BF) {
+        if constexpr (AG) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+        else asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+    } else {
+        if constexpr (AG) asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+        else asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+    }
+}
+
+enum : int { EL_I8 = 0, EL_F8 = 1, EL_F16 = 2, EL_BF16 = 3 };
+
+template <int FN, int OUT_DT, int EL = EL_I8, bool MXS = false>
 __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, int tiles_m, int tiles_n)
 {
+    constexpr bool F8 = EL == EL_F8;
     static_assert(!MXS || F8, "block scales ride on the fp8 form");
     constexpr int SLOTS = F8 ? 8 : 16;   // MFMAs per x2 fragment
     constexpr int NT = 256, BM = 256, TM = 128, FM = TM / 16, TN = 16 * FN, BN = 2 * TN, BK = 128, STAGES = 2;
@@ -190,7 +210,12 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
         for_copies([&](auto c) { issue_piece(kt, kt % STAGES, c); });
     };
 
-    using acc_t = std::conditional_t<F8, v4f, v4i>;
+    using acc_t = std::conditional_t<EL == EL_I8, v4i, v4f>;
+    auto mma = [&](auto ag, acc_t& c, const v4i a, const v4i b) {   // (the fp8 forms have their own loop)
+        constexpr bool AG = decltype(ag)::value;
+        if constexpr (EL == EL_I8) mfma_i8_16x16x64<AG>(c, a, b);
+        else if constexpr (EL == EL_F16 || EL == EL_BF16) mfma_16_16x16x32<AG, EL == EL_BF16>(c, a, b);
+    };
     acc_t acc[FN][FM];
 #pragma unroll
     for (int i = 0; i < FN; i++)
@@ -345,8 +370,8 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
             // the two instructions of a fragment pair are eight instructions apart: no back-to-back dependent MFMAs
 #pragma unroll
             for (int j = 0; j < FM; j++) {
-                if (i * FM + j < 64) mfma_i8_16x16x64<true>(acc[i][j], blo, fal[j]);
-                else mfma_i8_16x16x64<false>(acc[i][j], blo, fal[j]);
+                if (i * FM + j < 64) mma(std::true_type{}, acc[i][j], blo, fal[j]);
+                else mma(std::false_type{}, acc[i][j], blo, fal[j]);
                 __builtin_amdgcn_sched_barrier(0);
                 spread_copies(i * 16 + j);
                 if (i == FN - 1) fal[j] = load_lo(stn, a_rowbase + j * 16 * BK);
@@ -358,8 +383,8 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
             }
 #pragma unroll
             for (int j = 0; j < FM; j++) {
-                if (i * FM + j < 64) mfma_i8_16x16x64<true>(acc[i][j], bhi, fah[j]);
-                else mfma_i8_16x16x64<false>(acc[i][j], bhi, fah[j]);
+                if (i * FM + j < 64) mma(std::true_type{}, acc[i][j], bhi, fah[j]);
+                else mma(std::false_type{}, acc[i][j], bhi, fah[j]);
                 __builtin_amdgcn_sched_barrier(0);
                 spread_copies(i * 16 + 8 + j);
                 if (i == FN - 1) {
@@ -389,7 +414,7 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
             if (n >= p.N) n = p.N - 1;
             const int64_t si = p.x2s_len == 1 ? 0 : n;
             float sv = 1.0f;
-            if constexpr (!MXS) {
+            if (!MXS && (EL == EL_I8 || EL == EL_F8 || p.x2s)) {
                 sv = p.x2s_dt == DT_U64 ? u2f((uint32_t)((const uint64_t*)p.x2s)[si]) : load_scalar_as_f32(p.x2s, p.x2s_dt, si);
                 if (p.x2s_trunc || p.x2s_dt == DT_U64) sv = u2f(f2u(sv) & 0xFFFFE000u);
             }
@@ -407,7 +432,7 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
         // Integer outputs (no per-row scale): INT32 = acc + ib[n]; INT8 = clip(s9(s9(fp32(acc + ib[n]) * s2[n]) + s9(off[n])), the
         // offset from p.x2off or from bits 37..45 of a UINT64 scale word, s9 = round half to even and clamp to [-256, 255].
         // They leave straight from the registers: four consecutive columns of one row per lane and fragment.
-        static_assert(!F8 && !MXS, "integer outputs belong to the int8 mode");
+        static_assert(EL == EL_I8, "integer outputs belong to the int8 mode");
         float* sOff = (float*)smem + 3 * BN + BM;
         const bool has_off = p.x2off != nullptr || p.x2s_dt == DT_U64;
         if (OUT_DT == DT_I8 && has_off) {
@@ -495,7 +520,7 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
 #pragma unroll
             for (int e = 0; e < 4; e++) {
                 float tv;
-                if constexpr (F8) tv = acc[i][j][e];
+                if constexpr (EL != EL_I8) tv = acc[i][j][e];
                 else tv = (float)(acc[i][j][e] + ib[e]);
                 tv = tv * s2[e];
                 tv = tv * s1;
@@ -515,13 +540,13 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
     }
 }
 
-template <int FN, int OUT_DT, bool F8 = false, bool MXS = false>
+template <int FN, int OUT_DT, int EL = EL_I8, bool MXS = false>
 static int launch_wide_one(const QgemmParams& p, int64_t batch, hipStream_t st)
 {
     constexpr int BM = 256, BN = 32 * FN, BK = 128;
     const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
     const size_t lds = (size_t)2 * (BM + BN) * BK + (MXS ? (size_t)2 * ((BM + BN + 255) / 256) * 4096 : 0);
-    auto k = qgemm_i8_wide_kernel<FN, OUT_DT, F8, MXS>;
+    auto k = qgemm_i8_wide_kernel<FN, OUT_DT, EL, MXS>;
     static std::atomic<uint64_t> attr_set{0};   // one bit per device: the attribute belongs to the (kernel, device) pair
     if (!device_flag_test(attr_set)) {
         hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -570,10 +595,10 @@ int launch_f8_wide(const QgemmParams& p, int fn, int64_t batch, int out_dt, hipS
     if (out_dt != DT_BF16 && out_dt != DT_F16) return OPSNN_NOT_TAKEN;
     const bool bf = out_dt == DT_BF16;
     switch (fn) {
-        case 8: return bf ? launch_wide_one<8, DT_BF16, true>(p, batch, st) : launch_wide_one<8, DT_F16, true>(p, batch, st);
-        case 9: return bf ? launch_wide_one<9, DT_BF16, true>(p, batch, st) : launch_wide_one<9, DT_F16, true>(p, batch, st);
-        case 10: return bf ? launch_wide_one<10, DT_BF16, true>(p, batch, st) : launch_wide_one<10, DT_F16, true>(p, batch, st);
-        case 11: return bf ? launch_wide_one<11, DT_BF16, true>(p, batch, st) : launch_wide_one<11, DT_F16, true>(p, batch, st);
+        case 8: return bf ? launch_wide_one<8, DT_BF16, EL_F8>(p, batch, st) : launch_wide_one<8, DT_F16, EL_F8>(p, batch, st);
+        case 9: return bf ? launch_wide_one<9, DT_BF16, EL_F8>(p, batch, st) : launch_wide_one<9, DT_F16, EL_F8>(p, batch, st);
+        case 10: return bf ? launch_wide_one<10, DT_BF16, EL_F8>(p, batch, st) : launch_wide_one<10, DT_F16, EL_F8>(p, batch, st);
+        case 11: return bf ? launch_wide_one<11, DT_BF16, EL_F8>(p, batch, st) : launch_wide_one<11, DT_F16, EL_F8>(p, batch, st);
         default: return OPSNN_NOT_TAKEN;
     }
 }
@@ -591,10 +616,34 @@ int launch_mxfp8_wide(const QgemmParams& p, int fn, int64_t batch, int out_dt, h
     if (out_dt != DT_BF16 && out_dt != DT_F16) return OPSNN_NOT_TAKEN;
     const bool bf = out_dt == DT_BF16;
     switch (fn) {
-        case 8: return bf ? launch_wide_one<8, DT_BF16, true, true>(p, batch, st) : launch_wide_one<8, DT_F16, true, true>(p, batch, st);
-        case 9: return bf ? launch_wide_one<9, DT_BF16, true, true>(p, batch, st) : launch_wide_one<9, DT_F16, true, true>(p, batch, st);
+        case 8: return bf ? launch_wide_one<8, DT_BF16, EL_F8, true>(p, batch, st) : launch_wide_one<8, DT_F16, EL_F8, true>(p, batch, st);
+        case 9: return bf ? launch_wide_one<9, DT_BF16, EL_F8, true>(p, batch, st) : launch_wide_one<9, DT_F16, EL_F8, true>(p, batch, st);
         default: return OPSNN_NOT_TAKEN;
     }
+}
+
+}  // namespace opsnn
+
+namespace opsnn {
+
+// fp16 x fp16 or bf16 x bf16 (both operands K-contiguous, KB = 2 K bytes, K % 64 == 0), 16-bit output, epilogue as for fp8:
+// p.x1s / p.x2s (either may be null: no scale) and a floating bias.
+template <int EL>
+static int launch_16_wide_el(const QgemmParams& p, int fn, int64_t batch, bool bf, hipStream_t st)
+{
+    switch (fn) {
+        case 8: return bf ? launch_wide_one<8, DT_BF16, EL>(p, batch, st) : launch_wide_one<8, DT_F16, EL>(p, batch, st);
+        case 9: return bf ? launch_wide_one<9, DT_BF16, EL>(p, batch, st) : launch_wide_one<9, DT_F16, EL>(p, batch, st);
+        case 10: return bf ? launch_wide_one<10, DT_BF16, EL>(p, batch, st) : launch_wide_one<10, DT_F16, EL>(p, batch, st);
+        case 11: return bf ? launch_wide_one<11, DT_BF16, EL>(p, batch, st) : launch_wide_one<11, DT_F16, EL>(p, batch, st);
+        default: return OPSNN_NOT_TAKEN;
+    }
+}
+int launch_16_wide(const QgemmParams& p, int fn, bool bf16_operands, int64_t batch, int out_dt, hipStream_t st)
+{
+    if (p.KB % 128 != 0 || p.KB < 128) return OPSNN_NOT_TAKEN;
+    if (out_dt != DT_BF16 && out_dt != DT_F16) return OPSNN_NOT_TAKEN;
+    return bf16_operands ? launch_16_wide_el<EL_BF16>(p, fn, batch, out_dt == DT_BF16, st) : launch_16_wide_el<EL_F16>(p, fn, batch, out_dt == DT_BF16, st);
 }
 
 }  // namespace opsnn

@@ -1,0 +1,230 @@
+// Weight-only matmul with many rows of x: the weight is dequantised ONCE per call to x's own type, K-contiguous, into the
+// workspace, and the product is a dense 16-bit one (gemm16.hip).
+//
+//   w16[n][k] = T(T(w[k,n] + offset[g,n]) * scale[g,n])      the two roundings of the formula, as in wqmm_stream.hip.h
+//
+// Cost of the pass: half or one byte read and two bytes written per weight; the streaming kernels dequantise in registers
+// once per 256 rows instead, so the pass pays from a few hundred rows on, and from far fewer where those kernels do not
+// run (N no multiple of 32, K no whole number of x slabs, groups of 64, [K, N] storage): it takes every layout, group and N.
+#include "gemm16.h"
+#include "launch.h"
+#include "wqmm_stream.hip.h"
+
+extern "C" int opsnn_wq_tile_min();   // dispatch.hip
+namespace opsnn {
+
+// [N, K] storage: a lane turns 8 consecutive k of one row into 16 bytes; a wave covers 512 k of a row per step.
+template <int XDT, int WBITS, bool HAS_OFF>
+__global__ __launch_bounds__(256) void wq_dequant_nk_kernel(WqParams p, uint16_t* __restrict__ out, int steps)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t n = (int64_t)blockIdx.y * 4 + (threadIdx.x >> 6);
+    if (n >= p.N) return;
+    const uint8_t* w = p.w + n * p.ldw;
+    const uint16_t* sc = p.scale + n * p.s_cs;
+    const uint16_t* of = HAS_OFF ? p.offset + n * p.s_cs : nullptr;
+    const DqConst dqc = make_dq_const();
+    const int Ki = (int)p.K, groupi = (int)p.group;
+#pragma unroll 4
+    for (int s = 0; s < steps; s++) {
+        const int k = ((int)blockIdx.x * steps + s) * 512 + lane * 8;
+        if (k >= Ki) break;
+        v4i q = {0, 0, 0, 0};
+        if constexpr (WBITS == 4) q[0] = *(const int*)(w + k / 2);
+        else { const v2i t = *(const v2i*)(w + k); q[0] = t[0]; q[1] = t[1]; }
+        const int g = p.group_shift >= 0 ? k >> p.group_shift : k / groupi;
+        const uint16_t sb = sc[(int64_t)g * p.s_rs], ob = HAS_OFF ? of[(int64_t)g * p.s_rs] : (uint16_t)0;
+        *(v4i*)(out + n * p.K + k) = dequant8<XDT, WBITS, HAS_OFF, true>(q, 0, sb, ob, dqc);
+    }
+}
+
+// [K, N] storage: a lane takes 8 rows of k and 8 neighbouring columns, dequantises along the columns (that is how the codes
+// and the scales lie) and writes, per column, 16 bytes of 8 consecutive k; 16 lanes side by side in k make 256 contiguous
+// bytes of an output row.  The 8 x 8 transposition is byte permutes in registers (bf16: the packing conversion itself).
+template <int XDT, int WBITS, bool HAS_OFF>
+__global__ __launch_bounds__(256) void wq_dequant_kn_kernel(WqParams p, uint16_t* __restrict__ out)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t k0 = (int64_t)blockIdx.y * 128 + (lane & 15) * 8;
+    const int64_t n0 = ((int64_t)blockIdx.x * 16 + wave * 4 + (lane >> 4)) * 8;
+    if (k0 >= p.K || n0 >= p.N) return;
+    const int cols = p.N - n0 < 8 ? (int)(p.N - n0) : 8;
+    const int g = p.group_shift >= 0 ? (int)k0 >> p.group_shift : (int)k0 / (int)p.group;
+    // codes: row i of the block in q[i] (int4: one dword, int8: two)
+    constexpr int DW = WBITS / 4;
+    uint32_t q[8][DW];
+    const uint8_t* src = p.w + k0 * p.ldw + n0 * WBITS / 8;
+    if (cols == 8) {
+#pragma unroll
+        for (int i = 0; i < 8; i++) __builtin_memcpy(q[i], src + i * p.ldw, 4 * DW);
+    } else {   // the matrix edge: byte by byte (4-bit: N is even)
+        for (int i = 0; i < 8; i++) {
+            uint8_t b[4 * DW] = {};
+            for (int j = 0; j * 8 / WBITS < cols; j++) b[j] = src[i * p.ldw + j];
+            __builtin_memcpy(q[i], b, 4 * DW);
+        }
+    }
+    uint16_t sb[8], ob[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) {
+        const int64_t n = n0 + (j < cols ? j : cols - 1);
+        sb[j] = p.scale[(int64_t)g * p.s_rs + n * p.s_cs];
+        ob[j] = HAS_OFF ? p.offset[(int64_t)g * p.s_rs + n * p.s_cs] : (uint16_t)0;
+    }
+    uint32_t o[8][4];   // o[column][pair of k]
+    if constexpr (XDT == DT_F16) {
+        // per row of k: four pairs of columns -- int4: (0,4) (1,5) (2,6) (3,7), the order of the nibble splice; int8: (0,1) ...
+        h2 sc[4], of[4];
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int a = WBITS == 4 ? t : 2 * t, b = WBITS == 4 ? t + 4 : 2 * t + 1;
+            sc[t] = (h2){__builtin_bit_cast(_Float16, sb[a]), __builtin_bit_cast(_Float16, sb[b])};
+            of[t] = (h2){__builtin_bit_cast(_Float16, ob[a]), __builtin_bit_cast(_Float16, ob[b])};
+        }
+        const h2 c1032 = {(_Float16)-1032.0f, (_Float16)-1032.0f}, c72 = {(_Float16)-72.0f, (_Float16)-72.0f}, r16 = {(_Float16)0.0625f, (_Float16)0.0625f};
+        const h2 c1152 = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+#pragma unroll
+        for (int i = 0; i < 8; i += 2) {
+            uint32_t row[2][4];
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                h2 t[4];
+                if constexpr (WBITS == 4) {
+                    const uint32_t u = q[i + r][0], u8 = u >> 8;
+                    t[0] = __builtin_bit_cast(h2, (u & 0x000F000Fu) ^ 0x64086408u) + c1032;
+                    t[1] = __builtin_elementwise_fma(__builtin_bit_cast(h2, (u & 0x00F000F0u) ^ 0x64806480u), r16, c72);
+                    t[2] = __builtin_bit_cast(h2, (u8 & 0x000F000Fu) ^ 0x64086408u) + c1032;
+                    t[3] = __builtin_elementwise_fma(__builtin_bit_cast(h2, (u8 & 0x00F000F0u) ^ 0x64806480u), r16, c72);
+                } else {
+                    const uint32_t qa = q[i + r][0] ^ 0x80808080u, qb = q[i + r][DW - 1] ^ 0x80808080u, magic = 0x64646464u;
+                    t[0] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(magic, qa, 0x04010400u)) + c1152;
+                    t[1] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(magic, qa, 0x04030402u)) + c1152;
+                    t[2] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(magic, qb, 0x04010400u)) + c1152;
+                    t[3] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(magic, qb, 0x04030402u)) + c1152;
+                }
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    if constexpr (HAS_OFF) t[c] = t[c] + of[c];
+                    row[r][c] = u32(t[c] * sc[c]);
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const int a = WBITS == 4 ? c : 2 * c, b = WBITS == 4 ? c + 4 : 2 * c + 1;
+                o[a][i / 2] = __builtin_amdgcn_perm(row[1][c], row[0][c], 0x05040100u);
+                o[b][i / 2] = __builtin_amdgcn_perm(row[1][c], row[0][c], 0x07060302u);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const float scf = bf16_to_f32(sb[j]), off = bf16_to_f32(ob[j]);
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) {
+                float w[2];
+#pragma unroll
+                for (int r = 0; r < 2; r++) {
+                    if constexpr (WBITS == 4) w[r] = (float)((int)(q[i + r][0] << (28 - 4 * j)) >> 28);
+                    else w[r] = (float)((int)(q[i + r][j / 4 * (DW - 1)] << (24 - 8 * (j & 3))) >> 24);
+                }
+                if constexpr (HAS_OFF) {
+                    const uint32_t pk = pack2_bf16((v2f){w[0] + off, w[1] + off});
+                    w[0] = u2f(pk << 16);
+                    w[1] = u2f(pk & 0xffff0000u);
+                }
+                o[j][i / 2] = pack2_bf16((v2f){w[0] * scf, w[1] * scf});
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < 8; j++)
+        if (j < cols) *(v4i*)(out + (n0 + j) * p.K + k0) = (v4i){(int)o[j][0], (int)o[j][1], (int)o[j][2], (int)o[j][3]};
+}
+
+template <int XDT, int WBITS, bool HAS_OFF>
+static int launch_dequant(const WqParams& p, bool kn, uint16_t* out, hipStream_t st)
+{
+    if (kn) {
+        const dim3 grid((unsigned)((p.N + 127) / 128), (unsigned)((p.K + 127) / 128));
+        hipLaunchKernelGGL((wq_dequant_kn_kernel<XDT, WBITS, HAS_OFF>), grid, dim3(256), 0, st, p, out);
+    } else {
+        const int steps = 4;
+        const dim3 grid((unsigned)((p.K + 512 * steps - 1) / (512 * steps)), (unsigned)((p.N + 3) / 4));
+        hipLaunchKernelGGL((wq_dequant_nk_kernel<XDT, WBITS, HAS_OFF>), grid, dim3(256), 0, st, p, out, steps);
+    }
+    return (int)hipGetLastError();
+}
+
+static uint64_t dense_weight_bytes(const OpsnnWqmmArgs& a) { return ((uint64_t)a.N * (uint64_t)a.K * 2 + 255) / 256 * 256; }
+
+// Does the call run on this route?  Looks at what phase 1 knows (shapes, types, layouts, addresses), so that both phases agree.
+//
+// The pass moves 2.5 (8-bit weights: 3) bytes per weight at 4.4 TB/s, the product takes what gemm16_plan estimates.  Against
+// it stands the many-rows streaming kernel where it runs (wqmm.hip: [N, K] storage, N % 32 == 0, whole x slabs and groups of
+// whole chunks), which keeps 0.78 Pflop/s from 256 rows on if K is a whole number of rounds for its 256-row instance, a
+// third of that if not; everywhere else the general kernel re-reads the weight per 64 rows at a fraction of its speed, and this
+// route takes every call of more than 64 rows.  (Measured: 1999 x 4096 x 11008 bf16 x int4 228 -> 156 us, [K, N] storage
+// 613 -> 162; 1024 x 8192 x 28672 497 against 499, 512 rows 254 against 330.)
+bool wq_dense_wanted(const OpsnnWqmmArgs& a)
+{
+    if (a.w_dtype != DT_I4 && a.w_dtype != DT_I8) return false;
+    if (a.x_dtype != DT_F16 && a.x_dtype != DT_BF16) return false;
+    if (a.scale_dtype != a.x_dtype || a.force_variant == OPSNN_VARIANT_PLAIN) return false;
+    if (opsnn_wq_tile_min() <= 128) return false;   // (test hook: such calls are sent to the tile kernel of wqmm_tile.hip)
+    if (a.M <= 64 || a.K % 64 != 0 || a.N < 128 || (uintptr_t)a.x % 16) return false;
+    if (a.K >= (1ll << 22) || a.N >= (1ll << 30)) return false;
+    if (a.group > 0 && a.group % 8 != 0) return false;
+    const bool nk = a.w.row_stride == 1 && a.w.col_stride == a.K, kn = a.w.col_stride == 1 && a.w.row_stride == a.N;
+    if (!nk && !kn) return false;
+    if (a.w_dtype == DT_I4 && !nk && a.N % 2 != 0) return false;
+    const int wbits = a.w_dtype == DT_I4 ? 4 : 8;
+    const int64_t kc = 4 * (128 / wbits);
+    const int64_t cpg = a.group > 0 && a.group < a.K ? a.group / kc : 1;
+    const bool rows_kernel = nk && a.N % 32 == 0 && a.N >= 256 && a.K % (2 * kc) == 0 &&
+                             (a.group <= 0 || a.group >= a.K || (a.group % kc == 0 && (cpg & (cpg - 1)) == 0));
+    if (!rows_kernel) return true;
+    const double flops = 2.0 * (double)a.M * (double)a.N * (double)a.K;
+    const double rows_us = flops / (a.M <= 128 || a.K % (8 * kc) == 0 ? 0.78e9 : 0.26e9);
+    const double dense_us = (double)a.N * (double)a.K * (2.0 + wbits / 8.0) / 4.4e6 + gemm16_plan(a.M, a.N, a.K, 1).us;
+    return dense_us < rows_us;
+}
+uint64_t wq_dense_workspace(const OpsnnWqmmArgs& a)
+{
+    const Gemm16Plan pl = gemm16_plan(a.M, a.N, a.K, 1);
+    return dense_weight_bytes(a) + gemm16_part_bytes(pl, a.M, a.N, 1);
+}
+
+int launch_wq_dense(const OpsnnWqmmArgs& a, hipStream_t st)
+{
+    if (!a.workspace || !wq_dense_wanted(a)) return OPSNN_NOT_TAKEN;
+    const int wbits = a.w_dtype == DT_I4 ? 4 : 8;
+    const bool kn = a.w.row_stride != 1;
+    uint16_t* w16 = (uint16_t*)a.workspace;
+    WqParams p{};
+    p.w = (const uint8_t*)a.w.ptr;
+    p.ldw = (kn ? a.w.row_stride : a.w.col_stride) * wbits / 8;
+    p.scale = (const uint16_t*)a.scale.ptr; p.offset = (const uint16_t*)a.offset;
+    p.s_rs = a.scale.row_stride; p.s_cs = a.scale_n == 1 ? 0 : a.scale.col_stride;
+    p.M = a.M; p.N = a.N; p.K = a.K;
+    p.group = a.group > 0 ? a.group : a.K;
+    p.group_shift = (p.group & (p.group - 1)) == 0 ? __builtin_ctzll((unsigned long long)p.group) : p.group >= p.K ? 31 : -1;
+    const bool f16 = a.x_dtype == DT_F16;
+    int rc;
+    if (f16) {
+        if (wbits == 4) rc = a.offset ? launch_dequant<DT_F16, 4, true>(p, kn, w16, st) : launch_dequant<DT_F16, 4, false>(p, kn, w16, st);
+        else rc = a.offset ? launch_dequant<DT_F16, 8, true>(p, kn, w16, st) : launch_dequant<DT_F16, 8, false>(p, kn, w16, st);
+    } else {
+        if (wbits == 4) rc = a.offset ? launch_dequant<DT_BF16, 4, true>(p, kn, w16, st) : launch_dequant<DT_BF16, 4, false>(p, kn, w16, st);
+        else rc = a.offset ? launch_dequant<DT_BF16, 8, true>(p, kn, w16, st) : launch_dequant<DT_BF16, 8, false>(p, kn, w16, st);
+    }
+    if (rc != 0) return rc;
+    const Gemm16Plan pl = gemm16_plan(a.M, a.N, a.K, 1);
+    QgemmParams g{};
+    g.a = (const int8_t*)a.x; g.b = (const int8_t*)w16;
+    g.lda = 2 * a.K; g.ldb = 2 * a.K; g.KB = 2 * a.K;
+    g.out = a.y; g.M = a.M; g.N = a.N; g.ldc = a.N;
+    g.bias = a.bias; g.bias_dt = a.bias_dtype;
+    return launch_gemm16(g, pl, !f16, 1, a.x_dtype, (float*)((char*)a.workspace + dense_weight_bytes(a)), st);
+}
+
+}  // namespace opsnn
