@@ -33,27 +33,6 @@ __device__ __forceinline__ uint16_t bf16_bits(float f)
     u += 0x7fffu + ((u >> 16) & 1u);
     return (uint16_t)(u >> 16);
 }
-// Element i of the sum, in split order, of `splits` partial arrays of `total` elements each (the K split of the tile
-// kernels); four loads in flight at a time.
-template <typename T>
-__device__ __forceinline__ T splitk_sum(const T* part, int splits, int64_t total, int64_t i)
-{
-    T v = part[i];
-    int s = 1;
-    for (; s + 3 < splits; s += 4) {
-        const T a = part[(int64_t)s * total + i], b = part[(int64_t)(s + 1) * total + i];
-        const T c = part[(int64_t)(s + 2) * total + i], d = part[(int64_t)(s + 3) * total + i];
-        v = v + a; v = v + b; v = v + c; v = v + d;
-    }
-    for (; s < splits; s++) v = v + part[(int64_t)s * total + i];
-    return v;
-}
-// Blocks of 256 threads for a grid-stride loop with one element per thread and pass.
-inline unsigned splitk_reduce_grid(int64_t total)
-{
-    const int64_t want = (total + 255) / 256;
-    return (unsigned)(want < 1 ? 1 : want > (1 << 20) ? (1 << 20) : want);
-}
 __device__ __forceinline__ float bf16_to_f32(uint16_t h) { return u2f((uint32_t)h << 16); }
 __device__ __forceinline__ uint16_t f16_bits(float f)
 {
@@ -172,6 +151,71 @@ __device__ __forceinline__ float e8m0_to_f32(uint32_t b)
     if (b == 0xffu) return u2f(0x7fc00000u);
     if (b == 0u) return u2f(0x00400000u);
     return u2f(b << 23);
+}
+
+// The sum, in split order, of `splits` partial arrays [rows][N] that lie `slice` elements apart (the K split of every kernel
+// family), four neighbouring columns of one row per thread: emit(row, n0, cols, v) with cols = 4 except at the end of a
+// row.  The row comes from blockIdx.y and the columns from blockIdx.x, so no element costs a division (one 64-bit division is
+// several dozen instructions: with two or three of them per element the second kernel of a split took 106 us for 500 x 8192
+// outputs in two slices, where the 50 MB it moves are 10 us), and eight slices are in flight at a time.
+template <typename T, typename F>
+__device__ __forceinline__ void splitk_rows(const T* part, int splits, int64_t slice, int64_t rows, int64_t N, F&& emit)
+{
+    typedef T quad __attribute__((ext_vector_type(4)));
+    const int64_t n0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (n0 >= N) return;
+    const int cols = N - n0 < 4 ? (int)(N - n0) : 4;
+    const bool vec = (N % 4) == 0 && (slice % 4) == 0 && ((uintptr_t)part % 16) == 0;
+    for (int64_t row = blockIdx.y; row < rows; row += gridDim.y) {
+        const T* at = part + row * N + n0;
+        auto load = [&](int s) -> quad {
+            const T* q = at + (int64_t)s * slice;
+            if (vec) return *(const quad*)q;
+            quad r = {0, 0, 0, 0};
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (e < cols) r[e] = q[e];
+            return r;
+        };
+        quad v = load(0);
+        int s = 1;
+        for (; s + 7 < splits; s += 8) {
+            quad t[8];
+#pragma unroll
+            for (int j = 0; j < 8; j++) t[j] = load(s + j);
+#pragma unroll
+            for (int j = 0; j < 8; j++) v = v + t[j];
+        }
+        for (; s + 1 < splits; s += 2) {
+            const quad t0 = load(s), t1 = load(s + 1);
+            v = v + t0; v = v + t1;
+        }
+        if (s < splits) v = v + load(s);
+        emit(row, n0, cols, v);
+    }
+}
+inline dim3 splitk_rows_grid(int64_t rows, int64_t N)
+{
+    return dim3((unsigned)((N + 1023) / 1024), (unsigned)(rows < 65535 ? rows : 65535));
+}
+// cols (1 .. 4) neighbouring outputs of one row, rounded to out_dt (bf16, fp16 or fp32), at element `at` of out
+__device__ __forceinline__ void store_quad(void* out, int out_dt, int64_t at, int cols, v4f v)
+{
+    if (out_dt == DT_F32) {
+        float* o = (float*)out + at;
+        if (cols == 4 && ((uintptr_t)o % 16) == 0) { *(v4f*)o = v; return; }
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (e < cols) o[e] = v[e];
+        return;
+    }
+    const v4us q = out_dt == DT_BF16 ? (v4us){bf16_bits(v[0]), bf16_bits(v[1]), bf16_bits(v[2]), bf16_bits(v[3])}
+                                     : (v4us){f16_bits(v[0]), f16_bits(v[1]), f16_bits(v[2]), f16_bits(v[3])};
+    uint16_t* o = (uint16_t*)out + at;
+    if (cols == 4 && ((uintptr_t)o % 8) == 0) { *(v4us*)o = q; return; }
+#pragma unroll
+    for (int e = 0; e < 4; e++)
+        if (e < cols) o[e] = q[e];
 }
 
 // Decode element i of a dense buffer of 8-bit or 4-bit quantised values.

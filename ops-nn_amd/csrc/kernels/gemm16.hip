@@ -9,54 +9,21 @@ namespace opsnn {
 
 int launch_16_wide(const QgemmParams& p, int fn, bool bf16_operands, int64_t batch, int out_dt, hipStream_t st);   // qmm_int8_wide.hip
 
-// out[b, m, n] = rounded(sum over the splits, in split order, * x2s[n] * x1s[m] + bias[n]).  One row per blockIdx.y, four
-// columns per thread: no divisions (the row and column come from the block index), 16-byte loads where N % 4 == 0.
-template <int OUT_DT>
-__global__ __launch_bounds__(256) void gemm16_splitk_reduce_kernel(QgemmParams p, int64_t total)
+// out[b, m, n] = rounded(sum over the splits, in split order, * x2s[n] * x1s[m] + bias[n])
+__global__ __launch_bounds__(256) void gemm16_splitk_reduce_kernel(QgemmParams p, int64_t rows, int out_dt)
 {
-    const int64_t n0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
-    if (n0 >= p.N) return;
-    const float* part = (const float*)p.part;
-    const bool vec = (p.N % 4) == 0;
-    for (int64_t row = blockIdx.y; row < total / p.N; row += gridDim.y) {
-        const int64_t bz = row / p.M, m = row - bz * p.M, at = row * p.N + n0;
-        const int cols = p.N - n0 < 4 ? (int)(p.N - n0) : 4;
-        v4f v = {0, 0, 0, 0};
-        auto load = [&](int s) -> v4f {
-            const float* q = part + (int64_t)s * total + at;
-            if (vec) return *(const v4f*)q;
-            v4f r = {0, 0, 0, 0};
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (e < cols) r[e] = q[e];
-            return r;
-        };
-        v = load(0);
-        int s = 1;
-        for (; s + 3 < p.splits; s += 4) {
-            const v4f a = load(s), b = load(s + 1), c = load(s + 2), d = load(s + 3);
-            v = v + a; v = v + b; v = v + c; v = v + d;
-        }
-        for (; s < p.splits; s++) v = v + load(s);
+    splitk_rows((const float*)p.part, p.splits, rows * p.N, rows, p.N, [&](int64_t row, int64_t n0, int cols, v4f v) {
+        const int64_t bz = rows == p.M ? 0 : row / p.M, m = row - bz * p.M;
         const float s1 = p.x1s ? p.x1s[p.x1s_one ? 0 : m] : 1.0f;
-        uint16_t o[4];
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             const int64_t n = n0 + (e < cols ? e : cols - 1);
-            float t = v[e];
-            if (p.x2s) t = t * load_scalar_as_f32(p.x2s, p.x2s_dt, p.x2s_len == 1 ? 0 : n);
-            t = t * s1;
-            if (p.bias) t = t + load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + n);
-            o[e] = to_b16<OUT_DT>(t);
+            if (p.x2s) v[e] = v[e] * load_scalar_as_f32(p.x2s, p.x2s_dt, p.x2s_len == 1 ? 0 : n);
+            v[e] = v[e] * s1;
+            if (p.bias) v[e] = v[e] + load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + n);
         }
-        uint16_t* out = (uint16_t*)p.out + row * p.ldc + n0;
-        if (vec && ((uintptr_t)p.out % 8) == 0) *(v4us*)out = (v4us){o[0], o[1], o[2], o[3]};
-        else {
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (e < cols) out[e] = o[e];
-        }
-    }
+        store_quad(p.out, out_dt, row * p.ldc + n0, cols, v);
+    });
 }
 
 template <int MODE, int BM, int BN, int WGM, int WGN>
@@ -77,9 +44,7 @@ static int launch_split16(const QgemmParams& p, int64_t batch, int out_dt, hipSt
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     const int64_t rows = batch * p.M;
-    const dim3 grid((unsigned)((p.N + 1023) / 1024), (unsigned)(rows < 65535 ? rows : 65535));
-    if (out_dt == DT_BF16) hipLaunchKernelGGL(gemm16_splitk_reduce_kernel<DT_BF16>, grid, dim3(256), 0, st, p, rows * p.N);
-    else hipLaunchKernelGGL(gemm16_splitk_reduce_kernel<DT_F16>, grid, dim3(256), 0, st, p, rows * p.N);
+    hipLaunchKernelGGL(gemm16_splitk_reduce_kernel, splitk_rows_grid(rows, p.N), dim3(256), 0, st, p, rows, out_dt);
     return (int)hipGetLastError();
 }
 

@@ -59,10 +59,6 @@ struct QgemmParams {
     const uint8_t* sa;
     const uint8_t* sb;
     int64_t sa_rs, sb_rs, sa_bs, sb_bs;
-    // When set: the launch computes only if one of gate[0 .. gate_n) is non-zero (the flags of the pass that prepares the
-    // exact MX route, whose kernel then left the call to this one); otherwise every workgroup returns at once.
-    const int* gate;
-    int gate_n;
     // K split over `splits` workgroups per tile (SPLIT instantiations, grid.z): partial sums [splits][batch][M][N] -- int32
     // for MODE_I8 (qg_i8_splitk_reduce_kernel adds them exactly and applies the epilogue), fp32 with the MX scales applied
     // for the MX modes (qg_mx_splitk_reduce_kernel adds them in split order, then the bias)
@@ -136,13 +132,6 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave / WGN, wn = wave % WGN;
-    if constexpr (MX) {
-        if (p.gate) {
-            int f = 0;
-            for (int i = 0; i < p.gate_n; i++) f |= p.gate[i];   // every thread reads every flag: uniform loads, no LDS for a vote
-            if (!f) return;
-        }
-    }
 
     // Tile order: each XCD (own L2) gets a contiguous range of ids, and ids run down groups of GM row tiles and across the
     // columns inside a group, so that the 32 tiles an XCD works on at a time form a GM x (32 / GM) block sharing GM x1
@@ -730,51 +719,50 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
 
 // MODE_I8 after a K split: out[b, m, n] = rounded(fp32(sum of the partial sums + ib[n]) * x2s[n] * x1s[m] + fb[n]), the
 // terms as the tile kernel's epilogue stages them
-template <int OUT_DT>
-__global__ __launch_bounds__(256) void qg_i8_splitk_reduce_kernel(QgemmParams p, int64_t total)
+static __global__ __launch_bounds__(256) void qg_i8_splitk_reduce_kernel(QgemmParams p, int64_t rows, int out_dt)
 {
-    const int64_t MN = p.M * p.N, stride = (int64_t)gridDim.x * blockDim.x;
     const bool has_ib = p.bias && p.bias_dt == DT_I32, has_fb = p.bias && p.bias_dt != DT_I32;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        const int32_t a = splitk_sum(p.part, p.splits, total, i);
-        const int64_t bz = i / MN, m = (i % MN) / p.N, n = i % p.N;
-        const int64_t si = p.x2s_len == 1 ? 0 : n;
-        float sv = p.x2s_dt == DT_U64 ? u2f((uint32_t)((const uint64_t*)p.x2s)[si]) : load_scalar_as_f32(p.x2s, p.x2s_dt, si);
-        if (p.x2s_trunc || p.x2s_dt == DT_U64) sv = u2f(f2u(sv) & 0xFFFFE000u);
-        const int32_t ib = has_ib ? ((const int32_t*)p.bias)[bz * p.bias_bs + n] : 0;
-        const float fb = has_fb ? load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + n) : -0.0f;
+    splitk_rows(p.part, p.splits, rows * p.N, rows, p.N, [&](int64_t row, int64_t n0, int cols, v4i a) {
+        const int64_t bz = rows == p.M ? 0 : row / p.M, m = row - bz * p.M;
         const float s1 = p.x1s ? p.x1s[m] : 1.0f;
-        float tv = (float)(a + ib);
-        tv = tv * sv;
-        tv = tv * s1;
-        const float v = tv + fb;
-        ((uint16_t*)p.out)[(bz * p.M + m) * p.ldc + n] = OUT_DT == DT_BF16 ? bf16_bits(v) : f16_bits(v);
-    }
+        v4f v;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int64_t n = n0 + (e < cols ? e : cols - 1), si = p.x2s_len == 1 ? 0 : n;
+            float sv = p.x2s_dt == DT_U64 ? u2f((uint32_t)((const uint64_t*)p.x2s)[si]) : load_scalar_as_f32(p.x2s, p.x2s_dt, si);
+            if (p.x2s_trunc || p.x2s_dt == DT_U64) sv = u2f(f2u(sv) & 0xFFFFE000u);
+            const int32_t ib = has_ib ? ((const int32_t*)p.bias)[bz * p.bias_bs + n] : 0;
+            const float fb = has_fb ? load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + n) : -0.0f;
+            float tv = (float)(a[e] + ib);
+            tv = tv * sv;
+            tv = tv * s1;
+            v[e] = tv + fb;
+        }
+        store_quad(p.out, out_dt, row * p.ldc + n0, cols, v);
+    });
 }
 
 // The MX modes after a K split: out[b, m, n] = rounded(sum of the fp32 partial sums, in split order, + bias[n])
-template <int OUT_DT>
-__global__ __launch_bounds__(256) void qg_mx_splitk_reduce_kernel(QgemmParams p, int64_t total)
+static __global__ __launch_bounds__(256) void qg_mx_splitk_reduce_kernel(QgemmParams p, int64_t rows, int out_dt)
 {
-    const int64_t MN = p.M * p.N, stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        float v = splitk_sum((const float*)p.part, p.splits, total, i);
-        const int64_t bz = i / MN, m = (i % MN) / p.N, n = i % p.N;
-        if (p.bias) v = v + load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + n);
-        const int64_t o = (bz * p.M + m) * p.ldc + n;
-        if constexpr (OUT_DT == DT_F32) ((float*)p.out)[o] = v;
-        else ((uint16_t*)p.out)[o] = OUT_DT == DT_BF16 ? bf16_bits(v) : f16_bits(v);
-    }
+    splitk_rows((const float*)p.part, p.splits, rows * p.N, rows, p.N, [&](int64_t row, int64_t n0, int cols, v4f v) {
+        const int64_t bz = rows == p.M ? 0 : row / p.M;
+        if (p.bias) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = v[e] + load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + n0 + (e < cols ? e : cols - 1));
+        }
+        store_quad(p.out, out_dt, row * p.ldc + n0, cols, v);
+    });
 }
 
-// The K split of an MX mode (p.splits > 1, whole K tiles, no gate): the tile kernel per split, then the reduction.
+// The K split of an MX mode (p.splits > 1, whole K tiles): the tile kernel per split, then the reduction.
 template <int MODE, int BM, int BN, int BK, int WGM, int WGN, int STAGES, int MINWG>
 static int qgemm_launch_split_mx(const QgemmParams& p, int64_t batch, int out_dt, hipStream_t st)
 {
     static_assert(mode_is_mx(MODE), "the MX modes");
     constexpr int SCB = BK / (MODE == MODE_MXFP8 ? 32 : 16);
     constexpr int U = SCB == 8 ? 2 : 1;
-    if (!p.part || p.splits < 2 || p.gate || (p.KB % (BK * U)) != 0 || p.splits > p.KB / BK / U / 2) return -1;
+    if (!p.part || p.splits < 2 || (p.KB % (BK * U)) != 0 || p.splits > p.KB / BK / U / 2) return -1;
     int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
     dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch, (unsigned)p.splits);
     const size_t lds = SCB == 8 ? (size_t)STAGES * (BM + BN) * BK + 2 * (BM + BN) * 16 : (size_t)STAGES * ((BM + BN) * BK + (BM + BN) * SCB);
@@ -788,12 +776,8 @@ static int qgemm_launch_split_mx(const QgemmParams& p, int64_t batch, int out_dt
     hipLaunchKernelGGL(k, grid, dim3(WGM * WGN * 64), lds, st, p, tiles_m, tiles_n);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
-    const int64_t total = batch * p.M * p.N;
-    const unsigned rgrid = splitk_reduce_grid(total);
-    if (out_dt == DT_BF16) hipLaunchKernelGGL(qg_mx_splitk_reduce_kernel<DT_BF16>, dim3(rgrid), dim3(256), 0, st, p, total);
-    else if (out_dt == DT_F16) hipLaunchKernelGGL(qg_mx_splitk_reduce_kernel<DT_F16>, dim3(rgrid), dim3(256), 0, st, p, total);
-    else if (out_dt == DT_F32) hipLaunchKernelGGL(qg_mx_splitk_reduce_kernel<DT_F32>, dim3(rgrid), dim3(256), 0, st, p, total);
-    else return -2;
+    if (out_dt != DT_BF16 && out_dt != DT_F16 && out_dt != DT_F32) return -2;
+    hipLaunchKernelGGL(qg_mx_splitk_reduce_kernel, splitk_rows_grid(batch * p.M, p.N), dim3(256), 0, st, p, batch * p.M, out_dt);
     return (int)hipGetLastError();
 }
 
@@ -816,10 +800,7 @@ static int qgemm_launch_split_i8(const QgemmParams& p, int64_t batch, int out_dt
     hipLaunchKernelGGL(k, grid, dim3(WGM * WGN * 64), lds, st, p, tiles_m, tiles_n);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
-    const int64_t total = batch * p.M * p.N;
-    const unsigned rgrid = splitk_reduce_grid(total);
-    if (out_dt == DT_BF16) hipLaunchKernelGGL(qg_i8_splitk_reduce_kernel<DT_BF16>, dim3(rgrid), dim3(256), 0, st, p, total);
-    else hipLaunchKernelGGL(qg_i8_splitk_reduce_kernel<DT_F16>, dim3(rgrid), dim3(256), 0, st, p, total);
+    hipLaunchKernelGGL(qg_i8_splitk_reduce_kernel, splitk_rows_grid(batch * p.M, p.N), dim3(256), 0, st, p, batch * p.M, out_dt);
     return (int)hipGetLastError();
 }
 

@@ -489,16 +489,17 @@ __global__ __launch_bounds__(WGM * 128, 1) void qmm_fp8_block_kernel(Fp8BlkParam
 }
 
 // out[b, m, n] = rounded(sum over the splits, in split order, of part[s, b, m, n] + bias[b, n])
-template <int OUT_DT>
-__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* part, int splits, int64_t total, int64_t MN, int64_t N,
-                                                            const void* bias, int bias_dt, int64_t bias_bs, uint16_t* out)
+__global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* part, int splits, int64_t rows, int64_t M, int64_t N,
+                                                            const void* bias, int bias_dt, int64_t bias_bs, void* out, int out_dt)
 {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        float v = splitk_sum(part, splits, total, i);
-        if (bias) v = v + load_scalar_as_f32(bias, bias_dt, (i / MN) * bias_bs + i % N);
-        out[i] = OUT_DT == DT_BF16 ? bf16_bits(v) : f16_bits(v);
-    }
+    splitk_rows(part, splits, rows * N, rows, N, [&](int64_t row, int64_t n0, int cols, v4f v) {
+        const int64_t bz = rows == M ? 0 : row / M;
+        if (bias) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = v[e] + load_scalar_as_f32(bias, bias_dt, bz * bias_bs + n0 + (e < cols ? e : cols - 1));
+        }
+        store_quad(out, out_dt, row * N + n0, cols, v);
+    });
 }
 
 template <int WGM, int STAGES, int OUT_DT, int MODE = FP8_BLOCK>
@@ -522,10 +523,8 @@ static int launch_fp8_block(const Fp8BlkParams& p, int64_t batch, hipStream_t st
             hipLaunchKernelGGL(ks, grid, dim3(WGM * 128), lds, st, p, tiles_m, tiles_n);
             hipError_t e = hipGetLastError();
             if (e != hipSuccess) return (int)e;
-            const int64_t total = batch * p.M * p.N;
-            const unsigned rgrid = splitk_reduce_grid(total);
-            hipLaunchKernelGGL(splitk_reduce_kernel<OUT_DT>, dim3(rgrid), dim3(256), 0, st, (const float*)p.part, p.splits, total,
-                               p.M * p.N, p.N, (const void*)p.bias, MODE == FP8_MX_W4 ? p.bias_dt : DT_F32, p.bias_bs, (uint16_t*)p.out);
+            hipLaunchKernelGGL(splitk_reduce_kernel, splitk_rows_grid(batch * p.M, p.N), dim3(256), 0, st, (const float*)p.part, p.splits, batch * p.M,
+                               p.M, p.N, (const void*)p.bias, MODE == FP8_MX_W4 ? p.bias_dt : DT_F32, p.bias_bs, p.out, OUT_DT);
             return (int)hipGetLastError();
         }
     }

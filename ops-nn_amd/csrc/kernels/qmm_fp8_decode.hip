@@ -210,16 +210,15 @@ __global__ __launch_bounds__(NW * 64) void fp8_block_decode_kernel(Fp8DecParams 
 template <bool RC>
 __global__ __launch_bounds__(256) void fp8dec_reduce_kernel(Fp8DecParams p, int splits)
 {
-    const int64_t total = p.M * p.N, stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        float v = p.part[i];
-        for (int s = 1; s < splits; s++) v = v + p.part[(int64_t)s * p.part_slice + i];
-        const int64_t m = i / p.N, n = i - m * p.N;
-        if constexpr (RC) v = (v * p.cs[n * p.cs_stride]) * p.rs[m * p.rs_stride];
-        if (p.bias) v = v + p.bias[n];
-        if (p.out_dt == DT_F32) ((float*)p.out)[i] = v;
-        else ((uint16_t*)p.out)[i] = p.out_dt == DT_BF16 ? bf16_bits(v) : f16_bits(v);
-    }
+    splitk_rows((const float*)p.part, splits, p.part_slice, p.M, p.N, [&](int64_t m, int64_t n0, int cols, v4f v) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            const int64_t n = n0 + (e < cols ? e : cols - 1);
+            if constexpr (RC) v[e] = (v[e] * p.cs[n * p.cs_stride]) * p.rs[m * p.rs_stride];
+            if (p.bias) v[e] = v[e] + p.bias[n];
+        }
+        store_quad(p.out, p.out_dt, m * p.N + n0, cols, v);
+    });
 }
 
 template <int NW, int NBLK, bool RC, bool I8 = false, bool SEG = false>
@@ -236,7 +235,7 @@ int launch_decode_one(const Fp8DecParams& p, hipStream_t st, int splits = 1)
     const size_t lds = (size_t)2 * NW * 256 * sizeof(float);
     hipLaunchKernelGGL((fp8_block_decode_kernel<NW, NBLK, RC, I8, SEG>), dim3((unsigned)grid, (unsigned)splits), dim3(NW * 64), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
-    hipLaunchKernelGGL(fp8dec_reduce_kernel<RC>, dim3(splitk_reduce_grid(p.M * p.N)), dim3(256), 0, st, p, splits);
+    hipLaunchKernelGGL(fp8dec_reduce_kernel<RC>, splitk_rows_grid(p.M, p.N), dim3(256), 0, st, p, splits);
     return (int)hipGetLastError();
 }
 
@@ -401,13 +400,13 @@ __global__ __launch_bounds__(NW * 64) void mx_a8w4_decode_kernel(MxW4DecParams p
 // out = cast(sum over the K segments, in order, of part[s] + bias) for one pass of up to 16 rows
 __global__ __launch_bounds__(256) void mxw4dec_reduce_kernel(MxW4DecParams p, int splits)
 {
-    const int64_t total = p.M * p.N, stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        float v = p.part[i];
-        for (int s = 1; s < splits; s++) v = v + p.part[(int64_t)s * p.part_slice + i];
-        if (p.bias) v = v + load_scalar_as_f32(p.bias, p.bias_dt, i % p.N);
-        ((uint16_t*)p.out)[i] = p.out_dt == DT_BF16 ? bf16_bits(v) : f16_bits(v);
-    }
+    splitk_rows((const float*)p.part, splits, p.part_slice, p.M, p.N, [&](int64_t m, int64_t n0, int cols, v4f v) {
+        if (p.bias) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = v[e] + load_scalar_as_f32(p.bias, p.bias_dt, n0 + (e < cols ? e : cols - 1));
+        }
+        store_quad(p.out, p.out_dt, m * p.N + n0, cols, v);
+    });
 }
 
 template <int NW, int NCH, bool SEG = false>
@@ -424,7 +423,7 @@ int launch_mxw4_one(const MxW4DecParams& p, hipStream_t st, int splits = 1)
     const size_t lds = (size_t)2 * NW * 256 * sizeof(float);
     hipLaunchKernelGGL((mx_a8w4_decode_kernel<NW, NCH, SEG>), dim3((unsigned)grid, (unsigned)splits), dim3(NW * 64), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
-    hipLaunchKernelGGL(mxw4dec_reduce_kernel, dim3(splitk_reduce_grid(p.M * p.N)), dim3(256), 0, st, p, splits);
+    hipLaunchKernelGGL(mxw4dec_reduce_kernel, splitk_rows_grid(p.M, p.N), dim3(256), 0, st, p, splits);
     return (int)hipGetLastError();
 }
 
@@ -577,14 +576,13 @@ __global__ __launch_bounds__(NW * 64) void mx8_decode_kernel(Mx8DecParams p)
 // out = cast(sum over the K segments, in order, of part[s] + bias) for one pass of up to 16 rows
 __global__ __launch_bounds__(256) void mx8dec_reduce_kernel(Mx8DecParams p, int splits)
 {
-    const int64_t total = p.M * p.N, stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        float v = p.part[i];
-        for (int s = 1; s < splits; s++) v = v + p.part[(int64_t)s * p.part_slice + i];
-        if (p.bias) v = v + p.bias[i % p.N];
-        if (p.out_dt == DT_F32) ((float*)p.out)[i] = v;
-        else ((uint16_t*)p.out)[i] = p.out_dt == DT_BF16 ? bf16_bits(v) : f16_bits(v);
-    }
+    splitk_rows((const float*)p.part, splits, p.part_slice, p.M, p.N, [&](int64_t m, int64_t n0, int cols, v4f v) {
+        if (p.bias) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = v[e] + p.bias[n0 + (e < cols ? e : cols - 1)];
+        }
+        store_quad(p.out, p.out_dt, m * p.N + n0, cols, v);
+    });
 }
 
 template <int NW, int NBLK>
@@ -598,7 +596,7 @@ int launch_mx8_one(const Mx8DecParams& p, hipStream_t st, int splits)
     const size_t lds = (size_t)2 * NW * 256 * sizeof(float);
     hipLaunchKernelGGL((mx8_decode_kernel<NW, NBLK>), dim3((unsigned)grid, (unsigned)splits), dim3(NW * 64), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
-    hipLaunchKernelGGL(mx8dec_reduce_kernel, dim3(splitk_reduce_grid(p.M * p.N)), dim3(256), 0, st, p, splits);
+    hipLaunchKernelGGL(mx8dec_reduce_kernel, splitk_rows_grid(p.M, p.N), dim3(256), 0, st, p, splits);
     return (int)hipGetLastError();
 }
 

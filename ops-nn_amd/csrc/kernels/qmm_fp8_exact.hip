@@ -51,17 +51,10 @@ struct Fp8xParams {
     int64_t bias_bs;
     int64_t rs_bs, cs_bs;   // batch strides of rs / cs in elements (0: shared by all batches)
     // MX mode (template flag MXS): one e8m0 byte per 32 K and row, four per K tile (sa, sb: K-contiguous, 4-byte aligned
-    // rows).  Every row has a base exponent; the widening conversion multiplies a block by 2^(byte - base), exactly (the
-    // result is an fp16 value as long as byte - base is in [-15, 7]), and 2^(base - 127) comes back in through rs / cs.
-    // a_c / b_c hold 127 - base per row; gate[0 .. gate_n) are flags of the pass that chose the bases: any flag set means
-    // some row's bytes do not fit that window, and the kernel leaves the whole call to the launch that follows it.
+    // rows), folded into the widening to bf16; cs is null and the epilogue adds the bias only.
     const uint8_t* sa;
     const uint8_t* sb;
     int64_t sa_rs, sb_rs, sa_bs, sb_bs;
-    const int* a_c;
-    const int* b_c;
-    const int* gate;
-    int gate_n;
     // K split over `splits` workgroups per tile (SPLIT instantiations, grid.z): fp32 partial sums [splits][batch][M][N] --
     // block scales already applied, row / column scales and bias not yet (fp8x_splitk_reduce_kernel applies them)
     int splits;
@@ -96,34 +89,37 @@ template <bool E5> __device__ __forceinline__ v8h widen8(int d0, int d1)
     return (v8h){a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
-// the same with the power of two `sc` multiplied in (e4m3 only): exact while the scaled value is an fp16 value
+// the MX form: two of a dword's four e4m3 codes -> bf16 with the power of two `sc` multiplied in (the bits of a bf16 pair, carried
+// in the fp16 vector type of the other forms): exact wherever fp32 itself would hold the scaled value
+template <bool HI> __device__ __forceinline__ v2h cvt_mx(uint32_t d, float sc) { return __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d, sc, HI)); }
 __device__ __forceinline__ v8h widen8_scaled(int d0, int d1, float sc)
 {
-    const v2h a = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((uint32_t)d0, sc, false), b = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((uint32_t)d0, sc, true);
-    const v2h c = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((uint32_t)d1, sc, false), d = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((uint32_t)d1, sc, true);
+    const v2h a = cvt_mx<false>((uint32_t)d0, sc), b = cvt_mx<true>((uint32_t)d0, sc);
+    const v2h c = cvt_mx<false>((uint32_t)d1, sc), d = cvt_mx<true>((uint32_t)d1, sc);
     return (v8h){a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
 // FMT: bit 0 set = x1 holds e5m2 codes, bit 1 set = x2 does (else e4m3)
-// MXS: MX block scales (e8m0 per 32 K) folded into the widening conversion; row / column epilogue (RC) with the bases
-// The epilogue of the row / column scale forms for one output (Fp8xParams::ep_mode); rs = the row's scale (1 if none)
-__device__ __forceinline__ float fp8x_rowcol_epilogue(const Fp8xParams& p, float v, float rs, int64_t bz, int64_t ni)
+// MXS: MX block scales (e8m0 per 32 K) folded into the widening conversion, to bf16; the epilogue (RC) only adds the bias
+// The epilogue of the row / column scale forms (Fp8xParams::ep_mode): the column's scale and bias (neutral elements where there
+// are none), and the operations on one output; rs = the row's scale (1 if none).  -0.0f + v is v for every v.
+__device__ __forceinline__ float fp8x_col_scale(const Fp8xParams& p, int64_t bz, int64_t ni)
 {
+    if (!p.cs) return 1.0f;   // MX: the scales are in the sum
     const int64_t ci = bz * p.cs_bs + ni * p.cs_stride;
-    float csv;
-    if (p.cs_dt == DT_U64) csv = u2f((uint32_t)((const uint64_t*)p.cs)[ci] & 0xFFFFE000u);
-    else if (p.cs_dt == DT_BF16) csv = bf16_to_f32(((const uint16_t*)p.cs)[ci]);
-    else csv = ((const float*)p.cs)[ci];
-    if (p.ep_mode == 1) {
-        if (p.bias) v = v + load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + ni);
-        v = v * csv;
-    } else if (p.ep_mode == 2) {
-        v = v * u2f(f2u(csv * rs) & 0xFFFFE000u);
-    } else {
-        v = (v * csv) * rs;
-        if (p.bias) v = v + load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + ni);
-    }
-    return v;
+    if (p.cs_dt == DT_U64) return u2f((uint32_t)((const uint64_t*)p.cs)[ci] & 0xFFFFE000u);
+    if (p.cs_dt == DT_BF16) return bf16_to_f32(((const uint16_t*)p.cs)[ci]);
+    return ((const float*)p.cs)[ci];
+}
+__device__ __forceinline__ float fp8x_col_bias(const Fp8xParams& p, int64_t bz, int64_t ni)
+{
+    return p.bias ? load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + ni) : -0.0f;
+}
+__device__ __forceinline__ float fp8x_rowcol_epilogue(int ep_mode, float v, float rs, float csv, float bias)
+{
+    if (ep_mode == 1) return (v + bias) * csv;
+    if (ep_mode == 2) return v * u2f(f2u(csv * rs) & 0xFFFFE000u);
+    return (v * csv) * rs + bias;
 }
 
 template <int OUT_DT, bool RC, int FMT = 0, bool MXS = false, bool SPLIT = false>
@@ -152,11 +148,6 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-    if constexpr (MXS) {
-        int f = 0;
-        for (int i = 0; i < p.gate_n; i++) f |= p.gate[i];   // (every thread reads every flag: uniform loads)
-        if (f) return;   // some row's scale bytes do not fit the exact window: the next launch computes the call
-    }
 
     // Tile order: each XCD (own L2) gets a contiguous range of ids, and ids run down groups of GM row tiles and across
     // the columns inside a group, so the 32 tiles an XCD works on at a time form a GM x (32 / GM) block that shares
@@ -278,28 +269,17 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
     float sc[FM], scp[FM], s1raw[FM], s2raw = 0.0f;
     v4f part[2][FM];
     (void)sc; (void)scp; (void)s1raw; (void)s2raw; (void)part;
-    // MX: raw scale dwords of the tile being converted (one per fragment row of this lane), 127 - base of those rows, and
-    // the powers of two for the lane's two K blocks of a tile: bytes [16q, 16q+16) lie in block q/2, [64+16q, ..) in 2 + q/2
+    // MX: raw scale dwords of the tile being converted (one per fragment row of this lane) and the powers of two for the lane's two K blocks of a tile: bytes [16q, 16q+16) lie in block q/2, [64+16q, ..) in 2 + q/2
     uint32_t a_sraw[FM], b_sraw[FN];
-    int a_c[FM], b_c[FN];
     float a_lo[FM], a_hi[FM], b_lo[FN], b_hi[FN];
-    (void)a_sraw; (void)b_sraw; (void)a_c; (void)b_c; (void)a_lo; (void)a_hi; (void)b_lo; (void)b_hi;
+    (void)a_sraw; (void)b_sraw; (void)a_lo; (void)a_hi; (void)b_lo; (void)b_hi;
     const int sblk = 8 * (fq >> 1);
-    if constexpr (MXS) {
-#pragma unroll
-        for (int j = 0; j < FM; j++) {
-            const int r = wm * TM + j * 16 + frow;
-            a_c[j] = p.a_c[bz * p.rs_bs + m0 + (r < a_rows ? r : a_rows - 1)];
-        }
-#pragma unroll
-        for (int i = 0; i < FN; i++) {
-            const int r = wn * TN + i * 16 + frow;
-            b_c[i] = p.b_c[bz * p.cs_bs + n0 + (r < b_rows ? r : b_rows - 1)];
-        }
-    }
-    auto mx_pow = [&](uint32_t raw, int c, float& lo, float& hi) {
-        lo = u2f((((raw >> sblk) & 0xFFu) + (uint32_t)c) << 23);
-        hi = u2f((((raw >> (16 + sblk)) & 0xFFu) + (uint32_t)c) << 23);
+    // 2^(byte - 127) as the conversion's scale operand, which is read as an exponent only: exponent 0 is 2^-127 and 255 gives
+    // NaN results (both checked on the device), as the e8m0 codes 0 and 255 mean
+    auto mx_pow = [&](uint32_t raw, float& lo, float& hi) {
+        const uint32_t t = raw >> sblk;
+        lo = u2f((t << 23) & 0x7F800000u);
+        hi = u2f((t << 7) & 0x7F800000u);
     };
     auto read_scales = [&](const char* st) {
         if constexpr (MXS) {
@@ -318,8 +298,8 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
     auto widen4 = [&](int d, v8h& h, int half, float scl) {   // four bytes -> elements 4*half .. 4*half+3
         v2h lo, hi;
         if constexpr (MXS) {
-            lo = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((uint32_t)d, scl, false);
-            hi = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8((uint32_t)d, scl, true);
+            lo = cvt_mx<false>((uint32_t)d, scl);
+            hi = cvt_mx<true>((uint32_t)d, scl);
         } else {
             lo = cvt_lo<BE5>((uint32_t)d); hi = cvt_hi<BE5>((uint32_t)d);
         }
@@ -334,8 +314,8 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
         if constexpr (MXS) {
 #pragma unroll
             for (int j = 0; j < FM; j++) {
-                mx_pow(a_sraw[j], a_c[j], a_lo[j], a_hi[j]);
-                mx_pow(b_sraw[j], b_c[j], b_lo[j], b_hi[j]);
+                mx_pow(a_sraw[j], a_lo[j], a_hi[j]);
+                mx_pow(b_sraw[j], b_lo[j], b_hi[j]);
             }
         }
 #pragma unroll
@@ -415,7 +395,9 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
             for (int s = 0; s < 4; s++) {
 #pragma unroll
                 for (int j = 0; j < FM; j++) {
-                    if constexpr (RC) {
+                    if constexpr (MXS) {
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, fbc[i & 1][s]), __builtin_bit_cast(v8bf, fa[j][s]), acc[i][j], 0, 0, 0);
+                    } else if constexpr (RC) {
                         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fbc[i & 1][s], fa[j][s], acc[i][j], 0, 0, 0);
                     } else {
                         part[i & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fbc[i & 1][s], fa[j][s], s == 0 ? v4f{0.0f, 0.0f, 0.0f, 0.0f} : part[i & 1][j], 0, 0, 0);
@@ -428,8 +410,8 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
                         // current tile's has been issued (x2 fragments 1 .. FN-1 during the earlier fragments, the x1 high
                         // halves during the first)
                         if (i == FN - 1 && s == 1) {
-                            mx_pow(a_sraw[j], a_c[j], a_lo[j], a_hi[j]);
-                            mx_pow(b_sraw[j], b_c[j], b_lo[j], b_hi[j]);
+                            mx_pow(a_sraw[j], a_lo[j], a_hi[j]);
+                            mx_pow(b_sraw[j], b_lo[j], b_hi[j]);
                         }
                     }
                     if (s >= 2) {   // next x2 fragment: half a K step per instruction
@@ -515,9 +497,20 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
     uint16_t* out = (uint16_t*)p.out + bz * p.M * p.N;
     const bool vec_ok = (p.N % 8) == 0 && ((uintptr_t)p.out % 16) == 0;
     const int er = lane >> 3, ec = lane & 7;
+    // (the terms of a lane's 16 columns are fetched once, not once per row block)
     float rs_j[FM];
-    (void)rs_j;
+    v4f csv[FN], cbv[FN];
+    (void)rs_j; (void)csv; (void)cbv;
     if constexpr (RC) {
+#pragma unroll
+        for (int i = 0; i < FN; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                int64_t n = n0 + wn * TN + i * 16 + 4 * fq + r;
+                n = n < p.N ? n : p.N - 1;
+                csv[i][r] = fp8x_col_scale(p, bz, n);
+                cbv[i][r] = fp8x_col_bias(p, bz, n);
+            }
 #pragma unroll
         for (int j = 0; j < FM; j++) {
             const int64_t mrow = m0 + wm * TM + j * 16 + frow;
@@ -530,9 +523,8 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
         for (int i = 0; i < FN; i++) {
             v4f v = acc[i][j];
             if constexpr (RC) {   // (sum * x2Scale[n]) * x1Scale[m] + bias[n], each operation rounded, as compute_pertoken orders them
-                const int64_t nb = n0 + wn * TN + i * 16 + 4 * fq;
 #pragma unroll
-                for (int r = 0; r < 4; r++) v[r] = fp8x_rowcol_epilogue(p, v[r], rs_j[j], bz, nb + r < p.N ? nb + r : p.N - 1);
+                for (int r = 0; r < 4; r++) v[r] = fp8x_rowcol_epilogue(p.ep_mode, v[r], rs_j[j], csv[i][r], cbv[i][r]);
             }
             if constexpr (OUT_DT == DT_F32) {
                 // fp32 output: the lane's four neighbouring columns are 16 bytes, four lanes a 64-byte piece of a row: stored as they are
@@ -572,25 +564,22 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
 }
 
 // out[b, m, n] = the sum over the splits, in split order, of part[s, b, m, n], then the row / column epilogue (RC) and
-// the rounding.  With gate flags (the MX mode) nothing is written when one is set: the launch that follows computes the call.
-template <int OUT_DT, bool RC>
-__global__ __launch_bounds__(256) void fp8x_splitk_reduce_kernel(Fp8xParams p, int64_t total)
+// the rounding
+template <bool RC>
+__global__ __launch_bounds__(256) void fp8x_splitk_reduce_kernel(Fp8xParams p, int64_t rows, int out_dt)
 {
-    if (p.gate) {
-        int f = 0;
-        for (int i = 0; i < p.gate_n; i++) f |= p.gate[i];
-        if (f) return;
-    }
-    const int64_t MN = p.M * p.N, stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        float v = splitk_sum(p.part, p.splits, total, i);
+    splitk_rows((const float*)p.part, p.splits, rows * p.N, rows, p.N, [&](int64_t row, int64_t n0, int cols, v4f v) {
         if constexpr (RC) {
-            const int64_t bz = i / MN, m = (i % MN) / p.N, n = i % p.N;
-            v = fp8x_rowcol_epilogue(p, v, p.rs ? p.rs[bz * p.rs_bs + m * p.rs_stride] : 1.0f, bz, n);
+            const int64_t bz = rows == p.M ? 0 : row / p.M, m = row - bz * p.M;
+            const float rs = p.rs ? p.rs[bz * p.rs_bs + m * p.rs_stride] : 1.0f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int64_t n = n0 + (e < cols ? e : cols - 1);
+                v[e] = fp8x_rowcol_epilogue(p.ep_mode, v[e], rs, fp8x_col_scale(p, bz, n), fp8x_col_bias(p, bz, n));
+            }
         }
-        if constexpr (OUT_DT == DT_F32) ((float*)p.out)[i] = v;
-        else ((uint16_t*)p.out)[i] = OUT_DT == DT_BF16 ? bf16_bits(v) : f16_bits(v);
-    }
+        store_quad(p.out, out_dt, row * p.N + n0, cols, v);
+    });
 }
 
 template <int OUT_DT, bool RC, int FMT = 0, bool MXS = false>
@@ -612,9 +601,7 @@ static int launch_fp8_exact(const Fp8xParams& p, int64_t batch, hipStream_t st)
         hipLaunchKernelGGL(ks, grid, dim3(512), lds, st, p, tiles_m, tiles_n);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
-        const int64_t total = batch * p.M * p.N;
-        const unsigned rgrid = splitk_reduce_grid(total);
-        hipLaunchKernelGGL((fp8x_splitk_reduce_kernel<OUT_DT, RC>), dim3(rgrid), dim3(256), 0, st, p, total);
+        hipLaunchKernelGGL(fp8x_splitk_reduce_kernel<RC>, splitk_rows_grid(batch * p.M, p.N), dim3(256), 0, st, p, batch * p.M, OUT_DT);
         return (int)hipGetLastError();
     }
     auto k = qmm_fp8_exact_kernel<OUT_DT, RC, FMT, MXS>;
@@ -690,50 +677,10 @@ int launch_rowcol_exact(const OpsnnQmmArgs& a, hipStream_t st, int ep_mode, Spli
 }
 
 // ---- MX (e8m0 scale per 32 K) on exact products ----
-// Per row of a scale table [rows, K/32] (K-contiguous, nd = K/128 dwords per row): base = max byte - 7, c = 127 - base and
-// 2^(base - 127).  With byte - base in [-15, 7] an e4m3 value times 2^(byte - base) is an fp16 value (largest 448 * 2^7,
-// smallest 2^-9 * 2^-15 = 2^-24).  flags[block] = 1 when one of the block's rows holds a byte below max - 22 or the NaN
-// code 255.  One wave per row at a time, 64 rows per workgroup.
-__global__ __launch_bounds__(256) void mx_row_base_kernel(const uint8_t* __restrict__ s, int64_t rs, int64_t bs, int64_t rows, int64_t total, int nd,
-                                                          int* __restrict__ c_out, float* __restrict__ pow_out, int* __restrict__ flags)
-{
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int bad = 0;
-    for (int i = 0; i < 16; i++) {
-        const int64_t r = (int64_t)blockIdx.x * 64 + wave * 16 + i;
-        if (r >= total) break;
-        const uint32_t* row = (const uint32_t*)(s + (r / rows) * bs + (r % rows) * rs);
-        uint32_t mn = 255, mx = 0;
-        for (int d = lane; d < nd; d += 64) {
-            const uint32_t w = row[d];
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                const uint32_t v = (w >> (8 * b)) & 0xFFu;
-                mn = v < mn ? v : mn;
-                mx = v > mx ? v : mx;
-            }
-        }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const uint32_t a = (uint32_t)__shfl_xor((int)mn, o), b = (uint32_t)__shfl_xor((int)mx, o);
-            mn = a < mn ? a : mn;
-            mx = b > mx ? b : mx;
-        }
-        const int base = (int)mx - 7;
-        if (lane == 0) {
-            c_out[r] = 127 - base;
-            pow_out[r] = ldexpf(1.0f, base - 127);
-        }
-        bad |= (mx == 255u || mx - mn > 22u) ? 1 : 0;
-    }
-    const int any = __syncthreads_or(bad);
-    if (threadIdx.x == 0) flags[blockIdx.x] = any ? 1 : 0;
-}
-
 static inline uint64_t up256(uint64_t v) { return (v + 255) / 256 * 256; }
 
-// Bytes of workspace the exact MXFP8 route wants in front of everything else: 127 - base and 2^(base - 127) per row of
-// both operands, and the flags.
+// What phase 1 has always put in front of the workspace of an MXFP8 call.  The kernel below no longer needs the tables that it
+// was for; the size stays what callers of phase 1 have planned with.
 uint64_t mx_exact_bytes(const OpsnnQmmArgs& a)
 {
     if (a.x1_dtype != DT_E4M3 || a.x2_dtype != DT_E4M3) return 0;
@@ -742,18 +689,19 @@ uint64_t mx_exact_bytes(const OpsnnQmmArgs& a)
     return up256(rows * 8) + up256(((rows + 63) / 64 + 2) * 4);
 }
 
-// MXFP8 with exact products: the bases pass, this kernel, and -- computing
-// only when a flag is set -- the tile kernel on the scaled 8-bit instruction.  `a`: both operands e4m3, K-contiguous,
-// K % 128 == 0, scale rows K-contiguous; `region`: mx_exact_bytes(a) bytes.  OPSNN_NOT_TAKEN before anything is launched.
-int launch_mx_exact(const OpsnnQmmArgs& a, void* region, hipStream_t st, SplitK sk)
+// MXFP8 with exact products, one launch: an e4m3 value times the power of two of its block is a bf16 value wherever fp32 itself
+// would hold it, so both operands are widened to bf16 with their block's scale as the conversion's scale operand and
+// v_mfma_f32_16x16x32_bf16 sums exact products in fp32 -- the arithmetic of mx8_decode_kernel.  (Widened to fp16 the scaled
+// values need a base per row: two passes over the scale tables in front and a gated launch of the scaled-instruction kernel
+// behind, for rows whose scales spread too far -- 42 us of the 215 us that 500 x 8192 x 8192 took.)  `a`: both operands e4m3,
+// K-contiguous, K % 128 == 0, scale rows K-contiguous.
+int launch_mx_exact(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
 {
-    if (!region || (uintptr_t)region % 16) return OPSNN_NOT_TAKEN;
     if (a.x1_dtype != DT_E4M3 || a.x2_dtype != DT_E4M3) return OPSNN_NOT_TAKEN;
     if (a.out_dtype != DT_BF16 && a.out_dtype != DT_F16 && a.out_dtype != DT_F32) return OPSNN_NOT_TAKEN;
     if (a.bias && a.bias_dtype != DT_F32 && a.bias_dtype != DT_BF16 && a.bias_dtype != DT_F16) return OPSNN_NOT_TAKEN;
     if (a.K % 128 != 0 || a.M * a.N < 64 * 64 || a.x1.col_stride != 1 || a.x2.row_stride != 1) return OPSNN_NOT_TAKEN;
     if (a.x1_scale_mat.col_stride != 2 || a.x2_scale_mat.col_stride != 2) return OPSNN_NOT_TAKEN;
-    const int64_t nb1 = a.x1_scale_mat.batch_stride == 0 ? 1 : a.batch, nb2 = a.x2_scale_mat.batch_stride == 0 ? 1 : a.batch;
     Fp8xParams p{};
     p.a = (const int8_t*)a.x1.ptr; p.b = (const int8_t*)a.x2.ptr;
     p.lda = a.x1.row_stride; p.ldb = a.x2.col_stride; p.a_bs = a.x1.batch_stride; p.b_bs = a.x2.batch_stride;
@@ -763,35 +711,11 @@ int launch_mx_exact(const OpsnnQmmArgs& a, void* region, hipStream_t st, SplitK 
     p.sa_bs = a.x1_scale_mat.batch_stride; p.sb_bs = a.x2_scale_mat.batch_stride;
     if (((uintptr_t)p.a | (uintptr_t)p.b | (uint64_t)p.lda | (uint64_t)p.ldb | (uint64_t)p.a_bs | (uint64_t)p.b_bs) % 16) return OPSNN_NOT_TAKEN;
     if (((uintptr_t)p.sa | (uintptr_t)p.sb | (uint64_t)p.sa_rs | (uint64_t)p.sb_rs | (uint64_t)p.sa_bs | (uint64_t)p.sb_bs) % 4) return OPSNN_NOT_TAKEN;
-    const int64_t rows1 = nb1 * a.M, rows2 = nb2 * a.N;
-    const uint64_t all_rows = (uint64_t)a.batch * (uint64_t)(a.M + a.N);
-    int* c1 = (int*)region;
-    int* c2 = c1 + rows1;
-    float* pw1 = (float*)((char*)region + all_rows * 4);
-    float* pw2 = pw1 + rows1;
-    int* flags = (int*)((char*)region + up256(all_rows * 8));
-    const int g1 = (int)((rows1 + 63) / 64), g2 = (int)((rows2 + 63) / 64), nd = (int)(a.K / 128);
-    hipLaunchKernelGGL(mx_row_base_kernel, dim3((unsigned)g1), dim3(256), 0, st, p.sa, p.sa_rs, p.sa_bs, a.M, rows1, nd, c1, pw1, flags);
-    hipLaunchKernelGGL(mx_row_base_kernel, dim3((unsigned)g2), dim3(256), 0, st, p.sb, p.sb_rs, p.sb_bs, a.N, rows2, nd, c2, pw2, flags + g1);
-    p.a_c = c1; p.b_c = c2;
-    p.rs = pw1; p.rs_stride = 1; p.rs_bs = nb1 == 1 ? 0 : a.M;
-    p.cs = pw2; p.cs_stride = 1; p.cs_bs = nb2 == 1 ? 0 : a.N; p.cs_dt = DT_F32;
-    p.ep_mode = 0;
     p.bias = a.bias; p.bias_dt = a.bias_dtype; p.bias_bs = a.bias_batch_stride;
-    p.gate = flags; p.gate_n = g1 + g2;
     p.splits = sk.splits; p.part = sk.part;
-    const int rc = a.out_dtype == DT_F32    ? launch_fp8_exact<DT_F32, true, 0, true>(p, a.batch, st)
-                   : a.out_dtype == DT_BF16 ? launch_fp8_exact<DT_BF16, true, 0, true>(p, a.batch, st)
-                                            : launch_fp8_exact<DT_F16, true, 0, true>(p, a.batch, st);
-    if (rc != 0) return rc;
-    QgemmParams g{};
-    g.a = p.a; g.b = p.b; g.lda = p.lda; g.ldb = p.ldb; g.a_bs = p.a_bs; g.b_bs = p.b_bs;
-    g.out = a.out; g.M = a.M; g.N = a.N; g.ldc = a.N; g.KB = a.K;
-    g.bias = a.bias; g.bias_dt = a.bias_dtype; g.bias_bs = a.bias_batch_stride;
-    g.sa = p.sa; g.sb = p.sb; g.sa_rs = p.sa_rs; g.sb_rs = p.sb_rs; g.sa_bs = p.sa_bs; g.sb_bs = p.sb_bs;
-    g.gate = flags; g.gate_n = g1 + g2;
-    if (a.M <= 128 || a.N <= 128) return qgemm_launch<MODE_MXFP8, 128, 128, 128, 2, 2, 2, 1>(g, a.batch, a.out_dtype, st);
-    return qgemm_launch<MODE_MXFP8, 256, 256, 128, 2, 2, 2, 1>(g, a.batch, a.out_dtype, st);
+    return a.out_dtype == DT_F32    ? launch_fp8_exact<DT_F32, true, 0, true>(p, a.batch, st)
+           : a.out_dtype == DT_BF16 ? launch_fp8_exact<DT_BF16, true, 0, true>(p, a.batch, st)
+                                    : launch_fp8_exact<DT_F16, true, 0, true>(p, a.batch, st);
 }
 
 }  // namespace opsnn

@@ -70,8 +70,8 @@ __global__ __launch_bounds__(256) void mx_pad_rows_kernel(const uint8_t* __restr
     if constexpr (E == 16) {
         *(uint4*)d = c * E < kb ? *(const uint4*)s : make_uint4(fill, fill, fill, fill);
     } else {
-        // the tail repeats the row's last valid scale byte (its elements are zero, so any finite scale will do, and this
-        // one leaves the spread of the row's scales as it was: the exact MXFP8 route looks at that spread)
+        // the tail repeats the row's last valid scale byte (its elements are zero, so any finite scale will do; a row whose
+        // scales are finite gets no other kind)
         (void)fill;
         const uint32_t last = (src + (int64_t)blockIdx.z * bs + r * ld)[kb - 1];
         uint16_t v = (uint16_t)(last | (last << 8));
@@ -146,7 +146,7 @@ static int mx_pad_prestep(OpsnnQmmArgs& a, const MxPad& L, hipStream_t st)
 }
 
 uint64_t mx_exact_bytes(const OpsnnQmmArgs& a);           // qmm_fp8_exact.hip
-int launch_mx_exact(const OpsnnQmmArgs& a, void* region, hipStream_t st, SplitK sk);
+int launch_mx_exact(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk);
 
 // ---- x2 stored [K, N] with N contiguous (data dense, scales [K/64, N, 2]) ----
 // The kernels stream K-contiguous operands: data and scales are first re-laid out, per batch, at 256-byte aligned pitches.
@@ -274,20 +274,15 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
     const bool fp8 = a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E4M3;
     // MXFP8 runs on exact products by default (with two 8-bit operands the scaled matrix instruction aligns its products in
     // a window narrower than fp32: measured on 4096 x 8192 x 8192 with scale exponents in [-4, 4], 1 % of the bf16 outputs
-    // one ulp off and the largest relative error above 2^-7); opsnnSetFp8Fast(1) asks for the 8-bit instruction.  The exact
-    // route's tables sit in front of the workspace.  With a 4-bit x2 the same instruction is as close to the fp32 sums as
+    // one ulp off and the largest relative error above 2^-7); opsnnSetFp8Fast(1) asks for the 8-bit instruction.  With a 4-bit x2 the same instruction is as close to the fp32 sums as
     // exact products are (measured on the same shapes), so that mode keeps it.
     char* rows_region = nullptr;
     if (const uint64_t rb = mx_rows_bytes(a0); rb && a.workspace) {
         rows_region = (char*)a.workspace;
         a.workspace = rows_region + rb;
     }
-    char* mxx = nullptr;
-    if (const uint64_t front = mx_exact_bytes(a0); front && a.workspace) {
-        mxx = (char*)a.workspace;
-        a.workspace = mxx + front;
-    }
-    const bool exact = mxx && !opsnnGetFp8Fast();
+    if (const uint64_t front = mx_exact_bytes(a0); front && a.workspace) a.workspace = (char*)a.workspace + front;
+    const bool exact = !opsnnGetFp8Fast();
 
     // Pre-steps, planned in full before the first of them is launched: an N-contiguous x2 is re-laid out K-contiguous (into
     // the weight cache's buffer for this operand when the cache is on -- a hit skips the passes -- else into the workspace);
@@ -359,8 +354,8 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
     g.sa_bs = a.x1_scale_mat.batch_stride; g.sb_bs = a.x2_scale_mat.batch_stride;
     if (((uintptr_t)g.a | (uintptr_t)g.b | (uint64_t)g.lda | (uint64_t)g.ldb | (uint64_t)g.a_bs | (uint64_t)g.b_bs) % 16) return OPSNN_NOT_TAKEN;
     if (((uintptr_t)g.sa | (uintptr_t)g.sb | (uint64_t)g.sa_rs | (uint64_t)g.sb_rs | (uint64_t)g.sa_bs | (uint64_t)g.sb_bs) % 4) return OPSNN_NOT_TAKEN;
-    if (fp8 && exact) {
-        const int rc = launch_mx_exact(a, mxx, st, sk);
+    if (fp8 && exact && a.force_variant != OPSNN_VARIANT_MX_FP8_MFMA && a.force_variant != OPSNN_VARIANT_MX_128) {
+        const int rc = launch_mx_exact(a, st, sk);
         if (rc != OPSNN_NOT_TAKEN) return rc;
     }
     const bool small = a.M <= 128 || a.N <= 128;

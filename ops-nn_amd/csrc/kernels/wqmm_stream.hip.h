@@ -1429,36 +1429,36 @@ static int launch_resx_one(const WqParams& p, hipStream_t st)
 }
 
 // y[m, n] = rounded(sum over the K segments, in order, of part[s, m, n] + bias[n])
-template <int XDT>
-__global__ __launch_bounds__(256) void wq_splitk_reduce_kernel(const float* part, int splits, int64_t total, int64_t N, const void* bias, int bias_dt,
-                                                               uint16_t* y)
+static __global__ __launch_bounds__(256) void wq_splitk_reduce_kernel(const float* part, int splits, int64_t M, int64_t N, const void* bias, int bias_dt,
+                                                                      void* y, int y_dt)
 {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        float v = splitk_sum(part, splits, total, i);
-        if (bias) v = v + load_scalar_as_f32(bias, bias_dt, i % N);
-        y[i] = bits_x<XDT>(v);
-    }
+    splitk_rows(part, splits, M * N, M, N, [&](int64_t row, int64_t n0, int cols, v4f v) {
+        if (bias) {
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = v[e] + load_scalar_as_f32(bias, bias_dt, n0 + (e < cols ? e : cols - 1));
+        }
+        store_quad(y, y_dt, row * N + n0, cols, v);
+    });
 }
 
 // the fp8 forms of the many-rows kernel: out[m, n] = cast(epilogue(sum over the K segments, in order, of part[s, m, n])); the
 // block-scale form has folded its scales in already, the row / column scale form (RC) computes
 // (sum * x2Scale[n]) * x1Scale[m] + bias[n] here as the kernel's own epilogue does
 template <bool RC>
-__global__ __launch_bounds__(256) void rows_bs_splitk_reduce_kernel(const float* part, int splits, int64_t total, int64_t N, const float* rs, int64_t rs_stride,
-                                                                    const float* cs, int64_t cs_stride, const float* bias, void* out, int out_dt)
+static __global__ __launch_bounds__(256) void rows_bs_splitk_reduce_kernel(const float* part, int splits, int64_t M, int64_t N, const float* rs, int64_t rs_stride,
+                                                                           const float* cs, int64_t cs_stride, const float* bias, void* out, int out_dt)
 {
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        float v = splitk_sum(part, splits, total, i);
+    splitk_rows(part, splits, M * N, M, N, [&](int64_t row, int64_t n0, int cols, v4f v) {
         if constexpr (RC) {
-            const int64_t m = i / N, n = i - m * N;
-            v = (v * cs[n * cs_stride]) * rs[m * rs_stride];
-            if (bias) v = v + bias[n];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const int64_t n = n0 + (e < cols ? e : cols - 1);
+                v[e] = (v[e] * cs[n * cs_stride]) * rs[row * rs_stride];
+                if (bias) v[e] = v[e] + bias[n];
+            }
         }
-        if (out_dt == DT_F32) ((float*)out)[i] = v;
-        else ((uint16_t*)out)[i] = out_dt == DT_BF16 ? bf16_bits(v) : f16_bits(v);
-    }
+        store_quad(out, out_dt, row * N + n0, cols, v);
+    });
 }
 
 // One workgroup per CU (its waves fill the register file), or one per row block when there are fewer; with K split into
@@ -1492,9 +1492,8 @@ static int launch_xreg_one(const WqParams& p, hipStream_t st, int splits = 1)
     hipLaunchKernelGGL(k, dim3((unsigned)(nblocks < g ? nblocks : g), (unsigned)splits), dim3(NW * 64), lds, st, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || splits == 1) return (int)e;
-    const int64_t total = p.M * p.N;
-    hipLaunchKernelGGL(wq_splitk_reduce_kernel<XDT>, dim3(splitk_reduce_grid(total)), dim3(256), 0, st, (const float*)p.part, splits, total, p.N, p.bias,
-                       p.bias_dt, p.y);
+    hipLaunchKernelGGL(wq_splitk_reduce_kernel, splitk_rows_grid(p.M, p.N), dim3(256), 0, st, (const float*)p.part, splits, p.M, p.N, p.bias, p.bias_dt,
+                       (void*)p.y, XDT);
     return (int)hipGetLastError();
 }
 
@@ -1636,19 +1635,18 @@ static int launch_rows_one(const WqParams& p, hipStream_t st)
     hipLaunchKernelGGL(k, dim3(grid, (unsigned)slabs, split ? (unsigned)p.ksplit : 1u), dim3(512), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
     if (split) {
-        const int64_t total = p.M * p.N;
+        const dim3 rgrid = splitk_rows_grid(p.M, p.N);
         if constexpr (WF == 3) {
-            hipLaunchKernelGGL(rows_bs_splitk_reduce_kernel<false>, dim3(splitk_reduce_grid(total)), dim3(256), 0, st, (const float*)p.part, p.ksplit, total,
+            hipLaunchKernelGGL(rows_bs_splitk_reduce_kernel<false>, rgrid, dim3(256), 0, st, (const float*)p.part, p.ksplit, p.M,
                                p.N, (const float*)nullptr, (int64_t)0, (const float*)nullptr, (int64_t)0, (const float*)nullptr, (void*)p.y, p.bs_out_dt);
             return (int)hipGetLastError();
         }
         if constexpr (WF == 4) {
-            hipLaunchKernelGGL(rows_bs_splitk_reduce_kernel<true>, dim3(splitk_reduce_grid(total)), dim3(256), 0, st, (const float*)p.part, p.ksplit, total,
+            hipLaunchKernelGGL(rows_bs_splitk_reduce_kernel<true>, rgrid, dim3(256), 0, st, (const float*)p.part, p.ksplit, p.M,
                                p.N, p.bs1, p.bs1_rs, p.bs2, p.bs2_cs, (const float*)p.bias, (void*)p.y, p.bs_out_dt);
             return (int)hipGetLastError();
         }
-        hipLaunchKernelGGL(wq_splitk_reduce_kernel<XDT>, dim3(splitk_reduce_grid(total)), dim3(256), 0, st, (const float*)p.part, p.ksplit, total, p.N,
-                           p.bias, p.bias_dt, p.y);
+        hipLaunchKernelGGL(wq_splitk_reduce_kernel, rgrid, dim3(256), 0, st, (const float*)p.part, p.ksplit, p.M, p.N, p.bias, p.bias_dt, (void*)p.y, XDT);
         return (int)hipGetLastError();
     }
     return 0;
