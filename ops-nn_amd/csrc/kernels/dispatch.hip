@@ -32,6 +32,9 @@ int launch_wqmm_mfma(const OpsnnWqmmArgs& a, hipStream_t st);
 bool wq_dense_wanted(const OpsnnWqmmArgs& a);   // wq_dense.hip
 uint64_t wq_dense_workspace(const OpsnnWqmmArgs& a);
 int launch_wq_dense(const OpsnnWqmmArgs& a, hipStream_t st);
+bool wq_kn_wanted(const OpsnnWqmmArgs& a);   // wq_kn.hip
+uint64_t wq_kn_workspace(const OpsnnWqmmArgs& a);
+int launch_wq_kn(const OpsnnWqmmArgs& a, hipStream_t st);
 uint64_t mx_workspace_bytes(const OpsnnQmmArgs& a);
 }  // namespace opsnn
 
@@ -447,6 +450,8 @@ extern "C" int opsnnWqmm(const OpsnnWqmmArgs* a, void* stream)
     if (a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain()) {
         int rc = launch_wq_dense(*a, (hipStream_t)stream);
         if (rc != OPSNN_NOT_TAKEN) return rc;
+        rc = launch_wq_kn(*a, (hipStream_t)stream);
+        if (rc != OPSNN_NOT_TAKEN) return rc;
         rc = launch_wqmm_mfma(*a, (hipStream_t)stream);
         if (rc != OPSNN_NOT_TAKEN) return rc;
         if (a->force_variant != 0) return -4;
@@ -504,5 +509,8 @@ extern "C" uint64_t opsnnWqmmWorkspace(const OpsnnWqmmArgs* a)
         part = ((uint64_t)xs * (uint64_t)a->M * (uint64_t)a->N * 4 + 255) / 256 * 256;
     if (a->w.row_stride == 1 || a->K == 1) return part;
     if (a->w.col_stride != 1 || a->w.row_stride != a->N) return part;
-    return part + (uint64_t)a->N * (uint64_t)a->K * bits / 8;
+    const uint64_t relaid = part + (uint64_t)a->N * (uint64_t)a->K * bits / 8;
+    // few rows: the kernel that streams the weight as it lies, or (weight cache on, but without room) the re-layout
+    if (wq_kn_wanted(*a) && !opsnn_force_plain()) { const uint64_t kn = wq_kn_workspace(*a); return kn > relaid ? kn : relaid; }
+    return relaid;
 }

@@ -118,6 +118,9 @@ WeightCacheScope::~WeightCacheScope()
     if (--t_scope.depth == 0) unpin_all();
 }
 
+// Whether the cache may serve this thread's calls at the moment.
+bool weight_cache_on() { return __atomic_load_n(&g_limit, __ATOMIC_RELAXED) != 0 && !t_scope.bypass; }
+
 // A buffer of `bytes` that belongs to the operand (src, src2, src3 -- e.g. data, scales and offsets --, shape, element width,
 // batch count):
 // on a hit (*fresh = false) it holds what an earlier call put there and is ordered behind that call's writes on `st`; on a

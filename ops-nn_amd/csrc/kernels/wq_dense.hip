@@ -8,6 +8,7 @@
 // run (N no multiple of 32, K no whole number of x slabs, groups of 64, [K, N] storage): it takes every layout, group and N.
 #include "gemm16.h"
 #include "launch.h"
+#include "wq_kn.hip.h"
 #include "wqmm_stream.hip.h"
 
 extern "C" int opsnn_wq_tile_min();   // dispatch.hip
@@ -38,9 +39,8 @@ __global__ __launch_bounds__(256) void wq_dequant_nk_kernel(WqParams p, uint16_t
     }
 }
 
-// [K, N] storage: a lane takes 8 rows of k and 8 neighbouring columns, dequantises along the columns (that is how the codes
-// and the scales lie) and writes, per column, 16 bytes of 8 consecutive k; 16 lanes side by side in k make 256 contiguous
-// bytes of an output row.  The 8 x 8 transposition is byte permutes in registers (bf16: the packing conversion itself).
+// [K, N] storage: a lane takes 8 rows of k and 8 neighbouring columns (dequant_8x8) and writes, per column, 16 bytes of 8
+// consecutive k; 16 lanes side by side in k make 256 contiguous bytes of an output row.
 template <int XDT, int WBITS, bool HAS_OFF>
 __global__ __launch_bounds__(256) void wq_dequant_kn_kernel(WqParams p, uint16_t* __restrict__ out)
 {
@@ -71,71 +71,13 @@ __global__ __launch_bounds__(256) void wq_dequant_kn_kernel(WqParams p, uint16_t
         sb[j] = p.scale[(int64_t)g * p.s_rs + n * p.s_cs];
         ob[j] = HAS_OFF ? p.offset[(int64_t)g * p.s_rs + n * p.s_cs] : (uint16_t)0;
     }
-    uint32_t o[8][4];   // o[column][pair of k]
-    if constexpr (XDT == DT_F16) {
-        // per row of k: four pairs of columns -- int4: (0,4) (1,5) (2,6) (3,7), the order of the nibble splice; int8: (0,1) ...
-        h2 sc[4], of[4];
+    uint32_t o[8][4], scw[4], ofw[4];   // o[column][pair of k]
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            const int a = WBITS == 4 ? t : 2 * t, b = WBITS == 4 ? t + 4 : 2 * t + 1;
-            sc[t] = (h2){__builtin_bit_cast(_Float16, sb[a]), __builtin_bit_cast(_Float16, sb[b])};
-            of[t] = (h2){__builtin_bit_cast(_Float16, ob[a]), __builtin_bit_cast(_Float16, ob[b])};
-        }
-        const h2 c1032 = {(_Float16)-1032.0f, (_Float16)-1032.0f}, c72 = {(_Float16)-72.0f, (_Float16)-72.0f}, r16 = {(_Float16)0.0625f, (_Float16)0.0625f};
-        const h2 c1152 = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-#pragma unroll
-        for (int i = 0; i < 8; i += 2) {
-            uint32_t row[2][4];
-#pragma unroll
-            for (int r = 0; r < 2; r++) {
-                h2 t[4];
-                if constexpr (WBITS == 4) {
-                    const uint32_t u = q[i + r][0], u8 = u >> 8;
-                    t[0] = __builtin_bit_cast(h2, (u & 0x000F000Fu) ^ 0x64086408u) + c1032;
-                    t[1] = __builtin_elementwise_fma(__builtin_bit_cast(h2, (u & 0x00F000F0u) ^ 0x64806480u), r16, c72);
-                    t[2] = __builtin_bit_cast(h2, (u8 & 0x000F000Fu) ^ 0x64086408u) + c1032;
-                    t[3] = __builtin_elementwise_fma(__builtin_bit_cast(h2, (u8 & 0x00F000F0u) ^ 0x64806480u), r16, c72);
-                } else {
-                    const uint32_t qa = q[i + r][0] ^ 0x80808080u, qb = q[i + r][DW - 1] ^ 0x80808080u, magic = 0x64646464u;
-                    t[0] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(magic, qa, 0x04010400u)) + c1152;
-                    t[1] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(magic, qa, 0x04030402u)) + c1152;
-                    t[2] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(magic, qb, 0x04010400u)) + c1152;
-                    t[3] = __builtin_bit_cast(h2, __builtin_amdgcn_perm(magic, qb, 0x04030402u)) + c1152;
-                }
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    if constexpr (HAS_OFF) t[c] = t[c] + of[c];
-                    row[r][c] = u32(t[c] * sc[c]);
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const int a = WBITS == 4 ? c : 2 * c, b = WBITS == 4 ? c + 4 : 2 * c + 1;
-                o[a][i / 2] = __builtin_amdgcn_perm(row[1][c], row[0][c], 0x05040100u);
-                o[b][i / 2] = __builtin_amdgcn_perm(row[1][c], row[0][c], 0x07060302u);
-            }
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const float scf = bf16_to_f32(sb[j]), off = bf16_to_f32(ob[j]);
-#pragma unroll
-            for (int i = 0; i < 8; i += 2) {
-                float w[2];
-#pragma unroll
-                for (int r = 0; r < 2; r++) {
-                    if constexpr (WBITS == 4) w[r] = (float)((int)(q[i + r][0] << (28 - 4 * j)) >> 28);
-                    else w[r] = (float)((int)(q[i + r][j / 4 * (DW - 1)] << (24 - 8 * (j & 3))) >> 24);
-                }
-                if constexpr (HAS_OFF) {
-                    const uint32_t pk = pack2_bf16((v2f){w[0] + off, w[1] + off});
-                    w[0] = u2f(pk << 16);
-                    w[1] = u2f(pk & 0xffff0000u);
-                }
-                o[j][i / 2] = pack2_bf16((v2f){w[0] * scf, w[1] * scf});
-            }
-        }
+    for (int t = 0; t < 4; t++) {
+        scw[t] = sb[2 * t] | ((uint32_t)sb[2 * t + 1] << 16);
+        ofw[t] = ob[2 * t] | ((uint32_t)ob[2 * t + 1] << 16);
     }
+    dequant_8x8<XDT, WBITS, HAS_OFF>(q, scw, ofw, o);
 #pragma unroll
     for (int j = 0; j < 8; j++)
         if (j < cols) *(v4i*)(out + (n0 + j) * p.K + k0) = (v4i){(int)o[j][0], (int)o[j][1], (int)o[j][2], (int)o[j][3]};

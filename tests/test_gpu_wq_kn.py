@@ -1,0 +1,30 @@
+"""Weight-only calls with up to 64 rows against a weight in [K, N] storage, streamed as it lies (wq_kn.hip): the edges of its
+row blocks (16, 32, 64), a ragged last strip of columns at every alignment, K of a few steps, K in segments, short last
+groups, groups of 32 to K, one scale for the whole weight."""
+import pytest
+
+import cases
+import oracle_api as orc
+from test_gpu_shape_sweep import _b16_bar
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,K,N,group", [
+    (1, 256, 256, 0), (16, 288, 258, 128), (17, 1024, 520, 64), (32, 4096, 1002, 128), (33, 2080, 384, 32), (64, 8192, 300, 128),
+    (7, 4160, 2048, 128), (3, 18432, 1026, 0), (48, 3008, 4098, 64), (15, 11008, 770, 352),
+])
+@pytest.mark.parametrize("w_dt,x_dt,off", [("i4", "f16", True), ("i4", "bf16", False), ("i8", "f16", False), ("i8", "bf16", True)])
+def test_kn_stream(gpu, M, K, N, group, w_dt, x_dt, off):
+    m = gpu
+    xd = m.ACL_FLOAT16 if x_dt == "f16" else m.ACL_BF16
+    n = N + (1 if w_dt == "i8" and N % 16 == 2 else 0)   # (odd N with 8-bit weights)
+    inp = cases.make_wq_inputs(m, M, K, n, M + K, xd, m.ACL_INT4 if w_dt == "i4" else m.ACL_INT8, group, False, off, xd if M % 2 else None)
+    print(f"case kn M={M} K={K} N={n} g={group} {w_dt} {x_dt}", flush=True)
+    _b16_bar(cases.run_wq_aclnn(m, inp, M, K, n), cases.oracle_wq(m, inp, M, K, n), orc.F16 if x_dt == "f16" else orc.BF16, "kn stream", K)
+
+
+def test_kn_one_scale(gpu):
+    m = gpu
+    inp = cases.make_wq_inputs(m, 9, 512, 272, 3, m.ACL_FLOAT16, m.ACL_INT8, 0, False, True, None, per_tensor=True)
+    _b16_bar(cases.run_wq_aclnn(m, inp, 9, 512, 272), cases.oracle_wq(m, inp, 9, 512, 272), orc.F16, "kn one scale", 512)
