@@ -35,6 +35,9 @@ int launch_wq_dense(const OpsnnWqmmArgs& a, hipStream_t st);
 bool wq_kn_wanted(const OpsnnWqmmArgs& a);   // wq_kn.hip
 uint64_t wq_kn_workspace(const OpsnnWqmmArgs& a);
 int launch_wq_kn(const OpsnnWqmmArgs& a, hipStream_t st);
+bool wq_nk_wanted(const OpsnnWqmmArgs& a);   // wq_nk.hip
+uint64_t wq_nk_workspace(const OpsnnWqmmArgs& a);
+int launch_wq_nk(const OpsnnWqmmArgs& a, hipStream_t st);
 uint64_t mx_workspace_bytes(const OpsnnQmmArgs& a);
 }  // namespace opsnn
 
@@ -452,6 +455,8 @@ extern "C" int opsnnWqmm(const OpsnnWqmmArgs* a, void* stream)
         if (rc != OPSNN_NOT_TAKEN) return rc;
         rc = launch_wq_kn(*a, (hipStream_t)stream);
         if (rc != OPSNN_NOT_TAKEN) return rc;
+        rc = launch_wq_nk(*a, (hipStream_t)stream);
+        if (rc != OPSNN_NOT_TAKEN) return rc;
         rc = launch_wqmm_mfma(*a, (hipStream_t)stream);
         if (rc != OPSNN_NOT_TAKEN) return rc;
         if (a->force_variant != 0) return -4;
@@ -507,6 +512,7 @@ extern "C" uint64_t opsnnWqmmWorkspace(const OpsnnWqmmArgs* a)
     uint64_t part = 0;
     if (const int xs = wq_part_slices((int)bits, a->M, a->N, a->K, a->group > 0 ? a->group : a->K, opsnn_wq_narrow_slabs() != 0); xs > 1 && a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain())
         part = ((uint64_t)xs * (uint64_t)a->M * (uint64_t)a->N * 4 + 255) / 256 * 256;
+    if (wq_nk_wanted(*a) && !opsnn_force_plain()) return wq_nk_workspace(*a);   // few rows, a shape outside the specialised kernels
     if (a->w.row_stride == 1 || a->K == 1) return part;
     if (a->w.col_stride != 1 || a->w.row_stride != a->N) return part;
     const uint64_t relaid = part + (uint64_t)a->N * (uint64_t)a->K * bits / 8;

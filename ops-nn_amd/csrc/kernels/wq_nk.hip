@@ -1,0 +1,284 @@
+// Weight-only matmul with few rows of x (up to 64) against a weight in [N, K] storage whose shape the specialised streaming
+// kernels of wqmm_stream.hip.h do not take: any N, K a multiple of 32 (8-bit weights: 16 would do), any group that is a multiple
+// of 32.  (Such calls -- N no multiple of 32, groups of 64, K % 128 = 64 -- ran on the general kernel: 17 x 5632 x 1453 49 us,
+// 3 x 16448 x 2560 131 us.)
+//
+// A wave owns NB blocks of 16 columns; lane (r = lane % 16, q = lane / 16) streams PB-byte pieces of the rows 16 j + r straight
+// into registers (32 int4 or 16 int8 with 16 bytes; 16 int4 with 8), two chunks ahead, and the pieces of x that go with them
+// straight from memory: with eight (four) column blocks per x fragment the fragments cost no more requests than the weights, so
+// there is no LDS and no barrier in the loop.  Scales and offsets lie in a table in LDS, one word per column and group, laid
+// down once per workgroup (fetched per chunk they are 2-byte gathers of 16 cache lines each, as many requests as the weights).
+// x is put into the order in which the nibble splice delivers the weights (one permute per register of x, shared by the
+// column blocks).
+//
+// Work split as in wq_kn.hip: the four waves of a workgroup take a quarter each of its chunks, blockIdx.y cuts K into
+// segments; sums meet in LDS in a fixed order, segments in `part`, added in order by wq_splitk_reduce_kernel.  A wave past the
+// edge of N repeats the last columns (stored twice, same bits).
+#include "launch.h"
+#include "wqmm_stream.hip.h"
+
+namespace opsnn {
+
+struct WqNkPlan {
+    int mb = 1, splits = 1;
+    int groups = 1;   // groups a workgroup's segment can touch: columns of its scale table
+};
+// column blocks of 16 per workgroup (with four row blocks of x: sums, x fragments and eight column blocks would not fit the registers)
+constexpr int nk_nb(int mb) { return mb == 4 ? 4 : 8; }
+static bool nk_plan(int wbits, int64_t M, int64_t N, int64_t K, int64_t group, WqNkPlan& pl)
+{
+    pl.mb = M <= 16 ? 1 : M <= 32 ? 2 : 4;
+    const int64_t cols = 16 * nk_nb(pl.mb), strips = (N + cols - 1) / cols, kc = (pl.mb == 4 || wbits == 8) ? 64 : 128, chunks = (K + kc - 1) / kc;
+    // (a chunk: 8 KB of codes per wave; four row blocks: 2 KB of 4-bit, 4 KB of 8-bit codes; eight waves of a CU at 5 TB/s)
+    const double t_chunk = pl.mb == 4 ? (wbits == 4 ? 1.4 : 2.0) : pl.mb == 2 ? 4.1 : 3.4;
+    double best = 1e30;
+    bool found = false;
+    for (int s = 1; s <= 16 && chunks / s >= 2; s++) {
+        const int64_t seg = (chunks + s - 1) / s * kc, g = group >= K ? 1 : (seg + group - 1) / group + 1;
+        if (g * cols * 4 > 32768) continue;
+        const double us = (double)((strips * s + 511) / 512) * ((double)((chunks + 4 * s - 1) / (4 * s)) * t_chunk + 4.0) +
+                          (s > 1 ? 3.0 + 8.0 * s * (double)M * (double)N / 4.0e6 : 0.0);
+        if (us < best) { best = us; pl.splits = s; pl.groups = (int)g; found = true; }
+    }
+    return found;
+}
+
+template <int XDT, int WBITS, int MB, bool HAS_OFF>
+__global__ __launch_bounds__(256, 2) void wq_nk_kernel(WqParams p, int splits, int gmax)
+{
+    constexpr int NB = nk_nb(MB), PF = 2;
+    constexpr int PB = (MB == 4 && WBITS == 4) ? 8 : 16;   // bytes of a lane's weight piece
+    constexpr int KPL = PB * 8 / WBITS, KC = 4 * KPL, STEPS = KPL / 8;
+    constexpr int DW = PB / 4;
+    extern __shared__ __attribute__((aligned(16))) float dyn[];   // the scale table; at the end two waves' sums
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    int64_t n0 = (int64_t)blockIdx.x * (16 * NB);
+    if (n0 + 16 * NB > p.N) n0 = p.N - 16 * NB;
+    const int Ki = (int)p.K, chunks = (Ki + KC - 1) / KC;
+    const int s0 = (int)((int64_t)blockIdx.y * chunks / splits), s1 = (int)((int64_t)(blockIdx.y + 1) * chunks / splits);
+    const int w0 = s0 + (s1 - s0) * wave / 4, w1 = s0 + (s1 - s0) * (wave + 1) / 4;   // this wave's chunks
+
+    // scale table: word (column, group - g_lo) = scale | offset << 16
+    const int groupi = (int)p.group;
+    auto group_at = [&](int k) { return p.group_shift >= 0 ? k >> p.group_shift : k / groupi; };
+    const int g_lo = group_at(s0 * KC), g_all = group_at(Ki - 1);
+    uint32_t* const tab = (uint32_t*)dyn;
+    for (int i = tid; i < 16 * NB * gmax; i += 256) {
+        const int col = i / gmax, gi = g_lo + i - col * gmax;
+        const int64_t at = (int64_t)(gi < g_all ? gi : g_all) * p.s_rs + (n0 + col) * p.s_cs;
+        uint32_t w = p.scale[at];
+        if constexpr (HAS_OFF) w |= (uint32_t)p.offset[at] << 16;
+        tab[col * gmax + i - col * gmax] = w;
+    }
+    __syncthreads();
+
+    const uint8_t* wbase = p.w + (n0 + r) * p.ldw;
+    const int64_t wblk = 16 * p.ldw;
+    const uint16_t* xrow[MB];
+#pragma unroll
+    for (int b = 0; b < MB; b++) {
+        const int64_t m = 16 * b + r;
+        xrow[b] = p.x + (m < p.M ? m : p.M - 1) * p.K;
+    }
+    uint32_t raw[PF][NB][DW];
+    v4i xf[PF][STEPS][MB];
+    auto fetch = [&](auto jc, int c) {
+        constexpr int j = decltype(jc)::value;
+        const int k0 = c * KC + q * KPL, k = k0 < Ki ? k0 : Ki - KPL;   // (past the end of K: the last piece, multiplied by zeros of x)
+        const uint8_t* w = wbase + (int64_t)k * WBITS / 8;
+#pragma unroll
+        for (int b = 0; b < NB; b++) __builtin_memcpy(raw[j][b], w + b * wblk, PB);
+#pragma unroll
+        for (int s = 0; s < STEPS; s++)
+#pragma unroll
+            for (int b = 0; b < MB; b++) xf[j][s][b] = *(const v4i*)(xrow[b] + k + 8 * s);
+    };
+    v4f acc[NB][MB];
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+#pragma unroll
+        for (int b = 0; b < MB; b++) acc[j][b] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
+    const DqConst dqc = make_dq_const();
+    auto chunk = [&](auto jc, int c) {
+        constexpr int j = decltype(jc)::value;
+        const int k = c * KC + q * KPL;
+        const int gi = group_at(k < Ki ? k : Ki - KPL) - g_lo;
+        if (c == chunks - 1 && k >= Ki) {
+#pragma unroll
+            for (int s = 0; s < STEPS; s++)
+#pragma unroll
+                for (int b = 0; b < MB; b++) xf[j][s][b] = (v4i){0, 0, 0, 0};
+        }
+        uint32_t sow[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) sow[b] = tab[(16 * b + r) * gmax + gi];
+#pragma unroll
+        for (int s = 0; s < STEPS; s++) {
+            v4i xo[MB];
+#pragma unroll
+            for (int b = 0; b < MB; b++) {
+                xo[b] = xf[j][s][b];
+                if constexpr (WBITS == 4) {   // halves [0..7] -> [0,4,1,5,2,6,3,7]
+                    const uint32_t a0 = (uint32_t)xo[b][0], a1 = (uint32_t)xo[b][1], a2 = (uint32_t)xo[b][2], a3 = (uint32_t)xo[b][3];
+                    xo[b] = (v4i){(int)__builtin_amdgcn_perm(a2, a0, 0x05040100u), (int)__builtin_amdgcn_perm(a2, a0, 0x07060302u),
+                                  (int)__builtin_amdgcn_perm(a3, a1, 0x05040100u), (int)__builtin_amdgcn_perm(a3, a1, 0x07060302u)};
+                }
+            }
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++) {
+                v4i piece = {0, 0, 0, 0};
+                if constexpr (WBITS == 4) piece[0] = (int)raw[j][nb][s];
+                else { piece[0] = (int)raw[j][nb][2 * s]; piece[1] = (int)raw[j][nb][2 * s + 1]; }
+                const v4i a = dequant8<XDT, WBITS, HAS_OFF>(piece, 0, (uint16_t)sow[nb], (uint16_t)(sow[nb] >> 16), dqc);
+#pragma unroll
+                for (int b = 0; b < MB; b++) {
+                    if constexpr (XDT == DT_F16) acc[nb][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, xo[b]), acc[nb][b], 0, 0, 0);
+                    else acc[nb][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, xo[b]), acc[nb][b], 0, 0, 0);
+                }
+            }
+        }
+        if (c + PF < w1) fetch(jc, c + PF);
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    if (w0 < w1) fetch(I0{}, w0);
+    if (w0 + 1 < w1) fetch(I1{}, w0 + 1);
+    for (int c = w0; c < w1; c += PF) {
+        chunk(I0{}, c);
+        if (c + 1 < w1) chunk(I1{}, c + 1);
+    }
+
+    // the four waves' sums in a fixed order: (0 + 2) + (1 + 3)
+    float* const red = dyn;
+    constexpr int SUMS = NB * MB * 4 * 64;
+    auto park = [&](float* to) {
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+#pragma unroll
+            for (int b = 0; b < MB; b++) *(v4f*)(to + ((j * MB + b) * 64 + lane) * 4) = acc[j][b];
+    };
+    auto add = [&](const float* from) {
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+#pragma unroll
+            for (int b = 0; b < MB; b++) acc[j][b] = acc[j][b] + *(const v4f*)(from + ((j * MB + b) * 64 + lane) * 4);
+    };
+    __syncthreads();   // the scale table makes room
+    if (wave >= 2) park(red + (wave - 2) * SUMS);
+    __syncthreads();
+    if (wave < 2) add(red + wave * SUMS);
+    __syncthreads();
+    if (wave == 1) park(red);
+    __syncthreads();
+    if (wave != 0) return;
+    add(red);
+
+    // acc[j][b][i] is out[m = 16 b + lane % 16][n = n0 + 16 j + 4 q + i]
+#pragma unroll
+    for (int b = 0; b < MB; b++) {
+        const int64_t m = 16 * b + r;
+        if (m >= p.M) continue;
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const int64_t n = n0 + 16 * j + 4 * q;
+            if (splits > 1) {
+                __builtin_memcpy(p.part + ((int64_t)blockIdx.y * p.M + m) * p.N + n, &acc[j][b], 16);
+                continue;
+            }
+            uint16_t o[4];
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                float v = acc[j][b][e];
+                if (p.bias) v = v + load_scalar_as_f32(p.bias, p.bias_dt, n + e);
+                o[e] = bits_x<XDT>(v);
+            }
+            __builtin_memcpy(p.y + m * p.N + n, o, 8);
+        }
+    }
+}
+
+template <int XDT, int WBITS, int MB, bool HAS_OFF>
+static int launch_nk_one(const WqParams& p, const WqNkPlan& pl, hipStream_t st)
+{
+    constexpr int NB = nk_nb(MB), COLS = 16 * NB;
+    const dim3 grid((unsigned)((p.N + COLS - 1) / COLS), (unsigned)pl.splits);
+    constexpr size_t lds_sum = (size_t)2 * NB * MB * 4 * 64 * 4;
+    const size_t lds_tab = (size_t)pl.groups * COLS * 4;
+    auto k = wq_nk_kernel<XDT, WBITS, MB, HAS_OFF>;
+    static std::atomic<uint64_t> attr_set{0};   // one bit per device: the attribute belongs to the (kernel, device) pair
+    if (!device_flag_test(attr_set)) {
+        hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(lds_sum > 32768 ? lds_sum : 32768));
+        if (e != hipSuccess) return (int)e;
+        device_flag_set(attr_set);
+    }
+    hipLaunchKernelGGL(k, grid, dim3(256), lds_sum > lds_tab ? lds_sum : lds_tab, st, p, pl.splits, pl.groups);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess || pl.splits == 1) return (int)e;
+    hipLaunchKernelGGL(wq_splitk_reduce_kernel, splitk_rows_grid(p.M, p.N), dim3(256), 0, st, (const float*)p.part, pl.splits, p.M, p.N, p.bias, p.bias_dt,
+                       (void*)p.y, XDT);
+    return (int)hipGetLastError();
+}
+template <int XDT, int WBITS, bool HAS_OFF>
+static int launch_nk_mb(const WqParams& p, const WqNkPlan& pl, hipStream_t st)
+{
+    if (pl.mb == 1) return launch_nk_one<XDT, WBITS, 1, HAS_OFF>(p, pl, st);
+    if (pl.mb == 2) return launch_nk_one<XDT, WBITS, 2, HAS_OFF>(p, pl, st);
+    return launch_nk_one<XDT, WBITS, 4, HAS_OFF>(p, pl, st);
+}
+
+// Does the call run here?  Looks at what phase 1 knows, so that both phases agree.  The specialised kernels keep what they take
+// (wqmm.hip): K in whole 128-element units, groups of whole chunks, and from 17 rows N % 32 == 0 and K in whole x slabs.
+bool wq_nk_wanted(const OpsnnWqmmArgs& a)
+{
+    if ((a.w_dtype != DT_I4 && a.w_dtype != DT_I8) || (a.x_dtype != DT_F16 && a.x_dtype != DT_BF16)) return false;
+    if (a.scale_dtype != a.x_dtype) return false;
+    if (a.M > 64 || a.K % 32 != 0 || a.K < 256 || a.N < 256 || a.K >= (1ll << 30) || a.N >= (1ll << 30)) return false;
+    if (a.w.row_stride != 1 || a.w.col_stride != a.K) return false;
+    const int64_t group = a.group > 0 && a.group < a.K ? a.group : a.K;
+    if (group < a.K && group % 32 != 0) return false;
+    if ((uintptr_t)a.x % 16 != 0 || (uintptr_t)a.w.ptr % 16 != 0) return false;
+    WqNkPlan pl;
+    if (!nk_plan(a.w_dtype == DT_I4 ? 4 : 8, a.M, a.N, a.K, group, pl)) return false;
+    if (a.force_variant != 0) return false;
+    const int wbits = a.w_dtype == DT_I4 ? 4 : 8;
+    const int64_t kc = 4 * (128 / wbits), cpg = group / kc;
+    const bool whole_groups = group >= a.K || (group % kc == 0 && (cpg & (cpg - 1)) == 0);
+    if (!whole_groups || a.K % kc != 0) return true;
+    if (a.M <= 16) return a.K % 128 != 0;
+    // (17 .. 32 rows against a narrow N and a K that the many-rows kernel does not cut: there the streaming kernel's workgroups are
+    // few -- 32 x 4096 x 4096 fp16 / bf16 17.1 / 21.1 us against 13.3 / 13.5 here; at N = 11008 it is 20 against 24)
+    if (a.M <= 32 && a.N <= 8192 && a.K < 8192) return true;
+    return a.N % 32 != 0 || a.K % (2 * kc) != 0;
+}
+uint64_t wq_nk_workspace(const OpsnnWqmmArgs& a)
+{
+    WqNkPlan pl;
+    if (!nk_plan(a.w_dtype == DT_I4 ? 4 : 8, a.M, a.N, a.K, a.group > 0 && a.group < a.K ? a.group : a.K, pl)) return 0;
+    return pl.splits > 1 ? ((uint64_t)pl.splits * (uint64_t)a.M * (uint64_t)a.N * 4 + 255) / 256 * 256 : 0;
+}
+int launch_wq_nk(const OpsnnWqmmArgs& a, hipStream_t st)
+{
+    if (!wq_nk_wanted(a)) return OPSNN_NOT_TAKEN;
+    const int wbits = a.w_dtype == DT_I4 ? 4 : 8;
+    WqParams p{};
+    p.group = a.group > 0 && a.group < a.K ? a.group : a.K;
+    WqNkPlan pl;
+    if (!nk_plan(wbits, a.M, a.N, a.K, p.group, pl) || (pl.splits > 1 && !a.workspace)) return OPSNN_NOT_TAKEN;
+    p.x = (const uint16_t*)a.x;
+    p.w = (const uint8_t*)a.w.ptr; p.ldw = a.w.col_stride * wbits / 8;
+    p.scale = (const uint16_t*)a.scale.ptr; p.offset = (const uint16_t*)a.offset;
+    p.s_rs = a.scale.row_stride; p.s_cs = a.scale_n == 1 ? 0 : a.scale.col_stride;
+    p.bias = a.bias; p.bias_dt = a.bias_dtype;
+    p.y = (uint16_t*)a.y; p.M = a.M; p.N = a.N; p.K = a.K;
+    p.group_shift = p.group >= p.K ? 31 : (p.group & (p.group - 1)) == 0 ? __builtin_ctzll((unsigned long long)p.group) : -1;
+    p.part = (float*)a.workspace;
+    if (a.x_dtype == DT_F16) {
+        if (wbits == 4) return a.offset ? launch_nk_mb<DT_F16, 4, true>(p, pl, st) : launch_nk_mb<DT_F16, 4, false>(p, pl, st);
+        return a.offset ? launch_nk_mb<DT_F16, 8, true>(p, pl, st) : launch_nk_mb<DT_F16, 8, false>(p, pl, st);
+    }
+    if (wbits == 4) return a.offset ? launch_nk_mb<DT_BF16, 4, true>(p, pl, st) : launch_nk_mb<DT_BF16, 4, false>(p, pl, st);
+    return a.offset ? launch_nk_mb<DT_BF16, 8, true>(p, pl, st) : launch_nk_mb<DT_BF16, 8, false>(p, pl, st);
+}
+
+}  // namespace opsnn
