@@ -249,17 +249,12 @@ static int splitk_for(const OpsnnQmmArgs& a, int mode)
     int64_t bm, bn = 256, kunit = 128;
     double tile_us;   // one K tile (kunit elements) of the kernel in question, measured on calls with few tiles
     double bytes_per_us = 5.0e6;   // what its partial sums' traffic was measured to cost (splitk_factor)
-    // int8 with per-token / per-channel scales on 128 x 128 tiles (the selector's choice up to 256 x 256 x 64 outputs; whole K
-    // tiles): integer partial sums, so the result stays bit-identical
-    if ((mode == 0 || (mode == 3 && !a.x1_scale)) && a.x1_dtype == DT_I8 && a.x2_dtype == DT_I8 && out16 && a.K % 128 == 0 &&
-        (a.M <= 128 || a.N <= 128 || a.M * a.N <= 256 * 256 * 64)) {
-        // (a 128 x 128 int8 tile is quick, and the partial sums cost their own traffic: measured at 4096 x 4096 in eight
-        // splits, 64 rows 20 -> 15 us, 128 rows 19.5 -> 22, 256 rows in four 21 -> 24)
-        bm = 128; bn = 128; tile_us = 0.55; bytes_per_us = 2.4e6;
-    }
-    else if (tiny) return 1;
+    // int8 with per-token / per-channel scales (whole K tiles): integer partial sums, so the result stays bit-identical
+    if ((mode == 0 || (mode == 3 && !a.x1_scale)) && a.x1_dtype == DT_I8 && a.x2_dtype == DT_I8 && out16 && a.K % 128 == 0)
+        return int8_tile_plan(a.M, a.N, a.K, a.batch, true).splits;
+    if (tiny) return 1;
     // MXFP4: 128 x 128 tiles when 256 x 256 ones would be few (the launcher's rule), K tiles counted in 256 elements
-    else if (mode == 2 && a.x1_dtype == DT_E2M1 && a.x2_dtype == DT_E2M1 && (out16 || a.out_dtype == DT_F32)) {
+    if (mode == 2 && a.x1_dtype == DT_E2M1 && a.x2_dtype == DT_E2M1 && (out16 || a.out_dtype == DT_F32)) {
         const int64_t t256 = ((a.M + 255) / 256) * ((a.N + 255) / 256) * a.batch;
         bm = bn = (a.M <= 128 || a.N <= 128 || t256 <= 64) ? 128 : 256;
         kunit = 256;

@@ -80,6 +80,56 @@ namespace opsnn {
 int launch_int8_wide(const QgemmParams& p, int fn, int64_t batch, int out_dt, hipStream_t st);   // qmm_int8_wide.hip
 }
 
+namespace opsnn {
+// The tiles for shapes that do not fill the chip with 256 x 256 ones.  What bounds them is the time from a copy's issue to its
+// arrival (about 1 us with HBM busy): a workgroup with two stages has one K tile on its way while it waits for the other, and a
+// 128 x 128 tile took 0.85 us per 128 bytes of K where its matrix instructions need 0.2.  So each tile keeps as many stages as
+// LDS holds with one workgroup per CU (32 x 64 and 64 x 64: two) -- 128 x 128 x 4 stages 0.5 us; small row counts get tiles no
+// taller than they need, and row counts just above a multiple of 256 those of 128 and 192.  Measured, weights from HBM, before
+// (128 x 128 and 256 x 128 tiles of two and three stages, the former with K split) and now, in us:
+//   16 x 3584 x 18944 29.6 -> 19.9   64 x 4096 x 4096 15.6 -> 10.8    64 x 8192 x 28672 64 -> 50     333 x 3584 x 18944 54 -> 34
+//   150 x 8192 x 8192 39.9 -> 34.3   333 x 14336 x 4096 58 -> 44      512 x 3584 x 18944 63 -> 46    512 x 18432 x 7168 122 -> 89
+// The estimates are fitted to a sweep of every tile over 1 .. 1600 rows and weights of 4096 x 4096 to 8192 x 28672: per K tile of
+// 128 bytes t0 + t1 * (share of the CUs at work), c beside, in whole rounds of the chip; the two small tiles share a CU, and
+// time grows with their number from the first that does.  Within the region the chosen tile is within 10 % of the best measured.
+Int8TilePlan int8_tile_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split)
+{
+    const int64_t cus = 256, kt = (K + 127) / 128;
+    auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
+    if (M > 128 && N > 128 && tiles(256, 256) >= cus) return {0, 1};
+    const double from_hbm = ((double)N + (double)M) * (double)K * (double)batch / 4.7e6 + 3.0;
+    Int8TilePlan best{0, 1};
+    double best_us = 1e30;
+    auto offer = [&](int variant, int splits, double us) {
+        if (us < from_hbm) us = from_hbm;
+        if (splits > 1) us += 4.4 + 8.0 * splits * (double)M * (double)N * (double)batch / 5.0e6;   // partial sums, second kernel
+        if (us < best_us) { best_us = us; best = {variant, splits}; }
+    };
+    auto rounds = [&](int64_t t, int64_t slots, double steps, double t0, double t1, double c) {
+        const int64_t full = t / slots, rest = t % slots;
+        return (double)full * (steps * (t0 + t1) + c) + (rest ? steps * (t0 + t1 * (double)rest / (double)slots) + c : 0.0);
+    };
+    auto shared = [&](int64_t t, double steps, double one, double two, double more) {
+        return t <= cus ? steps * one + 2.7 : steps * (more * t / cus > two ? more * t / cus : two) + 2.7;
+    };
+    for (int s = 1; s <= 16 && (s == 1 || (may_split && kt / s >= 4 && K % 128 == 0)); s++) {
+        const double steps = (double)((kt + s - 1) / s);
+        const int64_t t32 = tiles(32, 64) * s, t64 = tiles(64, 64) * s, t128 = tiles(128, 128) * s;
+        if (s == 1 || t32 <= 2 * cus) offer(OPSNN_VARIANT_I8_T32, s, shared(t32, steps, 0.24, 0.50, 0.265));
+        if (s == 1 || t64 <= 2 * cus) offer(OPSNN_VARIANT_I8_T64, s, shared(t64, steps, 0.27, 0.58, 0.31));
+        if (s == 1 || t128 <= cus) offer(OPSNN_VARIANT_I8_T128, s, rounds(t128, cus, steps, 0.40, 0.22, 3.0));
+    }
+    const double steps = (double)kt;
+    offer(OPSNN_VARIANT_I8_128, 1, rounds(tiles(128, 128), 2 * cus, steps, 0.95, 0.15, 3.0));   // two stages, two workgroups per CU
+    offer(OPSNN_VARIANT_I8_T128x256, 1, rounds(tiles(128, 256), cus, steps, 0.77, 0.20, 4.0));
+    offer(OPSNN_VARIANT_I8_T192, 1, rounds(tiles(192, 256), cus, steps, 1.12, 0.20, 4.0));
+    offer(OPSNN_VARIANT_I8_256_W8_K128, 1, rounds(tiles(256, 256), cus, steps, 1.20, 0.20, 8.0));
+    if (K % 128 == 0 && K >= 3072)   // (with fewer K tiles the eight-wave kernels are ahead of the four-wave one)
+        for (int fn = 8; fn <= 11; fn++) offer(fn, 1, rounds(tiles(256, 32 * fn), cus, steps, 0.1445 * fn, 0.0595 * fn, 8.0));
+    return best;
+}
+}  // namespace opsnn
+
 static int64_t cu_count()
 {
     static const int n = [] {
@@ -194,6 +244,20 @@ static int qmm_int8_impl(const OpsnnQmmArgs* a, void* stream, SplitK sk)
             }
             return qgemm_launch_int<256, 256, 128, 2, 4, 2, 1>(g, a->batch, p.out_dt, st);
         }
+        int splits = 1;
+        if (variant == OPSNN_VARIANT_AUTO) {   // the chip not filled by 256 x 256 tiles: the fitting tile, K split over workgroups where `sk` has room
+            const Int8TilePlan pl = int8_tile_plan(p.M, p.N, p.K, a->batch, sk.splits > 1);
+            variant = pl.variant;
+            splits = pl.splits <= sk.splits ? pl.splits : 1;
+        }
+        if (splits > 1) {   // (integer partial sums: the same bits)
+            g.splits = splits; g.part = (int32_t*)sk.part;
+            switch (variant) {
+                case OPSNN_VARIANT_I8_T32: return qgemm_launch_split_i8<32, 64, 128, 1, 2, 6, 1>(g, a->batch, p.out_dt, st);
+                case OPSNN_VARIANT_I8_T64: return qgemm_launch_split_i8<64, 64, 128, 2, 2, 5, 1>(g, a->batch, p.out_dt, st);
+                default: return qgemm_launch_split_i8<128, 128, 128, 2, 4, 4, 1>(g, a->batch, p.out_dt, st);
+            }
+        }
         if (variant >= OPSNN_VARIANT_I8_WIDE8 && variant <= OPSNN_VARIANT_I8_WIDE11) {
             const int rc = launch_int8_wide(g, variant, a->batch, p.out_dt, st);
             if (rc != OPSNN_NOT_TAKEN) return rc;
@@ -205,15 +269,15 @@ static int qmm_int8_impl(const OpsnnQmmArgs* a, void* stream, SplitK sk)
             case OPSNN_VARIANT_I8_256_W8: return qgemm_launch<MODE_I8, 256, 256, 64, 2, 4, 4, 1>(g, a->batch, p.out_dt, st);
             case OPSNN_VARIANT_I8_256_S4: return qgemm_launch<MODE_I8, 256, 256, 64, 2, 2, 4, 1>(g, a->batch, p.out_dt, st);
             case OPSNN_VARIANT_I8_256_W8_K128: return qgemm_launch<MODE_I8, 256, 256, 128, 2, 4, 2, 1>(g, a->batch, p.out_dt, st);
+            case OPSNN_VARIANT_I8_T32: return qgemm_launch<MODE_I8, 32, 64, 128, 1, 2, 6, 1>(g, a->batch, p.out_dt, st);
+            case OPSNN_VARIANT_I8_T64: return qgemm_launch<MODE_I8, 64, 64, 128, 2, 2, 5, 1>(g, a->batch, p.out_dt, st);
+            case OPSNN_VARIANT_I8_T128: return qgemm_launch<MODE_I8, 128, 128, 128, 2, 4, 4, 1>(g, a->batch, p.out_dt, st);
+            case OPSNN_VARIANT_I8_T128x256: return qgemm_launch<MODE_I8, 128, 256, 128, 2, 4, 3, 1>(g, a->batch, p.out_dt, st);
+            case OPSNN_VARIANT_I8_T192: return qgemm_launch<MODE_I8, 192, 256, 128, 2, 4, 2, 1>(g, a->batch, p.out_dt, st);
             default: break;
         }
-        if (p.M <= 128 || p.N <= 128 || p.M * p.N <= 256 * 256 * 64) {
-            if (sk.splits > 1 && p.K % 128 == 0) {   // few tiles against a long K: K split over workgroups, integer partial sums
-                g.splits = sk.splits; g.part = (int32_t*)sk.part;
-                return qgemm_launch_split_i8<128, 128, 128, 2, 2, 2, 1>(g, a->batch, p.out_dt, st);
-            }
+        if (p.M * p.N <= 256 * 256 * 64)   // (a batch of small products)
             return qgemm_launch<MODE_I8, 128, 128, 128, 2, 2, 2, 1>(g, a->batch, p.out_dt, st);
-        }
         // Large shapes: 256x256 tiles, one per CU at a time, are the most economical in operand traffic, but only
         // whole rounds of them keep every CU busy.  Columns that fill whole rounds go to that kernel; the remaining
         // columns (less than one round) go to 128x128 tiles, two workgroups per CU, in a second launch.
@@ -225,8 +289,8 @@ static int qmm_int8_impl(const OpsnnQmmArgs* a, void* stream, SplitK sk)
         int64_t wide_cost = INT64_MAX;
         int wide_fn = 0;
         // (from 24 K tiles up: with fewer the 8-wave kernels, whose second wave per SIMD covers prologue and epilogue,
-        // are ahead -- 8192 x 1024 x 8192: 96 against 114 us, 4096 x 2048 x 14336: 147 against 154; and from 3/4 of a round of 256 x 256 tiles up)
-        if (p.K % 128 == 0 && p.K >= 3072 && tm * tn * a->batch * 4 >= cus * 3) {
+        // are ahead -- 8192 x 1024 x 8192: 96 against 114 us, 4096 x 2048 x 14336: 147 against 154)
+        if (p.K % 128 == 0 && p.K >= 3072) {
             for (int fn = 8; fn <= 11; fn++) {
                 const int64_t tiles = tm * ((p.N + 32 * fn - 1) / (32 * fn)) * a->batch;
                 const int64_t cost = (tiles + cus - 1) / cus * (fn + 2);   // + 2: what a tile costs beyond its width (8192^3: 3 rounds of 352 columns 495 us, 4 of 256 529 us)
