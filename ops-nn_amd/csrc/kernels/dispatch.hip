@@ -251,7 +251,7 @@ static int splitk_for(const OpsnnQmmArgs& a, int mode)
     double bytes_per_us = 5.0e6;   // what its partial sums' traffic was measured to cost (splitk_factor)
     // int8 with per-token / per-channel scales (whole K tiles): integer partial sums, so the result stays bit-identical
     if ((mode == 0 || (mode == 3 && !a.x1_scale)) && a.x1_dtype == DT_I8 && a.x2_dtype == DT_I8 && out16 && a.K % 128 == 0)
-        return int8_tile_plan(a.M, a.N, a.K, a.batch, true).splits;
+        return tile_plan(a.M, a.N, a.K, a.batch, true).splits;
     if (tiny) return 1;
     // MXFP4: 128 x 128 tiles when 256 x 256 ones would be few (the launcher's rule), K tiles counted in 256 elements
     if (mode == 2 && a.x1_dtype == DT_E2M1 && a.x2_dtype == DT_E2M1 && (out16 || a.out_dtype == DT_F32)) {

@@ -6,10 +6,10 @@
 namespace opsnn {
 
 // How a [M, K] x [N, K] product of 16-bit operands is tiled.  cfg: 8 .. 11 the four-wave kernel with 256 x 32*cfg tiles
-// (qmm_int8_wide.hip); 2: 128 x 128 tiles, two workgroups per CU.  splits > 1 (cfg 2): K split over workgroups, fp32 partial
-// sums [splits][batch][M][N].  us: the estimate that the choice rests on.
+// (qmm_int8_wide.hip), else the OPSNN_VARIANT_I8_* tile of that number.  splits > 1: K split over workgroups, fp32 partial sums
+// [splits][batch][M][N].  us: the estimate that the choice rests on.
 struct Gemm16Plan {
-    int cfg = 2, splits = 1;
+    int cfg = OPSNN_VARIANT_I8_128, splits = 1;
     double us = 0;
 };
 Gemm16Plan gemm16_plan(int64_t M, int64_t N, int64_t K, int64_t batch);

@@ -26,10 +26,10 @@ __global__ __launch_bounds__(256) void gemm16_splitk_reduce_kernel(QgemmParams p
     });
 }
 
-template <int MODE, int BM, int BN, int WGM, int WGN>
+template <int MODE, int BM, int BN, int WGM, int WGN, int STAGES>
 static int launch_split16(const QgemmParams& p, int64_t batch, int out_dt, hipStream_t st)
 {
-    constexpr int BK = 128, STAGES = 2;
+    constexpr int BK = 128;
     if (!p.part || p.splits < 2 || (p.KB % BK) != 0 || p.splits > p.KB / BK / 2 || p.ldc != p.N) return -1;
     const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
     const size_t lds = (size_t)STAGES * (BM + BN) * BK;
@@ -51,36 +51,45 @@ static int launch_split16(const QgemmParams& p, int64_t batch, int out_dt, hipSt
 template <int MODE>
 static int launch16(const QgemmParams& p, const Gemm16Plan& pl, int64_t batch, int out_dt, hipStream_t st)
 {
-    if (pl.cfg >= 8) return launch_16_wide(p, pl.cfg, MODE == MODE_BF16, batch, out_dt, st);
-    if (pl.splits > 1) return launch_split16<MODE, 128, 128, 2, 2>(p, batch, out_dt, st);
-    return qgemm_launch<MODE, 128, 128, 128, 2, 2, 2, 1>(p, batch, out_dt, st);
+    if (pl.cfg >= OPSNN_VARIANT_I8_WIDE8 && pl.cfg <= OPSNN_VARIANT_I8_WIDE11) return launch_16_wide(p, pl.cfg, MODE == MODE_BF16, batch, out_dt, st);
+    if (pl.splits > 1) {
+        if (pl.cfg == OPSNN_VARIANT_I8_T64) return launch_split16<MODE, 64, 64, 2, 2, 5>(p, batch, out_dt, st);
+        return launch_split16<MODE, 128, 128, 2, 4, 4>(p, batch, out_dt, st);
+    }
+    switch (pl.cfg) {
+        case OPSNN_VARIANT_I8_T64: return qgemm_launch<MODE, 64, 64, 128, 2, 2, 5, 1>(p, batch, out_dt, st);
+        case OPSNN_VARIANT_I8_T128: return qgemm_launch<MODE, 128, 128, 128, 2, 4, 4, 1>(p, batch, out_dt, st);
+        case OPSNN_VARIANT_I8_T128x256: return qgemm_launch<MODE, 128, 256, 128, 2, 4, 3, 1>(p, batch, out_dt, st);
+        case OPSNN_VARIANT_I8_T192: return qgemm_launch<MODE, 192, 256, 128, 2, 4, 2, 1>(p, batch, out_dt, st);
+        case OPSNN_VARIANT_I8_256_W8_K128: return qgemm_launch<MODE, 256, 256, 128, 2, 4, 2, 1>(p, batch, out_dt, st);
+        default: return qgemm_launch<MODE, 128, 128, 128, 2, 2, 2, 1>(p, batch, out_dt, st);
+    }
 }
 
-// The estimate, in microseconds, for each tiling; fitted to one box (random operands, K = 4096 .. 18432):
+// Fewer 256 x 256 tiles than CUs: tile_plan (qmm_int8.hip), whose K tiles of 128 bytes take the same time here -- half as many
+// products per byte at half the rate.  Otherwise the estimate, in microseconds, of the two kernels for large shapes, fitted to
+// one box (random operands, K = 4096 .. 18432):
 //   four-wave kernel: 0.185 us per 32 columns of tile width and 64-element K tile, 8 us a round beside (4096^3: 99 us in one
 //   round of 256 x 256 tiles = 1.39 Pflop/s; 2048 x 4096 x 11008: 134 us in one round of 256 x 352);
-//   128 x 128 tiles: 0.65 us per K tile alone on a CU, 1.0 us for two that share one, 6 us beside;
-//   K split: the partial sums written and read back at 4 TB/s, and 5 us for the second kernel.
+//   128 x 128 tiles: 0.65 us per K tile alone on a CU, 1.0 us for two that share one, 6 us beside.
 Gemm16Plan gemm16_plan(int64_t M, int64_t N, int64_t K, int64_t batch)
 {
     const int64_t cus = 256, kt = K / 64;
     Gemm16Plan best;
+    if (const TilePlan t = tile_plan(M, N, 2 * K, batch, true, false); t.variant) {
+        best.cfg = t.variant; best.splits = t.splits; best.us = t.us;
+        return best;
+    }
     best.us = 1e30;
     const int64_t tm = (M + 255) / 256;
     for (int fn = 8; fn <= 11; fn++) {
         const int64_t tiles = tm * ((N + 32 * fn - 1) / (32 * fn)) * batch;
         const double us = (double)((tiles + cus - 1) / cus) * (0.185 * fn * (double)kt + 8.0);
-        if (us < best.us) { best.cfg = fn; best.splits = 1; best.us = us; }
+        if (us < best.us) { best.cfg = fn; best.us = us; }
     }
-    const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128) * batch;
-    for (int s = 1; s <= 16; s++) {
-        if (s > 1 && (t128 * s > 2 * cus || kt / s < 4)) break;
-        const int64_t per_cu = (t128 * s + cus - 1) / cus;
-        const double steps = (double)(kt + s - 1) / s;
-        double us = steps * ((double)(per_cu / 2) * 1.0 + (double)(per_cu % 2) * 0.65) + 6.0;
-        if (s > 1) us += 5.0 + 8.0 * s * (double)M * (double)N * (double)batch / 4.0e6;
-        if (us < best.us) { best.cfg = 2; best.splits = s; best.us = us; }
-    }
+    const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128) * batch, per_cu = (t128 + cus - 1) / cus;
+    const double us = (double)kt * ((double)(per_cu / 2) * 1.0 + (double)(per_cu % 2) * 0.65) + 6.0;
+    if (us < best.us) { best.cfg = OPSNN_VARIANT_I8_128; best.us = us; }
     return best;
 }
 

@@ -15,7 +15,7 @@ enum {
     OPSNN_VARIANT_I8_256_W8_K128 = 7,  // int8 MFMA, 256x256 tile, 8 waves, BK 128, 2 stages
     OPSNN_VARIANT_I8_WIDE8 = 8,   // int8 MFMA, 4 waves with 128 x 16n sub-tiles, 256 x 32n tile, n = 8..11 (ids 8..11)
     OPSNN_VARIANT_I8_WIDE11 = 11,
-    OPSNN_VARIANT_I8_T32 = 12,    // int8 MFMA, the tiles of int8_tile_plan: 32x64, 6 stages
+    OPSNN_VARIANT_I8_T32 = 12,    // int8 MFMA, the tiles of tile_plan: 32x64, 6 stages
     OPSNN_VARIANT_I8_T64 = 13,    // 64x64, 5 stages
     OPSNN_VARIANT_I8_T128 = 14,   // 128x128, 4 stages
     OPSNN_VARIANT_I8_T128x256 = 15,  // 128x256, 3 stages
@@ -73,12 +73,14 @@ inline int splitk_factor(int64_t tiles, int64_t ktiles, double tile_us, int64_t 
     }
     return best;
 }
-// How an int8 x int8 product whose 256 x 256 tiles would not fill the chip once (or of up to 128 rows or columns) is tiled
-// (qmm_int8.hip).  variant: the OPSNN_VARIANT_I8_* kernel, 0 if the shape is outside; splits: K segments.
-struct Int8TilePlan {
+// How a product of two K-contiguous operands whose 256 x 256 tiles would not fill the chip once (or of up to 128 rows or columns)
+// is tiled (qmm_int8.hip; int8, and the 16-bit operands of gemm16.hip).  KB: bytes of K.  variant: the OPSNN_VARIANT_I8_*
+// tile, 0 if the shape is outside; splits: K segments; us: the estimate that the choice rests on.
+struct TilePlan {
     int variant, splits;
+    double us;
 };
-Int8TilePlan int8_tile_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split);
+TilePlan tile_plan(int64_t M, int64_t N, int64_t KB, int64_t batch, bool may_split, bool tiles_of_32 = true);
 
 // How the x-in-registers kernel (weight-only, up to 16 rows of x) covers K.  A workgroup holds `nw` waves x `nch` chunks
 // (of 64 weight bytes): 16 x 4, 8-bit weights also 16 x 8, or 8 x 4 / 8 x 8.  A K that is exactly one such shape runs on

@@ -92,18 +92,17 @@ namespace opsnn {
 // The estimates are fitted to a sweep of every tile over 1 .. 1600 rows and weights of 4096 x 4096 to 8192 x 28672: per K tile of
 // 128 bytes t0 + t1 * (share of the CUs at work), c beside, in whole rounds of the chip; the two small tiles share a CU, and
 // time grows with their number from the first that does.  Within the region the chosen tile is within 10 % of the best measured.
-Int8TilePlan int8_tile_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split)
+TilePlan tile_plan(int64_t M, int64_t N, int64_t KB, int64_t batch, bool may_split, bool tiles_of_32)
 {
-    const int64_t cus = 256, kt = (K + 127) / 128;
+    const int64_t cus = 256, kt = (KB + 127) / 128;
     auto tiles = [&](int64_t bm, int64_t bn) { return ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch; };
-    if (M > 128 && N > 128 && tiles(256, 256) >= cus) return {0, 1};
-    const double from_hbm = ((double)N + (double)M) * (double)K * (double)batch / 4.7e6 + 3.0;
-    Int8TilePlan best{0, 1};
-    double best_us = 1e30;
+    if (M > 128 && N > 128 && tiles(256, 256) >= cus) return {0, 1, 0.0};
+    const double from_hbm = ((double)N + (double)M) * (double)KB * (double)batch / 4.7e6 + 3.0;
+    TilePlan best{0, 1, 1e30};
     auto offer = [&](int variant, int splits, double us) {
         if (us < from_hbm) us = from_hbm;
         if (splits > 1) us += 4.4 + 8.0 * splits * (double)M * (double)N * (double)batch / 5.0e6;   // partial sums, second kernel
-        if (us < best_us) { best_us = us; best = {variant, splits}; }
+        if (us < best.us) best = {variant, splits, us};
     };
     auto rounds = [&](int64_t t, int64_t slots, double steps, double t0, double t1, double c) {
         const int64_t full = t / slots, rest = t % slots;
@@ -112,10 +111,10 @@ Int8TilePlan int8_tile_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool
     auto shared = [&](int64_t t, double steps, double one, double two, double more) {
         return t <= cus ? steps * one + 2.7 : steps * (more * t / cus > two ? more * t / cus : two) + 2.7;
     };
-    for (int s = 1; s <= 16 && (s == 1 || (may_split && kt / s >= 4 && K % 128 == 0)); s++) {
+    for (int s = 1; s <= 16 && (s == 1 || (may_split && kt / s >= 4 && KB % 128 == 0)); s++) {
         const double steps = (double)((kt + s - 1) / s);
         const int64_t t32 = tiles(32, 64) * s, t64 = tiles(64, 64) * s, t128 = tiles(128, 128) * s;
-        if (s == 1 || t32 <= 2 * cus) offer(OPSNN_VARIANT_I8_T32, s, shared(t32, steps, 0.24, 0.50, 0.265));
+        if (tiles_of_32 && (s == 1 || t32 <= 2 * cus)) offer(OPSNN_VARIANT_I8_T32, s, shared(t32, steps, 0.24, 0.50, 0.265));
         if (s == 1 || t64 <= 2 * cus) offer(OPSNN_VARIANT_I8_T64, s, shared(t64, steps, 0.27, 0.58, 0.31));
         if (s == 1 || t128 <= cus) offer(OPSNN_VARIANT_I8_T128, s, rounds(t128, cus, steps, 0.40, 0.22, 3.0));
     }
@@ -124,7 +123,7 @@ Int8TilePlan int8_tile_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool
     offer(OPSNN_VARIANT_I8_T128x256, 1, rounds(tiles(128, 256), cus, steps, 0.77, 0.20, 4.0));
     offer(OPSNN_VARIANT_I8_T192, 1, rounds(tiles(192, 256), cus, steps, 1.12, 0.20, 4.0));
     offer(OPSNN_VARIANT_I8_256_W8_K128, 1, rounds(tiles(256, 256), cus, steps, 1.20, 0.20, 8.0));
-    if (K % 128 == 0 && K >= 3072)   // (with fewer K tiles the eight-wave kernels are ahead of the four-wave one)
+    if (KB % 128 == 0 && KB >= 3072)   // (with fewer K tiles the eight-wave kernels are ahead of the four-wave one)
         for (int fn = 8; fn <= 11; fn++) offer(fn, 1, rounds(tiles(256, 32 * fn), cus, steps, 0.1445 * fn, 0.0595 * fn, 8.0));
     return best;
 }
@@ -246,7 +245,7 @@ static int qmm_int8_impl(const OpsnnQmmArgs* a, void* stream, SplitK sk)
         }
         int splits = 1;
         if (variant == OPSNN_VARIANT_AUTO) {   // the chip not filled by 256 x 256 tiles: the fitting tile, K split over workgroups where `sk` has room
-            const Int8TilePlan pl = int8_tile_plan(p.M, p.N, p.K, a->batch, sk.splits > 1);
+            const TilePlan pl = tile_plan(p.M, p.N, p.K, a->batch, sk.splits > 1);
             variant = pl.variant;
             splits = pl.splits <= sk.splits ? pl.splits : 1;
         }

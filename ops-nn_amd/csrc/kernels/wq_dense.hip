@@ -99,14 +99,30 @@ static int launch_dequant(const WqParams& p, bool kn, uint16_t* out, hipStream_t
 
 static uint64_t dense_weight_bytes(const OpsnnWqmmArgs& a) { return ((uint64_t)a.N * (uint64_t)a.K * 2 + 255) / 256 * 256; }
 
+// What the many-rows streaming kernel takes, in us: a workgroup of 128 columns and R rows (64, 128, 192 or 256) walks 4096 k in
+// 14 + 0.21 R (measured 27, 38, 52 and 67; a quarter less where few CUs have one), a CU at a time; rows as wq_narrow_slab_rows deals them, or in passes of 256.  With
+// more than 128 rows and a K that is no whole number of x rounds of those instances, three times that.
+static double rows_kernel_us(const OpsnnWqmmArgs& a, int wbits, int64_t group)
+{
+    const int64_t wgs = (a.N + 127) / 128, kx = 2 * 4 * (128 / wbits), slab = wq_narrow_slab_rows(a.M, a.N, true);
+    const int64_t ks = wq_rows_ksplit(wbits, a.M, a.N, a.K, group, true);
+    auto launch_us = [&](int64_t rows, int64_t slabs) {
+        const int64_t r = (rows + 63) / 64 * 64, n = wgs * slabs * ks;
+        const double rounds = n < 256 ? 0.75 + 0.25 * (double)n / 256.0 : (double)((n + 255) / 256);
+        return rounds * (double)a.K / (4096.0 * (double)ks) * (14.0 + 0.21 * (double)r) * (r > 128 && a.K % (4 * kx) != 0 ? 3.0 : 1.0);
+    };
+    const double part_us = ks > 1 ? 4.0 + 8.0 * (double)ks * (double)a.M * (double)a.N / 5.0e6 : 0.0;
+    if (slab) return launch_us(slab, (a.M + slab - 1) / slab) + part_us;
+    return (double)(a.M / 256) * launch_us(256, 1) + (a.M % 256 ? launch_us(a.M % 256, 1) : 0.0) + part_us;
+}
+
 // Does the call run on this route?  Looks at what phase 1 knows (shapes, types, layouts, addresses), so that both phases agree.
 //
-// The pass moves 2.5 (8-bit weights: 3) bytes per weight at 4.4 TB/s, the product takes what gemm16_plan estimates.  Against
+// The pass moves 2.5 (8-bit weights: 3) bytes per weight at 5 TB/s, the product takes what gemm16_plan estimates.  Against
 // it stands the many-rows streaming kernel where it runs (wqmm.hip: [N, K] storage, N % 32 == 0, whole x slabs and groups of
-// whole chunks), which keeps 0.78 Pflop/s from 256 rows on if K is a whole number of rounds for its 256-row instance, a
-// third of that if not; everywhere else the general kernel re-reads the weight per 64 rows at a fraction of its speed, and this
+// whole chunks); everywhere else the general kernel re-reads the weight per 64 rows at a fraction of its speed, and this
 // route takes every call of more than 64 rows.  (Measured: 1999 x 4096 x 11008 bf16 x int4 228 -> 156 us, [K, N] storage
-// 613 -> 162; 1024 x 8192 x 28672 497 against 499, 512 rows 254 against 330.)
+// 613 -> 162; 700 x 4096 x 11008 134 -> 106; 1024 x 8192 x 28672 497 against 499, 512 rows 254 against 330.)
 bool wq_dense_wanted(const OpsnnWqmmArgs& a)
 {
     if (a.w_dtype != DT_I4 && a.w_dtype != DT_I8) return false;
@@ -125,9 +141,8 @@ bool wq_dense_wanted(const OpsnnWqmmArgs& a)
     const bool rows_kernel = nk && a.N % 32 == 0 && a.N >= 256 && a.K % (2 * kc) == 0 &&
                              (a.group <= 0 || a.group >= a.K || (a.group % kc == 0 && (cpg & (cpg - 1)) == 0));
     if (!rows_kernel) return true;
-    const double flops = 2.0 * (double)a.M * (double)a.N * (double)a.K;
-    const double rows_us = flops / (a.M <= 128 || a.K % (8 * kc) == 0 ? 0.78e9 : 0.26e9);
-    const double dense_us = (double)a.N * (double)a.K * (2.0 + wbits / 8.0) / 4.4e6 + gemm16_plan(a.M, a.N, a.K, 1).us;
+    const double rows_us = rows_kernel_us(a, wbits, a.group > 0 && a.group < a.K ? a.group : a.K);
+    const double dense_us = 2.0 + (double)a.N * (double)a.K * (2.0 + wbits / 8.0) / 5.0e6 + gemm16_plan(a.M, a.N, a.K, 1).us;
     return dense_us < rows_us;
 }
 uint64_t wq_dense_workspace(const OpsnnWqmmArgs& a)

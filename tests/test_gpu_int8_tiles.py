@@ -1,4 +1,4 @@
-"""int8 per-token x per-channel calls whose 256 x 256 tiles do not fill the chip (int8_tile_plan): each of their tiles, pinned, at
+"""int8 per-token x per-channel calls whose 256 x 256 tiles do not fill the chip (tile_plan): each of their tiles, pinned, at
 its edges -- one row, a row more and less than a tile, ragged N, fewer K tiles than stages, a K that ends inside a tile -- and
 shapes that the plan cuts along K.  Integer sums: bit-identical to the oracle."""
 import ctypes as C
