@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("M,K,N,group", [
     (1, 256, 256, 0), (16, 288, 258, 128), (17, 1024, 520, 64), (32, 4096, 1002, 128), (33, 2080, 384, 32), (64, 8192, 300, 128),
-    (7, 4160, 2048, 128), (3, 18432, 1026, 0), (48, 3008, 4098, 64), (15, 11008, 770, 352),
+    (7, 4160, 2048, 128), (3, 18432, 1026, 0), (48, 3008, 4098, 64), (15, 11008, 770, 352), (9, 8192, 2064, 0),
 ])
 @pytest.mark.parametrize("w_dt,x_dt,off", [("i4", "f16", True), ("i4", "bf16", False), ("i8", "f16", False), ("i8", "bf16", True)])
 def test_kn_stream(gpu, M, K, N, group, w_dt, x_dt, off):
@@ -28,3 +28,19 @@ def test_kn_one_scale(gpu):
     m = gpu
     inp = cases.make_wq_inputs(m, 9, 512, 272, 3, m.ACL_FLOAT16, m.ACL_INT8, 0, False, True, None, per_tensor=True)
     _b16_bar(cases.run_wq_aclnn(m, inp, 9, 512, 272), cases.oracle_wq(m, inp, 9, 512, 272), orc.F16, "kn one scale", 512)
+
+
+@pytest.mark.parametrize("M,K,N,w_dt", [(16, 1024, 512, "i4"), (1, 4096, 512, "i8"), (16, 4096, 1024, "i8")])
+def test_small_weights_give_the_bits_of_their_k_contiguous_form(gpu, M, K, N, w_dt):
+    import numpy as np
+    m = gpu
+    wd = m.ACL_INT4 if w_dt == "i4" else m.ACL_INT8
+    inp = cases.make_wq_inputs(m, M, K, N, 5, m.ACL_BF16, wd, 0, False, False, None)
+    w = inp["w"].reshape(K, -1)
+    if w_dt == "i4":
+        n = orc.unpack_nibbles(inp["w"]).reshape(K, N).T
+        w = ((n[:, 0::2] & 15) | (n[:, 1::2] << 4)).astype(np.uint8)
+    else:
+        w = w.T
+    other = dict(inp, w=np.ascontiguousarray(w), tW=True)
+    assert np.array_equal(cases.run_wq_aclnn(m, inp, M, K, N), cases.run_wq_aclnn(m, other, M, K, N))
