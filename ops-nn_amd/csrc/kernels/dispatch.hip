@@ -239,8 +239,8 @@ static int splitk_for(const OpsnnQmmArgs& a, int mode)
     if ((mode == 1 || mode == 3) && f8 && a.M <= 128) {
         if (const int sr = mode == 1 ? blockscale_rows_ksplit(a) : rowcol_rows_ksplit(a); sr > 1) return sr;
     }
-    // 33 .. 256 rows of MXFP8 on the many-rows kernel
-    if (mode == 2 && f8 && a.M <= 256) {
+    // 33 .. 128 rows of MXFP8 on the many-rows kernel
+    if (mode == 2 && f8 && a.M <= 128) {
         if (const int sr = mxfp8_rows_ksplit(a); sr > 1) return sr;
     }
     // (fewer than 64 x 64 outputs are the plain kernels' -- except int8 with few outputs against a long K, qmm_int8.hip)
@@ -263,10 +263,11 @@ static int splitk_for(const OpsnnQmmArgs& a, int mode)
     else if (a.M <= 16) return 1;   // (up to 16 rows the streaming kernels take the modes below)
     else if (mode == 2 && a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E2M1 && out16) { bm = 256; tile_us = 1.8; }
     else if (mode == 1 && a.x1_dtype == DT_I8 && a.x2_dtype == DT_I8 && a.gsK == 128 && a.gsN == 128 && out16) { bm = a.M >= 512 ? 256 : 128; tile_us = 1.8; }
-    else if (mode == 1 && f8 && a.gsK == 128 && a.gsN == 128 && !a.bias && a.M > 128 && (out16 || a.out_dtype == DT_F32)) { bm = 256; bn = 128; tile_us = 1.4; }
-    else if (mode == 2 && f8 && (out16 || a.out_dtype == DT_F32)) { bm = 256; bn = 128; tile_us = 1.4; }
+    // (the exact fp8 kernel)
+    else if (mode == 1 && f8 && a.gsK == 128 && a.gsN == 128 && !a.bias && a.M > 128 && (out16 || a.out_dtype == DT_F32)) return fp8x_plan(a.M, a.N, a.K, a.batch, mode == 3, true).splits;
+    else if (mode == 2 && f8 && (out16 || a.out_dtype == DT_F32)) return fp8x_plan(a.M, a.N, a.K, a.batch, mode == 3, true).splits;
     else if (mode == 3 && (a.x1_dtype == DT_E4M3 || a.x1_dtype == DT_E5M2) && (a.x2_dtype == DT_E4M3 || a.x2_dtype == DT_E5M2) && a.M > 128 &&
-             (out16 || a.out_dtype == DT_F32)) { bm = 256; bn = 128; tile_us = 1.4; }
+             (out16 || a.out_dtype == DT_F32)) return fp8x_plan(a.M, a.N, a.K, a.batch, mode == 3, true).splits;
     else return 1;
     const int64_t tiles = ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * a.batch;
     return splitk_factor(tiles, (a.K + kunit - 1) / kunit, tile_us, a.M * a.N * a.batch, bytes_per_us);

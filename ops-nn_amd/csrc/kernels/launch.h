@@ -20,8 +20,11 @@ enum {
     OPSNN_VARIANT_I8_T128 = 14,   // 128x128, 4 stages
     OPSNN_VARIANT_I8_T128x256 = 15,  // 128x256, 3 stages
     OPSNN_VARIANT_MX_128 = 16,    // MX MFMA, 128x128 tile
-    OPSNN_VARIANT_I8_T192 = 18,   // int8 MFMA, 192x256, 2 stages
     OPSNN_VARIANT_MX_FP8_MFMA = 17,  // MXFP8 on the MFMA path (reduced accumulation precision, see qmm_mx.hip)
+    OPSNN_VARIANT_I8_T192 = 18,   // int8 MFMA, 192x256, 2 stages
+    OPSNN_VARIANT_FP8X_256x128 = 32,   // the tiles of the exact fp8 kernel (qmm_fp8_exact.hip)
+    OPSNN_VARIANT_FP8X_128x256 = 33,
+    OPSNN_VARIANT_FP8X_128x128 = 34,
 };
 
 #ifdef __cplusplus
@@ -81,6 +84,13 @@ struct TilePlan {
     double us;
 };
 TilePlan tile_plan(int64_t M, int64_t N, int64_t KB, int64_t batch, bool may_split, bool tiles_of_32 = true);
+
+// The tile (OPSNN_VARIANT_FP8X_*) and the K segments of a call on the exact fp8 kernel (qmm_fp8_exact.hip); plain: row / column
+// scales only.
+struct Fp8xPlan {
+    int tile, splits;
+};
+Fp8xPlan fp8x_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool plain, bool may_split);
 
 // How the x-in-registers kernel (weight-only, up to 16 rows of x) covers K.  A workgroup holds `nw` waves x `nch` chunks
 // (of 64 weight bytes): 16 x 4, 8-bit weights also 16 x 8, or 8 x 4 / 8 x 8.  A K that is exactly one such shape runs on

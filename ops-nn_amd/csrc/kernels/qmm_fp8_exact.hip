@@ -15,7 +15,8 @@
 // (measured: bit-identical to the correctly rounded exact sum of 128 products in 99.5 % of cases, never further than
 // fp32 ascending-k summation), at half the matrix rate.
 //
-// Tiling: 256 x 128 output tile per workgroup, 4 x 2 waves of 64 x 64 (4 x 4 fragments of 16 x 16).  The operands stay
+// Tiling: waves of 64 x 64 (4 x 4 fragments of 16 x 16), 4 x 2 of them -- 256 x 128 output tile per workgroup --, 2 x 4 or
+// 2 x 2: which, says fp8x_tile.  The operands stay
 // e4m3 bytes on the way global -> LDS (16-byte asynchronous copies, rows XOR-swizzled) and LDS -> registers, exactly as
 // in qmm_fp8_block.hip; a lane's 32 bytes of a fragment become sixteen registers of fp16 pairs by sixteen
 // v_cvt_scalef32_pk_f16_fp8 (unit scale).  The x1 fragments are widened once per K tile and stay (64 registers), the
@@ -58,6 +59,7 @@ struct Fp8xParams {
     // K split over `splits` workgroups per tile (SPLIT instantiations, grid.z): fp32 partial sums [splits][batch][M][N] --
     // block scales already applied, row / column scales and bias not yet (fp8x_splitk_reduce_kernel applies them)
     int splits;
+    int tile;   // host only: the tile that `splits` was planned for
     float* part;
 #if QG_DBG
     unsigned long long* dbg;   // timing harness only: per wave, loop clocks / barrier-wait clocks / K tiles
@@ -122,19 +124,21 @@ __device__ __forceinline__ float fp8x_rowcol_epilogue(int ep_mode, float v, floa
     return (v * csv) * rs + bias;
 }
 
-template <int OUT_DT, bool RC, int FMT = 0, bool MXS = false, bool SPLIT = false>
-__global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int tiles_m, int tiles_n)
+template <int WGM, int WGN, int OUT_DT, bool RC, int FMT = 0, bool MXS = false, bool SPLIT = false>
+__global__ __launch_bounds__(WGM * WGN * 64, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int tiles_m, int tiles_n)
 {
     static_assert(!MXS || (RC && FMT == 0), "the MX mode is e4m3 x e4m3 with the row / column epilogue");
     constexpr bool AE5 = (FMT & 1) != 0, BE5 = (FMT & 2) != 0;
-    constexpr int BM = 256, BN = 128, BK = 128, NT = 512;
+    constexpr int BM = 64 * WGM, BN = 64 * WGN, BK = 128, NT = WGM * WGN * 64;
     constexpr int CPR = BK / 16, RPW = 16 / CPR;
     constexpr int TM = 64, TN = 64, FM = TM / 16, FN = TN / 16;
     constexpr int A_BYTES = BM * BK, B_BYTES = BN * BK;
     constexpr bool SCC = !RC || MXS;                 // a 4-byte copy per lane rides with every K tile
-    constexpr int SC_BYTES = SCC ? NT * 4 : 0;       // block scales: BM s1 floats + the s2 float of the tile's n block; MX: four e8m0 bytes per tile row
+    constexpr int SC_BYTES = SCC ? NT * 4 : 0;       // block scales: BM s1 floats + the s2 floats of the tile's n blocks; MX: four e8m0 bytes per tile row
+    static_assert(!MXS || NT >= BM + BN, "one scale copy per thread covers the tile's rows");
+    static_assert(BN == 128 || BN == 256, "whole n blocks");
     constexpr int STAGE = A_BYTES + B_BYTES + SC_BYTES;
-    constexpr int RPI = NT / CPR;                    // 64 tile rows per copy instruction of the workgroup
+    constexpr int RPI = NT / CPR;                    // tile rows per copy instruction of the workgroup
     constexpr int NA = BM / RPI, NB = BN / RPI;
     constexpr int CPT = NA + NB + (SCC ? 1 : 0);
     // Three stages: the tile being consumed, the next one (complete at this tile's barrier) and one more in flight, so a
@@ -147,7 +151,7 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave / WGN, wn = wave % WGN;
 
     // Tile order: each XCD (own L2) gets a contiguous range of ids, and ids run down groups of GM row tiles and across
     // the columns inside a group, so the 32 tiles an XCD works on at a time form a GM x (32 / GM) block that shares
@@ -173,7 +177,7 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
         B += (int64_t)kt_first * BK;
     }
 
-    // copies: instruction i of the workgroup fills tile rows i*64 .. i*64+63; this thread handles row i*64 + tid/8 and
+    // copies: instruction i of the workgroup fills tile rows i*RPI .. i*RPI+RPI-1; this thread handles row i*RPI + tid/8 and
     // the logical 16-byte chunk that belongs at position tid%8 of the swizzled row.  Rows past the matrix edge repeat
     // the last valid row: they only feed outputs that are never stored.
     const int crow = tid / CPR;
@@ -193,12 +197,12 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
         r = r < b_rows ? r : b_rows - 1;
         b_off[i] = (uint32_t)(r * ldb + cchunk * 16);
     }
-    // scale copy: lanes 0..255 (waves 0..3) fetch s1 of tile row `tid`, the others the s2 of this tile's n block: a
+    // scale copy: lanes 0..BM-1 (whole waves) fetch s1 of tile row `tid`, the others the s2 of this tile's n blocks: a
     // wave-uniform table base, a 32-bit byte offset per lane (the launcher checks that the tables stay below 4 GB)
     const char* sc_base = nullptr;
     uint32_t sc_off = 0;
     int64_t sc_step = 0;   // bytes per K tile
-    if constexpr (MXS) {   // lanes 0..255: the four bytes of x1 row `tid`; the others: of x2 row tid - 256 (the last 128 lanes repeat the last row)
+    if constexpr (MXS) {   // lanes 0..BM-1: the four bytes of x1 row `tid`; the others: of x2 row tid - BM (lanes past the last row repeat it)
         if (wave < BM / 64) {
             const int r = tid < a_rows ? tid : a_rows - 1;
             sc_base = (const char*)(p.sa + bz * p.sa_bs + m0 * p.sa_rs);
@@ -217,6 +221,7 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
             sc_step = p.s1_cs * 4;
         } else {
             sc_base = (const char*)(p.s2 + bz * p.s2_bs + (n0 / 128) * p.s2_cs);
+            if (BN == 256 && (tid & 1) && n0 + 128 < p.N) sc_off = (uint32_t)(p.s2_cs * 4);   // (two n blocks, in turn)
             sc_step = p.s2_rs * 4;
         }
     }
@@ -290,7 +295,7 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
             for (int i = 0; i < FN; i++) b_sraw[i] = sS[BM + wn * TN + i * 16 + frow];
         } else if constexpr (!RC) {
             const float* sS = (const float*)(st + A_BYTES + B_BYTES);
-            s2raw = sS[BM];
+            s2raw = sS[BM + wn * TN / 128];
 #pragma unroll
             for (int j = 0; j < FM; j++) s1raw[j] = sS[wm * TM + j * 16 + frow];
         }
@@ -493,7 +498,7 @@ __global__ __launch_bounds__(512, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int
     typedef v4i __attribute__((may_alias)) v4i_a;
     constexpr int EP_PITCH = TN * 2 + 16;
     char* ep = smem + wave * (16 * EP_PITCH);
-    static_assert(8 * 16 * EP_PITCH <= STAGES * STAGE, "epilogue staging fits in the operand stages");
+    static_assert(WGM * WGN * 16 * EP_PITCH <= STAGES * STAGE, "epilogue staging fits in the operand stages");
     uint16_t* out = (uint16_t*)p.out + bz * p.M * p.N;
     const bool vec_ok = (p.N % 8) == 0 && ((uintptr_t)p.out % 16) == 0;
     const int er = lane >> 3, ec = lane & 7;
@@ -582,15 +587,43 @@ __global__ __launch_bounds__(256) void fp8x_splitk_reduce_kernel(Fp8xParams p, i
     });
 }
 
-template <int OUT_DT, bool RC, int FMT = 0, bool MXS = false>
-static int launch_fp8_exact(const Fp8xParams& p, int64_t batch, hipStream_t st)
+// The tile and the K segments.  A tile of 256 rows wastes up to half of its work just above a multiple of 128 rows, and an extra
+// round of the chip costs a whole round: 333 x 3584 x 18944 ran as 296 tiles of 256 x 128 in two rounds, 96 us (row / column
+// scales; block scales 102, MX 107); 222 of 128 x 256 take 55 (57, 62).  128 x 128 tiles fill the chip where the others are half
+// as many and would be cut along K: 1024 x 4096 x 4096 47 -> 39 us (48 -> 42, 49 -> 43).  The chosen one has the smallest
+// estimate: per K tile t0 + t1 * (share of the CUs at work), 4 us a round beside, fitted to 14 shapes of 140 .. 2048 rows; the
+// row / column form (`plain`) has no scales to apply in its loop.
+Fp8xPlan fp8x_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool plain, bool may_split)
 {
-    const int tiles_m = (int)((p.M + 255) / 256), tiles_n = (int)((p.N + 127) / 128);
+    const int64_t cus = 256, kt = (K + 127) / 128;   // (a K tail runs padded)
+    Fp8xPlan best{OPSNN_VARIANT_FP8X_256x128, 1};
+    double best_us = 1e30;
+    auto offer = [&](int tile, int64_t bm, int64_t bn, double t0, double t1) {
+        const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch;
+        for (int s = 1; s <= 16 && (s == 1 || (may_split && tiles * s <= cus && kt / s >= 4)); s++) {
+            const double steps = (double)((kt + s - 1) / s);
+            const int64_t full = tiles * s / cus, rest = tiles * s % cus;
+            double us = (double)full * (steps * (t0 + t1) + 4.0) + (rest ? steps * (t0 + t1 * (double)rest / (double)cus) + 4.0 : 0.0);
+            if (s > 1) us += 5.0 + 8.0 * s * (double)M * (double)N * (double)batch / 6.0e6;   // partial sums, second kernel
+            if (us < best_us) { best_us = us; best = {tile, s}; }
+        }
+    };
+    offer(OPSNN_VARIANT_FP8X_256x128, 256, 128, plain ? 1.25 : 1.37, plain ? 0.40 : 0.46);
+    offer(OPSNN_VARIANT_FP8X_128x256, 128, 256, plain ? 1.25 : 1.37, plain ? 0.40 : 0.46);
+    offer(OPSNN_VARIANT_FP8X_128x128, 128, 128, plain ? 0.92 : 1.08, 0.12);
+    return best;
+}
+
+template <int WGM, int WGN, int OUT_DT, bool RC, int FMT, bool MXS>
+static int launch_fp8_exact_tile(const Fp8xParams& p, int64_t batch, hipStream_t st)
+{
+    constexpr int BM = 64 * WGM, BN = 64 * WGN, NT = WGM * WGN * 64;
+    const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
     dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch);
-    const size_t lds = 3 * (size_t)(256 * 128 + 128 * 128 + ((RC && !MXS) ? 0 : 512 * 4));
+    const size_t lds = 3 * (size_t)((BM + BN) * 128 + ((RC && !MXS) ? 0 : NT * 4));
     if (p.splits > 1) {   // K split over workgroups, then the sum of the partial sums, the epilogue and the rounding
         if (!p.part || p.splits > p.K / 128) return -1;
-        auto ks = qmm_fp8_exact_kernel<DT_F32, RC, FMT, MXS, true>;
+        auto ks = qmm_fp8_exact_kernel<WGM, WGN, DT_F32, RC, FMT, MXS, true>;
         static std::atomic<uint64_t> attr_set_s{0};
         if (!device_flag_test(attr_set_s)) {
             hipError_t e = hipFuncSetAttribute((const void*)ks, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -598,21 +631,32 @@ static int launch_fp8_exact(const Fp8xParams& p, int64_t batch, hipStream_t st)
             device_flag_set(attr_set_s);
         }
         grid.z = (unsigned)p.splits;
-        hipLaunchKernelGGL(ks, grid, dim3(512), lds, st, p, tiles_m, tiles_n);
+        hipLaunchKernelGGL(ks, grid, dim3(NT), lds, st, p, tiles_m, tiles_n);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
         hipLaunchKernelGGL(fp8x_splitk_reduce_kernel<RC>, splitk_rows_grid(batch * p.M, p.N), dim3(256), 0, st, p, batch * p.M, OUT_DT);
         return (int)hipGetLastError();
     }
-    auto k = qmm_fp8_exact_kernel<OUT_DT, RC, FMT, MXS>;
+    auto k = qmm_fp8_exact_kernel<WGM, WGN, OUT_DT, RC, FMT, MXS>;
     static std::atomic<uint64_t> attr_set{0};   // one bit per device: the attribute belongs to the (kernel, device) pair
     if (!device_flag_test(attr_set)) {
         hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return (int)e;
         device_flag_set(attr_set);
     }
-    hipLaunchKernelGGL(k, grid, dim3(512), lds, st, p, tiles_m, tiles_n);
+    hipLaunchKernelGGL(k, grid, dim3(NT), lds, st, p, tiles_m, tiles_n);
     return (int)hipGetLastError();
+}
+
+template <int OUT_DT, bool RC, int FMT = 0, bool MXS = false>
+static int launch_fp8_exact(const Fp8xParams& p, int64_t batch, int force_variant, hipStream_t st)
+{
+    int tile = p.splits > 1 ? p.tile : fp8x_plan(p.M, p.N, p.K, batch, RC && !MXS, false).tile;
+    if (force_variant >= OPSNN_VARIANT_FP8X_256x128 && force_variant <= OPSNN_VARIANT_FP8X_128x128) tile = force_variant;
+    if (256 * p.ldb >= (1ll << 32) || p.s2_cs < 0 || p.s2_cs >= (1ll << 29)) tile = OPSNN_VARIANT_FP8X_256x128;   // (32-bit offsets inside a tile)
+    if (tile == OPSNN_VARIANT_FP8X_128x128) return launch_fp8_exact_tile<2, 2, OUT_DT, RC, FMT, MXS>(p, batch, st);
+    if (tile == OPSNN_VARIANT_FP8X_128x256) return launch_fp8_exact_tile<2, 4, OUT_DT, RC, FMT, MXS>(p, batch, st);
+    return launch_fp8_exact_tile<4, 2, OUT_DT, RC, FMT, MXS>(p, batch, st);
 }
 
 // fp8 e4m3 block scales (G-B, B-B), K-contiguous operands, K % 128 == 0, 16-bit or fp32 output, no bias.
@@ -638,10 +682,10 @@ int launch_blockscale_exact(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
     // by 32-bit offsets from the tile's first row
     if (p.s1_rs < 0 || p.s1_cs < 0 || ((a.M + p.gsM - 1) / p.gsM) * p.s1_rs * 4 >= (1ll << 32)) return OPSNN_NOT_TAKEN;
     if (p.lda < 0 || p.ldb < 0 || 256 * p.lda >= (1ll << 32) || 128 * p.ldb >= (1ll << 32)) return OPSNN_NOT_TAKEN;
-    p.splits = sk.splits; p.part = sk.part;
-    if (a.out_dtype == DT_BF16) return launch_fp8_exact<DT_BF16, false>(p, a.batch, st);
-    if (a.out_dtype == DT_F32) return launch_fp8_exact<DT_F32, false>(p, a.batch, st);
-    return launch_fp8_exact<DT_F16, false>(p, a.batch, st);
+    p.splits = sk.splits; p.part = sk.part; p.tile = sk.splits > 1 ? fp8x_plan(a.M, a.N, a.K, a.batch, false, true).tile : 0;
+    if (a.out_dtype == DT_BF16) return launch_fp8_exact<DT_BF16, false>(p, a.batch, a.force_variant, st);
+    if (a.out_dtype == DT_F32) return launch_fp8_exact<DT_F32, false>(p, a.batch, a.force_variant, st);
+    return launch_fp8_exact<DT_F16, false>(p, a.batch, a.force_variant, st);
 }
 
 // fp8 (e4m3 or e5m2, each operand by itself) with scales applied to the finished sums: one fp32 scale per row of x1 (or
@@ -666,13 +710,13 @@ int launch_rowcol_exact(const OpsnnQmmArgs& a, hipStream_t st, int ep_mode, Spli
     p.ep_mode = ep_mode;
     p.bias = a.bias; p.bias_dt = a.bias_dtype; p.bias_bs = a.bias_batch_stride;
     if (((uintptr_t)p.a | (uintptr_t)p.b | (uint64_t)p.lda | (uint64_t)p.ldb | (uint64_t)p.a_bs | (uint64_t)p.b_bs) % 16) return OPSNN_NOT_TAKEN;
-    p.splits = sk.splits; p.part = sk.part;
+    p.splits = sk.splits; p.part = sk.part; p.tile = sk.splits > 1 ? fp8x_plan(a.M, a.N, a.K, a.batch, true, true).tile : 0;
     const bool bf = a.out_dtype == DT_BF16, f32 = a.out_dtype == DT_F32;
     switch ((e1 ? 1 : 0) | (e2 ? 2 : 0)) {
-        case 0: return f32 ? launch_fp8_exact<DT_F32, true, 0>(p, a.batch, st) : bf ? launch_fp8_exact<DT_BF16, true, 0>(p, a.batch, st) : launch_fp8_exact<DT_F16, true, 0>(p, a.batch, st);
-        case 1: return f32 ? launch_fp8_exact<DT_F32, true, 1>(p, a.batch, st) : bf ? launch_fp8_exact<DT_BF16, true, 1>(p, a.batch, st) : launch_fp8_exact<DT_F16, true, 1>(p, a.batch, st);
-        case 2: return f32 ? launch_fp8_exact<DT_F32, true, 2>(p, a.batch, st) : bf ? launch_fp8_exact<DT_BF16, true, 2>(p, a.batch, st) : launch_fp8_exact<DT_F16, true, 2>(p, a.batch, st);
-        default: return f32 ? launch_fp8_exact<DT_F32, true, 3>(p, a.batch, st) : bf ? launch_fp8_exact<DT_BF16, true, 3>(p, a.batch, st) : launch_fp8_exact<DT_F16, true, 3>(p, a.batch, st);
+        case 0: return f32 ? launch_fp8_exact<DT_F32, true, 0>(p, a.batch, a.force_variant, st) : bf ? launch_fp8_exact<DT_BF16, true, 0>(p, a.batch, a.force_variant, st) : launch_fp8_exact<DT_F16, true, 0>(p, a.batch, a.force_variant, st);
+        case 1: return f32 ? launch_fp8_exact<DT_F32, true, 1>(p, a.batch, a.force_variant, st) : bf ? launch_fp8_exact<DT_BF16, true, 1>(p, a.batch, a.force_variant, st) : launch_fp8_exact<DT_F16, true, 1>(p, a.batch, a.force_variant, st);
+        case 2: return f32 ? launch_fp8_exact<DT_F32, true, 2>(p, a.batch, a.force_variant, st) : bf ? launch_fp8_exact<DT_BF16, true, 2>(p, a.batch, a.force_variant, st) : launch_fp8_exact<DT_F16, true, 2>(p, a.batch, a.force_variant, st);
+        default: return f32 ? launch_fp8_exact<DT_F32, true, 3>(p, a.batch, a.force_variant, st) : bf ? launch_fp8_exact<DT_BF16, true, 3>(p, a.batch, a.force_variant, st) : launch_fp8_exact<DT_F16, true, 3>(p, a.batch, a.force_variant, st);
     }
 }
 
@@ -712,10 +756,10 @@ int launch_mx_exact(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
     if (((uintptr_t)p.a | (uintptr_t)p.b | (uint64_t)p.lda | (uint64_t)p.ldb | (uint64_t)p.a_bs | (uint64_t)p.b_bs) % 16) return OPSNN_NOT_TAKEN;
     if (((uintptr_t)p.sa | (uintptr_t)p.sb | (uint64_t)p.sa_rs | (uint64_t)p.sb_rs | (uint64_t)p.sa_bs | (uint64_t)p.sb_bs) % 4) return OPSNN_NOT_TAKEN;
     p.bias = a.bias; p.bias_dt = a.bias_dtype; p.bias_bs = a.bias_batch_stride;
-    p.splits = sk.splits; p.part = sk.part;
-    return a.out_dtype == DT_F32    ? launch_fp8_exact<DT_F32, true, 0, true>(p, a.batch, st)
-           : a.out_dtype == DT_BF16 ? launch_fp8_exact<DT_BF16, true, 0, true>(p, a.batch, st)
-                                    : launch_fp8_exact<DT_F16, true, 0, true>(p, a.batch, st);
+    p.splits = sk.splits; p.part = sk.part; p.tile = sk.splits > 1 ? fp8x_plan(a.M, a.N, a.K, a.batch, false, true).tile : 0;
+    return a.out_dtype == DT_F32    ? launch_fp8_exact<DT_F32, true, 0, true>(p, a.batch, a.force_variant, st)
+           : a.out_dtype == DT_BF16 ? launch_fp8_exact<DT_BF16, true, 0, true>(p, a.batch, a.force_variant, st)
+                                    : launch_fp8_exact<DT_F16, true, 0, true>(p, a.batch, a.force_variant, st);
 }
 
 }  // namespace opsnn

@@ -246,7 +246,7 @@ static uint64_t mx_rest_bytes(const OpsnnQmmArgs& a0)
 // re-laid-out and padded operand copies.
 uint64_t mxfp8_rows_workspace(const OpsnnQmmArgs& a);   // qmm_fp8_rows.hip
 int launch_mxfp8_rows(const OpsnnQmmArgs& a, void* region, hipStream_t st, SplitK sk);
-// (in front of that: the bf16 copy of x1 for MXFP8 with 33 .. 256 rows on the many-rows kernel)
+// (in front of that: the bf16 copy of x1 for MXFP8 with 17 .. 128 rows on the many-rows kernel)
 static uint64_t mx_rows_bytes(const OpsnnQmmArgs& a)
 {
     // (whether or not opsnnSetFp8Fast is on: a workspace must not depend on a switch that may change between the two phases)
@@ -322,7 +322,7 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         if (rc != 0) return rc;
     }
     if (a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E2M1) return launch_mx_a8w4_mfma(a, st, sk);   // fp8 x fp4: qmm_fp8_block.hip
-    if (fp8 && rows_region) {   // MXFP8 with 33 .. 256 rows: the many-rows streaming kernel on bf16 operands (exact products)
+    if (fp8 && rows_region) {   // MXFP8 with 17 .. 128 rows: the many-rows streaming kernel on bf16 operands (exact products)
         if (!opsnnGetFp8Fast()) {
             const int rc = launch_mxfp8_rows(a, rows_region, st, sk);
             if (rc != OPSNN_NOT_TAKEN) return rc;
