@@ -157,7 +157,7 @@ __device__ __forceinline__ float e8m0_to_f32(uint32_t b)
 // family), four neighbouring columns of one row per thread: emit(row, n0, cols, v) with cols = 4 except at the end of a
 // row.  The row comes from blockIdx.y and the columns from blockIdx.x, so no element costs a division (one 64-bit division is
 // several dozen instructions: with two or three of them per element the second kernel of a split took 106 us for 500 x 8192
-// outputs in two slices, where the 50 MB it moves are 10 us), and eight slices are in flight at a time.
+// outputs in two slices, where the 50 MB it moves are 10 us), and up to eight slices are in flight at a time.
 template <typename T, typename F>
 __device__ __forceinline__ void splitk_rows(const T* part, int splits, int64_t slice, int64_t rows, int64_t N, F&& emit)
 {
@@ -177,20 +177,22 @@ __device__ __forceinline__ void splitk_rows(const T* part, int splits, int64_t s
                 if (e < cols) r[e] = q[e];
             return r;
         };
-        quad v = load(0);
-        int s = 1;
-        for (; s + 7 < splits; s += 8) {
-            quad t[8];
+        const T z = (T)-0.0f;   // (-0.0f + v is v for every v)
+        quad v = {z, z, z, z};
+        int s = 0;
+        auto take = [&](auto nc) {
+            constexpr int n = decltype(nc)::value;
+            quad t[n];
 #pragma unroll
-            for (int j = 0; j < 8; j++) t[j] = load(s + j);
+            for (int j = 0; j < n; j++) t[j] = load(s + j);
 #pragma unroll
-            for (int j = 0; j < 8; j++) v = v + t[j];
-        }
-        for (; s + 1 < splits; s += 2) {
-            const quad t0 = load(s), t1 = load(s + 1);
-            v = v + t0; v = v + t1;
-        }
-        if (s < splits) v = v + load(s);
+            for (int j = 0; j < n; j++) v = v + t[j];
+            s += n;
+        };
+        while (s + 8 <= splits) take(std::integral_constant<int, 8>{});
+        if (s + 4 <= splits) take(std::integral_constant<int, 4>{});
+        if (s + 2 <= splits) take(std::integral_constant<int, 2>{});
+        if (s < splits) take(std::integral_constant<int, 1>{});
         emit(row, n0, cols, v);
     }
 }
