@@ -17,6 +17,7 @@
 #include "launch.h"
 #include "wqmm_stream.hip.h"
 
+extern "C" int opsnn_wq_narrow_slabs();   // dispatch.hip
 namespace opsnn {
 
 struct WqNkPlan {
@@ -248,7 +249,9 @@ bool wq_nk_wanted(const OpsnnWqmmArgs& a)
     if (a.M <= 16) return a.K % 128 != 0;
     // (17 .. 32 rows against a narrow N and a K that the many-rows kernel does not cut: there the streaming kernel's workgroups are
     // few -- 32 x 4096 x 4096 fp16 / bf16 17.1 / 21.1 us against 13.3 / 13.5 here; at N = 11008 it is 20 against 24)
-    if (a.M <= 32 && a.N <= 8192 && a.K < 8192) return true;
+    // (33 .. 64 rows: up to N = 5120 -- 64 x 4096 x 2048 20.0 -> 12.8 us, 64 x 7168 x 4096 29.2 -> 24.2, 64 x 4096 x 4096 20.2 -> 16.5;
+    // 40 x 4096 x 6144 19.3 against 19.6, 64 x 2048 x 8192 14.5 against 16.5, 40 x 14336 x 4096, cut along K there, 22.7 against 28.6)
+    if (opsnn_wq_narrow_slabs() && a.K < 8192 && a.N <= (a.M <= 32 ? 8192 : 5120)) return true;
     return a.N % 32 != 0 || a.K % (2 * kc) != 0;
 }
 uint64_t wq_nk_workspace(const OpsnnWqmmArgs& a)
