@@ -548,9 +548,7 @@ int launch_wq_mx8_rows(const WqParams& p0, hipStream_t st)
     WqParams p = p0;
     p.w_float = 1; p.scale_e8m0 = 1; p.mx8_rows = 1; p.group = 32; p.group_shift = 5; p.s_rs = 1; p.offset = nullptr;
     constexpr int64_t KC = 64;
-    if (p.M < 17 || p.K % (2 * KC) != 0 || p.N % 32 != 0 || p.N < 256 || p.K >= (1ll << 23)) return OPSNN_NOT_TAKEN;
-    const int64_t nslab = narrow_n_slab(p.M, p.N);
-    if ((p.K / KC) % 8 != 0 && (nslab ? nslab : p.M) > 128) return OPSNN_NOT_TAKEN;
+    if (p.M < 17 || p.M > 128 || p.K % (2 * KC) != 0 || p.N % 32 != 0 || p.N < 256 || p.K >= (1ll << 23)) return OPSNN_NOT_TAKEN;
     return launch_slabs_float<DT_BF16, 8>(p, st);
 }
 

@@ -1680,10 +1680,8 @@ int launch_wq_rows_float(const WqParams& p, hipStream_t st);
     int launch_wq_rows_float<XDT, WBITS>(const WqParams& p, hipStream_t st)                                         \
     {                                                                                                               \
         constexpr int WF = WBITS == 4 ? 2 : 1;                                                                      \
-        if constexpr (WBITS == 8) {   /* e4m3 codes with e8m0 scales per 32 (no 64-column instance) */                 \
+        if constexpr (WBITS == 8) {   /* e4m3 codes with e8m0 scales per 32, up to 128 rows (no 64-column instance) */ \
             if (p.scale_e8m0) {                                                                                     \
-                if (p.m_rows > 192) return launch_rows_one<XDT, WBITS, 16, 2, 4, 2, false, 2>(p, st);               \
-                if (p.m_rows > 128) return launch_rows_one<XDT, WBITS, 12, 2, 4, 2, false, 2>(p, st);               \
                 return p.m_rows > 64 ? launch_rows_one<XDT, WBITS, 8, 2, 4, 2, false, 2>(p, st)                     \
                                      : launch_rows_one<XDT, WBITS, 4, 2, 4, 2, false, 2>(p, st);                    \
             }                                                                                                       \
