@@ -162,7 +162,7 @@ template <typename T, typename F>
 __device__ __forceinline__ void splitk_rows(const T* part, int splits, int64_t slice, int64_t rows, int64_t N, F&& emit)
 {
     typedef T quad __attribute__((ext_vector_type(4)));
-    const int64_t n0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    const int64_t n0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
     if (n0 >= N) return;
     const int cols = N - n0 < 4 ? (int)(N - n0) : 4;
     const bool vec = (N % 4) == 0 && (slice % 4) == 0 && ((uintptr_t)part % 16) == 0;
@@ -196,9 +196,9 @@ __device__ __forceinline__ void splitk_rows(const T* part, int splits, int64_t s
         emit(row, n0, cols, v);
     }
 }
-inline dim3 splitk_rows_grid(int64_t rows, int64_t N)
+inline dim3 splitk_rows_grid(int64_t rows, int64_t N, int threads = 256)
 {
-    return dim3((unsigned)((N + 1023) / 1024), (unsigned)(rows < 65535 ? rows : 65535));
+    return dim3((unsigned)((N + 4 * threads - 1) / (4 * threads)), (unsigned)(rows < 65535 ? rows : 65535));
 }
 // cols (1 .. 4) neighbouring outputs of one row, rounded to out_dt (bf16, fp16 or fp32), at element `at` of out
 __device__ __forceinline__ void store_quad(void* out, int out_dt, int64_t at, int cols, v4f v)

@@ -1635,18 +1635,19 @@ static int launch_rows_one(const WqParams& p, hipStream_t st)
     hipLaunchKernelGGL(k, dim3(grid, (unsigned)slabs, split ? (unsigned)p.ksplit : 1u), dim3(512), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
     if (split) {
-        const dim3 rgrid = splitk_rows_grid(p.M, p.N);
+        constexpr int RT = 64;   // (few outputs: small workgroups deal them evenly over the CUs)
+        const dim3 rgrid = splitk_rows_grid(p.M, p.N, RT);
         if constexpr (WF == 3) {
-            hipLaunchKernelGGL(rows_bs_splitk_reduce_kernel<false>, rgrid, dim3(256), 0, st, (const float*)p.part, p.ksplit, p.M,
+            hipLaunchKernelGGL(rows_bs_splitk_reduce_kernel<false>, rgrid, dim3(RT), 0, st, (const float*)p.part, p.ksplit, p.M,
                                p.N, (const float*)nullptr, (int64_t)0, (const float*)nullptr, (int64_t)0, (const float*)nullptr, (void*)p.y, p.bs_out_dt);
             return (int)hipGetLastError();
         }
         if constexpr (WF == 4) {
-            hipLaunchKernelGGL(rows_bs_splitk_reduce_kernel<true>, rgrid, dim3(256), 0, st, (const float*)p.part, p.ksplit, p.M,
+            hipLaunchKernelGGL(rows_bs_splitk_reduce_kernel<true>, rgrid, dim3(RT), 0, st, (const float*)p.part, p.ksplit, p.M,
                                p.N, p.bs1, p.bs1_rs, p.bs2, p.bs2_cs, (const float*)p.bias, (void*)p.y, p.bs_out_dt);
             return (int)hipGetLastError();
         }
-        hipLaunchKernelGGL(wq_splitk_reduce_kernel, rgrid, dim3(256), 0, st, (const float*)p.part, p.ksplit, p.M, p.N, p.bias, p.bias_dt, (void*)p.y, XDT);
+        hipLaunchKernelGGL(wq_splitk_reduce_kernel, rgrid, dim3(RT), 0, st, (const float*)p.part, p.ksplit, p.M, p.N, p.bias, p.bias_dt, (void*)p.y, XDT);
         return (int)hipGetLastError();
     }
     return 0;
