@@ -508,7 +508,9 @@ extern "C" uint64_t opsnnWqmmWorkspace(const OpsnnWqmmArgs* a)
     uint64_t part = 0;
     if (const int xs = wq_part_slices((int)bits, a->M, a->N, a->K, a->group > 0 ? a->group : a->K, opsnn_wq_narrow_slabs() != 0); xs > 1 && a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain())
         part = ((uint64_t)xs * (uint64_t)a->M * (uint64_t)a->N * 4 + 255) / 256 * 256;
-    if (wq_nk_wanted(*a) && !opsnn_force_plain()) return wq_nk_workspace(*a);   // few rows, a shape outside the specialised kernels
+    // few rows, a shape outside the specialised kernels: the streaming kernel without shape conditions or, for a weight at an
+    // unaligned address, the kernels behind it (which of them is only known in phase 2)
+    if (wq_nk_wanted(*a) && !opsnn_force_plain()) { const uint64_t nk = wq_nk_workspace(*a); return nk > part ? nk : part; }
     if (a->w.row_stride == 1 || a->K == 1) return part;
     if (a->w.col_stride != 1 || a->w.row_stride != a->N) return part;
     const uint64_t relaid = part + (uint64_t)a->N * (uint64_t)a->K * bits / 8;

@@ -228,8 +228,10 @@ static int launch_nk_mb(const WqParams& p, const WqNkPlan& pl, hipStream_t st)
     return launch_nk_one<XDT, WBITS, 4, HAS_OFF>(p, pl, st);
 }
 
-// Does the call run here?  Looks at what phase 1 knows, so that both phases agree.  The specialised kernels keep what they take
-// (wqmm.hip): K in whole 128-element units, groups of whole chunks, and from 17 rows N % 32 == 0 and K in whole x slabs.
+// Does the call run here?  Looks at what both phases know: not at the weight's address, which for a FRACTAL_NZ weight is that of
+// its ND copy in phase 2 alone (launch_wq_nk declines an unaligned one; the workspace has room for either outcome).  The
+// specialised kernels keep what they take (wqmm.hip): K in whole 128-element units, groups of whole chunks, and from 17 rows
+// N % 32 == 0 and K in whole x slabs.
 bool wq_nk_wanted(const OpsnnWqmmArgs& a)
 {
     if ((a.w_dtype != DT_I4 && a.w_dtype != DT_I8) || (a.x_dtype != DT_F16 && a.x_dtype != DT_BF16)) return false;
@@ -238,7 +240,7 @@ bool wq_nk_wanted(const OpsnnWqmmArgs& a)
     if (a.w.row_stride != 1 || a.w.col_stride != a.K) return false;
     const int64_t group = a.group > 0 && a.group < a.K ? a.group : a.K;
     if (group < a.K && group % 32 != 0) return false;
-    if ((uintptr_t)a.x % 16 != 0 || (uintptr_t)a.w.ptr % 16 != 0) return false;
+    if ((uintptr_t)a.x % 16 != 0) return false;
     WqNkPlan pl;
     if (!nk_plan(a.w_dtype == DT_I4 ? 4 : 8, a.M, a.N, a.K, group, pl)) return false;
     if (a.force_variant != 0) return false;
@@ -262,7 +264,7 @@ uint64_t wq_nk_workspace(const OpsnnWqmmArgs& a)
 }
 int launch_wq_nk(const OpsnnWqmmArgs& a, hipStream_t st)
 {
-    if (!wq_nk_wanted(a)) return OPSNN_NOT_TAKEN;
+    if (!wq_nk_wanted(a) || (uintptr_t)a.w.ptr % 16 != 0) return OPSNN_NOT_TAKEN;
     const int wbits = a.w_dtype == DT_I4 ? 4 : 8;
     WqParams p{};
     p.group = a.group > 0 && a.group < a.K ? a.group : a.K;
