@@ -91,6 +91,7 @@ extern "C" aclnnStatus aclnnQuantMatmulWeightNzGetWorkspaceSize(const aclTensor*
     aclTensor nd = *x2;   // the same view over the dense ND matrix the pre-step will write
     nd.format = ACL_FORMAT_ND;
     nd.storage = nd.view;
+    if (nd.data) nd.data = nz_plan_address();
     uint64_t inner = 0;
     aclOpExecutor* ex = nullptr;
     const aclnnStatus rc = aclnnQuantMatmulV5GetWorkspaceSize(x1, &nd, x1Scale, x2Scale, yScale, x1Offset, x2Offset, yOffset, bias, transposeX1,

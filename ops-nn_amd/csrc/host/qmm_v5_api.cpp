@@ -499,6 +499,18 @@ OpsnnMat mat_of(const TView& t, bool transposed)
     return m;
 }
 
+// the mode number of opsnnQmmWorkspace
+int qmm_mode(OpKind k)
+{
+    switch (k) {
+        case OpKind::QmmBlockScale: return 1;
+        case OpKind::QmmMx: return 2;
+        case OpKind::QmmTc: return 3;
+        case OpKind::QmmGroup: return 4;
+        default: return 0;
+    }
+}
+
 }  // namespace
 
 extern "C" aclnnStatus aclnnQuantMatmulV5GetWorkspaceSize(const aclTensor* x1, const aclTensor* x2,
@@ -809,6 +821,10 @@ extern "C" aclnnStatus aclnnQuantMatmulV5(void* workspace, uint64_t workspaceSiz
         if (rc != 0) FAIL(ACLNN_ERR_RUNTIME_ERROR, "%s: FRACTAL_NZ re-layout failed with code %d", ex->api, rc);
         ex->qmm.x2.ptr = nd;
         ex->qmm.workspace = ex->workspace_size > front + nz_front_bytes(*ex) ? rest : nullptr;
+        // (phase 1 planned for an aligned copy.  In a workspace that is not aligned the plan may be another one: it runs if it
+        // fits, and without a workspace if not)
+        if ((uintptr_t)nd % 16 != 0 && opsnnQmmWorkspace(&ex->qmm, qmm_mode(ex->kind)) > ex->workspace_size - front - nz_front_bytes(*ex))
+            ex->qmm.workspace = nullptr;
     }
     auto launch = [&](const OpsnnQmmArgs& q) -> int {
         switch (ex->kind) {

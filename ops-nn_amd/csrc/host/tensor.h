@@ -111,6 +111,9 @@ void swap_last2(TView& v);
 // stored matrix is [.., rows, cols] (the view, or its last two dims swapped for a transposed view) and fills the step.
 // Returns false with the error text set.
 bool describe_nz_operand(const char* api, const char* name, const aclTensor* t, aclOpExecutorImpl::NzStep* step);
+// The address that phase 1 plans with for the ND copy: any aligned one, as the front of the workspace is.  (The launchers' plans
+// look at alignment; the NZ operand's own address says nothing about the copy's.)
+inline void* nz_plan_address() { return (void*)(uintptr_t)256; }
 // Phase 2 helper for executors with an NZ pre-step: runs it, returns the ND operand's address and the rest of the workspace.
 int run_nz_step(const aclOpExecutorImpl& ex, void* workspace, void* stream, const void** nd_ptr, void** rest);
 inline uint64_t nz_front_bytes(const aclOpExecutorImpl& ex) { return ex.nz.active ? (ex.nz.nd_bytes + 255) / 256 * 256 : 0; }

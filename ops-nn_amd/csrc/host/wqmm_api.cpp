@@ -282,6 +282,7 @@ aclnnStatus aclnnWeightQuantBatchMatmulNzGetWorkspaceSize(const aclTensor* x, co
     aclTensor nd = *weight;   // the same view over the dense ND matrix the pre-step will write
     nd.format = ACL_FORMAT_ND;
     nd.storage = nd.view;
+    if (nd.data) nd.data = nz_plan_address();
     uint64_t inner = 0;
     aclOpExecutor* ex = nullptr;
     const aclnnStatus rc = get_workspace(api, x, &nd, antiquantScale, antiquantOffsetOptional, quantScaleOptional, quantOffsetOptional,

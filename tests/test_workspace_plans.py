@@ -91,3 +91,99 @@ def test_nz_weight_at_an_unaligned_address_stays_inside_the_workspace(gpu, M, K,
     m.check(m.lib().aclrtSynchronizeDevice(), "sync")
     assert np.array_equal(d_y.to_host(np.uint16, (M, N)), want)
     assert (buf.to_host(np.uint8, (ws + guard,))[ws:] == 0xA5).all()
+
+
+def _v5_nz_call(mode, M, N, K, x2_ptr, nk):
+    """Phase 1 of aclnnQuantMatmulWeightNz: (status, workspace)."""
+    four = mode in ("mxfp4", "a8w4")
+    x1_dt, x2_dt = {"int8": (m.ACL_INT8, m.ACL_INT8), "mxfp4": (m.ACL_FLOAT4_E2M1,) * 2,
+                    "a8w4": (m.ACL_FLOAT8_E4M3FN, m.ACL_FLOAT4_E2M1)}.get(mode, (m.ACL_FLOAT8_E4M3FN,) * 2)
+    c0e, cols, rows = 32, K if nk else N, N if nk else K
+    x1 = m.Tensor((M, K), x1_dt, ALIGNED)
+    x2 = m.Tensor((K, N), x2_dt, x2_ptr, strides=(1, K) if nk else None, fmt=m.ACL_FORMAT_FRACTAL_NZ,
+                  storage_shape=(-(-cols // c0e), -(-rows // 16), 16, c0e))
+    out = m.Tensor((M, N), m.ACL_BF16, ALIGNED)
+    kw = {}
+    if mode in ("int8", "fp8_token"):
+        s1, s2 = m.Tensor((M,), m.ACL_FLOAT, ALIGNED), m.Tensor((N,), m.ACL_FLOAT, ALIGNED)
+    elif mode == "fp8_block":
+        KB, NB = -(-K // 128), -(-N // 128)
+        s1, s2 = m.Tensor((M, KB), m.ACL_FLOAT, ALIGNED), m.Tensor((KB, NB), m.ACL_FLOAT, ALIGNED, strides=(1, KB) if nk else None)
+        kw["group_size"] = (1 << 32) | (128 << 16) | 128
+    else:
+        KS = -(-K // 64)
+        s1 = m.Tensor((M, KS, 2), m.ACL_FLOAT8_E8M0, ALIGNED)
+        s2 = m.Tensor((KS, N, 2), m.ACL_FLOAT8_E8M0, ALIGNED, strides=(2, KS * 2, 1) if nk else None)
+        kw["group_size"] = (1 << 32) | (1 << 16) | 32
+    rc, ws, ex = m.quant_matmul_v5_get_workspace(x1, x2, s1, s2, out, weight_nz=True, **kw)
+    if ex:
+        m.lib().aclDestroyAclOpExecutor(ex)
+    return rc, ws
+
+
+@pytest.mark.parametrize("mode", ["int8", "fp8_token", "fp8_block", "mxfp4", "mxfp8", "a8w4"])
+def test_quant_matmul_nz_plan_does_not_depend_on_the_nz_address(mode):
+    """(MXFP4 with K % 128 == 64 and a K split: the padded copies were planned only for an aligned NZ address, and written in
+    phase 2, where the ND copy is aligned, all the same.)"""
+    rng = random.Random(9)
+    taken = 0
+    for i in range(300):
+        M, N, K = rng.choice([1, 16, 20, 33, 64, 128, 300]), rng.randrange(16, 600) * 16, rng.randrange(8, 160) * 64
+        if i == 0:
+            M, N, K = 64, 1024, 8256
+        nk = rng.random() < 0.7
+        rc, want = _v5_nz_call(mode, M, N, K, ALIGNED, nk)
+        if rc != 0:
+            continue
+        taken += 1
+        for ptr in (ODD, ALIGNED + 8):
+            assert _v5_nz_call(mode, M, N, K, ptr, nk) == (0, want), (M, N, K, nk, ptr)
+    assert taken > 50, m.err_msg()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("mode,M,K,N", [("mxfp4", 64, 8256, 1024), ("int8", 64, 8192, 512), ("int8", 64, 8192, 500)])
+@pytest.mark.parametrize("x2_off,ws_off", [(4, 0), (0, 4), (8, 8)])
+def test_quant_matmul_nz_stays_inside_the_workspace(gpu, mode, M, K, N, x2_off, ws_off):
+    """NZ operands and workspaces at addresses that are not 16-byte aligned."""
+    import numpy as np
+
+    import cases
+    import oracle_api as orc
+    from test_gpu_shape_sweep import _b16_bar
+    from test_nz_entry_points import nd_to_nz
+    if mode == "int8":
+        inp = cases.make_qmm_int8_inputs(m, M, K, N, 3, m.ACL_BF16, True)
+        want, dt, c0 = cases.run_qmm_int8_aclnn(m, inp, M, K, N, True, m.ACL_BF16)[0], m.ACL_INT8, 32
+        nz = nd_to_nz(inp["x2"][0].view(np.uint8), c0)
+    else:
+        inp = cases.make_mx_inputs(m, M, K, N, 3, True, True)
+        want, dt, c0 = cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_BF16)[0], m.ACL_FLOAT4_E2M1, 16
+        nz = nd_to_nz(inp["x2"][0].view(np.uint8).reshape(N, K // 2), c0)
+    d = {k: m.DeviceBuffer(host=v) for k, v in inp.items() if isinstance(v, np.ndarray) and k != "x2"}
+    d_x2 = m.DeviceBuffer(host=np.concatenate([np.zeros(x2_off, np.uint8), nz.reshape(-1)]))
+    d_out = m.DeviceBuffer(M * N * 2)
+    x1 = m.Tensor((M, K), dt, d["x1"])
+    x2 = m.Tensor((N, K), dt, d_x2.ptr + x2_off, fmt=m.ACL_FORMAT_FRACTAL_NZ, storage_shape=nz.shape[:2] + (16, 32))
+    kw = {}
+    if mode == "int8":
+        s1, s2 = m.Tensor((M,), m.ACL_FLOAT, d["s1"]), m.Tensor((N,), m.ACL_FLOAT, d["s2"])
+        kw["bias"] = m.Tensor((N,), m.ACL_BF16, d["bias"])
+    else:
+        s1, s2 = m.Tensor(inp["s1"].shape[1:], m.ACL_FLOAT8_E8M0, d["s1"]), m.Tensor(inp["s2"].shape[1:], m.ACL_FLOAT8_E8M0, d["s2"])
+        kw["group_size"] = (1 << 32) | (1 << 16) | 32
+    rc, ws, ex = m.quant_matmul_v5_get_workspace(x1, x2, s1, s2, m.Tensor((M, N), m.ACL_BF16, d_out), transpose_x2=True, weight_nz=True, **kw)
+    assert rc == 0, m.err_msg()
+    guard = (M + N) * K + 4096   # (more than padded copies of both operands would take)
+    buf = m.DeviceBuffer(ws_off + ws + guard)
+    buf.fill(0xA5)
+    print(f"case nz {mode} M={M} K={K} N={N} x2 +{x2_off} workspace +{ws_off}", flush=True)
+    m.check(m.lib().aclnnQuantMatmulWeightNz(buf.ptr + ws_off, ws, ex, None), "aclnnQuantMatmulWeightNz")
+    m.check(m.lib().aclrtSynchronizeDevice(), "sync")
+    got = d_out.to_host(np.uint16, (M, N))
+    if mode == "int8":
+        assert np.array_equal(got, want)
+    else:
+        _b16_bar(got, want, orc.BF16, "mxfp4 nz", K)
+    after = buf.to_host(np.uint8, (ws_off + ws + guard,))
+    assert (after[:ws_off] == 0xA5).all() and (after[ws_off + ws:] == 0xA5).all()
