@@ -501,13 +501,15 @@ static uint64_t qmm_workspace_base(const OpsnnQmmArgs* a, int mode)
 extern "C" uint64_t opsnnWqmmWorkspace(const OpsnnWqmmArgs* a)
 {
     if (!a || a->M <= 0 || a->N <= 0 || a->K <= 0) return 0;
-    if (wq_dense_wanted(*a)) return wq_dense_workspace(*a);   // many rows: the dequantised weight (and partial sums)
     const uint64_t bits = (a->w_dtype == DT_I4 || a->w_dtype == DT_E2M1) ? 4 : 8;
     // up to 16 rows against a long K: fp32 partial sums of the x-in-registers kernel's K split, in front of everything else
     // (from 17 rows against a narrow N and a long K: those of the many-rows kernel's K split)
     uint64_t part = 0;
     if (const int xs = wq_part_slices((int)bits, a->M, a->N, a->K, a->group > 0 ? a->group : a->K, opsnn_wq_narrow_slabs() != 0); xs > 1 && a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain())
         part = ((uint64_t)xs * (uint64_t)a->M * (uint64_t)a->N * 4 + 255) / 256 * 256;
+    // many rows: the dequantised weight (and partial sums); [K, N] storage with the weight cache on: the K split of the cached copy's
+    // kernel (whether it is on is only known in phase 2)
+    if (wq_dense_wanted(*a)) { const uint64_t dense = wq_dense_workspace(*a); return dense > part ? dense : part; }
     // few rows, a shape outside the specialised kernels: the streaming kernel without shape conditions or, for a weight at an
     // unaligned address, the kernels behind it (which of them is only known in phase 2)
     if (wq_nk_wanted(*a) && !opsnn_force_plain()) { const uint64_t nk = wq_nk_workspace(*a); return nk > part ? nk : part; }

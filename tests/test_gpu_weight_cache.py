@@ -272,3 +272,29 @@ def test_static_entry_point_leaves_the_cache_alone(cache):
     assert _stats(m) == before, (before, _stats(m))
     want, _ = cases.oracle_qmm_int8(m, inp, M, K, N, False, m.ACL_BF16)
     assert np.array_equal(out.to_host(np.uint16, (M, N)), want[0])
+
+
+@pytest.mark.parametrize("M,K,N", [(100, 1024, 512), (128, 16384, 512)])
+def test_many_rows_use_the_cached_copy(cache, M, K, N):
+    """65 rows and more against [K, N] storage: with the cache on, a call whose K-contiguous form runs on the streaming kernel
+    (the second shape with K in segments) runs there on the cached copy; the bits are those of the pre-packed weight."""
+    m = cache
+    print(f"case weight cache, many rows, weight-only int4 {M}x{K}x{N}", flush=True)
+    inp = cases.make_wq_inputs(m, M, K, N, 3, m.ACL_FLOAT16, m.ACL_INT4, 128, False, True, None)
+    d = {k: m.DeviceBuffer(host=v) for k, v in inp.items() if isinstance(v, np.ndarray)}
+    d_y = m.DeviceBuffer(M * N * 2)
+    e0, _, h0, m0 = _stats(m)
+    first = _wq_call(m, inp, d, d_y, M, K, N)
+    second = _wq_call(m, inp, d, d_y, M, K, N)
+    e1, _, h1, m1 = _stats(m)
+    assert (e1 - e0, m1 - m0, h1 - h0) == (1, 1, 1)
+    w = orc.unpack_nibbles(inp["w"]).reshape(K, N).T & 15
+    packed = dict(inp, w=np.ascontiguousarray((w[:, 0::2] | (w[:, 1::2] << 4)).astype(np.uint8)), tW=True,
+                  scale=np.ascontiguousarray(inp["scale"].T), offset=np.ascontiguousarray(inp["offset"].T))
+    assert np.array_equal(first, cases.run_wq_aclnn(m, packed, M, K, N)) and np.array_equal(first, second)
+    # the cache too small for this weight: the dequantising route, no entry
+    m.lib().opsnnSetWeightCache(1024)
+    third = _wq_call(m, inp, d, d_y, M, K, N)
+    assert _stats(m)[0] == 0
+    mx, mean = orc.rel_err_stats(orc.b16_to_f32(third, orc.F16), orc.b16_to_f32(first, orc.F16))
+    assert mx <= 2.0 ** -7 and mean <= 2.0 ** -10

@@ -187,3 +187,12 @@ def test_quant_matmul_nz_stays_inside_the_workspace(gpu, mode, M, K, N, x2_off, 
         _b16_bar(got, want, orc.BF16, "mxfp4 nz", K)
     after = buf.to_host(np.uint8, (ws_off + ws + guard,))
     assert (after[:ws_off] == 0xA5).all() and (after[ws_off + ws:] == 0xA5).all()
+
+
+def test_kn_storage_leaves_room_for_the_cached_copys_k_split():
+    """[K, N] storage with more than 64 rows: whether the weight cache serves the call is only known in phase 2, so the workspace
+    holds what the K-contiguous form asks for as well."""
+    for M, N, K, group, wbits in _wq_shapes(400):
+        M, N = M + 64, N + N % 2
+        nk = m.lib().opsnnWqmmWorkspace(C.byref(_wq_args(M, N, K, group, wbits, m.ACL_FLOAT16, ALIGNED, True)))
+        assert m.lib().opsnnWqmmWorkspace(C.byref(_wq_args(M, N, K, group, wbits, m.ACL_FLOAT16, ALIGNED, False))) >= nk, (M, N, K, group, wbits)
