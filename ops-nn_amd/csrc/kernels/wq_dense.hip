@@ -162,7 +162,7 @@ int launch_wq_dense(const OpsnnWqmmArgs& a, hipStream_t st)
     const bool kn = a.w.row_stride != 1;
     if (kn && weight_cache_on()) {
         // a caller who keeps K-contiguous copies in the weight cache: where that form runs on the streaming kernel, so does the
-        // copy (128 x 8192 x 28672 int4: 105 us, 222 with the pass here); phase 1 has left room for its partial sums
+        // copy (128 x 8192 x 28672 int4: 75 us, 329 with the pass here); phase 1 has left room for its partial sums
         OpsnnWqmmArgs b = a;
         b.w.row_stride = 1; b.w.col_stride = a.K;
         if (!wq_dense_wanted(b) && (b.w.ptr = weight_cache_get(a.w.ptr, a.K, a.N, wbits, 1, st)) != nullptr) {
