@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 namespace opsnn {
 
@@ -154,70 +155,64 @@ __device__ __forceinline__ float e8m0_to_f32(uint32_t b)
 }
 
 // The sum, in split order, of `splits` partial arrays [rows][N] that lie `slice` elements apart (the K split of every kernel
-// family), four neighbouring columns of one row per thread: emit(row, n0, cols, v) with cols = 4 except at the end of a
-// row.  The row comes from blockIdx.y and the columns from blockIdx.x, so no element costs a division (one 64-bit division is
-// several dozen instructions: with two or three of them per element the second kernel of a split took 106 us for 500 x 8192
-// outputs in two slices, where the 50 MB it moves are 10 us), and up to eight slices are in flight at a time.
-template <typename T, typename F>
+// family), W neighbouring columns of one row per thread: emit(row, n0, v) with v[W].  W = 4 wants N % 4 == 0.  The row comes
+// from blockIdx.y and the columns from blockIdx.x, so no element costs a division (one 64-bit division is several dozen
+// instructions: with two or three of them per element the second kernel of a split took 106 us for 500 x 8192 outputs in two
+// slices, where the 50 MB it moves are 10 us), and up to eight slices are in flight at a time.
+template <int W, typename T, typename F>
 __device__ __forceinline__ void splitk_rows(const T* part, int splits, int64_t slice, int64_t rows, int64_t N, F&& emit)
 {
-    typedef T quad __attribute__((ext_vector_type(4)));
-    const int64_t n0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
+    const int64_t n0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * W;
     if (n0 >= N) return;
-    const int cols = N - n0 < 4 ? (int)(N - n0) : 4;
-    const bool vec = (N % 4) == 0 && (slice % 4) == 0 && ((uintptr_t)part % 16) == 0;
     for (int64_t row = blockIdx.y; row < rows; row += gridDim.y) {
         const T* at = part + row * N + n0;
-        auto load = [&](int s) -> quad {
-            const T* q = at + (int64_t)s * slice;
-            if (vec) return *(const quad*)q;
-            quad r = {0, 0, 0, 0};
+        T v[W];
 #pragma unroll
-            for (int e = 0; e < 4; e++)
-                if (e < cols) r[e] = q[e];
-            return r;
-        };
-        const T z = (T)-0.0f;   // (-0.0f + v is v for every v)
-        quad v = {z, z, z, z};
+        for (int e = 0; e < W; e++) v[e] = (T)-0.0f;   // (-0.0f + v is v for every v)
         int s = 0;
         auto take = [&](auto nc) {
             constexpr int n = decltype(nc)::value;
-            quad t[n];
+            T t[n][W];
 #pragma unroll
-            for (int j = 0; j < n; j++) t[j] = load(s + j);
+            for (int j = 0; j < n; j++) __builtin_memcpy(t[j], at + (int64_t)(s + j) * slice, sizeof(t[j]));
 #pragma unroll
-            for (int j = 0; j < n; j++) v = v + t[j];
+            for (int j = 0; j < n; j++)
+#pragma unroll
+                for (int e = 0; e < W; e++) v[e] = v[e] + t[j][e];
             s += n;
         };
         while (s + 8 <= splits) take(std::integral_constant<int, 8>{});
         if (s + 4 <= splits) take(std::integral_constant<int, 4>{});
         if (s + 2 <= splits) take(std::integral_constant<int, 2>{});
         if (s < splits) take(std::integral_constant<int, 1>{});
-        emit(row, n0, cols, v);
+        emit(row, n0, v);
     }
 }
-inline dim3 splitk_rows_grid(int64_t rows, int64_t N, int threads = 256)
+// Launches such a kernel: launch(W, grid, block).  Few outputs are a matter of latency, not of bytes: one column per thread
+// makes four times the waves (5 x 14464 x 1568 bf16 x int4, four slices: 12.4 us a call with four columns, 11.2 with one;
+// 16 x 4992 x 5248 fp8 14.6 / 14.1; 46 x 9856 x 4424 int8 18.0 / 17.2), and so it stays for an N that is no multiple of four
+// (13 x 1792 x 7273 11.3 / 10.3).  From 2^18 outputs the bytes count and four columns are ahead (64 x 4096 outputs 24.2 / 24.4,
+// 64 x 7168 50.4 / 51.0, 500 x 8192 77.3 / 88.4).
+template <typename L>
+inline void splitk_launch(int64_t rows, int64_t N, L&& launch)
 {
-    return dim3((unsigned)((N + 4 * threads - 1) / (4 * threads)), (unsigned)(rows < 65535 ? rows : 65535));
+    const dim3 block(256);
+    const unsigned gy = (unsigned)(rows < 65535 ? rows : 65535);
+    if (N % 4 == 0 && rows * N >= (1 << 18)) launch(std::integral_constant<int, 4>{}, dim3((unsigned)((N + 1023) / 1024), gy), block);
+    else launch(std::integral_constant<int, 1>{}, dim3((unsigned)((N + 255) / 256), gy), block);
 }
-// cols (1 .. 4) neighbouring outputs of one row, rounded to out_dt (bf16, fp16 or fp32), at element `at` of out
-__device__ __forceinline__ void store_quad(void* out, int out_dt, int64_t at, int cols, v4f v)
+// W neighbouring outputs of one row, rounded to out_dt (bf16, fp16 or fp32), at element `at` of out
+template <int W>
+__device__ __forceinline__ void store_cols(void* out, int out_dt, int64_t at, const float (&v)[W])
 {
     if (out_dt == DT_F32) {
-        float* o = (float*)out + at;
-        if (cols == 4 && ((uintptr_t)o % 16) == 0) { *(v4f*)o = v; return; }
-#pragma unroll
-        for (int e = 0; e < 4; e++)
-            if (e < cols) o[e] = v[e];
+        __builtin_memcpy((float*)out + at, v, sizeof(v));
         return;
     }
-    const v4us q = out_dt == DT_BF16 ? (v4us){bf16_bits(v[0]), bf16_bits(v[1]), bf16_bits(v[2]), bf16_bits(v[3])}
-                                     : (v4us){f16_bits(v[0]), f16_bits(v[1]), f16_bits(v[2]), f16_bits(v[3])};
-    uint16_t* o = (uint16_t*)out + at;
-    if (cols == 4 && ((uintptr_t)o % 8) == 0) { *(v4us*)o = q; return; }
+    uint16_t o[W];
 #pragma unroll
-    for (int e = 0; e < 4; e++)
-        if (e < cols) o[e] = q[e];
+    for (int e = 0; e < W; e++) o[e] = out_dt == DT_BF16 ? bf16_bits(v[e]) : f16_bits(v[e]);
+    __builtin_memcpy((uint16_t*)out + at, o, sizeof(o));
 }
 
 // Decode element i of a dense buffer of 8-bit or 4-bit quantised values.

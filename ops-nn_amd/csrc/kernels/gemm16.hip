@@ -10,19 +10,20 @@ namespace opsnn {
 int launch_16_wide(const QgemmParams& p, int fn, bool bf16_operands, int64_t batch, int out_dt, hipStream_t st);   // qmm_int8_wide.hip
 
 // out[b, m, n] = rounded(sum over the splits, in split order, * x2s[n] * x1s[m] + bias[n])
+template <int W>
 __global__ __launch_bounds__(256) void gemm16_splitk_reduce_kernel(QgemmParams p, int64_t rows, int out_dt)
 {
-    splitk_rows((const float*)p.part, p.splits, rows * p.N, rows, p.N, [&](int64_t row, int64_t n0, int cols, v4f v) {
+    splitk_rows<W>((const float*)p.part, p.splits, rows * p.N, rows, p.N, [&](int64_t row, int64_t n0, float (&v)[W]) {
         const int64_t bz = rows == p.M ? 0 : row / p.M, m = row - bz * p.M;
         const float s1 = p.x1s ? p.x1s[p.x1s_one ? 0 : m] : 1.0f;
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int64_t n = n0 + (e < cols ? e : cols - 1);
+        for (int e = 0; e < W; e++) {
+            const int64_t n = n0 + e;
             if (p.x2s) v[e] = v[e] * load_scalar_as_f32(p.x2s, p.x2s_dt, p.x2s_len == 1 ? 0 : n);
             v[e] = v[e] * s1;
             if (p.bias) v[e] = v[e] + load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + n);
         }
-        store_quad(p.out, out_dt, row * p.ldc + n0, cols, v);
+        store_cols(p.out, out_dt, row * p.ldc + n0, v);
     });
 }
 
@@ -44,7 +45,7 @@ static int launch_split16(const QgemmParams& p, int64_t batch, int out_dt, hipSt
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     const int64_t rows = batch * p.M;
-    hipLaunchKernelGGL(gemm16_splitk_reduce_kernel, splitk_rows_grid(rows, p.N), dim3(256), 0, st, p, rows, out_dt);
+    splitk_launch(rows, p.N, [&](auto w, dim3 g, dim3 b) { hipLaunchKernelGGL(gemm16_splitk_reduce_kernel<decltype(w)::value>, g, b, 0, st, p, rows, out_dt); });
     return (int)hipGetLastError();
 }
 

@@ -719,16 +719,17 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
 
 // MODE_I8 after a K split: out[b, m, n] = rounded(fp32(sum of the partial sums + ib[n]) * x2s[n] * x1s[m] + fb[n]), the
 // terms as the tile kernel's epilogue stages them
+template <int W>
 static __global__ __launch_bounds__(256) void qg_i8_splitk_reduce_kernel(QgemmParams p, int64_t rows, int out_dt)
 {
     const bool has_ib = p.bias && p.bias_dt == DT_I32, has_fb = p.bias && p.bias_dt != DT_I32;
-    splitk_rows(p.part, p.splits, rows * p.N, rows, p.N, [&](int64_t row, int64_t n0, int cols, v4i a) {
+    splitk_rows<W>((const int32_t*)p.part, p.splits, rows * p.N, rows, p.N, [&](int64_t row, int64_t n0, int32_t (&a)[W]) {
         const int64_t bz = rows == p.M ? 0 : row / p.M, m = row - bz * p.M;
         const float s1 = p.x1s ? p.x1s[m] : 1.0f;
-        v4f v;
+        float v[W];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int64_t n = n0 + (e < cols ? e : cols - 1), si = p.x2s_len == 1 ? 0 : n;
+        for (int e = 0; e < W; e++) {
+            const int64_t n = n0 + e, si = p.x2s_len == 1 ? 0 : n;
             float sv = p.x2s_dt == DT_U64 ? u2f((uint32_t)((const uint64_t*)p.x2s)[si]) : load_scalar_as_f32(p.x2s, p.x2s_dt, si);
             if (p.x2s_trunc || p.x2s_dt == DT_U64) sv = u2f(f2u(sv) & 0xFFFFE000u);
             const int32_t ib = has_ib ? ((const int32_t*)p.bias)[bz * p.bias_bs + n] : 0;
@@ -738,20 +739,21 @@ static __global__ __launch_bounds__(256) void qg_i8_splitk_reduce_kernel(QgemmPa
             tv = tv * s1;
             v[e] = tv + fb;
         }
-        store_quad(p.out, out_dt, row * p.ldc + n0, cols, v);
+        store_cols(p.out, out_dt, row * p.ldc + n0, v);
     });
 }
 
 // The MX modes after a K split: out[b, m, n] = rounded(sum of the fp32 partial sums, in split order, + bias[n])
+template <int W>
 static __global__ __launch_bounds__(256) void qg_mx_splitk_reduce_kernel(QgemmParams p, int64_t rows, int out_dt)
 {
-    splitk_rows((const float*)p.part, p.splits, rows * p.N, rows, p.N, [&](int64_t row, int64_t n0, int cols, v4f v) {
+    splitk_rows<W>((const float*)p.part, p.splits, rows * p.N, rows, p.N, [&](int64_t row, int64_t n0, float (&v)[W]) {
         const int64_t bz = rows == p.M ? 0 : row / p.M;
         if (p.bias) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) v[e] = v[e] + load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + n0 + (e < cols ? e : cols - 1));
+            for (int e = 0; e < W; e++) v[e] = v[e] + load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + n0 + e);
         }
-        store_quad(p.out, out_dt, row * p.ldc + n0, cols, v);
+        store_cols(p.out, out_dt, row * p.ldc + n0, v);
     });
 }
 
@@ -777,7 +779,7 @@ static int qgemm_launch_split_mx(const QgemmParams& p, int64_t batch, int out_dt
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
     if (out_dt != DT_BF16 && out_dt != DT_F16 && out_dt != DT_F32) return -2;
-    hipLaunchKernelGGL(qg_mx_splitk_reduce_kernel, splitk_rows_grid(batch * p.M, p.N), dim3(256), 0, st, p, batch * p.M, out_dt);
+    splitk_launch(batch * p.M, p.N, [&](auto w, dim3 g, dim3 b) { hipLaunchKernelGGL(qg_mx_splitk_reduce_kernel<decltype(w)::value>, g, b, 0, st, p, batch * p.M, out_dt); });
     return (int)hipGetLastError();
 }
 
@@ -800,7 +802,7 @@ static int qgemm_launch_split_i8(const QgemmParams& p, int64_t batch, int out_dt
     hipLaunchKernelGGL(k, grid, dim3(WGM * WGN * 64), lds, st, p, tiles_m, tiles_n);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL(qg_i8_splitk_reduce_kernel, splitk_rows_grid(batch * p.M, p.N), dim3(256), 0, st, p, batch * p.M, out_dt);
+    splitk_launch(batch * p.M, p.N, [&](auto w, dim3 g, dim3 b) { hipLaunchKernelGGL(qg_i8_splitk_reduce_kernel<decltype(w)::value>, g, b, 0, st, p, batch * p.M, out_dt); });
     return (int)hipGetLastError();
 }
 

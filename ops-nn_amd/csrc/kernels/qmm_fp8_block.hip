@@ -489,16 +489,17 @@ __global__ __launch_bounds__(WGM * 128, 1) void qmm_fp8_block_kernel(Fp8BlkParam
 }
 
 // out[b, m, n] = rounded(sum over the splits, in split order, of part[s, b, m, n] + bias[b, n])
+template <int W>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* part, int splits, int64_t rows, int64_t M, int64_t N,
                                                             const void* bias, int bias_dt, int64_t bias_bs, void* out, int out_dt)
 {
-    splitk_rows(part, splits, rows * N, rows, N, [&](int64_t row, int64_t n0, int cols, v4f v) {
+    splitk_rows<W>(part, splits, rows * N, rows, N, [&](int64_t row, int64_t n0, float (&v)[W]) {
         const int64_t bz = rows == M ? 0 : row / M;
         if (bias) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) v[e] = v[e] + load_scalar_as_f32(bias, bias_dt, bz * bias_bs + n0 + (e < cols ? e : cols - 1));
+            for (int e = 0; e < W; e++) v[e] = v[e] + load_scalar_as_f32(bias, bias_dt, bz * bias_bs + n0 + e);
         }
-        store_quad(out, out_dt, row * N + n0, cols, v);
+        store_cols(out, out_dt, row * N + n0, v);
     });
 }
 
@@ -523,8 +524,10 @@ static int launch_fp8_block(const Fp8BlkParams& p, int64_t batch, hipStream_t st
             hipLaunchKernelGGL(ks, grid, dim3(WGM * 128), lds, st, p, tiles_m, tiles_n);
             hipError_t e = hipGetLastError();
             if (e != hipSuccess) return (int)e;
-            hipLaunchKernelGGL(splitk_reduce_kernel, splitk_rows_grid(batch * p.M, p.N), dim3(256), 0, st, (const float*)p.part, p.splits, batch * p.M,
-                               p.M, p.N, (const void*)p.bias, MODE == FP8_MX_W4 ? p.bias_dt : DT_F32, p.bias_bs, p.out, OUT_DT);
+            splitk_launch(batch * p.M, p.N, [&](auto w, dim3 g, dim3 b) {
+                hipLaunchKernelGGL(splitk_reduce_kernel<decltype(w)::value>, g, b, 0, st, (const float*)p.part, p.splits, batch * p.M, p.M, p.N,
+                                   (const void*)p.bias, MODE == FP8_MX_W4 ? p.bias_dt : DT_F32, p.bias_bs, p.out, OUT_DT);
+            });
             return (int)hipGetLastError();
         }
     }

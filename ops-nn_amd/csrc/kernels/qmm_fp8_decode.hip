@@ -207,17 +207,17 @@ __global__ __launch_bounds__(NW * 64) void fp8_block_decode_kernel(Fp8DecParams 
 
 // out = epilogue(sum over the K segments, in order, of part[s]) for one pass of up to 16 rows: the block-scale form adds the
 // bias, the row / column scale form (RC) computes (sum * x2Scale[n]) * x1Scale[m] + bias[n]
-template <bool RC>
+template <int W, bool RC>
 __global__ __launch_bounds__(256) void fp8dec_reduce_kernel(Fp8DecParams p, int splits)
 {
-    splitk_rows((const float*)p.part, splits, p.part_slice, p.M, p.N, [&](int64_t m, int64_t n0, int cols, v4f v) {
+    splitk_rows<W>((const float*)p.part, splits, p.part_slice, p.M, p.N, [&](int64_t m, int64_t n0, float (&v)[W]) {
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int64_t n = n0 + (e < cols ? e : cols - 1);
+        for (int e = 0; e < W; e++) {
+            const int64_t n = n0 + e;
             if constexpr (RC) v[e] = (v[e] * p.cs[n * p.cs_stride]) * p.rs[m * p.rs_stride];
             if (p.bias) v[e] = v[e] + p.bias[n];
         }
-        store_quad(p.out, p.out_dt, m * p.N + n0, cols, v);
+        store_cols(p.out, p.out_dt, m * p.N + n0, v);
     });
 }
 
@@ -235,7 +235,7 @@ int launch_decode_one(const Fp8DecParams& p, hipStream_t st, int splits = 1)
     const size_t lds = (size_t)2 * NW * 256 * sizeof(float);
     hipLaunchKernelGGL((fp8_block_decode_kernel<NW, NBLK, RC, I8, SEG>), dim3((unsigned)grid, (unsigned)splits), dim3(NW * 64), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
-    hipLaunchKernelGGL(fp8dec_reduce_kernel<RC>, splitk_rows_grid(p.M, p.N), dim3(256), 0, st, p, splits);
+    splitk_launch(p.M, p.N, [&](auto w, dim3 g, dim3 b) { hipLaunchKernelGGL((fp8dec_reduce_kernel<decltype(w)::value, RC>), g, b, 0, st, p, splits); });
     return (int)hipGetLastError();
 }
 
@@ -398,14 +398,15 @@ __global__ __launch_bounds__(NW * 64) void mx_a8w4_decode_kernel(MxW4DecParams p
 }
 
 // out = cast(sum over the K segments, in order, of part[s] + bias) for one pass of up to 16 rows
+template <int W>
 __global__ __launch_bounds__(256) void mxw4dec_reduce_kernel(MxW4DecParams p, int splits)
 {
-    splitk_rows((const float*)p.part, splits, p.part_slice, p.M, p.N, [&](int64_t m, int64_t n0, int cols, v4f v) {
+    splitk_rows<W>((const float*)p.part, splits, p.part_slice, p.M, p.N, [&](int64_t m, int64_t n0, float (&v)[W]) {
         if (p.bias) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) v[e] = v[e] + load_scalar_as_f32(p.bias, p.bias_dt, n0 + (e < cols ? e : cols - 1));
+            for (int e = 0; e < W; e++) v[e] = v[e] + load_scalar_as_f32(p.bias, p.bias_dt, n0 + e);
         }
-        store_quad(p.out, p.out_dt, m * p.N + n0, cols, v);
+        store_cols(p.out, p.out_dt, m * p.N + n0, v);
     });
 }
 
@@ -423,7 +424,7 @@ int launch_mxw4_one(const MxW4DecParams& p, hipStream_t st, int splits = 1)
     const size_t lds = (size_t)2 * NW * 256 * sizeof(float);
     hipLaunchKernelGGL((mx_a8w4_decode_kernel<NW, NCH, SEG>), dim3((unsigned)grid, (unsigned)splits), dim3(NW * 64), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
-    hipLaunchKernelGGL(mxw4dec_reduce_kernel, splitk_rows_grid(p.M, p.N), dim3(256), 0, st, p, splits);
+    splitk_launch(p.M, p.N, [&](auto w, dim3 g, dim3 b) { hipLaunchKernelGGL(mxw4dec_reduce_kernel<decltype(w)::value>, g, b, 0, st, p, splits); });
     return (int)hipGetLastError();
 }
 
@@ -574,14 +575,15 @@ __global__ __launch_bounds__(NW * 64) void mx8_decode_kernel(Mx8DecParams p)
 }
 
 // out = cast(sum over the K segments, in order, of part[s] + bias) for one pass of up to 16 rows
+template <int W>
 __global__ __launch_bounds__(256) void mx8dec_reduce_kernel(Mx8DecParams p, int splits)
 {
-    splitk_rows((const float*)p.part, splits, p.part_slice, p.M, p.N, [&](int64_t m, int64_t n0, int cols, v4f v) {
+    splitk_rows<W>((const float*)p.part, splits, p.part_slice, p.M, p.N, [&](int64_t m, int64_t n0, float (&v)[W]) {
         if (p.bias) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) v[e] = v[e] + p.bias[n0 + (e < cols ? e : cols - 1)];
+            for (int e = 0; e < W; e++) v[e] = v[e] + p.bias[n0 + e];
         }
-        store_quad(p.out, p.out_dt, m * p.N + n0, cols, v);
+        store_cols(p.out, p.out_dt, m * p.N + n0, v);
     });
 }
 
@@ -596,7 +598,7 @@ int launch_mx8_one(const Mx8DecParams& p, hipStream_t st, int splits)
     const size_t lds = (size_t)2 * NW * 256 * sizeof(float);
     hipLaunchKernelGGL((mx8_decode_kernel<NW, NBLK>), dim3((unsigned)grid, (unsigned)splits), dim3(NW * 64), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
-    hipLaunchKernelGGL(mx8dec_reduce_kernel, splitk_rows_grid(p.M, p.N), dim3(256), 0, st, p, splits);
+    splitk_launch(p.M, p.N, [&](auto w, dim3 g, dim3 b) { hipLaunchKernelGGL(mx8dec_reduce_kernel<decltype(w)::value>, g, b, 0, st, p, splits); });
     return (int)hipGetLastError();
 }
 

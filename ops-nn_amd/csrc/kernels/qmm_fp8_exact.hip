@@ -570,20 +570,20 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void qmm_fp8_exact_kernel(Fp8xPa
 
 // out[b, m, n] = the sum over the splits, in split order, of part[s, b, m, n], then the row / column epilogue (RC) and
 // the rounding
-template <bool RC>
+template <int W, bool RC>
 __global__ __launch_bounds__(256) void fp8x_splitk_reduce_kernel(Fp8xParams p, int64_t rows, int out_dt)
 {
-    splitk_rows((const float*)p.part, p.splits, rows * p.N, rows, p.N, [&](int64_t row, int64_t n0, int cols, v4f v) {
+    splitk_rows<W>((const float*)p.part, p.splits, rows * p.N, rows, p.N, [&](int64_t row, int64_t n0, float (&v)[W]) {
         if constexpr (RC) {
             const int64_t bz = rows == p.M ? 0 : row / p.M, m = row - bz * p.M;
             const float rs = p.rs ? p.rs[bz * p.rs_bs + m * p.rs_stride] : 1.0f;
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int64_t n = n0 + (e < cols ? e : cols - 1);
+            for (int e = 0; e < W; e++) {
+                const int64_t n = n0 + e;
                 v[e] = fp8x_rowcol_epilogue(p.ep_mode, v[e], rs, fp8x_col_scale(p, bz, n), fp8x_col_bias(p, bz, n));
             }
         }
-        store_quad(p.out, out_dt, row * p.N + n0, cols, v);
+        store_cols(p.out, out_dt, row * p.N + n0, v);
     });
 }
 
@@ -634,7 +634,7 @@ static int launch_fp8_exact_tile(const Fp8xParams& p, int64_t batch, hipStream_t
         hipLaunchKernelGGL(ks, grid, dim3(NT), lds, st, p, tiles_m, tiles_n);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
-        hipLaunchKernelGGL(fp8x_splitk_reduce_kernel<RC>, splitk_rows_grid(batch * p.M, p.N), dim3(256), 0, st, p, batch * p.M, OUT_DT);
+        splitk_launch(batch * p.M, p.N, [&](auto w, dim3 g, dim3 b) { hipLaunchKernelGGL((fp8x_splitk_reduce_kernel<decltype(w)::value, RC>), g, b, 0, st, p, batch * p.M, OUT_DT); });
         return (int)hipGetLastError();
     }
     auto k = qmm_fp8_exact_kernel<WGM, WGN, OUT_DT, RC, FMT, MXS>;

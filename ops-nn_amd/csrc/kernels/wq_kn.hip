@@ -217,8 +217,7 @@ static int launch_kn_one(const WqParams& p, int splits, hipStream_t st)
     }
     hipLaunchKernelGGL(k, grid, dim3(256), lds, st, p, splits);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
-    hipLaunchKernelGGL(wq_splitk_reduce_kernel, splitk_rows_grid(p.M, p.N), dim3(256), 0, st, (const float*)p.part, splits, p.M, p.N, p.bias, p.bias_dt,
-                       (void*)p.y, XDT);
+    launch_wq_splitk_reduce(p, splits, XDT, st);
     return (int)hipGetLastError();
 }
 template <int XDT, int WBITS, bool HAS_OFF>

@@ -216,8 +216,7 @@ static int launch_nk_one(const WqParams& p, const WqNkPlan& pl, hipStream_t st)
     }
     hipLaunchKernelGGL(k, grid, dim3(256), lds_sum > lds_tab ? lds_sum : lds_tab, st, p, pl.splits, pl.groups);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || pl.splits == 1) return (int)e;
-    hipLaunchKernelGGL(wq_splitk_reduce_kernel, splitk_rows_grid(p.M, p.N), dim3(256), 0, st, (const float*)p.part, pl.splits, p.M, p.N, p.bias, p.bias_dt,
-                       (void*)p.y, XDT);
+    launch_wq_splitk_reduce(p, pl.splits, XDT, st);
     return (int)hipGetLastError();
 }
 template <int XDT, int WBITS, bool HAS_OFF>

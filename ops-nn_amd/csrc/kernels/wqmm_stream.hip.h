@@ -1429,35 +1429,42 @@ static int launch_resx_one(const WqParams& p, hipStream_t st)
 }
 
 // y[m, n] = rounded(sum over the K segments, in order, of part[s, m, n] + bias[n])
+template <int W>
 static __global__ __launch_bounds__(256) void wq_splitk_reduce_kernel(const float* part, int splits, int64_t M, int64_t N, const void* bias, int bias_dt,
                                                                       void* y, int y_dt)
 {
-    splitk_rows(part, splits, M * N, M, N, [&](int64_t row, int64_t n0, int cols, v4f v) {
+    splitk_rows<W>(part, splits, M * N, M, N, [&](int64_t row, int64_t n0, float (&v)[W]) {
         if (bias) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) v[e] = v[e] + load_scalar_as_f32(bias, bias_dt, n0 + (e < cols ? e : cols - 1));
+            for (int e = 0; e < W; e++) v[e] = v[e] + load_scalar_as_f32(bias, bias_dt, n0 + e);
         }
-        store_quad(y, y_dt, row * N + n0, cols, v);
+        store_cols(y, y_dt, row * N + n0, v);
+    });
+}
+static void launch_wq_splitk_reduce(const WqParams& p, int splits, int y_dt, hipStream_t st)
+{
+    splitk_launch(p.M, p.N, [&](auto w, dim3 g, dim3 b) {
+        hipLaunchKernelGGL(wq_splitk_reduce_kernel<decltype(w)::value>, g, b, 0, st, (const float*)p.part, splits, p.M, p.N, p.bias, p.bias_dt, (void*)p.y, y_dt);
     });
 }
 
 // the fp8 forms of the many-rows kernel: out[m, n] = cast(epilogue(sum over the K segments, in order, of part[s, m, n])); the
 // block-scale form has folded its scales in already, the row / column scale form (RC) computes
 // (sum * x2Scale[n]) * x1Scale[m] + bias[n] here as the kernel's own epilogue does
-template <bool RC>
+template <int W, bool RC>
 static __global__ __launch_bounds__(256) void rows_bs_splitk_reduce_kernel(const float* part, int splits, int64_t M, int64_t N, const float* rs, int64_t rs_stride,
                                                                            const float* cs, int64_t cs_stride, const float* bias, void* out, int out_dt)
 {
-    splitk_rows(part, splits, M * N, M, N, [&](int64_t row, int64_t n0, int cols, v4f v) {
+    splitk_rows<W>(part, splits, M * N, M, N, [&](int64_t row, int64_t n0, float (&v)[W]) {
         if constexpr (RC) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) {
-                const int64_t n = n0 + (e < cols ? e : cols - 1);
+            for (int e = 0; e < W; e++) {
+                const int64_t n = n0 + e;
                 v[e] = (v[e] * cs[n * cs_stride]) * rs[row * rs_stride];
                 if (bias) v[e] = v[e] + bias[n];
             }
         }
-        store_quad(out, out_dt, row * N + n0, cols, v);
+        store_cols(out, out_dt, row * N + n0, v);
     });
 }
 
@@ -1492,8 +1499,7 @@ static int launch_xreg_one(const WqParams& p, hipStream_t st, int splits = 1)
     hipLaunchKernelGGL(k, dim3((unsigned)(nblocks < g ? nblocks : g), (unsigned)splits), dim3(NW * 64), lds, st, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || splits == 1) return (int)e;
-    hipLaunchKernelGGL(wq_splitk_reduce_kernel, splitk_rows_grid(p.M, p.N), dim3(256), 0, st, (const float*)p.part, splits, p.M, p.N, p.bias, p.bias_dt,
-                       (void*)p.y, XDT);
+    launch_wq_splitk_reduce(p, splits, XDT, st);
     return (int)hipGetLastError();
 }
 
@@ -1635,19 +1641,16 @@ static int launch_rows_one(const WqParams& p, hipStream_t st)
     hipLaunchKernelGGL(k, dim3(grid, (unsigned)slabs, split ? (unsigned)p.ksplit : 1u), dim3(512), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
     if (split) {
-        constexpr int RT = 64;   // (few outputs: small workgroups deal them evenly over the CUs)
-        const dim3 rgrid = splitk_rows_grid(p.M, p.N, RT);
-        if constexpr (WF == 3) {
-            hipLaunchKernelGGL(rows_bs_splitk_reduce_kernel<false>, rgrid, dim3(RT), 0, st, (const float*)p.part, p.ksplit, p.M,
-                               p.N, (const float*)nullptr, (int64_t)0, (const float*)nullptr, (int64_t)0, (const float*)nullptr, (void*)p.y, p.bs_out_dt);
-            return (int)hipGetLastError();
-        }
-        if constexpr (WF == 4) {
-            hipLaunchKernelGGL(rows_bs_splitk_reduce_kernel<true>, rgrid, dim3(RT), 0, st, (const float*)p.part, p.ksplit, p.M,
-                               p.N, p.bs1, p.bs1_rs, p.bs2, p.bs2_cs, (const float*)p.bias, (void*)p.y, p.bs_out_dt);
-            return (int)hipGetLastError();
-        }
-        hipLaunchKernelGGL(wq_splitk_reduce_kernel, rgrid, dim3(RT), 0, st, (const float*)p.part, p.ksplit, p.M, p.N, p.bias, p.bias_dt, (void*)p.y, XDT);
+        if constexpr (WF == 3 || WF == 4) {
+            splitk_launch(p.M, p.N, [&](auto w, dim3 g, dim3 b) {
+                if constexpr (WF == 3)
+                    hipLaunchKernelGGL((rows_bs_splitk_reduce_kernel<decltype(w)::value, false>), g, b, 0, st, (const float*)p.part, p.ksplit, p.M, p.N,
+                                       (const float*)nullptr, (int64_t)0, (const float*)nullptr, (int64_t)0, (const float*)nullptr, (void*)p.y, p.bs_out_dt);
+                else
+                    hipLaunchKernelGGL((rows_bs_splitk_reduce_kernel<decltype(w)::value, true>), g, b, 0, st, (const float*)p.part, p.ksplit, p.M, p.N,
+                                       p.bs1, p.bs1_rs, p.bs2, p.bs2_cs, (const float*)p.bias, (void*)p.y, p.bs_out_dt);
+            });
+        } else launch_wq_splitk_reduce(p, p.ksplit, XDT, st);
         return (int)hipGetLastError();
     }
     return 0;
