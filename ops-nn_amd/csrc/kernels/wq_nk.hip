@@ -87,7 +87,7 @@ __global__ __launch_bounds__(256, 2) void wq_nk_kernel(WqParams p, int splits, i
     v4i xf[PF][STEPS][MB];
     auto fetch = [&](auto jc, int c) {
         constexpr int j = decltype(jc)::value;
-        const int k0 = c * KC + q * KPL, k = k0 < Ki ? k0 : Ki - KPL;   // (past the end of K: the last piece, multiplied by zeros of x)
+        const int k0 = c * KC + q * KPL, k = k0 < Ki ? k0 : Ki - KPL;   // (past the end of K: the last piece, which counts as zero)
         const uint8_t* w = wbase + (int64_t)k * WBITS / 8;
 #pragma unroll
         for (int b = 0; b < NB; b++) __builtin_memcpy(raw[j][b], w + b * wblk, PB);
@@ -106,15 +106,17 @@ __global__ __launch_bounds__(256, 2) void wq_nk_kernel(WqParams p, int splits, i
         constexpr int j = decltype(jc)::value;
         const int k = c * KC + q * KPL;
         const int gi = group_at(k < Ki ? k : Ki - KPL) - g_lo;
-        if (c == chunks - 1 && k >= Ki) {
+        uint32_t sow[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++) sow[b] = tab[(16 * b + r) * gmax + gi];
+        if (c == chunks - 1 && k >= Ki) {   // past the end of K: both factors zero (0 * inf is no zero; a code's weight is, with scale and offset 0)
 #pragma unroll
             for (int s = 0; s < STEPS; s++)
 #pragma unroll
                 for (int b = 0; b < MB; b++) xf[j][s][b] = (v4i){0, 0, 0, 0};
-        }
-        uint32_t sow[NB];
 #pragma unroll
-        for (int b = 0; b < NB; b++) sow[b] = tab[(16 * b + r) * gmax + gi];
+            for (int b = 0; b < NB; b++) sow[b] = 0;
+        }
 #pragma unroll
         for (int s = 0; s < STEPS; s++) {
             v4i xo[MB];
