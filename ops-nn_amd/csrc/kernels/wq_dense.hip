@@ -19,7 +19,7 @@ template <int XDT, int WBITS, bool HAS_OFF>
 __global__ __launch_bounds__(256) void wq_dequant_nk_kernel(WqParams p, uint16_t* __restrict__ out, int steps)
 {
     const int lane = threadIdx.x & 63;
-    const int64_t n = (int64_t)blockIdx.y * 4 + (threadIdx.x >> 6);
+    const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // (N on grid.x: grid.y ends at 65535)
     if (n >= p.N) return;
     const uint8_t* w = p.w + n * p.ldw;
     const uint16_t* sc = p.scale + n * p.s_cs;
@@ -28,7 +28,7 @@ __global__ __launch_bounds__(256) void wq_dequant_nk_kernel(WqParams p, uint16_t
     const int Ki = (int)p.K, groupi = (int)p.group;
 #pragma unroll 4
     for (int s = 0; s < steps; s++) {
-        const int k = ((int)blockIdx.x * steps + s) * 512 + lane * 8;
+        const int k = ((int)blockIdx.y * steps + s) * 512 + lane * 8;
         if (k >= Ki) break;
         v4i q = {0, 0, 0, 0};
         if constexpr (WBITS == 4) q[0] = *(const int*)(w + k / 2);
@@ -91,7 +91,7 @@ static int launch_dequant(const WqParams& p, bool kn, uint16_t* out, hipStream_t
         hipLaunchKernelGGL((wq_dequant_kn_kernel<XDT, WBITS, HAS_OFF>), grid, dim3(256), 0, st, p, out);
     } else {
         const int steps = 4;
-        const dim3 grid((unsigned)((p.K + 512 * steps - 1) / (512 * steps)), (unsigned)((p.N + 3) / 4));
+        const dim3 grid((unsigned)((p.N + 3) / 4), (unsigned)((p.K + 512 * steps - 1) / (512 * steps)));
         hipLaunchKernelGGL((wq_dequant_nk_kernel<XDT, WBITS, HAS_OFF>), grid, dim3(256), 0, st, p, out, steps);
     }
     return (int)hipGetLastError();
@@ -130,7 +130,7 @@ bool wq_dense_wanted(const OpsnnWqmmArgs& a)
     if (a.scale_dtype != a.x_dtype || a.force_variant == OPSNN_VARIANT_PLAIN) return false;
     if (opsnn_wq_tile_min() <= 128) return false;   // (test hook: such calls are sent to the tile kernel of wqmm_tile.hip)
     if (a.M <= 64 || a.K % 64 != 0 || a.N < 128 || (uintptr_t)a.x % 16) return false;
-    if (a.K >= (1ll << 22) || a.N >= (1ll << 30)) return false;
+    if (a.K >= (1ll << 22) || a.N >= (1ll << 24)) return false;   // (grids: K / 128 on grid.y, 64 threads per column on grid.x)
     if (a.group > 0 && a.group % 8 != 0) return false;
     const bool nk = a.w.row_stride == 1 && a.w.col_stride == a.K, kn = a.w.col_stride == 1 && a.w.row_stride == a.N;
     if (!nk && !kn) return false;

@@ -27,3 +27,12 @@ def test_dense_route(gpu, M, K, N, group, tW, w_dt, x_dt, off):
     print(f"case dense M={M} K={K} N={N} g={group} tW={tW} {w_dt} {x_dt}", flush=True)
     got = cases.run_wq_aclnn(m, inp, M, K, N)
     _b16_bar(got, cases.oracle_wq(m, inp, M, K, N), orc.F16 if x_dt == "f16" else orc.BF16, "dense route", K)
+
+
+def test_more_columns_than_a_grid_dimension_holds(gpu):
+    """262152 columns: the pass over the weight has them on grid.x (four per workgroup on grid.y would be 65538)."""
+    m = gpu
+    M, K, N = 65, 64, 262152
+    inp = cases.make_wq_inputs(m, M, K, N, 9, m.ACL_FLOAT16, m.ACL_INT4, 0, True, False, None)
+    print(f"case dense M={M} K={K} N={N}", flush=True)
+    _b16_bar(cases.run_wq_aclnn(m, inp, M, K, N), cases.oracle_wq(m, inp, M, K, N), orc.F16, "dense, wide", K)
