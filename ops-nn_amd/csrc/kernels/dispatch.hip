@@ -29,14 +29,12 @@ int launch_kg_mfma(const OpsnnQmmArgs& a, hipStream_t st);   // qmm_i4_kg.hip
 uint64_t kg_workspace_bytes(const OpsnnQmmArgs& a);
 int launch_mx_mfma(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk = {});
 int launch_wqmm_mfma(const OpsnnWqmmArgs& a, hipStream_t st);
-bool wq_dense_wanted(const OpsnnWqmmArgs& a);   // wq_dense.hip
-uint64_t wq_dense_workspace(const OpsnnWqmmArgs& a);
+uint64_t wq_dense_workspace(const OpsnnWqmmArgs& a);   // wq_dense.hip
 int launch_wq_dense(const OpsnnWqmmArgs& a, hipStream_t st);
 bool wq_kn_wanted(const OpsnnWqmmArgs& a);   // wq_kn.hip
 uint64_t wq_kn_workspace(const OpsnnWqmmArgs& a);
 int launch_wq_kn(const OpsnnWqmmArgs& a, hipStream_t st);
-bool wq_nk_wanted(const OpsnnWqmmArgs& a);   // wq_nk.hip
-uint64_t wq_nk_workspace(const OpsnnWqmmArgs& a);
+bool wq_nk_wanted(const OpsnnWqmmArgs& a, uint64_t* workspace);   // wq_nk.hip
 int launch_wq_nk(const OpsnnWqmmArgs& a, hipStream_t st);
 uint64_t mx_workspace_bytes(const OpsnnQmmArgs& a);
 }  // namespace opsnn
@@ -509,10 +507,10 @@ extern "C" uint64_t opsnnWqmmWorkspace(const OpsnnWqmmArgs* a)
         part = ((uint64_t)xs * (uint64_t)a->M * (uint64_t)a->N * 4 + 255) / 256 * 256;
     // many rows: the dequantised weight (and partial sums); [K, N] storage with the weight cache on: the K split of the cached copy's
     // kernel (whether it is on is only known in phase 2)
-    if (wq_dense_wanted(*a)) { const uint64_t dense = wq_dense_workspace(*a); return dense > part ? dense : part; }
+    if (const uint64_t dense = wq_dense_workspace(*a)) return dense > part ? dense : part;
     // few rows, a shape outside the specialised kernels: the streaming kernel without shape conditions or, for a weight at an
     // unaligned address, the kernels behind it (which of them is only known in phase 2)
-    if (wq_nk_wanted(*a) && !opsnn_force_plain()) { const uint64_t nk = wq_nk_workspace(*a); return nk > part ? nk : part; }
+    if (uint64_t nk = 0; !opsnn_force_plain() && wq_nk_wanted(*a, &nk)) return nk > part ? nk : part;
     if (a->w.row_stride == 1 || a->K == 1) return part;
     if (a->w.col_stride != 1 || a->w.row_stride != a->N) return part;
     const uint64_t relaid = part + (uint64_t)a->N * (uint64_t)a->K * bits / 8;

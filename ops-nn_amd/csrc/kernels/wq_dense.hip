@@ -8,6 +8,7 @@
 // run (N no multiple of 32, K no whole number of x slabs, groups of 64, [K, N] storage): it takes every layout, group and N.
 #include "gemm16.h"
 #include "launch.h"
+#include "wq_cost.h"
 #include "wq_kn.hip.h"
 #include "wqmm_stream.hip.h"
 
@@ -19,7 +20,9 @@ template <int XDT, int WBITS, bool HAS_OFF>
 __global__ __launch_bounds__(256) void wq_dequant_nk_kernel(WqParams p, uint16_t* __restrict__ out, int steps)
 {
     const int lane = threadIdx.x & 63;
-    const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);   // (N on grid.x: grid.y ends at 65535)
+    const int kblocks = ((int)p.K + 512 * steps - 1) / (512 * steps);   // (one grid dimension, K first: grid.y ends at 65535)
+    const int64_t n = (int64_t)(blockIdx.x / (unsigned)kblocks) * 4 + (threadIdx.x >> 6);
+    const int kb = (int)(blockIdx.x % (unsigned)kblocks);
     if (n >= p.N) return;
     const uint8_t* w = p.w + n * p.ldw;
     const uint16_t* sc = p.scale + n * p.s_cs;
@@ -28,7 +31,7 @@ __global__ __launch_bounds__(256) void wq_dequant_nk_kernel(WqParams p, uint16_t
     const int Ki = (int)p.K, groupi = (int)p.group;
 #pragma unroll 4
     for (int s = 0; s < steps; s++) {
-        const int k = ((int)blockIdx.y * steps + s) * 512 + lane * 8;
+        const int k = (kb * steps + s) * 512 + lane * 8;
         if (k >= Ki) break;
         v4i q = {0, 0, 0, 0};
         if constexpr (WBITS == 4) q[0] = *(const int*)(w + k / 2);
@@ -91,7 +94,7 @@ static int launch_dequant(const WqParams& p, bool kn, uint16_t* out, hipStream_t
         hipLaunchKernelGGL((wq_dequant_kn_kernel<XDT, WBITS, HAS_OFF>), grid, dim3(256), 0, st, p, out);
     } else {
         const int steps = 4;
-        const dim3 grid((unsigned)((p.N + 3) / 4), (unsigned)((p.K + 512 * steps - 1) / (512 * steps)));
+        const dim3 grid((unsigned)((p.N + 3) / 4 * ((p.K + 512 * steps - 1) / (512 * steps))));
         hipLaunchKernelGGL((wq_dequant_nk_kernel<XDT, WBITS, HAS_OFF>), grid, dim3(256), 0, st, p, out, steps);
     }
     return (int)hipGetLastError();
@@ -99,55 +102,91 @@ static int launch_dequant(const WqParams& p, bool kn, uint16_t* out, hipStream_t
 
 static uint64_t dense_weight_bytes(const OpsnnWqmmArgs& a) { return ((uint64_t)a.N * (uint64_t)a.K * 2 + 255) / 256 * 256; }
 
-// What the many-rows streaming kernel takes, in us: a workgroup of 128 columns and R rows (64, 128, 192 or 256) walks 4096 k in
-// 14 + 0.21 R (measured 27, 38, 52 and 67; a quarter less where few CUs have one), a CU at a time; rows as wq_narrow_slab_rows deals them, or in passes of 256.  With
-// more than 128 rows and a K that is no whole number of x rounds of those instances, three times that.
+// What the many-rows streaming kernel takes, in us, fitted to 96 calls of 65 .. 2100 rows (median error 5 %): a workgroup of 128
+// columns and R rows (64, 128, 192 or 256) walks 4096 k in DQ + 0.242 R beside 7.5 us a launch, where DQ is what dequantising takes;
+// with 64 columns, where 64 rows leave the chip idle (use_cols64), 0.55 times that.  Rows as wq_narrow_slab_rows deals them, or
+// in passes of 256.  With more than 128 rows and a K that is no whole number of x rounds of those instances, three times that;
+// bf16 with 8-bit weights has no 256-row instance that fits and takes 1.6 times that there.
 static double rows_kernel_us(const OpsnnWqmmArgs& a, int wbits, int64_t group)
 {
-    const int64_t wgs = (a.N + 127) / 128, kx = 2 * 4 * (128 / wbits), slab = wq_narrow_slab_rows(a.M, a.N, true);
+    const int64_t wgs = (a.N + 127) / 128, kc = 4 * (128 / wbits), slab = wq_narrow_slab_rows(a.M, a.N, true);
     const int64_t ks = wq_rows_ksplit(wbits, a.M, a.N, a.K, group, true);
+    const bool bf16 = a.x_dtype == DT_BF16, ragged = a.K % (8 * kc) != 0;
+    const double dq = wq_rows_dequant_us(wbits, bf16);
     auto launch_us = [&](int64_t rows, int64_t slabs) {
         const int64_t r = (rows + 63) / 64 * 64, n = wgs * slabs * ks;
-        const double rounds = n < 256 ? 0.75 + 0.25 * (double)n / 256.0 : (double)((n + 255) / 256);
-        return rounds * (double)a.K / (4096.0 * (double)ks) * (14.0 + 0.21 * (double)r) * (r > 128 && a.K % (4 * kx) != 0 ? 3.0 : 1.0);
+        const bool cols64 = r <= 64 && ks == 1 && wgs * slabs <= 128 && a.K % (4 * kc) == 0;
+        const double rounds = cols64 ? 0.55 : n < 256 ? 0.94 + 0.06 * (double)n / 256.0 : (double)((n + 255) / 256);
+        const double more = r > 128 && ragged ? 3.0 : r > 192 && bf16 && wbits == 8 ? 1.6 : 1.0;
+        return 7.5 + rounds * (double)a.K / (4096.0 * (double)ks) * (dq + 0.242 * (double)r) * more;
     };
-    const double part_us = ks > 1 ? 4.0 + 8.0 * (double)ks * (double)a.M * (double)a.N / 5.0e6 : 0.0;
+    const double part_us = ks > 1 ? 2.0 + 8.0 * (double)ks * (double)a.M * (double)a.N / 5.0e6 : 0.0;
     if (slab) return launch_us(slab, (a.M + slab - 1) / slab) + part_us;
     return (double)(a.M / 256) * launch_us(256, 1) + (a.M % 256 ? launch_us(a.M % 256, 1) : 0.0) + part_us;
 }
+// The tile kernel of wqmm_tile.hip, from 129 rows, in passes of up to 256 rows and workgroups of 128 columns.
+static double tile_kernel_us(const OpsnnWqmmArgs& a, const WqForm& f)
+{
+    const double per = f.wbits == 8 ? 16.2 : f.group < 128 ? 15.6 : 14.65;
+    return (double)((a.M + 255) / 256) * (6.0 + per * (double)a.K / 1024.0 * (double)((a.N + 32767) / 32768));
+}
 
-// Does the call run on this route?  Looks at what phase 1 knows (shapes, types, layouts, addresses), so that both phases agree.
-//
-// The pass moves 2.5 (8-bit weights: 3) bytes per weight at 5 TB/s, the product takes what gemm16_plan estimates.  Against
-// it stands the many-rows streaming kernel where it runs (wqmm.hip: [N, K] storage, N % 32 == 0, whole x slabs and groups of
-// whole chunks); everywhere else the general kernel re-reads the weight per 64 rows at a fraction of its speed, and this
-// route takes every call of more than 64 rows.  (Measured: 1999 x 4096 x 11008 bf16 x int4 228 -> 156 us, [K, N] storage
-// 613 -> 162; 700 x 4096 x 11008 134 -> 106; 1024 x 8192 x 28672 497 against 499, 512 rows 254 against 330.)
-bool wq_dense_wanted(const OpsnnWqmmArgs& a)
+// Is this route faster than the kernel that would take the call otherwise?  The pass moves 2.5 (8-bit weights: 3) bytes per weight
+// at 6 TB/s ([K, N] storage: 3.5, 4.6 with 8-bit weights), the product takes product_us (gemm16_plan) and 0.2 us more per 10^6
+// weights, which it reads from beyond its L2.  Against it stand, with [K, N] storage behind a re-layout at 0.62 (0.73) TB/s of
+// codes: the many-rows kernel where its shape conditions hold (with groups in [K, N] storage its scale table, and so its
+// 192- and 256-row instances, do not apply); else, from 129 rows, the tile kernel and up to 128 rows the streaming kernel.
+// With groups that are not whole chunks the general kernel is left, which counts where wq_general_counts says so.
+// (Of 368 measured calls 362 go to the faster side or one within 3 % of it: 1999 x 4096 x 11008 bf16 x int4 228 -> 164 us, [K, N] storage 613 -> 162; 1000 x 8192 x 28672 fp16 x int4 stays on the many-rows
+// kernel, 477 against 526; 65 x 4096 x 22896 on the streaming kernel, 54 against 93; 192 x 8192 x 22896 on the tile kernel, 127
+// against 230; 128 x 11008 x 4096 in [K, N] storage with the re-layout, 61 against 75.)
+static bool dense_is_faster(const OpsnnWqmmArgs& a, double product_us)
+{
+    const WqForm f = wq_form(a);
+    const double codes = (double)a.N * (double)a.K;
+    double other;
+    const bool four = f.wbits == 4, tile_ok = a.K % (four ? 128 : 64) == 0 && f.group % 64 == 0;
+    const bool no_table = !f.nk && f.group < a.K;
+    const double tile_us = tile_kernel_us(a, f) * (no_table ? 1.25 : 1.0);
+    if (f.rows) {
+        const int64_t slab = wq_narrow_slab_rows(a.M, a.N, true);
+        if (no_table && (slab ? slab : a.M) > 128) other = tile_us;
+        else other = rows_kernel_us(a, f.wbits, f.group) * (no_table && a.x_dtype == DT_BF16 ? 1.25 : 1.0);
+    }
+    else if (a.M > 128 && tile_ok) other = tile_us;
+    else if (f.stream) other = wq_passes_of_64_us(a.M, [&](int64_t r) { return wq_stream_pass_us(f.wbits, a.x_dtype == DT_BF16, r, a.N, a.K); });
+    else if (wq_general_counts(a, f)) other = wq_passes_of_64_us(a.M, [&](int64_t r) { return wq_general_pass_us(r, a.N, a.K); });
+    else return true;
+    if (!f.nk) other += 2.0 + codes * f.wbits / 8.0 / (four ? 0.62e6 : 0.73e6);
+    const double pass_rate = f.nk ? 6.0e6 : four ? 3.5e6 : 4.6e6;
+    return 3.0 + codes * (2.0 + f.wbits / 8.0) / pass_rate + product_us + codes * 2.0e-7 < 0.97 * other;   // (in doubt without the pass)
+}
+
+// Can the call run here?
+static bool dense_takes(const OpsnnWqmmArgs& a, const WqForm& f)
 {
     if (a.w_dtype != DT_I4 && a.w_dtype != DT_I8) return false;
     if (a.x_dtype != DT_F16 && a.x_dtype != DT_BF16) return false;
     if (a.scale_dtype != a.x_dtype || a.force_variant == OPSNN_VARIANT_PLAIN) return false;
     if (opsnn_wq_tile_min() <= 128) return false;   // (test hook: such calls are sent to the tile kernel of wqmm_tile.hip)
     if (a.M <= 64 || a.K % 64 != 0 || a.N < 128 || (uintptr_t)a.x % 16) return false;
-    if (a.K >= (1ll << 22) || a.N >= (1ll << 24)) return false;   // (grids: K / 128 on grid.y, 64 threads per column on grid.x)
+    if (a.K >= (1ll << 22) || a.N >= (1ll << 24) || a.N * a.K >= (1ll << 36)) return false;   // (what the grids of the pass hold)
     if (a.group > 0 && a.group % 8 != 0) return false;
-    const bool nk = a.w.row_stride == 1 && a.w.col_stride == a.K, kn = a.w.col_stride == 1 && a.w.row_stride == a.N;
-    if (!nk && !kn) return false;
-    if (a.w_dtype == DT_I4 && !nk && a.N % 2 != 0) return false;
-    const int wbits = a.w_dtype == DT_I4 ? 4 : 8;
-    const int64_t kc = 4 * (128 / wbits);
-    const int64_t cpg = a.group > 0 && a.group < a.K ? a.group / kc : 1;
-    const bool rows_kernel = nk && a.N % 32 == 0 && a.N >= 256 && a.K % (2 * kc) == 0 &&
-                             (a.group <= 0 || a.group >= a.K || (a.group % kc == 0 && (cpg & (cpg - 1)) == 0));
-    if (!rows_kernel) return true;
-    const double rows_us = rows_kernel_us(a, wbits, a.group > 0 && a.group < a.K ? a.group : a.K);
-    const double dense_us = 2.0 + (double)a.N * (double)a.K * (2.0 + wbits / 8.0) / 5.0e6 + gemm16_plan(a.M, a.N, a.K, 1).us;
-    return dense_us < rows_us;
+    if (!f.nk && (a.w.col_stride != 1 || a.w.row_stride != a.N)) return false;
+    return a.w_dtype != DT_I4 || f.nk || a.N % 2 == 0;
 }
+// (K-contiguous outside the many-rows kernel's shapes: planned for in any case, since the other kernels take no weight at an
+// unaligned address)
+static bool always_planned(const WqForm& f) { return f.nk && !f.rows; }
+
+// Workspace of this route, 0 if phase 1 does not plan for it.  Looks at what both phases know: shapes, types and layouts, not the
+// weight's address.
 uint64_t wq_dense_workspace(const OpsnnWqmmArgs& a)
 {
+    const WqForm f = wq_form(a);
+    if (!dense_takes(a, f)) return 0;
     const Gemm16Plan pl = gemm16_plan(a.M, a.N, a.K, 1);
+    if (!always_planned(f) && !dense_is_faster(a, pl.us)) return 0;
     return dense_weight_bytes(a) + gemm16_part_bytes(pl, a.M, a.N, 1);
 }
 
@@ -157,15 +196,18 @@ int launch_wqmm_mfma(const OpsnnWqmmArgs& a, hipStream_t st);   // wqmm.hip
 
 int launch_wq_dense(const OpsnnWqmmArgs& a, hipStream_t st)
 {
-    if (!a.workspace || !wq_dense_wanted(a)) return OPSNN_NOT_TAKEN;
-    const int wbits = a.w_dtype == DT_I4 ? 4 : 8;
-    const bool kn = a.w.row_stride != 1;
+    const WqForm f = wq_form(a);
+    if (!a.workspace || !dense_takes(a, f)) return OPSNN_NOT_TAKEN;
+    const int wbits = f.wbits;
+    const bool kn = !f.nk, unaligned = (uintptr_t)a.w.ptr % 16 != 0;
+    const Gemm16Plan pl = gemm16_plan(a.M, a.N, a.K, 1);
+    if (!(always_planned(f) && unaligned) && !dense_is_faster(a, pl.us)) return OPSNN_NOT_TAKEN;
     if (kn && weight_cache_on()) {
-        // a caller who keeps K-contiguous copies in the weight cache: where that form runs on the streaming kernel, so does the
-        // copy (128 x 8192 x 28672 int4: 75 us, 329 with the pass here); phase 1 has left room for its partial sums
+        // a caller who keeps K-contiguous copies in the weight cache: where that form runs on another kernel, so does the copy
+        // (128 x 8192 x 28672 int4: 75 us, 329 with the pass here); phase 1 has left room for its partial sums
         OpsnnWqmmArgs b = a;
         b.w.row_stride = 1; b.w.col_stride = a.K;
-        if (!wq_dense_wanted(b) && (b.w.ptr = weight_cache_get(a.w.ptr, a.K, a.N, wbits, 1, st)) != nullptr) {
+        if (!dense_is_faster(b, pl.us) && (b.w.ptr = weight_cache_get(a.w.ptr, a.K, a.N, wbits, 1, st)) != nullptr) {
             const int rc = launch_wqmm_mfma(b, st);
             if (rc != OPSNN_NOT_TAKEN) return rc;
         }
@@ -189,7 +231,6 @@ int launch_wq_dense(const OpsnnWqmmArgs& a, hipStream_t st)
         else rc = a.offset ? launch_dequant<DT_BF16, 8, true>(p, kn, w16, st) : launch_dequant<DT_BF16, 8, false>(p, kn, w16, st);
     }
     if (rc != 0) return rc;
-    const Gemm16Plan pl = gemm16_plan(a.M, a.N, a.K, 1);
     QgemmParams g{};
     g.a = (const int8_t*)a.x; g.b = (const int8_t*)w16;
     g.lda = 2 * a.K; g.ldb = 2 * a.K; g.KB = 2 * a.K;

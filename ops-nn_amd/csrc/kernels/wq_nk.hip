@@ -15,6 +15,7 @@
 // segments; sums meet in LDS in a fixed order, segments in `part`, added in order by wq_splitk_reduce_kernel.  A wave past the
 // edge of N repeats the last columns (stored twice, same bits).
 #include "launch.h"
+#include "wq_cost.h"
 #include "wqmm_stream.hip.h"
 
 extern "C" int opsnn_wq_narrow_slabs();   // dispatch.hip
@@ -29,17 +30,22 @@ constexpr int nk_nb(int mb) { return mb == 4 ? 4 : 8; }
 static bool nk_plan(int wbits, int64_t M, int64_t N, int64_t K, int64_t group, WqNkPlan& pl)
 {
     pl.mb = M <= 16 ? 1 : M <= 32 ? 2 : 4;
-    const int64_t cols = 16 * nk_nb(pl.mb), strips = (N + cols - 1) / cols, kc = (pl.mb == 4 || wbits == 8) ? 64 : 128, chunks = (K + kc - 1) / kc;
+    // (32-bit: both phases of every call with few rows come here; N and K are below 2^30)
+    const uint32_t cols = 16 * nk_nb(pl.mb), strips = ((uint32_t)N + cols - 1) / cols, kc = (pl.mb == 4 || wbits == 8) ? 64 : 128;
+    const uint32_t chunks = ((uint32_t)K + kc - 1) / kc;
     // (a chunk: 8 KB of codes per wave; four row blocks: 2 KB of 4-bit, 4 KB of 8-bit codes; eight waves of a CU at 5 TB/s)
     const double t_chunk = pl.mb == 4 ? (wbits == 4 ? 1.4 : 2.0) : pl.mb == 2 ? 4.1 : 3.4;
+    const double slice_us = 8.0 * (double)M * (double)N / 4.0e6;
     double best = 1e30;
     bool found = false;
-    for (int s = 1; s <= 16 && chunks / s >= 2; s++) {
-        const int64_t seg = (chunks + s - 1) / s * kc, g = group >= K ? 1 : (seg + group - 1) / group + 1;
-        if (g * cols * 4 > 32768) continue;
-        const double us = (double)((strips * s + 511) / 512) * ((double)((chunks + 4 * s - 1) / (4 * s)) * t_chunk + 4.0) +
-                          (s > 1 ? 3.0 + 8.0 * s * (double)M * (double)N / 4.0e6 : 0.0);
-        if (us < best) { best = us; pl.splits = s; pl.groups = (int)g; found = true; }
+    for (uint32_t s = 1; s <= 16 && chunks >= 2 * s; s++) {
+        const uint32_t seg = (chunks + s - 1) / s * kc, per_wave = (chunks + 4 * s - 1) / (4 * s);
+        const uint32_t g = group >= K ? 1 : (seg + (uint32_t)group - 1) / (uint32_t)group + 1;
+        if (g <= 8192 / cols) {   // (a table of 32 KB)
+            const double us = (double)((strips * s + 511) / 512) * ((double)per_wave * t_chunk + 4.0) + (s > 1 ? 3.0 + slice_us * s : 0.0);
+            if (us < best) { best = us; pl.splits = (int)s; pl.groups = (int)g; found = true; }
+        }
+        if (per_wave == 1 && found) break;   // (more segments only add partial sums)
     }
     return found;
 }
@@ -229,48 +235,71 @@ static int launch_nk_mb(const WqParams& p, const WqNkPlan& pl, hipStream_t st)
     return launch_nk_one<XDT, WBITS, 4, HAS_OFF>(p, pl, st);
 }
 
+// What this kernel takes with its plan, in us (median error 6 %).
+static double nk_us(int wbits, bool bf16, int64_t M, int64_t N, int64_t K, const WqNkPlan& pl)
+{
+    const int64_t cols = 16 * nk_nb(pl.mb), kc = (pl.mb == 4 || wbits == 8) ? 64 : 128, chunks = (K + kc - 1) / kc;
+    const int64_t wgs = (N + cols - 1) / cols * pl.splits, per_wave = (chunks + 4 * pl.splits - 1) / (4 * pl.splits);
+    const double t = pl.mb == 4 ? 1.72 * (wbits == 8 ? 1.05 : 1.0) : (pl.mb == 2 ? 4.1 : 3.6) * (wbits == 8 ? 0.8 : 1.0);
+    const double share = wgs > 256 ? (pl.mb == 4 ? 1.7 : 1.5) : 1.0;   // two workgroups on a CU
+    return 6.4 + (double)per_wave * t * share * (double)((wgs + 511) / 512) * (bf16 ? 1.035 : 1.0) +
+           (pl.splits > 1 ? 0.7 + 8.0 * pl.splits * (double)M * (double)N / 4.0e6 : 0.0);
+}
+
 // Does the call run here?  Looks at what both phases know: not at the weight's address, which for a FRACTAL_NZ weight is that of
-// its ND copy in phase 2 alone (launch_wq_nk declines an unaligned one; the workspace has room for either outcome).  The
-// specialised kernels keep what they take (wqmm.hip): K in whole 128-element units, groups of whole chunks, and from 17 rows
-// N % 32 == 0 and K in whole x slabs.
-bool wq_nk_wanted(const OpsnnWqmmArgs& a)
+// its ND copy in phase 2 alone (launch_wq_nk declines an unaligned one; the workspace has room for either outcome).
+//
+// Up to 16 rows the specialised kernels keep what they take (wqmm.hip): K in whole 128-element units, groups of whole chunks.
+// Otherwise the estimates decide: against the streaming kernel (17 .. 32 rows, and from 33 where the many-rows kernel's shape
+// conditions fail), the many-rows kernel (from 33 rows, narrow weights), and the general kernel (groups that are not whole chunks;
+// fp16 with 4-bit weights, elsewhere it is never the faster one).  A short K or a wide N is theirs, a long K against a narrow N is
+// cut along K here: 17 x 1024 x 11016 fp16 x int4 7.5 us there and 11.4 here, 48 x 8192 x 22896 61 and 93, but 64 x 8192 x 4104
+// 50 and 25.5, 32 x 4096 x 4096 bf16 21.9 and 13.4, 64 x 4096 x 4096 23.8 and 17.5; groups of 64: 16 x 1024 x 11008 8.5 and 12.1,
+// 64 x 8192 x 2048 40 and 18.  (Of 513 measured calls 492 go to the faster kernel or one within 3 % of it.)
+static bool nk_wanted(const OpsnnWqmmArgs& a, WqNkPlan& pl)
 {
     if ((a.w_dtype != DT_I4 && a.w_dtype != DT_I8) || (a.x_dtype != DT_F16 && a.x_dtype != DT_BF16)) return false;
     if (a.scale_dtype != a.x_dtype) return false;
     if (a.M > 64 || a.K % 32 != 0 || a.K < 256 || a.N < 256 || a.K >= (1ll << 30) || a.N >= (1ll << 30)) return false;
     if (a.w.row_stride != 1 || a.w.col_stride != a.K) return false;
-    const int64_t group = a.group > 0 && a.group < a.K ? a.group : a.K;
-    if (group < a.K && group % 32 != 0) return false;
-    if ((uintptr_t)a.x % 16 != 0) return false;
-    WqNkPlan pl;
-    if (!nk_plan(a.w_dtype == DT_I4 ? 4 : 8, a.M, a.N, a.K, group, pl)) return false;
-    if (a.force_variant != 0) return false;
-    const int wbits = a.w_dtype == DT_I4 ? 4 : 8;
-    const int64_t kc = 4 * (128 / wbits), cpg = group / kc;
-    const bool whole_groups = group >= a.K || (group % kc == 0 && (cpg & (cpg - 1)) == 0);
-    if (!whole_groups || a.K % kc != 0) return true;
-    if (a.M <= 16) return a.K % 128 != 0;
-    // (17 .. 32 rows against a narrow N and a K that the many-rows kernel does not cut: there the streaming kernel's workgroups are
-    // few -- 32 x 4096 x 4096 fp16 / bf16 17.1 / 21.1 us against 13.3 / 13.5 here; at N = 11008 it is 20 against 24)
-    // (33 .. 64 rows: up to N = 5120 -- 64 x 4096 x 2048 20.0 -> 12.8 us, 64 x 7168 x 4096 29.2 -> 24.2, 64 x 4096 x 4096 20.2 -> 16.5;
-    // 40 x 4096 x 6144 19.3 against 19.6, 64 x 2048 x 8192 14.5 against 16.5, 40 x 14336 x 4096, cut along K there, 22.7 against 28.6)
-    if (opsnn_wq_narrow_slabs() && a.K < 8192 && a.N <= (a.M <= 32 ? 8192 : 5120)) return true;
-    return a.N % 32 != 0 || a.K % (2 * kc) != 0;
+    if ((uintptr_t)a.x % 16 != 0 || a.force_variant != 0) return false;
+    const WqForm f = wq_form(a);
+    if (f.group < a.K && f.group % 32 != 0) return false;
+    if (f.stream && a.M <= 16 && a.K % 128 == 0) return false;   // (the x-in-registers kernel)
+    if (!nk_plan(f.wbits, a.M, a.N, a.K, f.group, pl)) return false;
+    if (f.stream && a.M <= 16) return true;
+    const bool bf16 = a.x_dtype == DT_BF16;
+    double other;
+    if (f.stream && a.M > 32 && f.rows) {
+        if (!opsnn_wq_narrow_slabs() || a.K >= 8192 || a.N > 8192) return false;   // (wide, or cut along K there)
+        if (a.N > 5120 && wq_part_slices(f.wbits, a.M, a.N, a.K, f.group, true) > 1) return false;
+        const int64_t kc = 4 * (128 / f.wbits), wgs = (a.N + 127) / 128;
+        const double cols = wgs <= 128 && a.K % (4 * kc) == 0 ? 0.6 : (double)((wgs + 255) / 256);
+        other = 6.0 + cols * (double)a.K / 4096.0 * (wq_rows_dequant_us(f.wbits, bf16) + 15.5);
+    }
+    else if (f.stream) {
+        if (f.rows && (!opsnn_wq_narrow_slabs() || wq_part_slices(f.wbits, a.M, a.N, a.K, f.group, true) > 1)) return false;
+        other = wq_stream_pass_us(f.wbits, bf16, a.M, a.N, a.K);
+    }
+    else if (wq_general_counts(a, f)) other = 0.94 * wq_general_pass_us(a.M, a.N, a.K);   // (in doubt the general one)
+    else return true;
+    return nk_us(f.wbits, bf16, a.M, a.N, a.K, pl) < other;
 }
-uint64_t wq_nk_workspace(const OpsnnWqmmArgs& a)
+// ... and if so, the workspace it needs.
+bool wq_nk_wanted(const OpsnnWqmmArgs& a, uint64_t* workspace)
 {
     WqNkPlan pl;
-    if (!nk_plan(a.w_dtype == DT_I4 ? 4 : 8, a.M, a.N, a.K, a.group > 0 && a.group < a.K ? a.group : a.K, pl)) return 0;
-    return pl.splits > 1 ? ((uint64_t)pl.splits * (uint64_t)a.M * (uint64_t)a.N * 4 + 255) / 256 * 256 : 0;
+    if (!nk_wanted(a, pl)) return false;
+    *workspace = pl.splits > 1 ? ((uint64_t)pl.splits * (uint64_t)a.M * (uint64_t)a.N * 4 + 255) / 256 * 256 : 0;
+    return true;
 }
 int launch_wq_nk(const OpsnnWqmmArgs& a, hipStream_t st)
 {
-    if (!wq_nk_wanted(a) || (uintptr_t)a.w.ptr % 16 != 0) return OPSNN_NOT_TAKEN;
+    WqNkPlan pl;
+    if ((uintptr_t)a.w.ptr % 16 != 0 || !nk_wanted(a, pl) || (pl.splits > 1 && !a.workspace)) return OPSNN_NOT_TAKEN;
     const int wbits = a.w_dtype == DT_I4 ? 4 : 8;
     WqParams p{};
     p.group = a.group > 0 && a.group < a.K ? a.group : a.K;
-    WqNkPlan pl;
-    if (!nk_plan(wbits, a.M, a.N, a.K, p.group, pl) || (pl.splits > 1 && !a.workspace)) return OPSNN_NOT_TAKEN;
     p.x = (const uint16_t*)a.x;
     p.w = (const uint8_t*)a.w.ptr; p.ldw = a.w.col_stride * wbits / 8;
     p.scale = (const uint16_t*)a.scale.ptr; p.offset = (const uint16_t*)a.offset;
