@@ -31,7 +31,7 @@ template <int MODE, int BM, int BN, int WGM, int WGN, int STAGES>
 static int launch_split16(const QgemmParams& p, int64_t batch, int out_dt, hipStream_t st)
 {
     constexpr int BK = 128;
-    if (!p.part || p.splits < 2 || (p.KB % BK) != 0 || p.splits > p.KB / BK / 2 || p.ldc != p.N) return -1;
+    if (!p.part || p.splits < 2 || (p.KB % BK) != 0 || p.splits > p.KB / BK / 2) return -1;
     const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
     const size_t lds = (size_t)STAGES * (BM + BN) * BK;
     auto k = qgemm_kernel<MODE, BM, BN, BK, WGM, WGN, STAGES, 1, false, DT_BF16, true>;

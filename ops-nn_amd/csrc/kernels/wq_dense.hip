@@ -100,8 +100,39 @@ static int launch_dequant(const WqParams& p, bool kn, uint16_t* out, hipStream_t
     return (int)hipGetLastError();
 }
 
-static uint64_t dense_weight_bytes(const OpsnnWqmmArgs& a) { return ((uint64_t)a.N * (uint64_t)a.K * 2 + 255) / 256 * 256; }
-
+// The columns go in strips whose dequantised weight takes at most 1 GiB of workspace (a vocabulary of 152064 against 8192: 2.5 GB in
+// one piece).  Of the widths between half of that and all of it the one whose products have the smallest estimate: a strip that ends
+// in a nearly empty round of the chip loses a tenth (1000 x 8192 x 152064: 2335 us so,
+// 2315 in one piece, 2588 in five equal strips).
+constexpr int64_t STRIP_BYTES = 1ll << 30;
+struct DensePlan {
+    int64_t strip, strips;      // columns of a strip but the last one
+    Gemm16Plan full, last;
+    double us;                  // the products' estimate
+    uint64_t weight_bytes, part_bytes;
+};
+static DensePlan dense_plan(int64_t M, int64_t N, int64_t K)
+{
+    DensePlan best;
+    best.us = 1e30;
+    const int64_t most = STRIP_BYTES / (2 * K) / 256 * 256;
+    for (int i = 0; i < 8; i++) {
+        DensePlan d;
+        d.strip = most >= N ? N : most - most * i / 16 / 256 * 256;
+        if (d.strip < 256 && d.strip < N) d.strip = 256;
+        d.strips = (N + d.strip - 1) / d.strip;
+        const int64_t rest = N - (d.strips - 1) * d.strip;
+        d.last = gemm16_plan(M, rest, K, 1);
+        d.full = rest == d.strip ? d.last : gemm16_plan(M, d.strip, K, 1);
+        d.us = (double)(d.strips - 1) * (d.full.us + 5.0) + d.last.us;
+        d.weight_bytes = ((uint64_t)d.strip * (uint64_t)K * 2 + 255) / 256 * 256;
+        const uint64_t pa = d.strips > 1 ? gemm16_part_bytes(d.full, M, d.strip, 1) : 0, pb = gemm16_part_bytes(d.last, M, rest, 1);
+        d.part_bytes = pa > pb ? pa : pb;
+        if (d.us < best.us) best = d;
+        if (most >= N) break;
+    }
+    return best;
+}
 // What the many-rows streaming kernel takes, in us, fitted to 96 calls of 65 .. 2100 rows (median error 5 %): a workgroup of 128
 // columns and R rows (64, 128, 192 or 256) walks 4096 k in DQ + 0.242 R beside 7.5 us a launch, where DQ is what dequantising takes;
 // with 64 columns, where 64 rows leave the chip idle (use_cols64), 0.55 times that.  Rows as wq_narrow_slab_rows deals them, or
@@ -185,9 +216,9 @@ uint64_t wq_dense_workspace(const OpsnnWqmmArgs& a)
 {
     const WqForm f = wq_form(a);
     if (!dense_takes(a, f)) return 0;
-    const Gemm16Plan pl = gemm16_plan(a.M, a.N, a.K, 1);
+    const DensePlan pl = dense_plan(a.M, a.N, a.K);
     if (!always_planned(f) && !dense_is_faster(a, pl.us)) return 0;
-    return dense_weight_bytes(a) + gemm16_part_bytes(pl, a.M, a.N, 1);
+    return pl.weight_bytes + pl.part_bytes;
 }
 
 bool weight_cache_on();   // weight_cache.hip
@@ -200,7 +231,7 @@ int launch_wq_dense(const OpsnnWqmmArgs& a, hipStream_t st)
     if (!a.workspace || !dense_takes(a, f)) return OPSNN_NOT_TAKEN;
     const int wbits = f.wbits;
     const bool kn = !f.nk, unaligned = (uintptr_t)a.w.ptr % 16 != 0;
-    const Gemm16Plan pl = gemm16_plan(a.M, a.N, a.K, 1);
+    const DensePlan pl = dense_plan(a.M, a.N, a.K);
     if (!(always_planned(f) && unaligned) && !dense_is_faster(a, pl.us)) return OPSNN_NOT_TAKEN;
     if (kn && weight_cache_on()) {
         // a caller who keeps K-contiguous copies in the weight cache: where that form runs on another kernel, so does the copy
@@ -214,29 +245,37 @@ int launch_wq_dense(const OpsnnWqmmArgs& a, hipStream_t st)
     }
     uint16_t* w16 = (uint16_t*)a.workspace;
     WqParams p{};
-    p.w = (const uint8_t*)a.w.ptr;
     p.ldw = (kn ? a.w.row_stride : a.w.col_stride) * wbits / 8;
-    p.scale = (const uint16_t*)a.scale.ptr; p.offset = (const uint16_t*)a.offset;
     p.s_rs = a.scale.row_stride; p.s_cs = a.scale_n == 1 ? 0 : a.scale.col_stride;
-    p.M = a.M; p.N = a.N; p.K = a.K;
+    p.M = a.M; p.K = a.K;
     p.group = a.group > 0 ? a.group : a.K;
     p.group_shift = (p.group & (p.group - 1)) == 0 ? __builtin_ctzll((unsigned long long)p.group) : p.group >= p.K ? 31 : -1;
     const bool f16 = a.x_dtype == DT_F16;
-    int rc;
-    if (f16) {
-        if (wbits == 4) rc = a.offset ? launch_dequant<DT_F16, 4, true>(p, kn, w16, st) : launch_dequant<DT_F16, 4, false>(p, kn, w16, st);
-        else rc = a.offset ? launch_dequant<DT_F16, 8, true>(p, kn, w16, st) : launch_dequant<DT_F16, 8, false>(p, kn, w16, st);
-    } else {
-        if (wbits == 4) rc = a.offset ? launch_dequant<DT_BF16, 4, true>(p, kn, w16, st) : launch_dequant<DT_BF16, 4, false>(p, kn, w16, st);
-        else rc = a.offset ? launch_dequant<DT_BF16, 8, true>(p, kn, w16, st) : launch_dequant<DT_BF16, 8, false>(p, kn, w16, st);
+    const int bias_bytes = a.bias_dtype == DT_F32 ? 4 : 2;
+    for (int64_t i = 0; i < pl.strips; i++) {
+        const int64_t n0 = i * pl.strip;
+        p.N = i + 1 < pl.strips ? pl.strip : a.N - n0;
+        p.w = (const uint8_t*)a.w.ptr + (kn ? n0 * wbits / 8 : n0 * p.ldw);
+        p.scale = (const uint16_t*)a.scale.ptr + n0 * p.s_cs;
+        p.offset = a.offset ? (const uint16_t*)a.offset + n0 * p.s_cs : nullptr;
+        int rc;
+        if (f16) {
+            if (wbits == 4) rc = a.offset ? launch_dequant<DT_F16, 4, true>(p, kn, w16, st) : launch_dequant<DT_F16, 4, false>(p, kn, w16, st);
+            else rc = a.offset ? launch_dequant<DT_F16, 8, true>(p, kn, w16, st) : launch_dequant<DT_F16, 8, false>(p, kn, w16, st);
+        } else {
+            if (wbits == 4) rc = a.offset ? launch_dequant<DT_BF16, 4, true>(p, kn, w16, st) : launch_dequant<DT_BF16, 4, false>(p, kn, w16, st);
+            else rc = a.offset ? launch_dequant<DT_BF16, 8, true>(p, kn, w16, st) : launch_dequant<DT_BF16, 8, false>(p, kn, w16, st);
+        }
+        if (rc != 0) return rc;
+        QgemmParams g{};
+        g.a = (const int8_t*)a.x; g.b = (const int8_t*)w16;
+        g.lda = 2 * a.K; g.ldb = 2 * a.K; g.KB = 2 * a.K;
+        g.out = (uint16_t*)a.y + n0; g.M = a.M; g.N = p.N; g.ldc = a.N;
+        g.bias = a.bias ? (const char*)a.bias + n0 * bias_bytes : nullptr; g.bias_dt = a.bias_dtype;
+        rc = launch_gemm16(g, i + 1 < pl.strips ? pl.full : pl.last, !f16, 1, a.x_dtype, (float*)((char*)a.workspace + pl.weight_bytes), st);
+        if (rc != 0) return rc;
     }
-    if (rc != 0) return rc;
-    QgemmParams g{};
-    g.a = (const int8_t*)a.x; g.b = (const int8_t*)w16;
-    g.lda = 2 * a.K; g.ldb = 2 * a.K; g.KB = 2 * a.K;
-    g.out = a.y; g.M = a.M; g.N = a.N; g.ldc = a.N;
-    g.bias = a.bias; g.bias_dt = a.bias_dtype;
-    return launch_gemm16(g, pl, !f16, 1, a.x_dtype, (float*)((char*)a.workspace + dense_weight_bytes(a)), st);
+    return 0;
 }
 
 }  // namespace opsnn

@@ -36,3 +36,36 @@ def test_more_columns_than_a_grid_dimension_holds(gpu):
     inp = cases.make_wq_inputs(m, M, K, N, 9, m.ACL_FLOAT16, m.ACL_INT4, 0, True, False, None)
     print(f"case dense M={M} K={K} N={N}", flush=True)
     _b16_bar(cases.run_wq_aclnn(m, inp, M, K, N), cases.oracle_wq(m, inp, M, K, N), orc.F16, "dense, wide", K)
+
+
+@pytest.mark.parametrize("M,K,N,w_dt,x_dt,group,tW,off,bias", [(66, 16384, 33000, "i8", "bf16", 0, False, True, True), (300, 16384, 33003, "i4", "f16", 128, True, True, False),
+                                                               (520, 16384, 34000, "i4", "bf16", 64, False, False, True)])
+def test_column_strips(gpu, M, K, N, w_dt, x_dt, group, tW, off, bias):
+    """A weight of more than 1 GiB in 16 bits goes in strips of whole 256 columns: the columns at both ends and on both sides of every
+    place where a strip can end."""
+    import numpy as np
+    m = gpu
+    xd, od = (m.ACL_FLOAT16, orc.F16) if x_dt == "f16" else (m.ACL_BF16, orc.BF16)
+    inp = cases.make_wq_inputs(m, M, K, N, M, xd, m.ACL_INT4 if w_dt == "i4" else m.ACL_INT8, group, tW, off, xd if bias else None)
+    print(f"case strips M={M} K={K} N={N} {w_dt} {x_dt} tW={tW}", flush=True)
+    got = cases.run_wq_aclnn(m, inp, M, K, N)
+    at = np.unique(np.concatenate([np.arange(0, 24), (np.arange(256, N - 1, 256)[:, None] + np.arange(-2, 2)).ravel(), np.arange(N - 25, N)]))
+    at = np.unique(np.concatenate([at & ~1, at | 1]))   # whole pairs of columns
+    at = at[at < N - N % 2]
+    G = -(-K // group) if group else 1
+    sub = dict(inp)
+    if tW:
+        sub["w"] = np.ascontiguousarray(inp["w"].reshape(N, -1)[at])
+    elif w_dt == "i4":
+        sub["w"] = np.ascontiguousarray(inp["w"].reshape(K, N // 2)[:, at[::2] // 2])
+    else:
+        sub["w"] = np.ascontiguousarray(inp["w"].reshape(K, N)[:, at])
+    for k in ("scale", "offset"):
+        if inp[k] is not None:
+            v = inp[k].reshape((N, G) if tW else (G, N))
+            sub[k] = np.ascontiguousarray(v[at] if tW else v[:, at])
+    if bias:
+        sub["bias"] = np.ascontiguousarray(inp["bias"][at])
+    rows = np.linspace(0, M - 1, 40).astype(int)
+    want = cases.oracle_wq(m, sub, M, K, len(at), rows=rows)
+    _b16_bar(np.ascontiguousarray(got[rows][:, at]), want, od, "strips", K)

@@ -196,3 +196,11 @@ def test_kn_storage_leaves_room_for_the_cached_copys_k_split():
         M, N = M + 64, N + N % 2
         nk = m.lib().opsnnWqmmWorkspace(C.byref(_wq_args(M, N, K, group, wbits, m.ACL_FLOAT16, ALIGNED, True)))
         assert m.lib().opsnnWqmmWorkspace(C.byref(_wq_args(M, N, K, group, wbits, m.ACL_FLOAT16, ALIGNED, False))) >= nk, (M, N, K, group, wbits)
+
+
+@pytest.mark.parametrize("nk", [True, False])
+def test_dequantised_weight_is_bounded(nk):
+    """The 16-bit weight that many rows are multiplied with takes 1 GiB of workspace at most (beside a K split's partial sums)."""
+    for M, N, K in ((600, 152064, 8192), (2048, 57344, 8192), (300, 70000, 8192), (65, 1 << 20, 1024)):
+        ws = m.lib().opsnnWqmmWorkspace(C.byref(_wq_args(M, N, K, 64, 4, m.ACL_BF16, ALIGNED, nk)))
+        assert 0 < ws <= (1 << 30) + 256 * K * 2 + 16 * 4 * M * min(N, (1 << 30) // (2 * K) + 256), (M, N, K, ws)
