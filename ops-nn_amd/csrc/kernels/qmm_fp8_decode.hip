@@ -432,8 +432,8 @@ int launch_mxw4_one(const MxW4DecParams& p, hipStream_t st, int splits = 1)
 // ---- MXFP8: fp8 e4m3 x fp8 e4m3 with e8m0 scales per 32 elements of K on both operands (the MX mode of
 // quant_batch_matmul_v4, qbmmv4_kernel_golden.py:119-186), up to 16 rows of x1 per pass ----
 // The stream of fp8_block_decode_kernel with the scales folded into the widening conversion: an e4m3 value times a power of
-// two is a bf16 value (v_cvt_scalef32_pk_bf16_fp8 with the scale 2^(byte - 127): exact wherever fp32 itself would hold the
-// scaled value), the product of two bf16 values is an fp32 value, and v_mfma_f32_16x16x32_bf16 sums such products in fp32
+// two is a bf16 value (v_cvt_scalef32_pk_bf16_fp8 with the scale 2^(byte - 127): exact from byte 3 on; below, the smallest codes
+// are rounded to bf16's subnormal spacing of 2^-133), the product of two bf16 values is an fp32 value, and v_mfma_f32_16x16x32_bf16 sums such products in fp32
 // -- one chain over the wave's whole K range, no fold per block.  A lane's 16-byte piece lies inside one 32-element block,
 // so one scale byte serves it; x2's scale bytes arrive as words of four (128 elements) per row: lane (row, q) fetches word
 // 4 i + q of the wave's range and the word of chunk c comes over from lane (row, (c / 2) % 4).  K segments and idle

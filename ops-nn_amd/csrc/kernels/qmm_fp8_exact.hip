@@ -92,7 +92,8 @@ template <bool E5> __device__ __forceinline__ v8h widen8(int d0, int d1)
 }
 
 // the MX form: two of a dword's four e4m3 codes -> bf16 with the power of two `sc` multiplied in (the bits of a bf16 pair, carried
-// in the fp16 vector type of the other forms): exact wherever fp32 itself would hold the scaled value
+// in the fp16 vector type of the other forms): exact from scale byte 3 on; with the bytes 0 to 2 a small code's value can lie between
+// two subnormal bf16 values (multiples of 2^-133) and is rounded to the nearest
 template <bool HI> __device__ __forceinline__ v2h cvt_mx(uint32_t d, float sc) { return __builtin_bit_cast(v2h, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(d, sc, HI)); }
 __device__ __forceinline__ v8h widen8_scaled(int d0, int d1, float sc)
 {
@@ -733,8 +734,8 @@ uint64_t mx_exact_bytes(const OpsnnQmmArgs& a)
     return up256(rows * 8) + up256(((rows + 63) / 64 + 2) * 4);
 }
 
-// MXFP8 with exact products, one launch: an e4m3 value times the power of two of its block is a bf16 value wherever fp32 itself
-// would hold it, so both operands are widened to bf16 with their block's scale as the conversion's scale operand and
+// MXFP8 with exact products, one launch: an e4m3 value times the power of two of its block is a bf16 value (scale bytes 0 to 2 aside,
+// cvt_mx), so both operands are widened to bf16 with their block's scale as the conversion's scale operand and
 // v_mfma_f32_16x16x32_bf16 sums exact products in fp32 -- the arithmetic of mx8_decode_kernel.  (Widened to fp16 the scaled
 // values need a base per row: two passes over the scale tables in front and a gated launch of the scaled-instruction kernel
 // behind, for rows whose scales spread too far -- 42 us of the 215 us that 500 x 8192 x 8192 took.)  `a`: both operands e4m3,

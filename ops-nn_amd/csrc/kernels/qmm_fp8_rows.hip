@@ -146,8 +146,8 @@ int launch_rowcol_rows(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
 
 // ---- MXFP8 (e8m0 scales per 32 elements of K on both operands) with 17 .. 128 rows of x1 ----
 // The many-rows kernel in its weight-only form for e4m3 codes with e8m0 group scales and bf16 activations: a pre-step widens
-// x1 to bf16 with its block scales folded in (an e4m3 value times a power of two is a bf16 value wherever fp32 would hold
-// it: M * K * 2 bytes of workspace), the kernel widens x2's codes the same way (T(w * s) is exact) and
+// x1 to bf16 with its block scales folded in (an e4m3 value times a power of two is a bf16 value from scale byte 3 on,
+// below that rounded to bf16's subnormal spacing: M * K * 2 bytes of workspace), the kernel widens x2's codes the same way (T(w * s) is exact) and
 // v_mfma_f32_16x16x32_bf16 sums exact products in fp32 -- the arithmetic of mx8_decode_kernel (qmm_fp8_decode.hip).
 int launch_wq_mx8_rows(const WqParams& p, hipStream_t st);   // wqmm.hip
 

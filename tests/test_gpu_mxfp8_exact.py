@@ -1,5 +1,5 @@
-"""MXFP8 on the tile kernel that widens both operands to bf16 with their block scales: the ends of the e8m0 range, rows whose
-scales spread over the whole fp32 range, a NaN scale, a K split, and the second kernel of a split at every alignment of N."""
+"""MXFP8 on the kernels that widen both operands to bf16 with their block scales: rows with some scales up to 60 binades below the
+others, a NaN scale, a K split, the second kernel of a split at every alignment of N, and the whole e8m0 range on single products."""
 import numpy as np
 import pytest
 
@@ -40,3 +40,46 @@ def test_mxfp8_nan_scale_stays_in_its_row(gpu, M, K, N):
     keep[5], keep[:, 9] = False, False
     assert np.isfinite(got[keep]).all()
     assert np.mean(np.abs(got[keep] - want[keep])) <= 1e-3 * np.mean(np.abs(want[keep]))
+
+
+def _e4m3_values():
+    b = np.arange(256)
+    e, m = (b >> 3) & 15, b & 7
+    v = np.where(e == 0, m * 2.0 ** -9, (8 + m) * 2.0 ** (e - 10.0))
+    return np.where(b & 128, -v, v)   # (0x7f and 0xff are NaN and not drawn)
+
+
+@pytest.mark.parametrize("M", [16, 64, 300])
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+@pytest.mark.parametrize("lo1,hi1,lo2,hi2", [(0, 2, 200, 245), (3, 12, 100, 245), (0, 245, 0, 245), (236, 245, 0, 2)])
+def test_mxfp8_single_products_over_the_e8m0_range(gpu, M, out, lo1, hi1, lo2, hi2):
+    """One element of x1 per row is not zero, so every output is one product, which has to be exact.  Both operands are widened to
+    bf16: exact from scale byte 3 on; for the bytes 0 to 2 the smallest codes lie between bf16's subnormal values (multiples of
+    2^-133) and are rounded to the nearest.  (Bytes up to 245: no value beyond fp32.  Products below fp32's normal range aside.)"""
+    m = gpu
+    K, N = 256, 320
+    rng = np.random.default_rng(M + lo1)
+    vals = _e4m3_values()
+    codes = np.array([b for b in range(256) if b & 127 != 127], np.uint8)
+    x2 = rng.choice(codes, (1, N, K)).astype(np.uint8)
+    s1 = rng.integers(lo1, hi1 + 1, (1, M, K // 64, 2)).astype(np.uint8)
+    s2 = rng.integers(lo2, hi2 + 1, (1, N, K // 64, 2)).astype(np.uint8)
+    k, c = rng.integers(0, K, M), rng.choice(codes, M)
+    x1 = np.zeros((1, M, K), np.uint8)
+    x1[0, np.arange(M), k] = c
+
+    def widened(code, byte):
+        return np.round(np.ldexp(vals[code], byte.astype(np.int64) - 127 + 133)) * 2.0 ** -133   # (round: to even, as the conversion)
+    a = widened(c, s1.reshape(M, K // 32)[np.arange(M), k // 32])
+    b = widened(x2[0][:, k], s2.reshape(N, K // 32)[:, k // 32])          # [N, M]
+    want = (a[None, :] * b).T
+    with np.errstate(over="ignore"):
+        want32 = want.astype(np.float32)
+    print(f"case mxfp8 range M={M} {out} s1 {lo1}..{hi1} s2 {lo2}..{hi2}", flush=True)
+    got = cases.run_mx_aclnn(m, dict(x1=x1, x2=x2, s1=s1, s2=s2, fp4=False), M, K, N, True, m.ACL_FLOAT if out == "f32" else m.ACL_BF16)[0]
+    normal = np.abs(want) >= 2.0 ** -126
+    assert normal.mean() > 0.3
+    if out == "f32":
+        assert np.array_equal(got[normal], want32[normal])
+    else:
+        assert np.array_equal(got[normal], orc.f32_to_b16(want32, m.ACL_BF16)[normal])
