@@ -7,18 +7,18 @@ namespace opsnn {
 
 // How a [M, K] x [N, K] product of 16-bit operands is tiled.  cfg: 8 .. 11 the four-wave kernel with 256 x 32*cfg tiles
 // (qmm_int8_wide.hip), else the OPSNN_VARIANT_I8_* tile of that number.  splits > 1: K split over workgroups, fp32 partial sums
-// [splits][batch][M][N].  us: the estimate that the choice rests on.
+// [splits][M][N].  us: the estimate that the choice rests on.
 struct Gemm16Plan {
     int cfg = OPSNN_VARIANT_I8_128, splits = 1;
     double us = 0;
 };
-Gemm16Plan gemm16_plan(int64_t M, int64_t N, int64_t K, int64_t batch);
-inline uint64_t gemm16_part_bytes(const Gemm16Plan& pl, int64_t M, int64_t N, int64_t batch)
+Gemm16Plan gemm16_plan(int64_t M, int64_t N, int64_t K);
+inline uint64_t gemm16_part_bytes(const Gemm16Plan& pl, int64_t M, int64_t N)
 {
-    return pl.splits > 1 ? ((uint64_t)pl.splits * (uint64_t)batch * (uint64_t)M * (uint64_t)N * 4 + 255) / 256 * 256 : 0;
+    return pl.splits > 1 ? ((uint64_t)pl.splits * (uint64_t)M * (uint64_t)N * 4 + 255) / 256 * 256 : 0;
 }
-// p: a / b with strides in bytes, KB = 2 K, K % 64 == 0, out [batch, M, N] with ldc = N; x1s / x2s / bias as in QgemmParams
-// (each may be null).  `part`: gemm16_part_bytes of the plan.
-int launch_gemm16(QgemmParams p, const Gemm16Plan& pl, bool bf16_operands, int64_t batch, int out_dt, float* part, hipStream_t st);
+// p: a / b with strides in bytes, KB = 2 K, K % 64 == 0, out [M, N] of the operands' type with row pitch ldc, a floating bias (may be
+// null).  `part`: gemm16_part_bytes of the plan.
+int launch_gemm16(QgemmParams p, const Gemm16Plan& pl, bool bf16, float* part, hipStream_t st);
 
 }  // namespace opsnn

@@ -4,7 +4,7 @@
 //   MODE_I8     int8 x int8 -> int32 (v_mfma_i32_32x32x32_i8), per-token / per-channel dequant epilogue
 //   MODE_MXFP4  fp4 e2m1 x fp4 e2m1 with e8m0 scales per 32 K (v_mfma_scale_f32_32x32x64_f8f6f4), bias epilogue
 //   MODE_MXFP8  fp8 e4m3 x fp8 e4m3 with e8m0 scales per 32 K (same instruction, 8-bit formats)
-//   MODE_F16, MODE_BF16  16-bit floating operands (v_mfma_f32_32x32x16_{f16,bf16}), row / column scale and bias epilogue
+//   MODE_F16, MODE_BF16  16-bit floating operands (v_mfma_f32_32x32x16_{f16,bf16}), bias epilogue, output of the operands' type
 // Both operands are K-contiguous ("x2 stored [N, K]") with 16-byte aligned rows.  Everything is addressed in
 // BYTES of the packed operand rows, so int8 and fp4 share all data movement (32 bytes of K per row per MFMA)
 // and fp8 uses 64.
@@ -91,7 +91,7 @@ template <int MODE, int BM, int BN, int BK, int WGM, int WGN, int STAGES, int MI
 __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams p, int tiles_m, int tiles_n)
 {
     static_assert(!SPLIT || !KTAIL, "the K split: whole K tiles");
-    constexpr bool MX = mode_is_mx(MODE), E16 = mode_is_16(MODE);
+    constexpr bool MX = mode_is_mx(MODE);
     constexpr int NT = WGM * WGN * 64;
     constexpr int CPR = BK / 16;                 // 16-byte chunks per LDS row
     constexpr int RPW = 16 / CPR;                // rows per 256-byte LDS bank wrap
@@ -507,9 +507,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
         for (int i = tid; i < BN; i += NT) {
             int64_t n = n0 + i;
             if (n >= p.N) n = p.N - 1;
-            if constexpr (E16) {
-                sS2[i] = p.x2s ? load_scalar_as_f32(p.x2s, p.x2s_dt, p.x2s_len == 1 ? 0 : n) : 1.0f;
-            } else if constexpr (MODE == MODE_I8) {
+            if constexpr (MODE == MODE_I8) {
                 const int64_t si = p.x2s_len == 1 ? 0 : n;
                 float sv = p.x2s_dt == DT_U64 ? u2f((uint32_t)((const uint64_t*)p.x2s)[si]) : load_scalar_as_f32(p.x2s, p.x2s_dt, si);
                 if (p.x2s_trunc || p.x2s_dt == DT_U64) sv = u2f(f2u(sv) & 0xFFFFE000u);
@@ -518,11 +516,11 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
             }
             sFb[i] = has_fb ? load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + n) : -0.0f;
         }
-        if constexpr (MODE == MODE_I8 || E16) {
+        if constexpr (MODE == MODE_I8) {
             for (int i = tid; i < BM; i += NT) {
                 int64_t m = m0 + i;
                 if (m >= p.M) m = p.M - 1;
-                sS1[i] = p.x1s ? p.x1s[E16 && p.x1s_one ? 0 : m] : 1.0f;
+                sS1[i] = p.x1s ? p.x1s[m] : 1.0f;
             }
         }
     }
@@ -651,7 +649,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
     for (int j = 0; j < FM; j++) {
         const int ml = wm * TM + j * 32 + frow;
         float s1 = 1.0f;
-        if constexpr (MODE == MODE_I8 || E16) s1 = sS1[ml];
+        if constexpr (MODE == MODE_I8) s1 = sS1[ml];
 #pragma unroll
         for (int i = 0; i < FN; i++) {
 #pragma unroll
@@ -660,15 +658,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
                 const int nl = wn * TN + nw;
                 const v4f fbv = *(const v4f*)(sFb + nl);
                 v4f v;
-                if constexpr (E16) {
-                    const v4f s2 = *(const v4f*)(sS2 + nl);
-#pragma unroll
-                    for (int e = 0; e < 4; e++) {
-                        float tv = acc[i][j][q * 4 + e] * s2[e];
-                        tv = tv * s1;
-                        v[e] = tv + fbv[e];
-                    }
-                } else if constexpr (MODE == MODE_I8) {
+                if constexpr (MODE == MODE_I8) {
                     const v4f s2 = *(const v4f*)(sS2 + nl);
                     const v4i ib = *(const v4i*)(sIb + nl);
 #pragma unroll
@@ -841,7 +831,8 @@ static int qgemm_launch(const QgemmParams& p, int64_t batch, int out_dt, hipStre
     if constexpr (mode_is_mx(MODE)) {
         if (out_dt == DT_F32) return qgemm_launch_one<MODE, BM, BN, BK, WGM, WGN, STAGES, MINWG, false, DT_F32>(p, batch, st);
     }
-    return bf ? qgemm_launch_one<MODE, BM, BN, BK, WGM, WGN, STAGES, MINWG, false, DT_BF16>(p, batch, st)
+    if constexpr (mode_is_16(MODE)) return qgemm_launch_one<MODE, BM, BN, BK, WGM, WGN, STAGES, MINWG, false, MODE == MODE_BF16 ? DT_BF16 : DT_F16>(p, batch, st);
+    else return bf ? qgemm_launch_one<MODE, BM, BN, BK, WGM, WGN, STAGES, MINWG, false, DT_BF16>(p, batch, st)
               : qgemm_launch_one<MODE, BM, BN, BK, WGM, WGN, STAGES, MINWG, false, DT_F16>(p, batch, st);
 }
 

@@ -402,6 +402,7 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
 
     // Epilogue.  acc[i][j][r] is out[m = m_base + 16j + lane%16][n = n_base + 16i + 4*(lane/16) + r].  Per-row and
     // per-column terms are first widened to fp32 in LDS (absent terms are the neutral elements 1.0f, 0 and -0.0f).
+    constexpr bool E16 = EL == EL_F16 || EL == EL_BF16;   // (a floating bias is all there is)
     float* sS2 = (float*)smem;
     float* sFb = sS2 + BN;
     int32_t* sIb = (int32_t*)(sFb + BN);
@@ -414,7 +415,7 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
             if (n >= p.N) n = p.N - 1;
             const int64_t si = p.x2s_len == 1 ? 0 : n;
             float sv = 1.0f;
-            if (!MXS && (EL == EL_I8 || EL == EL_F8 || p.x2s)) {
+            if (!MXS && !E16) {
                 sv = p.x2s_dt == DT_U64 ? u2f((uint32_t)((const uint64_t*)p.x2s)[si]) : load_scalar_as_f32(p.x2s, p.x2s_dt, si);
                 if (p.x2s_trunc || p.x2s_dt == DT_U64) sv = u2f(f2u(sv) & 0xFFFFE000u);
             }
@@ -422,7 +423,7 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
             sIb[i] = has_ib ? ((const int32_t*)p.bias)[bz * p.bias_bs + n] : 0;
             sFb[i] = has_fb ? load_scalar_as_f32(p.bias, p.bias_dt, bz * p.bias_bs + n) : -0.0f;
         }
-        for (int i = tid; i < BM; i += NT) {
+        for (int i = tid; i < BM && !E16; i += NT) {
             int64_t m = m0 + i;
             if (m >= p.M) m = p.M - 1;
             sS1[i] = p.x1s ? p.x1s[p.x1s_one ? 0 : m] : 1.0f;
@@ -508,7 +509,7 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
     const bool vec_ok = (p.ldc % 4) == 0 && ((uintptr_t)p.out % 8) == 0;
 #pragma unroll
     for (int j = 0; j < FM; j++) {
-        const float s1 = sS1[wm * TM + j * 16 + frow];
+        const float s1 = E16 ? 1.0f : sS1[wm * TM + j * 16 + frow];
         const int64_t m = m0 + wm * TM + j * 16 + frow;
 #pragma unroll
         for (int i = 0; i < FN; i++) {
@@ -522,8 +523,10 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
                 float tv;
                 if constexpr (EL != EL_I8) tv = acc[i][j][e];
                 else tv = (float)(acc[i][j][e] + ib[e]);
-                tv = tv * s2[e];
-                tv = tv * s1;
+                if constexpr (!E16) {
+                    tv = tv * s2[e];
+                    tv = tv * s1;
+                }
                 v[e] = tv + fbv[e];
             }
             const v4us o4 = pack4_b16<OUT_DT>(v);
@@ -626,24 +629,23 @@ int launch_mxfp8_wide(const QgemmParams& p, int fn, int64_t batch, int out_dt, h
 
 namespace opsnn {
 
-// fp16 x fp16 or bf16 x bf16 (both operands K-contiguous, KB = 2 K bytes, K % 64 == 0), 16-bit output, epilogue as for fp8:
-// p.x1s / p.x2s (either may be null: no scale) and a floating bias.
+// fp16 x fp16 or bf16 x bf16 (both operands K-contiguous, KB = 2 K bytes, K % 64 == 0), a floating bias, output of the operands' type.
 template <int EL>
-static int launch_16_wide_el(const QgemmParams& p, int fn, int64_t batch, bool bf, hipStream_t st)
+static int launch_16_wide_el(const QgemmParams& p, int fn, hipStream_t st)
 {
+    constexpr int DT = EL == EL_BF16 ? DT_BF16 : DT_F16;
     switch (fn) {
-        case 8: return bf ? launch_wide_one<8, DT_BF16, EL>(p, batch, st) : launch_wide_one<8, DT_F16, EL>(p, batch, st);
-        case 9: return bf ? launch_wide_one<9, DT_BF16, EL>(p, batch, st) : launch_wide_one<9, DT_F16, EL>(p, batch, st);
-        case 10: return bf ? launch_wide_one<10, DT_BF16, EL>(p, batch, st) : launch_wide_one<10, DT_F16, EL>(p, batch, st);
-        case 11: return bf ? launch_wide_one<11, DT_BF16, EL>(p, batch, st) : launch_wide_one<11, DT_F16, EL>(p, batch, st);
+        case 8: return launch_wide_one<8, DT, EL>(p, 1, st);
+        case 9: return launch_wide_one<9, DT, EL>(p, 1, st);
+        case 10: return launch_wide_one<10, DT, EL>(p, 1, st);
+        case 11: return launch_wide_one<11, DT, EL>(p, 1, st);
         default: return OPSNN_NOT_TAKEN;
     }
 }
-int launch_16_wide(const QgemmParams& p, int fn, bool bf16_operands, int64_t batch, int out_dt, hipStream_t st)
+int launch_16_wide(const QgemmParams& p, int fn, bool bf16, hipStream_t st)
 {
     if (p.KB % 128 != 0 || p.KB < 128) return OPSNN_NOT_TAKEN;
-    if (out_dt != DT_BF16 && out_dt != DT_F16) return OPSNN_NOT_TAKEN;
-    return bf16_operands ? launch_16_wide_el<EL_BF16>(p, fn, batch, out_dt == DT_BF16, st) : launch_16_wide_el<EL_F16>(p, fn, batch, out_dt == DT_BF16, st);
+    return bf16 ? launch_16_wide_el<EL_BF16>(p, fn, st) : launch_16_wide_el<EL_F16>(p, fn, st);
 }
 
 }  // namespace opsnn

@@ -122,11 +122,11 @@ static DensePlan dense_plan(int64_t M, int64_t N, int64_t K)
         if (d.strip < 256 && d.strip < N) d.strip = 256;
         d.strips = (N + d.strip - 1) / d.strip;
         const int64_t rest = N - (d.strips - 1) * d.strip;
-        d.last = gemm16_plan(M, rest, K, 1);
-        d.full = rest == d.strip ? d.last : gemm16_plan(M, d.strip, K, 1);
+        d.last = gemm16_plan(M, rest, K);
+        d.full = rest == d.strip ? d.last : gemm16_plan(M, d.strip, K);
         d.us = (double)(d.strips - 1) * (d.full.us + 5.0) + d.last.us;
         d.weight_bytes = ((uint64_t)d.strip * (uint64_t)K * 2 + 255) / 256 * 256;
-        const uint64_t pa = d.strips > 1 ? gemm16_part_bytes(d.full, M, d.strip, 1) : 0, pb = gemm16_part_bytes(d.last, M, rest, 1);
+        const uint64_t pa = d.strips > 1 ? gemm16_part_bytes(d.full, M, d.strip) : 0, pb = gemm16_part_bytes(d.last, M, rest);
         d.part_bytes = pa > pb ? pa : pb;
         if (d.us < best.us) best = d;
         if (most >= N) break;
@@ -272,7 +272,7 @@ int launch_wq_dense(const OpsnnWqmmArgs& a, hipStream_t st)
         g.lda = 2 * a.K; g.ldb = 2 * a.K; g.KB = 2 * a.K;
         g.out = (uint16_t*)a.y + n0; g.M = a.M; g.N = p.N; g.ldc = a.N;
         g.bias = a.bias ? (const char*)a.bias + n0 * bias_bytes : nullptr; g.bias_dt = a.bias_dtype;
-        rc = launch_gemm16(g, i + 1 < pl.strips ? pl.full : pl.last, !f16, 1, a.x_dtype, (float*)((char*)a.workspace + pl.weight_bytes), st);
+        rc = launch_gemm16(g, i + 1 < pl.strips ? pl.full : pl.last, !f16, (float*)((char*)a.workspace + pl.weight_bytes), st);
         if (rc != 0) return rc;
     }
     return 0;

@@ -144,28 +144,7 @@ __global__ __launch_bounds__(256, 2) void wq_kn_kernel(WqParams p, int splits)
         if constexpr (PF == 3) { if (st + 2 < w1) step(I2{}, st + 2); }
     }
 
-    // the four waves' sums in a fixed order: (0 + 2) + (1 + 3)
-    constexpr int SUMS = CPL * MB * 4 * 64;
-    auto park = [&](float* to) {
-#pragma unroll
-        for (int c = 0; c < CPL; c++)
-#pragma unroll
-            for (int b = 0; b < MB; b++) *(v4f*)(to + ((c * MB + b) * 64 + lane) * 4) = acc[c][b];
-    };
-    auto add = [&](const float* from) {
-#pragma unroll
-        for (int c = 0; c < CPL; c++)
-#pragma unroll
-            for (int b = 0; b < MB; b++) acc[c][b] = acc[c][b] + *(const v4f*)(from + ((c * MB + b) * 64 + lane) * 4);
-    };
-    if (wave >= 2) park(red + (wave - 2) * SUMS);
-    __syncthreads();
-    if (wave < 2) add(red + wave * SUMS);
-    __syncthreads();
-    if (wave == 1) park(red);
-    __syncthreads();
-    if (wave != 0) return;
-    add(red);
+    if (!sum_of_four_waves(acc, red, wave, lane)) return;
 
     // acc[c][b][i] is out[m = 16 b + lane % 16][column c of the weight rows' lane 4 q + i]: CPL neighbouring columns per i
 #pragma unroll

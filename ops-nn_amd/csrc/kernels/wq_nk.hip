@@ -159,30 +159,8 @@ __global__ __launch_bounds__(256, 2) void wq_nk_kernel(WqParams p, int splits, i
         if (c + 1 < w1) chunk(I1{}, c + 1);
     }
 
-    // the four waves' sums in a fixed order: (0 + 2) + (1 + 3)
-    float* const red = dyn;
-    constexpr int SUMS = NB * MB * 4 * 64;
-    auto park = [&](float* to) {
-#pragma unroll
-        for (int j = 0; j < NB; j++)
-#pragma unroll
-            for (int b = 0; b < MB; b++) *(v4f*)(to + ((j * MB + b) * 64 + lane) * 4) = acc[j][b];
-    };
-    auto add = [&](const float* from) {
-#pragma unroll
-        for (int j = 0; j < NB; j++)
-#pragma unroll
-            for (int b = 0; b < MB; b++) acc[j][b] = acc[j][b] + *(const v4f*)(from + ((j * MB + b) * 64 + lane) * 4);
-    };
     __syncthreads();   // the scale table makes room
-    if (wave >= 2) park(red + (wave - 2) * SUMS);
-    __syncthreads();
-    if (wave < 2) add(red + wave * SUMS);
-    __syncthreads();
-    if (wave == 1) park(red);
-    __syncthreads();
-    if (wave != 0) return;
-    add(red);
+    if (!sum_of_four_waves(acc, dyn, wave, lane)) return;
 
     // acc[j][b][i] is out[m = 16 b + lane % 16][n = n0 + 16 j + 4 q + i]
 #pragma unroll
