@@ -262,10 +262,10 @@ static int splitk_for(const OpsnnQmmArgs& a, int mode)
     else if (mode == 2 && a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E2M1 && out16) { bm = 256; tile_us = 1.8; }
     else if (mode == 1 && a.x1_dtype == DT_I8 && a.x2_dtype == DT_I8 && a.gsK == 128 && a.gsN == 128 && out16) { bm = a.M >= 512 ? 256 : 128; tile_us = 1.8; }
     // (the exact fp8 kernel)
-    else if (mode == 1 && f8 && a.gsK == 128 && a.gsN == 128 && !a.bias && a.M > 128 && (out16 || a.out_dtype == DT_F32)) return fp8x_plan(a.M, a.N, a.K, a.batch, mode == 3, true).splits;
-    else if (mode == 2 && f8 && (out16 || a.out_dtype == DT_F32)) return fp8x_plan(a.M, a.N, a.K, a.batch, mode == 3, true).splits;
+    else if (mode == 1 && f8 && a.gsK == 128 && a.gsN == 128 && !a.bias && a.M > 128 && (out16 || a.out_dtype == DT_F32)) return fp8x_plan(a.M, a.N, a.K, a.batch, FP8X_BLOCK, true).splits;
+    else if (mode == 2 && f8 && (out16 || a.out_dtype == DT_F32)) return fp8x_plan(a.M, a.N, a.K, a.batch, FP8X_MX, true).splits;
     else if (mode == 3 && (a.x1_dtype == DT_E4M3 || a.x1_dtype == DT_E5M2) && (a.x2_dtype == DT_E4M3 || a.x2_dtype == DT_E5M2) && a.M > 128 &&
-             (out16 || a.out_dtype == DT_F32)) return fp8x_plan(a.M, a.N, a.K, a.batch, mode == 3, true).splits;
+             (out16 || a.out_dtype == DT_F32)) return fp8x_plan(a.M, a.N, a.K, a.batch, FP8X_PLAIN, true).splits;
     else return 1;
     const int64_t tiles = ((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn) * a.batch;
     return splitk_factor(tiles, (a.K + kunit - 1) / kunit, tile_us, a.M * a.N * a.batch, bytes_per_us);

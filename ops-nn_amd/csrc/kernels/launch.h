@@ -85,12 +85,12 @@ struct TilePlan {
 };
 TilePlan tile_plan(int64_t M, int64_t N, int64_t KB, int64_t batch, bool may_split, bool tiles_of_32 = true);
 
-// The tile (OPSNN_VARIANT_FP8X_*) and the K segments of a call on the exact fp8 kernel (qmm_fp8_exact.hip); plain: row / column
-// scales only.
+// The tile (OPSNN_VARIANT_FP8X_*) and the K segments of a call on the exact fp8 kernel (qmm_fp8_exact.hip).
 struct Fp8xPlan {
     int tile, splits;
 };
-Fp8xPlan fp8x_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool plain, bool may_split);
+enum Fp8xForm { FP8X_BLOCK, FP8X_PLAIN, FP8X_MX };   // block scales, row / column scales, MX scales
+Fp8xPlan fp8x_plan(int64_t M, int64_t N, int64_t K, int64_t batch, Fp8xForm form, bool may_split);
 
 // How the x-in-registers kernel (weight-only, up to 16 rows of x) covers K.  A workgroup holds `nw` waves x `nch` chunks
 // (of 64 weight bytes): 16 x 4, 8-bit weights also 16 x 8, or 8 x 4 / 8 x 8.  A K that is exactly one such shape runs on

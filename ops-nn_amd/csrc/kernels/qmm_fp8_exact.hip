@@ -592,11 +592,16 @@ __global__ __launch_bounds__(256) void fp8x_splitk_reduce_kernel(Fp8xParams p, i
 // round of the chip costs a whole round: 333 x 3584 x 18944 ran as 296 tiles of 256 x 128 in two rounds, 96 us (row / column
 // scales; block scales 102, MX 107); 222 of 128 x 256 take 55 (57, 62).  128 x 128 tiles fill the chip where the others are half
 // as many and would be cut along K: 1024 x 4096 x 4096 47 -> 39 us (48 -> 42, 49 -> 43).  The chosen one has the smallest
-// estimate: per K tile t0 + t1 * (share of the CUs at work), 4 us a round beside, fitted to 14 shapes of 140 .. 2048 rows; the
-// row / column form (`plain`) has no scales to apply in its loop.
-Fp8xPlan fp8x_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool plain, bool may_split)
+// estimate: per K tile t0 + t1 * (share of the CUs at work) and a few us a round beside, fitted to 14 shapes of 140 .. 2048 rows
+// (profiles/tile_plans.txt); the row / column form has no scales to apply in its loop.  The MX form's loop starts 4 us later than the
+// others' (the first tile's conversions and scales), and its second kernel has nothing but the sum to do: a short K is cut earlier
+// (129 x 1024 x 1024 16.1 -> 14.3 us, 129 x 1024 x 2080 17.0 -> 14.4 where the many-rows kernel had taken 16.1; 256 x 2048 x 6976 26.3 ->
+// 24.2.  132 x 1152 x 6976 is left at 18.5 against 17.8 there).
+Fp8xPlan fp8x_plan(int64_t M, int64_t N, int64_t K, int64_t batch, Fp8xForm form, bool may_split)
 {
+    const bool plain = form == FP8X_PLAIN, mx = form == FP8X_MX;
     const int64_t cus = 256, kt = (K + 127) / 128;   // (a K tail runs padded)
+    const double round_us = mx ? 8.0 : 4.0, split_us = mx ? 2.0 : 5.0, sums_per_us = mx ? 5.0e6 : 6.0e6;
     Fp8xPlan best{OPSNN_VARIANT_FP8X_256x128, 1};
     double best_us = 1e30;
     auto offer = [&](int tile, int64_t bm, int64_t bn, double t0, double t1) {
@@ -604,8 +609,8 @@ Fp8xPlan fp8x_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool plain, b
         for (int s = 1; s <= 16 && (s == 1 || (may_split && tiles * s <= cus && kt / s >= 4)); s++) {
             const double steps = (double)((kt + s - 1) / s);
             const int64_t full = tiles * s / cus, rest = tiles * s % cus;
-            double us = (double)full * (steps * (t0 + t1) + 4.0) + (rest ? steps * (t0 + t1 * (double)rest / (double)cus) + 4.0 : 0.0);
-            if (s > 1) us += 5.0 + 8.0 * s * (double)M * (double)N * (double)batch / 6.0e6;   // partial sums, second kernel
+            double us = (double)full * (steps * (t0 + t1) + round_us) + (rest ? steps * (t0 + t1 * (double)rest / (double)cus) + round_us : 0.0);
+            if (s > 1) us += split_us + 8.0 * s * (double)M * (double)N * (double)batch / sums_per_us;   // partial sums, second kernel
             if (us < best_us) { best_us = us; best = {tile, s}; }
         }
     };
@@ -652,7 +657,7 @@ static int launch_fp8_exact_tile(const Fp8xParams& p, int64_t batch, hipStream_t
 template <int OUT_DT, bool RC, int FMT = 0, bool MXS = false>
 static int launch_fp8_exact(const Fp8xParams& p, int64_t batch, int force_variant, hipStream_t st)
 {
-    int tile = p.splits > 1 ? p.tile : fp8x_plan(p.M, p.N, p.K, batch, RC && !MXS, false).tile;
+    int tile = p.splits > 1 ? p.tile : fp8x_plan(p.M, p.N, p.K, batch, MXS ? FP8X_MX : RC ? FP8X_PLAIN : FP8X_BLOCK, false).tile;
     if (force_variant >= OPSNN_VARIANT_FP8X_256x128 && force_variant <= OPSNN_VARIANT_FP8X_128x128) tile = force_variant;
     if (256 * p.ldb >= (1ll << 32) || p.s2_cs < 0 || p.s2_cs >= (1ll << 29)) tile = OPSNN_VARIANT_FP8X_256x128;   // (32-bit offsets inside a tile)
     if (tile == OPSNN_VARIANT_FP8X_128x128) return launch_fp8_exact_tile<2, 2, OUT_DT, RC, FMT, MXS>(p, batch, st);
@@ -683,7 +688,7 @@ int launch_blockscale_exact(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
     // by 32-bit offsets from the tile's first row
     if (p.s1_rs < 0 || p.s1_cs < 0 || ((a.M + p.gsM - 1) / p.gsM) * p.s1_rs * 4 >= (1ll << 32)) return OPSNN_NOT_TAKEN;
     if (p.lda < 0 || p.ldb < 0 || 256 * p.lda >= (1ll << 32) || 128 * p.ldb >= (1ll << 32)) return OPSNN_NOT_TAKEN;
-    p.splits = sk.splits; p.part = sk.part; p.tile = sk.splits > 1 ? fp8x_plan(a.M, a.N, a.K, a.batch, false, true).tile : 0;
+    p.splits = sk.splits; p.part = sk.part; p.tile = sk.splits > 1 ? fp8x_plan(a.M, a.N, a.K, a.batch, FP8X_BLOCK, true).tile : 0;
     if (a.out_dtype == DT_BF16) return launch_fp8_exact<DT_BF16, false>(p, a.batch, a.force_variant, st);
     if (a.out_dtype == DT_F32) return launch_fp8_exact<DT_F32, false>(p, a.batch, a.force_variant, st);
     return launch_fp8_exact<DT_F16, false>(p, a.batch, a.force_variant, st);
@@ -711,7 +716,7 @@ int launch_rowcol_exact(const OpsnnQmmArgs& a, hipStream_t st, int ep_mode, Spli
     p.ep_mode = ep_mode;
     p.bias = a.bias; p.bias_dt = a.bias_dtype; p.bias_bs = a.bias_batch_stride;
     if (((uintptr_t)p.a | (uintptr_t)p.b | (uint64_t)p.lda | (uint64_t)p.ldb | (uint64_t)p.a_bs | (uint64_t)p.b_bs) % 16) return OPSNN_NOT_TAKEN;
-    p.splits = sk.splits; p.part = sk.part; p.tile = sk.splits > 1 ? fp8x_plan(a.M, a.N, a.K, a.batch, true, true).tile : 0;
+    p.splits = sk.splits; p.part = sk.part; p.tile = sk.splits > 1 ? fp8x_plan(a.M, a.N, a.K, a.batch, FP8X_PLAIN, true).tile : 0;
     const bool bf = a.out_dtype == DT_BF16, f32 = a.out_dtype == DT_F32;
     switch ((e1 ? 1 : 0) | (e2 ? 2 : 0)) {
         case 0: return f32 ? launch_fp8_exact<DT_F32, true, 0>(p, a.batch, a.force_variant, st) : bf ? launch_fp8_exact<DT_BF16, true, 0>(p, a.batch, a.force_variant, st) : launch_fp8_exact<DT_F16, true, 0>(p, a.batch, a.force_variant, st);
@@ -757,7 +762,7 @@ int launch_mx_exact(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
     if (((uintptr_t)p.a | (uintptr_t)p.b | (uint64_t)p.lda | (uint64_t)p.ldb | (uint64_t)p.a_bs | (uint64_t)p.b_bs) % 16) return OPSNN_NOT_TAKEN;
     if (((uintptr_t)p.sa | (uintptr_t)p.sb | (uint64_t)p.sa_rs | (uint64_t)p.sb_rs | (uint64_t)p.sa_bs | (uint64_t)p.sb_bs) % 4) return OPSNN_NOT_TAKEN;
     p.bias = a.bias; p.bias_dt = a.bias_dtype; p.bias_bs = a.bias_batch_stride;
-    p.splits = sk.splits; p.part = sk.part; p.tile = sk.splits > 1 ? fp8x_plan(a.M, a.N, a.K, a.batch, false, true).tile : 0;
+    p.splits = sk.splits; p.part = sk.part; p.tile = sk.splits > 1 ? fp8x_plan(a.M, a.N, a.K, a.batch, FP8X_MX, true).tile : 0;
     return a.out_dtype == DT_F32    ? launch_fp8_exact<DT_F32, true, 0, true>(p, a.batch, a.force_variant, st)
            : a.out_dtype == DT_BF16 ? launch_fp8_exact<DT_BF16, true, 0, true>(p, a.batch, a.force_variant, st)
                                     : launch_fp8_exact<DT_F16, true, 0, true>(p, a.batch, a.force_variant, st);
