@@ -65,7 +65,8 @@ static int launch16(const QgemmParams& p, const Gemm16Plan& pl, hipStream_t st)
 
 // Fewer 256 x 256 tiles than CUs: tile_plan (qmm_int8.hip), whose K tiles of 128 bytes take the same time here -- half as many
 // products per byte at half the rate.  Otherwise the estimate, in microseconds, of the two kernels for large shapes, fitted to
-// one box (random operands, K = 4096 .. 18432):
+// random operands, K = 4096 .. 18432 (profiles/tile_plans.txt: the pass and this product together, 41 calls of 100 .. 1999 rows, 37 within
+// 3 % of the fastest tile, the worst 8 % behind):
 //   four-wave kernel: 0.185 us per 32 columns of tile width and 64-element K tile, 8 us a round beside (4096^3: 99 us in one
 //   round of 256 x 256 tiles = 1.39 Pflop/s; 2048 x 4096 x 11008: 134 us in one round of 256 x 352);
 //   128 x 128 tiles: 0.65 us per K tile alone on a CU, 1.0 us for two that share one, 6 us beside.

@@ -592,11 +592,12 @@ __global__ __launch_bounds__(256) void fp8x_splitk_reduce_kernel(Fp8xParams p, i
 // round of the chip costs a whole round: 333 x 3584 x 18944 ran as 296 tiles of 256 x 128 in two rounds, 96 us (row / column
 // scales; block scales 102, MX 107); 222 of 128 x 256 take 55 (57, 62).  128 x 128 tiles fill the chip where the others are half
 // as many and would be cut along K: 1024 x 4096 x 4096 47 -> 39 us (48 -> 42, 49 -> 43).  The chosen one has the smallest
-// estimate: per K tile t0 + t1 * (share of the CUs at work) and a few us a round beside, fitted to 14 shapes of 140 .. 2048 rows
-// (profiles/tile_plans.txt); the row / column form has no scales to apply in its loop.  The MX form's loop starts 4 us later than the
-// others' (the first tile's conversions and scales), and its second kernel has nothing but the sum to do: a short K is cut earlier
-// (129 x 1024 x 1024 16.1 -> 14.3 us, 129 x 1024 x 2080 17.0 -> 14.4 where the many-rows kernel had taken 16.1; 256 x 2048 x 6976 26.3 ->
-// 24.2.  132 x 1152 x 6976 is left at 18.5 against 17.8 there).
+// estimate: per K tile t0 + t1 * (share of the CUs at work) and a few us a round beside, fitted to 14 shapes of 140 .. 2048 rows;
+// of 45 calls 39 run within 3 % of the fastest tile or ahead of all (K cut), the worst 8 % behind (profiles/tile_plans.txt).  The row /
+// column form has no scales to apply in its loop.  The MX form's loop starts 4 us later than the others' (the first tile's conversions
+// and scales), and its second kernel has nothing but the sum to do: a short K is cut earlier (129 x 1024 x 1024 16.1 -> 14.3 us,
+// 129 x 1024 x 2080 17.0 -> 14.4 where the many-rows kernel had taken 16.1; 256 x 2048 x 6976 26.3 -> 24.2.  132 x 1152 x 6976 is left
+// at 18.5 against 17.8 there).
 Fp8xPlan fp8x_plan(int64_t M, int64_t N, int64_t K, int64_t batch, Fp8xForm form, bool may_split)
 {
     const bool plain = form == FP8X_PLAIN, mx = form == FP8X_MX;

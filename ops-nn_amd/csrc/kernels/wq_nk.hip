@@ -30,10 +30,13 @@ constexpr int nk_nb(int mb) { return mb == 4 ? 4 : 8; }
 static bool nk_plan(int wbits, int64_t M, int64_t N, int64_t K, int64_t group, WqNkPlan& pl)
 {
     pl.mb = M <= 16 ? 1 : M <= 32 ? 2 : 4;
-    // (32-bit: both phases of every call with few rows come here; N and K are below 2^30)
+    // (32-bit: both phases of every call with few rows come here; N and K are below 2^30.  512 below: two workgroups on each of the
+    // chip's 256 CUs, a constant, since phase 1 makes no HIP call)
     const uint32_t cols = 16 * nk_nb(pl.mb), strips = ((uint32_t)N + cols - 1) / cols, kc = (pl.mb == 4 || wbits == 8) ? 64 : 128;
     const uint32_t chunks = ((uint32_t)K + kc - 1) / kc;
-    // (a chunk: 8 KB of codes per wave; four row blocks: 2 KB of 4-bit, 4 KB of 8-bit codes; eight waves of a CU at 5 TB/s)
+    // (a chunk: 8 KB of codes per wave; four row blocks: 2 KB of 4-bit, 4 KB of 8-bit codes; eight waves of a CU at 5 TB/s.  Of 24
+    // calls 22 run within 10 % of the fastest count of segments; the worst, 16 x 8224 x 16384 int8, takes 54.6 us with its four and
+    // 40.8 with two: profiles/tile_plans.txt)
     const double t_chunk = pl.mb == 4 ? (wbits == 4 ? 1.4 : 2.0) : pl.mb == 2 ? 4.1 : 3.4;
     const double slice_us = 8.0 * (double)M * (double)N / 4.0e6;
     double best = 1e30;
