@@ -92,8 +92,8 @@ namespace opsnn {
 // The estimates are fitted to a sweep of every tile over 1 .. 1600 rows and weights of 4096 x 4096 to 8192 x 28672: per K tile of
 // 128 bytes t0 + t1 * (share of the CUs at work), c beside, in whole rounds of the chip; the two small tiles share a CU, and
 // time grows with their number from the first that does.  Of 77 calls of 1 .. 1600 rows 59 run within 3 % of the fastest tile or ahead
-of all (K cut), 72 within 10 %; the worst are 333 x 4096 x 4096 18.3 us (64 x 64 tiles: 15.7) and 128 x 4096 x 11008 24.5 (21.9)
-(profiles/tile_plans.txt).  256: the whole chip's CUs, a constant, since phase 1 plans too and makes no HIP call.
+// of all (K cut), 72 within 10 %; the worst are 333 x 4096 x 4096 18.3 us (64 x 64 tiles: 15.7) and 128 x 4096 x 11008 24.5 (21.9)
+// (profiles/tile_plans.txt).  256: the whole chip's CUs, a constant, since phase 1 plans too and makes no HIP call.
 TilePlan tile_plan(int64_t M, int64_t N, int64_t KB, int64_t batch, bool may_split, bool tiles_of_32)
 {
     const int64_t cus = 256, kt = (KB + 127) / 128;
