@@ -168,8 +168,8 @@ static double tile_kernel_us(const OpsnnWqmmArgs& a, const WqForm& f)
 // codes: the many-rows kernel where its shape conditions hold (with groups in [K, N] storage its scale table, and so its
 // 192- and 256-row instances, do not apply); else, from 129 rows, the tile kernel and up to 128 rows the streaming kernel.
 // With groups that are not whole chunks the general kernel is left, which counts where wq_general_counts says so.
-// (Of 368 measured calls 362 go to the faster side or one within 3 % of it: 1999 x 4096 x 11008 bf16 x int4 228 -> 164 us, [K, N] storage 613 -> 162; 1000 x 8192 x 28672 fp16 x int4 stays on the many-rows
-// kernel, 477 against 526; 65 x 4096 x 22896 on the streaming kernel, 54 against 93; 192 x 8192 x 22896 on the tile kernel, 127
+// (Of 368 measured calls 362 go to the faster side or one within 3 % of it (profiles/weight_only_routes.txt): 1999 x 4096 x 11008
+// bf16 x int4 228 -> 164 us, [K, N] storage 613 -> 162; 1000 x 8192 x 28672 fp16 x int4 stays on the many-rows kernel, 477 against 526; 65 x 4096 x 22896 on the streaming kernel, 54 against 93; 192 x 8192 x 22896 on the tile kernel, 127
 // against 230; 128 x 11008 x 4096 in [K, N] storage with the re-layout, 61 against 75.)
 static bool dense_is_faster(const OpsnnWqmmArgs& a, double product_us)
 {

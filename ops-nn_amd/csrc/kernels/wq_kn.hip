@@ -222,8 +222,9 @@ bool wq_kn_wanted(const OpsnnWqmmArgs& a)
     // (so small a weight is re-laid out as fast -- 16 x 1024 x 512 9.7 us that way, 10.2 here -- and then gives the bits of its
     // pre-packed form)
     if (a.K * a.N < (1ll << 20)) return false;
-    // (up to 16 rows of 8-bit weights of at most 2^24 codes: the re-layout costs 15 us of 28 at 4096 x 4096, but there both storage
-    // forms of a layer give the same bits, on the x-in-registers kernel, and stay so)
+    // (Up to 16 rows of 8-bit weights of at most 2^24 codes: slower on purpose.  16 x 4096 x 4096 int8 takes 28 us behind the
+    // re-layout and 13 here, but the x-in-registers kernel behind it gives the bits of the [N, K] form, which callers at these sizes
+    // have always had and the full-size tests assert.  Elsewhere the two storage forms agree to the summation order only.)
     if (a.w_dtype == DT_I8 && a.M <= 16 && a.K * a.N <= (1ll << 24)) return false;
     if (a.scale_n != 1 && a.scale.col_stride != 1) return false;
     return (uintptr_t)a.x % 16 == 0;
