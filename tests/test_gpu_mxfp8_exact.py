@@ -25,6 +25,28 @@ def test_mxfp8_tiles(gpu, M, K, N, spread):
     _b16_bar(got, cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16), orc.BF16, "mxfp8 tiles", K)
 
 
+@pytest.mark.parametrize("M,K,N", [(129, 992, 1024), (129, 1024, 1024), (129, 1024, 2080), (192, 1152, 515), (256, 2048, 6976)])
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+def test_mxfp8_short_k_split(gpu, M, K, N, out):
+    """Around the K of eight tiles of 128 from which the exact kernel's plan may cut it.  Two fp32 sums of the same exact products differ by
+    at most K roundings each, relative to the sum of the terms' magnitudes; the stated bar holds for bf16."""
+    m = gpu
+    inp = cases.make_mx_inputs(m, M, K, N, M + N, True, False, exp_range=4)
+    dt = m.ACL_FLOAT if out == "f32" else m.ACL_BF16
+    print(f"case mxfp8 short K M={M} K={K} N={N} {out}", flush=True)
+    got, want = cases.run_mx_aclnn(m, inp, M, K, N, True, dt), cases.oracle_mx(m, inp, M, K, N, True, dt)
+    if out == "bf16":
+        _b16_bar(got, want, orc.BF16, "mxfp8 short K", K)
+    else:
+        vals = np.abs(_e4m3_values())
+
+        def wide(x, s):
+            e = s.reshape(x.shape[1], -1)[:, : K // 32, None].astype(np.int64) - 127
+            return np.ldexp(vals[x[0] & 127].reshape(x.shape[1], K // 32, 32), e).reshape(x.shape[1], K)
+        terms = wide(inp["x1"], inp["s1"]) @ wide(inp["x2"], inp["s2"]).T
+        assert (np.abs(got.reshape(M, N).astype(np.float64) - want.reshape(M, N)) <= 2 * K * 2.0 ** -24 * terms).all()
+
+
 @pytest.mark.parametrize("M,K,N", [(300, 512, 260), (300, 4096, 256)])
 def test_mxfp8_nan_scale_stays_in_its_row(gpu, M, K, N):
     m = gpu
