@@ -8,9 +8,10 @@
 //   y = int8 / int4: round half to even;  e4m3 / e5m2: the cast rounds
 // HBM-bound: 2 bytes read and 1 (or 1/2) written per element, one pass.  A row lives in registers between the reduction and
 // the quantisation: up to 8 pieces of 8 elements per thread, one wave per row up to 2048 columns, or 4096 with many rows (four rows
-// per workgroup, reduction by lane exchange only), and one workgroup per row up to 16384 (partial results of the four waves
-// through LDS).  Rows that are longer, or whose length is not a multiple of 8, take the two-pass kernel that reads x
-// twice (the second time from cache).
+// per workgroup, reduction by lane exchange only), and one workgroup per row beyond, of 256 threads, or 1024 with few rows and above
+// 16384 columns (partial results of the waves through LDS).  Rows longer than 65536, or whose length is not a multiple of 8, take
+// the two-pass kernel that reads x twice (the second time from cache; 8 x 17536, which used to run there, 46 -> 5.5 us, 1000 x 18432
+// 66.8 -> 16.2).
 #include "common.hip.h"
 #include "launch.h"
 
@@ -45,11 +46,23 @@ __device__ __forceinline__ float x_to_f32(uint32_t h)
     else return f16_to_f32((uint16_t)h);
 }
 
+// The largest value of a wave, in every lane.  Lane exchange by DPP inside rows of 16 and across them (the shuffle's way over
+// the LDS crossbar is some 60 clocks a step).
+template <int CTRL>
+__device__ __forceinline__ float dpp_max(float v)
+{
+    const int o = __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, v), __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false);
+    return fmaxf(v, __builtin_bit_cast(float, o));
+}
 __device__ __forceinline__ float wave_max(float v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
-    return v;
+    v = dpp_max<0x111>(v);   // row_shr:1, 2, 4, 8: lane 15 of each row of 16 has its row's
+    v = dpp_max<0x112>(v);
+    v = dpp_max<0x114>(v);
+    v = dpp_max<0x118>(v);
+    v = dpp_max<0x142>(v);   // row_bcast:15 and 31: lane 63 has the wave's
+    v = dpp_max<0x143>(v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
 // How a row's elements are divided by its scale.  An IEEE division costs about a dozen instructions per element; with the
@@ -109,18 +122,21 @@ __device__ __forceinline__ RowQuant row_params(const DynQuantParams& p, float am
     return r;
 }
 
-// TPR threads per row (64: one wave, 256: the workgroup), pieces of 8 elements held in registers.
-template <int X_DT, int Y_DT, bool ASYM, int TPR>
-__global__ __launch_bounds__(256) void dynamic_quant_rows_kernel(DynQuantParams p)
+// TPR threads per row (64: one wave, 256 or 1024: the workgroup), MAXP pieces of 8 elements per thread held in registers.
+// Few rows leave the chip to one chain of latencies: every piece of a row is requested before the first is looked at (a load under
+// its own test waited for the one before it), a row has as many threads as it has pieces where the rows do not fill the chip, and
+// the lanes' extremes meet by DPP, not through the LDS crossbar.
+template <int X_DT, int Y_DT, bool ASYM, int TPR, int MAXP>
+__global__ __launch_bounds__(TPR < 256 ? 256 : TPR) void dynamic_quant_rows_kernel(DynQuantParams p)
 {
-    constexpr int RPW = 256 / TPR;   // rows per workgroup
-    constexpr int MAXP = 8;
-    __shared__ float red[3][4];
+    constexpr int WG = TPR < 256 ? 256 : TPR, NW = WG / 64;
+    constexpr int RPW = WG / TPR;   // rows per workgroup
+    __shared__ float red[2][NW];
     const int t = threadIdx.x % TPR;
     const int64_t row = (int64_t)blockIdx.x * RPW + threadIdx.x / TPR;
     const int64_t srow = row < p.rows ? smooth_row_of(p, row) : -1;
     const bool live = row < p.rows && srow >= 0;   // whole waves: TPR is a multiple of 64
-    const int64_t pieces = p.cols / 8;
+    const int pieces = (int)(p.cols / 8);
     const uint4* smr = (const uint4*)(p.smooth + (srow > 0 ? srow : 0) * p.cols);
     const uint4* xr = (const uint4*)(p.x + (live ? row : 0) * p.cols);
     uint4 buf[MAXP];
@@ -131,30 +147,35 @@ __global__ __launch_bounds__(256) void dynamic_quant_rows_kernel(DynQuantParams 
         if (p.smooth) v = __fmul_rn(v, x_to_f32<X_DT>((sw[e >> 1] >> (16 * (e & 1))) & 0xffffu));
         return v;
     };
+    // (past the row's end a thread looks at the row's last piece once more: the extremes are the same)
+    auto at = [&](int i) { const int c = i * TPR + t; return c < pieces ? c : pieces - 1; };
+#pragma unroll
+    for (int i = 0; i < MAXP; i++) buf[i] = xr[at(i)];
 #pragma unroll
     for (int i = 0; i < MAXP; i++) {
-        const int64_t c = (int64_t)i * TPR + t;
-        if (live && c < pieces) {
-            buf[i] = xr[c];
-            uint4 sm = make_uint4(0, 0, 0, 0);
-            if (p.smooth) sm = smr[c];
+        uint4 sm = make_uint4(0, 0, 0, 0);
+        if (p.smooth) sm = smr[at(i)];
 #pragma unroll
-            for (int e = 0; e < 8; e++) {
-                const float v = element(buf[i], sm, e);
-                if (ASYM) { vmax = fmaxf(vmax, v); vmin = fminf(vmin, v); }
-                else amax = fmaxf(amax, fabsf(v));
-            }
+        for (int e = 0; e < 8; e++) {
+            const float v = element(buf[i], sm, e);
+            if (ASYM) { vmax = fmaxf(vmax, v); vmin = fminf(vmin, v); }
+            else amax = fmaxf(amax, fabsf(v));
         }
     }
     if (ASYM) { vmax = wave_max(vmax); vmin = -wave_max(-vmin); }
     else amax = wave_max(amax);
-    if constexpr (TPR == 256) {
+    if constexpr (RPW == 1) {
         const int w = threadIdx.x >> 6;
-        if ((threadIdx.x & 63) == 0) { red[0][w] = amax; red[1][w] = vmax; red[2][w] = vmin; }
+        if ((threadIdx.x & 63) == 0) { red[0][w] = ASYM ? vmax : amax; red[1][w] = vmin; }
         __syncthreads();
-        amax = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
-        vmax = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
-        vmin = fminf(fminf(red[2][0], red[2][1]), fminf(red[2][2], red[2][3]));
+        float hi = red[0][0], lo = red[1][0];
+#pragma unroll
+        for (int i = 1; i < NW; i++) {
+            hi = fmaxf(hi, red[0][i]);
+            if (ASYM) lo = fminf(lo, red[1][i]);
+        }
+        amax = vmax = hi;
+        vmin = lo;
     }
     if (!live) return;
     const RowQuant r = row_params<ASYM>(p, amax, vmax, vmin);
@@ -164,7 +185,7 @@ __global__ __launch_bounds__(256) void dynamic_quant_rows_kernel(DynQuantParams 
     }
 #pragma unroll
     for (int i = 0; i < MAXP; i++) {
-        const int64_t c = (int64_t)i * TPR + t;
+        const int c = i * TPR + t;
         if (c < pieces) {
             uint4 sm = make_uint4(0, 0, 0, 0);
             if (p.smooth) sm = smr[c];
@@ -226,22 +247,41 @@ __global__ __launch_bounds__(256) void dynamic_quant_two_pass_kernel(DynQuantPar
     }
 }
 
+template <int X_DT, int Y_DT, bool ASYM, int TPR, int MAXP>
+static int launch_quant_rows(const DynQuantParams& p, hipStream_t st)
+{
+    constexpr int WG = TPR < 256 ? 256 : TPR;
+    hipLaunchKernelGGL((dynamic_quant_rows_kernel<X_DT, Y_DT, ASYM, TPR, MAXP>), dim3((unsigned)((p.rows * TPR + WG - 1) / WG)), dim3(WG), 0, st, p);
+    return (int)hipGetLastError();
+}
 template <int X_DT, int Y_DT, bool ASYM>
 static int launch_dynamic_quant(const DynQuantParams& p, int variant, hipStream_t st)
 {
-    const bool vec = p.cols % 8 == 0 && p.cols <= 8 * 8 * 256 && (uintptr_t)p.x % 16 == 0 && (uintptr_t)p.y % 8 == 0 &&
+    const bool vec = p.cols % 8 == 0 && p.cols <= 8 * 8 * 1024 && (uintptr_t)p.x % 16 == 0 && (uintptr_t)p.y % 8 == 0 &&
                      (!p.smooth || (uintptr_t)p.smooth % 16 == 0);
     if (variant == 2 || !vec) {
         if (variant == 1) return -4;
         hipLaunchKernelGGL((dynamic_quant_two_pass_kernel<X_DT, Y_DT, ASYM>), dim3((unsigned)p.rows), dim3(256), 0, st, p);
-    } else if (p.cols <= 2048 || (p.cols <= 4096 && p.rows >= 16384)) {
-        // one wave per row: no barrier, no LDS.  Up to 4096 columns (8 pieces per lane) when there are rows enough to
-        // fill the SIMDs with such waves (65536 x 4096: 182 against 209 us; 2048 x 4096: 9.9 against 8.1 us)
-        hipLaunchKernelGGL((dynamic_quant_rows_kernel<X_DT, Y_DT, ASYM, 64>), dim3((unsigned)((p.rows + 3) / 4)), dim3(256), 0, st, p);
-    } else {
-        hipLaunchKernelGGL((dynamic_quant_rows_kernel<X_DT, Y_DT, ASYM, 256>), dim3((unsigned)p.rows), dim3(256), 0, st, p);
+        return (int)hipGetLastError();
     }
-    return (int)hipGetLastError();
+    // Up to 512 rows the workgroups do not fill the CUs and a row's own chain (load, reduction, conversion) is the time: a thread per
+    // piece (8 x 4096 5.9 -> 4.7 us, 2 x 10496 9.8 -> 4.4, 200 x 8192 7.9 -> 4.8, 333 x 3584 5.8 -> 5.0; under the profiler).  Beyond,
+    // the wider workgroups only wait longer for each other (2048 x 4096 10.9 us so and 13.5 with 1024 threads, 700 x 4096 5.9 and 6.8).
+    const bool few = p.rows <= 512;
+    if (p.cols > 16384 || (few && p.cols > 2048)) {
+        if (p.cols <= 8192) return launch_quant_rows<X_DT, Y_DT, ASYM, 1024, 1>(p, st);
+        if (p.cols <= 16384) return launch_quant_rows<X_DT, Y_DT, ASYM, 1024, 2>(p, st);
+        if (p.cols <= 32768) return launch_quant_rows<X_DT, Y_DT, ASYM, 1024, 4>(p, st);
+        return launch_quant_rows<X_DT, Y_DT, ASYM, 1024, 8>(p, st);
+    }
+    if (few) return launch_quant_rows<X_DT, Y_DT, ASYM, 256, 1>(p, st);
+    // one wave per row: no barrier, no LDS.  Up to 4096 columns (8 pieces per lane) when there are rows enough to
+    // fill the SIMDs with such waves (65536 x 4096: 182 against 209 us; 2048 x 4096: 9.9 against 8.1 us)
+    if (p.cols <= 2048) return launch_quant_rows<X_DT, Y_DT, ASYM, 64, 4>(p, st);
+    if (p.cols <= 4096 && p.rows >= 16384) return launch_quant_rows<X_DT, Y_DT, ASYM, 64, 8>(p, st);
+    if (p.cols <= 4096) return launch_quant_rows<X_DT, Y_DT, ASYM, 256, 2>(p, st);
+    if (p.cols <= 8192) return launch_quant_rows<X_DT, Y_DT, ASYM, 256, 4>(p, st);
+    return launch_quant_rows<X_DT, Y_DT, ASYM, 256, 8>(p, st);
 }
 
 // ---------------------------------------------------------------------------------------------------------------------

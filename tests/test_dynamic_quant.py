@@ -303,6 +303,16 @@ def test_gpu_dynamic_quant_is_bit_identical(gpu, shape, x_dt, y_dt, symmetric, w
 
 
 @pytest.mark.gpu
+# either side of every rule that picks the kernel's threads per row and pieces per thread: columns 2048, 4096, 8192, 16384, 32768 and
+# 65536 (the last that stays in registers), rows 512; rows of one piece
+@pytest.mark.parametrize("shape", [(3, 8), (512, 2048), (513, 2048), (513, 2056), (2, 2056), (513, 4104), (1, 8192), (3, 8200), (515, 8200),
+                                   (2, 16392), (514, 16392), (2, 32768), (2, 32776), (1, 65536), (1, 65544), (16384, 2056)])
+@pytest.mark.parametrize("x_dt,y_dt,symmetric,with_smooth", [(orc.BF16, orc.I8, True, False), (orc.BF16, orc.E4M3, True, True), (orc.F16, orc.I4, False, True)])
+def test_gpu_dynamic_quant_row_instances(gpu, shape, x_dt, y_dt, symmetric, with_smooth):
+    test_gpu_dynamic_quant_is_bit_identical(gpu, shape, x_dt, y_dt, symmetric, with_smooth)
+
+
+@pytest.mark.gpu
 def test_gpu_int32_carrier_holds_the_int4_bytes(gpu):
     m = gpu
     rng = np.random.default_rng(1)
