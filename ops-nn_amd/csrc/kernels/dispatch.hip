@@ -37,6 +37,7 @@ int launch_wq_kn(const OpsnnWqmmArgs& a, hipStream_t st);
 bool wq_nk_wanted(const OpsnnWqmmArgs& a, uint64_t* workspace);   // wq_nk.hip
 int launch_wq_nk(const OpsnnWqmmArgs& a, hipStream_t st);
 uint64_t mx_workspace_bytes(const OpsnnQmmArgs& a);
+bool mxfp4_rows_wanted(const OpsnnQmmArgs& a);   // qmm_mxfp4_rows.hip
 }  // namespace opsnn
 
 using namespace opsnn;
@@ -251,8 +252,9 @@ static int splitk_for(const OpsnnQmmArgs& a, int mode)
     if ((mode == 0 || (mode == 3 && !a.x1_scale)) && a.x1_dtype == DT_I8 && a.x2_dtype == DT_I8 && out16 && a.K % 128 == 0)
         return tile_plan(a.M, a.N, a.K, a.batch, true).splits;
     if (tiny) return 1;
-    // MXFP4: 128 x 128 tiles when 256 x 256 ones would be few (the launcher's rule), K tiles counted in 256 elements
+    // MXFP4 with few rows: one launch whatever K (qmm_mxfp4_rows.hip).  Else 128 x 128 tiles when 256 x 256 ones would be few (the launcher's rule), K tiles counted in 256 elements
     if (mode == 2 && a.x1_dtype == DT_E2M1 && a.x2_dtype == DT_E2M1 && (out16 || a.out_dtype == DT_F32)) {
+        if (mxfp4_rows_wanted(a)) return 1;
         const int64_t t256 = ((a.M + 255) / 256) * ((a.N + 255) / 256) * a.batch;
         bm = bn = (a.M <= 128 || a.N <= 128 || t256 <= 64) ? 128 : 256;
         kunit = 256;

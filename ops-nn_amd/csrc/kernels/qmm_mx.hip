@@ -8,6 +8,7 @@
 // the matrix core its 32 K elements together with the e8m0 byte that scales exactly those 32 elements, so the
 // MX block size (32) and the hardware operand block coincide and no dequantised copy is ever formed.
 //
+// Few rows of fp4: the stream kernel of qmm_mxfp4_rows.hip, whatever K's tail.
 // Fast paths: operands and scales K-contiguous, K % 128 == 0, 16-bit output.  fp4: qgemm_core.hip.h, MODE_MXFP4
 // (K % 512 == 0 takes 256-element K tiles, otherwise 128-element ones); fp8: the MX mode of the kernel in
 // qmm_fp8_block.hip.  An N-contiguous x2 (data [K, N], scales [K/64, N, 2]) is first re-laid out into the
@@ -200,6 +201,8 @@ static int mx_relayout_run(const OpsnnQmmArgs& a, const MxRelayout& R, char* w, 
     return (int)hipGetLastError();
 }
 
+bool mxfp4_rows_wanted(const OpsnnQmmArgs& a);   // qmm_mxfp4_rows.hip
+int launch_mxfp4_rows(const OpsnnQmmArgs& a, hipStream_t st);
 // What every matrix-core route of this file needs of the call, whatever x2's layout and K's tail: checked before any
 // pre-step is launched or a cache entry made.
 static bool mx_call_ok(const OpsnnQmmArgs& a)
@@ -218,7 +221,7 @@ static bool mx_call_ok(const OpsnnQmmArgs& a)
     if (a.out_dtype != DT_BF16 && a.out_dtype != DT_F16 && a.out_dtype != DT_F32) return false;
     if (a.bias && a.bias_dtype != DT_F32) return false;
     // (fewer than 64 x 64 outputs: only MXFP8's few-rows stream over x2, which wants 256 columns)
-    if (a.K % 32 != 0 || (a.M * a.N < 64 * 64 && !(fp8 && a.M <= 32 && a.N >= 256 && a.batch == 1 && a.K % 128 == 0))) return false;
+    if (a.K % 32 != 0 || (a.M * a.N < 64 * 64 && !(fp8 && a.M <= 32 && a.N >= 256 && a.batch == 1 && a.K % 128 == 0) && !mxfp4_rows_wanted(a))) return false;
     const int64_t ks = (a.K + 63) / 64, epb = fp4 ? 2 : 1;
     if (a.x1.col_stride != 1 || a.x1_scale_mat.col_stride != 2 || a.x1_scale_mat.row_stride != ks * 2) return false;
     if (((uintptr_t)a.x1.ptr | (uint64_t)(a.x1.row_stride / epb) | (uint64_t)(a.x1.batch_stride / epb)) % 16) return false;
@@ -238,7 +241,7 @@ static uint64_t mx_rest_bytes(const OpsnnQmmArgs& a0)
         mx_relayout_view(a, R, (char*)(uintptr_t)256);   // any aligned address: only the layout matters below
     }
     MxPad L;
-    if (mx_pad_layout(a, L)) total += L.total;
+    if (mx_pad_layout(a, L)) total += L.total;   // (few rows of fp4 leave it unused: the size stays what it always was)
     return total;
 }
 
@@ -293,8 +296,9 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
     OpsnnQmmArgs planned = a;
     if (relayout) mx_relayout_view(planned, R, (char*)(uintptr_t)256);
     MxPad L;
-    const bool pad = mx_pad_layout(planned, L);
-    if (!pad && planned.K % 128 != 0) return OPSNN_NOT_TAKEN;
+    const bool rows4 = fp4 && mxfp4_rows_wanted(a);   // few rows of MXFP4: the kernel that takes a K tail as it is
+    const bool pad = !rows4 && mx_pad_layout(planned, L);
+    if (!pad && !rows4 && planned.K % 128 != 0) return OPSNN_NOT_TAKEN;
     if (planned.x2_scale_mat.col_stride != 2 || (fp4 || fp8 ? planned.x2_scale_mat.row_stride != (planned.K + 63) / 64 * 2 : planned.x2_scale_mat.row_stride % 4 != 0)) return OPSNN_NOT_TAKEN;
     if (pad && (!a.workspace || (uintptr_t)a.workspace % 16)) return OPSNN_NOT_TAKEN;
     if (relayout) {
@@ -316,6 +320,7 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         if (cached && fresh) weight_cache_commit(w, st);
         mx_relayout_view(a, R, w);
     }
+    if (rows4) return launch_mxfp4_rows(a, st);
     if (pad) {
         if (!mx_pad_layout(a, L)) return OPSNN_NOT_TAKEN;   // (the same answer as for the planned view: its conditions do not look at x2's address beyond its alignment)
         const int rc = mx_pad_prestep(a, L, st);
