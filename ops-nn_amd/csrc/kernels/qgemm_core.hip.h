@@ -121,7 +121,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
     static_assert(!MX || SCB == 4 || SCB == 8, "MX tiles carry four or eight scale bytes per row");
     static_assert(!MX || (SC16 ? (BM + BN) % NT == 0 : ((BM + BN) * SCW) % NT == 0), "scale copy mapping");
     static_assert(!SC16 || STAGES == 2, "paired scale copies are waited for with the two-stage counts");
-    static_assert(!MX || !KTAIL, "MX fast path takes whole K tiles only");
+    static_assert(!MX || !KTAIL || SC16, "MX: a K tail on the tiles whose scales travel in pairs only");
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
 #if QG_DBG
@@ -206,31 +206,48 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
         }
     }
 
-    auto issue_tile = [&](int kt, auto with_scales) {   // with_scales: SC16 only, true for even tiles
+    // tail (MX with a K tail): this tile or its pair of scale words may reach past the end of K
+    auto issue_tile = [&](int kt, auto with_scales, auto tail) {   // with_scales: SC16 only, true for even tiles
         (void)with_scales;
+        constexpr bool TAIL = KTAIL && (!MX || decltype(tail)::value);
         char* sA = smem + (kt % STAGES) * STAGE + wave * 1024;
         char* sB = sA + A_BYTES;
         const int64_t k0 = (int64_t)kt * BK;
         const int8_t* Ak = A + k0;
         const int8_t* Bk = B + k0;
-        const bool kok = !KTAIL || (k0 + cchunk * 16) < K;
+        const bool kok = !TAIL || (k0 + cchunk * 16) < K;
 #pragma unroll
         for (int i = 0; i < NA; i++) {
             const int8_t* g = Ak + a_off[i];
-            if constexpr (KTAIL) g = kok ? g : zero_page;
+            if constexpr (TAIL) g = kok ? g : zero_page;
             async_copy16(g, sA + i * NT * 16);
         }
 #pragma unroll
         for (int i = 0; i < NB; i++) {
             const int8_t* g = Bk + b_off[i];
-            if constexpr (KTAIL) g = kok ? g : zero_page;
+            if constexpr (TAIL) g = kok ? g : zero_page;
             async_copy16(g, sB + i * NT * 16);
         }
         if constexpr (SC16) {
             if constexpr (decltype(with_scales)::value) {   // scales of tiles kt and kt+1; the slot's last reader was tile kt-1
-                char* sS = smem + SC_RING + ((kt >> 1) & 1) * ((BM + BN) * 16) + wave * 1024;
+                char* sS = smem + SC_RING + ((kt >> 1) & 1) * ((BM + BN) * 16);
+                const int at = (kt >> 1) * 16;
+                const int words = (int)((K + 63) / 64);   // scale words of a row (the last one filled up where K ends inside it)
+                if (TAIL && at + 16 > 4 * words) {
+                    // the row's last words, four lanes to a row, the last one again past its end (those elements are zeros)
+                    const int last = words - at / 4 - 1;
+#pragma unroll 1
+                    for (int i = 0; i < (BM + BN) * 4 / NT; i++) {
+                        const int c = i * NT + tid, r = c >> 2, part = (c & 3) < last ? (c & 3) : last;
+                        const uint8_t* g;
+                        if (r < BM) g = p.sa + bz * p.sa_bs + (m0 + (r < a_rows ? r : a_rows - 1)) * p.sa_rs;
+                        else g = p.sb + bz * p.sb_bs + (n0 + (r - BM < b_rows ? r - BM : b_rows - 1)) * p.sb_rs;
+                        async_copy4(g + at + 4 * part, sS + wave * 256 + i * NT * 4);
+                    }
+                } else {
 #pragma unroll
-                for (int i = 0; i < NSC; i++) async_copy16(sc_src[i] + (int64_t)(kt >> 1) * 16, sS + i * NT * 16);
+                    for (int i = 0; i < NSC; i++) async_copy16(sc_src[i] + (int64_t)at, sS + wave * 1024 + i * NT * 16);
+                }
             }
         } else if constexpr (MX) {
             char* sS = smem + (kt % STAGES) * STAGE + A_BYTES + B_BYTES + wave * 256;
@@ -383,8 +400,8 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
 #pragma unroll
     for (int i = 0; i < STAGES; i++)
         if (i < KT) {
-            if (i % 2 == 0) issue_tile(i, std::true_type{});
-            else issue_tile(i, std::false_type{});
+            if (i % 2 == 0) issue_tile(i, std::true_type{}, std::true_type{});
+            else issue_tile(i, std::false_type{}, std::true_type{});
         }
     if (KT >= STAGES) wait_vmcnt<(STAGES - 1) * CPT>();
     else wait_vmcnt<0>();
@@ -396,7 +413,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
     load_frags(0, 0, 0);
     load_scales(0);
 
-    auto k_tile = [&](int kt, auto issue, auto next, auto even) {
+    auto k_tile = [&](int kt, auto issue, auto next, auto even, auto tail) {
         constexpr bool ISSUE = decltype(issue)::value, NEXT = decltype(next)::value;
         raw_t ra[FM], rb[FN];   // raw scale bytes of the next tile on their way in
         (void)ra; (void)rb;
@@ -438,7 +455,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
             read_scales_raw(kt + 1, ra, rb);
             __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (ISSUE) issue_tile(kt + STAGES, even);
+        if constexpr (ISSUE) issue_tile(kt + STAGES, even, tail);
         if constexpr (NEXT) load_frags(kt + 1, 0, 0);
         mma(1, std::integral_constant<int, KS - 1>{});
         if constexpr (NEXT) interleave(ISSUE);
@@ -450,16 +467,24 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
     using T = std::true_type;
     using F = std::false_type;
     int kt = 0;
-    if constexpr (SC16) {   // KT is even: tiles go in pairs, the even one also starts the pair's scale copy
+    if constexpr (SC16 && KTAIL) {   // whole pairs of tiles first; the last one or two may end early
+        const int whole = (int)(K / 256) * 2;
+        for (; kt + 3 < whole; kt += 2) {
+            k_tile(kt, T{}, T{}, T{}, F{});
+            k_tile(kt + 1, T{}, T{}, F{}, F{});
+        }
+        if (kt + 2 < KT) { k_tile(kt, T{}, T{}, T{}, T{}); kt++; }
+        if (kt + 2 < KT) { k_tile(kt, T{}, T{}, F{}, T{}); kt++; }
+    } else if constexpr (SC16) {   // KT is even: tiles go in pairs, the even one also starts the pair's scale copy
         for (; kt + STAGES < KT; kt += 2) {
-            k_tile(kt, T{}, T{}, T{});
-            k_tile(kt + 1, T{}, T{}, F{});
+            k_tile(kt, T{}, T{}, T{}, F{});
+            k_tile(kt + 1, T{}, T{}, F{}, F{});
         }
     } else {
-        for (; kt + STAGES < KT; kt++) k_tile(kt, T{}, T{}, F{});
+        for (; kt + STAGES < KT; kt++) k_tile(kt, T{}, T{}, F{}, T{});
     }
-    for (; kt + 1 < KT; kt++) k_tile(kt, F{}, T{}, F{});
-    k_tile(kt, F{}, F{}, F{});
+    for (; kt + 1 < KT; kt++) k_tile(kt, F{}, T{}, F{}, F{});
+    k_tile(kt, F{}, F{}, F{}, F{});
     if constexpr (SPLIT) {
         // partial sums straight from the registers (acc[i][j][r]: n = n_base + 8*(r/4) + 4*(lane/32) + r%4, m = m_base + lane%32)
         typedef std::conditional_t<MODE == MODE_I8, v4i, v4f> quad_t;
@@ -824,6 +849,13 @@ static int qgemm_launch(const QgemmParams& p, int64_t batch, int out_dt, hipStre
     if constexpr (MODE == MODE_I8) {
         if (out_dt == DT_I32 || out_dt == DT_I8) return -2;   // qgemm_launch_int
         if ((p.KB % BK) != 0) {
+            return bf ? qgemm_launch_one<MODE, BM, BN, BK, WGM, WGN, STAGES, MINWG, true, DT_BF16>(p, batch, st)
+                      : qgemm_launch_one<MODE, BM, BN, BK, WGM, WGN, STAGES, MINWG, true, DT_F16>(p, batch, st);
+        }
+    }
+    if constexpr (MODE == MODE_MXFP4 && BK == 128) {
+        if ((p.KB % (2 * BK)) != 0) {
+            if (out_dt == DT_F32) return qgemm_launch_one<MODE, BM, BN, BK, WGM, WGN, STAGES, MINWG, true, DT_F32>(p, batch, st);
             return bf ? qgemm_launch_one<MODE, BM, BN, BK, WGM, WGN, STAGES, MINWG, true, DT_BF16>(p, batch, st)
                       : qgemm_launch_one<MODE, BM, BN, BK, WGM, WGN, STAGES, MINWG, true, DT_F16>(p, batch, st);
         }

@@ -9,12 +9,13 @@
 // MX block size (32) and the hardware operand block coincide and no dequantised copy is ever formed.
 //
 // Few rows of fp4: the stream kernel of qmm_mxfp4_rows.hip, whatever K's tail.
-// Fast paths: operands and scales K-contiguous, K % 128 == 0, 16-bit output.  fp4: qgemm_core.hip.h, MODE_MXFP4
-// (K % 512 == 0 takes 256-element K tiles, otherwise 128-element ones); fp8: the MX mode of the kernel in
-// qmm_fp8_block.hip.  An N-contiguous x2 (data [K, N], scales [K/64, N, 2]) is first re-laid out into the
-// workspace.  K % 128 != 0 (K a whole number of 32-element blocks): both operands and both scale tables (x2's after that re-layout, if it was needed) are first
-// copied into the workspace with K rounded up to 128, the new elements zero and their scales a repeat of the row's last one (zero products
-// change no sum).  All of this is planned before the first pre-step is launched.  Everything else runs the plain kernel.
+// Fast paths: operands and scales K-contiguous, 16-bit or fp32 output.  fp4: qgemm_core.hip.h, MODE_MXFP4 (256 x 256 tiles: K tiles of
+// 256 elements, a K that is no whole pair of them ending in zeros inside the kernel; 128 x 128 tiles: of 128); fp8: the MX mode of the
+// kernel in qmm_fp8_block.hip.  An N-contiguous x2 (data [K, N], scales [K/64, N, 2]) is first re-laid out into the workspace.
+// K % 128 != 0 (K a whole number of 32-element blocks): both operands and both scale tables (x2's after that re-layout, if it was needed)
+// are first copied into the workspace with K rounded up to 128, the new elements zero and their scales a repeat of the row's last one
+// (zero products change no sum); the 256 x 256 fp4 tiles need the scale tables alone.  All of this is planned before the first
+// pre-step is launched.  Everything else runs the plain kernel.
 #include "launch.h"
 #include "qgemm_core.hip.h"
 
@@ -116,6 +117,37 @@ static bool mx_pad_layout(const OpsnnQmmArgs& a, MxPad& L)
     L.o_s2 = L.o_s1 + align_up((uint64_t)L.snb1 * a.M * ksp * 2, 256);
     L.total = L.o_s2 + align_up((uint64_t)L.snb2 * a.N * ksp * 2, 256);
     return true;
+}
+
+// The scale tables alone, both in one launch (rows of x1's, then of x2's along grid.y): for fp4 on the tiles that end a K inside a
+// tile by themselves, whose scales come in whole words.
+__global__ __launch_bounds__(256) void mx_pad_scales_kernel(const uint8_t* __restrict__ s1, int64_t bs1, uint8_t* __restrict__ d1, int64_t rows1, int64_t nb1,
+                                                            const uint8_t* __restrict__ s2, int64_t bs2, uint8_t* __restrict__ d2, int64_t rows2, int64_t nb2,
+                                                            int64_t ld, int64_t kb, int64_t kbp)
+{
+    const int64_t c = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63), b = blockIdx.z;
+    int64_t r = (int64_t)blockIdx.y * 4 + (threadIdx.x >> 6);
+    const bool second = r >= rows1;
+    if (second) r -= rows1;
+    if (c * 2 >= kbp || r >= (second ? rows2 : rows1) || b >= (second ? nb2 : nb1)) return;
+    const uint8_t* s = (second ? s2 + b * bs2 : s1 + b * bs1) + r * ld;
+    uint8_t* d = (second ? d2 + b * rows2 * kbp : d1 + b * rows1 * kbp) + r * kbp + 2 * c;
+    const uint8_t last = s[kb - 1];
+    d[0] = 2 * c < kb ? s[2 * c] : last;
+    d[1] = 2 * c + 1 < kb ? s[2 * c + 1] : last;
+}
+static int mx_pad_scales(OpsnnQmmArgs& a, const MxPad& L, hipStream_t st)
+{
+    if (!a.workspace || (uintptr_t)a.workspace % 16) return OPSNN_NOT_TAKEN;
+    uint8_t* w = (uint8_t*)a.workspace;
+    const int64_t ksp2 = L.Kp / 64 * 2, nb = L.snb1 > L.snb2 ? L.snb1 : L.snb2;
+    const dim3 grid((unsigned)((ksp2 / 2 + 63) / 64), (unsigned)((a.M + a.N + 3) / 4), (unsigned)nb);
+    hipLaunchKernelGGL(mx_pad_scales_kernel, grid, dim3(256), 0, st, (const uint8_t*)a.x1_scale_mat.ptr, a.x1_scale_mat.batch_stride, w + L.o_s1, a.M, L.snb1,
+                       (const uint8_t*)a.x2_scale_mat.ptr, a.x2_scale_mat.batch_stride, w + L.o_s2, a.N, L.snb2, (a.K + 63) / 64 * 2, a.K / 32, ksp2);
+    a.x1_scale_mat = OpsnnMat{w + L.o_s1, ksp2, 2, L.snb1 == 1 && a.batch > 1 ? 0 : a.M * ksp2};
+    a.x2_scale_mat = OpsnnMat{w + L.o_s2, ksp2, 2, L.snb2 == 1 && a.batch > 1 ? 0 : a.N * ksp2};
+    a.workspace = nullptr;
+    return (int)hipGetLastError();
 }
 
 // Launches the four copies and rewrites `a` as the same call on the padded operands.
@@ -321,9 +353,12 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         mx_relayout_view(a, R, w);
     }
     if (rows4) return launch_mxfp4_rows(a, st);
+    const bool small = a.M <= 128 || a.N <= 128;
+    // 128 x 128 tiles also when 256 x 256 ones would be at most 64, a quarter of the CUs (1024 x 4096 x 4096: 22.9 against 28.0 us; at 128 tiles of 256 x 256 it is 42 against 32)
+    const bool fp4_small = small || ((a.M + 255) / 256) * ((a.N + 255) / 256) * a.batch <= 64 || a.force_variant == OPSNN_VARIANT_MX_128;
     if (pad) {
         if (!mx_pad_layout(a, L)) return OPSNN_NOT_TAKEN;   // (the same answer as for the planned view: its conditions do not look at x2's address beyond its alignment)
-        const int rc = mx_pad_prestep(a, L, st);
+        const int rc = fp4 && !fp4_small ? mx_pad_scales(a, L, st) : mx_pad_prestep(a, L, st);
         if (rc != 0) return rc;
     }
     if (a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E2M1) return launch_mx_a8w4_mfma(a, st, sk);   // fp8 x fp4: qmm_fp8_block.hip
@@ -363,28 +398,21 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         const int rc = launch_mx_exact(a, st, sk);
         if (rc != OPSNN_NOT_TAKEN) return rc;
     }
-    const bool small = a.M <= 128 || a.N <= 128;
     if (fp4) {
         // few tiles against a long K: K split over workgroups (fp32 partial sums in front of the workspace), on the tiles
         // chosen below
         const bool split = sk.splits > 1 && sk.part && a.force_variant == 0 && a.K % 256 == 0;
         if (split) { g.splits = sk.splits; g.part = (int32_t*)sk.part; }
-        // 128 x 128 tiles also when 256 x 256 ones would be at most 64, a quarter of the CUs (1024 x 4096 x 4096: 22.9 against 28.0 us; at 128 tiles of 256 x 256 it is 42 against 32)
-        const int64_t t256 = ((a.M + 255) / 256) * ((a.N + 255) / 256) * a.batch;
-        if (small || t256 <= 64 || a.force_variant == OPSNN_VARIANT_MX_128) {
+        if (fp4_small) {
             if (split) return qgemm_launch_split_mx<MODE_MXFP4, 128, 128, 64, 2, 2, 4, 1>(g, a.batch, a.out_dtype, st);
             return qgemm_launch<MODE_MXFP4, 128, 128, 64, 2, 2, 4, 1>(g, a.batch, a.out_dtype, st);
         }
-        // K tiles of 128 bytes (256 elements) with the scales of two tiles per 16-byte copy: needs an even number of
-        // such tiles and 16-byte aligned scale rows
-        const bool sc16 = a.K % 512 == 0 &&
-                          (((uintptr_t)g.sa | (uintptr_t)g.sb | (uint64_t)g.sa_rs | (uint64_t)g.sb_rs | (uint64_t)g.sa_bs | (uint64_t)g.sb_bs) % 16) == 0;
-        if (sc16) {
-            if (split) return qgemm_launch_split_mx<MODE_MXFP4, 256, 256, 128, 2, 4, 2, 1>(g, a.batch, a.out_dtype, st);
-            return qgemm_launch<MODE_MXFP4, 256, 256, 128, 2, 4, 2, 1>(g, a.batch, a.out_dtype, st);
-        }
-        if (split) return qgemm_launch_split_mx<MODE_MXFP4, 256, 256, 64, 2, 2, 4, 1>(g, a.batch, a.out_dtype, st);
-        return qgemm_launch<MODE_MXFP4, 256, 256, 64, 2, 2, 4, 1>(g, a.batch, a.out_dtype, st);
+        // K tiles of 128 bytes (256 elements) with the scales of two tiles per 16-byte copy; a K that is no whole pair of tiles ends in
+        // zeros from the kernel's own page.  (Against 64-byte tiles, on which such a K ran: 2 x 1864 x 1408 x 13208 94 -> 85 us,
+        // 4 x 1828 x 3840 x 11712 284 -> 229, 2048 x 8064 x 14336 189 -> 150.)  The K split deals whole pairs.
+        if (split && a.K % 512 != 0) return qgemm_launch_split_mx<MODE_MXFP4, 256, 256, 64, 2, 2, 4, 1>(g, a.batch, a.out_dtype, st);
+        if (split) return qgemm_launch_split_mx<MODE_MXFP4, 256, 256, 128, 2, 4, 2, 1>(g, a.batch, a.out_dtype, st);
+        return qgemm_launch<MODE_MXFP4, 256, 256, 128, 2, 4, 2, 1>(g, a.batch, a.out_dtype, st);
     }
     // FLOAT output: the tile kernel, whose epilogue stores fp32 straight from the registers
     if (a.out_dtype == DT_F32 || a.force_variant == OPSNN_VARIANT_MX_FP8_MFMA || a.force_variant == OPSNN_VARIANT_MX_128) {   // (also the chained-K variants of the tests)

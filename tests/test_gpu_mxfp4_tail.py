@@ -1,0 +1,46 @@
+"""MXFP4 on 256 x 256 tiles with a K that is no whole pair of 256-element K tiles: the tiles end in zeros, the last scale words by
+word, and a K inside a word behind scale rows that are copied (the data is read as it lies)."""
+import numpy as np
+import pytest
+
+import cases
+import oracle_api as orc
+from test_gpu_other_modes import check_close
+
+pytestmark = pytest.mark.gpu
+
+
+# 65 batches of one tile: more than the 64 tiles below which 128 x 128 ones take over.  One K tile and less, an odd and an even count,
+# a last tile of a quarter, a half and three quarters, and (32, 96, 160 mod 128) a last scale word that is not full
+@pytest.mark.parametrize("K", [32, 96, 128, 160, 256, 384, 544, 640, 768, 992, 1088, 1152, 1408])
+@pytest.mark.parametrize("tB", [True, False])
+def test_k_tail_on_whole_tiles(gpu, K, tB):
+    m = gpu
+    B, M, N = 65, 131, 140
+    print(f"case mxfp4 tail B={B} M={M} K={K} N={N} tB={tB}", flush=True)
+    m.lib().opsnnSetForcePlain(0)
+    inp = cases.make_mx_inputs(m, M, K, N, K, tB, True, batch=B)
+    if K % 64:   # the byte behind the last block scales nothing: a NaN code there must not reach any sum
+        inp["s1"][..., -1, 1] = 0xFF
+        if tB:
+            inp["s2"][..., -1, 1] = 0xFF
+        else:
+            inp["s2"][:, -1, :, 1] = 0xFF
+    bias = np.random.default_rng(1).normal(0, 1, N).astype(np.float32)
+    want = cases.oracle_mx(m, inp, M, K, N, tB, m.ACL_BF16, bias)
+    got = cases.run_mx_aclnn(m, inp, M, K, N, tB, m.ACL_BF16, bias)
+    check_close(got, want, orc.BF16, "mxfp4 tail")
+
+
+def test_neighbours_with_infinite_scales_stay_out(gpu):
+    """Rows whose scales are NaN codes reach their own outputs only: nothing of a row is read for the tail of the row in front of it."""
+    m = gpu
+    B, M, N, K = 65, 131, 140, 640
+    m.lib().opsnnSetForcePlain(0)
+    inp = cases.make_mx_inputs(m, M, K, N, 7, True, True, batch=B)
+    inp["s1"][:, 1::2] = 0xFF
+    inp["s2"][:, 1::2] = 0xFF
+    got = orc.b16_to_f32(cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_BF16, None), orc.BF16).reshape(B, M, N)
+    want = orc.b16_to_f32(cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, None), orc.BF16).reshape(B, M, N)
+    assert np.isnan(got[:, 1::2]).all() and np.isnan(got[:, :, 1::2]).all()
+    assert np.isfinite(got[:, ::2, ::2]).all() and np.allclose(got[:, ::2, ::2], want[:, ::2, ::2], rtol=1e-2, atol=1e-2)
