@@ -147,11 +147,12 @@ __device__ __forceinline__ float e2m1_to_f32(uint32_t c)
     float v = (e == 0u) ? 0.5f * (float)m : u2f(((e + 126u) << 23) | (m << 22));
     return (c & 8u) ? -v : v;
 }
+// 2^(b - 127), NaN for 0xff.  Without conditions: as branches on b the two special codes were a quarter of the instructions of the
+// loops that widen with a scale per 32 elements.
 __device__ __forceinline__ float e8m0_to_f32(uint32_t b)
 {
-    if (b == 0xffu) return u2f(0x7fc00000u);
-    if (b == 0u) return u2f(0x00400000u);
-    return u2f(b << 23);
+    const uint32_t u = b << 23;
+    return u2f((u > 0x00400000u ? u : 0x00400000u) | (((b + 1u) >> 8) << 22));
 }
 
 // The sum, in split order, of `splits` partial arrays [rows][N] that lie `slice` elements apart (the K split of every kernel

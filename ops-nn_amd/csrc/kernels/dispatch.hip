@@ -16,13 +16,9 @@ int launch_wqmm_plain(const OpsnnWqmmArgs& a, hipStream_t st);
 int launch_blockscale_mfma(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk = {});
 int launch_fp8_rowcol_mfma(const OpsnnQmmArgs& a, hipStream_t st, bool merged_scales_ok, SplitK sk = {});
 int launch_rowcol_exact(const OpsnnQmmArgs& a, hipStream_t st, int ep_mode, SplitK sk = {});   // qmm_fp8_exact.hip
-int launch_rowcol_decode(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk);   // qmm_fp8_decode.hip
-uint64_t blockscale_rows_workspace(const OpsnnQmmArgs& a);         // qmm_fp8_rows.hip
-int blockscale_rows_ksplit(const OpsnnQmmArgs& a);
-uint64_t rowcol_rows_workspace(const OpsnnQmmArgs& a);
-int launch_rowcol_rows(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk);
-int rowcol_rows_ksplit(const OpsnnQmmArgs& a);
-int mxfp8_rows_ksplit(const OpsnnQmmArgs& a);
+int launch_fp8_stream(const OpsnnQmmArgs& a, Fp8xForm form, SplitK sk, hipStream_t st);   // qmm_fp8_stream.hip
+uint64_t blockscale_rows_reserve(const OpsnnQmmArgs& a, int* segments);
+int mxfp8_rows_ksplit(const OpsnnQmmArgs& a);   // qmm_fp8_rows.hip
 int launch_tcg_mfma(const OpsnnQmmArgs& a, hipStream_t st);
 uint64_t tcg_workspace_bytes(const OpsnnQmmArgs& a);
 int launch_kg_mfma(const OpsnnQmmArgs& a, hipStream_t st);   // qmm_i4_kg.hip
@@ -175,6 +171,8 @@ int64_t k_pad_for(const OpsnnQmmArgs& a, int mode)
         // (the fp8 members of this family have no transposition step of their own)
         const bool f8_16 = f8any && (a.out_dtype == DT_BF16 || a.out_dtype == DT_F16 || a.out_dtype == DT_F32) && (!a.bias || a.bias_dtype == DT_F32);
         tail = (i8 && !a.x1_scale && (a.K % 16 != 0 || !x1_ok || !(x2_k || x2_n))) || (f8_16 && (a.K % 128 != 0 || !x1_ok || !x2_k));
+        // (few rows: the stream kernel ends a K of half a block by itself)
+        if (Fp8StreamPlan pl; tail && f8 && x1_ok && x2_k && fp8_stream_plan(a, FP8X_PLAIN, false, pl)) tail = false;
     }
     if (!tail || a.K < 16) return 0;
     if (a.x1.batch_stride < 0 || a.x2.batch_stride < 0) return 0;
@@ -222,21 +220,14 @@ static int splitk_for(const OpsnnQmmArgs& a, int mode)
     if (a.force_variant != 0 || opsnn_force_plain()) return 1;   // (a pinned kernel variant runs as it is)
     const bool out16 = a.out_dtype == DT_BF16 || a.out_dtype == DT_F16;
     const bool f8 = a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E4M3;
-    // up to 32 rows of fp8 with block scales or row / column scales, or of int8 per-tile: the decode kernel's K segments
+    // few rows of fp8: the stream kernel's
+    if (Fp8StreamPlan pl; f8 && mode >= 1 && mode <= 3 && fp8_stream_plan(a, mode == 1 ? FP8X_BLOCK : mode == 2 ? FP8X_MX : FP8X_PLAIN, true, pl)) return pl.splits;
+    // up to 16 rows of fp8 with block or MX scales, of int8 per-tile and of fp8 x fp4 MX: the decode kernels' K segments
     const bool a8w4 = mode == 2 && a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E2M1;
     const bool i8pt = mode == 1 && a.x1_dtype == DT_I8 && a.x2_dtype == DT_I8;
-    if (a.M <= ((i8pt || a8w4) ? 16 : 32) && a.batch == 1 && a.N >= 256 &&
-        ((mode == 1 && (f8 || i8pt) && a.gsK == 128 && a.gsN == 128) ||
-         (mode == 3 && f8 && a.x1_scale && a.x2_scale) || (a8w4 && out16) || (mode == 2 && f8))) {
+    if (a.M <= 16 && a.batch == 1 && a.N >= 256 && ((mode == 1 && (f8 || i8pt) && a.gsK == 128 && a.gsN == 128) || (a8w4 && out16) || (mode == 2 && f8))) {
         QmmDecodePlan pl;
-        const int sd = qmm_decode_plan(a.K, true, pl, a8w4) ? pl.splits : 1;
-        // (17 .. 32 rows of fp8 with block scales may also run on the many-rows kernel, with its own segments: room for either)
-        const int sr = mode == 1 && f8 ? blockscale_rows_ksplit(a) : mode == 3 && f8 ? rowcol_rows_ksplit(a) : mode == 2 && f8 ? mxfp8_rows_ksplit(a) : 1;
-        return sd > sr ? sd : sr;
-    }
-    // 33 .. 128 rows of fp8 with block scales or row / column scales on the many-rows kernel
-    if ((mode == 1 || mode == 3) && f8 && a.M <= 128) {
-        if (const int sr = mode == 1 ? blockscale_rows_ksplit(a) : rowcol_rows_ksplit(a); sr > 1) return sr;
+        return qmm_decode_plan(a.K, true, pl, a8w4) ? pl.splits : 1;
     }
     // 33 .. 128 rows of MXFP8 on the many-rows kernel
     if (mode == 2 && f8 && a.M <= 128) {
@@ -390,14 +381,12 @@ extern "C" int opsnnQmmTc(const OpsnnQmmArgs* a, void* stream)
     // the other two forms run here.
     if (f8 && a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain()) {
         const int ep = !a->x1_scale ? 1 : (a->x1_scale_len == 1 && a->x2_scale_len == 1 && !a->bias) ? 2 : 0;
-        if (ep == 0) {   // 17 .. 128 rows: the many-rows streaming kernel; up to 16 (32 in two passes where that does not apply): x1 in registers
-            int rc = launch_rowcol_rows(*a, (hipStream_t)stream, sk);
-            if (rc != OPSNN_NOT_TAKEN) return rc;
-            rc = launch_rowcol_decode(*a, (hipStream_t)stream, sk);
+        if (ep == 0) {   // up to 128 rows: the stream kernel
+            const int rc = launch_fp8_stream(*a, FP8X_PLAIN, sk, (hipStream_t)stream);
             if (rc != OPSNN_NOT_TAKEN) return rc;
         }
-        // (up to 32 rows the partial sums were laid out for the kernel above; the tile kernels run unsplit)
-        const SplitK sk_tiles = a->M <= 32 ? SplitK{} : sk;
+        // (up to 128 rows the partial sums were laid out for the kernel above; the tile kernels run unsplit)
+        const SplitK sk_tiles = a->M <= 128 ? SplitK{} : sk;
         const bool e4 = a->x1_dtype == DT_E4M3 && a->x2_dtype == DT_E4M3;
         if (ep != 0 || !e4 || a->x2_scale_dtype != DT_F32 || a->out_dtype == DT_F32) {
             const int rc = launch_rowcol_exact(*a, (hipStream_t)stream, ep, sk_tiles);
@@ -407,7 +396,7 @@ extern "C" int opsnnQmmTc(const OpsnnQmmArgs* a, void* stream)
     // fp8 e4m3 operands with a row scale and a column scale that are multiplied in separately (K-C, K-T, T-C with the
     // one-element x1Scale): matrix-core kernel when the layout allows, else the plain kernel
     if (f8 && a->x1_scale && a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain()) {
-        const int rc = launch_fp8_rowcol_mfma(*a, (hipStream_t)stream, false, a->M <= 32 ? SplitK{} : sk);
+        const int rc = launch_fp8_rowcol_mfma(*a, (hipStream_t)stream, false, a->M <= 128 ? SplitK{} : sk);
         if (rc != OPSNN_NOT_TAKEN) return rc;
     }
     NOTE_PLAIN("per-tensor / per-channel quant matmul", a);
@@ -468,7 +457,9 @@ extern "C" int opsnnWqmm(const OpsnnWqmmArgs* a, void* stream)
 extern "C" uint64_t opsnnQmmWorkspace(const OpsnnQmmArgs* a, int mode)
 {
     if (!a) return 0;
-    return splitk_bytes(*a, splitk_for(*a, mode)) + qmm_workspace_base(a, mode);   // partial sums of a K split in front
+    const uint64_t need = splitk_bytes(*a, splitk_for(*a, mode)) + qmm_workspace_base(a, mode);   // partial sums of a K split in front
+    const uint64_t reserve = mode == 1 && !opsnn_force_plain() ? blockscale_rows_reserve(*a, nullptr) : 0;
+    return need > reserve ? need : reserve;
 }
 
 extern "C" __attribute__((visibility("hidden"))) uint64_t opsnn_qmm_workspace_base(const OpsnnQmmArgs* a, int mode)
@@ -480,13 +471,7 @@ static uint64_t qmm_workspace_base(const OpsnnQmmArgs* a, int mode)
 {
     if (const int64_t Kp = k_pad_for(*a, mode)) return k_pad_bytes(*a, Kp);
     if (mode == 2) return mx_workspace_bytes(*a);
-    if (mode == 1 && a->x2.row_stride == 1 && a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain()) {
-        if (const uint64_t b = blockscale_rows_workspace(*a)) return b;   // fp8 block scales with 17 .. 128 rows: x1 widened to fp16
-    }
     // per-tensor / per-channel family: int8 operands share the int8 kernels and their re-layout; fp8 needs none
-    if (mode == 3 && a->x2.row_stride == 1 && a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain()) {
-        if (const uint64_t b = rowcol_rows_workspace(*a)) return b;   // fp8 row / column scales with 17 .. 128 rows: x1 widened to fp16
-    }
     if (mode == 3 && !(a->x1_dtype == DT_I8 && a->x2_dtype == DT_I8 && !a->x1_scale)) return 0;
     // K-group modes: the re-quantised weight of the fp8 x fp4 group-scale mode; the widened operands, row sums and fp32
     // scale / offset copies of the int4 mode with offsets

@@ -92,6 +92,14 @@ struct Fp8xPlan {
 enum Fp8xForm { FP8X_BLOCK, FP8X_PLAIN, FP8X_MX };   // block scales, row / column scales, MX scales
 Fp8xPlan fp8x_plan(int64_t M, int64_t N, int64_t K, int64_t batch, Fp8xForm form, bool may_split);
 
+// Whether a call of fp8 operands with few rows runs on the stream kernel of qmm_fp8_stream.hip, and how: row and column blocks of 16 per
+// workgroup, K segments (sizes, types and strides only: both phases of a call ask).
+struct Fp8StreamPlan {
+    int mb, nb, splits;
+    bool wide;   // the waves share x1 and each K tile, or each has a quarter of K
+};
+bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8StreamPlan& pl);
+
 // How the x-in-registers kernel (weight-only, up to 16 rows of x) covers K.  A workgroup holds `nw` waves x `nch` chunks
 // (of 64 weight bytes): 16 x 4, 8-bit weights also 16 x 8, or 8 x 4 / 8 x 8.  A K that is exactly one such shape runs on
 // one workgroup per row block range; any other K of whole 128-element units goes in `splits` segments of 16 x 4 chunks
@@ -175,7 +183,7 @@ inline int wq_part_slices(int wbits, int64_t M, int64_t N, int64_t K, int64_t gr
     if (M <= 16) return wq_xreg_splits(wbits, M, K);
     return wq_rows_ksplit(wbits, M, N, K, group, narrow_on);
 }
-// The fp8 / int8 decode kernel (qmm_fp8_decode.hip, up to 32 rows of x1): K in blocks of 128 that the NW = 16 or 8 waves
+// The fp8 / int8 decode kernel (qmm_fp8_decode.hip, up to 16 rows of x1): K in blocks of 128 that the NW = 16 or 8 waves
 // of a workgroup share, NBLK each (a wave keeps its blocks of x1 in registers: 16 waves up to 4, not 3; 8 waves up to 7).
 // A K that the waves of one workgroup share exactly runs as one segment; any other whole number of blocks in 1 .. 16
 // segments of NW * NBLK blocks, the last one with idle waves (K a whole number of NBLK blocks): the layout with the fewest

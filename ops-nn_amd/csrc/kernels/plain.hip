@@ -301,8 +301,7 @@ __global__ void qmm_i4_asym_plain(OpsnnQmmArgs a)
 }
 int launch_fp8_rowcol_mfma(const OpsnnQmmArgs& a, hipStream_t st, bool merged_scales_ok, SplitK sk = {});   // qmm_fp8_block.hip
 
-int launch_rowcol_rows(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk);      // qmm_fp8_rows.hip
-int launch_rowcol_decode(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk);    // qmm_fp8_decode.hip
+int launch_fp8_stream(const OpsnnQmmArgs& a, Fp8xForm form, SplitK sk, hipStream_t st);   // qmm_fp8_stream.hip
 void* weight_cache_blob3(const void* src, const void* src2, const void* src3, int64_t K, int64_t N, int bits, int64_t nb, uint64_t bytes, hipStream_t st,
                          bool* fresh);   // weight_cache.hip
 void weight_cache_commit(void* buffer, hipStream_t st);
@@ -313,8 +312,6 @@ static inline int64_t tcg_kp(const OpsnnQmmArgs& a) { return (a.K + 127) / 128 *
 static inline uint64_t tcg_blob_bytes(const OpsnnQmmArgs& a) { return align256((uint64_t)a.N * tcg_kp(a)) + align256((uint64_t)a.N * 4) + 256; }
 // a K tail: x1 copied into rows of Kp bytes behind the blob
 static inline uint64_t tcg_x1pad_bytes(const OpsnnQmmArgs& a) { return tcg_kp(a) != a.K ? align256((uint64_t)a.M * tcg_kp(a)) : 0; }
-// 17 .. 128 rows go to the many-rows streaming kernel, which wants x1 widened to fp16 (M * Kp * 2 bytes behind those)
-static inline uint64_t tcg_rows_bytes(const OpsnnQmmArgs& a) { return a.M > 16 && a.M <= 128 ? (uint64_t)a.M * tcg_kp(a) * 2 : 0; }
 // Workspace of the matrix-core path of the fp8 x fp4 group-scale mode (0: the shape stays on the plain kernel).
 uint64_t tcg_workspace_bytes(const OpsnnQmmArgs& a)
 {
@@ -326,7 +323,7 @@ uint64_t tcg_workspace_bytes(const OpsnnQmmArgs& a)
     if (((uintptr_t)a.x1.ptr | (uint64_t)a.x1.row_stride) % 16 != 0 || a.x1.row_stride < a.K) return 0;
     if (a.out_dtype != DT_BF16 && a.out_dtype != DT_F16) return 0;
     if (a.bias && a.bias_dtype != DT_F32) return 0;
-    return tcg_blob_bytes(a) + tcg_x1pad_bytes(a) + tcg_rows_bytes(a);
+    return tcg_blob_bytes(a) + tcg_x1pad_bytes(a);
 }
 // Re-quantise x2 into the workspace -- or, with the weight cache on and dense scales, once into a cached buffer that
 // later calls with the same x2, scales and output scale find again -- then an fp8 kernel with a column scale (the
@@ -366,11 +363,9 @@ int launch_tcg_mfma(const OpsnnQmmArgs& a, hipStream_t st)
     b.x2.ptr = w8; b.x2_dtype = DT_E4M3; b.x2.row_stride = 1; b.x2.col_stride = Kp; b.x2.batch_stride = 0;
     b.x1_scale = one; b.x1_scale_len = 1;
     b.x2_scale = cs; b.x2_scale_dtype = DT_F32; b.x2_scale_len = a.N;
-    b.workspace = tcg_rows_bytes(a) ? (char*)a.workspace + blob + tcg_x1pad_bytes(a) : nullptr;
+    b.workspace = nullptr;
     if (a.force_variant == 0) {
-        int rc = launch_rowcol_rows(b, st, SplitK{});
-        if (rc != OPSNN_NOT_TAKEN) return rc;
-        rc = launch_rowcol_decode(b, st, SplitK{});
+        const int rc = launch_fp8_stream(b, FP8X_PLAIN, SplitK{}, st);
         if (rc != OPSNN_NOT_TAKEN) return rc;
     }
     return launch_fp8_rowcol_mfma(b, st, true);

@@ -610,7 +610,7 @@ int launch_mx_a8w4_decode(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk);   /
 int launch_mx_a8w4_mfma(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
 {
     if (a.x1_dtype != DT_E4M3 || a.x2_dtype != DT_E2M1) return OPSNN_NOT_TAKEN;
-    {   // up to 32 rows: the stream over x2 with x1 in registers
+    {   // up to 16 rows: the stream over x2 with x1 in registers
         const int rc = launch_mx_a8w4_decode(a, st, sk);
         if (rc != OPSNN_NOT_TAKEN) return rc;
         if (a.M <= 16) sk = SplitK{};   // (the partial sums were laid out for the kernel above; the tile kernel runs unsplit)
@@ -700,8 +700,8 @@ int launch_fp8_rowcol_mfma(const OpsnnQmmArgs& a, hipStream_t st, bool merged_sc
     return launch_fp8_block<2, 2, DT_F16, FP8_ROWCOL>(p, a.batch, st);
 }
 
+int launch_fp8_stream(const OpsnnQmmArgs& a, Fp8xForm form, SplitK sk, hipStream_t st);   // qmm_fp8_stream.hip
 int launch_blockscale_decode(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk);   // qmm_fp8_decode.hip
-int launch_blockscale_rows(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk);     // qmm_fp8_rows.hip
 
 int launch_blockscale_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
 {
@@ -730,16 +730,16 @@ int launch_blockscale_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         }
         a.x2.row_stride = 1; a.x2.col_stride = a.K;
     }
-    if (!i8 && a0.x2.row_stride == 1) {   // 17 .. 128 rows: x1 widened into the workspace, then the many-rows streaming kernel
-        const int rc = launch_blockscale_rows(a, st, sk);
+    if (!i8) {   // up to 128 rows: the stream kernel
+        const int rc = launch_fp8_stream(a, FP8X_BLOCK, sk, st);
         if (rc != OPSNN_NOT_TAKEN) return rc;
     }
-    {   // up to 16 rows (32 in two passes where the kernel above does not apply): the stream over x2 with x1 in registers
+    {   // up to 16 rows: the stream over x2 with x1 in registers
         const int rc = launch_blockscale_decode(a, st, sk);
         if (rc != OPSNN_NOT_TAKEN) return rc;
     }
     if (tiny) return OPSNN_NOT_TAKEN;
-    if (a.M <= (i8 ? 16 : 32)) sk = SplitK{};   // (with so few rows the partial sums were laid out for the kernel above; the tile kernels run unsplit)
+    if (a.M <= (i8 ? 16 : 128)) sk = SplitK{};   // (with so few rows the partial sums were laid out for the kernels above; the tile kernels run unsplit)
     if (!i8 && (!opsnnGetFp8Fast() || out32)) {   // exact products and sums unless the caller asked for the 8-bit matrix instruction
         const int rc = launch_blockscale_exact(a, st, sk);
         if (rc != OPSNN_NOT_TAKEN || out32) return rc;

@@ -37,9 +37,7 @@ struct Fp8DecParams {
     const float* s1; int64_t s1_rs, s1_cs;
     const float* s2; int64_t s2_rs, s2_cs;
     int gsM;
-    // row / column scale form (RC): out = (sum * cs[n * cs_stride]) * rs[m * rs_stride] + bias[n]; strides 0 (one scale) or 1
-    const float* rs; const float* cs; const float* bias;
-    int rs_stride, cs_stride;
+    const float* bias;
     // K in segments (SEG instantiations, gridDim.y of them): fp32 sums of this pass's rows, slice s at part + s * part_slice
     float* part; int64_t part_slice;
 };
@@ -61,10 +59,9 @@ __device__ __forceinline__ v4i widen8_e4m3(uint32_t d0, uint32_t d1)
 // NBLK blocks from (s NW + w) NBLK on, and a wave whose blocks lie past the end of K (in the last segment; K is a whole
 // number of NBLK blocks) runs along on the last blocks and contributes zeros.  With more than one segment the
 // workgroup stores its fp32 sums for fp8dec_reduce_kernel, which adds the segments in order and applies the epilogue.
-template <int NW, int NBLK, bool RC, bool I8 = false, bool SEG = false>
+template <int NW, int NBLK, bool I8 = false, bool SEG = false>
 __global__ __launch_bounds__(NW * 64) void fp8_block_decode_kernel(Fp8DecParams p)
 {
-    static_assert(!(RC && I8), "int8: the block-scale form only");
     constexpr int NCH = 2 * NBLK;                    // 64-byte chunks of an x2 row in a wave's K range
     constexpr int PF = NW == 16 ? (NCH < 4 ? NCH : 4) : NCH;   // pieces in flight per lane; divides NCH
     static_assert(NCH % PF == 0, "a piece's slot must not depend on the column block");
@@ -99,11 +96,9 @@ __global__ __launch_bounds__(NW * 64) void fp8_block_decode_kernel(Fp8DecParams 
     }
     // the scales of this lane's row of x1 for the wave's blocks (rows past M: the last row's, their outputs are not stored)
     float s1v[NBLK];
-    if constexpr (!RC) {
-        const int64_t mr = (nrow < M ? nrow : M - 1) / p.gsM;
+    const int64_t mr = (nrow < M ? nrow : M - 1) / p.gsM;
 #pragma unroll
-        for (int j = 0; j < NBLK; j++) s1v[j] = p.s1[mr * p.s1_rs + (kb0 + j) * p.s1_cs];
-    }
+    for (int j = 0; j < NBLK; j++) s1v[j] = p.s1[mr * p.s1_rs + (kb0 + j) * p.s1_cs];
 
     auto wload = [&](int rb, int c) {
         const int64_t n = (int64_t)rb * 16 + nrow;
@@ -118,14 +113,12 @@ __global__ __launch_bounds__(NW * 64) void fp8_block_decode_kernel(Fp8DecParams 
         const int rbn = rb + (int)gridDim.x < nblocks ? rb + (int)gridDim.x : rb;   // past the end: a harmless reload
         const int64_t n0 = (int64_t)rb * 16;
         float s2v[NBLK];
-        if constexpr (!RC) {
 #pragma unroll
-            for (int j = 0; j < NBLK; j++) s2v[j] = p.s2[(kb0 + j) * p.s2_rs + (n0 / 128) * p.s2_cs];
-        }
+        for (int j = 0; j < NBLK; j++) s2v[j] = p.s2[(kb0 + j) * p.s2_rs + (n0 / 128) * p.s2_cs];
         v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int j = 0; j < NBLK; j++) {
-            v4f t = RC ? acc : (v4f){0.0f, 0.0f, 0.0f, 0.0f};   // RC: one chain over the whole range
+            v4f t = {0.0f, 0.0f, 0.0f, 0.0f};
             v4i ti = {0, 0, 0, 0};
 #pragma unroll
             for (int cc = 0; cc < 2; cc++) {
@@ -141,12 +134,9 @@ __global__ __launch_bounds__(NW * 64) void fp8_block_decode_kernel(Fp8DecParams 
                 }
             }
             if constexpr (I8) t = (v4f){(float)ti[0], (float)ti[1], (float)ti[2], (float)ti[3]};
-            if constexpr (RC) acc = t;
-            else {
-                const float sc = s1v[j] * s2v[j];
+            const float sc = s1v[j] * s2v[j];
 #pragma unroll
-                for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf(t[r], sc, acc[r]);
-            }
+            for (int r = 0; r < 4; r++) acc[r] = __builtin_fmaf(t[r], sc, acc[r]);
         }
         // acc[r]: m = lane % 16, n = n0 + 4 (lane / 16) + r, over this wave's K range
         if constexpr (SEG) {
@@ -175,15 +165,7 @@ __global__ __launch_bounds__(NW * 64) void fp8_block_decode_kernel(Fp8DecParams 
                 continue;
             }
         }
-        if constexpr (RC) {   // (sum * x2Scale[n]) * x1Scale[m] + bias[n], each operation rounded
-            const float rsv = p.rs[(int64_t)nrow * p.rs_stride];
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int64_t ni = n + r < p.N ? n + r : p.N - 1;
-                sum[r] = (sum[r] * p.cs[ni * p.cs_stride]) * rsv;
-                if (p.bias) sum[r] = sum[r] + p.bias[ni];
-            }
-        } else if (p.bias) {
+        if (p.bias) {
 #pragma unroll
             for (int r = 0; r < 4; r++) sum[r] = sum[r] + p.bias[n + r < p.N ? n + r : p.N - 1];
         }
@@ -205,27 +187,25 @@ __global__ __launch_bounds__(NW * 64) void fp8_block_decode_kernel(Fp8DecParams 
     }
 }
 
-// out = epilogue(sum over the K segments, in order, of part[s]) for one pass of up to 16 rows: the block-scale form adds the
-// bias, the row / column scale form (RC) computes (sum * x2Scale[n]) * x1Scale[m] + bias[n]
-template <int W, bool RC>
+// out = cast(sum over the K segments, in order, of part[s] + bias)
+template <int W>
 __global__ __launch_bounds__(256) void fp8dec_reduce_kernel(Fp8DecParams p, int splits)
 {
     splitk_rows<W>((const float*)p.part, splits, p.part_slice, p.M, p.N, [&](int64_t m, int64_t n0, float (&v)[W]) {
 #pragma unroll
         for (int e = 0; e < W; e++) {
             const int64_t n = n0 + e;
-            if constexpr (RC) v[e] = (v[e] * p.cs[n * p.cs_stride]) * p.rs[m * p.rs_stride];
             if (p.bias) v[e] = v[e] + p.bias[n];
         }
         store_cols(p.out, p.out_dt, m * p.N + n0, v);
     });
 }
 
-template <int NW, int NBLK, bool RC, bool I8 = false, bool SEG = false>
+template <int NW, int NBLK, bool I8 = false, bool SEG = false>
 int launch_decode_one(const Fp8DecParams& p, hipStream_t st, int splits = 1)
 {
     if constexpr (!SEG) {
-        if (splits > 1 || p.K != (int64_t)NW * NBLK * 128) return launch_decode_one<NW, NBLK, RC, I8, true>(p, st, splits);
+        if (splits > 1 || p.K != (int64_t)NW * NBLK * 128) return launch_decode_one<NW, NBLK, I8, true>(p, st, splits);
     }
     const int64_t nbk = p.K / 128;
     if (splits < 1 || splits > 16 || nbk % NBLK != 0 || nbk < NBLK || (int64_t)splits * NW * NBLK < nbk || (splits > 1 && !p.part)) return -1;
@@ -233,29 +213,29 @@ int launch_decode_one(const Fp8DecParams& p, hipStream_t st, int splits = 1)
     const int cus = 256 / splits;   // the CUs shared between the segments' workgroup columns
     const int grid = nblocks < cus ? nblocks : cus;
     const size_t lds = (size_t)2 * NW * 256 * sizeof(float);
-    hipLaunchKernelGGL((fp8_block_decode_kernel<NW, NBLK, RC, I8, SEG>), dim3((unsigned)grid, (unsigned)splits), dim3(NW * 64), lds, st, p);
+    hipLaunchKernelGGL((fp8_block_decode_kernel<NW, NBLK, I8, SEG>), dim3((unsigned)grid, (unsigned)splits), dim3(NW * 64), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
-    splitk_launch(p.M, p.N, [&](auto w, dim3 g, dim3 b) { hipLaunchKernelGGL((fp8dec_reduce_kernel<decltype(w)::value, RC>), g, b, 0, st, p, splits); });
+    splitk_launch(p.M, p.N, [&](auto w, dim3 g, dim3 b) { hipLaunchKernelGGL((fp8dec_reduce_kernel<decltype(w)::value>), g, b, 0, st, p, splits); });
     return (int)hipGetLastError();
 }
 
-template <bool RC, bool I8 = false>
+template <bool I8>
 int launch_decode_split(const Fp8DecParams& p, int nw, int nblk, hipStream_t st, int splits = 1)
 {
     if (nw == 16) {
-        if (nblk == 1) return launch_decode_one<16, 1, RC, I8>(p, st, splits);
-        if (nblk == 2) return launch_decode_one<16, 2, RC, I8>(p, st, splits);
-        if (nblk == 4) return launch_decode_one<16, 4, RC, I8>(p, st, splits);
+        if (nblk == 1) return launch_decode_one<16, 1, I8>(p, st, splits);
+        if (nblk == 2) return launch_decode_one<16, 2, I8>(p, st, splits);
+        if (nblk == 4) return launch_decode_one<16, 4, I8>(p, st, splits);
         return -1;
     }
     switch (nblk) {
-        case 1: return launch_decode_one<8, 1, RC, I8>(p, st, splits);
-        case 2: return launch_decode_one<8, 2, RC, I8>(p, st, splits);
-        case 3: return launch_decode_one<8, 3, RC, I8>(p, st, splits);
-        case 4: return launch_decode_one<8, 4, RC, I8>(p, st, splits);
-        case 5: return launch_decode_one<8, 5, RC, I8>(p, st, splits);
-        case 6: return launch_decode_one<8, 6, RC, I8>(p, st, splits);
-        case 7: return launch_decode_one<8, 7, RC, I8>(p, st, splits);
+        case 1: return launch_decode_one<8, 1, I8>(p, st, splits);
+        case 2: return launch_decode_one<8, 2, I8>(p, st, splits);
+        case 3: return launch_decode_one<8, 3, I8>(p, st, splits);
+        case 4: return launch_decode_one<8, 4, I8>(p, st, splits);
+        case 5: return launch_decode_one<8, 5, I8>(p, st, splits);
+        case 6: return launch_decode_one<8, 6, I8>(p, st, splits);
+        case 7: return launch_decode_one<8, 7, I8>(p, st, splits);
         default: return -1;
     }
 }
@@ -604,8 +584,8 @@ int launch_mx8_one(const Mx8DecParams& p, hipStream_t st, int splits)
 
 }  // namespace
 
-// fp8 e4m3 block scales (or int8 per-tile: the same scales, an fp32 bias, 16-bit output) with up to 32 rows of x1 (two
-// passes beyond 16), K-contiguous operands, K a whole number of 128-element blocks as qmm_decode_plan lays them out (more
+// fp8 e4m3 block scales (or int8 per-tile: the same scales, an fp32 bias, 16-bit output) with up to 16 rows of x1,
+// K-contiguous operands, K a whole number of 128-element blocks as qmm_decode_plan lays them out (more
 // than one segment only with room for the partial sums in sk); OPSNN_NOT_TAKEN otherwise.
 int launch_blockscale_decode(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
 {
@@ -613,8 +593,7 @@ int launch_blockscale_decode(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
     if ((!i8 && (a.x1_dtype != DT_E4M3 || a.x2_dtype != DT_E4M3)) || a.batch != 1) return OPSNN_NOT_TAKEN;
     if (a.out_dtype != DT_BF16 && a.out_dtype != DT_F16 && !(a.out_dtype == DT_F32 && !i8)) return OPSNN_NOT_TAKEN;
     if (a.bias && !(i8 && a.bias_dtype == DT_F32)) return OPSNN_NOT_TAKEN;
-    // (int8: 17 .. 32 rows are one pass of the tile kernel with K split, ahead of two passes here: 32 x 18432 x 7168 66 us here, 42 there)
-    if (a.M > (i8 ? 16 : 32) || a.N < 256) return OPSNN_NOT_TAKEN;
+    if (a.M > 16 || a.N < 256) return OPSNN_NOT_TAKEN;
     if (a.gsK != 128 || a.gsN != 128 || (a.gsM != 1 && a.gsM != 128)) return OPSNN_NOT_TAKEN;
     if (a.K % 128 != 0 || a.x1.col_stride != 1 || a.x2.row_stride != 1) return OPSNN_NOT_TAKEN;
     if (((uintptr_t)a.x1.ptr | (uintptr_t)a.x2.ptr | (uint64_t)a.x1.row_stride | (uint64_t)a.x2.col_stride) % 16) return OPSNN_NOT_TAKEN;
@@ -622,56 +601,20 @@ int launch_blockscale_decode(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
     if (a.x1.row_stride < a.K || a.x2.col_stride < a.K) return OPSNN_NOT_TAKEN;
     QmmDecodePlan pl;
     if (!qmm_decode_plan(a.K, sk.part != nullptr, pl) || pl.splits > (sk.part ? sk.splits : 1)) return OPSNN_NOT_TAKEN;
-    for (int64_t m0 = 0; m0 < a.M; m0 += 16) {
-        Fp8DecParams p{};
-        p.M = a.M - m0 < 16 ? a.M - m0 : 16; p.N = a.N; p.K = a.K;
-        p.a = (const uint8_t*)a.x1.ptr + m0 * a.x1.row_stride; p.b = (const uint8_t*)a.x2.ptr;
-        p.lda = a.x1.row_stride; p.ldb = a.x2.col_stride;
-        p.out_dt = a.out_dtype;
-        p.out = (char*)a.out + m0 * a.N * (a.out_dtype == DT_F32 ? 4 : 2);
-        p.part = sk.part ? sk.part + m0 * a.N : nullptr; p.part_slice = a.M * a.N;
-        p.gsM = (int)a.gsM;
-        // gsM 1: the pass's own rows of the scale table; gsM 128: up to 32 rows share row 0
-        p.s1 = (const float*)a.x1_scale_mat.ptr + (a.gsM == 1 ? m0 * a.x1_scale_mat.row_stride : 0);
-        p.s1_rs = a.x1_scale_mat.row_stride; p.s1_cs = a.x1_scale_mat.col_stride;
-        p.s2 = (const float*)a.x2_scale_mat.ptr; p.s2_rs = a.x2_scale_mat.row_stride; p.s2_cs = a.x2_scale_mat.col_stride;
-        p.bias = (const float*)a.bias;
-        const int rc = i8 ? launch_decode_split<false, true>(p, pl.nw, pl.nblk, st, pl.splits) : launch_decode_split<false>(p, pl.nw, pl.nblk, st, pl.splits);
-        if (rc != 0) return rc;
-    }
-    return 0;
+    Fp8DecParams p{};
+    p.M = a.M; p.N = a.N; p.K = a.K;
+    p.a = (const uint8_t*)a.x1.ptr; p.b = (const uint8_t*)a.x2.ptr;
+    p.lda = a.x1.row_stride; p.ldb = a.x2.col_stride;
+    p.out_dt = a.out_dtype; p.out = a.out;
+    p.part = sk.part; p.part_slice = a.M * a.N;
+    p.gsM = (int)a.gsM;
+    p.s1 = (const float*)a.x1_scale_mat.ptr; p.s1_rs = a.x1_scale_mat.row_stride; p.s1_cs = a.x1_scale_mat.col_stride;
+    p.s2 = (const float*)a.x2_scale_mat.ptr; p.s2_rs = a.x2_scale_mat.row_stride; p.s2_cs = a.x2_scale_mat.col_stride;
+    p.bias = (const float*)a.bias;
+    return i8 ? launch_decode_split<true>(p, pl.nw, pl.nblk, st, pl.splits) : launch_decode_split<false>(p, pl.nw, pl.nblk, st, pl.splits);
 }
 
-// fp8 e4m3 with one fp32 scale per row of x1 (or one) and one per column of x2 (or one), optional fp32 bias -- the form
-// (sum * x2Scale) * x1Scale + bias of compute_pertoken (qbmmv3_kernel_golden.py:361-387) -- for up to 32 rows.
-int launch_rowcol_decode(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
-{
-    if (a.x1_dtype != DT_E4M3 || a.x2_dtype != DT_E4M3 || a.batch != 1) return OPSNN_NOT_TAKEN;
-    if (a.out_dtype != DT_BF16 && a.out_dtype != DT_F16 && a.out_dtype != DT_F32) return OPSNN_NOT_TAKEN;
-    if (!a.x1_scale || !a.x2_scale || a.x2_scale_dtype != DT_F32 || (a.bias && a.bias_dtype != DT_F32)) return OPSNN_NOT_TAKEN;
-    if (a.M > 32 || a.N < 256 || a.x1.col_stride != 1 || a.x2.row_stride != 1) return OPSNN_NOT_TAKEN;
-    if (((uintptr_t)a.x1.ptr | (uintptr_t)a.x2.ptr | (uint64_t)a.x1.row_stride | (uint64_t)a.x2.col_stride) % 16) return OPSNN_NOT_TAKEN;
-    if (a.x1.row_stride < a.K || a.x2.col_stride < a.K) return OPSNN_NOT_TAKEN;
-    QmmDecodePlan pl;
-    if (!qmm_decode_plan(a.K, sk.part != nullptr, pl) || pl.splits > (sk.part ? sk.splits : 1)) return OPSNN_NOT_TAKEN;
-    for (int64_t m0 = 0; m0 < a.M; m0 += 16) {
-        Fp8DecParams p{};
-        p.M = a.M - m0 < 16 ? a.M - m0 : 16; p.N = a.N; p.K = a.K;
-        p.a = (const uint8_t*)a.x1.ptr + m0 * a.x1.row_stride; p.b = (const uint8_t*)a.x2.ptr;
-        p.lda = a.x1.row_stride; p.ldb = a.x2.col_stride;
-        p.out_dt = a.out_dtype;
-        p.out = (char*)a.out + m0 * a.N * (a.out_dtype == DT_F32 ? 4 : 2);
-        p.rs_stride = a.x1_scale_len == 1 ? 0 : 1; p.cs_stride = a.x2_scale_len == 1 ? 0 : 1;
-        p.rs = (const float*)a.x1_scale + (p.rs_stride ? m0 : 0);
-        p.cs = (const float*)a.x2_scale; p.bias = (const float*)a.bias;
-        p.part = sk.part ? sk.part + m0 * a.N : nullptr; p.part_slice = a.M * a.N;
-        const int rc = launch_decode_split<true>(p, pl.nw, pl.nblk, st, pl.splits);
-        if (rc != 0) return rc;
-    }
-    return 0;
-}
-
-// fp8 x fp4 MX with up to 32 rows of x1 (two passes beyond 16): K a whole number of 128-element chunks that 16 waves
+// fp8 x fp4 MX with up to 16 rows of x1: K a whole number of 128-element chunks that 16 waves
 // share 2 or 4 each, or 8 waves 1 .. 7 each; K-contiguous operands and scales; OPSNN_NOT_TAKEN otherwise.
 int launch_mx_a8w4_decode(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
 {
@@ -717,13 +660,13 @@ int launch_mx_a8w4_decode(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
     return 0;
 }
 
-// MXFP8 with up to 32 rows of x1 (two passes beyond 16): K-contiguous operands and scale rows ([rows, K / 64, 2] bytes), K a
+// MXFP8 with up to 16 rows of x1: K-contiguous operands and scale rows ([rows, K / 64, 2] bytes), K a
 // whole number of 128-element blocks as qmm_decode_plan lays them out; OPSNN_NOT_TAKEN otherwise.
 int launch_mxfp8_decode(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
 {
     if (a.x1_dtype != DT_E4M3 || a.x2_dtype != DT_E4M3 || a.batch != 1) return OPSNN_NOT_TAKEN;
     if (a.out_dtype != DT_BF16 && a.out_dtype != DT_F16 && a.out_dtype != DT_F32) return OPSNN_NOT_TAKEN;
-    if (a.M > 32 || a.N < 256 || a.K % 128 != 0 || a.x1.col_stride != 1 || a.x2.row_stride != 1) return OPSNN_NOT_TAKEN;
+    if (a.M > 16 || a.N < 256 || a.K % 128 != 0 || a.x1.col_stride != 1 || a.x2.row_stride != 1) return OPSNN_NOT_TAKEN;
     if (a.x1_scale_mat.col_stride != 2 || a.x2_scale_mat.col_stride != 2) return OPSNN_NOT_TAKEN;   // [rows, K / 64, 2]: a row's bytes contiguous
     if (a.bias && a.bias_dtype != DT_F32) return OPSNN_NOT_TAKEN;
     if (a.x1.row_stride < a.K || a.x2.col_stride < a.K) return OPSNN_NOT_TAKEN;
@@ -732,32 +675,29 @@ int launch_mxfp8_decode(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk)
     if (a.x1_scale_mat.row_stride < a.K / 32 || a.x2_scale_mat.row_stride < a.K / 32) return OPSNN_NOT_TAKEN;
     QmmDecodePlan pl;
     if (!qmm_decode_plan(a.K, sk.part != nullptr, pl) || pl.splits > (sk.part ? sk.splits : 1)) return OPSNN_NOT_TAKEN;
-    for (int64_t m0 = 0; m0 < a.M; m0 += 16) {
-        Mx8DecParams p{};
-        p.M = a.M - m0 < 16 ? a.M - m0 : 16; p.N = a.N; p.K = a.K;
-        p.a = (const uint8_t*)a.x1.ptr + m0 * a.x1.row_stride; p.b = (const uint8_t*)a.x2.ptr;
-        p.lda = a.x1.row_stride; p.ldb = a.x2.col_stride;
-        p.sa = (const uint8_t*)a.x1_scale_mat.ptr + m0 * a.x1_scale_mat.row_stride; p.sb = (const uint8_t*)a.x2_scale_mat.ptr;
-        p.sa_rs = a.x1_scale_mat.row_stride; p.sb_rs = a.x2_scale_mat.row_stride;
-        p.out_dt = a.out_dtype; p.out = (char*)a.out + m0 * a.N * (a.out_dtype == DT_F32 ? 4 : 2);
-        p.bias = (const float*)a.bias;
-        p.part = sk.part ? sk.part + m0 * a.N : nullptr; p.part_slice = a.M * a.N;
-        int rc = -1;
-        if (pl.nw == 16) rc = pl.nblk == 1 ? launch_mx8_one<16, 1>(p, st, pl.splits) : pl.nblk == 2 ? launch_mx8_one<16, 2>(p, st, pl.splits)
-                              : pl.nblk == 4 ? launch_mx8_one<16, 4>(p, st, pl.splits) : -1;
-        else switch (pl.nblk) {
-            case 1: rc = launch_mx8_one<8, 1>(p, st, pl.splits); break;
-            case 2: rc = launch_mx8_one<8, 2>(p, st, pl.splits); break;
-            case 3: rc = launch_mx8_one<8, 3>(p, st, pl.splits); break;
-            case 4: rc = launch_mx8_one<8, 4>(p, st, pl.splits); break;
-            case 5: rc = launch_mx8_one<8, 5>(p, st, pl.splits); break;
-            case 6: rc = launch_mx8_one<8, 6>(p, st, pl.splits); break;
-            case 7: rc = launch_mx8_one<8, 7>(p, st, pl.splits); break;
-            default: break;
-        }
-        if (rc != 0) return rc;
+    Mx8DecParams p{};
+    p.M = a.M; p.N = a.N; p.K = a.K;
+    p.a = (const uint8_t*)a.x1.ptr; p.b = (const uint8_t*)a.x2.ptr;
+    p.lda = a.x1.row_stride; p.ldb = a.x2.col_stride;
+    p.sa = (const uint8_t*)a.x1_scale_mat.ptr; p.sb = (const uint8_t*)a.x2_scale_mat.ptr;
+    p.sa_rs = a.x1_scale_mat.row_stride; p.sb_rs = a.x2_scale_mat.row_stride;
+    p.out_dt = a.out_dtype; p.out = a.out;
+    p.bias = (const float*)a.bias;
+    p.part = sk.part; p.part_slice = a.M * a.N;
+    int rc = -1;
+    if (pl.nw == 16) rc = pl.nblk == 1 ? launch_mx8_one<16, 1>(p, st, pl.splits) : pl.nblk == 2 ? launch_mx8_one<16, 2>(p, st, pl.splits)
+                          : pl.nblk == 4 ? launch_mx8_one<16, 4>(p, st, pl.splits) : -1;
+    else switch (pl.nblk) {
+        case 1: rc = launch_mx8_one<8, 1>(p, st, pl.splits); break;
+        case 2: rc = launch_mx8_one<8, 2>(p, st, pl.splits); break;
+        case 3: rc = launch_mx8_one<8, 3>(p, st, pl.splits); break;
+        case 4: rc = launch_mx8_one<8, 4>(p, st, pl.splits); break;
+        case 5: rc = launch_mx8_one<8, 5>(p, st, pl.splits); break;
+        case 6: rc = launch_mx8_one<8, 6>(p, st, pl.splits); break;
+        case 7: rc = launch_mx8_one<8, 7>(p, st, pl.splits); break;
+        default: break;
     }
-    return 0;
+    return rc;
 }
 
 }  // namespace opsnn

@@ -235,6 +235,7 @@ static int mx_relayout_run(const OpsnnQmmArgs& a, const MxRelayout& R, char* w, 
 
 bool mxfp4_rows_wanted(const OpsnnQmmArgs& a);   // qmm_mxfp4_rows.hip
 int launch_mxfp4_rows(const OpsnnQmmArgs& a, hipStream_t st);
+int launch_fp8_stream(const OpsnnQmmArgs& a, Fp8xForm form, SplitK sk, hipStream_t st);   // qmm_fp8_stream.hip
 // What every matrix-core route of this file needs of the call, whatever x2's layout and K's tail: checked before any
 // pre-step is launched or a cache entry made.
 static bool mx_call_ok(const OpsnnQmmArgs& a)
@@ -242,7 +243,7 @@ static bool mx_call_ok(const OpsnnQmmArgs& a)
     const bool fp4 = a.x1_dtype == DT_E2M1 && a.x2_dtype == DT_E2M1, fp8 = a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E4M3;
     const bool a8w4 = a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E2M1;
     if (!fp4 && !fp8 && !a8w4) return false;
-    if (a8w4) {   // launch_mx_a8w4_mfma (qmm_fp8_block.hip): a tile kernel, and a streaming kernel for up to 32 rows
+    if (a8w4) {   // launch_mx_a8w4_mfma (qmm_fp8_block.hip): a tile kernel, and a streaming kernel for up to 16 rows
         if (a.out_dtype != DT_BF16 && a.out_dtype != DT_F16) return false;
         if (a.bias && a.bias_dtype != DT_F32 && a.bias_dtype != DT_BF16 && a.bias_dtype != DT_F16) return false;
         if (a.K % 32 != 0 || a.x1.col_stride != 1 || a.x1_scale_mat.col_stride != 2) return false;
@@ -286,7 +287,7 @@ static uint64_t mx_rows_bytes(const OpsnnQmmArgs& a)
 {
     // (whether or not opsnnSetFp8Fast is on: a workspace must not depend on a switch that may change between the two phases)
     if (a.force_variant == OPSNN_VARIANT_PLAIN || opsnn_force_plain() || !mx_call_ok(a)) return 0;
-    return align_up(mxfp8_rows_workspace(a), 256);
+    return align_up(mxfp8_rows_workspace(a), 256);   // (few enough rows for the stream kernel leave it unused)
 }
 uint64_t mx_workspace_bytes(const OpsnnQmmArgs& a)
 {
@@ -328,9 +329,11 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
     OpsnnQmmArgs planned = a;
     if (relayout) mx_relayout_view(planned, R, (char*)(uintptr_t)256);
     MxPad L;
-    const bool rows4 = fp4 && mxfp4_rows_wanted(a);   // few rows of MXFP4: the kernel that takes a K tail as it is
-    const bool pad = !rows4 && mx_pad_layout(planned, L);
-    if (!pad && !rows4 && planned.K % 128 != 0) return OPSNN_NOT_TAKEN;
+    // few rows: the kernels that take a K tail as it is
+    Fp8StreamPlan spl;
+    const bool rows4 = fp4 && mxfp4_rows_wanted(a), rows8 = fp8 && exact && fp8_stream_plan(a, FP8X_MX, sk.part != nullptr, spl);
+    const bool pad = !rows4 && !rows8 && mx_pad_layout(planned, L);
+    if (!pad && !rows4 && !rows8 && planned.K % 128 != 0) return OPSNN_NOT_TAKEN;
     if (planned.x2_scale_mat.col_stride != 2 || (fp4 || fp8 ? planned.x2_scale_mat.row_stride != (planned.K + 63) / 64 * 2 : planned.x2_scale_mat.row_stride % 4 != 0)) return OPSNN_NOT_TAKEN;
     if (pad && (!a.workspace || (uintptr_t)a.workspace % 16)) return OPSNN_NOT_TAKEN;
     if (relayout) {
@@ -353,6 +356,7 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         mx_relayout_view(a, R, w);
     }
     if (rows4) return launch_mxfp4_rows(a, st);
+    if (rows8) return launch_fp8_stream(a, FP8X_MX, sk, st);
     const bool small = a.M <= 128 || a.N <= 128;
     // 128 x 128 tiles also when 256 x 256 ones would be at most 64, a quarter of the CUs (1024 x 4096 x 4096: 22.9 against 28.0 us; at 128 tiles of 256 x 256 it is 42 against 32)
     const bool fp4_small = small || ((a.M + 255) / 256) * ((a.N + 255) / 256) * a.batch <= 64 || a.force_variant == OPSNN_VARIANT_MX_128;
@@ -362,14 +366,14 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         if (rc != 0) return rc;
     }
     if (a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E2M1) return launch_mx_a8w4_mfma(a, st, sk);   // fp8 x fp4: qmm_fp8_block.hip
-    if (fp8 && rows_region) {   // MXFP8 with 17 .. 128 rows: the many-rows streaming kernel on bf16 operands (exact products)
+    if (fp8 && rows_region) {   // MXFP8 with 65 .. 128 rows of a large x2: the many-rows streaming kernel on bf16 operands (exact products)
         if (!opsnnGetFp8Fast()) {
             const int rc = launch_mxfp8_rows(a, rows_region, st, sk);
             if (rc != OPSNN_NOT_TAKEN) return rc;
         }
         sk = SplitK{};   // (any partial sums were laid out for the kernel above; the tile kernels run unsplit)
     }
-    if (fp8 && a.M <= 32) {   // MXFP8 with up to 32 rows: the stream over x2 with x1 in registers (exact products)
+    if (fp8 && a.M <= 16) {   // MXFP8 with up to 16 rows: the stream over x2 with x1 in registers (exact products)
         const int rc = launch_mxfp8_decode(a, st, sk);
         if (rc != OPSNN_NOT_TAKEN) return rc;
         if (a.M * a.N < 64 * 64) return OPSNN_NOT_TAKEN;

@@ -411,14 +411,6 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 8
 // WF: 0 integer codes; 1 floating-point codes (e4m3) with one scale of x's type per channel; 2 e2m1 codes with e8m0
 // scales per 32 k, a row's scale bytes contiguous: a lane's 32 weights of a chunk are exactly one group, so its scale
 // is one byte per chunk, fetched with the weights like the 16-bit scales of the other forms.
-// WF 3: the fp8 block-scale matmul (quant_batch_matmul_v3, G-B / B-B) with 17 .. 128 rows (MB = 4 up to 64 rows, else 8): x is x1 widened to fp16 by a
-// pre-step, w is x2 in e4m3, widened in registers without a scale (exact products); a slab of x is exactly one
-// 128-element scale block (WK = 2 chunks of 64), each wave chains its chunk's two instructions from a zero accumulator
-// and folds the partial block sum in with one fused multiply-add by s1[m, kb] * s2[kb, n / 128] -- the products of the
-// two scales for all blocks and the slab's rows are laid down in LDS once per workgroup (its 128 columns lie in one
-// scale block of w).  The output type is the call's (bf16, fp16 or fp32).
-// WF 4: the fp8 row / column scale form (K-C, K-T) of the same operands: one chain over all of K, and the epilogue
-// computes (sum * x2Scale[n]) * x1Scale[m] + bias[n] (bs2 / bs1 with element strides bs2_cs / bs1_rs of 0 or 1).
 // SLDS (integer codes, a row's scales contiguous, power-of-two group count): the workgroup lays all scales and offsets of
 // its columns down in LDS once, one 32-bit word (scale | offset << 16) per column and group, instead of fetching two
 // 16-bit values per row block and chunk from global memory.  Such a load is one instruction per 16-bit value and touches
@@ -429,13 +421,10 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 8
 template <int XDT, int WBITS, int MB, int NB, int WN, int WK, bool HAS_OFF, int WF = 0, bool SLDS = false, bool KSP = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void wqmm_rows_kernel(WqParams p)
 {
-    static_assert(!KSP || WF <= 4, "K in segments: the weight-only forms and the fp8 forms");
     static_assert(WN * WK == 8, "eight waves");
     static_assert(!SLDS || WF == 0 || WF == 2, "the scale table serves the integer forms and the e8m0 bytes of e2m1 codes");
     static_assert(WF == 0 || !HAS_OFF, "floating-point weight codes have no offset");
     static_assert(WF != 2 || WBITS == 4 || (WBITS == 8 && WK == 2), "e8m0 group scales: e2m1 codes, or e4m3 codes on the instances with two K waves");
-    static_assert(WF != 3 || (WBITS == 8 && XDT == DT_F16 && WK == 2 && NB == 2), "the block-scale form: fp16 x, e4m3 w, a slab per 128-block");
-    static_assert(WF != 4 || (WBITS == 8 && XDT == DT_F16 && !HAS_OFF), "the row / column scale form: fp16 x, e4m3 w");
     constexpr int NT = 512;
     if (p.m_slab > 0) {   // several row slabs in one launch: this workgroup's is number blockIdx.y
         p.m_base += (int64_t)blockIdx.y * p.m_slab;
@@ -459,7 +448,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
     constexpr int XPR = KX / 8 / XH;     // 16-byte pieces per x row per slab
     constexpr int XBUF = 16 * MB * XROW; // one slab buffer
     constexpr int XITEMS = 16 * MB * XPR / NT;
-    constexpr int NBL = (WF >= 3 || WF == 1 || SLDS) ? NB : NB * (HAS_OFF ? 3 : 2);   // loads of one weight fetch
+    constexpr int NBL = (WF == 1 || SLDS) ? NB : NB * (HAS_OFF ? 3 : 2);   // loads of one weight fetch
     constexpr int LDS_MAIN = (2 * XBUF > WN * (WK - 1) * NB * MB * 4 * 64 * 4) ? 2 * XBUF : WN * (WK - 1) * NB * MB * 4 * 64 * 4;
     static_assert((16 * MB * XPR) % NT == 0 && XPR >= 16 && PF >= 2 && PPH >= 1 && STEPS == PPH * XH, "staging and prefetch shape");
     static_assert(MB <= 8 || (WF == 0 && SLDS) || WF == 1 || WF == 2, "the 192- / 256-row instances: integer codes with the scale table in LDS, or floating-point codes");
@@ -480,10 +469,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
             p.x += k0;
             p.w += k0 * WBITS / 8;
             if constexpr (WF == 2) p.scale = (const uint16_t*)((const uint8_t*)p.scale + k0 / 32);   // one e8m0 byte per 32 k
-            else if constexpr (WF == 3) {   // the block scales of the segment's first 128-block
-                p.bs1 += (k0 / 128) * p.bs1_cs;
-                p.bs2 += (k0 / 128) * p.bs2_rs;
-            }
             else if (p.group < p.K) {
                 const int64_t g0 = (k0 / p.group) * p.s_rs;
                 p.scale += g0;
@@ -593,18 +578,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
         for (int b = 0; b < MB; b++) acc[q][b] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
     const DqConst dqc = make_dq_const();
 
-    // WF 3: sct[kb][r] = s1[row r of the slab, kb] * s2[kb, this workgroup's column block], behind the x buffers (and the
-    // partial sums that take their place at the end); complete behind the loop's first barrier
-    float* sct = (float*)(sx + LDS_MAIN);
-    if constexpr (WF == 3) {
-        const int64_t nbw = ((int64_t)blockIdx.x * (16 * NB * WN)) / 128;
-        for (int i = tid; i < NSLAB * 16 * MB; i += NT) {
-            const int kb = i / (16 * MB), r = i - kb * (16 * MB);
-            const int64_t m = p.m_base + (r < rows ? r : rows - 1);
-            sct[i] = p.bs1[(m / p.bs_gsm) * p.bs1_rs + kb * p.bs1_cs] * p.bs2[kb * p.bs2_rs + nbw * p.bs2_cs];
-        }
-    }
-
     // SLDS: word (row rw of the workgroup's 16 NB WN columns, group gi) at stab[rw * P + (gi ^ swizzle(rw))], P = the power of
     // two at or above the groups per row; the swizzle (4 * (rw % 16), kept below P) spreads the 16 rows that one read touches
     // over the banks.  The table is complete behind the loop's first barrier.
@@ -658,14 +631,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
                 wq[j][q] = *(const v4i*)(wptr + q * wblk + (int64_t)cw * (WK * 64));
             }
             if constexpr (SLDS) { sq[j][q] = 0; oq[j][q] = 0; continue; }
-            if constexpr (WF >= 3 || WF == 1) sq[j][q] = 0;
+            if constexpr (WF == 1) sq[j][q] = 0;
             else if constexpr (WF == 2) sq[j][q] = srow8[q * sblk + (cw * WK + wk) * (KC / 32)];
             else sq[j][q] = srow[q * sblk + so];
             if constexpr (HAS_OFF) oq[j][q] = orow[q * sblk + so];
             else oq[j][q] = 0;
         }
     };
-    // pieces of a chunk's work (all forms but the block-scale one, which has its own order below)
+    // pieces of a chunk's work
     v4i aop[NB];                   // the dequantised weights of the K step about to be multiplied
     auto load_sow = [&](int cw, uint32_t (&sow)[NB]) {
         if constexpr (SLDS) {
@@ -689,14 +662,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
             if constexpr (WF == 0 && SLDS) out[q] = dequant8<XDT, WBITS, HAS_OFF, true>(wq[j][q], s, (uint16_t)sow[q], (uint16_t)(sow[q] >> 16), dqc);
             else if constexpr (WF == 0) out[q] = dequant8<XDT, WBITS, HAS_OFF, true>(wq[j][q], s, sq[j][q], oq[j][q], dqc);
             else if constexpr (WF == 1 || (WF == 2 && SLDS)) out[q] = dequant8_float<XDT, WBITS, true>(wq[j][q], s, (uint16_t)sow[q]);
-            else if constexpr (WF == 4) {
-                typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-                const uint32_t d0 = (uint32_t)wq[j][q][2 * s], d1 = (uint32_t)wq[j][q][2 * s + 1];
-                const h2v w0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d0, 1.0f, false), w1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d0, 1.0f, true);
-                const h2v w2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d1, 1.0f, false), w3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d1, 1.0f, true);
-                out[q] = (v4i){(int)__builtin_bit_cast(uint32_t, w0), (int)__builtin_bit_cast(uint32_t, w1),
-                               (int)__builtin_bit_cast(uint32_t, w2), (int)__builtin_bit_cast(uint32_t, w3)};
-            }
             else out[q] = dequant8_float<XDT, WBITS, true>(wq[j][q], s, bits_x<XDT>(e8m0_to_f32(sq[j][q])));
         }
     };
@@ -755,127 +720,46 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
             const bool more_x = sl + 1 < NSLAB * XH;
             if (!SPREAD && more_x) issue_x(sl + 1);
             const char* xs = sx + (sl & 1) * XBUF;
-            if constexpr (WF != 3) { if (h == 0) load_sow(cw, sow); }   // (behind the barrier: the first one also completes the scale table)
-            if constexpr (WF == 3) {
-                // this wave's half of block cw: two instructions per fragment pair from zero, then the fold
-                v4i aw[NB][2];
+            if (h == 0) load_sow(cw, sow);   // (behind the barrier: the first one also completes the scale table)
+            // A slab's work: per K step the x fragments are requested first, so that they arrive in the shadow of the
+            // step's dequantisation (vector ALU) instead of each pair of matrix instructions waiting for a read issued
+            // just in front of it.
 #pragma unroll
-                for (int q = 0; q < NB; q++) {
-                    const v4i pc = wq[j][q];
-#pragma unroll
-                    for (int s = 0; s < 2; s++) {
-                        typedef _Float16 h2v __attribute__((ext_vector_type(2)));
-                        const uint32_t d0 = (uint32_t)pc[2 * s], d1 = (uint32_t)pc[2 * s + 1];
-                        const h2v w0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d0, 1.0f, false), w1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d0, 1.0f, true);
-                        const h2v w2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d1, 1.0f, false), w3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(d1, 1.0f, true);
-                        aw[q][s] = (v4i){(int)__builtin_bit_cast(uint32_t, w0), (int)__builtin_bit_cast(uint32_t, w1),
-                                         (int)__builtin_bit_cast(uint32_t, w2), (int)__builtin_bit_cast(uint32_t, w3)};
+            for (int s = 0; s < PPH; s++) {
+                if constexpr (MB <= 8) {
+                    v4i bops[MB];
+                    read_frags(xs, s, bops);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (SPREAD) {   // the next slab's copies in two halves, behind the fragment requests of the first two steps
+                        constexpr int CPH = (XITEMS + 1) / 2;
+                        if (s < 2 && more_x) issue_x_part(sl + 1, s * CPH, CPH);
                     }
-                }
-                const float* scr = sct + cw * (16 * MB) + nrow;
-                if constexpr (MB > 4) {
-                    // 128 rows: two row blocks at a time, and the fold of a pair rides behind the next pair's matrix
-                    // instructions.  The empty asm statements pin each fold where it is written: left alone the compiler
-                    // postpones the folds, keeps all eight blocks' partial sums alive and spills the weight prefetch.
-                    v4f tp[2][NB];
-                    float scp[2] = {0.0f, 0.0f};
-#pragma unroll
-                    for (int bp = 0; bp <= MB / 2; bp++) {
-                        v4f tc[2][NB];
-                        float scc[2] = {0.0f, 0.0f};
-                        if (bp < MB / 2) {
-#pragma unroll
-                            for (int h = 0; h < 2; h++) {
-                                const int b = 2 * bp + h;
-                                const v4i b0 = *(const v4i*)(xs + xoff_at(b, 0)), b1 = *(const v4i*)(xs + xoff_at(b, 1));
-                                scc[h] = scr[16 * b];
-#pragma unroll
-                                for (int q = 0; q < NB; q++)
-                                    tc[h][q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, aw[q][0]), __builtin_bit_cast(v8h, b0), (v4f){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-                                for (int q = 0; q < NB; q++)
-                                    tc[h][q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, aw[q][1]), __builtin_bit_cast(v8h, b1), tc[h][q], 0, 0, 0);
-                            }
-                        }
-                        if (bp > 0) {
-#pragma unroll
-                            for (int h = 0; h < 2; h++)
-#pragma unroll
-                                for (int q = 0; q < NB; q++) {
-                                    v4f& a = acc[q][2 * (bp - 1) + h];
-#pragma unroll
-                                    for (int i = 0; i < 4; i++) a[i] = __builtin_fmaf(tp[h][q][i], scp[h], a[i]);
-                                    asm volatile("" : "+v"(a));
-                                }
-                        }
-#pragma unroll
-                        for (int h = 0; h < 2; h++) {
-                            scp[h] = scc[h];
-#pragma unroll
-                            for (int q = 0; q < NB; q++) tp[h][q] = tc[h][q];
-                        }
-                        __builtin_amdgcn_sched_barrier(0);
-                    }
+                    dequant_step(j, h * PPH + s, sow, aop);
+                    mma_step(aop, bops);
                 } else {
-#pragma unroll
-                for (int b = 0; b < MB; b++) {
-                    const v4i b0 = *(const v4i*)(xs + xoff_at(b, 0)), b1 = *(const v4i*)(xs + xoff_at(b, 1));
-                    const float sc = scr[16 * b];
-                    v4f t[NB];
-#pragma unroll
-                    for (int q = 0; q < NB; q++)
-                        t[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, aw[q][0]), __builtin_bit_cast(v8h, b0), (v4f){0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-#pragma unroll
-                    for (int q = 0; q < NB; q++)
-                        t[q] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, aw[q][1]), __builtin_bit_cast(v8h, b1), t[q], 0, 0, 0);
-#pragma unroll
-                    for (int q = 0; q < NB; q++)
-#pragma unroll
-                        for (int i = 0; i < 4; i++) acc[q][b][i] = __builtin_fmaf(t[q][i], sc, acc[q][b][i]);
-                }
-                }
-            }
-            if constexpr (WF != 3) {
-                // A slab's work: per K step the x fragments are requested first, so that they arrive in the shadow of the
-                // step's dequantisation (vector ALU) instead of each pair of matrix instructions waiting for a read issued
-                // just in front of it.
-#pragma unroll
-                for (int s = 0; s < PPH; s++) {
-                    if constexpr (MB <= 8) {
-                        v4i bops[MB];
-                        read_frags(xs, s, bops);
-                        __builtin_amdgcn_sched_barrier(0);
-                        if constexpr (SPREAD) {   // the next slab's copies in two halves, behind the fragment requests of the first two steps
-                            constexpr int CPH = (XITEMS + 1) / 2;
-                            if (s < 2 && more_x) issue_x_part(sl + 1, s * CPH, CPH);
-                        }
-                        dequant_step(j, h * PPH + s, sow, aop);
-                        mma_step(aop, bops);
-                    } else {
-                        // 256 rows: the fragments in four groups of four, two groups requested ahead of the matrix
-                        // instructions that use them (all sixteen at once would need 64 registers beside 128 sums)
-                        constexpr int Q = MB / 4;
-                        v4i b0[Q], b1[Q], b2[Q], b3[Q];
-                        read_frags_part(std::integral_constant<int, 0>{}, xs, s, b0);
-                        read_frags_part(std::integral_constant<int, Q>{}, xs, s, b1);
-                        __builtin_amdgcn_sched_barrier(0);
-                        dequant_step(j, h * PPH + s, sow, aop);
-                        __builtin_amdgcn_sched_barrier(0);
-                        constexpr int CPG = (XITEMS + 3) / 4;   // copies behind each of the first step's four groups
-                        if (s == 0 && more_x) issue_x_part(sl + 1, 0, CPG);
-                        mma_part(std::integral_constant<int, 0>{}, aop, b0);
-                        read_frags_part(std::integral_constant<int, 2 * Q>{}, xs, s, b2);
-                        if (s == 0 && more_x) issue_x_part(sl + 1, CPG, CPG);
-                        __builtin_amdgcn_sched_barrier(0);
-                        mma_part(std::integral_constant<int, Q>{}, aop, b1);
-                        read_frags_part(std::integral_constant<int, 3 * Q>{}, xs, s, b3);
-                        if (s == 0 && more_x) issue_x_part(sl + 1, 2 * CPG, CPG);
-                        __builtin_amdgcn_sched_barrier(0);
-                        mma_part(std::integral_constant<int, 2 * Q>{}, aop, b2);
-                        if (s == 0 && more_x) issue_x_part(sl + 1, 3 * CPG, CPG);
-                        __builtin_amdgcn_sched_barrier(0);
-                        mma_part(std::integral_constant<int, 3 * Q>{}, aop, b3);
-                    }
+                    // 256 rows: the fragments in four groups of four, two groups requested ahead of the matrix
+                    // instructions that use them (all sixteen at once would need 64 registers beside 128 sums)
+                    constexpr int Q = MB / 4;
+                    v4i b0[Q], b1[Q], b2[Q], b3[Q];
+                    read_frags_part(std::integral_constant<int, 0>{}, xs, s, b0);
+                    read_frags_part(std::integral_constant<int, Q>{}, xs, s, b1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    dequant_step(j, h * PPH + s, sow, aop);
+                    __builtin_amdgcn_sched_barrier(0);
+                    constexpr int CPG = (XITEMS + 3) / 4;   // copies behind each of the first step's four groups
+                    if (s == 0 && more_x) issue_x_part(sl + 1, 0, CPG);
+                    mma_part(std::integral_constant<int, 0>{}, aop, b0);
+                    read_frags_part(std::integral_constant<int, 2 * Q>{}, xs, s, b2);
+                    if (s == 0 && more_x) issue_x_part(sl + 1, CPG, CPG);
+                    __builtin_amdgcn_sched_barrier(0);
+                    mma_part(std::integral_constant<int, Q>{}, aop, b1);
+                    read_frags_part(std::integral_constant<int, 3 * Q>{}, xs, s, b3);
+                    if (s == 0 && more_x) issue_x_part(sl + 1, 2 * CPG, CPG);
+                    __builtin_amdgcn_sched_barrier(0);
+                    mma_part(std::integral_constant<int, 2 * Q>{}, aop, b2);
+                    if (s == 0 && more_x) issue_x_part(sl + 1, 3 * CPG, CPG);
+                    __builtin_amdgcn_sched_barrier(0);
+                    mma_part(std::integral_constant<int, 3 * Q>{}, aop, b3);
                 }
             }
             }
@@ -946,15 +830,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 v[i] = acc[q][b][i];
-                if constexpr (WF == 4) v[i] = (v[i] * p.bs2[(nn0 + i) * p.bs2_cs]) * p.bs1[m * p.bs1_rs];
                 if (p.bias) v[i] = v[i] + load_scalar_as_f32(p.bias, p.bias_dt, nn0 + i);
                 if constexpr (XDT == DT_BF16) v[i] = bf16_to_f32(bf16_bits(v[i]));   // the golden rounds bf16 results twice (a no-op)
-            }
-            if constexpr (WF >= 3) {
-                const v4f vv = {v[0], v[1], v[2], v[3]};
-                if (p.bs_out_dt == DT_F32) *(v4f*)((float*)p.y + m * p.N + nn0) = vv;
-                else *(v4us*)(p.y + m * p.N + nn0) = p.bs_out_dt == DT_BF16 ? pack4_b16<DT_BF16>(vv) : pack4_b16<DT_F16>(vv);
-                continue;
             }
             const v4us o = {bits_x<XDT>(v[0]), bits_x<XDT>(v[1]), bits_x<XDT>(v[2]), bits_x<XDT>(v[3])};
             *(v4us*)(p.y + m * p.N + nn0) = o;   // N % 16 == 0 here: 8-byte aligned
@@ -1448,26 +1325,6 @@ static void launch_wq_splitk_reduce(const WqParams& p, int splits, int y_dt, hip
     });
 }
 
-// the fp8 forms of the many-rows kernel: out[m, n] = cast(epilogue(sum over the K segments, in order, of part[s, m, n])); the
-// block-scale form has folded its scales in already, the row / column scale form (RC) computes
-// (sum * x2Scale[n]) * x1Scale[m] + bias[n] here as the kernel's own epilogue does
-template <int W, bool RC>
-static __global__ __launch_bounds__(256) void rows_bs_splitk_reduce_kernel(const float* part, int splits, int64_t M, int64_t N, const float* rs, int64_t rs_stride,
-                                                                           const float* cs, int64_t cs_stride, const float* bias, void* out, int out_dt)
-{
-    splitk_rows<W>(part, splits, M * N, M, N, [&](int64_t row, int64_t n0, float (&v)[W]) {
-        if constexpr (RC) {
-#pragma unroll
-            for (int e = 0; e < W; e++) {
-                const int64_t n = n0 + e;
-                v[e] = (v[e] * cs[n * cs_stride]) * rs[row * rs_stride];
-                if (bias) v[e] = v[e] + bias[n];
-            }
-        }
-        store_cols(out, out_dt, row * N + n0, v);
-    });
-}
-
 // One workgroup per CU (its waves fill the register file), or one per row block when there are fewer; with K split into
 // `splits` segments one workgroup column per segment, the CUs shared between the columns.
 template <int XDT, int WBITS, int NW, int NCH, bool HAS_OFF, int SCM, bool WFLT = false, bool TWO = false>
@@ -1585,7 +1442,7 @@ static int launch_rows_one(const WqParams& p, hipStream_t st)
 {
     if constexpr (!KSP) {   // K in segments: the instantiations of the 64-row instance with 128-column workgroups that know them
         if (p.ksplit > 1) {
-            if constexpr (MB == 4 && NB == 2 && WN == 4 && WK == 2 && WF <= 4 && !SLDS) return launch_rows_one<XDT, WBITS, MB, NB, WN, WK, HAS_OFF, WF, false, true>(p, st);
+            if constexpr (MB == 4 && NB == 2 && WN == 4 && WK == 2 && !SLDS) return launch_rows_one<XDT, WBITS, MB, NB, WN, WK, HAS_OFF, WF, false, true>(p, st);
             else return -1;
         }
     }
@@ -1625,32 +1482,21 @@ static int launch_rows_one(const WqParams& p, hipStream_t st)
     if constexpr (SLDS) lds_stab = (size_t)(16 * NB * WN) * GP * 4;
     constexpr size_t lds_red = (size_t)WN * (WK - 1) * NB * MB * 4 * 64 * 4;
     constexpr size_t lds_main = lds_x > lds_red ? lds_x : lds_red;
-    constexpr size_t lds_table = WF == 3 ? 65536 : 0;   // products of the block scales: (K / 128) * 16 MB floats, at most this
-    const size_t lds = lds_main + (WF == 3 ? (size_t)(kseg / 128) * 16 * MB * 4 : 0) + lds_stab;
-    if (lds > lds_main + lds_table + lds_stab) return OPSNN_NOT_TAKEN;
+    const size_t lds = lds_main + lds_stab;
     const unsigned grid = (unsigned)((p.N + 16 * NB * WN - 1) / (16 * NB * WN));
     const int64_t slabs = p.m_slab > 0 ? (p.m_end - p.m_base + p.m_slab - 1) / p.m_slab : 1;
     if (slabs < 1 || slabs > 65535 || p.m_rows > 16 * MB || (p.m_slab > 0 && p.m_slab != p.m_rows)) return -1;
     auto k = wqmm_rows_kernel<XDT, WBITS, MB, NB, WN, WK, HAS_OFF, WF, SLDS, KSP>;
     static std::atomic<uint64_t> attr_set{0};   // one bit per device: the attribute belongs to the (kernel, device) pair
     if (!device_flag_test(attr_set)) {
-        hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(SLDS ? 160 * 1024 : lds_main + lds_table));
+        hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(SLDS ? 160 * 1024 : lds_main));
         if (e != hipSuccess) return (int)e;
         device_flag_set(attr_set);
     }
     hipLaunchKernelGGL(k, dim3(grid, (unsigned)slabs, split ? (unsigned)p.ksplit : 1u), dim3(512), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
     if (split) {
-        if constexpr (WF == 3 || WF == 4) {
-            splitk_launch(p.M, p.N, [&](auto w, dim3 g, dim3 b) {
-                if constexpr (WF == 3)
-                    hipLaunchKernelGGL((rows_bs_splitk_reduce_kernel<decltype(w)::value, false>), g, b, 0, st, (const float*)p.part, p.ksplit, p.M, p.N,
-                                       (const float*)nullptr, (int64_t)0, (const float*)nullptr, (int64_t)0, (const float*)nullptr, (void*)p.y, p.bs_out_dt);
-                else
-                    hipLaunchKernelGGL((rows_bs_splitk_reduce_kernel<decltype(w)::value, true>), g, b, 0, st, (const float*)p.part, p.ksplit, p.M, p.N,
-                                       p.bs1, p.bs1_rs, p.bs2, p.bs2_cs, (const float*)p.bias, (void*)p.y, p.bs_out_dt);
-            });
-        } else launch_wq_splitk_reduce(p, p.ksplit, XDT, st);
+        launch_wq_splitk_reduce(p, p.ksplit, XDT, st);
         return (int)hipGetLastError();
     }
     return 0;
