@@ -78,7 +78,11 @@ template <int N>
 __device__ __forceinline__ void wait_copies()
 {
     static_assert(N >= 0 && N < 64, "vmcnt range");
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" : : "n"(N) : "memory");
+    // (the builtin, not its text: the compiler has to see that its own loads are in, or it waits for them again, and with them for
+    // every copy under way)
+    asm volatile("" : : : "memory");
+    __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4) << 14 | 7 << 4);
+    asm volatile("" : : : "memory");
 }
 
 // bytes of a K tile in a wave's ring, copies per tile
@@ -299,6 +303,7 @@ __global__ __launch_bounds__(256, 1) void fp8_stream_kernel(Fp8StreamParams p)
             wait_copies<(S - 2) * CPT>();
             issue(t + S, at); at = next(at);
             read(f1, at);
+            __builtin_amdgcn_sched_barrier(0);
             float sc = 1.0f;
             if constexpr (FORM == FP8X_BLOCK) sc = *(const float*)(smem + 4 * S * TILE + wave * (4 * FS_MOST_BLOCKS) + 4 * (t >> 1));
             open();
@@ -310,6 +315,7 @@ __global__ __launch_bounds__(256, 1) void fp8_stream_kernel(Fp8StreamParams p)
             wait_copies<(S - 2) * CPT>();
             issue(t + 1 + S, at); at = next(at);
             read(f0, at);
+            __builtin_amdgcn_sched_barrier(0);
             multiply(f1, std::true_type{}, sc);
         }
     }
@@ -488,6 +494,7 @@ __global__ __launch_bounds__(256, 2) void fp8_wide_kernel(Fp8StreamParams p)
             issue(t + S, at);
             at = at + 1 < S ? at + 1 : 0;
             read(then, at);
+            __builtin_amdgcn_sched_barrier(0);
             float sc = 1.0f;
             if constexpr (FORM == FP8X_BLOCK) sc = *(const float*)(smem + S * TILE + wave * (4 * FS_MOST_BLOCKS) + 4 * t);
             multiply(now, sc);
