@@ -61,19 +61,24 @@ __device__ __forceinline__ void dequant_8x8(const uint32_t (&q)[8][WBITS / 4], c
             }
         }
     } else {
+        // (4 bits: signed bytes of 16 times the weight, as in dequant8)
+        uint32_t even[8], odd[8];
+#pragma unroll
+        for (int i = 0; i < 8; i++) { odd[i] = q[i][0] & 0xf0f0f0f0u; even[i] = (q[i][0] << 4) & 0xf0f0f0f0u; }
 #pragma unroll
         for (int j = 0; j < 8; j++) {
-            const float scf = u2f((j & 1) ? scw[j / 2] & 0xffff0000u : scw[j / 2] << 16), off = u2f((j & 1) ? ofw[j / 2] & 0xffff0000u : ofw[j / 2] << 16);
+            const float sc1 = u2f((j & 1) ? scw[j / 2] & 0xffff0000u : scw[j / 2] << 16), scf = WBITS == 4 && !HAS_OFF ? 0.0625f * sc1 : sc1, off = u2f((j & 1) ? ofw[j / 2] & 0xffff0000u : ofw[j / 2] << 16);
 #pragma unroll
             for (int i = 0; i < 8; i += 2) {
                 float w[2];
 #pragma unroll
                 for (int r = 0; r < 2; r++) {
-                    if constexpr (WBITS == 4) w[r] = (float)((int)(q[i + r][0] << (28 - 4 * j)) >> 28);
+                    if constexpr (WBITS == 4) w[r] = (float)((int)((j & 1 ? odd : even)[i + r] << (24 - 8 * (j >> 1))) >> 24);
                     else w[r] = (float)((int)(q[i + r][j / 4 * (DW - 1)] << (24 - 8 * (j & 3))) >> 24);
                 }
                 if constexpr (HAS_OFF) {
-                    const uint32_t pk = pack2_bf16((v2f){w[0] + off, w[1] + off});
+                    const float one = WBITS == 4 ? 0.0625f : 1.0f;
+                    const uint32_t pk = pack2_bf16((v2f){__builtin_fmaf(w[0], one, off), __builtin_fmaf(w[1], one, off)});
                     w[0] = u2f(pk << 16);
                     w[1] = u2f(pk & 0xffff0000u);
                 }

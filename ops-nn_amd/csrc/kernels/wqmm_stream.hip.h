@@ -78,13 +78,20 @@ __device__ __forceinline__ v4i dequant8(const v4i& piece, int s, uint16_t sb, ui
     } else {
         // bf16: no packed bf16 arithmetic on this chip, so the two steps run in fp32 with a hardware
         // round-to-nearest-even conversion to bf16 after each
-        const float scf = bf16_to_f32(sb), off = bf16_to_f32(ob);
+        // 4 bits: a nibble at the top of its byte is a signed byte, 16 times the weight, which the conversion reads as it lies (exact, and so
+        // is the scale's sixteenth: 23 operations for 8 weights, 28 with every nibble moved to the bottom first; with an offset
+        // the many-columns kernels spill that way, and keep to the bottom)
+        const float scf = WBITS == 4 && !HAS_OFF ? 0.0625f * bf16_to_f32(sb) : bf16_to_f32(sb), off = bf16_to_f32(ob);
         float w[8];
         if constexpr (WBITS == 4) {
-            const uint32_t q = (uint32_t)piece[s];
+            const uint32_t q = (uint32_t)piece[s], odd = q & 0xf0f0f0f0u, even = (q << 4) & 0xf0f0f0f0u;
             const int ord[8] = {0, 4, 1, 5, 2, 6, 3, 7};
 #pragma unroll
-            for (int j = 0; j < 8; j++) w[j] = (float)(((int)(q << (28 - 4 * (NATURAL ? j : ord[j])))) >> 28);
+            for (int j = 0; j < 8; j++) {
+                const int i = NATURAL ? j : ord[j];
+                if constexpr (HAS_OFF) w[j] = (float)(((int)(q << (28 - 4 * i))) >> 28);
+                else w[j] = (float)(((int)((i & 1 ? odd : even) << (24 - 8 * (i >> 1)))) >> 24);
+            }
         } else {
 #pragma unroll
             for (int j = 0; j < 8; j++) w[j] = (float)(((int)((uint32_t)piece[2 * s + (j >> 2)] << (24 - 8 * (j & 3)))) >> 24);
