@@ -280,6 +280,18 @@ __device__ __forceinline__ void copy4_sbase(const void* base, uint32_t voff, uin
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dword %1, %2" : : "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
 }
 
+// All but the last N vector memory operations are done, and all LDS reads.
+template <int N>
+__device__ __forceinline__ void wait_copies()
+{
+    static_assert(N >= 0 && N < 64, "vmcnt range");
+    // (the builtin, not its text: the compiler has to see that its own loads are in, or it waits for them again, and with them for
+    // every copy under way)
+    asm volatile("" : : : "memory");
+    __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4) << 14 | 7 << 4);
+    asm volatile("" : : : "memory");
+}
+
 // Workgroup ids are dealt round-robin over the 8 XCDs; give each XCD (own L2) a contiguous
 // range of logical tile ids so that neighbouring tiles share operand panels in one L2.
 __device__ __forceinline__ uint32_t xcd_remap(uint32_t wg, uint32_t total)

@@ -32,6 +32,8 @@ uint64_t wq_kn_workspace(const OpsnnWqmmArgs& a);
 int launch_wq_kn(const OpsnnWqmmArgs& a, hipStream_t st);
 bool wq_nk_wanted(const OpsnnWqmmArgs& a, uint64_t* workspace);   // wq_nk.hip
 int launch_wq_nk(const OpsnnWqmmArgs& a, hipStream_t st);
+bool wq_wide_wanted(const OpsnnWqmmArgs& a, uint64_t* workspace);   // wq_wide.hip
+int launch_wq_wide(const OpsnnWqmmArgs& a, hipStream_t st);
 uint64_t mx_workspace_bytes(const OpsnnQmmArgs& a);
 bool mxfp4_rows_wanted(const OpsnnQmmArgs& a);   // qmm_mxfp4_rows.hip
 }  // namespace opsnn
@@ -436,7 +438,9 @@ extern "C" int opsnnWqmm(const OpsnnWqmmArgs* a, void* stream)
     WeightCacheScope cache_scope;
     if (!a || !a->x || !a->w.ptr || !a->scale.ptr || !a->y || a->M <= 0 || a->N <= 0 || a->K <= 0) return -1;
     if (a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain()) {
-        int rc = launch_wq_dense(*a, (hipStream_t)stream);
+        int rc = launch_wq_wide(*a, (hipStream_t)stream);
+        if (rc != OPSNN_NOT_TAKEN) return rc;
+        rc = launch_wq_dense(*a, (hipStream_t)stream);
         if (rc != OPSNN_NOT_TAKEN) return rc;
         rc = launch_wq_kn(*a, (hipStream_t)stream);
         if (rc != OPSNN_NOT_TAKEN) return rc;
@@ -483,9 +487,18 @@ static uint64_t qmm_workspace_base(const OpsnnQmmArgs* a, int mode)
     return ((uint64_t)a->N * (uint64_t)a->K * bits / 8) * nb;
 }
 
+static uint64_t wqmm_workspace_others(const OpsnnWqmmArgs* a);
 extern "C" uint64_t opsnnWqmmWorkspace(const OpsnnWqmmArgs* a)
 {
     if (!a || a->M <= 0 || a->N <= 0 || a->K <= 0) return 0;
+    // (the wide kernel's partial sums, or what the kernels behind it need for a weight at an unaligned address, which only phase 2 knows)
+    uint64_t wide = 0;
+    if (opsnn_force_plain() || a->force_variant == OPSNN_VARIANT_PLAIN || !wq_wide_wanted(*a, &wide)) wide = 0;
+    const uint64_t others = wqmm_workspace_others(a);
+    return wide > others ? wide : others;
+}
+static uint64_t wqmm_workspace_others(const OpsnnWqmmArgs* a)
+{
     const uint64_t bits = (a->w_dtype == DT_I4 || a->w_dtype == DT_E2M1) ? 4 : 8;
     // up to 16 rows against a long K: fp32 partial sums of the x-in-registers kernel's K split, in front of everything else
     // (from 17 rows against a narrow N and a long K: those of the many-rows kernel's K split)

@@ -74,16 +74,6 @@ __device__ __forceinline__ void copy2_lanes(const void* base, uint32_t voff, uin
     asm volatile("s_mov_b64 %0, exec\n\ts_mov_b64 exec, %4\n\ts_mov_b32 m0, %1\n\ts_nop 4\n\tglobal_load_lds_ushort %2, %3\n\ts_mov_b64 exec, %0"
                  : "=&s"(all) : "s"(lds), "v"(voff), "s"(base), "s"(LANES >= 64 ? ~0ull : (1ull << (LANES & 63)) - 1) : "memory", "m0");
 }
-template <int N>
-__device__ __forceinline__ void wait_copies()
-{
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    // (the builtin, not its text: the compiler has to see that its own loads are in, or it waits for them again, and with them for
-    // every copy under way)
-    asm volatile("" : : : "memory");
-    __builtin_amdgcn_s_waitcnt((N & 15) | (N >> 4) << 14 | 7 << 4);
-    asm volatile("" : : : "memory");
-}
 
 // bytes of a K tile in a wave's ring, copies per tile
 template <int MB, int NB, int FORM> constexpr int fs_tile = (MB + NB) * 1024 + (FORM == FP8X_BLOCK ? 256 : FORM == FP8X_MX ? 256 + (NB + 3) / 4 * 256 : 0);

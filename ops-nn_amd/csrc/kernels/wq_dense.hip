@@ -171,7 +171,8 @@ static double tile_kernel_us(const OpsnnWqmmArgs& a, const WqForm& f)
 // (Of 368 measured calls 362 go to the faster side or one within 3 % of it (profiles/weight_only_routes.txt): 1999 x 4096 x 11008
 // bf16 x int4 228 -> 164 us, [K, N] storage 613 -> 162; 1000 x 8192 x 28672 fp16 x int4 stays on the many-rows kernel, 477 against 526; 65 x 4096 x 22896 on the streaming kernel, 54 against 93; 192 x 8192 x 22896 on the tile kernel, 127
 // against 230; 128 x 11008 x 4096 in [K, N] storage with the re-layout, 61 against 75.)
-static bool dense_is_faster(const OpsnnWqmmArgs& a, double product_us)
+struct DenseEstimate { double here, other; };
+static DenseEstimate dense_estimate(const OpsnnWqmmArgs& a, double product_us)
 {
     const WqForm f = wq_form(a);
     const double codes = (double)a.N * (double)a.K;
@@ -179,6 +180,8 @@ static bool dense_is_faster(const OpsnnWqmmArgs& a, double product_us)
     const bool four = f.wbits == 4, tile_ok = a.K % (four ? 128 : 64) == 0 && f.group % 64 == 0;
     const bool no_table = !f.nk && f.group < a.K;
     const double tile_us = tile_kernel_us(a, f) * (no_table ? 1.25 : 1.0);
+    const double pass_rate = f.nk ? 6.0e6 : four ? 3.5e6 : 4.6e6;
+    const double here = 3.0 + codes * (2.0 + f.wbits / 8.0) / pass_rate + product_us + codes * 2.0e-7;
     if (f.rows) {
         const int64_t slab = wq_narrow_slab_rows(a.M, a.N, true);
         if (no_table && (slab ? slab : a.M) > 128) other = tile_us;
@@ -187,10 +190,22 @@ static bool dense_is_faster(const OpsnnWqmmArgs& a, double product_us)
     else if (a.M > 128 && tile_ok) other = tile_us;
     else if (f.stream) other = wq_passes_of_64_us(a.M, [&](int64_t r) { return wq_stream_pass_us(f.wbits, a.x_dtype == DT_BF16, r, a.N, a.K); });
     else if (wq_general_counts(a, f)) other = wq_passes_of_64_us(a.M, [&](int64_t r) { return wq_general_pass_us(r, a.N, a.K); });
-    else return true;
+    else return {here, 1e30};
     if (!f.nk) other += 2.0 + codes * f.wbits / 8.0 / (four ? 0.62e6 : 0.73e6);
-    const double pass_rate = f.nk ? 6.0e6 : four ? 3.5e6 : 4.6e6;
-    return 3.0 + codes * (2.0 + f.wbits / 8.0) / pass_rate + product_us + codes * 2.0e-7 < 0.97 * other;   // (in doubt without the pass)
+    return {here, other};
+}
+static bool dense_is_faster(const OpsnnWqmmArgs& a, double product_us)
+{
+    const DenseEstimate e = dense_estimate(a, product_us);
+    return e.here < 0.97 * e.other;   // (in doubt without the pass)
+}
+// What a K-contiguous call takes without the wide kernel (wq_wide.hip), from 33 rows: for its rule.
+double wq_many_rows_estimate(const OpsnnWqmmArgs& a)
+{
+    const WqForm f = wq_form(a);
+    if (a.M <= 64) return f.rows ? rows_kernel_us(a, f.wbits, f.group) : 1e30;
+    const DenseEstimate e = dense_estimate(a, dense_plan(a.M, a.N, a.K).us);
+    return a.K % 64 == 0 && a.N >= 128 && e.here < e.other ? e.here : e.other;
 }
 
 // Can the call run here?

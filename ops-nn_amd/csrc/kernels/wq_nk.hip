@@ -266,6 +266,14 @@ static bool nk_wanted(const OpsnnWqmmArgs& a, WqNkPlan& pl)
     else return true;
     return nk_us(f.wbits, bf16, a.M, a.N, a.K, pl) < other;
 }
+// What the kernel takes for a call of up to 64 rows with a shape of its own (others: a large number), for other kernels' rules.
+double wq_nk_estimate(const OpsnnWqmmArgs& a)
+{
+    WqNkPlan pl;
+    const WqForm f = wq_form(a);
+    if (a.M > 64 || a.K % 32 != 0 || a.K < 256 || a.N < 256 || !nk_plan(f.wbits, a.M, a.N, a.K, f.group, pl)) return 1e30;
+    return nk_us(f.wbits, a.x_dtype == DT_BF16, a.M, a.N, a.K, pl);
+}
 // ... and if so, the workspace it needs.
 bool wq_nk_wanted(const OpsnnWqmmArgs& a, uint64_t* workspace)
 {
