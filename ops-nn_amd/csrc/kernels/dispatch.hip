@@ -217,13 +217,13 @@ extern "C" __attribute__((visibility("hidden"))) int opsnn_qmm_k_pad(const Opsnn
 // per-tile from 33 rows) or on the exact fp8 kernel of qmm_fp8_exact.hip (fp8 block scales from 129 rows, MXFP8 from 33):
 // 1 = none.  Looks only at what the caller passed (shapes, types), so that the workspace query and the launch agree; a
 // route that ends on another kernel leaves the partial sums' share of the workspace unused.
-static int splitk_for(const OpsnnQmmArgs& a, int mode)
+static int splitk_for(const OpsnnQmmArgs& a, int mode, bool stream = true)
 {
     if (a.force_variant != 0 || opsnn_force_plain()) return 1;   // (a pinned kernel variant runs as it is)
     const bool out16 = a.out_dtype == DT_BF16 || a.out_dtype == DT_F16;
     const bool f8 = a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E4M3;
     // few rows of fp8: the stream kernel's
-    if (Fp8StreamPlan pl; f8 && mode >= 1 && mode <= 3 && fp8_stream_plan(a, mode == 1 ? FP8X_BLOCK : mode == 2 ? FP8X_MX : FP8X_PLAIN, true, pl)) return pl.splits;
+    if (Fp8StreamPlan pl; stream && f8 && mode >= 1 && mode <= 3 && fp8_stream_plan(a, mode == 1 ? FP8X_BLOCK : mode == 2 ? FP8X_MX : FP8X_PLAIN, true, pl)) return pl.splits;
     // up to 16 rows of fp8 with block or MX scales, of int8 per-tile and of fp8 x fp4 MX: the decode kernels' K segments
     const bool a8w4 = mode == 2 && a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E2M1;
     const bool i8pt = mode == 1 && a.x1_dtype == DT_I8 && a.x2_dtype == DT_I8;
@@ -383,22 +383,23 @@ extern "C" int opsnnQmmTc(const OpsnnQmmArgs* a, void* stream)
     // the other two forms run here.
     if (f8 && a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain()) {
         const int ep = !a->x1_scale ? 1 : (a->x1_scale_len == 1 && a->x2_scale_len == 1 && !a->bias) ? 2 : 0;
-        if (ep == 0) {   // up to 128 rows: the stream kernel
+        if (ep == 0) {   // few rows, small products: the stream kernel
             const int rc = launch_fp8_stream(*a, FP8X_PLAIN, sk, (hipStream_t)stream);
             if (rc != OPSNN_NOT_TAKEN) return rc;
         }
-        // (up to 128 rows the partial sums were laid out for the kernel above; the tile kernels run unsplit)
-        const SplitK sk_tiles = a->M <= 128 ? SplitK{} : sk;
+        // (partial sums that were laid out for the kernel above: the tile kernels run unsplit)
+        Fp8StreamPlan pl;
+        if (a->M <= 128 || fp8_stream_plan(*a, FP8X_PLAIN, true, pl)) sk = SplitK{};
         const bool e4 = a->x1_dtype == DT_E4M3 && a->x2_dtype == DT_E4M3;
         if (ep != 0 || !e4 || a->x2_scale_dtype != DT_F32 || a->out_dtype == DT_F32) {
-            const int rc = launch_rowcol_exact(*a, (hipStream_t)stream, ep, sk_tiles);
+            const int rc = launch_rowcol_exact(*a, (hipStream_t)stream, ep, sk);
             if (rc != OPSNN_NOT_TAKEN) return rc;
         }
     }
     // fp8 e4m3 operands with a row scale and a column scale that are multiplied in separately (K-C, K-T, T-C with the
     // one-element x1Scale): matrix-core kernel when the layout allows, else the plain kernel
     if (f8 && a->x1_scale && a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain()) {
-        const int rc = launch_fp8_rowcol_mfma(*a, (hipStream_t)stream, false, a->M <= 128 ? SplitK{} : sk);
+        const int rc = launch_fp8_rowcol_mfma(*a, (hipStream_t)stream, false, sk);
         if (rc != OPSNN_NOT_TAKEN) return rc;
     }
     NOTE_PLAIN("per-tensor / per-channel quant matmul", a);
@@ -462,7 +463,9 @@ extern "C" uint64_t opsnnQmmWorkspace(const OpsnnQmmArgs* a, int mode)
 {
     if (!a) return 0;
     const uint64_t need = splitk_bytes(*a, splitk_for(*a, mode)) + qmm_workspace_base(a, mode);   // partial sums of a K split in front
-    const uint64_t reserve = mode == 1 && !opsnn_force_plain() ? blockscale_rows_reserve(*a, nullptr) : 0;
+    uint64_t reserve = mode == 1 && !opsnn_force_plain() ? blockscale_rows_reserve(*a, nullptr) : 0;
+    // (above 128 rows: no less than what the tile kernels would use, which the stream kernel's rule stands in for)
+    if (a->M > 128 && mode >= 1 && mode <= 3) reserve = splitk_bytes(*a, splitk_for(*a, mode, false)) + qmm_workspace_base(a, mode);
     return need > reserve ? need : reserve;
 }
 

@@ -730,7 +730,7 @@ int launch_blockscale_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         }
         a.x2.row_stride = 1; a.x2.col_stride = a.K;
     }
-    if (!i8) {   // up to 128 rows: the stream kernel
+    if (!i8) {   // few rows, small products: the stream kernel
         const int rc = launch_fp8_stream(a, FP8X_BLOCK, sk, st);
         if (rc != OPSNN_NOT_TAKEN) return rc;
     }
@@ -739,7 +739,8 @@ int launch_blockscale_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         if (rc != OPSNN_NOT_TAKEN) return rc;
     }
     if (tiny) return OPSNN_NOT_TAKEN;
-    if (a.M <= (i8 ? 16 : 128)) sk = SplitK{};   // (with so few rows the partial sums were laid out for the kernels above; the tile kernels run unsplit)
+    // (partial sums that were laid out for the kernels above: the tile kernels run unsplit)
+    if (Fp8StreamPlan pl; a.M <= (i8 ? 16 : 128) || (!i8 && fp8_stream_plan(a0, FP8X_BLOCK, true, pl))) sk = SplitK{};
     if (!i8 && (!opsnnGetFp8Fast() || out32)) {   // exact products and sums unless the caller asked for the 8-bit matrix instruction
         const int rc = launch_blockscale_exact(a, st, sk);
         if (rc != OPSNN_NOT_TAKEN || out32) return rc;

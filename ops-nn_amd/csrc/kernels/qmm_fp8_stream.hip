@@ -621,14 +621,22 @@ uint64_t blockscale_rows_reserve(const OpsnnQmmArgs& a, int* segments)
 // Does a call run here, and how?  (Sizes, types, strides and which operands there are: both phases ask.  x2 K-contiguous, or re-laid
 // out so by then.)
 //
+// From 129 to 512 rows, in slabs of 64, K from 1024: small products, which leave most of the exact tile kernel's 128 x 128 tiles without a CU's worth
+// of work (row / column scales 181 x 2560 x 2368 16.4 us there, 11.1 here, 140 x 1536 x 17344 30.5 and 25.1; block scales 158 x 1152 x 2112 15.3
+// and 9.2, 405 x 1664 x 3848 24.2 and 18.9; MX 298 x 1280 x 1152 19.3 and 13.0; but 223 x 1024 x 15488 22.0 and 23.4, 258 x 3072 x 13440 41.8 and
+// 49.5), and, with row / column scales, somewhat larger ones with a
+// last half K tile, which run on padded copies there (246 x 12224 x 2560 76 and 49).
+//
 // Up to 128 rows.  Row / column scales always; block scales but for a K that the x-in-registers kernel of qmm_fp8_decode.hip shares
 // out evenly, up to 16 rows (16 x 7168 x 18432 29.9 us there, 32.8 here; 8 x 9856 x 23040, which it cuts, 61 and 44); MX the same, and from 65
 // rows on the many-rows kernel's large weights (128 x 11392 x 27904 132 there, 147 here; 128 x 9856 x 8128 82 and 50).
+constexpr int64_t FS_MANY_ROWS = 3200000000, FS_MANY_ROWS_TAIL = 12000000000;   // multiplications
 bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8StreamPlan& pl)
 {
     if (a.x1_dtype != DT_E4M3 || a.x2_dtype != DT_E4M3 || a.batch != 1 || a.force_variant != 0) return false;
     if (a.out_dtype != DT_BF16 && a.out_dtype != DT_F16 && a.out_dtype != DT_F32) return false;
-    if (a.M > 128 || a.N < 256 || a.K < 128 || a.K % 64 != 0 || a.K >= (1ll << 30) || a.N >= (1ll << 30)) return false;
+    if (a.M > 512 || a.N < 256 || a.K < 128 || a.K % 64 != 0 || a.K >= (1ll << 30) || a.N >= (1ll << 30)) return false;
+    if (a.M > 128 && (a.K < 1024 || a.M * a.N * a.K > (form == FP8X_PLAIN && a.K % 128 ? FS_MANY_ROWS_TAIL : FS_MANY_ROWS))) return false;
     const int64_t ldb = a.x2.row_stride == 1 ? a.x2.col_stride : a.K;
     if (a.x1.row_stride < 0 || a.x1.row_stride >= (1ll << 24) || ldb < 0 || ldb >= (1ll << 24)) return false;   // (32-bit lane offsets)
     if (form == FP8X_BLOCK) {
@@ -683,6 +691,7 @@ bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8St
 int launch_fp8_stream(const OpsnnQmmArgs& a, Fp8xForm form, SplitK sk, hipStream_t st)
 {
     Fp8StreamPlan pl;
+    if (a.M > 128 && a.K % 128 == 0 && opsnnGetFp8Fast()) return OPSNN_NOT_TAKEN;   // (the caller asked for the 8-bit instruction)
     if (!fp8_stream_plan(a, form, sk.part != nullptr, pl)) return OPSNN_NOT_TAKEN;
     // (partial sums laid out for other segments: a call that another layout of its operands has changed on the way)
     if (pl.splits > 1 && sk.splits < pl.splits && !fp8_stream_plan(a, form, false, pl)) return OPSNN_NOT_TAKEN;

@@ -253,8 +253,9 @@ static bool mx_call_ok(const OpsnnQmmArgs& a)
     }
     if (a.out_dtype != DT_BF16 && a.out_dtype != DT_F16 && a.out_dtype != DT_F32) return false;
     if (a.bias && a.bias_dtype != DT_F32) return false;
-    // (fewer than 64 x 64 outputs: only MXFP8's few-rows stream over x2, which wants 256 columns)
-    if (a.K % 32 != 0 || (a.M * a.N < 64 * 64 && !(fp8 && a.M <= 32 && a.N >= 256 && a.batch == 1 && a.K % 128 == 0) && !mxfp4_rows_wanted(a))) return false;
+    // (fewer than 64 x 64 outputs: only MXFP8's few-rows streams over x2, which want 256 columns and whole half tiles of K: on one thread
+    // per output 3 x 15168 x 1088 took 12.4 ms, 16 us here)
+    if (a.K % 32 != 0 || (a.M * a.N < 64 * 64 && !(fp8 && a.M <= 32 && a.N >= 256 && a.batch == 1 && a.K % 64 == 0) && !mxfp4_rows_wanted(a))) return false;
     const int64_t ks = (a.K + 63) / 64, epb = fp4 ? 2 : 1;
     if (a.x1.col_stride != 1 || a.x1_scale_mat.col_stride != 2 || a.x1_scale_mat.row_stride != ks * 2) return false;
     if (((uintptr_t)a.x1.ptr | (uint64_t)(a.x1.row_stride / epb) | (uint64_t)(a.x1.batch_stride / epb)) % 16) return false;

@@ -1,4 +1,4 @@
-"""fp8 with up to 128 rows of x1 on the stream kernels (qmm_fp8_stream.hip) through the two-phase entry point, against the oracle."""
+"""fp8 with up to 128 rows of x1, or small products of up to 512 rows, on the stream kernels (qmm_fp8_stream.hip) through the two-phase entry point, against the oracle."""
 import numpy as np
 import pytest
 
@@ -18,7 +18,8 @@ def _reset(gpu):
 # rows on either side of each row-block count and slab; columns that end inside a block of 16, of a wave and of a workgroup, and odd
 # counts; K of one block, fewer blocks than waves or stages, a wave with one block less than the others, segments with partial sums
 SHAPES = [(1, 128, 256), (15, 256, 257), (16, 1152, 300), (17, 384, 271), (32, 640, 1033), (33, 1280, 260), (48, 512, 2050), (64, 2176, 515),
-          (65, 1024, 258), (100, 640, 1100), (128, 1408, 530), (5, 2048, 4361), (40, 896, 8200), (64, 4608, 1030), (16, 13440, 258), (24, 8320, 390), (128, 7040, 280)]
+          (65, 1024, 258), (100, 640, 1100), (128, 1408, 530), (5, 2048, 4361), (40, 896, 8200), (64, 4608, 1030), (16, 13440, 258), (24, 8320, 390), (128, 7040, 280),
+          (129, 1024, 520), (193, 1152, 1030), (300, 3072, 771), (512, 1024, 257)]
 
 
 @pytest.mark.parametrize("M,K,N", SHAPES)
@@ -39,7 +40,8 @@ def test_block_scales(gpu, M, K, N, gsM, out):
 
 
 # (K % 128 == 64 as well: the narrow kernel, with four column blocks where N is wide)
-@pytest.mark.parametrize("M,K,N", SHAPES + [(3, 192, 256), (16, 320, 300), (33, 1088, 4500), (70, 1984, 1030), (12, 704, 9001), (32, 4160, 17000)])
+@pytest.mark.parametrize("M,K,N", SHAPES + [(3, 192, 256), (16, 320, 300), (33, 1088, 4500), (70, 1984, 1030), (12, 704, 9001), (32, 4160, 17000), (161, 2496, 300),
+                                            (3, 2112, 1088), (2, 1088, 260)])   # (the last two: fewer than 64 x 64 outputs)
 @pytest.mark.parametrize("form", ["rowcol", "mx"])
 def test_row_column_and_mx_scales(gpu, form, M, K, N):
     """fp32 outputs: exact products, fp32 sums of at most 8 terms a step inside the instruction and K / 128 steps beyond, so within
