@@ -134,8 +134,12 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
     const char* const xbase = (const char*)(p.x + (int64_t)m0 * Ki);
     const char* const wbase = (const char*)(KN ? p.w + (int64_t)n0 * WBITS / 8 : p.w + (int64_t)n0 * p.ldw);
     const uint32_t ring = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)smem;
-    auto issue = [&](int t, int stage) {
-        const int64_t k = __builtin_amdgcn_readfirstlane(base_of(t < nt ? t : nt - 1));
+    // (bases only grow, so that the last one bounds them all: past the end it is fetched and read again)
+    const int k_last = __builtin_amdgcn_readfirstlane(base_of(nt - 1));
+    int k_issue = __builtin_amdgcn_readfirstlane(t0 * WW_KT), k_read = k_issue;
+    auto issue = [&](int stage) {
+        const int64_t k = k_issue < k_last ? k_issue : k_last;
+        k_issue += WW_KT;
         const uint32_t at = __builtin_amdgcn_readfirstlane(ring + stage * TILE);
 #pragma unroll
         for (int i = 0; i < WC; i++) copy16_sbase(wbase + (KN ? k * p.ldw : k * WBITS / 8), wo[i], at + MB * 4096 + (wave * WC + i) * 1024);
@@ -155,7 +159,9 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
         uint32_t w[KN ? 8 : WBITS == 4 ? NB : 2 * NB];   // NK: column j's 8 codes; KN: row i of four columns
         uint32_t so[NB];
     };
-    auto read = [&](Frags& f, int t, int stage) {
+    auto read = [&](Frags& f, int stage) {
+        const int k = k_read < k_last ? k_read : k_last;
+        k_read += WW_KT;
         const char* const at = smem + stage * TILE;
 #pragma unroll
         for (int b = 0; b < MB; b++) f.x[b] = *(const v4i*)(at + (16 * b + r) * 256 + 16 * ((4 * kw + q) ^ r));
@@ -177,7 +183,7 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
                 else __builtin_memcpy(f.w + 2 * j, __builtin_assume_aligned(row + 16 * ((2 * kw + (q >> 1)) ^ (r >> 1)) + 8 * (q & 1), 8), 8);
             }
         }
-        const int g = group_at(base_of(t) + 32 * kw) - g_lo;
+        const int g = group_at(k + 32 * kw) - g_lo;
 #pragma unroll
         for (int j = 0; j < NB; j++) f.so[j] = tab[g * WW_COLS + wn * 64 + (KN ? 4 * r + j : 16 * j + r)];
     };
@@ -255,7 +261,7 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
         if (32 < gmax + 7) load8(v1, 1);
         wait_copies<0>();   // (these loads, for the compiler)
 #pragma unroll
-        for (int i = 0; i < S; i++) issue(i, i);
+        for (int i = 0; i < S; i++) issue(i);
         store8(v0, 0);
         if (32 < gmax + 7) store8(v1, 1);
     }
@@ -264,25 +270,25 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
     const bool rest = base_of(nt - 1) + 32 * kw >= (t0 + nt - 1) * WW_KT;   // (a partial tile: the others were counted with the one before)
     if constexpr (MB <= 4) {
         Frags f0, f1;
-        read(f0, 0, 0);
+        read(f0, 0);
         int t = 0, at = 0;
         // tile t + 1 is read while tile t multiplies; tile t + S goes where tile t was, whose fragments every wave holds by then
-        auto step = [&](const Frags& now, Frags& then, int t) {
+        auto step = [&](const Frags& now, Frags& then) {
             wait_copies<(S - 2) * CPT>();
             __builtin_amdgcn_s_barrier();
             asm volatile("" : : : "memory");
-            issue(t + S, at);
+            issue(at);
             at = at + 1 < S ? at + 1 : 0;
-            read(then, t + 1, at);
+            read(then, at);
             __builtin_amdgcn_sched_barrier(0);
             multiply(now);
         };
         for (; t + 2 < nt; t += 2) {
-            step(f0, f1, t);
-            step(f1, f0, t + 1);
+            step(f0, f1);
+            step(f1, f0);
         }
         if (t + 1 < nt) {
-            step(f0, f1, t);
+            step(f0, f1);
             if (rest) multiply(f1);
         } else if (rest) multiply(f0);
     } else {   // (no registers for a second set of fragments: tile t + S - 1 goes where tile t - 1 was)
@@ -292,8 +298,8 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
             wait_copies<(S - 2) * CPT>();
             __builtin_amdgcn_s_barrier();
             asm volatile("" : : : "memory");
-            if (t > 0) issue(t + S - 1, free);
-            read(f, t, at);
+            if (t > 0) issue(free);
+            read(f, at);
             if (t + 1 < nt || rest) multiply(f);
             free = at;
             at = at + 1 < S ? at + 1 : 0;
