@@ -245,15 +245,10 @@ static int splitk_for(const OpsnnQmmArgs& a, int mode, bool stream = true)
     if ((mode == 0 || (mode == 3 && !a.x1_scale)) && a.x1_dtype == DT_I8 && a.x2_dtype == DT_I8 && out16 && a.K % 128 == 0)
         return tile_plan(a.M, a.N, a.K, a.batch, true).splits;
     if (tiny) return 1;
-    // MXFP4 with few rows: one launch whatever K (qmm_mxfp4_rows.hip).  Else 128 x 128 tiles when 256 x 256 ones would be few (the launcher's rule), K tiles counted in 256 elements
-    if (mode == 2 && a.x1_dtype == DT_E2M1 && a.x2_dtype == DT_E2M1 && (out16 || a.out_dtype == DT_F32)) {
-        if (mxfp4_rows_wanted(a)) return 1;
-        const int64_t t256 = ((a.M + 255) / 256) * ((a.N + 255) / 256) * a.batch;
-        bm = bn = (a.M <= 128 || a.N <= 128 || t256 <= 64) ? 128 : 256;
-        kunit = 256;
-        tile_us = bm == 128 ? 0.6 : 1.3; bytes_per_us = 2.4e6;
-    }
-    else if (a.M <= 16) return 1;   // (up to 16 rows the streaming kernels take the modes below)
+    // MXFP4 with few rows: one launch whatever K (qmm_mxfp4_rows.hip); else by its tiles
+    if (mode == 2 && a.x1_dtype == DT_E2M1 && a.x2_dtype == DT_E2M1 && (out16 || a.out_dtype == DT_F32))
+        return mxfp4_rows_wanted(a) ? 1 : mxfp4_tile_plan(a.M, a.N, a.K, a.batch, true).splits;
+    if (a.M <= 16) return 1;   // (up to 16 rows the streaming kernels take the modes below)
     else if (mode == 2 && a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E2M1 && out16) { bm = 256; tile_us = 1.8; }
     else if (mode == 1 && a.x1_dtype == DT_I8 && a.x2_dtype == DT_I8 && a.gsK == 128 && a.gsN == 128 && out16) { bm = a.M >= 512 ? 256 : 128; tile_us = 1.8; }
     // (the exact fp8 kernel)

@@ -76,6 +76,28 @@ inline int splitk_factor(int64_t tiles, int64_t ktiles, double tile_us, int64_t 
     }
     return best;
 }
+// MXFP4 on the tile kernels: 128 x 128 or 256 x 256 tiles, and how many K segments.  A K tile of 256 elements takes a CU 1.4 us in the
+// small tile, 2.3 in the large one, which computes four times as much; partial sums move at 4 bytes a ps, behind a second launch.  Small
+// tiles where large ones would be at most 64, a quarter of the CUs, unless the large ones in segments are ahead (505 x 17536 x 6208 108 us on
+// small tiles; 1024 x 4096 x 4096 22.9 against 28.0 on large ones, at 128 large tiles it is 42 against 32).
+struct Mxfp4Plan {
+    bool small;
+    int splits;
+};
+inline Mxfp4Plan mxfp4_tile_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split)
+{
+    const int64_t ktiles = (K + 255) / 256, out = M * N * batch;
+    auto best = [&](int64_t bm, double t, int& splits) {
+        const int64_t tiles = ((M + bm - 1) / bm) * ((N + bm - 1) / bm) * batch;
+        splits = may_split ? splitk_factor(tiles, ktiles, t, out, 4.0e6) : 1;
+        return (double)((tiles * splits + 255) / 256) * (double)((ktiles + splits - 1) / splits) * t + (splits > 1 ? 4.0 + 8.0 * splits * (double)out / 4.0e6 : 0.0);
+    };
+    int s128, s256;
+    const double us128 = best(128, 1.4, s128), us256 = best(256, 2.3, s256);
+    const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256) * batch;
+    const bool small = M <= 128 || N <= 128 || (t256 <= 64 && us128 < 1.05 * us256);
+    return {small, small ? s128 : s256};
+}
 // How a product of two K-contiguous operands whose 256 x 256 tiles would not fill the chip once (or of up to 128 rows or columns)
 // is tiled (qmm_int8.hip; int8, and the 16-bit operands of gemm16.hip).  KB: bytes of K.  variant: the OPSNN_VARIANT_I8_*
 // tile, 0 if the shape is outside; splits: K segments; us: the estimate that the choice rests on.

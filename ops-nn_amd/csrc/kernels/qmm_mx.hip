@@ -359,8 +359,7 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
     if (rows4) return launch_mxfp4_rows(a, st);
     if (rows8) return launch_fp8_stream(a, FP8X_MX, sk, st);
     const bool small = a.M <= 128 || a.N <= 128;
-    // 128 x 128 tiles also when 256 x 256 ones would be at most 64, a quarter of the CUs (1024 x 4096 x 4096: 22.9 against 28.0 us; at 128 tiles of 256 x 256 it is 42 against 32)
-    const bool fp4_small = small || ((a.M + 255) / 256) * ((a.N + 255) / 256) * a.batch <= 64 || a.force_variant == OPSNN_VARIANT_MX_128;
+    const bool fp4_small = a.force_variant == OPSNN_VARIANT_MX_128 || mxfp4_tile_plan(a.M, a.N, a.K, a.batch, sk.splits > 1 && a.force_variant == 0).small;
     if (pad) {
         if (!mx_pad_layout(a, L)) return OPSNN_NOT_TAKEN;   // (the same answer as for the planned view: its conditions do not look at x2's address beyond its alignment)
         const int rc = fp4 && !fp4_small ? mx_pad_scales(a, L, st) : mx_pad_prestep(a, L, st);
@@ -405,8 +404,8 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
     }
     if (fp4) {
         // few tiles against a long K: K split over workgroups (fp32 partial sums in front of the workspace), on the tiles
-        // chosen below
-        const bool split = sk.splits > 1 && sk.part && a.force_variant == 0 && a.K % 256 == 0;
+        // chosen below, whole ones
+        const bool split = sk.splits > 1 && sk.part && a.force_variant == 0 && a.K % 128 == 0;
         if (split) { g.splits = sk.splits; g.part = (int32_t*)sk.part; }
         if (fp4_small) {
             if (split) return qgemm_launch_split_mx<MODE_MXFP4, 128, 128, 64, 2, 2, 4, 1>(g, a.batch, a.out_dtype, st);

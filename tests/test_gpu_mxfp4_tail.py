@@ -44,3 +44,12 @@ def test_neighbours_with_infinite_scales_stay_out(gpu):
     want = orc.b16_to_f32(cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, None), orc.BF16).reshape(B, M, N)
     assert np.isnan(got[:, 1::2]).all() and np.isnan(got[:, :, 1::2]).all()
     assert np.isfinite(got[:, ::2, ::2]).all() and np.allclose(got[:, ::2, ::2], want[:, ::2, ::2], rtol=1e-2, atol=1e-2)
+
+
+# few tiles of either size against a long K: K in segments of whole tiles of 128 elements, an odd count of them and a shorter last segment
+@pytest.mark.parametrize("M,K,N", [(130, 6272, 260), (200, 4480, 390), (65, 8320, 520), (2100, 6272, 2090)])
+def test_segments_of_odd_tiles(gpu, M, K, N):
+    m = gpu
+    print(f"case mxfp4 segments M={M} K={K} N={N}", flush=True)
+    inp = cases.make_mx_inputs(m, M, K, N, K + N, True, True)
+    check_close(cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_BF16, None), cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, None), orc.BF16, "mxfp4 in segments")
