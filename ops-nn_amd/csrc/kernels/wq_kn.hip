@@ -9,6 +9,11 @@
 // columns becomes 8 consecutive k: the operand of one v_mfma_f32_16x16x32 whose row r is column n0 + CPL r + c.  x is the
 // other operand straight from memory (16 bytes per lane and 16 rows; it stays in L2).  No LDS in the loop, no barrier.
 //
+// The loads of a step are held or in flight while others multiply, which the compiler's waits have to see: with conditions on the fetches
+// and on the scales it waits for every load under way in each step.  From some twelve steps a wave (TABLE, up to 16 rows) the loop has
+// none: the fetches go on past the end, and the scales of a window of steps lie in LDS (16 x 8192 x 28672 int4 44.4 -> 40.7 us, 3 x 11904 x 21504
+// 41.4 -> 38.2).
+//
 // Work split: a workgroup is four waves on the same 16 CPL columns, each with a quarter of the workgroup's steps; blockIdx.y
 // cuts K into segments so that the chip has two workgroups per CU.  The waves' sums meet in LDS in a fixed order; with more
 // than one segment they go to `part` as fp32 and wq_splitk_reduce_kernel adds the segments in order.
@@ -21,6 +26,8 @@ namespace opsnn {
 struct WqKnPlan {
     int mb = 1, splits = 1;
 };
+constexpr int KN_GROUPS = 16;   // groups in a wave's table of scales
+constexpr int kn_pf(int wbits, int mb) { return (mb == 2 || (mb == 1 && wbits == 4)) ? 3 : 2; }   // steps held or in flight per wave
 constexpr int kn_cpl(int mb) { return mb == 1 ? 16 : 8; }   // codes per lane: with 16 and two row blocks the loop spills
 
 // Segments of K: as many workgroups as two per CU, less what a slice of partial sums costs.  (A step is 4 KB (int8: 8 KB) per
@@ -42,13 +49,13 @@ static WqKnPlan kn_plan(int wbits, int64_t M, int64_t N, int64_t K)
     return pl;
 }
 
-template <int XDT, int WBITS, int MB, bool HAS_OFF>
-__global__ __launch_bounds__(256, 2) void wq_kn_kernel(WqParams p, int splits)
+template <int XDT, int WBITS, int MB, bool HAS_OFF, bool TABLE>
+__global__ __launch_bounds__(256, 2) void wq_kn_kernel(WqParams p, int splits, int window)
 {
     constexpr int CPL = kn_cpl(MB);
     constexpr int DW = CPL * WBITS / 32;          // dwords of codes per lane and row: 1, 2 or 4
     constexpr int OCT = CPL / 8;                  // 8 x 8 blocks per step
-    constexpr int PF = (MB == 2 || (MB == 1 && WBITS == 4)) ? 3 : 2;   // steps held or in flight per wave
+    constexpr int PF = kn_pf(WBITS, MB);
     extern __shared__ __attribute__((aligned(16))) float red[];   // two waves' sums
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -73,53 +80,19 @@ __global__ __launch_bounds__(256, 2) void wq_kn_kernel(WqParams p, int splits)
     const int groupi = (int)p.group;
     auto group_of = [&](int st) { return p.group_shift >= 0 ? (st * 32) >> p.group_shift : (st * 32) / groupi; };
 
-    uint32_t raw[PF][8][DW];
-    v4i xf[PF][MB];
-    uint32_t sc[OCT][4], of[OCT][4];
-#pragma unroll
-    for (int t = 0; t < OCT; t++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) sc[t][e] = of[t][e] = 0;
-    auto fetch = [&](auto jc, int st) {
-        constexpr int j = decltype(jc)::value;
-        const uint8_t* w = wbase + (int64_t)st * 32 * ldw;
-#pragma unroll
-        for (int i = 0; i < 8; i++) __builtin_memcpy(raw[j][i], w + i * ldw, 4 * DW);
-#pragma unroll
-        for (int b = 0; b < MB; b++) xf[j][b] = *(const v4i*)(xrow[b] + st * 32);
-    };
-    auto load_scales = [&](int g) {
-        if (p.s_cs == 1) {
-            __builtin_memcpy(sc, sbase + (int64_t)g * p.s_rs, sizeof(sc));
-            if constexpr (HAS_OFF) __builtin_memcpy(of, obase + (int64_t)g * p.s_rs, sizeof(of));
-        } else {   // one scale for all columns (s_cs == 0)
-#pragma unroll
-            for (int t = 0; t < OCT; t++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    sc[t][e] = sbase[(int64_t)g * p.s_rs] * 0x00010001u;
-                    if constexpr (HAS_OFF) of[t][e] = obase[(int64_t)g * p.s_rs] * 0x00010001u;
-                }
-        }
-    };
     v4f acc[CPL][MB];
 #pragma unroll
     for (int c = 0; c < CPL; c++)
 #pragma unroll
         for (int b = 0; b < MB; b++) acc[c][b] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
-
-    int g_cur = -1;
-    auto step = [&](auto jc, int st) {
-        constexpr int j = decltype(jc)::value;
-        const int g = group_of(st);
-        if (g != g_cur) { load_scales(g); g_cur = g; }
+    auto multiply = [&](const uint32_t (&rw)[8][DW], const v4i (&x)[MB], const uint32_t (&sc)[OCT][4], const uint32_t (&of)[OCT][4]) __attribute__((always_inline)) {
 #pragma unroll
         for (int t = 0; t < OCT; t++) {
             uint32_t q8[8][WBITS / 4], o[8][4];
 #pragma unroll
             for (int i = 0; i < 8; i++)
 #pragma unroll
-                for (int d = 0; d < WBITS / 4; d++) q8[i][d] = raw[j][i][t * (WBITS / 4) + d];
+                for (int d = 0; d < WBITS / 4; d++) q8[i][d] = rw[i][t * (WBITS / 4) + d];
             dequant_8x8<XDT, WBITS, HAS_OFF>(q8, sc[t], of[t], o);
 #pragma unroll
             for (int c = 0; c < 8; c++) {
@@ -127,23 +100,124 @@ __global__ __launch_bounds__(256, 2) void wq_kn_kernel(WqParams p, int splits)
 #pragma unroll
                 for (int b = 0; b < MB; b++) {
                     v4f& d = acc[t * 8 + c][b];
-                    if constexpr (XDT == DT_F16) d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, xf[j][b]), d, 0, 0, 0);
-                    else d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, xf[j][b]), d, 0, 0, 0);
+                    if constexpr (XDT == DT_F16) d = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, x[b]), d, 0, 0, 0);
+                    else d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, x[b]), d, 0, 0, 0);
                 }
             }
         }
-        if (st + PF < w1) fetch(jc, st + PF);
     };
-    using I0 = std::integral_constant<int, 0>;
-    using I1 = std::integral_constant<int, 1>;
-    using I2 = std::integral_constant<int, PF - 1>;
-    if (w0 < w1) fetch(I0{}, w0);
-    if (w0 + 1 < w1) fetch(I1{}, w0 + 1);
-    if constexpr (PF == 3) { if (w0 + 2 < w1) fetch(I2{}, w0 + 2); }
-    for (int st = w0; st < w1; st += PF) {
-        step(I0{}, st);
-        if (st + 1 < w1) step(I1{}, st + 1);
-        if constexpr (PF == 3) { if (st + 2 < w1) step(I2{}, st + 2); }
+    if constexpr (TABLE) {
+        uint32_t raw[PF][8][DW];
+        v4i xf[PF][MB];
+        auto fetch = [&](auto jc, int st) {   // (past the end: the last step again, so that every step waits for the same count of loads)
+            constexpr int j = decltype(jc)::value;
+            const int sc = st < w1 ? st : w1 - 1;
+            const uint8_t* w = wbase + (int64_t)sc * 32 * ldw;
+#pragma unroll
+            for (int i = 0; i < 8; i++) __builtin_memcpy(raw[j][i], w + i * ldw, 4 * DW);
+#pragma unroll
+            for (int b = 0; b < MB; b++) xf[j][b] = *(const v4i*)(xrow[b] + sc * 32);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+
+        // scales of a window of steps: rows of 16 CPL columns, this wave's own
+        char* const tab = (char*)red + wave * (KN_GROUPS * 32 * CPL * (HAS_OFF ? 2 : 1));
+        int g_lo = 0;
+        auto load_window = [&](int st, int end) {
+            g_lo = group_of(st);
+            const int n_groups = group_of(end - 1) - g_lo + 1;
+            for (int g = q; g < n_groups; g += 4) {   // (lane r: its own CPL columns)
+                uint32_t v[HAS_OFF ? 2 : 1][CPL / 2];
+                if (p.s_cs == 1) {
+                    __builtin_memcpy(v[0], sbase + (int64_t)(g_lo + g) * p.s_rs, 2 * CPL);
+                    if constexpr (HAS_OFF) __builtin_memcpy(v[1], obase + (int64_t)(g_lo + g) * p.s_rs, 2 * CPL);
+                } else {   // one scale for all columns (s_cs == 0)
+#pragma unroll
+                    for (int e = 0; e < CPL / 2; e++) {
+                        v[0][e] = sbase[(int64_t)(g_lo + g) * p.s_rs] * 0x00010001u;
+                        if constexpr (HAS_OFF) v[1][e] = obase[(int64_t)(g_lo + g) * p.s_rs] * 0x00010001u;
+                    }
+                }
+                __builtin_memcpy(tab + g * (32 * CPL) + r * (2 * CPL), v[0], 2 * CPL);
+                if constexpr (HAS_OFF) __builtin_memcpy(tab + (KN_GROUPS + g) * (32 * CPL) + r * (2 * CPL), v[1], 2 * CPL);
+            }
+        };
+        auto step = [&](auto jc, int st) __attribute__((always_inline)) {
+            constexpr int j = decltype(jc)::value;
+            const char* const at = tab + (group_of(st) - g_lo) * (32 * CPL) + r * (2 * CPL);
+            uint32_t sc[OCT][4], of[OCT][4] = {};
+            __builtin_memcpy(sc, __builtin_assume_aligned(at, 16), sizeof(sc));
+            if constexpr (HAS_OFF) __builtin_memcpy(of, __builtin_assume_aligned(at + KN_GROUPS * (32 * CPL), 16), sizeof(of));
+            multiply(raw[j], xf[j], sc, of);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto each = [&](auto&& f) {
+            [&]<int... J>(std::integer_sequence<int, J...>) { (f(std::integral_constant<int, J>{}), ...); }(std::make_integer_sequence<int, PF>{});
+        };
+        if (w0 < w1) {
+            each([&](auto j) { fetch(j, w0 + j); });
+            int st = w0;
+            while (w1 - st >= PF) {   // windows of whole rounds of PF steps
+                int end = w1 - st > window ? st + window : st + (w1 - st) / PF * PF;
+                load_window(st, end);
+                for (; st < end; st += PF) each([&](auto j) __attribute__((always_inline)) { step(j, st + j); fetch(j, st + j + PF); });
+            }
+            if (st < w1) {
+                load_window(st, w1);
+                each([&](auto j) __attribute__((always_inline)) { if (st + j < w1) step(j, st + j); });
+            }
+        }
+        __syncthreads();   // the tables make room for the sums
+    } else {
+        uint32_t raw[PF][8][DW];
+        v4i xf[PF][MB];
+        uint32_t sc[OCT][4], of[OCT][4];
+#pragma unroll
+        for (int t = 0; t < OCT; t++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) sc[t][e] = of[t][e] = 0;
+        auto fetch = [&](auto jc, int st) {
+            constexpr int j = decltype(jc)::value;
+            const uint8_t* w = wbase + (int64_t)st * 32 * ldw;
+#pragma unroll
+            for (int i = 0; i < 8; i++) __builtin_memcpy(raw[j][i], w + i * ldw, 4 * DW);
+#pragma unroll
+            for (int b = 0; b < MB; b++) xf[j][b] = *(const v4i*)(xrow[b] + st * 32);
+        };
+        auto load_scales = [&](int g) {
+            if (p.s_cs == 1) {
+                __builtin_memcpy(sc, sbase + (int64_t)g * p.s_rs, sizeof(sc));
+                if constexpr (HAS_OFF) __builtin_memcpy(of, obase + (int64_t)g * p.s_rs, sizeof(of));
+            } else {   // one scale for all columns (s_cs == 0)
+#pragma unroll
+                for (int t = 0; t < OCT; t++)
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        sc[t][e] = sbase[(int64_t)g * p.s_rs] * 0x00010001u;
+                        if constexpr (HAS_OFF) of[t][e] = obase[(int64_t)g * p.s_rs] * 0x00010001u;
+                    }
+            }
+        };
+
+        int g_cur = -1;
+        auto step = [&](auto jc, int st) {
+            constexpr int j = decltype(jc)::value;
+            const int g = group_of(st);
+            if (g != g_cur) { load_scales(g); g_cur = g; }
+            multiply(raw[j], xf[j], sc, of);
+            if (st + PF < w1) fetch(jc, st + PF);
+        };
+        using I0 = std::integral_constant<int, 0>;
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, PF - 1>;
+        if (w0 < w1) fetch(I0{}, w0);
+        if (w0 + 1 < w1) fetch(I1{}, w0 + 1);
+        if constexpr (PF == 3) { if (w0 + 2 < w1) fetch(I2{}, w0 + 2); }
+        for (int st = w0; st < w1; st += PF) {
+            step(I0{}, st);
+            if (st + 1 < w1) step(I1{}, st + 1);
+            if constexpr (PF == 3) { if (st + 2 < w1) step(I2{}, st + 2); }
+        }
     }
 
     if (!sum_of_four_waves(acc, red, wave, lane)) return;
@@ -183,20 +257,24 @@ __global__ __launch_bounds__(256, 2) void wq_kn_kernel(WqParams p, int splits)
     }
 }
 
-template <int XDT, int WBITS, int MB, bool HAS_OFF>
+template <int XDT, int WBITS, int MB, bool HAS_OFF, bool TABLE = false>
 static int launch_kn_one(const WqParams& p, int splits, hipStream_t st)
 {
-    constexpr int CPL = kn_cpl(MB);
+    constexpr int CPL = kn_cpl(MB), PF = kn_pf(WBITS, MB);
     const dim3 grid((unsigned)((p.N + 16 * CPL - 1) / (16 * CPL)), (unsigned)splits);
-    const size_t lds = (size_t)2 * CPL * MB * 4 * 64 * 4;
-    auto k = wq_kn_kernel<XDT, WBITS, MB, HAS_OFF>;
+    constexpr size_t lds_sum = (size_t)2 * CPL * MB * 4 * 64 * 4, lds_tab = TABLE ? (size_t)4 * KN_GROUPS * 32 * CPL * (HAS_OFF ? 2 : 1) : 0;
+    constexpr size_t lds = lds_sum > lds_tab ? lds_sum : lds_tab;
+    // steps whose groups fit a table wherever they start, in whole rounds of the loop
+    const int64_t steps = p.K / 32, fit = p.group >= p.K ? steps + PF : (KN_GROUPS - (p.group > 32)) * p.group / 32;
+    const int window = (int)((fit < steps + PF ? fit : steps + PF) / PF * PF);
+    auto k = wq_kn_kernel<XDT, WBITS, MB, HAS_OFF, TABLE>;
     static std::atomic<uint64_t> attr_set{0};   // one bit per device: the attribute belongs to the (kernel, device) pair
     if (!device_flag_test(attr_set)) {
         hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
         if (e != hipSuccess) return (int)e;
         device_flag_set(attr_set);
     }
-    hipLaunchKernelGGL(k, grid, dim3(256), lds, st, p, splits);
+    hipLaunchKernelGGL(k, grid, dim3(256), lds, st, p, splits, window);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
     launch_wq_splitk_reduce(p, splits, XDT, st);
     return (int)hipGetLastError();
@@ -204,7 +282,11 @@ static int launch_kn_one(const WqParams& p, int splits, hipStream_t st)
 template <int XDT, int WBITS, bool HAS_OFF>
 static int launch_kn_mb(const WqParams& p, const WqKnPlan& pl, hipStream_t st)
 {
-    if (pl.mb == 1) return launch_kn_one<XDT, WBITS, 1, HAS_OFF>(p, pl.splits, st);
+    if (pl.mb == 1) {
+        // (the table pays for itself from some twelve steps a wave: 16 x 8192 x 28672, sixteen, 44.4 -> 41.3 us; 4 x 3072 x 1872, six, 9.0 -> 10.4)
+        if (p.K / 32 >= 48 * pl.splits) return launch_kn_one<XDT, WBITS, 1, HAS_OFF, true>(p, pl.splits, st);
+        return launch_kn_one<XDT, WBITS, 1, HAS_OFF>(p, pl.splits, st);
+    }
     if (pl.mb == 2) return launch_kn_one<XDT, WBITS, 2, HAS_OFF>(p, pl.splits, st);
     return launch_kn_one<XDT, WBITS, 4, HAS_OFF>(p, pl.splits, st);
 }
