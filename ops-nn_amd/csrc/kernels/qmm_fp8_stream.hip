@@ -638,16 +638,18 @@ bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8St
     if (a.M > 512 || a.N < 256 || a.K < 128 || a.K % 64 != 0 || a.K >= (1ll << 30) || a.N >= (1ll << 30)) return false;
     if (a.M > 128 && (a.K < 1024 || a.M * a.N * a.K > (form == FP8X_PLAIN && a.K % 128 ? FS_MANY_ROWS_TAIL : FS_MANY_ROWS))) return false;
     const int64_t ldb = a.x2.row_stride == 1 ? a.x2.col_stride : a.K;
-    if (a.x1.row_stride < 0 || a.x1.row_stride >= (1ll << 24) || ldb < 0 || ldb >= (1ll << 24)) return false;   // (32-bit lane offsets)
+    // (32-bit lane offsets: from the first row of x1 and of its scales, from the workgroup's first column of x2)
+    auto offsets_ok = [](int64_t rows, int64_t bytes) { return bytes >= 0 && bytes < (1ll << 31) / rows; };
+    if (!offsets_ok(a.M, a.x1.row_stride) || ldb < 0 || ldb >= (1ll << 24)) return false;
     if (form == FP8X_BLOCK) {
         if (a.K % 128 != 0 || a.bias || a.gsK != 128 || a.gsN != 128 || (a.gsM != 1 && a.gsM != 128)) return false;
-        if (a.x1_scale_mat.row_stride < 0 || a.x1_scale_mat.row_stride >= (1ll << 22) || a.x2_scale_mat.row_stride < 0 || a.x2_scale_mat.row_stride >= (1ll << 20)) return false;
+        if (!offsets_ok(a.M, 4 * a.x1_scale_mat.row_stride) || a.x2_scale_mat.row_stride < 0 || a.x2_scale_mat.row_stride >= (1ll << 20)) return false;
     } else if (form == FP8X_PLAIN) {
         if (!a.x1_scale || !a.x2_scale || a.x2_scale_dtype != DT_F32 || (a.bias && a.bias_dtype != DT_F32)) return false;
         if (a.x1_scale_len == 1 && a.x2_scale_len == 1 && !a.bias) return false;   // (that case merges and truncates the scales)
     } else {
-        if ((a.bias && a.bias_dtype != DT_F32) || a.x1_scale_mat.row_stride < 0 || a.x2_scale_mat.row_stride < 0) return false;
-        if (a.x1_scale_mat.row_stride >= (1ll << 24) || a.x2_scale_mat.row_stride >= (1ll << 24)) return false;
+        if ((a.bias && a.bias_dtype != DT_F32) || !offsets_ok(a.M, a.x1_scale_mat.row_stride) || a.x2_scale_mat.row_stride < 0) return false;
+        if (a.x2_scale_mat.row_stride >= (1ll << 24)) return false;
     }
     const int mb = a.M <= 16 ? 1 : a.M <= 32 ? 2 : 4;
     const int64_t slabs = (a.M + 16 * mb - 1) / (16 * mb), units = (a.K + 127) / 128;

@@ -87,6 +87,32 @@ def test_row_column_and_mx_scales(gpu, form, M, K, N):
     del keep
 
 
+# rows of x1 so far apart that the last ones lie 2^32 bytes and more behind the first: the stream kernels' lane offsets have 32 bits
+@pytest.mark.parametrize("M,K,N", [(300, 1024, 256), (300, 1088, 260)])
+def test_rows_far_apart(gpu, M, K, N):
+    m = gpu
+    stride = (1 << 24) - 128
+    print(f"case fp8 stream rowcol, rows {stride} apart M={M} K={K} N={N}", flush=True)
+    rng = np.random.default_rng(M + K)
+    x1, x2 = cases.gen_fp8(rng, (M, K)), cases.gen_fp8(rng, (N, K))
+    s1, s2 = rng.uniform(0.5, 2, M).astype(np.float32), rng.uniform(0.5, 2, N).astype(np.float32)
+    d = {k: m.DeviceBuffer(host=v) for k, v in dict(x2=x2, s1=s1, s2=s2).items()}
+    d["x1"] = m.DeviceBuffer((M - 1) * stride + K)
+    for r in range(M):
+        m.check(m.lib().aclrtMemcpy(d["x1"].ptr + r * stride, K, x1[r].ctypes.data, K, m.binding.H2D), "aclrtMemcpy H2D")
+    d_out = m.DeviceBuffer(M * N * 4)
+    acl = m.ACL_FLOAT8_E4M3FN
+    keep = m.quant_matmul_v5(m.Tensor((M, K), acl, d["x1"], strides=(stride, 1), storage_shape=((M - 1) * stride + K,)), m.Tensor((N, K), acl, d["x2"]),
+                             m.Tensor((M,), m.ACL_FLOAT, d["s1"]), m.Tensor((N,), m.ACL_FLOAT, d["s2"]), m.Tensor((M, N), m.ACL_FLOAT, d_out), transpose_x2=True)
+    m.check(m.lib().aclrtSynchronizeDevice(), "sync")
+    got = d_out.to_host(np.float32, (M, N)).astype(np.float64)
+    code = _codes()
+    a, b = code[x1] * s1[:, None].astype(np.float64), code[x2] * s2[:, None].astype(np.float64)
+    err = np.abs(got - a @ b.T)
+    assert (err <= 2.0 ** -18 * (np.abs(a) @ np.abs(b).T) + 1e-30).all(), f"worst {err.max():.3e}"
+    del keep
+
+
 def _codes():
     c = np.arange(256)
     e, f, s = (c >> 3) & 15, c & 7, np.where(c & 128, -1.0, 1.0)
