@@ -119,14 +119,14 @@ static bool mx_pad_layout(const OpsnnQmmArgs& a, MxPad& L)
     return true;
 }
 
-// The scale tables alone, both in one launch (rows of x1's, then of x2's along grid.y): for fp4 on the tiles that end a K inside a
+// The scale tables alone, both in one launch (rows of x1's, then of x2's along grid.x, which takes their sum): for fp4 on the tiles that end a K inside a
 // tile by themselves, whose scales come in whole words.
 __global__ __launch_bounds__(256) void mx_pad_scales_kernel(const uint8_t* __restrict__ s1, int64_t bs1, uint8_t* __restrict__ d1, int64_t rows1, int64_t nb1,
                                                             const uint8_t* __restrict__ s2, int64_t bs2, uint8_t* __restrict__ d2, int64_t rows2, int64_t nb2,
                                                             int64_t ld, int64_t kb, int64_t kbp)
 {
-    const int64_t c = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63), b = blockIdx.z;
-    int64_t r = (int64_t)blockIdx.y * 4 + (threadIdx.x >> 6);
+    const int64_t c = (int64_t)blockIdx.y * 64 + (threadIdx.x & 63), b = blockIdx.z;
+    int64_t r = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const bool second = r >= rows1;
     if (second) r -= rows1;
     if (c * 2 >= kbp || r >= (second ? rows2 : rows1) || b >= (second ? nb2 : nb1)) return;
@@ -141,7 +141,7 @@ static int mx_pad_scales(OpsnnQmmArgs& a, const MxPad& L, hipStream_t st)
     if (!a.workspace || (uintptr_t)a.workspace % 16) return OPSNN_NOT_TAKEN;
     uint8_t* w = (uint8_t*)a.workspace;
     const int64_t ksp2 = L.Kp / 64 * 2, nb = L.snb1 > L.snb2 ? L.snb1 : L.snb2;
-    const dim3 grid((unsigned)((ksp2 / 2 + 63) / 64), (unsigned)((a.M + a.N + 3) / 4), (unsigned)nb);
+    const dim3 grid((unsigned)((a.M + a.N + 3) / 4), (unsigned)((ksp2 / 2 + 63) / 64), (unsigned)nb);
     hipLaunchKernelGGL(mx_pad_scales_kernel, grid, dim3(256), 0, st, (const uint8_t*)a.x1_scale_mat.ptr, a.x1_scale_mat.batch_stride, w + L.o_s1, a.M, L.snb1,
                        (const uint8_t*)a.x2_scale_mat.ptr, a.x2_scale_mat.batch_stride, w + L.o_s2, a.N, L.snb2, (a.K + 63) / 64 * 2, a.K / 32, ksp2);
     a.x1_scale_mat = OpsnnMat{w + L.o_s1, ksp2, 2, L.snb1 == 1 && a.batch > 1 ? 0 : a.M * ksp2};

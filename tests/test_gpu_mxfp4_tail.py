@@ -53,3 +53,12 @@ def test_segments_of_odd_tiles(gpu, M, K, N):
     print(f"case mxfp4 segments M={M} K={K} N={N}", flush=True)
     inp = cases.make_mx_inputs(m, M, K, N, K + N, True, True)
     check_close(cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_BF16, None), cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, None), orc.BF16, "mxfp4 in segments")
+
+
+def test_scale_rows_of_both_operands_beyond_the_grids_second_axis(gpu):
+    """M + N rows of scales are copied by one launch, four a workgroup: more workgroups than the second and third axis of a grid hold."""
+    m = gpu
+    M, K, N = 260, 32, 262000
+    print(f"case mxfp4 tail M={M} K={K} N={N}", flush=True)
+    inp = cases.make_mx_inputs(m, M, K, N, 5, True, True)
+    check_close(cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_BF16, None), cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, None), orc.BF16, "mxfp4 tail, many scale rows")
