@@ -257,7 +257,8 @@ static int launch_quant_rows(const DynQuantParams& p, hipStream_t st)
 template <int X_DT, int Y_DT, bool ASYM>
 static int launch_dynamic_quant(const DynQuantParams& p, int variant, hipStream_t st)
 {
-    const bool vec = p.cols % 8 == 0 && p.cols <= 8 * 8 * 1024 && (uintptr_t)p.x % 16 == 0 && (uintptr_t)p.y % 8 == 0 &&
+    // (a launch has fewer than 2^32 threads)
+    const bool vec = p.cols % 8 == 0 && p.cols <= (p.rows < (1ll << 22) ? 8 * 8 * 1024 : 8 * 8 * 256) && (uintptr_t)p.x % 16 == 0 && (uintptr_t)p.y % 8 == 0 &&
                      (!p.smooth || (uintptr_t)p.smooth % 16 == 0);
     if (variant == 2 || !vec) {
         if (variant == 1) return -4;
