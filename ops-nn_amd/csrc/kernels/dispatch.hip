@@ -87,6 +87,15 @@ extern "C" int opsnnDebugFillLds(void* stream)
     return (int)hipGetLastError();
 }
 
+static thread_local const char* t_route = "";
+static thread_local int t_route_splits = 1;
+void opsnn::note_route(const char* kernel, int splits) { t_route = kernel; t_route_splits = splits; }
+extern "C" const char* opsnnDebugLastRoute(int* splits)
+{
+    if (splits) *splits = t_route_splits;
+    return t_route;
+}
+
 // fp8 x fp8 arithmetic of the block-scale and row/column-scale modes: 0 (default) exact products and sums on the fp16
 // matrix instruction, 1 the 8-bit matrix instruction (about 1.5x faster, sums aligned in a narrower window).  The
 // initial value comes from OPSNN_FP8_FAST, read once.
@@ -100,6 +109,7 @@ extern "C" int opsnnGetFp8Fast(void) { return __atomic_load_n(&g_fp8_fast, __ATO
 static const bool g_log = [] { const char* e = getenv("OPSNN_LOG"); return e && *e && *e != '0'; }();
 extern "C" __attribute__((visibility("hidden"))) void opsnn_note_plain(const char* mode, int forced, int64_t batch, int64_t M, int64_t N, int64_t K)
 {
+    opsnn::note_route("plain");
     if (!g_log || forced || opsnn_force_plain()) return;
     const double macs = (double)batch * (double)M * (double)N * (double)K;
     if (macs <= 1e7) return;
@@ -288,6 +298,7 @@ extern "C" __attribute__((visibility("hidden"))) void opsnn_qmm_splitk_carve(con
 extern "C" int opsnnQmmBlockScale(const OpsnnQmmArgs* a0, void* stream)
 {
     WeightCacheScope cache_scope;
+    note_route("other");
     if (!qmm_args_ok(a0) || !a0->x1_scale_mat.ptr || !a0->x2_scale_mat.ptr) return -1;
     const OpsnnQmmArgs* a = a0;
     if (a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain()) {
@@ -311,6 +322,7 @@ extern "C" int opsnnQmmBlockScale(const OpsnnQmmArgs* a0, void* stream)
 extern "C" int opsnnQmmMx(const OpsnnQmmArgs* a, void* stream)
 {
     WeightCacheScope cache_scope;
+    note_route("other");
     if (!qmm_args_ok(a) || !a->x1_scale_mat.ptr || !a->x2_scale_mat.ptr) return -1;
     if (a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain()) {
         OpsnnQmmArgs c;
@@ -331,6 +343,7 @@ extern "C" __attribute__((visibility("hidden"))) int opsnn_qmm_int8_impl(const O
 extern "C" int opsnnQmmTc(const OpsnnQmmArgs* a, void* stream)
 {
     WeightCacheScope cache_scope;
+    note_route("other");
     if (!qmm_args_ok(a) || !a->x2_scale) return -1;
     const bool i8 = a->x1_dtype == DT_I8 && a->x2_dtype == DT_I8;
     const bool f8 = (a->x1_dtype == DT_E4M3 || a->x1_dtype == DT_E5M2) && (a->x2_dtype == DT_E4M3 || a->x2_dtype == DT_E5M2);
@@ -404,6 +417,7 @@ extern "C" int opsnnQmmTc(const OpsnnQmmArgs* a, void* stream)
 extern "C" int opsnnQmmGroup(const OpsnnQmmArgs* a, void* stream)
 {
     WeightCacheScope cache_scope;
+    note_route("other");
     if (!qmm_args_ok(a) || a->batch != 1 || a->gsK <= 0 || !a->x2_scale_mat.ptr) return -1;
     const bool tcg = a->x1_dtype == DT_E4M3 && a->x2_dtype == DT_E2M1;
     const bool i4 = a->x1_dtype == DT_I4 && a->x2_dtype == DT_I4;
@@ -432,6 +446,7 @@ extern "C" int opsnnQmmGroup(const OpsnnQmmArgs* a, void* stream)
 extern "C" int opsnnWqmm(const OpsnnWqmmArgs* a, void* stream)
 {
     WeightCacheScope cache_scope;
+    note_route("other");
     if (!a || !a->x || !a->w.ptr || !a->scale.ptr || !a->y || a->M <= 0 || a->N <= 0 || a->K <= 0) return -1;
     if (a->force_variant != OPSNN_VARIANT_PLAIN && !opsnn_force_plain()) {
         int rc = launch_wq_wide(*a, (hipStream_t)stream);

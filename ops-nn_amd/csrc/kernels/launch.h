@@ -52,6 +52,8 @@ namespace opsnn {
 // `splits` workgroups per tile each take a contiguous range of K tiles and leave fp32 partial sums in `part`
 // ([splits][batch][M][N], at the front of the call's workspace); a second kernel adds them in split order, adds the bias
 // and rounds.  splits <= 1: one workgroup per tile, no partial sums.
+// The kernel that this thread launched last, a literal, and its K segments (opsnnDebugLastRoute).
+void note_route(const char* kernel, int splits = 1);   // dispatch.hip
 struct SplitK {
     int splits = 1;
     float* part = nullptr;

@@ -213,6 +213,7 @@ int launch_decode_one(const Fp8DecParams& p, hipStream_t st, int splits = 1)
     const int cus = 256 / splits;   // the CUs shared between the segments' workgroup columns
     const int grid = nblocks < cus ? nblocks : cus;
     const size_t lds = (size_t)2 * NW * 256 * sizeof(float);
+    note_route("fp8_decode", splits);
     hipLaunchKernelGGL((fp8_block_decode_kernel<NW, NBLK, I8, SEG>), dim3((unsigned)grid, (unsigned)splits), dim3(NW * 64), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
     splitk_launch(p.M, p.N, [&](auto w, dim3 g, dim3 b) { hipLaunchKernelGGL((fp8dec_reduce_kernel<decltype(w)::value>), g, b, 0, st, p, splits); });
@@ -576,6 +577,7 @@ int launch_mx8_one(const Mx8DecParams& p, hipStream_t st, int splits)
     const int cus = 256 / splits;   // the CUs shared between the segments' workgroup columns
     const int grid = nblocks < cus ? nblocks : cus;
     const size_t lds = (size_t)2 * NW * 256 * sizeof(float);
+    note_route("fp8_decode", splits);
     hipLaunchKernelGGL((mx8_decode_kernel<NW, NBLK>), dim3((unsigned)grid, (unsigned)splits), dim3(NW * 64), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
     splitk_launch(p.M, p.N, [&](auto w, dim3 g, dim3 b) { hipLaunchKernelGGL(mx8dec_reduce_kernel<decltype(w)::value>, g, b, 0, st, p, splits); });

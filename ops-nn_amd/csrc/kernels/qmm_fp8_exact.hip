@@ -628,6 +628,7 @@ static int launch_fp8_exact_tile(const Fp8xParams& p, int64_t batch, hipStream_t
     const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
     dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch);
     const size_t lds = 3 * (size_t)((BM + BN) * 128 + ((RC && !MXS) ? 0 : NT * 4));
+    note_route("fp8_exact", p.splits > 1 ? p.splits : 1);
     if (p.splits > 1) {   // K split over workgroups, then the sum of the partial sums, the epilogue and the rounding
         if (!p.part || p.splits > p.K / 128) return -1;
         auto ks = qmm_fp8_exact_kernel<WGM, WGN, DT_F32, RC, FMT, MXS, true>;

@@ -538,6 +538,7 @@ int launch_one(const Fp8StreamParams& p, hipStream_t st)
         if (e != hipSuccess) return (int)e;
         device_flag_set(attr_set);
     }
+    note_route("fp8_stream", p.splits);
     hipLaunchKernelGGL(k, grid, dim3(256), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || p.splits == 1) return (int)e;
     return launch_reduce<FORM>(p, st);
@@ -558,6 +559,7 @@ int launch_wide_one(const Fp8StreamParams& p, hipStream_t st)
         if (e != hipSuccess) return (int)e;
         device_flag_set(attr_set);
     }
+    note_route("fp8_wide", p.splits);
     hipLaunchKernelGGL(k, grid, dim3(256), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || p.splits == 1) return (int)e;
     return launch_reduce<FORM>(p, st);

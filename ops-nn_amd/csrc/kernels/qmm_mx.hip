@@ -407,6 +407,7 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         // chosen below, whole ones
         const bool split = sk.splits > 1 && sk.part && a.force_variant == 0 && a.K % 128 == 0;
         if (split) { g.splits = sk.splits; g.part = (int32_t*)sk.part; }
+        note_route(fp4_small ? "mxfp4_tiles_128" : "mxfp4_tiles_256", split ? sk.splits : 1);
         if (fp4_small) {
             if (split) return qgemm_launch_split_mx<MODE_MXFP4, 128, 128, 64, 2, 2, 4, 1>(g, a.batch, a.out_dtype, st);
             return qgemm_launch<MODE_MXFP4, 128, 128, 64, 2, 2, 4, 1>(g, a.batch, a.out_dtype, st);

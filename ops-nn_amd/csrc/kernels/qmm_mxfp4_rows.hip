@@ -199,6 +199,7 @@ int launch_one(const Mx4RowsParams& p, int64_t batch, hipStream_t st)
             device_flag_set(attr_set);
         }
     }
+    note_route("mxfp4_rows");
     hipLaunchKernelGGL(k, grid, dim3(NW * 64), lds, st, p);
     return (int)hipGetLastError();
 }

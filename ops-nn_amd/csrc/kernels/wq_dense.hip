@@ -258,6 +258,7 @@ int launch_wq_dense(const OpsnnWqmmArgs& a, hipStream_t st)
             if (rc != OPSNN_NOT_TAKEN) return rc;
         }
     }
+    note_route("wq_dense");
     uint16_t* w16 = (uint16_t*)a.workspace;
     WqParams p{};
     p.ldw = (kn ? a.w.row_stride : a.w.col_stride) * wbits / 8;

@@ -274,6 +274,7 @@ static int launch_kn_one(const WqParams& p, int splits, hipStream_t st)
         if (e != hipSuccess) return (int)e;
         device_flag_set(attr_set);
     }
+    note_route(TABLE ? "wq_kn_table" : "wq_kn", splits);
     hipLaunchKernelGGL(k, grid, dim3(256), lds, st, p, splits, window);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
     launch_wq_splitk_reduce(p, splits, XDT, st);

@@ -203,6 +203,7 @@ static int launch_nk_one(const WqParams& p, const WqNkPlan& pl, hipStream_t st)
         if (e != hipSuccess) return (int)e;
         device_flag_set(attr_set);
     }
+    note_route("wq_nk", pl.splits);
     hipLaunchKernelGGL(k, grid, dim3(256), lds_sum > lds_tab ? lds_sum : lds_tab, st, p, pl.splits, pl.groups);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || pl.splits == 1) return (int)e;
     launch_wq_splitk_reduce(p, pl.splits, XDT, st);

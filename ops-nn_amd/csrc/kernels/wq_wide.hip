@@ -376,6 +376,7 @@ int launch_one(const WqParams& p, const WqWidePlan& pl, hipStream_t st)
     }
     const int tiles = (int)((p.K + WW_KT - 1) / WW_KT);
     const dim3 grid((unsigned)((p.N + WW_COLS - 1) / WW_COLS), (unsigned)pl.splits, (unsigned)((p.M + 16 * MB - 1) / (16 * MB)));
+    note_route("wq_wide", pl.splits);
     hipLaunchKernelGGL(k, grid, dim3(512), ww_ring(WBITS, MB) + pl.groups * WW_COLS * 4, st, p, tiles, pl.splits, pl.groups);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || pl.splits == 1) return (int)e;
     launch_wq_splitk_reduce(p, pl.splits, XDT, st);

@@ -1360,6 +1360,7 @@ static int launch_xreg_one(const WqParams& p, hipStream_t st, int splits = 1)
         if (e != hipSuccess) return (int)e;
         device_flag_set(attr_set);
     }
+    note_route("wq_xreg", splits);
     hipLaunchKernelGGL(k, dim3((unsigned)(nblocks < g ? nblocks : g), (unsigned)splits), dim3(NW * 64), lds, st, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || splits == 1) return (int)e;

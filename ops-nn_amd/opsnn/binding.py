@@ -200,6 +200,7 @@ _SIGS = {
     "opsnnTranspose4": (C.c_int, [C.c_void_p, C.c_void_p, C.c_int64, C.c_int64, C.c_int64, C.c_void_p]),
     "opsnnSetFp8Fast": (None, [C.c_int]),
     "opsnnSetForcePlain": (None, [C.c_int]),
+    "opsnnDebugLastRoute": (C.c_char_p, [C.POINTER(C.c_int)]),
     "opsnnSetMx8Wide": (None, [C.c_int]),
     "opsnnSetWqTileMin": (None, [C.c_int]),
     "opsnnGetFp8Fast": (C.c_int, []),
