@@ -292,6 +292,14 @@ __device__ __forceinline__ void wait_copies()
     asm volatile("" : : : "memory");
 }
 
+// LDS that lanes of one wave exchange: what is written in front is there for every lane behind, and what is read in front has been read
+// before anything behind overwrites it (a wave's LDS operations execute in order; this keeps the compiler to it).
+__device__ __forceinline__ void wave_lds_fence()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Workgroup ids are dealt round-robin over the 8 XCDs; give each XCD (own L2) a contiguous
 // range of logical tile ids so that neighbouring tiles share operand panels in one L2.
 __device__ __forceinline__ uint32_t xcd_remap(uint32_t wg, uint32_t total)

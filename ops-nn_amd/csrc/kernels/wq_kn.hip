@@ -126,6 +126,7 @@ __global__ __launch_bounds__(256, 2) void wq_kn_kernel(WqParams p, int splits, i
         auto load_window = [&](int st, int end) {
             g_lo = group_of(st);
             const int n_groups = group_of(end - 1) - g_lo + 1;
+            wave_lds_fence();   // (other lanes of the wave read what a lane writes here, and read the window before until now)
             for (int g = q; g < n_groups; g += 4) {   // (lane r: its own CPL columns)
                 uint32_t v[HAS_OFF ? 2 : 1][CPL / 2];
                 if (p.s_cs == 1) {
@@ -141,6 +142,7 @@ __global__ __launch_bounds__(256, 2) void wq_kn_kernel(WqParams p, int splits, i
                 __builtin_memcpy(tab + g * (32 * CPL) + r * (2 * CPL), v[0], 2 * CPL);
                 if constexpr (HAS_OFF) __builtin_memcpy(tab + (KN_GROUPS + g) * (32 * CPL) + r * (2 * CPL), v[1], 2 * CPL);
             }
+            wave_lds_fence();
         };
         auto step = [&](auto jc, int st) __attribute__((always_inline)) {
             constexpr int j = decltype(jc)::value;

@@ -44,3 +44,16 @@ def test_small_weights_give_the_bits_of_their_k_contiguous_form(gpu, M, K, N, w_
         w = w.T
     other = dict(inp, w=np.ascontiguousarray(w), tW=True)
     assert np.array_equal(cases.run_wq_aclnn(m, inp, M, K, N), cases.run_wq_aclnn(m, other, M, K, N))
+
+
+# groups of 32 against a wave's 13 steps: the table of scales is laid down again while the loop runs
+@pytest.mark.parametrize("w_dt,x_dt,off", [("i4", "f16", True), ("i4", "bf16", False)])
+def test_table_of_scales_in_several_windows(gpu, w_dt, x_dt, off):
+    m = gpu
+    M, K, N = 5, 16384, 12290
+    xd = m.ACL_FLOAT16 if x_dt == "f16" else m.ACL_BF16
+    inp = cases.make_wq_inputs(m, M, K, N, 11, xd, m.ACL_INT4, 32, False, off, None)
+    print(f"case kn windows M={M} K={K} N={N} {x_dt}", flush=True)
+    got = cases.run_wq_aclnn(m, inp, M, K, N)
+    assert m.lib().opsnnDebugLastRoute(None) == b"wq_kn_table"
+    _b16_bar(got, cases.oracle_wq(m, inp, M, K, N), orc.F16 if x_dt == "f16" else orc.BF16, "kn windows", K)
