@@ -78,27 +78,62 @@ inline int splitk_factor(int64_t tiles, int64_t ktiles, double tile_us, int64_t 
     }
     return best;
 }
-// MXFP4 on the tile kernels: 128 x 128 or 256 x 256 tiles, and how many K segments.  A K tile of 256 elements takes a CU 1.4 us in the
-// small tile, 2.3 in the large one, which computes four times as much; partial sums move at 4 bytes a ps, behind a second launch.  Small
-// tiles where large ones would be at most 64, a quarter of the CUs, unless the large ones in segments are ahead (505 x 17536 x 6208 108 us on
-// small tiles; 1024 x 4096 x 4096 22.9 against 28.0 on large ones, at 128 large tiles it is 42 against 32).
+// MXFP4 on the tile kernels: 128 x 128 or 256 x 256 tiles, how many K segments, and the time in us that the choice rests on.
+// Fitted to 1210 timed launches of 350 calls (M 17 .. 4096, K 1024 .. 18432 with and without a tail, N 1024 .. 28672, 1 to 4 batches), each
+// as the geometric mean of its time with the weight from memory and from the last-level cache: a start, K steps of 256 elements for as
+// many workgroups as a CU takes one after the other -- two small ones side by side --, the operands' bytes, the second kernel of a K split, and
+// for a K that is no whole 128 the padded copies, which small tiles and segments run on and large tiles in one piece do not (median error
+// 4 % on small tiles, 8 on large ones).  The launcher asks with the same sizes: what is planned cut is launched cut.
+// (Planned in segments but launched in one, 594 x 16320 x 5312 took 127 us, 2456 x 10816 x 1211 105; 83 and 73 now.)
 struct Mxfp4Plan {
     bool small;
     int splits;
+    double us;
 };
+inline double mxfp4_tiles_us(bool small, int64_t M, int64_t N, int64_t K, int64_t batch, int splits)
+{
+    static const struct { double start, step, round, two, reduce, reduce_mb, copy, copy_mb, mb; } cost[3] = {   // mb: us per 10^6 bytes
+        {3.25, 0.81, 0.0, 1.95, 2.5, 2.9, 8.5, 0.19, 0.072},    // small, up to 128 rows
+        {2.8, 1.05, 0.0, 1.9, 2.6, 2.2, 9.6, 0.14, 0.114},      // small
+        {3.75, 1.67, 6.5, 1.0, 3.2, 1.5, 8.3, 0.12, 0.15}};     // large
+    const auto& c = cost[small ? (M <= 128 ? 0 : 1) : 2];
+    const int64_t bm = small ? 128 : 256, wgs = ((M + bm - 1) / bm) * ((N + bm - 1) / bm) * batch * splits;
+    const int64_t steps = ((K + 255) / 256 + splits - 1) / splits;
+    double turns = (double)((wgs + 255) / 256);
+    if (small && wgs > 256) turns = wgs <= 512 ? c.two : c.two * 0.5 * ((double)wgs / 512.0 + (double)((wgs + 511) / 512));
+    const double mb = (double)(M + N) * (double)K * (double)batch * 0.5e-6, out = (double)M * (double)N * (double)batch * (N % 4 ? 2e-6 : 1e-6);
+    return c.start + turns * ((double)steps * c.step + c.round) + mb * c.mb + (splits > 1 ? c.reduce + c.reduce_mb * splits * out : 0.0) +
+           (K % 128 && (small || splits > 1) ? c.copy + 2.0 * mb * c.copy_mb : 0.0);
+}
 inline Mxfp4Plan mxfp4_tile_plan(int64_t M, int64_t N, int64_t K, int64_t batch, bool may_split)
 {
-    const int64_t ktiles = (K + 255) / 256, out = M * N * batch;
-    auto best = [&](int64_t bm, double t, int& splits) {
-        const int64_t tiles = ((M + bm - 1) / bm) * ((N + bm - 1) / bm) * batch;
-        splits = may_split ? splitk_factor(tiles, ktiles, t, out, 4.0e6) : 1;
-        return (double)((tiles * splits + 255) / 256) * (double)((ktiles + splits - 1) / splits) * t + (splits > 1 ? 4.0 + 8.0 * splits * (double)out / 4.0e6 : 0.0);
-    };
-    int s128, s256;
-    const double us128 = best(128, 1.4, s128), us256 = best(256, 2.3, s256);
-    const int64_t t256 = ((M + 255) / 256) * ((N + 255) / 256) * batch;
-    const bool small = M <= 128 || N <= 128 || (t256 <= 64 && us128 < 1.05 * us256);
-    return {small, small ? s128 : s256};
+    Mxfp4Plan best{true, 1, 1e30};
+    if (M > 128 && N > 128 && K % 128 == 0) {
+        // Whole K tiles: small ones where large ones would be at most 64, a quarter of the CUs, unless the large ones in segments are
+        // ahead, at 1.4 and 2.3 us a K tile (505 x 17536 x 6208 108 us on small tiles; 1024 x 4096 x 4096 22.9 against 28.0 on large ones, at 128
+        // large tiles it is 42 against 32).  The estimate above chooses no better here: of 55 calls 6 became faster, 5 slower.
+        const int64_t ktiles = (K + 255) / 256, out = M * N * batch;
+        auto plan = [&](int64_t bm, double t, int& splits) {
+            const int64_t tiles = ((M + bm - 1) / bm) * ((N + bm - 1) / bm) * batch;
+            splits = may_split ? splitk_factor(tiles, ktiles, t, out, 4.0e6) : 1;
+            return (double)((tiles * splits + 255) / 256) * (double)((ktiles + splits - 1) / splits) * t + (splits > 1 ? 4.0 + 8.0 * splits * (double)out / 4.0e6 : 0.0);
+        };
+        int s128, s256;
+        const double us128 = plan(128, 1.4, s128), us256 = plan(256, 2.3, s256);
+        best.small = ((M + 255) / 256) * ((N + 255) / 256) * batch <= 64 && us128 < 1.05 * us256;
+        best.splits = best.small ? s128 : s256;
+        best.us = mxfp4_tiles_us(best.small, M, N, K, batch, best.splits);
+        return best;
+    }
+    for (int small = 1; small >= (M <= 128 || N <= 128 ? 1 : 0); small--) {
+        const int64_t bm = small ? 128 : 256, tiles = ((M + bm - 1) / bm) * ((N + bm - 1) / bm) * batch;
+        for (int s : {1, 2, 3, 4, 5, 6, 8, 12, 16}) {
+            if (s > 1 && (!may_split || (K + 255) / 256 < 4 * s || tiles * s > 256)) break;
+            const double us = mxfp4_tiles_us(small != 0, M, N, K, batch, s) * (s > 1 ? 1.03 : 1.0);   // (in doubt in one piece)
+            if (us < best.us) best = {small != 0, s, us};
+        }
+    }
+    return best;
 }
 // How a product of two K-contiguous operands whose 256 x 256 tiles would not fill the chip once (or of up to 128 rows or columns)
 // is tiled (qmm_int8.hip; int8, and the 16-bit operands of gemm16.hip).  KB: bytes of K.  variant: the OPSNN_VARIANT_I8_*

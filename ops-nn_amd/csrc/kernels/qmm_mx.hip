@@ -359,10 +359,14 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
     if (rows4) return launch_mxfp4_rows(a, st);
     if (rows8) return launch_fp8_stream(a, FP8X_MX, sk, st);
     const bool small = a.M <= 128 || a.N <= 128;
-    const bool fp4_small = a.force_variant == OPSNN_VARIANT_MX_128 || mxfp4_tile_plan(a.M, a.N, a.K, a.batch, sk.splits > 1 && a.force_variant == 0).small;
+    // (the plan that the partial sums were laid out for, or, where a call comes without them, one that leaves K in one piece)
+    Mxfp4Plan fp4_plan = mxfp4_tile_plan(a.M, a.N, a.K, a.batch, a.force_variant == 0);
+    if (fp4_plan.splits > 1 && (!sk.part || sk.splits != fp4_plan.splits)) fp4_plan = mxfp4_tile_plan(a.M, a.N, a.K, a.batch, false);
+    const bool fp4_small = a.force_variant == OPSNN_VARIANT_MX_128 || fp4_plan.small, fp4_cut = fp4_plan.splits > 1 && a.force_variant == 0;
     if (pad) {
         if (!mx_pad_layout(a, L)) return OPSNN_NOT_TAKEN;   // (the same answer as for the planned view: its conditions do not look at x2's address beyond its alignment)
-        const int rc = fp4 && !fp4_small ? mx_pad_scales(a, L, st) : mx_pad_prestep(a, L, st);
+        // (large fp4 tiles in segments deal whole tiles of 128 elements: their operands are padded like everybody's)
+        const int rc = fp4 && !fp4_small && !fp4_cut ? mx_pad_scales(a, L, st) : mx_pad_prestep(a, L, st);
         if (rc != 0) return rc;
     }
     if (a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E2M1) return launch_mx_a8w4_mfma(a, st, sk);   // fp8 x fp4: qmm_fp8_block.hip
@@ -405,7 +409,7 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
     if (fp4) {
         // few tiles against a long K: K split over workgroups (fp32 partial sums in front of the workspace), on the tiles
         // chosen below, whole ones
-        const bool split = sk.splits > 1 && sk.part && a.force_variant == 0 && a.K % 128 == 0;
+        const bool split = fp4_cut;
         if (split) { g.splits = sk.splits; g.part = (int32_t*)sk.part; }
         note_route(fp4_small ? "mxfp4_tiles_128" : "mxfp4_tiles_256", split ? sk.splits : 1);
         if (fp4_small) {

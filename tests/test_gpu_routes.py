@@ -33,3 +33,29 @@ def test_names(gpu):
     assert block_route(m, 40, 1024, 512)[0] in ("fp8_stream", "fp8_wide")
     m.lib().opsnnSetForcePlain(1)
     assert block_route(m, 4, 256, 300) == ("plain", 1)
+
+
+def mx_route(m, M, K, N, fp4=True, batch=1, out=None, bias=None, tB=True):
+    cases.run_mx_aclnn(m, cases.make_mx_inputs(m, M, K, N, M + N + K, tB, fp4, batch=batch), M, K, N, tB, m.ACL_BF16 if out is None else out, bias)
+    return route(m)
+
+
+# K % 128 == 64: what the plan cuts along K is launched cut, and large tiles in one piece are never few
+@pytest.mark.parametrize("M,K,N", [(514, 2624, 13504), (505, 6208, 17472), (594, 16320, 5312), (2642, 12736, 1088), (200, 9024, 390), (130, 6208, 260)])
+def test_mxfp4_tail_is_launched_as_planned(gpu, M, K, N):
+    name, segments = mx_route(gpu, M, K, N)
+    tiles = -(-M // 256) * -(-N // 256)
+    assert name == "mxfp4_tiles_128" or (name == "mxfp4_tiles_256" and (segments > 1 or tiles > 128)), (name, segments)
+
+
+# (some rows of large tiles in segments, all of small ones)
+@pytest.mark.parametrize("M,K,N,rows", [(594, 16320, 5312, [0, 1, 255, 256, 511, 512, 593]), (200, 9024, 390, None), (130, 6208, 260, None)])
+def test_mxfp4_tail_in_segments(gpu, M, K, N, rows):
+    import oracle_api as orc
+    from test_gpu_other_modes import check_close
+    m = gpu
+    print(f"case mxfp4 tail segments M={M} K={K} N={N}", flush=True)
+    inp = cases.make_mx_inputs(m, M, K, N, K + N, True, True)
+    got = cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_BF16, None)
+    assert route(m)[1] > 1
+    check_close(got if rows is None else np.ascontiguousarray(got[:, rows]), cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, rows=rows), orc.BF16, "mxfp4 tail in segments")
