@@ -14,6 +14,8 @@
 // in flight, and meet in LDS at the end, added in wave order.  K is cut by waves only, so a call is one launch.
 // K need be no multiple of 128: what is left behind the last whole unit goes to the waves step by step, requested ahead of the
 // loop, lanes past the end of K with zeros for x1 and a unit scale on both sides.
+#include <cmath>
+
 #include "launch.h"
 #include "common.hip.h"
 
@@ -210,9 +212,10 @@ int launch_one(const Mx4RowsParams& p, int64_t batch, hipStream_t st)
 //
 // Up to 16 rows always: 1 x 7040 x 10176 32.5 us on the tile kernel and 10.7 here, 16 x 8192 x 8192 17.2 and 11.7, 16 x 4096 x 28672
 // 19.5 and 19.4, 16 x 1984 x 1056 in 8 batches (K padded by four launches there) 21.6 and 6.8.  With more rows each workgroup reads x1
-// as often as its columns' share of x2, and a large x2 is faster on the tiles where those can cut K: the two estimates below, fitted
-// to 45 calls of 24 .. 128 rows, in us (24 x 4480 x 15680 24.1 there and 14.4 here, 64 x 4480 x 1280 17.7 and 7.7, but 64 x 4096 x 28672
-// 22.0 and 43.8).
+// as often as its columns' share of x2, and a large x2 is faster on the tiles where those can cut K: the estimate below, fitted to 210
+// calls of 17 .. 128 rows, each as the geometric mean of its time with the weight from memory and from the last-level cache (median
+// error 7 %), against that of mxfp4_tile_plan (24 x 4480 x 15680 24.1 there and 14.4 here, 64 x 4480 x 1280 17.7 and 7.7, but
+// 64 x 4096 x 28672 22.0 and 43.8, 50 x 18176 x 1088 13.0 and 25.3).
 bool mxfp4_rows_wanted(const OpsnnQmmArgs& a)
 {
     if (a.x1_dtype != DT_E2M1 || a.x2_dtype != DT_E2M1 || a.force_variant != 0) return false;
@@ -221,21 +224,15 @@ bool mxfp4_rows_wanted(const OpsnnQmmArgs& a)
     if (a.x1.row_stride < 0 || a.x2.col_stride < 0 || a.x1_scale_mat.row_stride < 0 || a.x2_scale_mat.row_stride < 0) return false;
     if (a.x1.row_stride / 2 >= (1ll << 32) / MX4_MAX_ROWS || a.N * ((a.x2.row_stride == 1 ? a.x2.col_stride : a.K) / 2) >= (1ll << 32)) return false;
     if (a.M <= 16) return true;
-    static const double per_mb[5] = {0.0, 0.26, 0.40, 0.52, 0.62};   // by row blocks of 16, per 10^6 bytes of x2
-    const int64_t out = a.M * a.N * a.batch, tiles = (a.N + 127) / 128 * a.batch, steps = (a.K + 127) / 128;
-    const int64_t slabs = (a.M + 63) / 64;   // (above 64 rows in slabs of 64)
-    double here = (slabs > 1 ? per_mb[4] * (double)slabs : per_mb[(a.M + 15) / 16]) * 1e-6 * (double)(a.K / 2 * a.N * a.batch);
-    if (a.M > 32) {   // one workgroup a CU: its last round may be nearly empty, and a round is 3 us of latency at least
-        const double wgs = (double)((a.N + 31) / 32 * a.batch * slabs), rounds = (double)(int64_t)((wgs + 255.0) / 256.0);
-        if (wgs > 256.0) here *= 256.0 * rounds / wgs;
-        if (here < 3.2 * rounds) here = 3.2 * rounds;
-    }
-    here += 2.0;
-    const int s = a.K % 256 == 0 ? splitk_factor(tiles, a.K / 256, 0.6, out, 2.4e6) : 1;
-    double there = 3.5 + 0.55 * (double)steps / s * (double)((tiles * s + 511) / 512);
-    if (s > 1) there += 4.0 + 8.0 * s * (double)out / 2.4e6;
-    if (a.K % 128 != 0) there += 12.0;
-    return here < 0.93 * there;
+    // K steps of 128 elements in turns of eight waves; workgroups of 16 or 32 columns and up to 64 rows, two to a CU up to 32 rows
+    const int64_t w1 = (a.N + 15) / 16 * a.batch, slabs = (a.M + 63) / 64, mb = a.M > 64 ? 4 : (a.M + 15) / 16;
+    const int64_t nb = w1 <= 128 ? 1 : 2, wgs = (nb == 1 ? w1 : (a.N + 31) / 32 * a.batch) * slabs;
+    double turns = (double)((wgs + 255) / 256);
+    if (a.M <= 32 && wgs > 256) turns = wgs <= 512 ? 1.42 : 0.71 * ((double)wgs / 512.0 + (double)((wgs + 511) / 512));
+    const double steps = (double)((a.K + 1023) / 1024);
+    const double here = 2.05 + turns * steps * (0.276 + 0.026 * (double)(mb * nb) + 0.193 * (double)mb) +
+                        (double)a.batch * (double)a.N * (double)a.K * 0.5e-6 / 5.23 * std::sqrt((double)slabs);
+    return 0.98 * here < mxfp4_tile_plan(a.M, a.N, a.K, a.batch, true).us;
 }
 int launch_mxfp4_rows(const OpsnnQmmArgs& a, hipStream_t st)
 {

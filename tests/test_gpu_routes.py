@@ -59,3 +59,13 @@ def test_mxfp4_tail_in_segments(gpu, M, K, N, rows):
     got = cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_BF16, None)
     assert route(m)[1] > 1
     check_close(got if rows is None else np.ascontiguousarray(got[:, rows]), cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, rows=rows), orc.BF16, "mxfp4 tail in segments")
+
+
+# 17 to 128 rows of MXFP4: short K and many columns on the few-rows kernel, long K against few columns on tiles that cut it, whatever
+# K's tail
+@pytest.mark.parametrize("M,K,N,batch,want", [
+    (50, 18176, 1088, 1, "mxfp4_tiles_128"), (62, 11264, 1472, 1, "mxfp4_tiles_128"), (79, 15104, 1408, 1, "mxfp4_tiles_128"),
+    (44, 11200, 2504, 1, "mxfp4_rows"), (84, 2752, 4096, 1, "mxfp4_rows"), (24, 4480, 4096, 1, "mxfp4_rows"), (64, 4480, 1280, 1, "mxfp4_rows"),
+    (36, 5952, 2064, 2, "mxfp4_rows"), (64, 4096, 28672, 1, "mxfp4_tiles_128"), (16, 18176, 1088, 1, "mxfp4_rows")])
+def test_mxfp4_rows_or_tiles(gpu, M, K, N, batch, want):
+    assert mx_route(gpu, M, K, N, batch=batch)[0] == want
