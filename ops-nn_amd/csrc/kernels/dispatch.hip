@@ -17,7 +17,6 @@ int launch_blockscale_mfma(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk = {}
 int launch_fp8_rowcol_mfma(const OpsnnQmmArgs& a, hipStream_t st, bool merged_scales_ok, SplitK sk = {});
 int launch_rowcol_exact(const OpsnnQmmArgs& a, hipStream_t st, int ep_mode, SplitK sk = {});   // qmm_fp8_exact.hip
 int launch_fp8_stream(const OpsnnQmmArgs& a, Fp8xForm form, SplitK sk, hipStream_t st);   // qmm_fp8_stream.hip
-uint64_t blockscale_rows_reserve(const OpsnnQmmArgs& a, int* segments);
 int mxfp8_rows_ksplit(const OpsnnQmmArgs& a);   // qmm_fp8_rows.hip
 int launch_tcg_mfma(const OpsnnQmmArgs& a, hipStream_t st);
 uint64_t tcg_workspace_bytes(const OpsnnQmmArgs& a);
@@ -473,7 +472,7 @@ extern "C" uint64_t opsnnQmmWorkspace(const OpsnnQmmArgs* a, int mode)
 {
     if (!a) return 0;
     const uint64_t need = splitk_bytes(*a, splitk_for(*a, mode)) + qmm_workspace_base(a, mode);   // partial sums of a K split in front
-    uint64_t reserve = mode == 1 && !opsnn_force_plain() ? blockscale_rows_reserve(*a, nullptr) : 0;
+    uint64_t reserve = 0;
     // (above 128 rows: no less than what the tile kernels would use, which the stream kernel's rule stands in for)
     if (a->M > 128 && mode >= 1 && mode <= 3) reserve = splitk_bytes(*a, splitk_for(*a, mode, false)) + qmm_workspace_base(a, mode);
     return need > reserve ? need : reserve;

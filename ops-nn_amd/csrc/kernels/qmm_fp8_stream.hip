@@ -608,18 +608,6 @@ constexpr int narrow_per_cu(int mb, int nb)
 
 }  // namespace
 
-// Block scales, 17 .. 128 rows against whole scale blocks of columns: phase 1 reports no less than what it used to, an fp16 copy of x1
-// and the partial sums of `segments` K segments.  Where there were several, and above 64 rows, the segments here make do with that.
-uint64_t blockscale_rows_reserve(const OpsnnQmmArgs& a, int* segments)
-{
-    if (a.x1_dtype != DT_E4M3 || a.x2_dtype != DT_E4M3 || a.batch != 1 || a.bias || a.force_variant != 0) return 0;
-    if (a.M <= 16 || a.M > 128 || a.N % 128 != 0 || a.N < 256 || a.K % 128 != 0 || a.gsK != 128 || a.gsN != 128 || a.x2.row_stride != 1) return 0;
-    const int64_t slab = wq_narrow_slab_rows(a.M, a.N, true);
-    const int s = (slab ? slab : a.M) > 64 ? 1 : wq_rows_ksplit(8, a.M, a.N, a.K, a.K, true);
-    if (segments) *segments = s;
-    return (s > 1 ? ((uint64_t)s * (uint64_t)a.M * (uint64_t)a.N * 4 + 255) / 256 * 256 : 0) + (uint64_t)a.M * (uint64_t)a.K * 2;
-}
-
 // Does a call run here, and how?  (Sizes, types, strides and which operands there are: both phases ask.  x2 K-contiguous, or re-laid
 // out so by then.)
 //
@@ -657,17 +645,12 @@ bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8St
     const int64_t slabs = (a.M + 16 * mb - 1) / (16 * mb), units = (a.K + 127) / 128;
     const bool whole = a.K % 128 == 0;
     const float x2_mb = (float)a.N * (float)a.K * 1e-6f, out_m = (float)a.M * (float)a.N * 1e-6f;
-    uint64_t most = ~0ull;   // bytes of partial sums
-    if (int segments = 1; form == FP8X_BLOCK) {
-        const uint64_t reserve = blockscale_rows_reserve(a, &segments);
-        if (segments > 1 || (reserve && a.M > 64)) most = reserve;
-    }
     pl.mb = mb;
     float best = 1e30f;
     auto consider = [&](bool wide, int nb, int splits, int per_cu) {
         const int64_t strips = (a.N + (wide ? 64 : 16) * nb - 1) / ((wide ? 64 : 16) * nb), seg = (units + splits - 1) / splits;
         const int64_t per_wave = wide ? seg : (seg + 3) / 4;
-        if (splits > 1 && (!may_split || units < 4 * splits || (uint64_t)splits * (uint64_t)a.M * (uint64_t)a.N * 4 > most)) return;
+        if (splits > 1 && (!may_split || units < 4 * splits)) return;
         if (form == FP8X_BLOCK && per_wave > FS_MOST_BLOCKS) return;
         // (partial sums of a row that is no whole number of quads: stored piece by piece, added one column per thread)
         const float us = stream_us(wide ? wide_cost[form] : narrow_cost[form], mb, nb, strips * splits * slabs, wide ? seg : 2 * per_wave, slabs, splits, per_cu, x2_mb, a.N % 4 ? 2.0f * out_m : out_m);

@@ -69,3 +69,10 @@ def test_mxfp4_tail_in_segments(gpu, M, K, N, rows):
     (36, 5952, 2064, 2, "mxfp4_rows"), (64, 4096, 28672, 1, "mxfp4_tiles_128"), (16, 18176, 1088, 1, "mxfp4_rows")])
 def test_mxfp4_rows_or_tiles(gpu, M, K, N, batch, want):
     assert mx_route(gpu, M, K, N, batch=batch)[0] == want
+
+
+# fp8 block scales with whole scale blocks of columns: few workgroups against a long K run in segments, as with a ragged last block
+@pytest.mark.parametrize("M,K,N", [(128, 7168, 2048), (128, 8192, 1024), (72, 12288, 2560), (40, 16384, 1024)])
+def test_block_scales_are_cut_for_any_columns(gpu, M, K, N):
+    whole, ragged = block_route(gpu, M, K, N), block_route(gpu, M, K, N - 28)
+    assert whole == ragged and whole[1] > 1, (whole, ragged)
