@@ -8,6 +8,7 @@ acceptance rule (>= 99.9 % of elements within rtol = atol = 1e-3).  The fp8 bloc
 and the MX modes with fp8 operands run by default on exact fp16 products (that bar); their opt-in 8-bit
 matrix-instruction form (opsnnSetFp8Fast) is held to the looser bars written out in check_close.
 """
+import ctypes
 import os
 
 import numpy as np
@@ -114,36 +115,6 @@ def test_fp8_blockscale_fp32_output(gpu, M, K, N, tB, gsM, fast):
     assert np.array_equal(cases.run_blockscale_aclnn(m, inp, M, K, N, tB, m.ACL_FLOAT), want)
 
 
-def _rows_ksplit(wbits, M, N, K, group):
-    """The many-rows kernel's K segments (the library's rule, restated): 1 = K in one piece."""
-    if M < 17 or N % 32 or N < 256 or K < 4096:
-        return 1
-    wg = -(-N // 128)
-    slabs = 1
-    if M > 64:
-        if wg > 128:
-            return 1
-        n = max(min(256 // wg, -(-M // 64)), -(-M // 256))
-        if n < 2:
-            return 1
-        slab = -(-(-(-M // n)) // 16) * 16
-        slabs = -(-M // slab)
-    wgs, kx = slabs * wg, 2 * 4 * (128 // wbits)
-    unit = kx
-    if group < K:
-        unit = max(kx, group)
-        if unit % group or unit % kx:
-            return 1
-    if wgs > 128 or K % unit:
-        return 1
-    if K < 8192 and (K % (2 * kx) == 0 or wgs > 64 or M < 33):
-        return 1
-    s = min(256 // wgs, 8, K // 2048, K // unit)
-    if s == 2 and wgs > 64 and K < 12288:
-        return 1
-    return s if s >= 2 else 1
-
-
 @pytest.mark.parametrize("M,K,N,gsM,out", [
     # up to 16 rows (one pass): K shared by 16 waves (2048, 4096, 8192) or by 8 (1024, 3072, 5120, 6144, 7168); ragged columns;
     # more column blocks than workgroups (N = 8192: 512 blocks on 256 workgroups) and fewer
@@ -185,15 +156,17 @@ def test_fp8_blockscale_decode_rows(gpu, M, K, N, gsM, out):
         differ = float(np.mean(got != want))
         print(f"   {differ:.2e} of outputs differ from the ascending-block oracle", flush=True)
         assert differ < 2e-2
-    if M > 32 and N % 128 == 0:   # phase 1 plans the fp16 copy of x1 (and the partial sums of a K split): the many-rows route is the one taken
+    if M > 32 and N % 128 == 0:   # the stream kernels are taken, and phase 1 has left room for the partial sums of the segments they run in
+        segments = ctypes.c_int(0)
+        assert m.lib().opsnnDebugLastRoute(ctypes.byref(segments)) in (b"fp8_stream", b"fp8_wide")
         d = {k: m.DeviceBuffer(host=v) for k, v in inp.items() if isinstance(v, np.ndarray)}
         x1 = m.Tensor((M, K), m.ACL_FLOAT8_E4M3FN, d["x1"]); x2 = m.Tensor((N, K), m.ACL_FLOAT8_E4M3FN, d["x2"])
         s1 = m.Tensor(inp["s1"].shape[1:], m.ACL_FLOAT, d["s1"]); s2 = m.Tensor(inp["s2"].shape[1:], m.ACL_FLOAT, d["s2"])
         o = m.Tensor((M, N), dt, m.DeviceBuffer(M * N * 4))
         rc, ws, ex = m.quant_matmul_v5_get_workspace(x1, x2, s1, s2, o, transpose_x2=True, group_size=(gsM << 32) | (128 << 16) | 128)
-        ks = _rows_ksplit(8, M, N, K, K)
+        ks = segments.value
         part = -(-ks * M * N * 4 // 256) * 256 if ks > 1 else 0
-        assert rc == 0 and ws == part + M * K * 2, (rc, ws, ks)
+        assert rc == 0 and ws == part, (rc, ws, ks)
         m.lib().aclDestroyAclOpExecutor(ex)
     plain(True)
     assert np.array_equal(cases.run_blockscale_aclnn(m, inp, M, K, N, True, dt), want)
