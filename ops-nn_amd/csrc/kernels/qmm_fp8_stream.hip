@@ -20,6 +20,8 @@
 // 24 x 2560 x 1536 19.8 -> 7.0, 64 x 18432 x 7168 50.2 -> 40.3 -- 3.3 TB/s, of 5.6 that the copies alone reach --, 32 x 7296 x 22529 92 -> 40,
 // MX 64 x 10496 x 1152 25.0 -> 14.3.)
 // An operand piece of 16 bytes is two k steps of v_mfma_f32_16x16x32_{f16,bf16}, cut the same way for x1 and x2.
+#include <cmath>
+
 #include "launch.h"
 #include "common.hip.h"
 
@@ -576,7 +578,7 @@ int launch_form(const Fp8StreamParams& p, const Fp8StreamPlan& pl, hipStream_t s
     return -1;
 }
 
-// What a launch takes, in us, fitted to 2700 timed launches of 216 calls (M 4 .. 128, K 1024 .. 16384, N 1024 .. 28000; median error 3 %
+// Which layout is best: what a launch takes, in us, x2 from memory, fitted to 2700 timed launches of 216 calls (M 4 .. 128, K 1024 .. 16384, N 1024 .. 28000; median error 3 %
 // on the wide kernel, 10 % on the other): a start, the K tiles of a workgroup by its row and column blocks -- more than one workgroup a
 // CU taking turns --, x2's stream as the other bound, and the second kernel of a K split.
 struct StreamCost {
@@ -586,17 +588,48 @@ const StreamCost narrow_cost[3] = {   // by Fp8xForm
     {3.5f, 0.116f, 0.039f, 0.108f, 1.88f, 3.2f, 8.0f, 3.5f, 0.0f}, {4.8f, 0.088f, 0.013f, 0.094f, 1.81f, 2.1f, 8.0f, 3.7f, 1.0f}, {3.7f, 0.235f, 0.052f, 0.078f, 1.64f, 3.0f, 8.0f, 3.5f, 0.0f}};
 const StreamCost wide_cost[3] = {
     {5.2f, 0.241f, 0.050f, 0.021f, 1.61f, 2.6f, 2.1f, 5.6f, 0.15f}, {5.5f, 0.193f, 0.051f, 0.010f, 1.70f, 1.9f, 2.4f, 5.8f, 0.4f}, {4.7f, 0.296f, 0.055f, 0.025f, 1.73f, 3.0f, 2.1f, 4.3f, 0.33f}};
+float turns(int64_t wgs, int per_cu, float two)   // workgroups one after the other, or two at a time
+{
+    const float w = (float)wgs / 256.0f;
+    if (w <= 1.0f) return 1.0f;
+    if (per_cu < 2) return (float)((wgs + 255) / 256);
+    return w <= 2.0f ? two : two * 0.5f * (0.5f * w + (float)((wgs + 256 * per_cu - 1) / (256 * per_cu)));
+}
 float stream_us(const StreamCost& c, int mb, int nb, int64_t wgs, int64_t tiles, int64_t slabs, int splits, int per_cu, float x2_mb, float out_m)
 {
-    const float w = (float)wgs / 256.0f, t = c.tile + c.tile_mn * (float)(mb * nb) + c.tile_m * (float)mb;
-    float load = 1.0f;   // rounds: one workgroup after the other, or two at a time
-    if (w > 1.0f) {
-        const float r = per_cu >= 2 ? 0.5f * w : w, whole = (float)((wgs + 256 * per_cu - 1) / (256 * per_cu));
-        load = per_cu >= 2 ? (w <= 2.0f ? c.two : c.two * 0.5f * (r + whole)) : whole;
-    }
-    const float cu = (float)tiles * t * load, hbm = x2_mb / c.bw * (1.0f + c.again * (float)(slabs - 1));
+    const float t = c.tile + c.tile_mn * (float)(mb * nb) + c.tile_m * (float)mb;
+    const float cu = (float)tiles * t * turns(wgs, per_cu, c.two), hbm = x2_mb / c.bw * (1.0f + c.again * (float)(slabs - 1));
     const float most = cu > hbm ? cu : hbm, least = cu > hbm ? hbm : cu, q = least / most;
     return c.start + most * (1.0f + 0.19f * q * q * q * q) + (splits > 1 ? c.reduce + c.reduce_mb * (float)splits * out_m : 0.0f);
+}
+// Whether a call runs here at all: what the chosen layout typically takes, the geometric mean of its time with x2 from memory and with
+// x2 in the last-level cache.  Fitted to 12200 launches of 1190 calls in both states (M 1 .. 512, K 1024 .. 18432, N 1024 .. 28672; median error
+// 4 %).  `round`: a workgroup's start and end; `few`: x2's rate falls with that power of the share of CUs that have a workgroup.
+struct StreamTime {
+    float start, tile, tile_mn, tile_m, round, two, bw, again, few, reduce, reduce_mb;
+};
+const StreamTime narrow_time[3] = {   // by Fp8xForm; its copies and products add up (a workgroup a CU, one ring a wave)
+    {1.48f, 0.026f, 0.027f, 0.076f, 2.26f, 1.44f, 9.7f, 0.50f, 0.67f, 0.0f, 0.0f}, {1.44f, 0.010f, 0.027f, 0.051f, 2.2f, 1.33f, 9.4f, 0.61f, 0.58f, 0.0f, 0.0f},
+    {1.0f, 0.018f, 0.028f, 0.089f, 2.7f, 1.34f, 6.3f, 0.59f, 0.71f, 0.0f, 0.0f}};
+const StreamTime wide_time[3] = {
+    {3.26f, 0.204f, 0.063f, 0.004f, 0.87f, 1.6f, 5.9f, 0.67f, 0.0f, 2.3f, 1.44f}, {3.21f, 0.160f, 0.064f, 0.002f, 1.09f, 1.65f, 5.95f, 0.65f, 0.0f, 2.05f, 1.26f},
+    {2.84f, 0.221f, 0.075f, 0.017f, 1.16f, 1.61f, 4.9f, 0.37f, 0.48f, 2.7f, 1.43f}};
+float stream_typical_us(const StreamTime& c, const Fp8StreamPlan& pl, int64_t wgs, int64_t tiles, int64_t slabs, int per_cu, float x2_mb, float out_m)
+{
+    const float t = c.tile + c.tile_mn * (float)(pl.mb * pl.nb) + c.tile_m * (float)pl.mb;
+    const float cu = turns(wgs, per_cu, c.two) * ((float)tiles * t + c.round);
+    const float hbm = x2_mb / c.bw * (1.0f + c.again * (float)(slabs - 1)) * (wgs < 256 ? powf(256.0f / (float)wgs, c.few) : 1.0f);
+    const float both = pl.wide ? cbrtf(cu * cu * cu + hbm * hbm * hbm) : cu + hbm;
+    return c.start + both + (pl.splits > 1 ? c.reduce + c.reduce_mb * (float)pl.splits * out_m : 0.0f);
+}
+// The x-in-registers kernel of qmm_fp8_decode.hip on the same terms (292 calls of up to 16 rows, median error 4 %): its workgroups take
+// blocks of 16 columns in turns; idle waves read what others read, which costs no bytes from memory.
+float decode_typical_us(const QmmDecodePlan& pl, bool mx, int64_t N, float x2_mb, float out_m)
+{
+    const int64_t cus = 256 / pl.splits, rounds = ((N + 15) / 16 + cus - 1) / cus;
+    const float block = mx ? 0.685f : 0.81f, wide = pl.nw == 16 ? (mx ? 2.04f : 1.8f) : 1.0f;
+    const float cu = (float)rounds * ((float)pl.nblk * block * wide + (mx ? 0.435f : 0.28f)), hbm = x2_mb / (mx ? 10.6f : 12.0f);
+    return (mx ? 3.35f : 3.18f) + cbrtf(cu * cu * cu + hbm * hbm * hbm) + (pl.splits > 1 ? 1.9f + (mx ? 3.2f : 2.6f) * (float)pl.splits * out_m : 0.0f);
 }
 template <int FORM>
 constexpr int narrow_per_cu(int mb, int nb)
@@ -617,9 +650,9 @@ constexpr int narrow_per_cu(int mb, int nb)
 // 49.5), and, with row / column scales, somewhat larger ones with a
 // last half K tile, which run on padded copies there (246 x 12224 x 2560 76 and 49).
 //
-// Up to 128 rows.  Row / column scales always; block scales but for a K that the x-in-registers kernel of qmm_fp8_decode.hip shares
-// out evenly, up to 16 rows (16 x 7168 x 18432 29.9 us there, 32.8 here; 8 x 9856 x 23040, which it cuts, 61 and 44); MX the same, and from 65
-// rows on the many-rows kernel's large weights (128 x 11392 x 27904 132 there, 147 here; 128 x 9856 x 8128 82 and 50).
+// Up to 128 rows.  Row / column scales always; block and MX scales with up to 16 rows where the x-in-registers kernel of qmm_fp8_decode.hip
+// is not ahead by the estimates above (x2 from memory, there and here: 16 x 7168 x 18432 29.9 and 32.8 us, MX 3 x 6272 x 19456 32.8 and 42,
+// 8 x 3200 x 1920 7.7 and 10.8; 8 x 9856 x 23040, which it cuts, 61 and 44); MX from 65 rows but on the many-rows kernel's large weights (128 x 11392 x 27904 132 there, 147 here; 128 x 9856 x 8128 82 and 50).
 constexpr int64_t FS_MANY_ROWS = 3200000000, FS_MANY_ROWS_TAIL = 12000000000;   // multiplications
 bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8StreamPlan& pl)
 {
@@ -647,6 +680,8 @@ bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8St
     const float x2_mb = (float)a.N * (float)a.K * 1e-6f, out_m = (float)a.M * (float)a.N * 1e-6f;
     pl.mb = mb;
     float best = 1e30f;
+    int64_t wgs = 0, k_tiles = 0;   // of the best so far
+    int cu_wgs = 1;
     auto consider = [&](bool wide, int nb, int splits, int per_cu) {
         const int64_t strips = (a.N + (wide ? 64 : 16) * nb - 1) / ((wide ? 64 : 16) * nb), seg = (units + splits - 1) / splits;
         const int64_t per_wave = wide ? seg : (seg + 3) / 4;
@@ -654,7 +689,7 @@ bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8St
         if (form == FP8X_BLOCK && per_wave > FS_MOST_BLOCKS) return;
         // (partial sums of a row that is no whole number of quads: stored piece by piece, added one column per thread)
         const float us = stream_us(wide ? wide_cost[form] : narrow_cost[form], mb, nb, strips * splits * slabs, wide ? seg : 2 * per_wave, slabs, splits, per_cu, x2_mb, a.N % 4 ? 2.0f * out_m : out_m);
-        if (us < best) { best = us; pl.wide = wide; pl.nb = nb; pl.splits = splits; }
+        if (us < best) { best = us; pl.wide = wide; pl.nb = nb; pl.splits = splits; wgs = strips * splits * slabs; k_tiles = wide ? seg : 2 * per_wave; cu_wgs = per_cu; }
     };
     // the narrow kernel where one round of workgroups is enough, the wide one for the rest; a last half K tile is the narrow one's
     static const int steps[8] = {1, 2, 3, 4, 6, 8, 12, 16};
@@ -666,11 +701,8 @@ bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8St
     for (int i = 0; !whole && i < 6; i++) consider(false, 4, steps[i], 1);
     if (best >= 1e30f) return false;
     if (a.M <= 16 && whole && form != FP8X_PLAIN) {
-        QmmDecodePlan dp;
-        if (qmm_decode_plan(a.K, may_split, dp)) {
-            const float slots = (float)(dp.splits * dp.nw * dp.nblk) / (float)units;
-            if (4.5f + x2_mb / (form == FP8X_MX ? 4.4f : 5.2f) * slots + (dp.splits > 1 ? 3.5f : 0.0f) < best) return false;
-        }
+        const float out = a.N % 4 ? 2.0f * out_m : out_m, here = stream_typical_us((pl.wide ? wide_time : narrow_time)[form], pl, wgs, k_tiles, slabs, cu_wgs, x2_mb, out);
+        if (QmmDecodePlan dp; qmm_decode_plan(a.K, may_split, dp) && decode_typical_us(dp, form == FP8X_MX, a.N, x2_mb, out) < here) return false;
     }
     return !(form == FP8X_MX && whole && a.M > 64 && x2_mb > 100.0f && a.out_dtype == DT_BF16 && a.N % 32 == 0);
 }
@@ -679,9 +711,9 @@ int launch_fp8_stream(const OpsnnQmmArgs& a, Fp8xForm form, SplitK sk, hipStream
 {
     Fp8StreamPlan pl;
     if (a.M > 128 && a.K % 128 == 0 && opsnnGetFp8Fast()) return OPSNN_NOT_TAKEN;   // (the caller asked for the 8-bit instruction)
-    if (!fp8_stream_plan(a, form, sk.part != nullptr, pl)) return OPSNN_NOT_TAKEN;
-    // (partial sums laid out for other segments: a call that another layout of its operands has changed on the way)
-    if (pl.splits > 1 && sk.splits < pl.splits && !fp8_stream_plan(a, form, false, pl)) return OPSNN_NOT_TAKEN;
+    if (!fp8_stream_plan(a, form, true, pl)) return OPSNN_NOT_TAKEN;
+    // (no partial sums, or laid out for other segments: a call that another layout of its operands has changed on the way)
+    if (pl.splits > 1 && (!sk.part || sk.splits < pl.splits) && !fp8_stream_plan(a, form, false, pl)) return OPSNN_NOT_TAKEN;
     const int splits = pl.splits;
     if (a.x1.col_stride != 1 || a.x2.row_stride != 1) return OPSNN_NOT_TAKEN;
     Fp8StreamParams p{};

@@ -332,7 +332,7 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
     MxPad L;
     // few rows: the kernels that take a K tail as it is
     Fp8StreamPlan spl;
-    const bool rows4 = fp4 && mxfp4_rows_wanted(a), rows8 = fp8 && exact && fp8_stream_plan(a, FP8X_MX, sk.part != nullptr, spl);
+    const bool rows4 = fp4 && mxfp4_rows_wanted(a), rows8 = fp8 && exact && fp8_stream_plan(a, FP8X_MX, true, spl);
     const bool pad = !rows4 && !rows8 && mx_pad_layout(planned, L);
     if (!pad && !rows4 && !rows8 && planned.K % 128 != 0) return OPSNN_NOT_TAKEN;
     if (planned.x2_scale_mat.col_stride != 2 || (fp4 || fp8 ? planned.x2_scale_mat.row_stride != (planned.K + 63) / 64 * 2 : planned.x2_scale_mat.row_stride % 4 != 0)) return OPSNN_NOT_TAKEN;
@@ -357,7 +357,11 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         mx_relayout_view(a, R, w);
     }
     if (rows4) return launch_mxfp4_rows(a, st);
-    if (rows8) return launch_fp8_stream(a, FP8X_MX, sk, st);
+    if (rows8) {
+        const int rc = launch_fp8_stream(a, FP8X_MX, sk, st);
+        if (rc != OPSNN_NOT_TAKEN || a.K % 128 != 0) return rc;   // (a K tail was left as it is)
+        sk = SplitK{};
+    }
     const bool small = a.M <= 128 || a.N <= 128;
     // (the plan that the partial sums were laid out for, or, where a call comes without them, one that leaves K in one piece)
     Mxfp4Plan fp4_plan = mxfp4_tile_plan(a.M, a.N, a.K, a.batch, a.force_variant == 0);

@@ -74,5 +74,15 @@ def test_mxfp4_rows_or_tiles(gpu, M, K, N, batch, want):
 # fp8 block scales with whole scale blocks of columns: few workgroups against a long K run in segments, as with a ragged last block
 @pytest.mark.parametrize("M,K,N", [(128, 7168, 2048), (128, 8192, 1024), (72, 12288, 2560), (40, 16384, 1024)])
 def test_block_scales_are_cut_for_any_columns(gpu, M, K, N):
-    whole, ragged = block_route(gpu, M, K, N), block_route(gpu, M, K, N - 28)
-    assert whole == ragged and whole[1] > 1, (whole, ragged)
+    for n in (N, N - 28):
+        assert block_route(gpu, M, K, n)[1] > 1, n
+
+
+# up to 16 rows of fp8: shapes that were measured on both kernels, the weight from memory and from the last-level cache
+@pytest.mark.parametrize("mode,M,K,N,want", [
+    ("mx", 8, 3200, 1920, "fp8_decode"), ("mx", 16, 2688, 9728, "fp8_decode"), ("mx", 1, 1792, 8192, "fp8_decode"),
+    ("block", 1, 1792, 4096, "fp8_decode"),
+    ("mx", 1, 12800, 4096, "fp8_wide"), ("block", 1, 12800, 4096, "fp8_wide")])
+def test_up_to_16_rows_of_fp8(gpu, mode, M, K, N, want):
+    got = mx_route(gpu, M, K, N, False) if mode == "mx" else block_route(gpu, M, K, N)
+    assert got[0] == want, got
