@@ -17,7 +17,6 @@ int launch_blockscale_mfma(const OpsnnQmmArgs& a, hipStream_t st, SplitK sk = {}
 int launch_fp8_rowcol_mfma(const OpsnnQmmArgs& a, hipStream_t st, bool merged_scales_ok, SplitK sk = {});
 int launch_rowcol_exact(const OpsnnQmmArgs& a, hipStream_t st, int ep_mode, SplitK sk = {});   // qmm_fp8_exact.hip
 int launch_fp8_stream(const OpsnnQmmArgs& a, Fp8xForm form, SplitK sk, hipStream_t st);   // qmm_fp8_stream.hip
-int mxfp8_rows_ksplit(const OpsnnQmmArgs& a);   // qmm_fp8_rows.hip
 int launch_tcg_mfma(const OpsnnQmmArgs& a, hipStream_t st);
 uint64_t tcg_workspace_bytes(const OpsnnQmmArgs& a);
 int launch_kg_mfma(const OpsnnQmmArgs& a, hipStream_t st);   // qmm_i4_kg.hip
@@ -239,10 +238,6 @@ static int splitk_for(const OpsnnQmmArgs& a, int mode, bool stream = true)
     if (a.M <= 16 && a.batch == 1 && a.N >= 256 && ((mode == 1 && (f8 || i8pt) && a.gsK == 128 && a.gsN == 128) || (a8w4 && out16) || (mode == 2 && f8))) {
         QmmDecodePlan pl;
         return qmm_decode_plan(a.K, true, pl, a8w4) ? pl.splits : 1;
-    }
-    // 33 .. 128 rows of MXFP8 on the many-rows kernel
-    if (mode == 2 && f8 && a.M <= 128) {
-        if (const int sr = mxfp8_rows_ksplit(a); sr > 1) return sr;
     }
     // (fewer than 64 x 64 outputs are the plain kernels' -- except int8 with few outputs against a long K, qmm_int8.hip)
     const bool tiny = a.M * a.N < 64 * 64;

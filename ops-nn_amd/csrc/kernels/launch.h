@@ -147,6 +147,7 @@ TilePlan tile_plan(int64_t M, int64_t N, int64_t KB, int64_t batch, bool may_spl
 // The tile (OPSNN_VARIANT_FP8X_*) and the K segments of a call on the exact fp8 kernel (qmm_fp8_exact.hip).
 struct Fp8xPlan {
     int tile, splits;
+    double us;   // the estimate that the choice rests on
 };
 enum Fp8xForm { FP8X_BLOCK, FP8X_PLAIN, FP8X_MX };   // block scales, row / column scales, MX scales
 Fp8xPlan fp8x_plan(int64_t M, int64_t N, int64_t K, int64_t batch, Fp8xForm form, bool may_split);

@@ -603,8 +603,7 @@ Fp8xPlan fp8x_plan(int64_t M, int64_t N, int64_t K, int64_t batch, Fp8xForm form
     const bool plain = form == FP8X_PLAIN, mx = form == FP8X_MX;
     const int64_t cus = 256, kt = (K + 127) / 128;   // (a K tail runs padded)
     const double round_us = mx ? 8.0 : 4.0, split_us = mx ? 2.0 : 5.0, sums_per_us = mx ? 5.0e6 : 6.0e6;
-    Fp8xPlan best{OPSNN_VARIANT_FP8X_256x128, 1};
-    double best_us = 1e30;
+    Fp8xPlan best{OPSNN_VARIANT_FP8X_256x128, 1, 1e30};
     auto offer = [&](int tile, int64_t bm, int64_t bn, double t0, double t1) {
         const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch;
         for (int s = 1; s <= 16 && (s == 1 || (may_split && tiles * s <= cus && kt / s >= 4)); s++) {
@@ -612,7 +611,7 @@ Fp8xPlan fp8x_plan(int64_t M, int64_t N, int64_t K, int64_t batch, Fp8xForm form
             const int64_t full = tiles * s / cus, rest = tiles * s % cus;
             double us = (double)full * (steps * (t0 + t1) + round_us) + (rest ? steps * (t0 + t1 * (double)rest / (double)cus) + round_us : 0.0);
             if (s > 1) us += split_us + 8.0 * s * (double)M * (double)N * (double)batch / sums_per_us;   // partial sums, second kernel
-            if (us < best_us) { best_us = us; best = {tile, s}; }
+            if (us < best.us) best = {tile, s, us};
         }
     };
     offer(OPSNN_VARIANT_FP8X_256x128, 256, 128, plain ? 1.25 : 1.37, plain ? 0.40 : 0.46);

@@ -631,6 +631,17 @@ float decode_typical_us(const QmmDecodePlan& pl, bool mx, int64_t N, float x2_mb
     const float cu = (float)rounds * ((float)pl.nblk * block * wide + (mx ? 0.435f : 0.28f)), hbm = x2_mb / (mx ? 10.6f : 12.0f);
     return (mx ? 3.35f : 3.18f) + cbrtf(cu * cu * cu + hbm * hbm * hbm) + (pl.splits > 1 ? 1.9f + (mx ? 3.2f : 2.6f) * (float)pl.splits * out_m : 0.0f);
 }
+// The exact tiles of qmm_fp8_exact.hip on the same terms: their plan's estimate with what it leaves out, and corrected where it is off
+// (524 calls of 65 .. 512 rows, median error 2 %).  K is cut there from 129 rows, MX from 65.
+float tiles_typical_us(int64_t M, int64_t N, int64_t K, Fp8xForm form, bool may_split)
+{
+    static const struct { float scale, start, out, out_odd, odd, split; } cost[3] = {   // by Fp8xForm
+        {0.978f, 1.85f, 0.38f, 1.42f, 1.09f, -0.96f}, {0.898f, 6.49f, 0.431f, 1.53f, 1.15f, -4.33f}, {1.03f, -0.78f, 0.434f, 2.02f, 0.29f, -1.2f}};
+    const auto& c = cost[form];
+    const Fp8xPlan pl = fp8x_plan(M, N, K, 1, form, may_split && (M > 128 || form == FP8X_MX));
+    const float out_m = (float)M * (float)N * 1e-6f;
+    return c.scale * (float)pl.us + c.start + out_m * (c.out + (N % 4 ? c.out_odd * (float)pl.splits : 0.0f)) + (N % 8 ? c.odd : 0.0f) + (pl.splits > 1 ? c.split : 0.0f);
+}
 template <int FORM>
 constexpr int narrow_per_cu(int mb, int nb)
 {
@@ -644,22 +655,22 @@ constexpr int narrow_per_cu(int mb, int nb)
 // Does a call run here, and how?  (Sizes, types, strides and which operands there are: both phases ask.  x2 K-contiguous, or re-laid
 // out so by then.)
 //
-// From 129 to 512 rows, in slabs of 64, K from 1024: small products, which leave most of the exact tile kernel's 128 x 128 tiles without a CU's worth
-// of work (row / column scales 181 x 2560 x 2368 16.4 us there, 11.1 here, 140 x 1536 x 17344 30.5 and 25.1; block scales 158 x 1152 x 2112 15.3
-// and 9.2, 405 x 1664 x 3848 24.2 and 18.9; MX 298 x 1280 x 1152 19.3 and 13.0; but 223 x 1024 x 15488 22.0 and 23.4, 258 x 3072 x 13440 41.8 and
-// 49.5), and, with row / column scales, somewhat larger ones with a
-// last half K tile, which run on padded copies there (246 x 12224 x 2560 76 and 49).
-//
-// Up to 128 rows.  Row / column scales always; block and MX scales with up to 16 rows where the x-in-registers kernel of qmm_fp8_decode.hip
+// Up to 64 rows.  Row / column scales always; block and MX scales with up to 16 rows where the x-in-registers kernel of qmm_fp8_decode.hip
 // is not ahead by the estimates above (x2 from memory, there and here: 16 x 7168 x 18432 29.9 and 32.8 us, MX 3 x 6272 x 19456 32.8 and 42,
-// 8 x 3200 x 1920 7.7 and 10.8; 8 x 9856 x 23040, which it cuts, 61 and 44); MX from 65 rows but on the many-rows kernel's large weights (128 x 11392 x 27904 132 there, 147 here; 128 x 9856 x 8128 82 and 50).
-constexpr int64_t FS_MANY_ROWS = 3200000000, FS_MANY_ROWS_TAIL = 12000000000;   // multiplications
+// 8 x 3200 x 1920 7.7 and 10.8; 8 x 9856 x 23040, which it cuts, 61 and 44).
+//
+// From 65 to 512 rows, in slabs of 64: products that leave most of the exact tiles without a CU's worth of work, by the estimates
+// (typical times there and here, MX 65 x 2048 x 2304 13.4 and 10.1 us, 128 x 1664 x 1472 15.2 and 8.9, 128 x 13568 x 8960 52 and 67,
+// 96 x 7424 x 18816 55 and 77; row / column scales 181 x 2560 x 2368 16.4 and 11.1, 114 x 11520 x 22208 89 and 108; block scales
+// 405 x 1664 x 3848 24.2 and 18.9).  A last half K tile runs on padded copies there: here up to so many multiplications above 128 rows (row /
+// column scales 246 x 12224 x 2560 76 and 49).
+constexpr int64_t FS_MANY_ROWS_TAIL = 3200000000, FS_MANY_ROWS_TAIL_PLAIN = 12000000000;
 bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8StreamPlan& pl)
 {
     if (a.x1_dtype != DT_E4M3 || a.x2_dtype != DT_E4M3 || a.batch != 1 || a.force_variant != 0) return false;
     if (a.out_dtype != DT_BF16 && a.out_dtype != DT_F16 && a.out_dtype != DT_F32) return false;
     if (a.M > 512 || a.N < 256 || a.K < 128 || a.K % 64 != 0 || a.K >= (1ll << 30) || a.N >= (1ll << 30)) return false;
-    if (a.M > 128 && (a.K < 1024 || a.M * a.N * a.K > (form == FP8X_PLAIN && a.K % 128 ? FS_MANY_ROWS_TAIL : FS_MANY_ROWS))) return false;
+    if (a.M > 128 && (a.K < 1024 || (a.K % 128 && a.M * a.N * a.K > (form == FP8X_PLAIN ? FS_MANY_ROWS_TAIL_PLAIN : FS_MANY_ROWS_TAIL)))) return false;
     const int64_t ldb = a.x2.row_stride == 1 ? a.x2.col_stride : a.K;
     // (32-bit lane offsets: from the first row of x1 and of its scales, from the workgroup's first column of x2)
     auto offsets_ok = [](int64_t rows, int64_t bytes) { return bytes >= 0 && bytes < (1ll << 31) / rows; };
@@ -700,11 +711,12 @@ bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8St
     }
     for (int i = 0; !whole && i < 6; i++) consider(false, 4, steps[i], 1);
     if (best >= 1e30f) return false;
-    if (a.M <= 16 && whole && form != FP8X_PLAIN) {
+    if (whole && (a.M > 64 || (a.M <= 16 && form != FP8X_PLAIN))) {
         const float out = a.N % 4 ? 2.0f * out_m : out_m, here = stream_typical_us((pl.wide ? wide_time : narrow_time)[form], pl, wgs, k_tiles, slabs, cu_wgs, x2_mb, out);
+        if (a.M > 64) return here <= tiles_typical_us(a.M, a.N, a.K, form, may_split);
         if (QmmDecodePlan dp; qmm_decode_plan(a.K, may_split, dp) && decode_typical_us(dp, form == FP8X_MX, a.N, x2_mb, out) < here) return false;
     }
-    return !(form == FP8X_MX && whole && a.M > 64 && x2_mb > 100.0f && a.out_dtype == DT_BF16 && a.N % 32 == 0);
+    return true;
 }
 
 int launch_fp8_stream(const OpsnnQmmArgs& a, Fp8xForm form, SplitK sk, hipStream_t st)

@@ -431,7 +431,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
     static_assert(WN * WK == 8, "eight waves");
     static_assert(!SLDS || WF == 0 || WF == 2, "the scale table serves the integer forms and the e8m0 bytes of e2m1 codes");
     static_assert(WF == 0 || !HAS_OFF, "floating-point weight codes have no offset");
-    static_assert(WF != 2 || WBITS == 4 || (WBITS == 8 && WK == 2), "e8m0 group scales: e2m1 codes, or e4m3 codes on the instances with two K waves");
+    static_assert(WF != 2 || WBITS == 4, "e8m0 group scales: e2m1 codes");
     constexpr int NT = 512;
     if (p.m_slab > 0) {   // several row slabs in one launch: this workgroup's is number blockIdx.y
         p.m_base += (int64_t)blockIdx.y * p.m_slab;
@@ -460,9 +460,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
     static_assert((16 * MB * XPR) % NT == 0 && XPR >= 16 && PF >= 2 && PPH >= 1 && STEPS == PPH * XH, "staging and prefetch shape");
     static_assert(MB <= 8 || (WF == 0 && SLDS) || WF == 1 || WF == 2, "the 192- / 256-row instances: integer codes with the scale table in LDS, or floating-point codes");
     static_assert(!(SLDS && WF == 2 && MB > 8) || WK == 2, "8-byte pieces: byte position of a lane's e8m0 scale inside the table word");
-    // a lane's piece holds half a group of 32 codes (8-byte pieces of e2m1 codes, 16-byte pieces of e4m3 codes): two lane
-    // groups share an e8m0 byte, a chunk of the wave holds two bytes and the table word of 128 k serves the chunks of both K waves
-    constexpr bool E8H = (MB > 8 && WBITS == 4) || (WF == 2 && WBITS == 8);
+    // an 8-byte piece of e2m1 codes holds half a group of 32: two lane groups share an e8m0 byte, a chunk of the wave holds two bytes
+    // and the table word of 128 k serves the chunks of both K waves
+    constexpr bool E8H = MB > 8 && WBITS == 4;
     // K in segments: this workgroup's is number blockIdx.z.  Segments are whole units of p.kunit k (whole slabs of x and
     // whole groups), as equal as that allows, the longer ones first.  From here on p.K is the segment's length and x, w, the scales and
     // offsets start at the segment; a row of x keeps its pitch ldx.
@@ -1480,8 +1480,7 @@ static int launch_rows_one(const WqParams& p, hipStream_t st)
         // beside the x buffers (e2m1 codes: one word per 128 k, the four e8m0 bytes of a row read as a word; the caller
         // passes cpg_shift 0)
         const size_t red = (size_t)WN * (WK - 1) * NB * MB * 4 * 64 * 4;
-        // (the caller counts a table word of 128 k in chunks: one of e2m1 codes, two of e4m3 codes)
-        const bool rows_ok = WF == 2 ? (p.s_cs % 4 == 0 && (uintptr_t)p.scale % 4 == 0 && p.cpg_shift == (WBITS == 8 ? 1 : 0)) : (p.s_rs == 1 || G == 1);
+        const bool rows_ok = WF == 2 ? (p.s_cs % 4 == 0 && (uintptr_t)p.scale % 4 == 0 && p.cpg_shift == 0) : (p.s_rs == 1 || G == 1);
         if (rows_ok && (lds_x > red ? lds_x : red) + (size_t)(16 * NB * WN) * GP * 4 <= 160 * 1024)
             return launch_rows_one<XDT, WBITS, MB, NB, WN, WK, HAS_OFF, WF, true, KSP>(p, st);
     }
@@ -1538,12 +1537,6 @@ int launch_wq_rows_float(const WqParams& p, hipStream_t st);
     int launch_wq_rows_float<XDT, WBITS>(const WqParams& p, hipStream_t st)                                         \
     {                                                                                                               \
         constexpr int WF = WBITS == 4 ? 2 : 1;                                                                      \
-        if constexpr (WBITS == 8) {   /* e4m3 codes with e8m0 scales per 32, up to 128 rows (no 64-column instance) */ \
-            if (p.scale_e8m0) {                                                                                     \
-                return p.m_rows > 64 ? launch_rows_one<XDT, WBITS, 8, 2, 4, 2, false, 2>(p, st)                     \
-                                     : launch_rows_one<XDT, WBITS, 4, 2, 4, 2, false, 2>(p, st);                    \
-            }                                                                                                       \
-        }                                                                                                           \
         if (p.m_rows > 192) return launch_rows_one<XDT, WBITS, 16, 2, 4, 2, false, WF>(p, st);                      \
         if (p.m_rows > 128) return launch_rows_one<XDT, WBITS, 12, 2, 4, 2, false, WF>(p, st);                      \
         if (p.cols64 && p.m_rows <= 64) return launch_rows_one<XDT, WBITS, 4, 2, 2, 4, false, WF>(p, st);           \

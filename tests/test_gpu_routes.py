@@ -86,3 +86,13 @@ def test_block_scales_are_cut_for_any_columns(gpu, M, K, N):
 def test_up_to_16_rows_of_fp8(gpu, mode, M, K, N, want):
     got = mx_route(gpu, M, K, N, False) if mode == "mx" else block_route(gpu, M, K, N)
     assert got[0] == want, got
+
+
+# from 65 rows: small products on the stream kernels, the others on the exact tiles, by measured shapes
+@pytest.mark.parametrize("mode,M,K,N,want", [
+    ("mx", 65, 2048, 2304, "fp8_wide fp8_stream"), ("mx", 128, 1664, 1472, "fp8_wide fp8_stream"), ("mx", 128, 13568, 4096, "fp8_exact"),
+    ("mx", 70, 13440, 4096, "fp8_exact"), ("mx", 64, 13440, 4096, "fp8_wide"), ("block", 100, 2048, 2304, "fp8_wide fp8_stream"),
+    ("block", 405, 1664, 3848, "fp8_wide"), ("block", 512, 4096, 8192, "fp8_exact"), ("mx", 300, 1280, 1152, "fp8_wide fp8_stream"), ("mx", 512, 8192, 4096, "fp8_exact")])
+def test_from_65_rows_of_fp8(gpu, mode, M, K, N, want):
+    got = mx_route(gpu, M, K, N, False) if mode == "mx" else block_route(gpu, M, K, N)
+    assert got[0] in want.split(), got
