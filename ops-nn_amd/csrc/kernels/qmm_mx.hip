@@ -316,9 +316,12 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
     OpsnnQmmArgs planned = a;
     if (relayout) mx_relayout_view(planned, R, (char*)(uintptr_t)256);
     MxPad L;
-    // few rows: the kernels that take a K tail as it is
+    // few rows: the kernels that take a K tail as it is.  With the 8-bit instruction asked for too, but for shapes whose 8-bit tiles fill half
+    // the CUs and are as fast with x2 from memory, faster from the last-level cache (51 x 3328 x 18624 29.0 and 21.0 us, stream 29.4 and 27.3;
+    // 56 x 2944 x 11264 24.7 and 17.9, 19.4 and 18.4; 64 x 5888 x 12288 49 and 35, 32 and 29)
+    const bool stream8 = exact || a.M <= 32 || (a.M <= 128 && (a.N <= 16384 || a.K % 128 != 0));
     Fp8StreamPlan spl;
-    const bool rows4 = fp4 && mxfp4_rows_wanted(a), rows8 = fp8 && exact && fp8_stream_plan(a, FP8X_MX, true, spl);
+    const bool rows4 = fp4 && mxfp4_rows_wanted(a), rows8 = fp8 && stream8 && fp8_stream_plan(a, FP8X_MX, true, spl);
     const bool pad = !rows4 && !rows8 && mx_pad_layout(planned, L);
     if (!pad && !rows4 && !rows8 && planned.K % 128 != 0) return OPSNN_NOT_TAKEN;
     if (planned.x2_scale_mat.col_stride != 2 || (fp4 || fp8 ? planned.x2_scale_mat.row_stride != (planned.K + 63) / 64 * 2 : planned.x2_scale_mat.row_stride % 4 != 0)) return OPSNN_NOT_TAKEN;

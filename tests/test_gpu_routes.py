@@ -96,3 +96,16 @@ def test_up_to_16_rows_of_fp8(gpu, mode, M, K, N, want):
 def test_from_65_rows_of_fp8(gpu, mode, M, K, N, want):
     got = mx_route(gpu, M, K, N, False) if mode == "mx" else block_route(gpu, M, K, N)
     assert got[0] in want.split(), got
+
+
+# with the 8-bit instruction asked for, MXFP8 with few rows keeps its kernels, also below 64 x 64 outputs
+@pytest.mark.parametrize("M,K,N", [(1, 2176, 256), (1, 3968, 3968), (1, 10624, 3968), (2, 2112, 1088), (16, 3200, 1920), (24, 1536, 512), (100, 1664, 1472)])
+def test_mxfp8_few_rows_with_the_8_bit_instruction(gpu, M, K, N):
+    m = gpu
+    print(f"case mxfp8 fast few rows M={M} K={K} N={N}", flush=True)
+    inp = cases.make_mx_inputs(m, M, K, N, M + N + K, True, False)
+    exact, exact_route = cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_FLOAT), route(m)
+    m.lib().opsnnSetFp8Fast(1)
+    fast, fast_route = cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_FLOAT), route(m)
+    assert fast_route == exact_route and exact_route[0].startswith("fp8_"), (exact_route, fast_route)
+    assert np.array_equal(fast, exact)
