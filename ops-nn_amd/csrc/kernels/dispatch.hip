@@ -34,6 +34,7 @@ bool wq_wide_wanted(const OpsnnWqmmArgs& a, uint64_t* workspace);   // wq_wide.h
 int launch_wq_wide(const OpsnnWqmmArgs& a, hipStream_t st);
 uint64_t mx_workspace_bytes(const OpsnnQmmArgs& a);
 bool mxfp4_rows_wanted(const OpsnnQmmArgs& a);   // qmm_mxfp4_rows.hip
+bool mxfp8_few_outputs(const OpsnnQmmArgs& a);   // qmm_mx.hip
 }  // namespace opsnn
 
 using namespace opsnn;
@@ -230,6 +231,7 @@ static int splitk_for(const OpsnnQmmArgs& a, int mode, bool stream = true)
     if (a.force_variant != 0 || opsnn_force_plain()) return 1;   // (a pinned kernel variant runs as it is)
     const bool out16 = a.out_dtype == DT_BF16 || a.out_dtype == DT_F16;
     const bool f8 = a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E4M3;
+    if (mode == 2 && mxfp8_few_outputs(a)) return 1;
     // few rows of fp8: the stream kernel's
     if (Fp8StreamPlan pl; stream && f8 && mode >= 1 && mode <= 3 && fp8_stream_plan(a, mode == 1 ? FP8X_BLOCK : mode == 2 ? FP8X_MX : FP8X_PLAIN, true, pl)) return pl.splits;
     // up to 16 rows of fp8 with block or MX scales, of int8 per-tile and of fp8 x fp4 MX: the decode kernels' K segments

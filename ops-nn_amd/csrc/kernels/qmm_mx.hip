@@ -233,6 +233,99 @@ static int mx_relayout_run(const OpsnnQmmArgs& a, const MxRelayout& R, char* w, 
     return (int)hipGetLastError();
 }
 
+// ---- MXFP8 with fewer than 64 x 64 outputs and a last half K tile ----
+// fp32 operands, x1 * 2^(a - 127) and x2 * 2^(b - 127) rounded nowhere down to scale byte 0, and fp32 sums, as on the plain kernel, which
+// took these calls before (3 x 15168 x 1088 12.4 ms on one thread per output); in bf16, as the matrix instructions would have them,
+// scale bytes 0 to 2 lose bits.  A workgroup per column of x2: its threads take pieces of 16 k in turns, multiply them with every row of x1,
+// and their sums meet in LDS.  Bound by vector instructions, some 40 a piece and row, against x2's bytes at few rows.
+template <int ROWS>
+__global__ __launch_bounds__(256) void mxfp8_few_outputs_kernel(OpsnnQmmArgs a)
+{
+    __shared__ float red[4][ROWS];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t n = blockIdx.x;
+    const uint8_t* w = (const uint8_t*)a.x2.ptr + n * a.x2.col_stride;
+    const uint8_t* ws = (const uint8_t*)a.x2_scale_mat.ptr + n * a.x2_scale_mat.row_stride;
+    float acc[ROWS];
+#pragma unroll
+    for (int m = 0; m < ROWS; m++) acc[m] = 0.0f;
+    auto widen = [](const uint4& v, float s, float (&o)[16]) {
+        const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8((int)d[i], false), hi = __builtin_amdgcn_cvt_pk_f32_fp8((int)d[i], true);
+            o[4 * i] = lo[0] * s; o[4 * i + 1] = lo[1] * s; o[4 * i + 2] = hi[0] * s; o[4 * i + 3] = hi[1] * s;
+        }
+    };
+    const uint8_t* const x = (const uint8_t*)a.x1.ptr;
+    const uint8_t* const xs = (const uint8_t*)a.x1_scale_mat.ptr;
+    struct Pieces { uint4 w, x[ROWS]; uint8_t ws, xs[ROWS]; };
+    auto fetch = [&](Pieces& f, int p) {
+        f.w = *(const uint4*)(w + 16 * p);
+        f.ws = ws[p >> 1];
+#pragma unroll
+        for (int m = 0; m < ROWS; m++) {
+            const int64_t r = m < a.M ? m : a.M - 1;   // (past the last row: that row again, not stored)
+            f.x[m] = *(const uint4*)(x + r * a.x1.row_stride + 16 * p);
+            f.xs[m] = xs[r * a.x1_scale_mat.row_stride + (p >> 1)];
+        }
+    };
+    auto multiply = [&](const Pieces& f) {
+        float wf[16];
+        widen(f.w, e8m0_to_f32(f.ws), wf);
+#pragma unroll
+        for (int m = 0; m < ROWS; m++) {
+            float xf[16];
+            widen(f.x[m], e8m0_to_f32(f.xs[m]), xf);
+#pragma unroll
+            for (int e = 0; e < 16; e++) acc[m] = __builtin_fmaf(xf[e], wf[e], acc[m]);
+        }
+    };
+    // (a turn's pieces are requested together, in front of the turn before's products: loaded row by row, 15 x 9152 x 272 took 37 us)
+    const int pieces = (int)(a.K / 16);
+    if (tid < pieces) {
+        Pieces now, next;
+        fetch(now, tid);
+        for (int p = tid; p < pieces; p += 256) {
+            fetch(next, p + 256 < pieces ? p + 256 : p);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(now);
+            now = next;
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < ROWS; m++) {
+        float v = acc[m];
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+        if (lane == 0) red[wave][m] = v;
+    }
+    __syncthreads();
+    if (tid < a.M) {
+        float v = ((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid];
+        if (a.bias) v = v + ((const float*)a.bias)[n];
+        store_f32_as(a.out, a.out_dtype, (int64_t)tid * a.N + n, v);
+    }
+}
+bool mxfp8_few_outputs(const OpsnnQmmArgs& a)
+{
+    return a.x1_dtype == DT_E4M3 && a.x2_dtype == DT_E4M3 && a.force_variant == 0 && a.batch == 1 && a.N >= 256 && a.M * a.N < 64 * 64 && a.K % 128 == 64;
+}
+// (`a` as mx_call_ok has passed it, x2 K-contiguous)
+static int launch_mxfp8_few_outputs(const OpsnnQmmArgs& a, hipStream_t st)
+{
+    if (((uintptr_t)a.x2.ptr | (uint64_t)a.x2.col_stride) % 16 || a.x2_scale_mat.col_stride != 2) return OPSNN_NOT_TAKEN;
+    note_route("mxfp8_few_outputs");
+    const dim3 grid((unsigned)a.N), block(256);
+    if (a.M == 1) hipLaunchKernelGGL(mxfp8_few_outputs_kernel<1>, grid, block, 0, st, a);
+    else if (a.M == 2) hipLaunchKernelGGL(mxfp8_few_outputs_kernel<2>, grid, block, 0, st, a);
+    else if (a.M == 3) hipLaunchKernelGGL(mxfp8_few_outputs_kernel<3>, grid, block, 0, st, a);
+    else if (a.M == 4) hipLaunchKernelGGL(mxfp8_few_outputs_kernel<4>, grid, block, 0, st, a);
+    else if (a.M <= 8) hipLaunchKernelGGL(mxfp8_few_outputs_kernel<8>, grid, block, 0, st, a);
+    else hipLaunchKernelGGL(mxfp8_few_outputs_kernel<16>, grid, block, 0, st, a);   // (fewer than 64 x 64 outputs and 256 columns: 15 rows at most)
+    return (int)hipGetLastError();
+}
+
 bool mxfp4_rows_wanted(const OpsnnQmmArgs& a);   // qmm_mxfp4_rows.hip
 int launch_mxfp4_rows(const OpsnnQmmArgs& a, hipStream_t st);
 int launch_fp8_stream(const OpsnnQmmArgs& a, Fp8xForm form, SplitK sk, hipStream_t st);   // qmm_fp8_stream.hip
@@ -321,9 +414,10 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
     // 56 x 2944 x 11264 24.7 and 17.9, 19.4 and 18.4; 64 x 5888 x 12288 49 and 35, 32 and 29)
     const bool stream8 = exact || a.M <= 32 || (a.M <= 128 && (a.N <= 16384 || a.K % 128 != 0));
     Fp8StreamPlan spl;
-    const bool rows4 = fp4 && mxfp4_rows_wanted(a), rows8 = fp8 && stream8 && fp8_stream_plan(a, FP8X_MX, true, spl);
+    const bool rows4 = fp4 && mxfp4_rows_wanted(a), few_outputs = mxfp8_few_outputs(a);
+    const bool rows8 = fp8 && !few_outputs && stream8 && fp8_stream_plan(a, FP8X_MX, true, spl);
     const bool pad = !rows4 && !rows8 && mx_pad_layout(planned, L);
-    if (!pad && !rows4 && !rows8 && planned.K % 128 != 0) return OPSNN_NOT_TAKEN;
+    if (!pad && !rows4 && !rows8 && !few_outputs && planned.K % 128 != 0) return OPSNN_NOT_TAKEN;
     if (planned.x2_scale_mat.col_stride != 2 || (fp4 || fp8 ? planned.x2_scale_mat.row_stride != (planned.K + 63) / 64 * 2 : planned.x2_scale_mat.row_stride % 4 != 0)) return OPSNN_NOT_TAKEN;
     if (pad && (!a.workspace || (uintptr_t)a.workspace % 16)) return OPSNN_NOT_TAKEN;
     if (relayout) {
@@ -346,6 +440,7 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         mx_relayout_view(a, R, w);
     }
     if (rows4) return launch_mxfp4_rows(a, st);
+    if (few_outputs) return launch_mxfp8_few_outputs(a, st);
     if (rows8) {
         const int rc = launch_fp8_stream(a, FP8X_MX, sk, st);
         if (rc != OPSNN_NOT_TAKEN || a.K % 128 != 0) return rc;   // (a K tail was left as it is)

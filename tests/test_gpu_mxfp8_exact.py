@@ -105,3 +105,32 @@ def test_mxfp8_single_products_over_the_e8m0_range(gpu, M, out, lo1, hi1, lo2, h
         assert np.array_equal(got[normal], want32[normal])
     else:
         assert np.array_equal(got[normal], orc.f32_to_b16(want32, m.ACL_BF16)[normal])
+
+
+# fewer than 64 x 64 outputs, K % 128 == 64: the operands stay in 32 bits, also where x1's scale bytes are 0 to 2 (2^-127 .. 2^-125), which
+# bf16 holds only in part.  fp32 sums of exact products in chains of at most K / 4096 + 8 steps of 16: within 2^-18 of the sum of magnitudes
+@pytest.mark.parametrize("M,K,N", [(1, 192, 256), (1, 2112, 4000), (2, 1088, 1500), (3, 704, 1300), (4, 64, 700), (7, 4160, 513), (8, 1984, 300), (15, 320, 257)])
+@pytest.mark.parametrize("tB", [True, False])
+def test_few_outputs_keep_32_bit_operands(gpu, M, K, N, tB):
+    m = gpu
+    m.lib().opsnnSetForcePlain(0)
+    print(f"case mxfp8 few outputs M={M} K={K} N={N} tB={tB}", flush=True)
+    inp = cases.make_mx_inputs(m, M, K, N, M + N + K, tB, False)
+    rng = np.random.default_rng(M)
+    inp["s1"] = rng.integers(0, 4, inp["s1"].shape).astype(np.uint8)
+    inp["s2"] = rng.integers(232, 238, inp["s2"].shape).astype(np.uint8)
+    bias = rng.normal(0, 2.0 ** -12, N).astype(np.float32) if M % 2 else None
+    c = np.arange(256)
+    e, f, s = (c >> 3) & 15, c & 7, np.where(c & 128, -1.0, 1.0)
+    code = np.where((e == 15) & (f == 7), np.nan, s * np.where(e == 0, f * 2.0 ** -9, (8 + f) * 2.0 ** (e - 10.0)))
+    s1 = np.exp2(inp["s1"][0].reshape(M, -1).astype(np.float64) - 127)
+    s2 = np.exp2((inp["s2"][0] if tB else np.moveaxis(inp["s2"][0], 1, 0)).reshape(N, -1).astype(np.float64) - 127)
+    a = code[inp["x1"][0]] * np.repeat(s1, 32, 1)[:, :K]
+    b = code[inp["x2"][0] if tB else inp["x2"][0].T] * np.repeat(s2, 32, 1)[:, :K]
+    want, terms = a @ b.T, np.abs(a) @ np.abs(b).T
+    if bias is not None:
+        want, terms = want + bias, terms + np.abs(bias)
+    got = cases.run_mx_aclnn(m, inp, M, K, N, tB, m.ACL_FLOAT, bias).reshape(M, N).astype(np.float64)
+    assert m.lib().opsnnDebugLastRoute(None) == b"mxfp8_few_outputs"
+    err = np.abs(got - want)
+    assert (err <= 2.0 ** -18 * terms).all(), f"worst error / sum of magnitudes {float((err / terms).max()):.3e}"
