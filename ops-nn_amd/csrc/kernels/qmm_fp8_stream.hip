@@ -722,7 +722,8 @@ bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8St
 int launch_fp8_stream(const OpsnnQmmArgs& a, Fp8xForm form, SplitK sk, hipStream_t st)
 {
     Fp8StreamPlan pl;
-    if (a.M > 128 && a.K % 128 == 0 && opsnnGetFp8Fast()) return OPSNN_NOT_TAKEN;   // (the caller asked for the 8-bit instruction)
+    // (the caller asked for the 8-bit instruction, which has no fp32 outputs but for MX)
+    if (a.M > 128 && a.K % 128 == 0 && (a.out_dtype != DT_F32 || form == FP8X_MX) && opsnnGetFp8Fast()) return OPSNN_NOT_TAKEN;
     if (!fp8_stream_plan(a, form, true, pl)) return OPSNN_NOT_TAKEN;
     // (no partial sums, or laid out for other segments: a call that another layout of its operands has changed on the way)
     if (pl.splits > 1 && (!sk.part || sk.splits < pl.splits) && !fp8_stream_plan(a, form, false, pl)) return OPSNN_NOT_TAKEN;

@@ -109,3 +109,15 @@ def test_mxfp8_few_rows_with_the_8_bit_instruction(gpu, M, K, N):
     fast, fast_route = cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_FLOAT), route(m)
     assert fast_route == exact_route and exact_route[0] in ("fp8_stream", "fp8_wide", "fp8_decode", "mxfp8_few_outputs"), (exact_route, fast_route)
     assert np.array_equal(fast, exact)
+
+
+# fp32 outputs have no 8-bit form: with the switch on they go where they go without it
+@pytest.mark.parametrize("M,K,N", [(200, 4096, 1024), (300, 3072, 771), (512, 8192, 4096)])
+def test_fp32_outputs_with_the_8_bit_instruction(gpu, M, K, N):
+    m = gpu
+    inp = cases.make_blockscale_inputs(m, M, K, N, M + N + K, True)
+    exact, exact_route = cases.run_blockscale_aclnn(m, inp, M, K, N, True, m.ACL_FLOAT), route(m)
+    m.lib().opsnnSetFp8Fast(1)
+    fast, fast_route = cases.run_blockscale_aclnn(m, inp, M, K, N, True, m.ACL_FLOAT), route(m)
+    assert fast_route == exact_route, (exact_route, fast_route)
+    assert np.array_equal(fast, exact)
