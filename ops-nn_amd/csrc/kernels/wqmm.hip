@@ -282,6 +282,7 @@ static int launch_decode(const WqParams& p, hipStream_t st)
         if (e != hipSuccess) return (int)e;
         device_flag_set(attr_set);
     }
+    note_route("wq_general");
     hipLaunchKernelGGL(k, dim3(grid), dim3(256), lds, st, p);
     return (int)hipGetLastError();
 }

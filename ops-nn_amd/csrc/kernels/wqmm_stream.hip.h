@@ -1308,6 +1308,7 @@ static int launch_resx_one(const WqParams& p, hipStream_t st)
         if (e != hipSuccess) return (int)e;
         device_flag_set(attr_set);
     }
+    note_route("wq_resx");
     hipLaunchKernelGGL(k, dim3(resx_grid((p.N + 15) / 16)), dim3(256), lds, st, p);
     return (int)hipGetLastError();
 }
@@ -1441,6 +1442,7 @@ static int launch_stream_one(const WqParams& p, hipStream_t st)
         if (e != hipSuccess) return (int)e;
         device_flag_set(attr_set);
     }
+    note_route("wq_stream");
     hipLaunchKernelGGL(k, dim3(grid), dim3(NW * 64), lds, st, p);
     return (int)hipGetLastError();
 }
@@ -1500,6 +1502,7 @@ static int launch_rows_one(const WqParams& p, hipStream_t st)
         if (e != hipSuccess) return (int)e;
         device_flag_set(attr_set);
     }
+    note_route("wq_rows", split ? (int)p.ksplit : 1);
     hipLaunchKernelGGL(k, dim3(grid, (unsigned)slabs, split ? (unsigned)p.ksplit : 1u), dim3(512), lds, st, p);
     if (hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
     if (split) {

@@ -345,6 +345,7 @@ static int launch_tile_bm(const WqParams& p, hipStream_t st)
             if (hipMalloc((void**)&d, n * sizeof(WqAudit)) != hipSuccess) return -100;
             WqParams q = p;
             q.m_base = (int64_t)(uintptr_t)d;
+            note_route("wq_tile");
             hipLaunchKernelGGL(kern, grid, dim3(512), lds, st, q);
             std::vector<WqAudit> h(n);
             if (hipStreamSynchronize(st) != hipSuccess || hipMemcpy(h.data(), d, n * sizeof(WqAudit), hipMemcpyDeviceToHost) != hipSuccess) return -101;
@@ -370,6 +371,7 @@ static int launch_tile_bm(const WqParams& p, hipStream_t st)
             return bad ? -102 : -103;   // either way the real kernel does not run in this build
         }
 #endif
+        note_route("wq_tile");
         hipLaunchKernelGGL(kern, grid, dim3(512), lds, st, p);
         return (int)hipGetLastError();
     };
