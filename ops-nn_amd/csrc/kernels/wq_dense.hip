@@ -199,13 +199,29 @@ static bool dense_is_faster(const OpsnnWqmmArgs& a, double product_us)
     const DenseEstimate e = dense_estimate(a, product_us);
     return e.here < 0.97 * e.other;   // (in doubt without the pass)
 }
-// What a K-contiguous call takes without the wide kernel (wq_wide.hip), from 33 rows: for its rule.
-double wq_many_rows_estimate(const OpsnnWqmmArgs& a)
+// What a call of 33 rows and more typically takes without the wide kernel (wq_wide.hip), for its rule: the many-rows kernel's estimate as
+// corrected by 396 calls (median error 3 to 4 %), the pass by 944 (5 %).
+static double rows_typical_us(const OpsnnWqmmArgs& a, const WqForm& f)
+{
+    static const double rate[2][2][2] = {{{1.19, 1.02}, {1.1, 1.1}}, {{1.025, 0.977}, {1.0, 1.035}}};               // [from 65 rows][8 bits][bf16]
+    static const double offs[2][2][2] = {{{0.03, 0.28}, {0.12, 0.11}}, {{0.02, 0.27}, {0.07, 0.1}}};
+    const int many = a.M > 64, w8 = f.wbits == 8, bf = a.x_dtype == DT_BF16;
+    return rows_kernel_us(a, f.wbits, f.group) * rate[many][w8][bf] * (a.offset ? 1.0 + offs[many][w8][bf] : 1.0) - (many ? 1.36 : 3.88) +
+           (many ? 0.18e-6 : 1.49e-6) * (double)a.M * (double)a.N;
+}
+double wq_many_rows_typical_us(const OpsnnWqmmArgs& a)
 {
     const WqForm f = wq_form(a);
-    if (a.M <= 64) return f.rows ? rows_kernel_us(a, f.wbits, f.group) : 1e30;
-    const DenseEstimate e = dense_estimate(a, dense_plan(a.M, a.N, a.K).us);
-    return a.K % 64 == 0 && a.N >= 128 && e.here < e.other ? e.here : e.other;
+    if (a.M <= 64) return f.rows && f.nk ? rows_typical_us(a, f) : 1e30;
+    const double product_us = dense_plan(a.M, a.N, a.K).us;
+    const DenseEstimate e = dense_estimate(a, product_us);
+    if (a.K % 64 == 0 && a.N >= 128 && e.here < 0.97 * e.other) {
+        static const double pass[2][2] = {{0.467, 0.49}, {0.427, 0.421}};   // [K-contiguous][8 bits]: us per 10^6 codes
+        const double codes = (double)a.N * (double)a.K * 1e-6;
+        return 7.85 + codes * pass[f.nk][f.wbits == 8] * (1.0 + 0.299 * (codes < 200.0 ? codes / 100.0 : 2.0)) + 0.766 * product_us +
+               0.682e-6 * (double)a.M * (double)a.N;
+    }
+    return f.rows && f.nk ? rows_typical_us(a, f) : e.other;
 }
 
 // Can the call run here?

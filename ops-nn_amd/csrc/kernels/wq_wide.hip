@@ -32,8 +32,11 @@
 extern "C" int opsnn_wq_tile_min();   // dispatch.hip
 extern "C" int opsnn_wq_narrow_slabs();
 namespace opsnn {
-double wq_nk_estimate(const OpsnnWqmmArgs& a);          // wq_nk.hip
-double wq_many_rows_estimate(const OpsnnWqmmArgs& a);   // wq_dense.hip
+bool wq_nk_wanted(const OpsnnWqmmArgs& a, uint64_t* workspace);   // wq_nk.hip
+double wq_nk_typical_us(const OpsnnWqmmArgs& a);
+bool wq_kn_wanted(const OpsnnWqmmArgs& a);   // wq_kn.hip
+double wq_kn_typical_us(const OpsnnWqmmArgs& a);
+double wq_many_rows_typical_us(const OpsnnWqmmArgs& a);   // wq_dense.hip
 bool weight_cache_on();                                 // weight_cache.hip
 const void* weight_cache_get(const void* src, int64_t K, int64_t N, int bits, int64_t nb, hipStream_t st);
 namespace {
@@ -397,7 +400,7 @@ int launch_mb(const WqParams& p, const WqWidePlan& pl, hipStream_t st)
     return launch_one<XDT, WBITS, 8, HAS_OFF, false>(p, pl, st);
 }
 
-// What a launch takes, in us, fitted to 1460 timed launches of 160 calls (M 1 .. 400, K 1024 .. 18432, N 1024 .. 28672; median error 5 %):
+// Which layout is best: what a launch takes, in us, the weight from memory, fitted to 1460 timed launches of 160 calls (M 1 .. 400, K 1024 .. 18432, N 1024 .. 28672; median error 5 %):
 // workgroups one a CU, in rounds, their K tiles by type and row blocks, the scale table, the weight's stream as the other bound, the
 // outputs, and the second kernel of a K split.
 float wide_us(const OpsnnWqmmArgs& a, int wbits, bool kn, int mb, int splits, int64_t groups)
@@ -434,14 +437,44 @@ bool wide_plan(const OpsnnWqmmArgs& a, const WqForm& f, WqWidePlan& pl)
     return pl.us < 1e30f;
 }
 
+// Whether a call runs here at all: what the chosen layout typically takes (median error 3 %; see wq_cost.h).
+double wide_typical_us(const OpsnnWqmmArgs& a, int wbits, const WqWidePlan& pl)
+{
+    static const double tile[2][2][2] = {{{0.343, 0.444}, {0.486, 0.82}}, {{0.407, 0.502}, {0.449, 0.802}}};   // [8 bits][bf16][offset]
+    const int64_t strips = (a.N + WW_COLS - 1) / WW_COLS, tiles = (a.K + WW_KT - 1) / WW_KT, slabs = (a.M + 16 * pl.mb - 1) / (16 * pl.mb);
+    const double t = tile[wbits == 8][a.x_dtype == DT_BF16][a.offset != nullptr] + 0.066 * pl.mb + (pl.kn ? 0.056 : 0.0), out_m = (double)a.M * (double)a.N * 1e-6;
+    const double cu = (double)((strips * slabs * pl.splits + 255) / 256) * ((double)((tiles + pl.splits - 1) / pl.splits) * t + 1.91 + 0.355 * pl.mb + 0.0143 * pl.groups);
+    return 2.39 + 1.33 * out_m + wq_typical_both(cu, wq_typical_mb(wbits, a.N, a.K) / 6.56) + (pl.splits > 1 ? 2.9 + 2.09 * pl.splits * out_m * (a.N % 4 ? 2.0 : 1.0) : 0.0);
+}
+// What the call typically takes on the kernel that it runs on otherwise.
+double others_typical_us(const OpsnnWqmmArgs& a, const WqForm& f)
+{
+    if (a.M > 64) return wq_many_rows_typical_us(a);
+    if (!f.nk) return wq_kn_wanted(a) ? wq_kn_typical_us(a) : 1e30;   // (else behind a re-layout)
+    if (a.M <= 16 && f.stream && a.K % 128 == 0) {
+        // up to 16 rows, whole chunks: x in registers, x whole in LDS, or the streaming kernel
+        WqXregPlan x;
+        const bool resx = a.K / (4 * (128 / f.wbits)) % 4 == 0 && (a.M + 1) * (a.K * 2 + 16) <= 65536;
+        if (wq_xreg_plan(f.wbits, a.M, a.K, x) && (a.M >= 4 || (x.splits > 1 && !resx))) return x.splits == 1 ? 0.0 : wq_xreg_typical_us(a, f, x);
+        return resx ? wq_resx_typical_us(a, f) : wq_stream_typical_us(a, f);
+    }
+    if (uint64_t bytes; wq_nk_wanted(a, &bytes)) return wq_nk_typical_us(a);
+    if (f.rows && (a.M > 32 || wq_part_slices(f.wbits, a.M, a.N, a.K, f.group, true) > 1)) return wq_many_rows_typical_us(a);
+    if (f.stream) return wq_stream_typical_us(a, f);
+    return wq_general_counts(a, f) ? wq_general_typical_us(a) : 1e30;
+}
+
 // Does the call run here?  Looks at what both phases know: not at the weight's address (launch_wq_wide declines an unaligned one).
 //
-// [K, N] storage in whole 16-byte pieces of a row: from 65 rows always (241 x 1024 x 1664 is the least: 13.3 us with the pass, 14.6 here),
-// from 17 unless the weight is small (wq_kn.hip: 32 x 2304 x 2176 10.5 and 11.9, 28 x 8832 x 4032 19.2 and 17.6), up to 16 unless it is
-// large and wide (3 x 17664 x 15040 53 and 67, 16 x 8192 x 28672 44 and 51; 10 x 15104 x 1472 24 and 18, 15 x 9984 x 7808 24 and 21).
-// [N, K] storage, up to 16 rows: from 8 MB, unless K is one whole shape of the x-in-registers kernel (16 x 8192 x 28672 36 there, 44
-// here; 15 x 8448 x 4288, which that kernel cuts, 44 and 20; 4 x 3072 x 3128 7.3 and 10.5).  More rows: where the estimates say so
-// (20 x 13568 x 8656 37 and 30, 24 x 1024 x 11016 7.0 and 8.9).  From 513 rows the dequantising pass is ahead of a fifth slab.
+// Where the two estimates above say so.  (Of 5380 calls timed on either side, the weight from memory and in the last-level cache, 3670 run here,
+// 103 of them 5 % slower or more than there, 36 by 10 %, the worst 1.4 times: 339 x 15872 x 12160 bf16 x int8 226 us, 162 on the many-rows kernel.
+// Before there were estimates for [K, N] storage and up to 16 rows, and with the other estimates fitted to the weight from memory, 297
+// were, 170 by 10 %: 491 x 8448 x 2112 [K, N] int8 48 us with the pass and 75 here, 27 x 17920 x 25376 [K, N] bf16 124 and 156, 3 x 1536 x 13184
+// bf16 10.7 and 13.6, 18 x 3328 x 1152 bf16 x int8 9.8 and 11.1.)  Below 2^20 codes nothing was timed; from 65 rows the pass
+// is ahead below 2^21 (189 x 1152 x 1088 12.1 there, 13.7 here).  Up to 16 rows, [K, N] storage: not
+// where the weight is large and wide, of 68 such calls 56 faster there (16 x 8192 x 28672 40.7 us, 47.9 here; 5 x 12288 x 27072 61 and 86); [N, K]
+// storage: from 8 MB, and not where K is one whole shape of the x-in-registers kernel (16 x 8192 x 28672 36 there, 44 here; 4 x 3072 x 3128 7.3 and
+// 10.5).  From 513 rows the dequantising pass is ahead of a fifth slab.
 bool wide_wanted(const OpsnnWqmmArgs& a, WqWidePlan& pl)
 {
     if ((a.w_dtype != DT_I4 && a.w_dtype != DT_I8) || (a.x_dtype != DT_F16 && a.x_dtype != DT_BF16)) return false;
@@ -453,22 +486,10 @@ bool wide_wanted(const OpsnnWqmmArgs& a, WqWidePlan& pl)
     pl.kn = !f.nk;
     if (pl.kn && (a.w.col_stride != 1 || a.w.row_stride != a.N || a.N % (128 / f.wbits) != 0)) return false;
     if (f.group < a.K && (f.group < 32 || (f.group & (f.group - 1)) != 0)) return false;
-    if (pl.kn) {
-        if (codes < (a.M > 64 ? 1ll << 21 : a.M > 16 ? 1ll << 23 : 1ll << 20) || (a.w_dtype == DT_I8 && a.M <= 16 && codes <= (1ll << 24))) return false;   // (as in wq_kn.hip)
-        if (a.M <= 16 && codes > (1ll << 26) && a.N > 6144) return false;
-        return wide_plan(a, f, pl);
-    }
-    if (a.M <= 16) {
-        if (codes * f.wbits < (1ll << 26)) return false;
-        if (WqXregPlan x; f.stream && wq_xreg_plan(f.wbits, a.M, a.K, x) && x.splits == 1) return false;
-        return wide_plan(a, f, pl);
-    }
-    if (!wide_plan(a, f, pl) || codes < (1ll << 21)) return false;
-    double other = wq_nk_estimate(a);
-    if (f.stream && a.M <= 64) { const double us = wq_stream_pass_us(f.wbits, a.x_dtype == DT_BF16, a.M, a.N, a.K); if (us < other) other = us; }
-    if (wq_general_counts(a, f) && a.M <= 64) { const double us = wq_general_pass_us(a.M, a.N, a.K); if (us < other) other = us; }
-    if (a.M > 32) { const double us = wq_many_rows_estimate(a); if (us < other) other = us; }
-    return pl.us < (f.wbits == 8 ? 1.07 : 0.97) * other;   // (8 bits: the others' estimates lie some 10 % low, 64 x 8192 x 28672 fp16 67 us for 57)
+    if (codes < (a.M > 64 ? 1ll << 21 : 1ll << 20)) return false;
+    if (pl.kn && a.w_dtype == DT_I8 && a.M <= 16 && codes <= (1ll << 24)) return false;   // (as in wq_kn.hip)
+    if (a.M <= 16 && (pl.kn ? codes > (1ll << 26) && a.N > 6144 : codes * f.wbits < (1ll << 26))) return false;
+    return wide_plan(a, f, pl) && wide_typical_us(a, f.wbits, pl) < others_typical_us(a, f);
 }
 }  // namespace
 

@@ -121,3 +121,18 @@ def test_fp32_outputs_with_the_8_bit_instruction(gpu, M, K, N):
     fast, fast_route = cases.run_blockscale_aclnn(m, inp, M, K, N, True, m.ACL_FLOAT), route(m)
     assert fast_route == exact_route, (exact_route, fast_route)
     assert np.array_equal(fast, exact)
+
+
+# weight-only: shapes that were timed on both sides, the weight from memory and in the last-level cache
+@pytest.mark.parametrize("M,K,N,group,w,x,nk,off,want", [
+    (491, 8448, 2112, 32, "i8", "f16", False, True, "wq_dense"), (27, 17920, 2112, 64, "i4", "bf16", False, False, "wq_wide"),
+    (30, 15360, 12288, 64, "i4", "bf16", False, True, "wq_kn"), (32, 2304, 2176, 128, "i4", "f16", False, True, "wq_kn"),
+    (110, 11008, 4096, 128, "i4", "f16", False, True, "wq_wide"), (9, 17280, 1888, 64, "i4", "f16", False, True, "wq_wide"),
+    (3, 1536, 13184, 0, "i4", "bf16", True, True, "wq_resx"), (9, 1536, 6144, 0, "i8", "f16", True, False, "wq_resx"),
+    (18, 3328, 1152, 0, "i8", "bf16", True, True, "wq_nk"), (57, 9856, 4352, 128, "i4", "f16", True, True, "wq_wide"),
+    (16, 8192, 28672, 128, "i4", "f16", False, True, "wq_kn_table"), (55, 2432, 1024, 128, "i4", "f16", True, False, "wq_nk"), (4, 3072, 3136, 128, "i4", "f16", True, False, "wq_resx")])
+def test_weight_only(gpu, M, K, N, group, w, x, nk, off, want):
+    m = gpu
+    xd = m.ACL_FLOAT16 if x == "f16" else m.ACL_BF16
+    cases.run_wq_aclnn(m, cases.make_wq_inputs(m, M, K, N, 1, xd, m.ACL_INT4 if w == "i4" else m.ACL_INT8, group, nk, off, None), M, K, N)
+    assert route(m)[0] == want, route(m)
