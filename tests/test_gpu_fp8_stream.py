@@ -5,6 +5,7 @@ import pytest
 import cases
 import oracle_api as orc
 from test_gpu_other_modes import check_close
+from test_gpu_routes import route
 
 pytestmark = pytest.mark.gpu
 
@@ -31,12 +32,17 @@ def test_block_scales(gpu, M, K, N, gsM, out):
     inp = cases.make_blockscale_inputs(m, M, K, N, M + N + K, True, gsM)
     want = cases.oracle_blockscale(m, inp, M, K, N, True, dt)
     got = cases.run_blockscale_aclnn(m, inp, M, K, N, True, dt)
+    assert route(m)[0] in STREAM, route(m)
     if out == "f32":
         assert np.isfinite(got).all()
         mx, mean = orc.rel_err_stats(got, want)
         assert mean <= 2.0 ** -16 and orc.isclose_fraction(got, want) == 0.0, f"max rel {mx:.3e} mean rel {mean:.3e}"
     else:
         check_close(got, want, orc.BF16, "fp8 stream, block scales")
+
+
+STREAM = ("fp8_stream", "fp8_wide")
+ELSEWHERE = {("mx", 5, 2048, 4361): "fp8_decode", ("mx", 3, 192, 256): "mxfp8_few_outputs", ("mx", 3, 2112, 1088): "mxfp8_few_outputs", ("mx", 2, 1088, 260): "mxfp8_few_outputs"}
 
 
 # (K % 128 == 64 as well: the narrow kernel, with four column blocks where N is wide)
@@ -79,6 +85,7 @@ def test_row_column_and_mx_scales(gpu, form, M, K, N):
     keep = m.quant_matmul_v5(m.Tensor((M, K), acl, d["x1"]), m.Tensor((N, K), acl, d["x2"]), m.Tensor(s1.shape, st, d["s1"]), m.Tensor(s2.shape, st, d["s2"]),
                              m.Tensor((M, N), m.ACL_FLOAT, d_out), **kw)
     m.check(m.lib().aclrtSynchronizeDevice(), "sync")
+    assert route(m)[0] in ([ELSEWHERE[form, M, K, N]] if (form, M, K, N) in ELSEWHERE else STREAM), route(m)
     raw = d_out.to_host(np.uint8, (M * N * 4 + 64,))
     assert (raw[M * N * 4:] == 0xEE).all(), "wrote past the output"
     got = raw[:M * N * 4].view(np.float32).reshape(M, N).astype(np.float64)
@@ -88,8 +95,9 @@ def test_row_column_and_mx_scales(gpu, form, M, K, N):
 
 
 # rows of x1 so far apart that the last ones lie 2^32 bytes and more behind the first: the stream kernels' lane offsets have 32 bits
-@pytest.mark.parametrize("M,K,N", [(300, 1024, 256), (300, 1088, 260)])
-def test_rows_far_apart(gpu, M, K, N):
+# (a K tail runs on padded copies, whose rows lie close together)
+@pytest.mark.parametrize("M,K,N,want", [(300, 1024, 256, "fp8_exact"), (300, 1088, 260, "fp8_stream")])
+def test_rows_far_apart(gpu, M, K, N, want):
     m = gpu
     stride = (1 << 24) - 128
     print(f"case fp8 stream rowcol, rows {stride} apart M={M} K={K} N={N}", flush=True)
@@ -105,6 +113,7 @@ def test_rows_far_apart(gpu, M, K, N):
     keep = m.quant_matmul_v5(m.Tensor((M, K), acl, d["x1"], strides=(stride, 1), storage_shape=((M - 1) * stride + K,)), m.Tensor((N, K), acl, d["x2"]),
                              m.Tensor((M,), m.ACL_FLOAT, d["s1"]), m.Tensor((N,), m.ACL_FLOAT, d["s2"]), m.Tensor((M, N), m.ACL_FLOAT, d_out), transpose_x2=True)
     m.check(m.lib().aclrtSynchronizeDevice(), "sync")
+    assert route(m)[0] == want, route(m)
     got = d_out.to_host(np.float32, (M, N)).astype(np.float64)
     code = _codes()
     a, b = code[x1] * s1[:, None].astype(np.float64), code[x2] * s2[:, None].astype(np.float64)

@@ -5,6 +5,7 @@ import pytest
 import cases
 import oracle_api as orc
 from test_gpu_other_modes import check_close
+from test_gpu_routes import route
 
 pytestmark = pytest.mark.gpu
 
@@ -39,6 +40,7 @@ def test_few_rows(gpu, M, K, N, tB, batch, out):
     bias = np.random.default_rng(1).normal(0, 1, N).astype(np.float32) if M % 2 == 0 else None
     want = cases.oracle_mx(m, inp, M, K, N, tB, dt, bias)
     got = cases.run_mx_aclnn(m, inp, M, K, N, tB, dt, bias)
+    assert route(m)[0] == "mxfp4_rows", route(m)
     if out == "f32":
         pos = dict(inp, x1=inp["x1"] & 0x77, x2=inp["x2"] & 0x77)
         abs_sum = cases.oracle_mx(m, pos, M, K, N, tB, dt).astype(np.float64) + (np.abs(bias) if bias is not None else 0.0)

@@ -6,6 +6,7 @@ import pytest
 import cases
 import oracle_api as orc
 from test_gpu_other_modes import check_close
+from test_gpu_routes import route
 
 pytestmark = pytest.mark.gpu
 
@@ -29,6 +30,7 @@ def test_k_tail_on_whole_tiles(gpu, K, tB):
     bias = np.random.default_rng(1).normal(0, 1, N).astype(np.float32)
     want = cases.oracle_mx(m, inp, M, K, N, tB, m.ACL_BF16, bias)
     got = cases.run_mx_aclnn(m, inp, M, K, N, tB, m.ACL_BF16, bias)
+    assert route(m) == ("mxfp4_tiles_256", 1), route(m)
     check_close(got, want, orc.BF16, "mxfp4 tail")
 
 
@@ -52,13 +54,19 @@ def test_segments_of_odd_tiles(gpu, M, K, N):
     m = gpu
     print(f"case mxfp4 segments M={M} K={K} N={N}", flush=True)
     inp = cases.make_mx_inputs(m, M, K, N, K + N, True, True)
-    check_close(cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_BF16, None), cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, None), orc.BF16, "mxfp4 in segments")
+    got = cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_BF16, None)
+    assert route(m)[1] > 1, route(m)
+    check_close(got, cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, None), orc.BF16, "mxfp4 in segments")
 
 
-def test_scale_rows_of_both_operands_beyond_the_grids_second_axis(gpu):
+# on small tiles the operands are copied as well; large ones copy the scale rows alone
+@pytest.mark.parametrize("M,K,N,want", [(260, 32, 262000, "mxfp4_tiles_128"), (512, 736, 262000, "mxfp4_tiles_256")])
+def test_scale_rows_of_both_operands_beyond_the_grids_second_axis(gpu, M, K, N, want):
     """M + N rows of scales are copied by one launch, four a workgroup: more workgroups than the second and third axis of a grid hold."""
     m = gpu
-    M, K, N = 260, 32, 262000
     print(f"case mxfp4 tail M={M} K={K} N={N}", flush=True)
     inp = cases.make_mx_inputs(m, M, K, N, 5, True, True)
-    check_close(cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_BF16, None), cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, None), orc.BF16, "mxfp4 tail, many scale rows")
+    got = cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_BF16, None)
+    assert route(m) == (want, 1), route(m)
+    rows = [0, 1, 130, 255, 256, M - 1]
+    check_close(np.ascontiguousarray(got[:, rows]), cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, rows=rows), orc.BF16, "mxfp4 tail, many scale rows")
