@@ -656,7 +656,7 @@ constexpr int narrow_per_cu(int mb, int nb)
 // out so by then.)
 //
 // Up to 64 rows.  Row / column scales always; block and MX scales with up to 16 rows where the x-in-registers kernel of qmm_fp8_decode.hip
-// is not ahead by the estimates above (x2 from memory, there and here: 16 x 7168 x 18432 29.9 and 32.8 us, MX 3 x 6272 x 19456 32.8 and 42,
+// is not ahead by the estimates above (x2 from memory, there and here: 16 x 7168 x 18432 37 and 35 us, MX 3 x 6272 x 19456 32.8 and 42,
 // 8 x 3200 x 1920 7.7 and 10.8; 8 x 9856 x 23040, which it cuts, 61 and 44).
 //
 // From 65 to 512 rows, in slabs of 64: products that leave most of the exact tiles without a CU's worth of work, by the estimates

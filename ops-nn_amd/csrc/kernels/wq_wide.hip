@@ -466,15 +466,16 @@ double others_typical_us(const OpsnnWqmmArgs& a, const WqForm& f)
 
 // Does the call run here?  Looks at what both phases know: not at the weight's address (launch_wq_wide declines an unaligned one).
 //
-// Where the two estimates above say so.  (Of 5380 calls timed on either side, the weight from memory and in the last-level cache, 3670 run here,
-// 103 of them 5 % slower or more than there, 36 by 10 %, the worst 1.4 times: 339 x 15872 x 12160 bf16 x int8 226 us, 162 on the many-rows kernel.
-// Before there were estimates for [K, N] storage and up to 16 rows, and with the other estimates fitted to the weight from memory, 297
-// were, 170 by 10 %: 491 x 8448 x 2112 [K, N] int8 48 us with the pass and 75 here, 27 x 17920 x 25376 [K, N] bf16 124 and 156, 3 x 1536 x 13184
-// bf16 10.7 and 13.6, 18 x 3328 x 1152 bf16 x int8 9.8 and 11.1.)  Below 2^20 codes nothing was timed; from 65 rows the pass
-// is ahead below 2^21 (189 x 1152 x 1088 12.1 there, 13.7 here).  Up to 16 rows, [K, N] storage: not
-// where the weight is large and wide, of 68 such calls 56 faster there (16 x 8192 x 28672 40.7 us, 47.9 here; 5 x 12288 x 27072 61 and 86); [N, K]
-// storage: from 8 MB, and not where K is one whole shape of the x-in-registers kernel (16 x 8192 x 28672 36 there, 44 here; 4 x 3072 x 3128 7.3 and
-// 10.5).  From 513 rows the dequantising pass is ahead of a fifth slab.
+// Where the two estimates above say so.  (Of 2989 calls beside the fitted ones, timed on either side with the weight from memory and in the
+// last-level cache, 1983 run here, 46 of them 5 % slower or more than there, 14 by 10 %, the worst 1.28 times; among the fitted ones the worst
+// is 1.4, 339 x 15872 x 12160 bf16 x int8 226 us, 162 on the many-rows kernel.  Before there were estimates for [K, N] storage and up to 16
+// rows, and with the other estimates fitted to the weight from memory, 153 were, 82 by 10 %: 491 x 8448 x 2112 [K, N] int8 48 us with the pass
+// and 75 here, 27 x 17920 x 25376 [K, N] bf16 124 and 156, 3 x 1536 x 13184 bf16 10.7 and 13.6, 18 x 3328 x 1152 bf16 x int8 9.8 and 11.1.)
+//
+// Below 2^20 codes nothing was timed; from 65 rows the pass is ahead below 2^21 (189 x 1152 x 1088 12.1 there, 13.7 here).  Up to 16 rows:
+// [K, N] storage not where the weight is large and wide, of 68 such calls 56 faster there (16 x 8192 x 28672 40.7 us, 47.9 here; 5 x 12288 x 27072 61
+// and 86); [N, K] storage from 8 MB, and not where K is one whole shape of the x-in-registers kernel (16 x 8192 x 28672 36 there, 44 here;
+// 4 x 3072 x 3128 7.3 and 10.5).  From 513 rows the dequantising pass is ahead of a fifth slab.
 bool wide_wanted(const OpsnnWqmmArgs& a, WqWidePlan& pl)
 {
     if ((a.w_dtype != DT_I4 && a.w_dtype != DT_I8) || (a.x_dtype != DT_F16 && a.x_dtype != DT_BF16)) return false;

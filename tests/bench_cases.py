@@ -35,9 +35,9 @@ PROFILED_TRAFFIC = {
     (8, None, None): (392.1e6, "profiles/block_quant_e4m3_128x128_18432x7168.txt"),
     (9, None, None): (674.5e6, "profiles/mx_quant_e2m1_32768x8192.txt"),
     (10, None, None): (290.3e6, "profiles/qmm_i4_kg_m4096_k4096_n4096.txt"),
-    (12, 16, "exact"): (136.9e6, "profiles/qmm_fp8_block_decode_m16_k7168_n18432.txt"),
+    (12, 16, "exact"): (133.8e6, "profiles/qmm_fp8_block_decode_m16_k7168_n18432.txt"),
     (12, 64, "exact"): (166.9e6, "profiles/qmm_fp8_block_rows_m64_k7168_n18432.txt"),
-    (12, 128, "exact"): (167.3e6, "profiles/qmm_fp8_block_rows_m128_k7168_n18432.txt"),
+    (12, 128, "exact"): (326.2e6, "profiles/qmm_fp8_block_rows_m128_k7168_n18432.txt"),
     (13, 16, None): (131.0e6, "profiles/qmm_mx_a8w4_decode_m16_k8192_n28672.txt"),
     (14, 16, None): (244.0e6, "profiles/qmm_i8_pertile_decode_m16_k8192_n28672.txt"),
     (11, 16, "warm"): (133.5e6, "profiles/wqmm_decode_mxfp4_m16_k8192_n28672.txt"),
@@ -213,7 +213,7 @@ class Config4Rows(Config4):
         M = args.m or 16
         super().__init__(m, args, M=M)
         self.instr_peak_key = None
-        self.kernel = "fp8_block_decode_kernel" if M <= 16 else "fp8_wide_kernel (+ fp8_stream_reduce_kernel where K is cut)" if M <= 128 else self.kernel
+        self.kernel = "fp8_wide_kernel (+ fp8_stream_reduce_kernel where K is cut), by estimate fp8_block_decode_kernel up to 16 rows" if M <= 128 else self.kernel
         self.config = dict(self.config, workload="aclnnQuantMatmulV5 fp8 e4m3 G-B (1x128 / 128x128 scales), bf16 out, decode rows")
 
 
@@ -327,7 +327,7 @@ class ConfigMxfp8Rows(Workload):
     bound = "hbm"
     peak_key = "fp8"
     dtype = "fp8_e4m3 x fp8_e4m3, both widened to bf16 with their e8m0 block scales (exact), fp32 sums"
-    kernel = "mx8_decode_kernel (v_mfma_f32_16x16x32_bf16); from 17 rows fp8_wide_kernel, from 65 wqmm_rows_kernel on e4m3 codes with e8m0 scales"
+    kernel = "mx8_decode_kernel (v_mfma_f32_16x16x32_bf16); from 17 rows fp8_wide_kernel, from 65 by estimate qmm_fp8_exact_kernel"
 
     def __init__(self, m, args, K=8192, N=28672):
         M = args.m or 16

@@ -21,9 +21,9 @@ WQ_CASES = [(8, 8192, 1024, True),     # x in registers, K split across workgrou
             (4, 2048, 4096, False),    # N-contiguous weight: re-laid out into the workspace first
             (200, 1024, 768, True)]    # row slabs in one launch
 FP8_CASES = [(16, 18432, 512, True),   # few rows: K in segments, partial sums, a kernel that adds them
-             (64, 18432, 1024, True),  # the many-rows kernel with K in segments
+             (64, 18432, 1024, True),  # the stream kernel with K in segments
              (300, 1024, 640, False)]  # tiles, N-contiguous x2 re-laid out into the workspace
-MX_CASES = [(64, 8192, 1024, False),   # MXFP8, 17 .. 256 rows: x1 widened into the workspace, the many-rows kernel
+MX_CASES = [(64, 8192, 1024, False),   # MXFP8, 17 .. 64 rows: the stream kernel
             (16, 8192, 512, False),    # MXFP8, few rows, K in segments
             (16, 8192, 512, True),     # MXFP4, few rows
             (300, 1024, 640, True)]    # MXFP4 tiles

@@ -125,22 +125,20 @@ def test_fp8_blockscale_fp32_output(gpu, M, K, N, tB, gsM, fast):
     # three of 8 x 6; 108: seven of 16 x 1; 19: three of 8 x 1; 148 in two passes: five of 16 x 2)
     (5, 3584, 264, 1, "f16"), (16, 11008, 512, 1, "bf16"), (16, 18432, 256, 1, "bf16"), (12, 13824, 384, 128, "f32"),
     (16, 2432, 256, 1, "f16"), (32, 18944, 264, 1, "bf16"), (4, 128, 256, 1, "bf16"), (16, 640, 272, 1, "f32"),
-    # 17 .. 32 rows where the many-rows kernel does not apply (N % 128, K % 512): two passes; one scale row for all of x1 (B-B)
+    # 17 .. 32 rows: the stream kernels; one scale row for all of x1 (B-B)
     (17, 2048, 520, 1, "bf16"), (32, 7168, 520, 128, "f16"), (24, 1024, 256, 1, "f32"), (20, 4096, 256, 1, "f32"),
-    # 17 .. 64 rows (N % 128 == 0, K % 512 == 0): x1 widened into the workspace, the many-rows streaming kernel
+    # 17 .. 64 rows, whole scale blocks of columns
     (33, 2048, 512, 1, "bf16"), (64, 8192, 1024, 1, "f16"), (50, 7168, 256, 128, "bf16"), (64, 512, 384, 1, "f32"),
     (40, 1536, 2304, 1, "bf16"),
-    # 65 .. 128 rows: the same kernel's 128-row instance
+    # 65 .. 128 rows: the stream kernels or the exact tiles
     (65, 2048, 512, 1, "bf16"), (128, 7168, 1024, 1, "f16"), (100, 1024, 256, 128, "f32"), (96, 16384, 256, 1, "bf16"),
-    # ... K in whole scale blocks but no whole rounds of the chunk pipeline; K segments against a narrow x2 (86 blocks in five,
-    # 148 in eight, 144 in four with two row slabs; 17 .. 32 rows as well)
+    # ... K in counts of blocks that no power of two divides, K segments against a narrow x2
     (40, 1664, 256, 1, "bf16"), (64, 11008, 512, 1, "f16"), (50, 18944, 256, 128, "bf16"), (128, 18432, 1024, 1, "f32"),
     (24, 13824, 384, 1, "bf16"),
 ])
 def test_fp8_blockscale_decode_rows(gpu, M, K, N, gsM, out):
-    """The block-scale modes with up to 32 rows of x1 (x2 K-contiguous): x1 stays in registers as exact fp16 and x2 is
-    streamed once per 16 rows; exact products, fp32 sums per block, one fused multiply-add per block (the exact tile
-    kernel's arithmetic, its bar)."""
+    """The block-scale modes with few rows of x1 (x2 K-contiguous), x2 streamed once: exact products, fp32 sums per block, one
+    fused multiply-add per block (the exact tile kernel's arithmetic, its bar)."""
     m = gpu
     dt = {"bf16": m.ACL_BF16, "f16": m.ACL_FLOAT16, "f32": m.ACL_FLOAT}[out]
     print(f"case fp8 block decode M={M} K={K} N={N} gsM={gsM} out={out}", flush=True)
@@ -295,8 +293,8 @@ def test_mxfp8_few_rows(gpu, M, K, N, exp_range, out):
     (130, 640, 16640, 4),       # (more than 128 rows per workgroup with a K that is no whole round of the 256-row instance: the tiles)
 ])
 def test_mxfp8_many_rows(gpu, M, K, N, exp_range):
-    """MXFP8 with 17 .. 256 rows: x1 widened to bf16 with its block scales into the workspace, then the many-rows streaming
-    kernel on e4m3 codes with e8m0 group scales (exact products, fp32 sums) -- the stated bar; the plain kernel bit-identical."""
+    """MXFP8 with 17 .. 256 rows, on the stream kernels or the exact tiles (exact products, fp32 sums) -- the stated bar; the plain
+    kernel bit-identical."""
     m = gpu
     print(f"case mxfp8 many rows M={M} K={K} N={N} exp_range={exp_range}", flush=True)
     inp = cases.make_mx_inputs(m, M, K, N, K + N + M, True, False, exp_range=exp_range)

@@ -247,16 +247,15 @@ def test_gpu_matches_oracle(gpu, M, K, N, in_dt, s_dt, s_len, bias_dt, out_dt, t
     (16, 11008, 256, "N", True, "f16", "M"),
     (9, 18432, 520, "N", False, "bf16", "M"),
     (16, 13824, 256, 1, True, "f16", True),
-    # 33 .. 64 rows (N % 32 == 0, K % 512 == 0): x1 widened into the workspace, the many-rows streaming kernel
+    # 33 .. 64 rows: the stream kernels
     (40, 2048, 512, "N", True, "bf16", "M"),
     (64, 7168, 288, "N", False, "f16", "M"),
     (33, 512, 256, 1, True, "f16", True),
-    # 65 .. 128 rows: the same kernel's 128-row instance
+    # 65 .. 128 rows: the stream kernels or the exact tiles
     (65, 1024, 288, "N", True, "bf16", "M"),
     (128, 3584, 512, "N", False, "f16", "M"),
     (100, 512, 256, 1, True, "bf16", True),
-    # ... K in whole 128-element blocks but no whole rounds of the chunk pipeline; K segments against a narrow x2 (86 blocks in
-    # five, 148 in eight, 144 in four with two row slabs, 108 at 17 .. 32 rows)
+    # ... K in counts of blocks that no power of two divides, K segments against a narrow x2
     (40, 1664, 256, "N", True, "bf16", "M"),
     (64, 11008, 512, "N", True, "f16", "M"),
     (50, 18944, 256, "N", False, "bf16", "M"),
