@@ -466,9 +466,9 @@ double others_typical_us(const OpsnnWqmmArgs& a, const WqForm& f)
 
 // Does the call run here?  Looks at what both phases know: not at the weight's address (launch_wq_wide declines an unaligned one).
 //
-// Where the two estimates above say so.  (Of 2989 calls beside the fitted ones, timed on either side with the weight from memory and in the
-// last-level cache, 1983 run here, 46 of them 5 % slower or more than there, 14 by 10 %, the worst 1.28 times; among the fitted ones the worst
-// is 1.4, 339 x 15872 x 12160 bf16 x int8 226 us, 162 on the many-rows kernel.  Before there were estimates for [K, N] storage and up to 16
+// Where the two estimates above say so.  (Of 2989 calls, 1797 of them drawn after the fit, timed on either side with the weight from memory and in
+// the last-level cache, 1983 run here, 46 of them 5 % slower or more than there, 14 by 10 %, the worst 1.28 times; among other fitted ones the
+// worst is 1.4, 339 x 15872 x 12160 bf16 x int8 226 us, 162 on the many-rows kernel.  Before there were estimates for [K, N] storage and up to 16
 // rows, and with the other estimates fitted to the weight from memory, 153 were, 82 by 10 %: 491 x 8448 x 2112 [K, N] int8 48 us with the pass
 // and 75 here, 27 x 17920 x 25376 [K, N] bf16 124 and 156, 3 x 1536 x 13184 bf16 10.7 and 13.6, 18 x 3328 x 1152 bf16 x int8 9.8 and 11.1.)
 //
