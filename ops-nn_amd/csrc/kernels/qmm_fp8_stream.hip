@@ -622,14 +622,16 @@ float stream_typical_us(const StreamTime& c, const Fp8StreamPlan& pl, int64_t wg
     const float both = pl.wide ? cbrtf(cu * cu * cu + hbm * hbm * hbm) : cu + hbm;
     return c.start + both + (pl.splits > 1 ? c.reduce + c.reduce_mb * (float)pl.splits * out_m : 0.0f);
 }
-// The x-in-registers kernel of qmm_fp8_decode.hip on the same terms (292 calls of up to 16 rows, median error 4 %): its workgroups take
-// blocks of 16 columns in turns; idle waves read what others read, which costs no bytes from memory.
-float decode_typical_us(const QmmDecodePlan& pl, bool mx, int64_t N, float x2_mb, float out_m)
+// The x-in-registers kernel of qmm_fp8_decode.hip on the same terms (900 calls of up to 16 rows, median error 3 %): its workgroups take
+// blocks of 16 columns in turns, behind the load of x1 into the waves' registers; idle waves read what others read, which costs no bytes
+// from memory.
+float decode_typical_us(const QmmDecodePlan& pl, bool mx, int64_t M, int64_t N, float x2_mb, float out_m)
 {
     const int64_t cus = 256 / pl.splits, rounds = ((N + 15) / 16 + cus - 1) / cus;
-    const float block = mx ? 0.685f : 0.81f, wide = pl.nw == 16 ? (mx ? 2.04f : 1.8f) : 1.0f;
-    const float cu = (float)rounds * ((float)pl.nblk * block * wide + (mx ? 0.435f : 0.28f)), hbm = x2_mb / (mx ? 10.6f : 12.0f);
-    return (mx ? 3.35f : 3.18f) + cbrtf(cu * cu * cu + hbm * hbm * hbm) + (pl.splits > 1 ? 1.9f + (mx ? 3.2f : 2.6f) * (float)pl.splits * out_m : 0.0f);
+    const float block = mx ? 0.602f : 0.659f, wide = pl.nw == 16 ? (mx ? 2.03f : 1.84f) : 1.0f;
+    const float cu = (float)rounds * ((float)pl.nblk * block * wide + (mx ? 0.511f : 0.41f)), hbm = x2_mb / (mx ? 6.43f : 6.85f);
+    return (mx ? 2.92f : 2.84f) + (mx ? 4.4e-3f : 2.6e-3f) * (float)(M * pl.nblk * pl.nw) + cbrtf(cu * cu * cu + hbm * hbm * hbm) +
+           (pl.splits > 1 ? (mx ? 2.06f : 2.17f) + (mx ? 1.53f : 1.76f) * (float)pl.splits * out_m : 0.0f);
 }
 // The exact tiles of qmm_fp8_exact.hip on the same terms: their plan's estimate with what it leaves out, and corrected where it is off
 // (524 calls of 65 .. 512 rows, median error 2 %).  K is cut there from 129 rows, MX from 65.
@@ -656,8 +658,8 @@ constexpr int narrow_per_cu(int mb, int nb)
 // out so by then.)
 //
 // Up to 64 rows.  Row / column scales always; block and MX scales with up to 16 rows where the x-in-registers kernel of qmm_fp8_decode.hip
-// is not ahead by the estimates above (x2 from memory, there and here: 16 x 7168 x 18432 37 and 35 us, MX 3 x 6272 x 19456 32.8 and 42,
-// 8 x 3200 x 1920 7.7 and 10.8; 8 x 9856 x 23040, which it cuts, 61 and 44).
+// is not ahead by the estimates above (x2 from memory, there and here: 16 x 7168 x 18432 37 and 35 us, MX 3 x 6272 x 19456 33 and 41,
+// 1 x 1792 x 8192 7.8 and 9.2, but 8 x 3200 x 1920 9.0 and 7.9; 8 x 9856 x 23040, which it cuts, 61 and 44).
 //
 // From 65 to 512 rows, in slabs of 64: products that leave most of the exact tiles without a CU's worth of work, by the estimates
 // (typical times there and here, MX 65 x 2048 x 2304 13.4 and 10.1 us, 128 x 1664 x 1472 15.2 and 8.9, 128 x 13568 x 8960 52 and 67,
@@ -714,7 +716,9 @@ bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8St
     if (whole && (a.M > 64 || (a.M <= 16 && form != FP8X_PLAIN))) {
         const float out = a.N % 4 ? 2.0f * out_m : out_m, here = stream_typical_us((pl.wide ? wide_time : narrow_time)[form], pl, wgs, k_tiles, slabs, cu_wgs, x2_mb, out);
         if (a.M > 64) return here <= tiles_typical_us(a.M, a.N, a.K, form, may_split);
-        if (QmmDecodePlan dp; qmm_decode_plan(a.K, may_split, dp) && decode_typical_us(dp, form == FP8X_MX, a.N, x2_mb, out) < here) return false;
+        // (1.04: this kernel's estimate is 2 to 10 % high up to 16 rows.  Of 700 calls drawn after the fit 33 are 5 % slower or more than on the other
+        // kernel, of 900 without x1's load and this factor 78.)
+        if (QmmDecodePlan dp; qmm_decode_plan(a.K, may_split, dp) && 1.04f * decode_typical_us(dp, form == FP8X_MX, a.M, a.N, x2_mb, out) < here) return false;
     }
     return true;
 }
