@@ -68,5 +68,6 @@ def test_scale_rows_of_both_operands_beyond_the_grids_second_axis(gpu, M, K, N, 
     inp = cases.make_mx_inputs(m, M, K, N, 5, True, True)
     got = cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_BF16, None)
     assert route(m) == (want, 1), route(m)
-    rows = [0, 1, 130, 255, 256, M - 1]
-    check_close(np.ascontiguousarray(got[:, rows]), cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, rows=rows), orc.BF16, "mxfp4 tail, many scale rows")
+    rows = None if K == 32 else [0, 1, 130, 255, 256, M - 1]   # (of the larger case some rows)
+    check_close(got if rows is None else np.ascontiguousarray(got[:, rows]), cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, rows=rows), orc.BF16,
+                "mxfp4 tail, many scale rows")
