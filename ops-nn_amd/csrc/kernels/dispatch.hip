@@ -241,9 +241,9 @@ static int splitk_for(const OpsnnQmmArgs& a, int mode, bool stream = true)
         QmmDecodePlan pl;
         return qmm_decode_plan(a.K, true, pl, a8w4) ? pl.splits : 1;
     }
-    // (fewer than 64 x 64 outputs are the plain kernels' -- except int8 with few outputs against a long K, qmm_int8.hip)
+    // (fewer than 64 x 64 outputs are the plain kernels' -- except int8 from 256 columns on, qmm_int8.hip)
     const bool tiny = a.M * a.N < 64 * 64;
-    if ((tiny && !(a.N >= 256 && a.M * a.N * a.K >= (1ll << 22))) || a.K < 1024) return 1;
+    if ((tiny && a.N < 256) || a.K < 1024) return 1;
     int64_t bm, bn = 256, kunit = 128;
     double tile_us;   // one K tile (kunit elements) of the kernel in question, measured on calls with few tiles
     double bytes_per_us = 5.0e6;   // what its partial sums' traffic was measured to cost (splitk_factor)

@@ -198,9 +198,11 @@ static int qmm_int8_impl(const OpsnnQmmArgs* a, void* stream, SplitK sk)
     bool b16 = (p.out_dt == DT_BF16 || p.out_dt == DT_F16) || int_out;
     int variant = a->force_variant;
     if (opsnn_force_plain()) variant = OPSNN_VARIANT_PLAIN;
-    // (fewer than 64 x 64 outputs stay on the plain kernel unless K is long: one row against 3584 x 18944 is no work for one
-    // thread per output -- 2.4 ms there, 20 us on a 128 x 128 tile with K split)
-    const bool enough = p.M * p.N >= 64 * 64 || (p.N >= 256 && p.M * p.N * p.K >= (1ll << 22));
+    // Fewer than 64 x 64 outputs: the plain kernel walks K in one thread per output, 125 ns an element whatever M and N; a tile takes
+    // the 8 us of a call's launch up to K = 1536 (a call of 1 to 15 rows and 256 to 4000 columns, plain and tile: K = 64 11 / 8.4 us,
+    // 128 19 / 8.2, 512 66 / 8.3, 1536 195 / 8.3; 1 x 18944 x 3584 2.4 ms / 20 us).  From K = 128, so that a [K, N] x2 pays for its
+    // re-layout too.
+    const bool enough = p.M * p.N >= 64 * 64 || (p.N >= 256 && p.K >= 128);
     bool want_fast = b16 && a_kmajor && variant != OPSNN_VARIANT_PLAIN && enough && (p.K % 16) == 0 &&
                      (p.a_rs % 16) == 0 && ((uintptr_t)p.a % 16) == 0 && (p.a_bs % 16) == 0;
     if (want_fast && !b_kmajor && p.b_cs == 1 && p.b_rs == p.N && (p.b_bs == 0 || p.b_bs == p.K * p.N)) {
@@ -251,6 +253,7 @@ static int qmm_int8_impl(const OpsnnQmmArgs* a, void* stream, SplitK sk)
             variant = pl.variant;
             splits = pl.splits <= sk.splits ? pl.splits : 1;
         }
+        note_route("int8_tiles", splits);
         if (splits > 1) {   // (integer partial sums: the same bits)
             g.splits = splits; g.part = (int32_t*)sk.part;
             switch (variant) {

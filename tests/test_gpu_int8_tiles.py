@@ -8,6 +8,7 @@ import pytest
 
 import cases
 import oracle_api as orc
+from test_gpu_routes import route
 
 pytestmark = pytest.mark.gpu
 
@@ -37,3 +38,14 @@ def test_planned_shapes_are_bit_identical(gpu, M, K, N):
     print(f"case int8 planned M={M} K={K} N={N}", flush=True)
     got, want, _ = cases.run_qmm_int8_case(m, orc, M, K, N, seed=M + N, out_dtype=m.ACL_BF16, bias_dtype=m.ACL_FLOAT if M % 2 else None, transpose_x2=True)
     assert np.array_equal(got, want)
+
+
+# fewer than 64 x 64 outputs: on the tiles from 256 columns and K = 128 on
+@pytest.mark.parametrize("transpose_x2", [True, False])
+@pytest.mark.parametrize("M,K,N,tiles", [(1, 128, 256, True), (1, 112, 256, False), (1, 1536, 255, False), (15, 144, 273, True), (1, 1024, 4095, True), (3, 1536, 1365, True), (1, 2048, 2040, True)])
+def test_few_outputs_are_bit_identical(gpu, M, K, N, tiles, transpose_x2):
+    m = gpu
+    print(f"case int8 few outputs M={M} K={K} N={N} transpose_x2={transpose_x2}", flush=True)
+    got, want, _ = cases.run_qmm_int8_case(m, orc, M, K, N, seed=M + N, out_dtype=m.ACL_BF16, bias_dtype=m.ACL_FLOAT if M % 2 else None, transpose_x2=transpose_x2)
+    assert np.array_equal(got, want)
+    assert route(m)[0] == ("int8_tiles" if tiles else "plain"), route(m)
