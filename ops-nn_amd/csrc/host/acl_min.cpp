@@ -68,7 +68,7 @@ const char* dtype_name(aclDataType d)
     }
 }
 
-std::string shape_str(const std::vector<int64_t>& s)
+std::string shape_str(const Dims& s)
 {
     std::string r = "[";
     for (size_t i = 0; i < s.size(); i++) { if (i) r += ","; r += std::to_string(s[i]); }

@@ -52,7 +52,7 @@ aclnnStatus aclnnDynamicBlockQuantGetWorkspaceSize(const aclTensor* x_, double m
     if (x.rank() != 2 && x.rank() != 3) INVALID("%s: x must have 2 or 3 dims, got %ld", kApi, (long)x.rank());
     if (y.shape != x.shape) INVALID("%s: yOut %s must have x's shape %s", kApi, shape_str(y.shape).c_str(), shape_str(x.shape).c_str());
     if (x.empty()) INVALID("%s: empty tensors are not supported", kApi);
-    std::vector<int64_t> want = x.shape;
+    Dims want = x.shape;
     want[want.size() - 2] = (x.dim(-2) + rowBlockSize - 1) / rowBlockSize;
     want[want.size() - 1] = (x.dim(-1) + colBlockSize - 1) / colBlockSize;
     if (sc.shape != want) INVALID("%s: scaleOut %s must be %s", kApi, shape_str(sc.shape).c_str(), shape_str(want).c_str());

@@ -58,7 +58,7 @@ aclnnStatus aclnnDynamicMxQuantGetWorkspaceSize(const aclTensor* x_, int64_t axi
     const int64_t ax = axis < 0 ? axis + x.rank() : axis;
     if (y.shape != x.shape) INVALID("%s: yOut %s must have x's shape %s", kApi, shape_str(y.shape).c_str(), shape_str(x.shape).c_str());
     if (fp4 && x.dim(-1) % 2 != 0) INVALID("%s: the last dim of x must be even for a FLOAT4 output, got %ld", kApi, (long)x.dim(-1));
-    std::vector<int64_t> want = x.shape;
+    Dims want = x.shape;
     want[(size_t)ax] = ((x.dim(ax) + blocksize - 1) / blocksize + 1) / 2;
     want.push_back(2);
     if (sc.shape != want) INVALID("%s: mxscaleOut %s must be %s", kApi, shape_str(sc.shape).c_str(), shape_str(want).c_str());

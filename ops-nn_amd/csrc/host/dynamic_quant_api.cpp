@@ -83,7 +83,7 @@ aclnnStatus get_workspace(const char* api, const aclTensor* x_, const aclTensor*
     if (pertensor) {
         if (sc.rank() != 1 || sc.dim(0) != 1) INVALID("%s: scaleOut must be [1] when quantMode is pertensor", api);
     } else if (perchannel) {
-        std::vector<int64_t> want(x.shape.begin(), x.shape.end() - 2);
+        Dims want(x.shape.begin(), x.shape.end() - 2);
         want.push_back(cols);
         if (sc.shape != want) INVALID("%s: scaleOut %s must be %s when quantMode is perchannel", api, shape_str(sc.shape).c_str(), shape_str(want).c_str());
     } else if (sc.rank() != x.rank() - 1 || !std::equal(sc.shape.begin(), sc.shape.end(), x.shape.begin()))

@@ -284,7 +284,7 @@ aclnnStatus check_dtype(const Ctx& c)
 }
 
 // ---- shape rules: quant_matmul_checker.cpp:453-1195 ----
-aclnnStatus check_shape(const Ctx& c, std::vector<int64_t>& batch)
+aclnnStatus check_shape(const Ctx& c, Dims& batch)
 {
     const uint64_t gk = (uint64_t)c.groupSize & kMask16, gn = ((uint64_t)c.groupSize >> 16) & kMask16, gm = ((uint64_t)c.groupSize >> 32) & kMask16;
     // scale ranks
@@ -612,7 +612,7 @@ extern "C" aclnnStatus aclnnQuantMatmulV5GetWorkspaceSize(const aclTensor* x1, c
         Ctx cc = c;
         cc.groupSize = gsReal;
         if ((rc = check_dtype(cc)) != ACLNN_SUCCESS) return rc;
-        std::vector<int64_t> batch;
+        Dims batch;
         if ((rc = check_shape(cc, batch)) != ACLNN_SUCCESS) return rc;
         if ((rc = check_format(cc)) != ACLNN_SUCCESS) return rc;
         if (cc.x1.empty() || cc.x2.empty()) INVALID("%s: x1 and x2 must not be empty", kApi);

@@ -1,5 +1,6 @@
 // Internal definitions behind the opaque aclTensor / aclOpExecutor handles.
 #pragma once
+#include <algorithm>
 #include <cstdarg>
 #include <cstdint>
 #include <string>
@@ -78,15 +79,61 @@ inline int dtype_bits(aclDataType d)
     }
 }
 const char* dtype_name(aclDataType d);
-std::string shape_str(const std::vector<int64_t>& s);
+
+// Extents or strides.  Up to eight of them lie in the object: phase 1 copies the views of up to ten tensors, and with a heap block for
+// every shape, stride and storage list those were a third of its time.
+class Dims {
+public:
+    Dims() = default;
+    Dims(const std::vector<int64_t>& v) { assign(v.data(), v.size()); }
+    Dims(const int64_t* first, const int64_t* last) { assign(first, (size_t)(last - first)); }
+    Dims(const Dims& o) { assign(o.data(), o.n_); }
+    Dims& operator=(const Dims& o)
+    {
+        if (this != &o) assign(o.data(), o.n_);
+        return *this;
+    }
+    size_t size() const { return n_; }
+    int64_t* data() { return n_ <= kHere ? here_ : more_.data(); }
+    const int64_t* data() const { return n_ <= kHere ? here_ : more_.data(); }
+    int64_t& operator[](size_t i) { return data()[i]; }
+    int64_t operator[](size_t i) const { return data()[i]; }
+    int64_t* begin() { return data(); }
+    int64_t* end() { return data() + n_; }
+    const int64_t* begin() const { return data(); }
+    const int64_t* end() const { return data() + n_; }
+    int64_t& back() { return data()[n_ - 1]; }
+    void clear() { n_ = 0; more_.clear(); }
+    void push_back(int64_t v)
+    {
+        if (n_ == kHere) more_.assign(here_, here_ + kHere);
+        if (n_ >= kHere) more_.push_back(v);
+        else here_[n_] = v;
+        n_++;
+    }
+    bool operator==(const Dims& o) const { return n_ == o.n_ && std::equal(begin(), end(), o.begin()); }
+    bool operator!=(const Dims& o) const { return !(*this == o); }
+private:
+    static constexpr size_t kHere = 8;
+    void assign(const int64_t* v, size_t n)
+    {
+        if (n <= kHere) std::copy(v, v + n, here_);
+        else more_.assign(v, v + n);
+        n_ = n;
+    }
+    int64_t here_[kHere];
+    size_t n_ = 0;
+    std::vector<int64_t> more_;   // all of them, where they are more (a wanted shape can have a dim more than a tensor)
+};
+std::string shape_str(const Dims& s);
 
 // A lightweight copy of a tensor's view that the checks may rewrite (swap dims, re-tag dtype).
 struct TView {
-    std::vector<int64_t> shape, strides;
+    Dims shape, strides;
     int64_t offset = 0;
     aclDataType dtype = ACL_DT_UNDEFINED;
     aclFormat format = ACL_FORMAT_ND;
-    std::vector<int64_t> storage;
+    Dims storage;
     void* data = nullptr;
     bool present = false;
     int64_t rank() const { return (int64_t)shape.size(); }

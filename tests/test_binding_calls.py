@@ -1,0 +1,100 @@
+"""The binding's extension (csrc/python/calls.cpp) against the same entry points called through ctypes: statuses, workspace sizes and
+whether an executor comes back, for calls that are accepted and for calls that are refused; and views of up to eight dims."""
+import ctypes as C
+
+import pytest
+
+import opsnn as m
+
+PTR = 1 << 20
+
+
+def _ctypes(name, *args):
+    fn = C.CDLL(m.LIB_PATH)[name]   # (a function object of its own)
+    fn.restype, fn.argtypes = m.binding._SIGS[name]
+    ws, ex = C.c_uint64(0), C.c_void_p()
+    rc = fn(*args, C.byref(ws), C.byref(ex))
+    return rc, ws.value, ex.value
+
+
+def _same(got, want):
+    for ex in (got[2], want[2]):
+        if ex:
+            m.check(m.lib().aclDestroyAclOpExecutor(ex))
+    assert got[:2] == want[:2] and (got[2] is None) == (want[2] is None), (got, want, m.err_msg())
+
+
+def _t(shape, dtype, **kw):
+    return m.Tensor(shape, dtype, PTR, **kw)
+
+
+def _h(t):
+    return t.handle if t is not None else None
+
+
+@pytest.mark.parametrize("M,K,N,wrong", [(8, 4096, 4096, None), (300, 2048, 1536, None), (8, 4096, 4096, "scale"), (8, 4096, 4096, "out"), (0, 4096, 64, None)])
+def test_quant_matmul_v5(M, K, N, wrong):
+    x1, x2 = _t((M, K), m.ACL_INT8), _t((N, K), m.ACL_INT8)
+    s1, s2 = _t((M,), m.ACL_FLOAT), _t((N + (wrong == "scale"),), m.ACL_FLOAT)
+    bias, y = _t((N,), m.ACL_BF16), (None if wrong == "out" else _t((M, N), m.ACL_BF16))
+    for b in (None, bias):
+        _same(m.quant_matmul_v5_get_workspace(x1, x2, s1, s2, y, bias=b, transpose_x2=True),
+              _ctypes("aclnnQuantMatmulV5GetWorkspaceSize", x1.handle, x2.handle, s1.handle, s2.handle, None, None, None, None, _h(b), False, True, 0, _h(y)))
+    assert m.quant_matmul_v5_get_workspace(x1, x2, s1, s2, y, transpose_x2=True, ws_ptr=False)[0] != 0
+    assert m.quant_matmul_v5_get_workspace(x1, x2, s1, s2, y, transpose_x2=True, ex_ptr=False)[0] != 0
+
+
+@pytest.mark.parametrize("group,off", [(128, True), (64, False), (0, False), (33, False)])
+def test_weight_quant(group, off):
+    M, K, N = 16, 4096, 1024
+    G = max(1, -(-K // group) if group else 1)
+    x, w, y = _t((M, K), m.ACL_FLOAT16), _t((K, N), m.ACL_INT4), _t((M, N), m.ACL_FLOAT16)
+    s = _t((G, N), m.ACL_FLOAT16)
+    o = _t((G, N), m.ACL_FLOAT16) if off else None
+    _same(m.weight_quant_batch_matmul_get_workspace(x, w, s, y, offset=o, group_size=group),
+          _ctypes("aclnnWeightQuantBatchMatmulV2GetWorkspaceSize", x.handle, w.handle, s.handle, _h(o), None, None, None, group, y.handle))
+
+
+@pytest.mark.parametrize("rows", [0, 5, 300])
+def test_quantizers(rows):
+    K = 2048
+    x, q8, s = _t((rows, K), m.ACL_BF16), _t((rows, K), m.ACL_INT8), _t((rows,), m.ACL_FLOAT)
+    f8, sb, sm = _t((rows, K), m.ACL_FLOAT8_E4M3FN), _t((rows, K // 128), m.ACL_FLOAT), _t((rows, K // 64, 2), m.ACL_FLOAT8_E8M0)
+    _same(m.dynamic_quant_get_workspace(x, q8, s), _ctypes("aclnnDynamicQuantGetWorkspaceSize", x.handle, None, q8.handle, s.handle))
+    _same(m.dynamic_quant_get_workspace(x, q8, sb), _ctypes("aclnnDynamicQuantGetWorkspaceSize", x.handle, None, q8.handle, sb.handle))
+    for mode in (b"rint", b"no such", None, C.c_char_p(b"rint")):
+        _same(m.dynamic_block_quant_get_workspace(x, f8, sb, round_mode=mode),
+              _ctypes("aclnnDynamicBlockQuantGetWorkspaceSize", x.handle, 0.0, mode, m.ACL_FLOAT8_E4M3FN, 1, 128, f8.handle, sb.handle))
+        _same(m.dynamic_mx_quant_get_workspace(x, f8, sm, round_mode=mode),
+              _ctypes("aclnnDynamicMxQuantGetWorkspaceSize", x.handle, -1, mode, m.ACL_FLOAT8_E4M3FN, 32, 0, f8.handle, sm.handle))
+
+
+def test_phase_2_refuses_as_through_ctypes():
+    lib = m.lib()
+    for name in ("aclnnQuantMatmulV5", "aclnnWeightQuantBatchMatmulV2", "aclnnDynamicQuant", "aclnnDynamicBlockQuant", "aclnnDynamicMxQuant"):
+        fn = C.CDLL(m.LIB_PATH)[name]
+        fn.restype, fn.argtypes = m.binding._SIGS[name]
+        assert getattr(lib, name)(None, 0, None, None) == fn(None, 0, None, None) != 0
+        assert getattr(lib, name)(None, 0, 4096, None) == fn(None, 0, 4096, None) != 0       # no live executor
+        some = (C.c_char * 16)()
+        for args in ((C.c_void_p(), C.c_uint64(0), C.c_void_p(4096), None), (some, 16, 4096, C.c_void_p(64)), (C.byref(some), 2 ** 64 - 1, some, None)):
+            assert getattr(lib, name)(*args) == fn(*args) != 0
+        with pytest.raises((TypeError, C.ArgumentError)):
+            getattr(lib, name)(None, 0, None)
+        with pytest.raises((TypeError, C.ArgumentError)):
+            getattr(lib, name)(None, 0.5, None, None)
+
+
+@pytest.mark.parametrize("rank", [2, 3, 7, 8])
+def test_an_extent_in_any_place_is_seen(rank):
+    shape = [2] * (rank - 2) + [3, 64]
+    x, y, s = _t(shape, m.ACL_BF16), _t(shape, m.ACL_INT8), _t(shape[:-1], m.ACL_FLOAT)
+    rc, ws, ex = m.dynamic_quant_get_workspace(x, y, s)
+    assert rc == 0, m.err_msg()
+    m.check(m.lib().aclDestroyAclOpExecutor(ex))
+    for at in range(rank):
+        other = list(shape)
+        other[at] += 1
+        assert m.dynamic_quant_get_workspace(x, _t(other, m.ACL_INT8), s)[0] != 0, at
+        if at < rank - 1:
+            assert m.dynamic_quant_get_workspace(x, y, _t(other[:-1], m.ACL_FLOAT))[0] != 0, at
