@@ -7,24 +7,27 @@
 // in K tiles of 128 for 128 columns and 16 MB rows, through a ring of as many stages as the LDS holds, one barrier a tile, and every
 // weight is dequantised once per 16 MB rows, in registers.
 //
-// Eight waves: two halves of the columns times four steps of 32 k.  A wave multiplies 64 columns (four blocks of 16) by all rows, so
-// that a fragment of x serves four column blocks; the four sums over k meet in LDS at the end, in order.  blockIdx.y cuts K further
-// (fp32 partial sums, added in order by wq_splitk_reduce_kernel), blockIdx.z takes further slabs of 16 MB rows.  The scales of the
-// workgroup's columns lie in LDS as a table, laid down once: a compiler's load in the loop would be waited for with every copy under
-// way.
+// Eight waves: two halves of the columns times four steps of 32 k.  A wave multiplies 64 columns by all rows with 32 x 32 x 16 products,
+// each fragment of x for both column blocks; the sums over k meet in LDS at the end, in order.  (One row block: four quarters of the
+// columns times two steps of 64 k, 16 x 16 x 32 products.)  blockIdx.y cuts K further (fp32 partial sums, added in order by
+// wq_splitk_reduce_kernel), blockIdx.z takes further slabs of 16 MB rows.  The scales of the workgroup's columns lie in LDS as a table,
+// laid down once: a compiler's load in the loop would be waited for with every copy under way.
 //
-// What bounds it now is the issue of vector instructions: dequantising takes some 20 per 8 weights of a lane, two of which a matrix
-// instruction hides (mfma_16x16x32 7.2 ns with none or two of them behind it, 18 with eight).  [K, N] storage: two rows of k of one
-// column share a dword once their 16-bit pieces are joined, so the splice delivers pairs in k order and x needs no permutation;
-// [N, K] storage permutes x.
+// What bounds it is the issue of vector instructions, from 33 rows against a wide N also the power: 64 x 8192 x 28672 fp16 runs at 1.96 GHz
+// (2.38 with x zero).  Two waves a SIMD issue a packed fp16 operation, permute, shift or conversion in 2.15 ns and an fp32 or bit operation
+// in 1.75; a 16 x 16 x 32 product stands in their way for 4 ns, a 32 x 32 x 16 one, twice the work, for as long.  So: the large products;
+// operands in k order, so that x needs no permutation (three operations more for eight codes of fp16 x int4, four fewer for a fragment of
+// x); [K, N] storage through the LDS reads that transpose, which deliver what the [N, K] form reads, where pairs of rows were
+// spliced before; bf16 x int4 without offsets through a conversion that takes two codes at a time.  Sixteen waves a workgroup, copies from
+// waves of their own, and reads and copies spread between the products changed nothing (57.6, 57.5, 58.6 us for 57.8, 64 x 8192 x 28672).
 //
 // LDS rows, conflict-free for the reads below: x 256 bytes, 16-byte chunk c of row r at c ^ (r % 16); [N, K] weights 64 bytes (4 bits),
-// c ^ (r / 4 % 4), or 128, c ^ (r / 2 % 8); [K, N] weights 64 bytes, row k at slot k ^ (k / 8 % 4), or 128, slot k ^ (k / 8 % 2) with
-// the halves swapped where k / 16 is odd.
+// c ^ (r / 4 % 4), or 128, c ^ (r / 2 % 8); [K, N] weights, a row of k each, 64 bytes, c ^ (k / 4 % 4), or 128, c ^ 2 (k / 2 % 4).
 //
-// Measured, the weight from memory, a call before and now: [K, N] int4, 110 x 11008 x 24768 fp16 346 -> 126 us, 73 x 6656 x 2752 34.9 -> 19.0,
-// 200-row slabs 195 x 7296 x 15680 154 -> 83, int8 67 x 3840 x 12864 65 -> 30; [N, K] int4 57 x 9856 x 24349 98 -> 63, 37 x 7936 x 8576 bf16 69 -> 33,
-// int8 118 x 14336 x 8512 bf16 135 -> 58; 341 drawn calls of 1 .. 600 rows 1.21 times as fast.
+// Measured, before these products and reads and with them, the weight in turn from three buffers: 121 drawn calls of 1 .. 512 rows 1.058 times as
+// fast, none slower by more than 2 %; bf16 x int4 499 x 13632 x 3052 77 -> 64 us, 129 x 14912 x 3328 41 -> 35; fp16 64 x 16384 x 5120 91 -> 81
+// (the kernel alone), [K, N] bf16 4 x 2240 x 4224 10.4 -> 8.9.  Against the kernels before this one: [K, N] int4, 110 x 11008 x 24768 fp16 346 ->
+// 126 us, 73 x 6656 x 2752 34.9 -> 19.0, int8 67 x 3840 x 12864 65 -> 30; [N, K] int4 57 x 9856 x 24349 98 -> 63, int8 118 x 14336 x 8512 bf16 135 -> 58.
 #include "launch.h"
 #include "wq_cost.h"
 #include "wqmm_stream.hip.h"
@@ -43,46 +46,80 @@ namespace {
 
 constexpr int WW_COLS = 128, WW_KT = 128;   // columns of a workgroup, k of a tile
 
-// [K, N] storage: two rows of k of column j -> a pair of values of x's type.  4 bits: w0 holds four columns of both rows; 8 bits: of one
-// row each.  The arithmetic and its roundings are dequant8's.
-template <int XDT, int WBITS, bool HAS_OFF>
-__device__ __forceinline__ int kn_pair(uint32_t w0, uint32_t w1, int j, uint32_t so, const DqConst& dc)
+// 8 codes of consecutive k (4 bits: one dword, 8 bits: two) -> an operand of the matrix instructions, in k order.  The arithmetic and its
+// two roundings are those of dequant8 in wqmm_stream.hip.h.
+struct WwConst {
+    uint32_t mask, flip;   // fp16, 4 bits: the low nibble of the low half, the high one of the high half; their sign bits under the exponent of 1024.0
+    h2 unit, base;
+};
+__device__ __forceinline__ WwConst ww_const()
 {
+    WwConst c = {0x00f0000fu, 0x64806408u, {(_Float16)1.0f, (_Float16)0.0625f}, {(_Float16)-1032.0f, (_Float16)-72.0f}};
+    asm volatile("" : "+v"(c.mask), "+v"(c.flip), "+v"(c.unit), "+v"(c.base));   // (registers: the three-operand forms take no literals)
+    return c;
+}
+// E4M3 (bf16, 4 bits, no offset): by way of e4m3 codes, for scales below 2^125
+template <int XDT, int WBITS, bool HAS_OFF, bool E4M3>
+__device__ __forceinline__ v4i ww_dequant(const uint32_t* w, uint32_t so, const WwConst& dc)
+{
+    v4i r;
     if constexpr (XDT == DT_F16) {
         const _Float16 sh = __builtin_bit_cast(_Float16, (uint16_t)so), oh = __builtin_bit_cast(_Float16, (uint16_t)(so >> 16));
-        h2 t;
-        if constexpr (WBITS == 4) {
-            const uint32_t q = j >= 2 ? w0 >> 8 : w0;
-            const h2 c1032 = {(_Float16)-1032.0f, (_Float16)-1032.0f}, c72 = {(_Float16)-72.0f, (_Float16)-72.0f}, r16 = {(_Float16)0.0625f, (_Float16)0.0625f};
-            if (j & 1) t = __builtin_elementwise_fma(__builtin_bit_cast(h2, (q & dc.mhi) ^ dc.chi), r16, c72);
-            else t = __builtin_bit_cast(h2, (q & dc.mlo) ^ dc.clo) + c1032;
-        } else {
-            const h2 c1152 = {(_Float16)-1152.0f, (_Float16)-1152.0f};
-            t = __builtin_bit_cast(h2, __builtin_amdgcn_perm(w1, w0, 0x0c000c00u | (uint32_t)j | (uint32_t)(4 + j) << 16) ^ 0x64806480u) + c1152;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            h2 t;
+            if constexpr (WBITS == 4) {   // byte i in both halves: 1024 + (w + 8) of its low nibble, 1024 + 16 (w + 8) of its high one
+                const uint32_t b = __builtin_amdgcn_perm(w[0], w[0], 0x0c000c00u | (uint32_t)i | (uint32_t)i << 16);
+                t = __builtin_elementwise_fma(__builtin_bit_cast(h2, (b & dc.mask) ^ dc.flip), dc.unit, dc.base);   // exact
+            } else {
+                const h2 c1152 = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+                t = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, w[i >> 1] ^ 0x80808080u, i & 1 ? 0x04030402u : 0x04010400u)) + c1152;
+            }
+            if constexpr (HAS_OFF) t = t + (h2){oh, oh};
+            r[i] = (int)u32(t * (h2){sh, sh});
         }
-        if constexpr (HAS_OFF) t = t + (h2){oh, oh};
-        return (int)u32(t * (h2){sh, sh});
     } else {
         const float sc = bf16_to_f32((uint16_t)so), off = bf16_to_f32((uint16_t)(so >> 16));
-        float a, b;
-        if constexpr (WBITS == 4) {   // (16 times the weight, see dequant8)
-            const uint32_t n = j & 1 ? w0 & 0xf0f0f0f0u : (w0 << 4) & 0xf0f0f0f0u;
-            a = (float)((int)(n << (24 - 8 * (j >> 1))) >> 24);
-            b = (float)((int)(n << (8 - 8 * (j >> 1))) >> 24);
+        float v[8];
+        if constexpr (E4M3) {
+            // w + 8 in a byte reads as the e4m3 value 2^-9 (w + 8): two conversions at a time, and the fma's (w + 8) s - 8 s is w s
+            const uint32_t lo = (w[0] & 0x0f0f0f0fu) ^ 0x08080808u, hi = ((w[0] >> 4) & 0x0f0f0f0fu) ^ 0x08080808u;
+            const v2f l0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.0f, false), l1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(lo, 512.0f, true);
+            const v2f h0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.0f, false), h1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hi, 512.0f, true);
+            const float s8 = -8.0f * sc;
+            v[0] = __builtin_fmaf(l0[0], sc, s8); v[1] = __builtin_fmaf(h0[0], sc, s8); v[2] = __builtin_fmaf(l0[1], sc, s8); v[3] = __builtin_fmaf(h0[1], sc, s8);
+            v[4] = __builtin_fmaf(l1[0], sc, s8); v[5] = __builtin_fmaf(h1[0], sc, s8); v[6] = __builtin_fmaf(l1[1], sc, s8); v[7] = __builtin_fmaf(h1[1], sc, s8);
         } else {
-            a = (float)((int)(w0 << (24 - 8 * j)) >> 24);
-            b = (float)((int)(w1 << (24 - 8 * j)) >> 24);
+            // (4 bits: a nibble at the top of its byte, 16 times the weight, converts as it lies)
+            const uint32_t odd = w[0] & 0xf0f0f0f0u, even = (w[0] << 4) & 0xf0f0f0f0u;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float c = WBITS == 4 ? (float)((int)((i & 1 ? odd : even) << (24 - 8 * (i >> 1))) >> 24) : (float)((int)(w[i >> 2] << (24 - 8 * (i & 3))) >> 24);
+                v[i] = HAS_OFF ? __builtin_fmaf(c, WBITS == 4 ? 0.0625f : 1.0f, off) : c;
+            }
+            if constexpr (HAS_OFF) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const uint32_t pk = pack2_bf16((v2f){v[2 * i], v[2 * i + 1]});
+                    v[2 * i] = u2f(pk << 16);
+                    v[2 * i + 1] = u2f(pk & 0xffff0000u);
+                }
+            }
+            const float unit = WBITS == 4 && !HAS_OFF ? 0.0625f * sc : sc;
+#pragma unroll
+            for (int i = 0; i < 8; i++) v[i] = v[i] * unit;
         }
-        float s = sc;
-        if constexpr (HAS_OFF) {
-            const float one = WBITS == 4 ? 0.0625f : 1.0f;
-            const uint32_t pk = pack2_bf16((v2f){__builtin_fmaf(a, one, off), __builtin_fmaf(b, one, off)});
-            a = u2f(pk << 16);
-            b = u2f(pk & 0xffff0000u);
-        } else if constexpr (WBITS == 4) s = 0.0625f * sc;
-        return (int)pack2_bf16((v2f){a * s, b * s});
+#pragma unroll
+        for (int i = 0; i < 4; i++) r[i] = (int)pack2_bf16((v2f){v[2 * i], v[2 * i + 1]});
     }
+    return r;
 }
+
+// Reads that transpose (lane layouts checked on the chip): of sixteen lanes, each at 8 bytes, lane l gets nibble l of all sixteen; or, in
+// pairs at 16 bytes of a row, byte l of the eight rows.
+typedef __attribute__((address_space(3))) v2i LdsV2i;
+__device__ __forceinline__ v2i lds_read_tr4(const char* at) { return __builtin_amdgcn_ds_read_tr4_b64_v2i32((LdsV2i*)at); }
+__device__ __forceinline__ v2i lds_read_tr8(const char* at) { return __builtin_amdgcn_ds_read_tr8_b64_v2i32((LdsV2i*)at); }
 
 // bytes of a tile, stages of the ring, bytes of the ring (at least what the sums need at the end), groups that the table has room for
 constexpr int ww_tile(int wbits, int mb) { return mb * 4096 + WW_COLS * WW_KT * wbits / 8; }
@@ -91,19 +128,25 @@ constexpr int ww_stages(int wbits, int mb)
     return wbits == 4 ? (mb <= 2 ? 6 : mb <= 4 ? 4 : 3) : (mb <= 4 ? 4 : 3);
 }
 constexpr int ww_ring(int wbits, int mb) { const int a = ww_tile(wbits, mb) * ww_stages(wbits, mb); return a > 65536 ? a : 65536; }
-constexpr int ww_groups(int wbits, int mb) { return (163840 - ww_ring(wbits, mb)) / (WW_COLS * 4); }
+constexpr int WW_FLAGS = 32;   // bytes behind the table, a word a wave
+constexpr int ww_groups(int wbits, int mb) { return (163840 - WW_FLAGS - ww_ring(wbits, mb)) / (WW_COLS * 4); }
 
 template <int XDT, int WBITS, int MB, bool HAS_OFF, bool KN>
 __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, int splits, int gmax)
 {
-    constexpr int NB = 4, TILE = ww_tile(WBITS, MB), S = ww_stages(WBITS, MB);
+    constexpr bool BIG = MB >= 2;                                            // 32 x 32 x 16, or 16 x 16 x 32
+    constexpr int LC = BIG ? 32 : 16, RB = BIG ? MB / 2 : MB, CB = 2;         // columns and rows of a block, row and column blocks of a wave
+    constexpr int WN = WW_COLS / (CB * LC), KW = 8 / WN, KS = WW_KT / KW;    // waves across columns and k, k of a wave's step
+    constexpr int E4 = BIG ? 4 : 1;                                          // quads of a block's sums that a lane has
+    constexpr int TILE = ww_tile(WBITS, MB), S = ww_stages(WBITS, MB);
     constexpr int XC = MB > 2 ? MB / 2 : 1, WC = WBITS / 4, CPT = XC + WC;   // copies per wave and tile
     constexpr int WROW = WW_KT * WBITS / 8;                                  // bytes of a weight row in a tile
+    typedef std::conditional_t<BIG, v16f, v4f> Acc;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wn = wave & 1, kw = wave >> 1;
-    const int r = lane & 15, q = lane >> 4;
+    const int wn = wave % WN, kw = wave / WN;
+    const int c = lane % LC, qh = lane / LC;
     const int Ni = (int)p.N, Ki = (int)p.K, Mi = (int)p.M;
     const int n0 = (int)blockIdx.x * WW_COLS, m0 = (int)blockIdx.z * (16 * MB);
     const int t0 = (int)((int64_t)blockIdx.y * tiles / splits), nt = (int)((int64_t)(blockIdx.y + 1) * tiles / splits) - t0;
@@ -121,17 +164,13 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
     }
 #pragma unroll
     for (int i = 0; i < WC; i++) {
-        const int row = WBITS == 4 ? wave * 16 + (lane >> 2) : (wave * 2 + i) * 8 + (lane >> 3);
+        const int row = WBITS == 4 ? wave * 16 + (lane >> 2) : (wave * 2 + i) * 8 + (lane >> 3);   // a column, or a row of k
         if constexpr (KN) {
-            // a tile row is a row of k; row k lies at slot k ^ (k / 8 % 4) (8 bits: k ^ (k / 8 % 2), and its halves swapped where k / 16 is odd)
-            const int k = WBITS == 4 ? row ^ ((row >> 3) & 3) : row ^ ((row >> 3) & 1);
-            const int c = WBITS == 4 ? (lane & 3) : (lane & 7) ^ (((row >> 4) & 1) << 2);
-            const int at = 16 * c, last = (Ni - n0) * WBITS / 8 - 16;
-            wo[i] = (uint32_t)k * (uint32_t)p.ldw + (at < last ? at : last);
+            const int at = 16 * (WBITS == 4 ? (lane & 3) ^ ((row >> 2) & 3) : (lane & 7) ^ (2 * ((row >> 1) & 3))), last = (Ni - n0) * WBITS / 8 - 16;
+            wo[i] = (uint32_t)row * (uint32_t)p.ldw + (at < last ? at : last);
         } else {
             const int n = n0 + row < Ni ? row : Ni - 1 - n0;
-            const int c = WBITS == 4 ? (lane & 3) ^ ((row >> 2) & 3) : (lane & 7) ^ ((row >> 1) & 7);
-            wo[i] = (uint32_t)n * (uint32_t)p.ldw + 16 * c;
+            wo[i] = (uint32_t)n * (uint32_t)p.ldw + 16 * (WBITS == 4 ? (lane & 3) ^ ((row >> 2) & 3) : (lane & 7) ^ ((row >> 1) & 7));
         }
     }
     const char* const xbase = (const char*)(p.x + (int64_t)m0 * Ki);
@@ -150,79 +189,79 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
         for (int i = 0; i < XC; i++) copy16_sbase(xbase + k * 2, xo[i], at + ((wave * XC + i) * 1024) % (MB * 4096));
     };
 
-    v4f acc[NB][MB];
-#pragma unroll
-    for (int j = 0; j < NB; j++)
-#pragma unroll
-        for (int b = 0; b < MB; b++) acc[j][b] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
-    const DqConst dqc = make_dq_const();
+    Acc acc[CB][RB] = {};
+    constexpr bool PERMUTE = !BIG && XDT == DT_F16 && WBITS == 4;   // one row block: four permutes for a fragment of x cost less than three more for each of its two operands
+    constexpr bool MAY_E4M3 = XDT == DT_BF16 && WBITS == 4 && !HAS_OFF;
+    const WwConst dqc = ww_const();
+    const DqConst dqp = make_dq_const();
     uint32_t* const tab = (uint32_t*)(smem + ww_ring(WBITS, MB));
+    // A lane multiplies k = KS kw + 16 qh .. + 15 of its columns and rows, eight at a time.
     struct Frags {
-        v4i x[MB];
-        uint32_t w[KN ? 8 : WBITS == 4 ? NB : 2 * NB];   // NK: column j's 8 codes; KN: row i of four columns
-        uint32_t so[NB];
+        v4i x[RB][2];
+        uint32_t w[CB][WBITS / 2];
+        uint32_t so[CB];
     };
+    const int ck = (KS * kw + 16 * qh) / 8;   // in pieces of 8 k
     auto read = [&](Frags& f, int stage) {
         const int k = k_read < k_last ? k_read : k_last;
         k_read += WW_KT;
         const char* const at = smem + stage * TILE;
+        const char* const wat = at + MB * 4096;
 #pragma unroll
-        for (int b = 0; b < MB; b++) f.x[b] = *(const v4i*)(at + (16 * b + r) * 256 + 16 * ((4 * kw + q) ^ r));
-        if constexpr (KN && WBITS == 4) {
+        for (int b = 0; b < RB; b++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {   // (row 32 kw + 8 q + i at the slot with i ^ q)
-                const char* const a = at + MB * 4096 + (32 * kw + 8 * q) * 64 + 32 * wn + 2 * r;
-                f.w[2 * i] = *(const uint16_t*)(a + ((2 * i) ^ q) * 64);
-                f.w[2 * i + 1] = *(const uint16_t*)(a + ((2 * i + 1) ^ q) * 64);
-            }
-        } else if constexpr (KN) {
+            for (int i = 0; i < 2; i++) f.x[b][i] = *(const v4i*)(at + (LC * b + c) * 256 + 16 * ((ck + i) ^ (c & 15)));
 #pragma unroll
-            for (int i = 0; i < 8; i++) f.w[i] = *(const uint32_t*)(at + MB * 4096 + (32 * kw + 8 * q + (i ^ (q & 1))) * 128 + 64 * (wn ^ (q >> 1)) + 4 * r);
-        } else {
+        for (int j = 0; j < CB; j++) {
+            const int col = (wn * CB + j) * LC + c;
+            if constexpr (!KN && WBITS == 4) __builtin_memcpy(f.w[j], __builtin_assume_aligned(wat + col * WROW + 16 * ((ck >> 2) ^ ((col >> 2) & 3)) + 4 * (ck & 2), 8), 8);
+            else if constexpr (!KN) __builtin_memcpy(f.w[j], __builtin_assume_aligned(wat + col * WROW + 16 * ((ck >> 1) ^ ((col >> 1) & 7)), 16), 16);
+            else {
+                // the transposing reads: sixteen lanes point at 16 k x 16 columns of 4 bits (8 k of 8 bits), and each gets a column's codes
+                const int n = (wn * CB + j) * LC + (BIG ? lane & 16 : 0);
+                if constexpr (WBITS == 4) {
+                    const int row = 8 * ck + (lane & 15);
+                    const v2i v = lds_read_tr4(wat + row * 64 + 16 * ((n >> 5) ^ ((row >> 2) & 3)) + ((n >> 1) & 8));
+                    f.w[j][0] = (uint32_t)v[0]; f.w[j][1] = (uint32_t)v[1];
+                } else {
 #pragma unroll
-            for (int j = 0; j < NB; j++) {
-                const char* const row = at + MB * 4096 + (wn * 64 + 16 * j + r) * WROW;
-                if constexpr (WBITS == 4) f.w[j] = *(const uint32_t*)(row + 16 * (kw ^ (r >> 2)) + 4 * q);
-                else __builtin_memcpy(f.w + 2 * j, __builtin_assume_aligned(row + 16 * ((2 * kw + (q >> 1)) ^ (r >> 1)) + 8 * (q & 1), 8), 8);
-            }
-        }
-        const int g = group_at(k + 32 * kw) - g_lo;
-#pragma unroll
-        for (int j = 0; j < NB; j++) f.so[j] = tab[g * WW_COLS + wn * 64 + (KN ? 4 * r + j : 16 * j + r)];
-    };
-    auto multiply = [&](const Frags& f) {
-        v4i xh[MB];
-        uint32_t pairs[4];   // KN, 4 bits: rows 2 i, 2 i + 1 of four columns
-        if constexpr (KN && WBITS == 4) {
-#pragma unroll
-            for (int i = 0; i < 4; i++) pairs[i] = f.w[2 * i] | f.w[2 * i + 1] << 16;
-        }
-#pragma unroll
-        for (int b = 0; b < MB; b++) {
-            xh[b] = f.x[b];
-            if constexpr (WBITS == 4 && !KN) {   // halves [0..7] -> [0,4,1,5,2,6,3,7]
-                const uint32_t a0 = (uint32_t)xh[b][0], a1 = (uint32_t)xh[b][1], a2 = (uint32_t)xh[b][2], a3 = (uint32_t)xh[b][3];
-                xh[b] = (v4i){(int)__builtin_amdgcn_perm(a2, a0, 0x05040100u), (int)__builtin_amdgcn_perm(a2, a0, 0x07060302u),
-                              (int)__builtin_amdgcn_perm(a3, a1, 0x05040100u), (int)__builtin_amdgcn_perm(a3, a1, 0x07060302u)};
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < NB; j++) {
-            v4i a;
-            if constexpr (KN) {
-#pragma unroll
-                for (int i = 0; i < 4; i++) {
-                    if constexpr (WBITS == 4) a[i] = kn_pair<XDT, 4, HAS_OFF>(pairs[i], 0, j, f.so[j], dqc);
-                    else a[i] = kn_pair<XDT, 8, HAS_OFF>(f.w[2 * i], f.w[2 * i + 1], j, f.so[j], dqc);
+                    for (int i = 0; i < 2; i++) {
+                        const int row = 8 * (ck + i) + ((lane & 15) >> 1);
+                        const v2i v = lds_read_tr8(wat + row * 128 + 16 * ((n >> 4) ^ (2 * ((row >> 1) & 3))) + 8 * (lane & 1));
+                        f.w[j][2 * i] = (uint32_t)v[0]; f.w[j][2 * i + 1] = (uint32_t)v[1];
+                    }
                 }
-            } else {
-                const v4i piece = {(int)f.w[WBITS == 4 ? j : 2 * j], WBITS == 8 ? (int)f.w[(2 * j + 1) % (2 * NB)] : 0, 0, 0};
-                a = dequant8<XDT, WBITS, HAS_OFF>(piece, 0, (uint16_t)f.so[j], (uint16_t)(f.so[j] >> 16), dqc);
+            }
+            f.so[j] = tab[(group_at(k + 8 * ck) - g_lo) * WW_COLS + col];
+        }
+    };
+    auto multiply = [&](const Frags& f, auto e4m3, bool part, bool counts) {
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            v4i xf[RB];
+#pragma unroll
+            for (int b = 0; b < RB; b++) {
+                xf[b] = f.x[b][i];
+                if constexpr (PERMUTE) {   // halves [0..7] -> [0,4,1,5,2,6,3,7]
+                    const uint32_t a0 = (uint32_t)xf[b][0], a1 = (uint32_t)xf[b][1], a2 = (uint32_t)xf[b][2], a3 = (uint32_t)xf[b][3];
+                    xf[b] = (v4i){(int)__builtin_amdgcn_perm(a2, a0, 0x05040100u), (int)__builtin_amdgcn_perm(a2, a0, 0x07060302u),
+                                  (int)__builtin_amdgcn_perm(a3, a1, 0x05040100u), (int)__builtin_amdgcn_perm(a3, a1, 0x07060302u)};
+                }
             }
 #pragma unroll
-            for (int b = 0; b < MB; b++) {
-                if constexpr (XDT == DT_F16) acc[j][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, xh[b]), acc[j][b], 0, 0, 0);
-                else acc[j][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, xh[b]), acc[j][b], 0, 0, 0);
+            for (int j = 0; j < CB; j++) {
+                v4i a;
+                if constexpr (PERMUTE) a = dequant8<XDT, WBITS, HAS_OFF>((v4i){(int)f.w[j][i], 0, 0, 0}, 0, (uint16_t)f.so[j], (uint16_t)(f.so[j] >> 16), dqp);
+                else a = ww_dequant<XDT, WBITS, HAS_OFF, decltype(e4m3)::value>(f.w[j] + i * (WBITS / 4), f.so[j], dqc);
+                if (part) a = counts ? a : (v4i){0, 0, 0, 0};
+#pragma unroll
+                for (int b = 0; b < RB; b++) {
+                    const v4i x = part && !counts ? (v4i){0, 0, 0, 0} : xf[b];
+                    if constexpr (BIG && XDT == DT_F16) acc[j][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, x), acc[j][b], 0, 0, 0);
+                    else if constexpr (BIG) acc[j][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, x), acc[j][b], 0, 0, 0);
+                    else if constexpr (XDT == DT_F16) acc[j][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, a), __builtin_bit_cast(v8h, x), acc[j][b], 0, 0, 0);
+                    else acc[j][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a), __builtin_bit_cast(v8bf, x), acc[j][b], 0, 0, 0);
+                }
             }
         }
     };
@@ -249,10 +288,12 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
             }
         }
     };
+    bool large = false;   // a scale from 2^125 on, an infinity or NaN
     auto store8 = [&](const Eight& v, int i) {
         const int g = t_g + 32 * i - g_lo;
 #pragma unroll
         for (int e = 0; e < 8; e++) {
+            if constexpr (MAY_E4M3) large = large || (v.s[e] & 0x7f80) >= 0x7e00;
             const int ge = g + (by_group ? e : 0), ne = t_col + (by_group ? 0 : e);
             if (ge >= 0 && ge < gmax) tab[ge * WW_COLS + ne] = HAS_OFF ? v.s[e] | (uint32_t)v.o[e] << 16 : v.s[e];
         }
@@ -268,67 +309,93 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
         store8(v0, 0);
         if (32 < gmax + 7) store8(v1, 1);
     }
+    uint32_t* const flags = tab + gmax * WW_COLS;
+    if constexpr (MAY_E4M3) {
+        const uint64_t any = __ballot(large);
+        if (lane == 0) flags[wave] = any != 0;
+    }
     wait_copies<(S - 1) * CPT>();
     __syncthreads();
-    const bool rest = base_of(nt - 1) + 32 * kw >= (t0 + nt - 1) * WW_KT;   // (a partial tile: the others were counted with the one before)
-    if constexpr (MB <= 4) {
-        Frags f0, f1;
-        read(f0, 0);
-        int t = 0, at = 0;
-        // tile t + 1 is read while tile t multiplies; tile t + S goes where tile t was, whose fragments every wave holds by then
-        auto step = [&](const Frags& now, Frags& then) {
-            wait_copies<(S - 2) * CPT>();
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" : : : "memory");
-            issue(at);
-            at = at + 1 < S ? at + 1 : 0;
-            read(then, at);
-            __builtin_amdgcn_sched_barrier(0);
-            multiply(now);
-        };
-        for (; t + 2 < nt; t += 2) {
-            step(f0, f1);
-            step(f1, f0);
+    // (a last, partial tile: what lies in front of it was counted with the one before)
+    const bool part = (t0 + nt) * WW_KT > Ki, counts = base_of(nt - 1) + 8 * ck >= (t0 + nt - 1) * WW_KT;
+    auto walk = [&](auto e4m3) {
+        if constexpr (MB <= 4) {
+            Frags f0, f1;
+            read(f0, 0);
+            int t = 0, at = 0;
+            // tile t + 1 is read while tile t multiplies; tile t + S goes where tile t was, whose fragments every wave holds by then
+            auto step = [&](const Frags& now, Frags& then) {
+                wait_copies<(S - 2) * CPT>();
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" : : : "memory");
+                issue(at);
+                at = at + 1 < S ? at + 1 : 0;
+                read(then, at);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(now, e4m3, false, true);
+            };
+            for (; t + 2 < nt; t += 2) {
+                step(f0, f1);
+                step(f1, f0);
+            }
+            if (t + 1 < nt) {
+                step(f0, f1);
+                multiply(f1, e4m3, part, counts);
+            } else multiply(f0, e4m3, part, counts);
+        } else {   // (no registers for a second set of fragments: tile t + S - 1 goes where tile t - 1 was)
+            Frags f;
+            int at = 0, free = S - 1;
+            for (int t = 0; t < nt; t++) {
+                wait_copies<(S - 2) * CPT>();
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" : : : "memory");
+                if (t > 0) issue(free);
+                read(f, at);
+                if (t + 1 < nt) multiply(f, e4m3, false, true);
+                free = at;
+                at = at + 1 < S ? at + 1 : 0;
+            }
+            multiply(f, e4m3, part, counts);
         }
-        if (t + 1 < nt) {
-            step(f0, f1);
-            if (rest) multiply(f1);
-        } else if (rest) multiply(f0);
-    } else {   // (no registers for a second set of fragments: tile t + S - 1 goes where tile t - 1 was)
-        Frags f;
-        int at = 0, free = S - 1;
-        for (int t = 0; t < nt; t++) {
-            wait_copies<(S - 2) * CPT>();
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" : : : "memory");
-            if (t > 0) issue(free);
-            read(f, at);
-            if (t + 1 < nt || rest) multiply(f);
-            free = at;
-            at = at + 1 < S ? at + 1 : 0;
-        }
-    }
+    };
+    if constexpr (MAY_E4M3) {
+        uint32_t any = 0;
+#pragma unroll
+        for (int i = 0; i < WW_FLAGS / 4; i++) any |= flags[i];
+        if (__builtin_amdgcn_readfirstlane(any)) walk(std::false_type{});
+        else walk(std::true_type{});
+    } else walk(std::false_type{});
     wait_copies<0>();
     __syncthreads();   // the ring makes room for the sums
 
-    // acc[j][b][e]: n = n0 + 64 wn + 16 j + 4 q + e (KN: 4 (4 q + e) + j), m = m0 + 16 b + r, over the k of kw
+    // The waves' sums over k, 8 KB of each wave at a time.  A quad: n = LC (CB wn + j) + 8 e + 4 qh .. + 3, m = LC b + c (16 x 16: n = 4 qh ..);
+    // lane l's lies at l ^ (its number), so that threads can take a row's quads one after the other.
     float* const red = (float*)smem;
+    constexpr int PIECES = CB * E4;   // of a round, which is a row block
 #pragma unroll
-    for (int b0 = 0; b0 < MB; b0 += 2) {
-        constexpr int RB = MB < 2 ? 1 : 2;
+    for (int rd = 0; rd < RB; rd++) {
 #pragma unroll
-        for (int j = 0; j < NB; j++)
+        for (int j = 0; j < CB; j++)
 #pragma unroll
-            for (int b = 0; b < RB; b++) *(v4f*)(red + ((kw * 2 + wn) * (NB * RB) + j * RB + b) * 256 + lane * 4) =
-                KN ? (v4f){acc[0][b0 + b][j], acc[1][b0 + b][j], acc[2][b0 + b][j], acc[3][b0 + b][j]} : acc[j][b0 + b];
+            for (int e = 0; e < E4; e++) {
+                v4f v;
+                if constexpr (BIG) v = (v4f){acc[j][rd][4 * e], acc[j][rd][4 * e + 1], acc[j][rd][4 * e + 2], acc[j][rd][4 * e + 3]};
+                else v = acc[j][rd];
+                const int piece = j * E4 + e;
+                *(v4f*)(red + (wave * PIECES + piece) * 256 + 4 * (lane ^ (BIG ? 2 * piece + qh : 4 * piece + qh))) = v;
+            }
         __syncthreads();
+        constexpr int QUADS = WW_COLS / 4;   // of a row
 #pragma unroll
-        for (int i = 0; i < RB; i++) {
-            const int t = tid + 512 * i, blk = t >> 6;   // block (wn, j, b)
-            v4f sum = *(const v4f*)(red + t * 4);
+        for (int i = 0; i < LC * QUADS / 512; i++) {
+            const int t = tid + 512 * i, nq = t % QUADS, ml = t / QUADS;
+            const int w_n = nq / (CB * LC / 4), in = nq % (CB * LC / 4);
+            const int piece = BIG ? in >> 1 : in >> 2, half = BIG ? in & 1 : in & 3;
+            const int slot = (half * LC + ml) ^ (BIG ? 2 * piece + half : 4 * piece + half);
+            v4f sum = *(const v4f*)(red + (w_n * PIECES + piece) * 256 + 4 * slot);
 #pragma unroll
-            for (int h = 1; h < 4; h++) sum = sum + *(const v4f*)(red + (h * 2 * NB * RB) * 256 + t * 4);
-            const int m = m0 + 16 * (b0 + blk % RB) + (t & 15), n = n0 + 64 * (blk / (NB * RB)) + (KN ? 4 : 16) * (blk / RB % NB) + (KN ? 16 : 4) * ((t >> 4) & 3);
+            for (int h = 1; h < KW; h++) sum = sum + *(const v4f*)(red + ((h * WN + w_n) * PIECES + piece) * 256 + 4 * slot);
+            const int m = m0 + LC * rd + ml, n = n0 + 4 * nq;
             if (m < Mi && n < Ni) {
                 const int cols = Ni - n < 4 ? Ni - n : 4;
                 if (splits > 1) {
@@ -357,7 +424,7 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
                 }
             }
         }
-        if (b0 + 2 < MB) __syncthreads();
+        if (rd + 1 < RB) __syncthreads();
     }
 }
 
@@ -380,7 +447,7 @@ int launch_one(const WqParams& p, const WqWidePlan& pl, hipStream_t st)
     const int tiles = (int)((p.K + WW_KT - 1) / WW_KT);
     const dim3 grid((unsigned)((p.N + WW_COLS - 1) / WW_COLS), (unsigned)pl.splits, (unsigned)((p.M + 16 * MB - 1) / (16 * MB)));
     note_route("wq_wide", pl.splits);
-    hipLaunchKernelGGL(k, grid, dim3(512), ww_ring(WBITS, MB) + pl.groups * WW_COLS * 4, st, p, tiles, pl.splits, pl.groups);
+    hipLaunchKernelGGL(k, grid, dim3(512), ww_ring(WBITS, MB) + pl.groups * WW_COLS * 4 + WW_FLAGS, st, p, tiles, pl.splits, pl.groups);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || pl.splits == 1) return (int)e;
     launch_wq_splitk_reduce(p, pl.splits, XDT, st);
     return (int)hipGetLastError();

@@ -115,3 +115,29 @@ def test_unaligned_weight_runs_elsewhere(gpu, M, K, N, nk):
     assert route(m)[0] != "wq_wide"
     assert (buf.to_host(np.uint8, (ws + guard,))[ws:] == 0xA5).all()
     _b16_bar(d_y.to_host(np.uint16, (M, N)), cases.oracle_wq(m, inp, M, K, N), orc.F16, "unaligned weight", K)
+
+
+@pytest.mark.parametrize("M,K,N,group,nk", [(40, 8192, 1056, 128, False), (1, 1056, 1024, 32, False), (40, 12544, 1793, 64, True), (130, 8832, 1026, 0, True)])
+def test_scales_at_the_end_of_the_range(gpu, M, K, N, group, nk):
+    """bf16 x int4 without offsets converts by way of w + 8, which is exact while eight scales are a number: an infinite, a NaN and a
+    scale of 2^126 in one column each, and in a workgroup without them nothing changes."""
+    m = gpu
+    print(f"case wide, large scales M={M} K={K} N={N} nk={nk}", flush=True)
+    inp = cases.make_wq_inputs(m, M, K, N, 5, m.ACL_BF16, m.ACL_INT4, group, nk, False, None)
+    inp["x"] = orc.f32_to_b16(np.abs(orc.b16_to_f32(inp["x"], orc.BF16)) * np.float32(2.0 ** -20), orc.BF16)
+    codes = orc.unpack_nibbles(inp["w"]).reshape((N, K) if nk else (K, N)) & 15
+    scale = inp["scale"].reshape((N, -1) if nk else (-1, N))
+    for col, s in ((3, np.inf), (N // 2, np.nan), (N - 2, 2.0 ** 126), (N - 1, -np.inf)):
+        c = np.random.default_rng(col).integers(1, 4, K).astype(codes.dtype)
+        (codes[col] if nk else codes[:, col])[...] = c
+        (scale[col] if nk else scale[:, col])[...] = orc.f32_to_b16(np.array([s], np.float32), orc.BF16)[0]
+    inp["w"], inp["scale"] = orc.pack_nibbles(codes.astype(np.uint8)), np.ascontiguousarray(scale.reshape(inp["scale"].shape))
+    got, want = cases.run_wq_aclnn(m, inp, M, K, N), cases.oracle_wq(m, inp, M, K, N)
+    assert route(m)[0] == "wq_wide", route(m)
+    g, w = orc.b16_to_f32(got, orc.BF16), orc.b16_to_f32(want, orc.BF16)
+    assert np.array_equal(np.isnan(g), np.isnan(w)) and np.array_equal(np.isinf(g), np.isinf(w)) and np.isinf(w[:, 3]).all() and np.isnan(w[:, N // 2]).all()
+    assert np.array_equal(np.sign(g[np.isinf(w)]), np.sign(w[np.isinf(w)])) and np.isfinite(w[:, N - 2]).all()
+    rest = np.isfinite(w).all(axis=0)
+    rest[N - 2] = False
+    _b16_bar(np.ascontiguousarray(got[:, rest]), np.ascontiguousarray(want[:, rest]), orc.BF16, "wide, other columns", K)
+    assert np.abs(g[:, N - 2] / w[:, N - 2] - 1).max() <= 2.0 ** -7
