@@ -275,6 +275,11 @@ __device__ __forceinline__ void copy16_sbase(const void* base, uint32_t voff, ui
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
 }
+// The same past the last-level cache (a nontemporal load).
+__device__ __forceinline__ void copy16_sbase_once(const void* base, uint32_t voff, uint32_t lds)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dwordx4 %1, %2 nt" : : "s"(lds), "v"(voff), "s"(base) : "memory", "m0");
+}
 __device__ __forceinline__ void copy4_sbase(const void* base, uint32_t voff, uint32_t lds)
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 4\n\tglobal_load_lds_dword %1, %2" : : "s"(lds), "v"(voff), "s"(base) : "memory", "m0");

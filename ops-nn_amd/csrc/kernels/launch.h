@@ -58,6 +58,12 @@ struct SplitK {
     int splits = 1;
     float* part = nullptr;
 };
+// Whether a weight that a call reads once goes past the last-level cache (256 MB): from 100 MB on.  A step works through three such weights
+// and more, of which none is found there again, and fetched without a line kept there they come faster.  Copies of 128-byte row
+// pieces into LDS, three weights in turn, plain / past the cache: 88 MB 14.2 / 23.4 us, 101 MB 23.5 / 23.6, 117 MB 26.7 / 24.7, 168 MB 34.1 / 30.2, 235 MB 43.3 /
+// 39.2 (one weight again and again, which is the other way round: 117 MB 17.0 / 24.5, 262 MB 38.9 / 40.9).  Not where the pieces are 64
+// bytes, half a line that is then fetched twice: 117 MB 25.0 / 27.5.
+inline bool weight_is_streamed(int64_t bytes) { return bytes > 100000000; }
 // How many ways a call with `tiles` output tiles, `ktiles` K tiles of `tile_us` microseconds each and `out_elems` outputs
 // is split: at most one workgroup per CU, at least four K tiles per workgroup, at most sixteen ways -- and among those the
 // count with the largest estimated gain, if that is at least 3 us: the loop time saved, ktiles * tile_us * (1 - 1/s), less

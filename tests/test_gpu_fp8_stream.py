@@ -94,6 +94,17 @@ def test_row_column_and_mx_scales(gpu, form, M, K, N):
     del keep
 
 
+# a weight from 100 MB on: the wide kernel's copies go past the last-level cache, a last strip of one column, segments
+@pytest.mark.parametrize("form,M,K,N", [("block", 17, 12288, 8193), ("rowcol", 33, 13568, 7400), ("mx", 20, 18432, 5440)])
+def test_weights_from_100_mb_on(gpu, form, M, K, N):
+    assert N * K > 100_000_000
+    if form == "block":
+        test_block_scales(gpu, M, K, N, 1, "bf16")
+    else:
+        test_row_column_and_mx_scales(gpu, form, M, K, N)
+    assert route(gpu)[0] == "fp8_wide", route(gpu)
+
+
 # rows of x1 so far apart that the last ones lie 2^32 bytes and more behind the first: the stream kernels' lane offsets have 32 bits
 # (a K tail runs on padded copies, whose rows lie close together)
 @pytest.mark.parametrize("M,K,N,want", [(300, 1024, 256, "fp8_exact"), (300, 1088, 260, "fp8_stream")])
