@@ -23,6 +23,8 @@
 //
 // LDS rows, conflict-free for the reads below: x 256 bytes, 16-byte chunk c of row r at c ^ (r % 16); [N, K] weights 64 bytes (4 bits),
 // c ^ (r / 4 % 4), or 128, c ^ (r / 2 % 8); [K, N] weights, a row of k each, 64 bytes, c ^ (k / 4 % 4), or 128, c ^ 2 (k / 2 % 4).
+// A [K, N] weight whose rows are whole dwords but not 16-byte pieces (N a multiple of 8 with 4 bits, of 4 with 8) is copied a dword a lane, four
+// copies for one (4 bits) and eight for two (8 bits) a wave and tile.  0.05 us a tile (4 bits) and 0.1 (8).
 //
 // Measured, before these products and reads and with them, the weight in turn from three buffers: 121 drawn calls of 1 .. 512 rows 1.058 times as
 // fast, none slower by more than 2 %; bf16 x int4 499 x 13632 x 3052 77 -> 64 us, 129 x 14912 x 3328 41 -> 35; fp16 64 x 16384 x 5120 91 -> 81
@@ -131,7 +133,10 @@ constexpr int ww_ring(int wbits, int mb) { const int a = ww_tile(wbits, mb) * ww
 constexpr int WW_FLAGS = 32;   // bytes behind the table, a word a wave
 constexpr int ww_groups(int wbits, int mb) { return (163840 - WW_FLAGS - ww_ring(wbits, mb)) / (WW_COLS * 4); }
 
-template <int XDT, int WBITS, int MB, bool HAS_OFF, bool KN>
+// [N, K] storage; [K, N] storage with rows of whole 16-byte pieces; of whole dwords
+enum WwStorage { WW_NK, WW_KN, WW_KN4 };
+
+template <int XDT, int WBITS, int MB, bool HAS_OFF, int STORAGE>
 __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, int splits, int gmax)
 {
     constexpr bool BIG = MB >= 2;                                            // 32 x 32 x 16, or 16 x 16 x 32
@@ -139,7 +144,9 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
     constexpr int WN = WW_COLS / (CB * LC), KW = 8 / WN, KS = WW_KT / KW;    // waves across columns and k, k of a wave's step
     constexpr int E4 = BIG ? 4 : 1;                                          // quads of a block's sums that a lane has
     constexpr int TILE = ww_tile(WBITS, MB), S = ww_stages(WBITS, MB);
-    constexpr int XC = MB > 2 ? MB / 2 : 1, WC = WBITS / 4, CPT = XC + WC;   // copies per wave and tile
+    constexpr bool KN = STORAGE != WW_NK;
+    constexpr int WP = STORAGE == WW_KN4 ? 4 : 16;                                       // bytes of a lane's copy of the weight
+    constexpr int XC = MB > 2 ? MB / 2 : 1, WC = WBITS / 4 * (16 / WP), CPT = XC + WC;   // copies per wave and tile
     constexpr int WROW = WW_KT * WBITS / 8;                                  // bytes of a weight row in a tile
     typedef std::conditional_t<BIG, v16f, v4f> Acc;
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -164,13 +171,13 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
     }
 #pragma unroll
     for (int i = 0; i < WC; i++) {
-        const int row = WBITS == 4 ? wave * 16 + (lane >> 2) : (wave * 2 + i) * 8 + (lane >> 3);   // a column, or a row of k
+        const int piece = (wave * WC + i) * 64 + lane, row = piece / (WROW / WP), b = piece % (WROW / WP) * WP;   // a column, or a row of k; byte of the LDS row
         if constexpr (KN) {
-            const int at = 16 * (WBITS == 4 ? (lane & 3) ^ ((row >> 2) & 3) : (lane & 7) ^ (2 * ((row >> 1) & 3))), last = (Ni - n0) * WBITS / 8 - 16;
+            const int at = (b ^ 16 * (WBITS == 4 ? (row >> 2) & 3 : 2 * ((row >> 1) & 3))), last = (Ni - n0) * WBITS / 8 - WP;
             wo[i] = (uint32_t)row * (uint32_t)p.ldw + (at < last ? at : last);
         } else {
             const int n = n0 + row < Ni ? row : Ni - 1 - n0;
-            wo[i] = (uint32_t)n * (uint32_t)p.ldw + 16 * (WBITS == 4 ? (lane & 3) ^ ((row >> 2) & 3) : (lane & 7) ^ ((row >> 1) & 7));
+            wo[i] = (uint32_t)n * (uint32_t)p.ldw + (b ^ 16 * (WBITS == 4 ? (row >> 2) & 3 : (row >> 1) & 7));
         }
     }
     const char* const xbase = (const char*)(p.x + (int64_t)m0 * Ki);
@@ -184,7 +191,10 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
         k_issue += WW_KT;
         const uint32_t at = __builtin_amdgcn_readfirstlane(ring + stage * TILE);
 #pragma unroll
-        for (int i = 0; i < WC; i++) copy16_sbase(wbase + (KN ? k * p.ldw : k * WBITS / 8), wo[i], at + MB * 4096 + (wave * WC + i) * 1024);
+        for (int i = 0; i < WC; i++) {
+            if constexpr (WP == 16) copy16_sbase(wbase + (KN ? k * p.ldw : k * WBITS / 8), wo[i], at + MB * 4096 + (wave * WC + i) * 1024);
+            else copy4_sbase(wbase + k * p.ldw, wo[i], at + MB * 4096 + (wave * WC + i) * 256);
+        }
 #pragma unroll
         for (int i = 0; i < XC; i++) copy16_sbase(xbase + k * 2, xo[i], at + ((wave * XC + i) * 1024) % (MB * 4096));
     };
@@ -430,14 +440,14 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
 
 struct WqWidePlan {
     int mb = 2, splits = 1, groups = 1;
-    bool kn = false;
+    bool kn = false, dwords = false;   // [K, N] storage; its rows are no whole 16-byte pieces
     float us = 0.0f;
 };
 
-template <int XDT, int WBITS, int MB, bool HAS_OFF, bool KN>
+template <int XDT, int WBITS, int MB, bool HAS_OFF, int STORAGE>
 int launch_one(const WqParams& p, const WqWidePlan& pl, hipStream_t st)
 {
-    auto k = wq_wide_kernel<XDT, WBITS, MB, HAS_OFF, KN>;
+    auto k = wq_wide_kernel<XDT, WBITS, MB, HAS_OFF, STORAGE>;
     static std::atomic<uint64_t> attr_set{0};   // one bit per device: the attribute belongs to the (kernel, device) pair
     if (!device_flag_test(attr_set)) {
         hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 163840);
@@ -452,19 +462,20 @@ int launch_one(const WqParams& p, const WqWidePlan& pl, hipStream_t st)
     launch_wq_splitk_reduce(p, pl.splits, XDT, st);
     return (int)hipGetLastError();
 }
-template <int XDT, int WBITS, bool HAS_OFF>
+template <int XDT, int WBITS, bool HAS_OFF, int STORAGE>
 int launch_mb(const WqParams& p, const WqWidePlan& pl, hipStream_t st)
 {
-    if (pl.kn) {
-        if (pl.mb == 1) return launch_one<XDT, WBITS, 1, HAS_OFF, true>(p, pl, st);
-        if (pl.mb == 2) return launch_one<XDT, WBITS, 2, HAS_OFF, true>(p, pl, st);
-        if (pl.mb == 4) return launch_one<XDT, WBITS, 4, HAS_OFF, true>(p, pl, st);
-        return launch_one<XDT, WBITS, 8, HAS_OFF, true>(p, pl, st);
-    }
-    if (pl.mb == 1) return launch_one<XDT, WBITS, 1, HAS_OFF, false>(p, pl, st);
-    if (pl.mb == 2) return launch_one<XDT, WBITS, 2, HAS_OFF, false>(p, pl, st);
-    if (pl.mb == 4) return launch_one<XDT, WBITS, 4, HAS_OFF, false>(p, pl, st);
-    return launch_one<XDT, WBITS, 8, HAS_OFF, false>(p, pl, st);
+    if (pl.mb == 1) return launch_one<XDT, WBITS, 1, HAS_OFF, STORAGE>(p, pl, st);
+    if (pl.mb == 2) return launch_one<XDT, WBITS, 2, HAS_OFF, STORAGE>(p, pl, st);
+    if (pl.mb == 4) return launch_one<XDT, WBITS, 4, HAS_OFF, STORAGE>(p, pl, st);
+    return launch_one<XDT, WBITS, 8, HAS_OFF, STORAGE>(p, pl, st);
+}
+template <int XDT, int WBITS>
+int launch_form(const WqParams& p, const WqWidePlan& pl, hipStream_t st)
+{
+    if (!pl.kn) return p.offset ? launch_mb<XDT, WBITS, true, WW_NK>(p, pl, st) : launch_mb<XDT, WBITS, false, WW_NK>(p, pl, st);
+    if (!pl.dwords) return p.offset ? launch_mb<XDT, WBITS, true, WW_KN>(p, pl, st) : launch_mb<XDT, WBITS, false, WW_KN>(p, pl, st);
+    return p.offset ? launch_mb<XDT, WBITS, true, WW_KN4>(p, pl, st) : launch_mb<XDT, WBITS, false, WW_KN4>(p, pl, st);
 }
 
 // Which layout is best: what a launch takes, in us, the weight from memory, fitted to 1460 timed launches of 160 calls (M 1 .. 400, K 1024 .. 18432, N 1024 .. 28672; median error 5 %):
@@ -509,7 +520,7 @@ double wide_typical_us(const OpsnnWqmmArgs& a, int wbits, const WqWidePlan& pl)
 {
     static const double tile[2][2][2] = {{{0.343, 0.444}, {0.486, 0.82}}, {{0.407, 0.502}, {0.449, 0.802}}};   // [8 bits][bf16][offset]
     const int64_t strips = (a.N + WW_COLS - 1) / WW_COLS, tiles = (a.K + WW_KT - 1) / WW_KT, slabs = (a.M + 16 * pl.mb - 1) / (16 * pl.mb);
-    const double t = tile[wbits == 8][a.x_dtype == DT_BF16][a.offset != nullptr] + 0.066 * pl.mb + (pl.kn ? 0.056 : 0.0), out_m = (double)a.M * (double)a.N * 1e-6;
+    const double t = tile[wbits == 8][a.x_dtype == DT_BF16][a.offset != nullptr] + 0.066 * pl.mb + (pl.kn ? 0.056 : 0.0) + (pl.dwords ? 0.0125 * wbits : 0.0), out_m = (double)a.M * (double)a.N * 1e-6;
     const double cu = (double)((strips * slabs * pl.splits + 255) / 256) * ((double)((tiles + pl.splits - 1) / pl.splits) * t + 1.91 + 0.355 * pl.mb + 0.0143 * pl.groups);
     return 2.39 + 1.33 * out_m + wq_typical_both(cu, wq_typical_mb(wbits, a.N, a.K) / 6.56) + (pl.splits > 1 ? 2.9 + 2.09 * pl.splits * out_m * (a.N % 4 ? 2.0 : 1.0) : 0.0);
 }
@@ -543,6 +554,11 @@ double others_typical_us(const OpsnnWqmmArgs& a, const WqForm& f)
 // [K, N] storage not where the weight is large and wide, of 68 such calls 56 faster there (16 x 8192 x 28672 40.7 us, 47.9 here; 5 x 12288 x 27072 61
 // and 86); [N, K] storage from 8 MB, and not where K is one whole shape of the x-in-registers kernel (16 x 8192 x 28672 36 there, 44 here;
 // 4 x 3072 x 3128 7.3 and 10.5).  From 513 rows the dequantising pass is ahead of a fifth slab.
+//
+// Rows in dwords: of 126 drawn calls of that kind 68 come here, 1.22 times as fast as on the pass (behind which the re-layout read the weight
+// column by column) and the [K, N] decode kernel: 156 x 7168 x 21520 int4 bf16 208 -> 100 us, 85 x 11008 x 2456 37 -> 21, 53 x 1408 x 22192 28 -> 15.
+// Not where the estimates were wrong about them: from 257 rows with few k (510 x 1152 x 5744 21 there, 24 here), int8 up to 16 rows
+// (10 x 13184 x 3944 20.7 and 22.0).
 bool wide_wanted(const OpsnnWqmmArgs& a, WqWidePlan& pl)
 {
     if ((a.w_dtype != DT_I4 && a.w_dtype != DT_I8) || (a.x_dtype != DT_F16 && a.x_dtype != DT_BF16)) return false;
@@ -552,7 +568,9 @@ bool wide_wanted(const OpsnnWqmmArgs& a, WqWidePlan& pl)
     const WqForm f = wq_form(a);
     const int64_t codes = a.N * a.K;
     pl.kn = !f.nk;
-    if (pl.kn && (a.w.col_stride != 1 || a.w.row_stride != a.N || a.N % (128 / f.wbits) != 0)) return false;
+    if (pl.kn && (a.w.col_stride != 1 || a.w.row_stride != a.N || a.N % (32 / f.wbits) != 0)) return false;
+    pl.dwords = pl.kn && a.N % (128 / f.wbits) != 0;
+    if (pl.dwords && ((a.M > 256 && a.K < 1536) || (a.M <= 16 && f.wbits == 8))) return false;
     if (f.group < a.K && (f.group < 32 || (f.group & (f.group - 1)) != 0)) return false;
     if (codes < (a.M > 64 ? 1ll << 21 : 1ll << 20)) return false;
     if (pl.kn && a.w_dtype == DT_I8 && a.M <= 16 && codes <= (1ll << 24)) return false;   // (as in wq_kn.hip)
@@ -608,12 +626,8 @@ int launch_wq_wide(const OpsnnWqmmArgs& a0, hipStream_t st)
     p.y = (uint16_t*)a.y; p.M = a.M; p.N = a.N; p.K = a.K;
     p.group_shift = p.group >= p.K ? 31 : __builtin_ctzll((unsigned long long)p.group);
     p.part = (float*)a.workspace;
-    if (a.x_dtype == DT_F16) {
-        if (wbits == 4) return a.offset ? launch_mb<DT_F16, 4, true>(p, pl, st) : launch_mb<DT_F16, 4, false>(p, pl, st);
-        return a.offset ? launch_mb<DT_F16, 8, true>(p, pl, st) : launch_mb<DT_F16, 8, false>(p, pl, st);
-    }
-    if (wbits == 4) return a.offset ? launch_mb<DT_BF16, 4, true>(p, pl, st) : launch_mb<DT_BF16, 4, false>(p, pl, st);
-    return a.offset ? launch_mb<DT_BF16, 8, true>(p, pl, st) : launch_mb<DT_BF16, 8, false>(p, pl, st);
+    if (a.x_dtype == DT_F16) return wbits == 4 ? launch_form<DT_F16, 4>(p, pl, st) : launch_form<DT_F16, 8>(p, pl, st);
+    return wbits == 4 ? launch_form<DT_BF16, 4>(p, pl, st) : launch_form<DT_BF16, 8>(p, pl, st);
 }
 
 }  // namespace opsnn

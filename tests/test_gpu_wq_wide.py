@@ -18,6 +18,8 @@ ELSEWHERE = {(17, 2080, 4128) + k: "wq_kn" for k in KINDS}
 ELSEWHERE.update({(17, 2080, 16416) + k: "wq_kn" for k in KINDS if k[1] == "bf16"})
 ELSEWHERE.update({(1, 1056, 16416) + k: "wq_kn" for k in KINDS if k[1:] == ("bf16", True)})
 ELSEWHERE.update({(1, 1056, 1024) + k: "wq_general" for k in KINDS if k[0] == "i8"})
+ELSEWHERE.update({shape + k: "wq_general" for shape in [(1, 4128, 1064), (16, 4128, 1080)] for k in KINDS if k[0] == "i8"})
+ELSEWHERE[(33, 8192, 1048, "i4", "bf16", False)] = "wq_kn"
 ELSEWHERE.update({(257, 7040, 1090) + k: "wq_dense" for k in KINDS if k[1:] == ("bf16", True)})
 
 
@@ -37,6 +39,17 @@ def _check(m, M, K, N, group, nk, w_dt, x_dt, off):
 ])
 @pytest.mark.parametrize("w_dt,x_dt,off", KINDS)
 def test_rows_of_k(gpu, M, K, N, group, w_dt, x_dt, off):
+    _check(gpu, M, K, N, group, False, w_dt, x_dt, off)
+
+
+@pytest.mark.parametrize("M,K,N,group", [
+    (1, 4128, 1064, 32), (16, 4128, 1080, 64), (33, 8192, 1048, 128), (64, 4160, 2088, 0), (65, 1344, 1672, 64), (96, 2080, 2124, 0),
+    (130, 2336, 1068, 0), (300, 4096, 552, 32), (400, 2080, 4104, 128),
+])
+@pytest.mark.parametrize("w_dt,x_dt,off", KINDS)
+def test_rows_of_k_in_whole_dwords(gpu, M, K, N, group, w_dt, x_dt, off):
+    if w_dt == "i4" and N % 8 != 0:
+        N += 4
     _check(gpu, M, K, N, group, False, w_dt, x_dt, off)
 
 
