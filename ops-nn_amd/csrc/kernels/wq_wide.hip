@@ -1,4 +1,4 @@
-// Weight-only matmul, up to 512 rows of x, either storage of the weight ([N, K] and [K, N]), any group that is a power of two from 32.
+// Weight-only matmul, up to 1024 rows of x, either storage of the weight ([N, K] and [K, N]), any group that is a power of two from 32.
 //
 // What bounded these calls (17 .. 64 rows on the kernels of wq_nk.hip, wq_kn.hip and wqmm_stream.hip.h, more rows on the dequantising
 // pass of wq_dense.hip): operands loaded straight into the layout of the matrix instructions, 16 rows per 16 lanes, take 66 clocks a KB
@@ -553,17 +553,19 @@ double others_typical_us(const OpsnnWqmmArgs& a, const WqForm& f)
 // Below 2^20 codes nothing was timed; from 65 rows the pass is ahead below 2^21 (189 x 1152 x 1088 12.1 there, 13.7 here).  Up to 16 rows:
 // [K, N] storage not where the weight is large and wide, of 68 such calls 56 faster there (16 x 8192 x 28672 40.7 us, 47.9 here; 5 x 12288 x 27072 61
 // and 86); [N, K] storage from 8 MB, and not where K is one whole shape of the x-in-registers kernel (16 x 8192 x 28672 36 there, 44 here;
-// 4 x 3072 x 3128 7.3 and 10.5).  From 513 rows the dequantising pass is ahead of a fifth slab.
+// 4 x 3072 x 3128 7.3 and 10.5).  To 1024 rows: of 70 drawn calls of 513 .. 1024 the estimates
+// send 26 here, 1.15 times as fast as on the pass and the many-rows kernel, one slower by more than 2 % (762 x 10624 x 24704 472 us there, 500
+// here): 630 x 9472 x 18624 int4 fp16 326 -> 268, 707 x 9024 x 4160 int8 99 -> 77, 580 x 1408 x 5231 27.5 -> 21.6; of seven beyond one gained (1.07)
+// and one lost (1534 x 1728 x 2184 21 -> 26).
 //
-// Rows in dwords: of 126 drawn calls of that kind 68 come here, 1.22 times as fast as on the pass (behind which the re-layout read the weight
-// column by column) and the [K, N] decode kernel: 156 x 7168 x 21520 int4 bf16 208 -> 100 us, 85 x 11008 x 2456 37 -> 21, 53 x 1408 x 22192 28 -> 15.
+// Rows in dwords: of 126 drawn calls of that kind 68 come here, 1.22 times as fast as on the pass and the [K, N] decode kernel: 156 x 7168 x 21520 int4 bf16 208 -> 100 us, 85 x 11008 x 2456 37 -> 21, 53 x 1408 x 22192 28 -> 15.
 // Not where the estimates were wrong about them: from 257 rows with few k (510 x 1152 x 5744 21 there, 24 here), int8 up to 16 rows
 // (10 x 13184 x 3944 20.7 and 22.0).
 bool wide_wanted(const OpsnnWqmmArgs& a, WqWidePlan& pl)
 {
     if ((a.w_dtype != DT_I4 && a.w_dtype != DT_I8) || (a.x_dtype != DT_F16 && a.x_dtype != DT_BF16)) return false;
     if (a.scale_dtype != a.x_dtype || a.force_variant != 0 || (uintptr_t)a.x % 16 != 0) return false;
-    if (a.M > 512 || a.K % 32 != 0 || a.K < 256 || a.N < 256 || a.K >= (1ll << 23) || a.N >= (1ll << 24)) return false;
+    if (a.M > 1024 || a.K % 32 != 0 || a.K < 256 || a.N < 256 || a.K >= (1ll << 23) || a.N >= (1ll << 24)) return false;
     if (opsnn_wq_tile_min() <= 128 || !opsnn_wq_narrow_slabs()) return false;   // (test hooks of the other kernels)
     const WqForm f = wq_form(a);
     const int64_t codes = a.N * a.K;

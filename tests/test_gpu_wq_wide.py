@@ -34,7 +34,7 @@ def _check(m, M, K, N, group, nk, w_dt, x_dt, off):
 
 @pytest.mark.parametrize("M,K,N,group", [
     (1, 1056, 1024, 32), (16, 16416, 1056, 128), (17, 2080, 4128, 64), (33, 8192, 1056, 128), (64, 4160, 2080, 0),
-    (65, 1344, 1664, 64), (128, 1120, 1920, 256), (130, 2336, 1056, 128), (200, 1536, 1568, 0), (300, 4096, 544, 32),
+    (65, 1344, 1664, 64), (128, 1120, 1920, 256), (130, 2336, 1056, 128), (200, 1536, 1568, 0), (300, 4096, 544, 32), (900, 1056, 2080, 128),
     (1, 1056, 16416, 32), (17, 2080, 16416, 64), (40, 8192, 1056, 128),
 ])
 @pytest.mark.parametrize("w_dt,x_dt,off", KINDS)
@@ -55,7 +55,7 @@ def test_rows_of_k_in_whole_dwords(gpu, M, K, N, group, w_dt, x_dt, off):
 
 @pytest.mark.parametrize("M,K,N,group", [
     (9, 17280, 1873, 64), (20, 13568, 1730, 128), (40, 12544, 1793, 64), (64, 12928, 802, 32), (67, 14976, 1111, 128),
-    (130, 8832, 1026, 0), (257, 7040, 1090, 128), (257, 3104, 1090, 128),
+    (130, 8832, 1026, 0), (257, 7040, 1090, 128), (257, 3104, 1090, 128), (641, 1440, 5231, 32),
 ])
 @pytest.mark.parametrize("w_dt,x_dt,off", KINDS)
 def test_rows_of_n(gpu, M, K, N, group, w_dt, x_dt, off):
