@@ -63,32 +63,64 @@ static int launch16(const QgemmParams& p, const Gemm16Plan& pl, hipStream_t st)
     }
 }
 
-// Fewer 256 x 256 tiles than CUs: tile_plan (qmm_int8.hip), whose K tiles of 128 bytes take the same time here -- half as many
-// products per byte at half the rate.  Otherwise the estimate, in microseconds, of the two kernels for large shapes, fitted to
-// random operands, K = 4096 .. 18432 (profiles/tile_plans.txt: the pass and this product together, 41 calls of 100 .. 1999 rows, 37 within
-// 3 % of the fastest tile, the worst 8 % behind):
-//   four-wave kernel: 0.185 us per 32 columns of tile width and 64-element K tile, 8 us a round beside (4096^3: 99 us in one
-//   round of 256 x 256 tiles = 1.39 Pflop/s; 2048 x 4096 x 11008: 134 us in one round of 256 x 352);
-//   128 x 128 tiles: 0.65 us per K tile alone on a CU, 1.0 us for two that share one, 6 us beside.
-Gemm16Plan gemm16_plan(int64_t M, int64_t N, int64_t K)
+// One launch.  Fewer 256 x 256 tiles than CUs: tile_plan (qmm_int8.hip), whose K tiles of 128 bytes take the same time here -- half as
+// many products per byte at half the rate.  Otherwise the estimates, in microseconds, of the kernels for large shapes, fitted to
+// 36 drawn shapes of 613 .. 3108 rows on each of them (the product alone, steady state; median error 4 %, 3 % and 5 %):
+//   four-wave kernel, tiles of 256 x 32 fn: a K tile of 64 takes (0.137 + 0.057 * share of the CUs at work) fn, 5.8 a round beside
+//   (4096^3: 99 us in one round of 256 x 256 tiles = 1.39 Pflop/s; 2048 x 4096 x 11008: 134 us in one round of 256 x 352);
+//   eight waves on 256 x 256 tiles: 0.140 + 0.065 times 8, ahead of the four-wave form of that tile where there are several rounds;
+//   128 x 128 tiles, two on a CU: 1.14 a K tile.  (0.65 alone on a CU, 1.0 for two was the estimate before: 775 x 11264 x 22888 was
+//   planned on them with 472 us and took 611, the eight-wave kernel takes 557.)
+static Gemm16Plan one_launch(int64_t M, int64_t N, int64_t K)
 {
-    const int64_t cus = 256, kt = K / 64;
+    const int64_t cus = 256, kt = K / 64, tm = (M + 255) / 256;
     Gemm16Plan best;
     if (const TilePlan t = tile_plan(M, N, 2 * K, 1, true, false); t.variant) {
         best.cfg = t.variant; best.splits = t.splits; best.us = t.us;
         return best;
     }
     best.us = 1e30;
-    const int64_t tm = (M + 255) / 256;
-    for (int fn = 8; fn <= 11; fn++) {
-        const int64_t tiles = tm * ((N + 32 * fn - 1) / (32 * fn));
-        const double us = (double)((tiles + cus - 1) / cus) * (0.185 * fn * (double)kt + 8.0);
-        if (us < best.us) { best.cfg = fn; best.us = us; }
-    }
-    const int64_t t128 = ((M + 127) / 128) * ((N + 127) / 128), per_cu = (t128 + cus - 1) / cus;
-    const double us = (double)kt * ((double)(per_cu / 2) * 1.0 + (double)(per_cu % 2) * 0.65) + 6.0;
-    if (us < best.us) { best.cfg = OPSNN_VARIANT_I8_128; best.us = us; }
+    auto offer = [&](int cfg, double us) { if (us < best.us) { best.cfg = cfg; best.us = us; } };
+    auto rounds = [&](int64_t tiles, int64_t slots, double tile, double share, double beside) {
+        const int64_t full = tiles / slots, rest = tiles % slots;
+        return (double)full * ((double)kt * (tile + share) + beside) + (rest ? (double)kt * (tile + share * (double)rest / (double)slots) + beside : 0.0);
+    };
+    for (int fn = 8; fn <= 11; fn++) offer(fn, rounds(tm * ((N + 32 * fn - 1) / (32 * fn)), cus, 0.1372 * fn, 0.0567 * fn, 5.8) + 3.7);
+    offer(OPSNN_VARIANT_I8_256_W8_K128, rounds(tm * ((N + 255) / 256), cus, 1.122, 0.516, 5.6) - 6.0);
+    offer(OPSNN_VARIANT_I8_128, rounds(((M + 127) / 128) * ((N + 127) / 128), 2 * cus, 0.108, 1.031, 0.0) + 5.0);
     return best;
+}
+
+// Two launches where one ends in a round of the chip that is nearly empty: the columns (or rows) whose tiles make whole rounds, and the
+// rest on what is best for that.  Only where the estimate of one is a tenth above the time of its products in whole rounds, and where
+// two are estimated below 0.95 of it.  (A whole call with its pass over the weight, int4 bf16: 775 x 11264 x 22888 739 -> 502 us, 997 x 8512 x 23552
+// 543 -> 405, 1488 x 6912 x 15680 397 -> 309, 2877 x 3712 x 7424 177 -> 146; of 62 drawn calls that fill the chip nine are 1.16 to 1.28
+// times as fast and none is slower by more than 3 %.)
+Gemm16Plan gemm16_plan(int64_t M, int64_t N, int64_t K)
+{
+    Gemm16Plan best = one_launch(M, N, K);
+    const int64_t cus = 256, kt = K / 64, tm = (M + 255) / 256;
+    if (M <= 128 || N <= 128 || tm * ((N + 255) / 256) < cus) return best;   // (tile_plan chose)
+    if (best.us < 1.1 * ((double)kt * (double)M * (double)N * (0.194 / (256.0 * 32.0 * 256.0)) + 9.5)) return best;
+    const double most = 0.95 * best.us;
+    Gemm16Plan two = best;
+    two.us = most;
+    auto consider = [&](int cfg, int64_t m, int64_t n, double us) {
+        if (us >= two.us || (m == M && n == N)) return;
+        const Gemm16Plan rest = one_launch(m < M ? M - m : M, n < N ? N - n : N, K);
+        if (us + rest.us + 4.0 >= two.us) return;
+        two.cfg = cfg; two.splits = 1; two.us = us + rest.us + 4.0;
+        two.rows = m < M ? m : 0; two.cols = n < N ? n : 0;
+        two.rest_cfg = rest.cfg; two.rest_splits = rest.splits;
+    };
+    for (int fn = 8; fn <= 11; fn++) {
+        const int64_t width = 32 * fn, tn = (N + width - 1) / width, full = tm * tn / cus;
+        if (full < 1) continue;
+        const double us = (double)full * ((double)kt * 0.1939 * fn + 5.8) + 3.7;
+        if (const int64_t c = full * cus / tm; c * width < N) consider(fn, M, c * width, us);
+        if (const int64_t r = full * cus / tn; r > 0 && r * 256 < M) consider(fn, r * 256, N, us);
+    }
+    return two.us < most ? two : best;
 }
 
 int launch_gemm16(QgemmParams p, const Gemm16Plan& pl, bool bf16, float* part, hipStream_t st)
@@ -96,9 +128,22 @@ int launch_gemm16(QgemmParams p, const Gemm16Plan& pl, bool bf16, float* part, h
     if (p.KB % 128 != 0 || p.KB < 128) return OPSNN_NOT_TAKEN;
     if (((uintptr_t)p.a | (uintptr_t)p.b | (uint64_t)p.lda | (uint64_t)p.ldb) % 16) return OPSNN_NOT_TAKEN;
     if (256 * p.lda >= (1ll << 31) || 352 * p.ldb >= (1ll << 31)) return OPSNN_NOT_TAKEN;   // 32-bit offsets inside a tile
-    p.splits = pl.splits;
     p.part = (int32_t*)part;
-    return bf16 ? launch16<MODE_BF16>(p, pl, st) : launch16<MODE_F16>(p, pl, st);
+    auto launch = [&](const QgemmParams& q, const Gemm16Plan& of) { return bf16 ? launch16<MODE_BF16>(q, of, st) : launch16<MODE_F16>(q, of, st); };
+    QgemmParams q = p;
+    q.splits = pl.splits;
+    if (pl.rows) q.M = pl.rows;
+    if (pl.cols) q.N = pl.cols;
+    int rc = launch(q, pl);
+    if (rc != 0 || (!pl.rows && !pl.cols)) return rc;
+    Gemm16Plan rest;
+    rest.cfg = pl.rest_cfg; rest.splits = q.splits = pl.rest_splits;
+    q.M = p.M - pl.rows; q.N = p.N - pl.cols;
+    q.a = p.a + pl.rows * p.lda;
+    q.b = p.b + pl.cols * p.ldb;
+    q.out = (uint16_t*)p.out + pl.rows * p.ldc + pl.cols;
+    if (p.bias) q.bias = (const char*)p.bias + pl.cols * (p.bias_dt == DT_F32 ? 4 : 2);
+    return launch(q, rest);
 }
 
 }  // namespace opsnn
