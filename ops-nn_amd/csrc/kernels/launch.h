@@ -25,6 +25,8 @@ enum {
     OPSNN_VARIANT_FP8X_256x128 = 32,   // the tiles of the exact fp8 kernel (qmm_fp8_exact.hip)
     OPSNN_VARIANT_FP8X_128x256 = 33,
     OPSNN_VARIANT_FP8X_128x128 = 34,
+    OPSNN_VARIANT_FP8X_192x128 = 35,
+    OPSNN_VARIANT_FP8X_64x256 = 36,
 };
 
 #ifdef __cplusplus

@@ -15,8 +15,10 @@
 // (measured: bit-identical to the correctly rounded exact sum of 128 products in 99.5 % of cases, never further than
 // fp32 ascending-k summation), at half the matrix rate.
 //
-// Tiling: waves of 64 x 64 (4 x 4 fragments of 16 x 16), 4 x 2 of them -- 256 x 128 output tile per workgroup --, 2 x 4 or
-// 2 x 2: which, says fp8x_tile.  The operands stay
+// Tiling: eight waves, two a SIMD, 4 x 2 or 2 x 4 of them, each 64, 48 or 32 rows by 64 columns: output tiles of 256, 192 and 128 x 128,
+// 128 and 64 x 256; which, says fp8x_plan.  (A 128 x 128 tile of four waves of 64 x 64 before, one a SIMD, with nobody to issue while it waits:
+// 561 x 5120 x 6656 block scales 63 -> 47 us, 406 x 4480 x 6752 44.6 -> 36.4 on the same tiles; 192 rows: 2690 x 7296 x 3648 180 -> 152, MX
+// 3213 x 17920 x 2560 472 -> 360; 64: row / column scales 179 x 12544 x 17544 118 -> 99.)  The operands stay
 // e4m3 bytes on the way global -> LDS (16-byte asynchronous copies, rows XOR-swizzled) and LDS -> registers, exactly as
 // in qmm_fp8_block.hip; a lane's 32 bytes of a fragment become sixteen registers of fp16 pairs by sixteen
 // v_cvt_scalef32_pk_f16_fp8 (unit scale).  The x1 fragments are widened once per K tile and stay (64 registers), the
@@ -125,14 +127,16 @@ __device__ __forceinline__ float fp8x_rowcol_epilogue(int ep_mode, float v, floa
     return (v * csv) * rs + bias;
 }
 
-template <int WGM, int WGN, int OUT_DT, bool RC, int FMT = 0, bool MXS = false, bool SPLIT = false>
+// FM: 16-row x1 fragments of a wave, its tile being 16 FM x 64
+template <int WGM, int WGN, int FM, int OUT_DT, bool RC, int FMT = 0, bool MXS = false, bool SPLIT = false>
 __global__ __launch_bounds__(WGM * WGN * 64, 1) void qmm_fp8_exact_kernel(Fp8xParams p, int tiles_m, int tiles_n)
 {
     static_assert(!MXS || (RC && FMT == 0), "the MX mode is e4m3 x e4m3 with the row / column epilogue");
     constexpr bool AE5 = (FMT & 1) != 0, BE5 = (FMT & 2) != 0;
-    constexpr int BM = 64 * WGM, BN = 64 * WGN, BK = 128, NT = WGM * WGN * 64;
+    constexpr int BM = 16 * FM * WGM, BN = 64 * WGN, BK = 128, NT = WGM * WGN * 64;
     constexpr int CPR = BK / 16, RPW = 16 / CPR;
-    constexpr int TM = 64, TN = 64, FM = TM / 16, FN = TN / 16;
+    constexpr int TM = 16 * FM, TN = 64, FN = TN / 16;
+    static_assert(FM >= 2 && FM <= 4 && BM % 64 == 0 && NT / 8 <= BM && BM % (NT / 8) == 0, "whole copies");
     constexpr int A_BYTES = BM * BK, B_BYTES = BN * BK;
     constexpr bool SCC = !RC || MXS;                 // a 4-byte copy per lane rides with every K tile
     constexpr int SC_BYTES = SCC ? NT * 4 : 0;       // block scales: BM s1 floats + the s2 floats of the tile's n blocks; MX: four e8m0 bytes per tile row
@@ -319,10 +323,9 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void qmm_fp8_exact_kernel(Fp8xPa
         read_scales(smem);
         if constexpr (MXS) {
 #pragma unroll
-            for (int j = 0; j < FM; j++) {
-                mx_pow(a_sraw[j], a_lo[j], a_hi[j]);
-                mx_pow(b_sraw[j], b_lo[j], b_hi[j]);
-            }
+            for (int j = 0; j < FM; j++) mx_pow(a_sraw[j], a_lo[j], a_hi[j]);
+#pragma unroll
+            for (int i = 0; i < FN; i++) mx_pow(b_sraw[i], b_lo[i], b_hi[i]);
         }
 #pragma unroll
         for (int j = 0; j < FM; j++) {
@@ -407,9 +410,10 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void qmm_fp8_exact_kernel(Fp8xPa
                         acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fbc[i & 1][s], fa[j][s], acc[i][j], 0, 0, 0);
                     } else {
                         part[i & 1][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fbc[i & 1][s], fa[j][s], s == 0 ? v4f{0.0f, 0.0f, 0.0f, 0.0f} : part[i & 1][j], 0, 0, 0);
-                        // fold element j of x1 fragment s of the previous x2 fragment (for i == 0: the previous tile's last, with its scales)
-                        if (i > 0) acc[i - 1][s][j] = __builtin_fmaf(part[(i - 1) & 1][s][j], sc[s], acc[i - 1][s][j]);
-                        else acc[FN - 1][s][j] = __builtin_fmaf(part[1][s][j], scp[s], acc[FN - 1][s][j]);
+                        // fold one of the 4 FM elements of the previous x2 fragment (for i == 0: the previous tile's last, with its scales)
+                        const int fj = (s * FM + j) / 4, fe = (s * FM + j) % 4;
+                        if (i > 0) acc[i - 1][fj][fe] = __builtin_fmaf(part[(i - 1) & 1][fj][fe], sc[fj], acc[i - 1][fj][fe]);
+                        else acc[FN - 1][fj][fe] = __builtin_fmaf(part[1][fj][fe], scp[fj], acc[FN - 1][fj][fe]);
                     }
                     if constexpr (MXS) {
                         // the next tile's scale bytes were requested behind the barrier; every conversion that used the
@@ -417,13 +421,15 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void qmm_fp8_exact_kernel(Fp8xPa
                         // halves during the first)
                         if (i == FN - 1 && s == 1) {
                             mx_pow(a_sraw[j], a_lo[j], a_hi[j]);
-                            mx_pow(b_sraw[j], b_lo[j], b_hi[j]);
+#pragma unroll
+                            for (int b = j * FN / FM; b < (j + 1) * FN / FM; b++) mx_pow(b_sraw[b], b_lo[b], b_hi[b]);
                         }
                     }
-                    if (s >= 2) {   // next x2 fragment: half a K step per instruction
-                        const int idx = (s - 2) * 4 + j;
-                        const int nf = (i + 1) % FN;
-                        widen4(b_raw[idx], fbc[(i + 1) & 1][idx / 2], idx % 2, idx / 2 < 2 ? b_lo[nf] : b_hi[nf]);
+                    if (s >= 2) {   // next x2 fragment: its eight half K steps over these 2 FM instructions
+                        const int nf = (i + 1) % FN, at = (s - 2) * FM + j;
+#pragma unroll
+                        for (int idx = at * 4 / FM; idx < (at + 1) * 4 / FM; idx++)
+                            widen4(b_raw[idx], fbc[(i + 1) & 1][idx / 2], idx % 2, idx / 2 < 2 ? b_lo[nf] : b_hi[nf]);
                     }
                     if (i == FN - 1 && s >= 2)                // next tile's x1 fragments, K step s - 2 (low halves)
                         fa[j][s - 2] = widen_a(a_half[j][2 * (s - 2)], a_half[j][2 * (s - 2) + 1], j, s - 2);
@@ -590,10 +596,12 @@ __global__ __launch_bounds__(256) void fp8x_splitk_reduce_kernel(Fp8xParams p, i
 
 // The tile and the K segments.  A tile of 256 rows wastes up to half of its work just above a multiple of 128 rows, and an extra
 // round of the chip costs a whole round: 333 x 3584 x 18944 ran as 296 tiles of 256 x 128 in two rounds, 96 us (row / column
-// scales; block scales 102, MX 107); 222 of 128 x 256 take 55 (57, 62).  128 x 128 tiles fill the chip where the others are half
-// as many and would be cut along K: 1024 x 4096 x 4096 47 -> 39 us (48 -> 42, 49 -> 43).  The chosen one has the smallest
-// estimate: per K tile t0 + t1 * (share of the CUs at work) and a few us a round beside, fitted to 14 shapes of 140 .. 2048 rows;
-// of 45 calls 39 run within 3 % of the fastest tile or ahead of all (K cut), the worst 8 % behind (profiles/tile_plans.txt).  The row /
+// scales; block scales 102, MX 107); 222 of 128 x 256 take 55 (57, 62).  The chosen one has the smallest estimate: per K tile
+// t0 + t1 * (share of the CUs at work) and a few us a round beside, fitted to 270 launches of 63 shapes of 175 .. 3692 rows on every tile (median
+// error 2 %; the tile chosen by them takes 1.0006 (row / column), 1.001 (block) and 1.000 (MX) times the best one's time on average); the
+// smaller tiles are some 2 to 5 % slower than that where there are several rounds.  Of 240 drawn calls of 65 .. 4096 rows 88 are more than 5 %
+// faster with the tiles of 192 and 64 rows and the eight-wave 128 x 128 one, three slower (109 x 16640 x 15253 95 us on the many-rows stream kernel, 108
+// here), all 1.055 times as fast.  The row /
 // column form has no scales to apply in its loop.  The MX form's loop starts 4 us later than the others' (the first tile's conversions
 // and scales), and its second kernel has nothing but the sum to do: a short K is cut earlier (129 x 1024 x 1024 16.1 -> 14.3 us,
 // 129 x 1024 x 2080 17.0 -> 14.4 where the many-rows kernel had taken 16.1; 256 x 2048 x 6976 26.3 -> 24.2.  132 x 1152 x 6976 is left
@@ -602,35 +610,42 @@ Fp8xPlan fp8x_plan(int64_t M, int64_t N, int64_t K, int64_t batch, Fp8xForm form
 {
     const bool plain = form == FP8X_PLAIN, mx = form == FP8X_MX;
     const int64_t cus = 256, kt = (K + 127) / 128;   // (a K tail runs padded)
-    const double round_us = mx ? 8.0 : 4.0, split_us = mx ? 2.0 : 5.0, sums_per_us = mx ? 5.0e6 : 6.0e6;
+    const double start = mx ? 4.0 : 0.0, round_us = 4.0, split_us = mx ? 1.0 : 4.0, sums_per_us = mx ? 5.0e6 : 6.0e6;
     Fp8xPlan best{OPSNN_VARIANT_FP8X_256x128, 1, 1e30};
-    auto offer = [&](int tile, int64_t bm, int64_t bn, double t0, double t1) {
+    auto offer = [&](int tile, int64_t bm, int64_t bn, double t0, double t1, double many = 1.0) {
         const int64_t tiles = ((M + bm - 1) / bm) * ((N + bn - 1) / bn) * batch;
         for (int s = 1; s <= 16 && (s == 1 || (may_split && tiles * s <= cus && kt / s >= 4)); s++) {
             const double steps = (double)((kt + s - 1) / s);
             const int64_t full = tiles * s / cus, rest = tiles * s % cus;
-            double us = (double)full * (steps * (t0 + t1) + round_us) + (rest ? steps * (t0 + t1 * (double)rest / (double)cus) + round_us : 0.0);
+            double us = (double)full * (steps * (t0 + t1) + round_us) + (rest ? steps * (t0 + t1 * (double)rest / (double)cus) + round_us : 0.0) + start;
+            if (full > 1) us *= many;
             if (s > 1) us += split_us + 8.0 * s * (double)M * (double)N * (double)batch / sums_per_us;   // partial sums, second kernel
             if (us < best.us) best = {tile, s, us};
         }
     };
-    offer(OPSNN_VARIANT_FP8X_256x128, 256, 128, plain ? 1.25 : 1.37, plain ? 0.40 : 0.46);
-    offer(OPSNN_VARIANT_FP8X_128x256, 128, 256, plain ? 1.25 : 1.37, plain ? 0.40 : 0.46);
-    offer(OPSNN_VARIANT_FP8X_128x128, 128, 128, plain ? 0.92 : 1.08, 0.12);
+    static const double cost[3][4][2] = {   // by form: 256 x 128 and 128 x 256, 192 x 128, 128 x 128, 64 x 256
+        {{1.150, 0.238}, {0.864, 0.247}, {0.712, 0.121}, {0.787, 0.114}}, {{1.364, 0.247}, {1.128, 0.161}, {0.831, 0.102}, {0.877, 0.101}},
+        {{1.519, 0.044}, {1.165, 0.052}, {0.885, 0.032}, {0.887, 0.071}}};
+    const auto& c = cost[plain ? 0 : mx ? 2 : 1];
+    offer(OPSNN_VARIANT_FP8X_256x128, 256, 128, c[0][0], c[0][1]);
+    offer(OPSNN_VARIANT_FP8X_128x256, 128, 256, c[0][0], c[0][1]);
+    offer(OPSNN_VARIANT_FP8X_192x128, 192, 128, c[1][0], c[1][1], 1.02);
+    offer(OPSNN_VARIANT_FP8X_128x128, 128, 128, c[2][0], c[2][1], 1.05);
+    offer(OPSNN_VARIANT_FP8X_64x256, 64, 256, c[3][0], c[3][1], 1.05);
     return best;
 }
 
-template <int WGM, int WGN, int OUT_DT, bool RC, int FMT, bool MXS>
+template <int WGM, int WGN, int FM, int OUT_DT, bool RC, int FMT, bool MXS>
 static int launch_fp8_exact_tile(const Fp8xParams& p, int64_t batch, hipStream_t st)
 {
-    constexpr int BM = 64 * WGM, BN = 64 * WGN, NT = WGM * WGN * 64;
+    constexpr int BM = 16 * FM * WGM, BN = 64 * WGN, NT = WGM * WGN * 64;
     const int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
     dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch);
     const size_t lds = 3 * (size_t)((BM + BN) * 128 + ((RC && !MXS) ? 0 : NT * 4));
     note_route("fp8_exact", p.splits > 1 ? p.splits : 1);
     if (p.splits > 1) {   // K split over workgroups, then the sum of the partial sums, the epilogue and the rounding
         if (!p.part || p.splits > p.K / 128) return -1;
-        auto ks = qmm_fp8_exact_kernel<WGM, WGN, DT_F32, RC, FMT, MXS, true>;
+        auto ks = qmm_fp8_exact_kernel<WGM, WGN, FM, DT_F32, RC, FMT, MXS, true>;
         static std::atomic<uint64_t> attr_set_s{0};
         if (!device_flag_test(attr_set_s)) {
             hipError_t e = hipFuncSetAttribute((const void*)ks, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -644,7 +659,7 @@ static int launch_fp8_exact_tile(const Fp8xParams& p, int64_t batch, hipStream_t
         splitk_launch(batch * p.M, p.N, [&](auto w, dim3 g, dim3 b) { hipLaunchKernelGGL((fp8x_splitk_reduce_kernel<decltype(w)::value, RC>), g, b, 0, st, p, batch * p.M, OUT_DT); });
         return (int)hipGetLastError();
     }
-    auto k = qmm_fp8_exact_kernel<WGM, WGN, OUT_DT, RC, FMT, MXS>;
+    auto k = qmm_fp8_exact_kernel<WGM, WGN, FM, OUT_DT, RC, FMT, MXS>;
     static std::atomic<uint64_t> attr_set{0};   // one bit per device: the attribute belongs to the (kernel, device) pair
     if (!device_flag_test(attr_set)) {
         hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -659,11 +674,13 @@ template <int OUT_DT, bool RC, int FMT = 0, bool MXS = false>
 static int launch_fp8_exact(const Fp8xParams& p, int64_t batch, int force_variant, hipStream_t st)
 {
     int tile = p.splits > 1 ? p.tile : fp8x_plan(p.M, p.N, p.K, batch, MXS ? FP8X_MX : RC ? FP8X_PLAIN : FP8X_BLOCK, false).tile;
-    if (force_variant >= OPSNN_VARIANT_FP8X_256x128 && force_variant <= OPSNN_VARIANT_FP8X_128x128) tile = force_variant;
+    if (force_variant >= OPSNN_VARIANT_FP8X_256x128 && force_variant <= OPSNN_VARIANT_FP8X_64x256) tile = force_variant;
     if (256 * p.ldb >= (1ll << 32) || p.s2_cs < 0 || p.s2_cs >= (1ll << 29)) tile = OPSNN_VARIANT_FP8X_256x128;   // (32-bit offsets inside a tile)
-    if (tile == OPSNN_VARIANT_FP8X_128x128) return launch_fp8_exact_tile<2, 2, OUT_DT, RC, FMT, MXS>(p, batch, st);
-    if (tile == OPSNN_VARIANT_FP8X_128x256) return launch_fp8_exact_tile<2, 4, OUT_DT, RC, FMT, MXS>(p, batch, st);
-    return launch_fp8_exact_tile<4, 2, OUT_DT, RC, FMT, MXS>(p, batch, st);
+    if (tile == OPSNN_VARIANT_FP8X_128x128) return launch_fp8_exact_tile<4, 2, 2, OUT_DT, RC, FMT, MXS>(p, batch, st);
+    if (tile == OPSNN_VARIANT_FP8X_128x256) return launch_fp8_exact_tile<2, 4, 4, OUT_DT, RC, FMT, MXS>(p, batch, st);
+    if (tile == OPSNN_VARIANT_FP8X_192x128) return launch_fp8_exact_tile<4, 2, 3, OUT_DT, RC, FMT, MXS>(p, batch, st);
+    if (tile == OPSNN_VARIANT_FP8X_64x256) return launch_fp8_exact_tile<2, 4, 2, OUT_DT, RC, FMT, MXS>(p, batch, st);
+    return launch_fp8_exact_tile<4, 2, 4, OUT_DT, RC, FMT, MXS>(p, batch, st);
 }
 
 // fp8 e4m3 block scales (G-B, B-B), K-contiguous operands, K % 128 == 0, 16-bit or fp32 output, no bias.

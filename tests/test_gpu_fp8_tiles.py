@@ -59,3 +59,11 @@ def test_planned_block_scale_shapes(gpu, M, K, N):
     print(f"case fp8 block planned M={M} K={K} N={N}", flush=True)
     inp = cases.make_blockscale_inputs(m, M, K, N, M + N, True)
     _b16_bar(cases.run_blockscale_aclnn(m, inp, M, K, N, True, m.ACL_BF16), cases.oracle_blockscale(m, inp, M, K, N, True, m.ACL_BF16), orc.BF16, "planned tiles", K)
+
+
+@pytest.mark.parametrize("M,K,N", [(193, 384, 257), (191, 128, 390), (383, 1152, 1001), (65, 256, 129), (449, 640, 520)])
+@pytest.mark.parametrize("mode", ["rowcol", "block", "mx"])
+def test_tiles_of_192_and_64_rows(gpu, monkeypatch, mode, M, K, N):
+    """OPSNN_VARIANT_FP8X_192x128 and _64x256, as above."""
+    monkeypatch.setitem(globals(), "TILES", (32, 35, 36))
+    test_each_tile_gives_the_same_bits(gpu, mode, M, K, N)
