@@ -156,15 +156,16 @@ __device__ __forceinline__ float e8m0_to_f32(uint32_t b)
 }
 
 // The sum, in split order, of `splits` partial arrays [rows][N] that lie `slice` elements apart (the K split of every kernel
-// family), W neighbouring columns of one row per thread: emit(row, n0, v) with v[W].  W = 4 wants N % 4 == 0.  The row comes
+// family), W neighbouring columns of one row per thread: emit(row, n0, v) with v[W].  W = 4 wants N >= 4.  The row comes
 // from blockIdx.y and the columns from blockIdx.x, so no element costs a division (one 64-bit division is several dozen
 // instructions: with two or three of them per element the second kernel of a split took 106 us for 500 x 8192 outputs in two
 // slices, where the 50 MB it moves are 10 us), and up to eight slices are in flight at a time.
 template <int W, typename T, typename F>
 __device__ __forceinline__ void splitk_rows(const T* part, int splits, int64_t slice, int64_t rows, int64_t N, F&& emit)
 {
-    const int64_t n0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * W;
+    int64_t n0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * W;
     if (n0 >= N) return;
+    if (n0 + W > N) n0 = N - W;   // (the last columns of such an N twice, the same both times)
     for (int64_t row = blockIdx.y; row < rows; row += gridDim.y) {
         const T* at = part + row * N + n0;
         T v[W];
@@ -191,17 +192,20 @@ __device__ __forceinline__ void splitk_rows(const T* part, int splits, int64_t s
 }
 // Launches such a kernel: launch(W, grid, block).  Few outputs are a matter of latency, not of bytes: one column per thread
 // makes four times the waves (5 x 14464 x 1568 bf16 x int4, four slices: 12.4 us a call with four columns, 11.2 with one;
-// 16 x 4992 x 5248 fp8 14.6 / 14.1; 46 x 9856 x 4424 int8 18.0 / 17.2), and so it stays for an N that is no multiple of four
-// (13 x 1792 x 7273 11.3 / 10.3).  From 2^18 outputs the bytes count and four columns are ahead (64 x 4096 outputs 24.2 / 24.4,
-// 64 x 7168 50.4 / 51.0, 500 x 8192 77.3 / 88.4).
+// 16 x 4992 x 5248 fp8 14.6 / 14.1; 46 x 9856 x 4424 int8 18.0 / 17.2;
+// 13 x 1792 x 7273 11.3 / 10.3).  From 2^18 outputs the bytes count and four columns are ahead (64 x 4096 outputs 24.2 / 24.4,
+// 64 x 7168 50.4 / 51.0, 500 x 8192 77.3 / 88.4), rows that are no whole quads of columns included (197 x 9600 x 7841 fp8 64.9 -> 53.6 with their stores).
 template <typename L>
 inline void splitk_launch(int64_t rows, int64_t N, L&& launch)
 {
     const dim3 block(256);
     const unsigned gy = (unsigned)(rows < 65535 ? rows : 65535);
-    if (N % 4 == 0 && rows * N >= (1 << 18)) launch(std::integral_constant<int, 4>{}, dim3((unsigned)((N + 1023) / 1024), gy), block);
+    if (N >= 4 && rows * N >= (1 << 18)) launch(std::integral_constant<int, 4>{}, dim3((unsigned)((N + 1023) / 1024), gy), block);
     else launch(std::integral_constant<int, 1>{}, dim3((unsigned)((N + 255) / 256), gy), block);
 }
+// Stores of several columns go through __builtin_memcpy: rows of an odd N lie at odd addresses, where a 16-byte store of a lane is still
+// one instruction (stored element by element, eight instructions that each touch every line: int8 2599 x 1472 x 22345 208 -> 135 us, MXFP4
+// 2463 x 2048 x 15131 111 -> 62, fp8 block scales 2977 x 1024 x 26682 281 -> 187; 96 drawn calls of N % 8 != 0 and more than 100 rows 1.16).
 // W neighbouring outputs of one row, rounded to out_dt (bf16, fp16 or fp32), at element `at` of out
 template <int W>
 __device__ __forceinline__ void store_cols(void* out, int out_dt, int64_t at, const float (&v)[W])

@@ -109,7 +109,7 @@ inline double mxfp4_tiles_us(bool small, int64_t M, int64_t N, int64_t K, int64_
     const int64_t steps = ((K + 255) / 256 + splits - 1) / splits;
     double turns = (double)((wgs + 255) / 256);
     if (small && wgs > 256) turns = wgs <= 512 ? c.two : c.two * 0.5 * ((double)wgs / 512.0 + (double)((wgs + 511) / 512));
-    const double mb = (double)(M + N) * (double)K * (double)batch * 0.5e-6, out = (double)M * (double)N * (double)batch * (N % 4 ? 2e-6 : 1e-6);
+    const double mb = (double)(M + N) * (double)K * (double)batch * 0.5e-6, out = (double)M * (double)N * (double)batch * 1e-6;
     return c.start + turns * ((double)steps * c.step + c.round) + mb * c.mb + (splits > 1 ? c.reduce + c.reduce_mb * splits * out : 0.0) +
            (K % 128 && (small || splits > 1) ? c.copy + 2.0 * mb * c.copy_mb : 0.0);
 }

@@ -490,7 +490,6 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
         typedef std::conditional_t<MODE == MODE_I8, v4i, v4f> quad_t;
         typedef std::conditional_t<MODE == MODE_I8, int32_t, float> elem_t;
         elem_t* part = (elem_t*)p.part + (((int64_t)blockIdx.z * gridDim.y + bz) * p.M) * p.N;
-        const bool vec_ok4 = (p.N % 4) == 0 && ((uintptr_t)p.part % 16) == 0;
 #pragma unroll
         for (int j = 0; j < FM; j++) {
             const int64_t m = m0 + wm * TM + j * 32 + (lane & 31);
@@ -501,8 +500,8 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
                     const int64_t n = n0 + wn * TN + i * 32 + 8 * q + 4 * (lane >> 5);
                     if (m >= p.M) continue;
                     const quad_t o = {acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]};
-                    if (vec_ok4 && n + 3 < p.N) {
-                        *(quad_t*)(part + m * p.N + n) = o;
+                    if (n + 3 < p.N) {
+                        __builtin_memcpy(part + m * p.N + n, &o, 16);
                     } else {
 #pragma unroll
                         for (int e = 0; e < 4; e++)
@@ -570,7 +569,6 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
             }
         }
         __syncthreads();
-        const bool vec_ok = (p.ldc % 4) == 0 && ((uintptr_t)p.out % 16) == 0;
 #pragma unroll
         for (int j = 0; j < FM; j++) {
             const int64_t m = m0 + wm * TM + j * 32 + frow;
@@ -587,7 +585,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
                         for (int e = 0; e < 4; e++) o[e] = acc[i][j][q * 4 + e] + ib[e];
                         if (m < p.M) {
                             int32_t* dst = (int32_t*)p.out + (bz * p.M + m) * p.ldc + n;
-                            if (vec_ok && n + 3 < p.N) *(v4i*)dst = o;
+                            if (n + 3 < p.N) __builtin_memcpy(dst, &o, 16);
                             else {
 #pragma unroll
                                 for (int e = 0; e < 4; e++)
@@ -608,7 +606,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
                         }
                         if (m < p.M) {
                             int8_t* dst = (int8_t*)p.out + (bz * p.M + m) * p.ldc + n;
-                            if (vec_ok && n + 3 < p.N) *(uint32_t*)dst = packed;
+                            if (n + 3 < p.N) __builtin_memcpy(dst, &packed, 4);
                             else {
 #pragma unroll
                                 for (int e = 0; e < 4; e++)
@@ -625,7 +623,6 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
         // FLOAT output (the MX modes): like the integer outputs, straight from the registers, 16 bytes per lane
         static_assert(MX, "only the MX modes have a FLOAT output here");
         __syncthreads();
-        const bool vec_ok = (p.ldc % 4) == 0 && ((uintptr_t)p.out % 16) == 0;
 #pragma unroll
         for (int j = 0; j < FM; j++) {
             const int64_t m = m0 + wm * TM + j * 32 + frow;
@@ -641,7 +638,7 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
                     for (int e = 0; e < 4; e++) v[e] = acc[i][j][q * 4 + e] + fbv[e];
                     if (m < p.M) {
                         float* dst = (float*)p.out + (bz * p.M + m) * p.ldc + n;
-                        if (vec_ok && n + 3 < p.N) *(v4f*)dst = v;
+                        if (n + 3 < p.N) __builtin_memcpy(dst, &v, 16);
                         else {
 #pragma unroll
                             for (int e = 0; e < 4; e++)
@@ -669,7 +666,6 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
     constexpr int LPR = TN / 8;          // lanes per row when every lane moves 16 bytes
     constexpr int RPI2 = 64 / LPR;       // rows per store instruction
     const int er = lane / LPR, ec = lane % LPR;
-    const bool vec_ok = (p.ldc % 8) == 0 && ((uintptr_t)p.out % 16) == 0;
 #pragma unroll
     for (int j = 0; j < FM; j++) {
         const int ml = wm * TM + j * 32 + frow;
@@ -708,8 +704,8 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
             const int64_t m = m0 + wm * TM + j * 32 + row;
             const int64_t n = n0 + wn * TN + ec * 8;
             if (m < p.M) {
-                if (vec_ok && n + 7 < p.N) {
-                    *(v4i*)(out + m * p.ldc + n) = o;
+                if (n + 7 < p.N) {
+                    __builtin_memcpy(out + m * p.ldc + n, &o, 16);
                 } else {
                     const uint16_t* oe = (const uint16_t*)&o;
 #pragma unroll

@@ -396,7 +396,6 @@ __global__ __launch_bounds__(WGM * 128, 1) void qmm_fp8_block_kernel(Fp8BlkParam
     if constexpr (SPLIT) {
         // partial sums straight from the registers: a lane holds four consecutive columns of one row per fragment
         float* part = p.part + (((int64_t)blockIdx.z * gridDim.y + bz) * p.M) * p.N;
-        const bool vec_ok4 = (p.N % 4) == 0 && ((uintptr_t)p.part % 16) == 0;
 #pragma unroll
         for (int j = 0; j < FM; j++) {
             const int64_t m = m0 + wm * TM + j * 16 + frow;
@@ -404,8 +403,8 @@ __global__ __launch_bounds__(WGM * 128, 1) void qmm_fp8_block_kernel(Fp8BlkParam
             for (int i = 0; i < FN; i++) {
                 const int64_t n = n0 + wn * TN + i * 16 + 4 * fq;
                 if (m >= p.M) continue;
-                if (vec_ok4 && n + 3 < p.N) {
-                    *(v4f*)(part + m * p.N + n) = acc[i][j];
+                if (n + 3 < p.N) {
+                    __builtin_memcpy(part + m * p.N + n, &acc[i][j], 16);
                 } else {
 #pragma unroll
                     for (int r = 0; r < 4; r++)
@@ -421,7 +420,6 @@ __global__ __launch_bounds__(WGM * 128, 1) void qmm_fp8_block_kernel(Fp8BlkParam
     char* ep = smem + wave * (16 * EP_PITCH);
     static_assert(WGM * 2 * 16 * EP_PITCH <= STAGES * STAGE, "epilogue staging fits in the operand stages");
     uint16_t* out = (uint16_t*)p.out + bz * p.M * p.N;
-    const bool vec_ok = (p.N % 8) == 0 && ((uintptr_t)p.out % 16) == 0;
     const int er = lane >> 4, ec = lane & 15;
     float rs_j[FM];   // row / column scale mode: the scale of this lane's output row in each x1 fragment
     (void)rs_j;
@@ -464,8 +462,8 @@ __global__ __launch_bounds__(WGM * 128, 1) void qmm_fp8_block_kernel(Fp8BlkParam
             const int64_t m = m0 + wm * TM + j * 16 + row;
             const int64_t n = n0 + wn * TN + ec * 8;
             if (m < p.M) {
-                if (vec_ok && n + 7 < p.N) {
-                    *(v4i*)(out + m * p.N + n) = o;
+                if (n + 7 < p.N) {
+                    __builtin_memcpy(out + m * p.N + n, &o, 16);
                 } else {
                     const uint16_t* oe = (const uint16_t*)&o;
 #pragma unroll

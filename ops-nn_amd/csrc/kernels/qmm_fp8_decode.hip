@@ -177,7 +177,7 @@ __global__ __launch_bounds__(NW * 64) void fp8_block_decode_kernel(Fp8DecParams 
         } else {
             const v4us o = p.out_dt == DT_BF16 ? pack4_b16<DT_BF16>(sum) : pack4_b16<DT_F16>(sum);
             uint16_t* dst = (uint16_t*)p.out + (int64_t)nrow * p.N + n;
-            if ((p.N % 4) == 0 && ((uintptr_t)p.out % 8) == 0 && n + 3 < p.N) *(v4us*)dst = o;
+            if (n + 3 < p.N) __builtin_memcpy(dst, &o, 8);
             else {
 #pragma unroll
                 for (int r = 0; r < 4; r++)
@@ -369,7 +369,7 @@ __global__ __launch_bounds__(NW * 64) void mx_a8w4_decode_kernel(MxW4DecParams p
         }
         const v4us o = p.out_dt == DT_BF16 ? pack4_b16<DT_BF16>(sum) : pack4_b16<DT_F16>(sum);
         uint16_t* dst = (uint16_t*)p.out + (int64_t)nrow * p.N + n;
-        if ((p.N % 4) == 0 && ((uintptr_t)p.out % 8) == 0 && n + 3 < p.N) *(v4us*)dst = o;
+        if (n + 3 < p.N) __builtin_memcpy(dst, &o, 8);
         else {
 #pragma unroll
             for (int r = 0; r < 4; r++)
@@ -545,7 +545,7 @@ __global__ __launch_bounds__(NW * 64) void mx8_decode_kernel(Mx8DecParams p)
         } else {
             const v4us o = p.out_dt == DT_BF16 ? pack4_b16<DT_BF16>(sum) : pack4_b16<DT_F16>(sum);
             uint16_t* dst = (uint16_t*)p.out + (int64_t)nrow * p.N + n;
-            if ((p.N % 4) == 0 && ((uintptr_t)p.out % 8) == 0 && n + 3 < p.N) *(v4us*)dst = o;
+            if (n + 3 < p.N) __builtin_memcpy(dst, &o, 8);
             else {
 #pragma unroll
                 for (int r = 0; r < 4; r++)

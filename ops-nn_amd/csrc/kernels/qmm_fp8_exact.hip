@@ -478,7 +478,6 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void qmm_fp8_exact_kernel(Fp8xPa
     if constexpr (SPLIT) {
         // partial sums straight from the registers: a lane holds four consecutive columns of one row per fragment
         float* part = p.part + (((int64_t)blockIdx.z * gridDim.y + bz) * p.M) * p.N;
-        const bool vec_ok4 = (p.N % 4) == 0 && ((uintptr_t)p.part % 16) == 0;
 #pragma unroll
         for (int j = 0; j < FM; j++) {
             const int64_t m = m0 + wm * TM + j * 16 + frow;
@@ -486,8 +485,8 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void qmm_fp8_exact_kernel(Fp8xPa
             for (int i = 0; i < FN; i++) {
                 const int64_t n = n0 + wn * TN + i * 16 + 4 * fq;
                 if (m >= p.M) continue;
-                if (vec_ok4 && n + 3 < p.N) {
-                    *(v4f*)(part + m * p.N + n) = acc[i][j];
+                if (n + 3 < p.N) {
+                    __builtin_memcpy(part + m * p.N + n, &acc[i][j], 16);
                 } else {
 #pragma unroll
                     for (int r = 0; r < 4; r++)
@@ -507,7 +506,6 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void qmm_fp8_exact_kernel(Fp8xPa
     char* ep = smem + wave * (16 * EP_PITCH);
     static_assert(WGM * WGN * 16 * EP_PITCH <= STAGES * STAGE, "epilogue staging fits in the operand stages");
     uint16_t* out = (uint16_t*)p.out + bz * p.M * p.N;
-    const bool vec_ok = (p.N % 8) == 0 && ((uintptr_t)p.out % 16) == 0;
     const int er = lane >> 3, ec = lane & 7;
     // (the terms of a lane's 16 columns are fetched once, not once per row block)
     float rs_j[FM];
@@ -543,7 +541,7 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void qmm_fp8_exact_kernel(Fp8xPa
                 float* outf = (float*)p.out + bz * p.M * p.N;
                 const int64_t m = m0 + wm * TM + j * 16 + frow, n = n0 + wn * TN + i * 16 + 4 * fq;
                 if (m < p.M) {
-                    if ((p.N % 4) == 0 && ((uintptr_t)p.out % 16) == 0 && n + 3 < p.N) *(v4f*)(outf + m * p.N + n) = v;
+                    if (n + 3 < p.N) __builtin_memcpy(outf + m * p.N + n, &v, 16);
                     else {
 #pragma unroll
                         for (int r = 0; r < 4; r++)
@@ -562,8 +560,8 @@ __global__ __launch_bounds__(WGM * WGN * 64, 1) void qmm_fp8_exact_kernel(Fp8xPa
             const int64_t m = m0 + wm * TM + j * 16 + row;
             const int64_t n = n0 + wn * TN + ec * 8;
             if (m < p.M) {
-                if (vec_ok && n + 7 < p.N) {
-                    *(v4i*)(out + m * p.N + n) = o;
+                if (n + 7 < p.N) {
+                    __builtin_memcpy(out + m * p.N + n, &o, 16);
                 } else {
                     const uint16_t* oe = (const uint16_t*)&o;
 #pragma unroll

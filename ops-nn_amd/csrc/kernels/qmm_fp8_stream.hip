@@ -643,12 +643,12 @@ float decode_typical_us(const QmmDecodePlan& pl, bool mx, int64_t M, int64_t N, 
 // (524 calls of 65 .. 512 rows, median error 2 %).  K is cut there from 129 rows, MX from 65.
 float tiles_typical_us(int64_t M, int64_t N, int64_t K, Fp8xForm form, bool may_split)
 {
-    static const struct { float scale, start, out, out_odd, odd, split; } cost[3] = {   // by Fp8xForm
-        {0.978f, 1.85f, 0.38f, 1.42f, 1.09f, -0.96f}, {0.898f, 6.49f, 0.431f, 1.53f, 1.15f, -4.33f}, {1.03f, -0.78f, 0.434f, 2.02f, 0.29f, -1.2f}};
+    static const struct { float scale, start, out, split; } cost[3] = {   // by Fp8xForm
+        {0.978f, 1.85f, 0.38f, -0.96f}, {0.898f, 6.49f, 0.431f, -4.33f}, {1.03f, -0.78f, 0.434f, -1.2f}};
     const auto& c = cost[form];
     const Fp8xPlan pl = fp8x_plan(M, N, K, 1, form, may_split && (M > 128 || form == FP8X_MX));
     const float out_m = (float)M * (float)N * 1e-6f;
-    return c.scale * (float)pl.us + c.start + out_m * (c.out + (N % 4 ? c.out_odd * (float)pl.splits : 0.0f)) + (N % 8 ? c.odd : 0.0f) + (pl.splits > 1 ? c.split : 0.0f);
+    return c.scale * (float)pl.us + c.start + out_m * c.out + (pl.splits > 1 ? c.split : 0.0f);
 }
 template <int FORM>
 constexpr int narrow_per_cu(int mb, int nb)

@@ -226,7 +226,6 @@ __global__ __launch_bounds__(512) void kg_gemm_kernel(const int8_t* __restrict__
         }
     }
 
-    const bool vec_ok = (N % 4) == 0 && ((uintptr_t)out % 8) == 0;
 #pragma unroll
     for (int j = 0; j < FM; j++) {
         const int64_t m = m0 + wm * 64 + 16 * j + frow;
@@ -239,7 +238,7 @@ __global__ __launch_bounds__(512) void kg_gemm_kernel(const int8_t* __restrict__
 #pragma unroll
             for (int r = 0; r < 4; r++) v[r] = v[r] * s1;
             const v4us o = pack4_b16<OUT_DT>(v);
-            if (vec_ok && n + 3 < N) *(v4us*)(out + m * N + n) = o;
+            if (n + 3 < N) __builtin_memcpy(out + m * N + n, &o, 8);
             else {
 #pragma unroll
                 for (int r = 0; r < 4; r++)

@@ -451,7 +451,6 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
             }
         }
         __syncthreads();
-        const bool vec_ok = (p.ldc % 4) == 0 && ((uintptr_t)p.out % 16) == 0;
 #pragma unroll
         for (int j = 0; j < FM; j++) {
             const int64_t m = m0 + wm * TM + j * 16 + frow;
@@ -466,7 +465,7 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
                     for (int e = 0; e < 4; e++) o[e] = acc[i][j][e] + ib[e];
                     if (m < p.M) {
                         int32_t* dst = (int32_t*)p.out + (bz * p.M + m) * p.ldc + n;
-                        if (vec_ok && n + 3 < p.N) *(v4i*)dst = o;
+                        if (n + 3 < p.N) __builtin_memcpy(dst, &o, 16);
                         else {
 #pragma unroll
                             for (int e = 0; e < 4; e++)
@@ -487,7 +486,7 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
                     }
                     if (m < p.M) {
                         int8_t* dst = (int8_t*)p.out + (bz * p.M + m) * p.ldc + n;
-                        if (vec_ok && n + 3 < p.N) *(uint32_t*)dst = packed;
+                        if (n + 3 < p.N) __builtin_memcpy(dst, &packed, 4);
                         else {
 #pragma unroll
                             for (int e = 0; e < 4; e++)
@@ -506,7 +505,6 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
     // nothing hides the patch's write-to-read round trips; the int32 output of the same kernel, stored directly, beat the
     // 16-bit one although it writes twice the bytes).
     uint16_t* out = (uint16_t*)p.out + bz * p.M * p.ldc;
-    const bool vec_ok = (p.ldc % 4) == 0 && ((uintptr_t)p.out % 8) == 0;
 #pragma unroll
     for (int j = 0; j < FM; j++) {
         const float s1 = E16 ? 1.0f : sS1[wm * TM + j * 16 + frow];
@@ -532,7 +530,7 @@ __global__ __launch_bounds__(256, 1) void qgemm_i8_wide_kernel(QgemmParams p, in
             const v4us o4 = pack4_b16<OUT_DT>(v);
             const int64_t n = n0 + nl;
             if (m < p.M) {
-                if (vec_ok && n + 3 < p.N) *(v4us*)(out + m * p.ldc + n) = o4;
+                if (n + 3 < p.N) __builtin_memcpy(out + m * p.ldc + n, &o4, 8);
                 else {
 #pragma unroll
                     for (int e = 0; e < 4; e++)

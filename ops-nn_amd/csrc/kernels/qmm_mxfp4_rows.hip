@@ -175,7 +175,7 @@ __global__ __launch_bounds__(NW * 64) void mxfp4_rows_kernel(Mx4RowsParams p)
         } else {
             const v4us o = p.out_dt == DT_BF16 ? pack4_b16<DT_BF16>(sum) : pack4_b16<DT_F16>(sum);
             uint16_t* dst = (uint16_t*)p.out + at;
-            if ((p.N % 4) == 0 && ((uintptr_t)p.out % 8) == 0) *(v4us*)dst = o;   // (n < N: n + 3 too)
+            if (n + 3 < p.N) __builtin_memcpy(dst, &o, 8);
             else {
 #pragma unroll
                 for (int e = 0; e < 4; e++)

@@ -258,9 +258,9 @@ __global__ __launch_bounds__(256, 2) void wqmm_decode_kernel(WqParams p)
             if constexpr (XDT == DT_BF16) v[i] = bf16_to_f32(bf16_bits(v[i]));   // the golden rounds bf16 results twice (a no-op)
         }
         const int64_t nn0 = n0 + 4 * g;
-        if (nn0 + 3 < p.N && (p.N % 4) == 0) {
+        if (nn0 + 3 < p.N) {
             const v4us o = {bits_x<XDT>(v[0]), bits_x<XDT>(v[1]), bits_x<XDT>(v[2]), bits_x<XDT>(v[3])};
-            *(v4us*)(p.y + m * p.N + nn0) = o;
+            __builtin_memcpy(p.y + m * p.N + nn0, &o, 8);
         } else {
 #pragma unroll
             for (int i = 0; i < 4; i++)

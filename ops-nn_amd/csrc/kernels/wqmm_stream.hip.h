@@ -386,9 +386,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 8
             if constexpr (XDT == DT_BF16) v[i] = bf16_to_f32(bf16_bits(v[i]));   // the golden rounds bf16 results twice (a no-op)
         }
         const int64_t nn0 = n0 + 4 * g;
-        if (nn0 + 3 < p.N && (p.N % 4) == 0) {
+        if (nn0 + 3 < p.N) {
             const v4us o = {bits_x<XDT>(v[0]), bits_x<XDT>(v[1]), bits_x<XDT>(v[2]), bits_x<XDT>(v[3])};
-            *(v4us*)(p.y + m * p.N + nn0) = o;
+            __builtin_memcpy(p.y + m * p.N + nn0, &o, 8);
         } else {
 #pragma unroll
             for (int i = 0; i < 4; i++)
@@ -841,7 +841,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void w
                 if constexpr (XDT == DT_BF16) v[i] = bf16_to_f32(bf16_bits(v[i]));   // the golden rounds bf16 results twice (a no-op)
             }
             const v4us o = {bits_x<XDT>(v[0]), bits_x<XDT>(v[1]), bits_x<XDT>(v[2]), bits_x<XDT>(v[3])};
-            *(v4us*)(p.y + m * p.N + nn0) = o;   // N % 16 == 0 here: 8-byte aligned
+            __builtin_memcpy(p.y + m * p.N + nn0, &o, 8);   // N % 16 == 0 here: 8-byte aligned
         }
     }
 }
@@ -1024,9 +1024,9 @@ __global__ __launch_bounds__(256, 2) void wqmm_resx_kernel(WqParams p)
                     if constexpr (XDT == DT_BF16) v[i] = bf16_to_f32(bf16_bits(v[i]));
                 }
                 const int64_t nn0 = n0 + 4 * g;
-                if (nn0 + 3 < p.N && (p.N % 4) == 0) {
+                if (nn0 + 3 < p.N) {
                     const v4us o = {bits_x<XDT>(v[0]), bits_x<XDT>(v[1]), bits_x<XDT>(v[2]), bits_x<XDT>(v[3])};
-                    *(v4us*)(p.y + m * p.N + nn0) = o;
+                    __builtin_memcpy(p.y + m * p.N + nn0, &o, 8);
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; i++)
@@ -1251,8 +1251,8 @@ __global__ __launch_bounds__(NW * 64) void wqmm_xreg_kernel(WqParams p)
             if (nrow < rows && gridDim.y > 1) {   // K split: this segment's sums, as they are, for wq_splitk_reduce_kernel
                 const int64_t m = p.m_base + nrow, nn0 = (int64_t)rb * 16 + 4 * g;
                 float* dst = p.part + ((int64_t)blockIdx.y * p.M + m) * p.N + nn0;
-                if (nn0 + 3 < p.N && (p.N % 4) == 0 && ((uintptr_t)p.part % 16) == 0) {
-                    *(v4f*)dst = sum;
+                if (nn0 + 3 < p.N) {
+                    __builtin_memcpy(dst, &sum, 16);
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; i++)
@@ -1270,9 +1270,9 @@ __global__ __launch_bounds__(NW * 64) void wqmm_xreg_kernel(WqParams p)
                     if constexpr (XDT == DT_BF16) v[i] = bf16_to_f32(bf16_bits(v[i]));
                 }
                 const int64_t nn0 = n0 + 4 * g;
-                if (nn0 + 3 < p.N && (p.N % 4) == 0) {
+                if (nn0 + 3 < p.N) {
                     const v4us o = {bits_x<XDT>(v[0]), bits_x<XDT>(v[1]), bits_x<XDT>(v[2]), bits_x<XDT>(v[3])};
-                    *(v4us*)(p.y + m * p.N + nn0) = o;
+                    __builtin_memcpy(p.y + m * p.N + nn0, &o, 8);
                 } else {
 #pragma unroll
                     for (int i = 0; i < 4; i++)

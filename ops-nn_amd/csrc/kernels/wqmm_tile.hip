@@ -315,8 +315,8 @@ __global__ __launch_bounds__(512, 1) void wqmm_tile_kernel(WqParams p)
             }
             const v4us o = pack4_b16<XDT>(v);
             uint16_t* dst = p.y + (int64_t)m * p.N + n;
-            if (n + 3 < p.N && (p.N % 4) == 0) {
-                *(v4us*)dst = o;
+            if (n + 3 < p.N) {
+                __builtin_memcpy(dst, &o, 8);
             } else {
 #pragma unroll
                 for (int r = 0; r < 4; r++)

@@ -67,3 +67,33 @@ def test_tiles_of_192_and_64_rows(gpu, monkeypatch, mode, M, K, N):
     """OPSNN_VARIANT_FP8X_192x128 and _64x256, as above."""
     monkeypatch.setitem(globals(), "TILES", (32, 35, 36))
     test_each_tile_gives_the_same_bits(gpu, mode, M, K, N)
+
+
+@pytest.mark.parametrize("N,shift", [(264, 2), (263, 0), (261, 6)])
+def test_rows_of_the_output_at_any_address(gpu, N, shift):
+    """The output at an address that is no multiple of 16, in whole and in ragged rows: the bits of the aligned, whole-row call, and nothing
+    beside them."""
+    m = gpu
+    M, K = 131, 256
+    rng = np.random.default_rng(N)
+    x1, x2 = cases.gen_fp8(rng, (M, K)), cases.gen_fp8(rng, (264, K))
+    s1, s2 = rng.uniform(0.5, 2, M).astype(np.float32), rng.uniform(0.5, 2, 264).astype(np.float32)
+    d1, d2, ds1, ds2 = (m.DeviceBuffer(host=v) for v in (x1, x2, s1, s2))
+    outs = []
+    for n, off in ((264, 0), (N, shift)):
+        a = m.OpsnnQmmArgs()
+        a.M, a.N, a.K, a.batch = M, n, K, 1
+        a.x1, a.x2 = m.OpsnnMat(d1.ptr, K, 1, 0), m.OpsnnMat(d2.ptr, 1, K, 0)
+        a.x1_dtype = a.x2_dtype = m.ACL_FLOAT8_E4M3FN
+        a.x1_scale, a.x1_scale_len, a.x2_scale, a.x2_scale_dtype, a.x2_scale_len = ds1.ptr, M, ds2.ptr, m.ACL_FLOAT, n
+        host = np.full(M * n + 64, 0x5a5a, np.uint16)
+        d_out = m.DeviceBuffer(host=host)
+        a.out, a.out_dtype, a.force_variant = d_out.ptr + 32 + off, m.ACL_BF16, 32
+        print(f"case fp8 out N={n} shift={off}", flush=True)
+        assert m.lib().opsnnQmmTc(C.byref(a), None) == 0
+        m.check(m.lib().aclrtSynchronizeDevice(), "sync")
+        got = d_out.to_host(np.uint16, (M * n + 64,))
+        at = 16 + off // 2
+        assert (got[:at] == 0x5a5a).all() and (got[at + M * n:] == 0x5a5a).all()
+        outs.append(got[at:at + M * n].reshape(M, n))
+    assert np.array_equal(outs[1], outs[0][:, :N])
