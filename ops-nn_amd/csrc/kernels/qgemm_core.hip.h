@@ -87,6 +87,9 @@ __device__ __forceinline__ void async_copy4(const void* g, void* lds)
                                      (__attribute__((address_space(3))) void*)lds, 4, 0, 0);
 }
 
+// LDS of a stage's scales that travel in 4-byte copies, one or more a thread (threads past the tile's rows copy the last one again)
+constexpr int qg_sc_bytes(int rows, int bytes_per_row, int threads) { return (rows * bytes_per_row + 4 * threads - 1) / (4 * threads) * (4 * threads); }
+
 template <int MODE, int BM, int BN, int BK, int WGM, int WGN, int STAGES, int MINWG, bool KTAIL, int OUT_DT, bool SPLIT = false>
 __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams p, int tiles_m, int tiles_n)
 {
@@ -107,19 +110,19 @@ __global__ __launch_bounds__(WGM* WGN * 64, MINWG) void qgemm_kernel(QgemmParams
     // (a 4-byte copy per row costs a whole cache-line request for 4 useful bytes, as many requests as the operands
     // themselves); they live in a ring of two slots behind the operand stages.
     constexpr bool SC16 = MX && SCB == 8;
-    constexpr int SC_BYTES = (MX && !SC16) ? (BM + BN) * SCB : 0;
+    constexpr int SC_BYTES = (MX && !SC16) ? qg_sc_bytes(BM + BN, SCB, NT) : 0;
     constexpr int STAGE = A_BYTES + B_BYTES + SC_BYTES;
     constexpr int SC_RING = STAGES * STAGE;              // SC16: two slots of (BM + BN) * 16 bytes from here
     constexpr int RPI = NT / CPR;                // tile rows covered by one copy instruction of the workgroup
     constexpr int NA = BM / RPI, NB = BN / RPI;  // copy instructions per thread per tile
-    constexpr int NSC = MX ? (SC16 ? (BM + BN) / NT : (BM + BN) * SCW / NT) : 0; // scale-copy instructions per thread (SC16: per tile pair)
+    constexpr int NSC = MX ? (SC16 ? (BM + BN) / NT : SC_BYTES / (4 * NT)) : 0; // scale-copy instructions per thread (SC16: per tile pair)
     constexpr int CPT = NA + NB + (SC16 ? 0 : NSC);     // copies per tile that the wait counts step by
     static_assert(CPR == 8 || CPR == 4, "BK must be 64 or 128");
     static_assert(BM % RPI == 0 && BN % RPI == 0, "tile rows must be a multiple of the rows one copy pass covers");
     static_assert(STAGES >= 2 && STAGES * CPT < 64, "stage count");
     static_assert(KS % 2 == 0, "operand double buffer parity");
     static_assert(!MX || SCB == 4 || SCB == 8, "MX tiles carry four or eight scale bytes per row");
-    static_assert(!MX || (SC16 ? (BM + BN) % NT == 0 : ((BM + BN) * SCW) % NT == 0), "scale copy mapping");
+    static_assert(!SC16 || (BM + BN) % NT == 0, "scale copy mapping");
     static_assert(!SC16 || STAGES == 2, "paired scale copies are waited for with the two-stage counts");
     static_assert(!MX || !KTAIL || SC16, "MX: a K tail on the tiles whose scales travel in pairs only");
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -778,7 +781,7 @@ static int qgemm_launch_split_mx(const QgemmParams& p, int64_t batch, int out_dt
     if (!p.part || p.splits < 2 || (p.KB % (BK * U)) != 0 || p.splits > p.KB / BK / U / 2) return -1;
     int tiles_m = (int)((p.M + BM - 1) / BM), tiles_n = (int)((p.N + BN - 1) / BN);
     dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch, (unsigned)p.splits);
-    const size_t lds = SCB == 8 ? (size_t)STAGES * (BM + BN) * BK + 2 * (BM + BN) * 16 : (size_t)STAGES * ((BM + BN) * BK + (BM + BN) * SCB);
+    const size_t lds = SCB == 8 ? (size_t)STAGES * (BM + BN) * BK + 2 * (BM + BN) * 16 : (size_t)STAGES * ((BM + BN) * BK + qg_sc_bytes(BM + BN, SCB, WGM * WGN * 64));
     auto k = qgemm_kernel<MODE, BM, BN, BK, WGM, WGN, STAGES, MINWG, false, DT_F32, true>;
     static std::atomic<uint64_t> attr_set{0};
     if (!device_flag_test(attr_set)) {
@@ -825,7 +828,7 @@ static int qgemm_launch_one(const QgemmParams& p, int64_t batch, hipStream_t st)
     dim3 grid((unsigned)(tiles_m * tiles_n), (unsigned)batch);
     constexpr int SCB = MX ? BK / (MODE == MODE_MXFP8 ? 32 : 16) : 0;   // scale bytes per row per tile
     size_t lds = SCB == 8 ? (size_t)STAGES * (BM + BN) * BK + 2 * (BM + BN) * 16   // scales in their own ring of two slots
-                          : (size_t)STAGES * ((BM + BN) * BK + (BM + BN) * SCB);
+                          : (size_t)STAGES * ((BM + BN) * BK + qg_sc_bytes(BM + BN, SCB, WGM * WGN * 64));
     auto k = qgemm_kernel<MODE, BM, BN, BK, WGM, WGN, STAGES, MINWG, KTAIL, OUT_DT>;
     static std::atomic<uint64_t> attr_set{0};   // one bit per device: the attribute belongs to the (kernel, device) pair
     if (!device_flag_test(attr_set)) {

@@ -494,6 +494,14 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         if (split) { g.splits = sk.splits; g.part = (int32_t*)sk.part; }
         note_route(fp4_small ? "mxfp4_tiles_128" : "mxfp4_tiles_256", split ? sk.splits : 1);
         if (fp4_small) {
+            // Eight waves of 64 x 32 where a CU has at most two workgroups of at most 18 K tiles of 128 each, which are a matter of latency (235 x 1536 x
+            // 7335 9.5 -> 8.1 us, 8 x 93 x 1152 x 1208 8.7 -> 7.2, 71 x 5120 x 5688 in four segments 14.6 -> 13.8); four of 64 x 64, with fewer reads,
+            // where there is more (486 x 5760 x 3584 in two 28.1 so, 29.2 on eight; 8 x 36 x 3840 x 10048 50.5 and 55.5).
+            const int64_t cut = split ? sk.splits : 1, wgs = (a.M + 127) / 128 * ((a.N + 127) / 128) * a.batch * cut;
+            if (wgs <= 512 && a.K <= 18 * 128 * cut) {
+                if (split) return qgemm_launch_split_mx<MODE_MXFP4, 128, 128, 64, 2, 4, 4, 1>(g, a.batch, a.out_dtype, st);
+                return qgemm_launch<MODE_MXFP4, 128, 128, 64, 2, 4, 4, 1>(g, a.batch, a.out_dtype, st);
+            }
             if (split) return qgemm_launch_split_mx<MODE_MXFP4, 128, 128, 64, 2, 2, 4, 1>(g, a.batch, a.out_dtype, st);
             return qgemm_launch<MODE_MXFP4, 128, 128, 64, 2, 2, 4, 1>(g, a.batch, a.out_dtype, st);
         }

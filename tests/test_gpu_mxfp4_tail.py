@@ -71,3 +71,20 @@ def test_scale_rows_of_both_operands_beyond_the_grids_second_axis(gpu, M, K, N, 
     rows = None if K == 32 else [0, 1, 130, 255, 256, M - 1]   # (of the larger case some rows)
     check_close(got if rows is None else np.ascontiguousarray(got[:, rows]), cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, rows=rows), orc.BF16,
                 "mxfp4 tail, many scale rows")
+
+
+@pytest.mark.parametrize("M,K,N", [(40, 256, 65408), (97, 384, 65500)])
+def test_eight_waves_and_four_give_the_same_bits(gpu, M, K, N):
+    """128 x 128 tiles on either side of the line between eight and four waves, 512 workgroups: the same columns by themselves and with 128 more."""
+    m = gpu
+    inp = cases.make_mx_inputs(m, M, K, N + 128, N, True, True)
+    few = dict(inp)
+    few["x2"], few["s2"] = (np.ascontiguousarray(inp[k][:, :N]) for k in ("x2", "s2"))
+    print(f"case mxfp4 eight and four waves M={M} K={K} N={N}", flush=True)
+    got = []
+    for i, n in ((few, N), (inp, N + 128)):
+        got.append(cases.run_mx_aclnn(m, i, M, K, n, True, m.ACL_BF16, None).reshape(M, n)[:, :N])
+        assert route(m) == ("mxfp4_tiles_128", 1), route(m)
+    assert np.array_equal(got[0], got[1])
+    rows = [0, 31, 32, M - 1]
+    check_close(np.ascontiguousarray(got[0][rows]).reshape(1, 4, N), cases.oracle_mx(m, few, M, K, N, True, m.ACL_BF16, rows=rows), orc.BF16, "mxfp4 eight waves")
