@@ -1,4 +1,4 @@
-"""ctypes binding of libopsnn_amd.so (the C ABI declared under include/).
+"""Binding of libopsnn_amd.so (the C ABI declared under include/): ctypes, and a CPython extension for the calls of a serving loop.
 
 The host side of this library is C++; this module only exists so that the Python
 test-suite and the benchmark can drive the C entry points.  It adds no compute

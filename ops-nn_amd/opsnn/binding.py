@@ -1,4 +1,5 @@
-"""Thin ctypes layer over include/acl/acl.h, include/aclnnop/*.h and include/opsnn_kernels.h."""
+"""Thin layer over include/acl/acl.h, include/aclnnop/*.h and include/opsnn_kernels.h: ctypes, and csrc/python/calls.cpp for what a serving
+loop calls."""
 import ctypes as C
 import importlib.util
 import os
