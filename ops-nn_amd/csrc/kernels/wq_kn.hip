@@ -15,7 +15,8 @@
 // 41.4 -> 38.2).
 //
 // Work split: a workgroup is four waves on the same 16 CPL columns, each with a quarter of the workgroup's steps; blockIdx.y
-// cuts K into segments so that the chip has two workgroups per CU.  The waves' sums meet in LDS in a fixed order; with more
+// cuts K into segments so that the chip has two workgroups per CU.  With the table and an even count of segments, two of them are one workgroup of
+// eight waves, which halves the partial sums (16 x 8192 x 28672 42.0 -> 40.4 us, 9 x 12032 x 19648 43.9 -> 42.5, int8 10 x 15616 x 12352 47.3 -> 45.6).  The waves' sums meet in LDS in a fixed order; with more
 // than one segment they go to `part` as fp32 and wq_splitk_reduce_kernel adds the segments in order.
 #include "launch.h"
 #include "wq_cost.h"
@@ -50,8 +51,8 @@ static WqKnPlan kn_plan(int wbits, int64_t M, int64_t N, int64_t K)
     return pl;
 }
 
-template <int XDT, int WBITS, int MB, bool HAS_OFF, bool TABLE>
-__global__ __launch_bounds__(256, 2) void wq_kn_kernel(WqParams p, int splits, int window)
+template <int XDT, int WBITS, int MB, bool HAS_OFF, bool TABLE, int NW>
+__global__ __launch_bounds__(64 * NW, 8 / NW) void wq_kn_kernel(WqParams p, int splits, int window)
 {
     constexpr int CPL = kn_cpl(MB);
     constexpr int DW = CPL * WBITS / 32;          // dwords of codes per lane and row: 1, 2 or 4
@@ -66,7 +67,7 @@ __global__ __launch_bounds__(256, 2) void wq_kn_kernel(WqParams p, int splits, i
     const int64_t nl = strip0 + r * CPL, n = nl + CPL <= p.N ? nl : p.N - CPL;
     const int steps = (int)(p.K / 32);
     const int s0 = (int)((int64_t)blockIdx.y * steps / splits), s1 = (int)((int64_t)(blockIdx.y + 1) * steps / splits);
-    const int w0 = s0 + (s1 - s0) * wave / 4, w1 = s0 + (s1 - s0) * (wave + 1) / 4;   // this wave's steps
+    const int w0 = s0 + (s1 - s0) * wave / NW, w1 = s0 + (s1 - s0) * (wave + 1) / NW;   // this wave's steps
 
     const uint8_t* wbase = p.w + (int64_t)8 * q * p.ldw + n * WBITS / 8;
     const int64_t ldw = p.ldw;
@@ -223,7 +224,7 @@ __global__ __launch_bounds__(256, 2) void wq_kn_kernel(WqParams p, int splits, i
         }
     }
 
-    if (!sum_of_four_waves(acc, red, wave, lane)) return;
+    if (!sum_of_waves<NW>(acc, red, wave, lane)) return;
 
     // acc[c][b][i] is out[m = 16 b + lane % 16][column c of the weight rows' lane 4 q + i]: CPL neighbouring columns per i
 #pragma unroll
@@ -260,17 +261,17 @@ __global__ __launch_bounds__(256, 2) void wq_kn_kernel(WqParams p, int splits, i
     }
 }
 
-template <int XDT, int WBITS, int MB, bool HAS_OFF, bool TABLE = false>
+template <int XDT, int WBITS, int MB, bool HAS_OFF, bool TABLE = false, int NW = 4>
 static int launch_kn_one(const WqParams& p, int splits, hipStream_t st)
 {
     constexpr int CPL = kn_cpl(MB), PF = kn_pf(WBITS, MB);
     const dim3 grid((unsigned)((p.N + 16 * CPL - 1) / (16 * CPL)), (unsigned)splits);
-    constexpr size_t lds_sum = (size_t)2 * CPL * MB * 4 * 64 * 4, lds_tab = TABLE ? (size_t)4 * KN_GROUPS * 32 * CPL * (HAS_OFF ? 2 : 1) : 0;
+    constexpr size_t lds_sum = (size_t)NW / 2 * CPL * MB * 4 * 64 * 4, lds_tab = TABLE ? (size_t)NW * KN_GROUPS * 32 * CPL * (HAS_OFF ? 2 : 1) : 0;
     constexpr size_t lds = lds_sum > lds_tab ? lds_sum : lds_tab;
     // steps whose groups fit a table wherever they start, in whole rounds of the loop
     const int64_t steps = p.K / 32, fit = p.group >= p.K ? steps + PF : (KN_GROUPS - (p.group > 32)) * p.group / 32;
     const int window = (int)((fit < steps + PF ? fit : steps + PF) / PF * PF);
-    auto k = wq_kn_kernel<XDT, WBITS, MB, HAS_OFF, TABLE>;
+    auto k = wq_kn_kernel<XDT, WBITS, MB, HAS_OFF, TABLE, NW>;
     static std::atomic<uint64_t> attr_set{0};   // one bit per device: the attribute belongs to the (kernel, device) pair
     if (!device_flag_test(attr_set)) {
         hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -278,7 +279,7 @@ static int launch_kn_one(const WqParams& p, int splits, hipStream_t st)
         device_flag_set(attr_set);
     }
     note_route(TABLE ? "wq_kn_table" : "wq_kn", splits);
-    hipLaunchKernelGGL(k, grid, dim3(256), lds, st, p, splits, window);
+    hipLaunchKernelGGL(k, grid, dim3(64 * NW), lds, st, p, splits, window);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
     launch_wq_splitk_reduce(p, splits, XDT, st);
     return (int)hipGetLastError();
@@ -288,6 +289,7 @@ static int launch_kn_mb(const WqParams& p, const WqKnPlan& pl, hipStream_t st)
 {
     if (pl.mb == 1) {
         // (the table pays for itself from some twelve steps a wave: 16 x 8192 x 28672, sixteen, 44.4 -> 41.3 us; 4 x 3072 x 1872, six, 9.0 -> 10.4)
+        if (p.K / 32 >= 48 * pl.splits && pl.splits % 2 == 0) return launch_kn_one<XDT, WBITS, 1, HAS_OFF, true, 8>(p, pl.splits / 2, st);
         if (p.K / 32 >= 48 * pl.splits) return launch_kn_one<XDT, WBITS, 1, HAS_OFF, true>(p, pl.splits, st);
         return launch_kn_one<XDT, WBITS, 1, HAS_OFF>(p, pl.splits, st);
     }

@@ -163,7 +163,7 @@ __global__ __launch_bounds__(256, 2) void wq_nk_kernel(WqParams p, int splits, i
     }
 
     __syncthreads();   // the scale table makes room
-    if (!sum_of_four_waves(acc, dyn, wave, lane)) return;
+    if (!sum_of_waves(acc, dyn, wave, lane)) return;
 
     // acc[j][b][i] is out[m = 16 b + lane % 16][n = n0 + 16 j + 4 q + i]
 #pragma unroll

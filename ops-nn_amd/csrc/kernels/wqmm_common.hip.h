@@ -97,10 +97,10 @@ __device__ __forceinline__ float dequant_one(float w, float off, float sc, bool 
 }
 
 
-// The sums of a workgroup's four waves in a fixed order, (0 + 2) + (1 + 3), through 2 * A * B * 256 floats of LDS: true in wave 0, which
-// then holds them.
-template <int A, int B>
-__device__ __forceinline__ bool sum_of_four_waves(v4f (&acc)[A][B], float* red, int wave, int lane)
+// The sums of a workgroup's NW waves in a fixed order, halves of them onto the others ((0 + 2) + (1 + 3) of four), through NW / 2 * A * B * 256
+// floats of LDS: true in wave 0, which then holds them.
+template <int NW = 4, int A, int B>
+__device__ __forceinline__ bool sum_of_waves(v4f (&acc)[A][B], float* red, int wave, int lane)
 {
     constexpr int SUMS = A * B * 4 * 64;
     auto park = [&](float* to) {
@@ -115,10 +115,13 @@ __device__ __forceinline__ bool sum_of_four_waves(v4f (&acc)[A][B], float* red, 
 #pragma unroll
             for (int b = 0; b < B; b++) acc[i][b] = acc[i][b] + *(const v4f*)(from + ((i * B + b) * 64 + lane) * 4);
     };
-    if (wave >= 2) park(red + (wave - 2) * SUMS);
-    __syncthreads();
-    if (wave < 2) add(red + wave * SUMS);
-    __syncthreads();
+#pragma unroll
+    for (int h = NW / 2; h > 1; h /= 2) {
+        if (wave >= h && wave < 2 * h) park(red + (wave - h) * SUMS);
+        __syncthreads();
+        if (wave < h) add(red + wave * SUMS);
+        __syncthreads();
+    }
     if (wave == 1) park(red);
     __syncthreads();
     if (wave != 0) return false;

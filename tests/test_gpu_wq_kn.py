@@ -57,3 +57,18 @@ def test_table_of_scales_in_several_windows(gpu, w_dt, x_dt, off):
     got = cases.run_wq_aclnn(m, inp, M, K, N)
     assert m.lib().opsnnDebugLastRoute(None) == b"wq_kn_table"
     _b16_bar(got, cases.oracle_wq(m, inp, M, K, N), orc.F16 if x_dt == "f16" else orc.BF16, "kn windows", K)
+
+
+@pytest.mark.parametrize("w_dt,x_dt,off", [("i4", "f16", True), ("i4", "bf16", False), ("i8", "bf16", True)])
+@pytest.mark.parametrize("M,K,N,group", [(16, 6176, 28674, 128), (5, 6432, 28416, 0)])
+def test_eight_waves(gpu, M, K, N, group, w_dt, x_dt, off):
+    """An even count of segments with the table of scales: two segments a workgroup of eight waves; steps that are no multiple of the waves', a
+    ragged last strip of columns."""
+    from test_gpu_routes import route
+    m = gpu
+    xd = m.ACL_FLOAT16 if x_dt == "f16" else m.ACL_BF16
+    inp = cases.make_wq_inputs(m, M, K, N, M + K, xd, m.ACL_INT4 if w_dt == "i4" else m.ACL_INT8, group, False, off, xd if M % 2 else None)
+    print(f"case kn eight waves M={M} K={K} N={N} g={group} {w_dt} {x_dt}", flush=True)
+    got = cases.run_wq_aclnn(m, inp, M, K, N)
+    assert route(m) == ("wq_kn_table", 2), route(m)
+    _b16_bar(got, cases.oracle_wq(m, inp, M, K, N), orc.F16 if x_dt == "f16" else orc.BF16, "kn eight waves", K)
