@@ -3,6 +3,7 @@ loop calls."""
 import ctypes as C
 import importlib.util
 import os
+import threading
 
 import numpy as np
 
@@ -211,19 +212,23 @@ _SIGS = {
 EXPORTED_SYMBOLS = sorted(_SIGS)
 
 _lib = None
+_lib_lock = threading.Lock()
 
 
 def lib():
     """The loaded shared library.  There is no fallback: a missing build is an error."""
     global _lib
     if _lib is None:
-        if not os.path.exists(LIB_PATH):
-            raise RuntimeError(f"{LIB_PATH} is not built; run `python -c 'import __graft_entry__ as g; g.build()'`")
-        _lib = C.CDLL(LIB_PATH)
-        for name, (res, args) in _SIGS.items():
-            fn = getattr(_lib, name)
-            fn.restype, fn.argtypes = res, args
-        _bind_calls(_lib)
+        with _lib_lock:
+            if _lib is None:
+                if not os.path.exists(LIB_PATH):
+                    raise RuntimeError(f"{LIB_PATH} is not built; run `python -c 'import __graft_entry__ as g; g.build()'`")
+                library = C.CDLL(LIB_PATH)
+                for name, (res, args) in _SIGS.items():
+                    fn = getattr(library, name)
+                    fn.restype, fn.argtypes = res, args
+                _bind_calls(library)
+                _lib = library   # (last: another thread, and a call after one that failed here, finds all of it or none)
     return _lib
 
 

@@ -1,6 +1,7 @@
 """The binding's extension (csrc/python/calls.cpp) against the same entry points called through ctypes: statuses, workspace sizes and
 whether an executor comes back, for calls that are accepted and for calls that are refused; and views of up to eight dims."""
 import ctypes as C
+import threading
 
 import pytest
 
@@ -98,3 +99,37 @@ def test_an_extent_in_any_place_is_seen(rank):
         assert m.dynamic_quant_get_workspace(x, _t(other, m.ACL_INT8), s)[0] != 0, at
         if at < rank - 1:
             assert m.dynamic_quant_get_workspace(x, y, _t(other[:-1], m.ACL_FLOAT))[0] != 0, at
+
+
+def test_a_binding_that_failed_leaves_nothing_behind(monkeypatch):
+    def fail(library):
+        raise OSError("not this one")
+
+    monkeypatch.setattr(m.binding, "_lib", None)
+    monkeypatch.setattr(m.binding, "_bind_calls", fail)
+    for _ in range(2):
+        with pytest.raises(OSError, match="not this one"):
+            m.lib()
+
+
+def test_threads_find_the_library_whole(monkeypatch):
+    bind, entered, go, seen = m.binding._bind_calls, threading.Event(), threading.Event(), []
+
+    def slow(library):
+        entered.set()
+        assert go.wait(30)
+        bind(library)
+
+    monkeypatch.setattr(m.binding, "_lib", None)
+    monkeypatch.setattr(m.binding, "_bind_calls", slow)
+    first = threading.Thread(target=lambda: seen.append(m.lib()))
+    first.start()
+    assert entered.wait(30)
+    second = threading.Thread(target=lambda: seen.append(m.lib()))
+    second.start()
+    second.join(0.2)
+    early = list(seen)
+    go.set()
+    first.join(30)
+    second.join(30)
+    assert early == [] and len(seen) == 2 and seen[0] is seen[1]
