@@ -19,84 +19,59 @@
 
 namespace {
 
-PyObject *g_handle, *g_value;   // interned attribute names
+PyObject* g_handle;   // interned attribute name
 
-// Address of an argument: None, an int, or a ctypes pointer-sized value.  False with a Python error set otherwise.
+// Of every argument only the plain form is taken here -- None, an int, a float, bytes, a Tensor whose handle is one of the first two --, with
+// the value that ctypes makes of it.  Anything else is left to ctypes, which knows what each parameter accepts: a phase 1 function then
+// returns NotImplemented, phase 2 calls the ctypes function itself.  The readers below return false for that, without a Python error.
+
+// None or an int, of which the low bits count.
 bool as_pointer(PyObject* o, void** out)
 {
     if (o == Py_None) { *out = nullptr; return true; }
-    if (PyLong_Check(o)) {
-        *out = (void*)(uintptr_t)PyLong_AsUnsignedLongLongMask(o);
-        return !PyErr_Occurred();
-    }
-    PyObject* v = PyObject_GetAttr(o, g_value);
-    if (!v) return false;
-    const bool ok = (v == Py_None || PyLong_Check(v)) && as_pointer(v, out);
-    if (!ok && !PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "an address (int or None) is wanted");
-    Py_DECREF(v);
-    return ok;
+    if (!PyLong_Check(o)) return false;
+    *out = (void*)(uintptr_t)PyLong_AsUnsignedLongLongMask(o);
+    return true;
 }
-// The handle of a Tensor, or null for None.
-bool as_tensor(PyObject* o, const aclTensor** out)
-{
-    if (o == Py_None) { *out = nullptr; return true; }
-    PyObject* h = PyObject_GetAttr(o, g_handle);
-    if (!h) return false;
-    void* p = nullptr;
-    const bool ok = as_pointer(h, &p);
-    Py_DECREF(h);
-    *out = (const aclTensor*)p;
-    return ok;
-}
-// (a ctypes number stands for its value, as it does for ctypes)
-PyObject* plain(PyObject* o) { return PyLong_Check(o) || PyFloat_Check(o) || !PyObject_HasAttr(o, g_value) ? Py_NewRef(o) : PyObject_GetAttr(o, g_value); }
 bool as_int64(PyObject* o, int64_t* out)
 {
-    PyObject* v = plain(o);
-    if (!v) return false;
-    *out = (int64_t)PyLong_AsLongLong(v);
-    Py_DECREF(v);
-    return *out != -1 || !PyErr_Occurred();
+    if (!PyLong_Check(o)) return false;
+    *out = (int64_t)PyLong_AsUnsignedLongLongMask(o);
+    return true;
 }
 bool as_double(PyObject* o, double* out)
 {
-    PyObject* v = plain(o);
-    if (!v) return false;
-    *out = PyFloat_AsDouble(v);
-    Py_DECREF(v);
-    return *out != -1.0 || !PyErr_Occurred();
+    if (!PyFloat_Check(o)) return false;
+    *out = PyFloat_AS_DOUBLE(o);
+    return true;
 }
 bool as_flag(PyObject* o, bool* out)
 {
-    const int t = PyObject_IsTrue(o);
-    *out = t != 0;
-    return t >= 0;
+    *out = o == Py_True;
+    return PyBool_Check(o);
 }
-// Bytes, None or a ctypes string, whose copy lives as long as the object.
-struct Text {
-    const char* c = nullptr;
-    PyObject* held = nullptr;
-    ~Text() { Py_XDECREF(held); }
-    bool from(PyObject* o)
-    {
-        if (o == Py_None) return true;
-        held = PyBytes_Check(o) ? Py_NewRef(o) : PyObject_GetAttr(o, g_value);
-        if (!held || held == Py_None) return held != nullptr;
-        c = PyBytes_AsString(held);
-        return c != nullptr;
-    }
-};
-bool tensors(PyObject* const* args, int n, const aclTensor** t)
+// (lives as long as the argument)
+bool as_text(PyObject* o, const char** out)
 {
-    for (int i = 0; i < n; i++)
-        if (!as_tensor(args[i], &t[i])) return false;
+    if (o == Py_None) { *out = nullptr; return true; }
+    if (!PyBytes_Check(o)) return false;
+    *out = PyBytes_AS_STRING(o);
     return true;
 }
-bool count(Py_ssize_t n, Py_ssize_t want)
+bool tensors(PyObject* const* args, int n, const aclTensor** t)
 {
-    if (n == want) return true;
-    PyErr_Format(PyExc_TypeError, "%zd arguments are wanted, %zd given", want, n);
-    return false;
+    for (int i = 0; i < n; i++) {
+        t[i] = nullptr;
+        if (args[i] == Py_None) continue;
+        PyObject* h = PyObject_GetAttr(args[i], g_handle);
+        if (!h) { PyErr_Clear(); return false; }
+        void* p = nullptr;
+        const bool ok = as_pointer(h, &p);
+        Py_DECREF(h);
+        if (!ok) return false;
+        t[i] = (const aclTensor*)p;
+    }
+    return true;
 }
 PyObject* phase1_result(aclnnStatus rc, uint64_t ws, const aclOpExecutor* ex)
 {
@@ -122,9 +97,12 @@ struct Entry {
 PyObject* bind(PyObject*, PyObject* const* args, Py_ssize_t n)
 {
     void* p[6];
-    if (!count(n, 6)) return nullptr;
-    for (int i = 0; i < 6; i++)
-        if (!as_pointer(args[i], &p[i])) return nullptr;
+    bool ok = n == 6;
+    for (int i = 0; ok && i < 6; i++) ok = as_pointer(args[i], &p[i]) && p[i];
+    if (!ok) {
+        PyErr_SetString(PyExc_TypeError, "six addresses are wanted");
+        return nullptr;
+    }
     g_entry.qmm = (decltype(g_entry.qmm))p[0];
     g_entry.qmm_nz = (decltype(g_entry.qmm_nz))p[1];
     g_entry.wqmm = (decltype(g_entry.wqmm))p[2];
@@ -140,8 +118,8 @@ PyObject* qmm(PyObject*, PyObject* const* args, Py_ssize_t n)
     const aclTensor* t[10];
     bool ta, tb, want_ws, want_ex, nz;
     int64_t group;
-    if (!count(n, 16) || !tensors(args, 10, t) || !as_flag(args[10], &ta) || !as_flag(args[11], &tb) || !as_int64(args[12], &group) ||
-        !as_flag(args[13], &want_ws) || !as_flag(args[14], &want_ex) || !as_flag(args[15], &nz)) return nullptr;
+    if (n != 16 || !tensors(args, 10, t) || !as_flag(args[10], &ta) || !as_flag(args[11], &tb) || !as_int64(args[12], &group) ||
+        !as_flag(args[13], &want_ws) || !as_flag(args[14], &want_ex) || !as_flag(args[15], &nz)) Py_RETURN_NOTIMPLEMENTED;
     uint64_t ws = 0;
     aclOpExecutor* ex = nullptr;
     aclnnStatus rc;
@@ -156,7 +134,7 @@ PyObject* wqmm(PyObject*, PyObject* const* args, Py_ssize_t n)
 {
     const aclTensor* t[8];
     int64_t group;
-    if (!count(n, 9) || !tensors(args, 8, t) || !as_int64(args[8], &group)) return nullptr;
+    if (n != 9 || !tensors(args, 8, t) || !as_int64(args[8], &group)) Py_RETURN_NOTIMPLEMENTED;
     uint64_t ws = 0;
     aclOpExecutor* ex = nullptr;
     aclnnStatus rc;
@@ -169,7 +147,7 @@ PyObject* wqmm(PyObject*, PyObject* const* args, Py_ssize_t n)
 PyObject* dynamic_quant(PyObject*, PyObject* const* args, Py_ssize_t n)
 {
     const aclTensor* t[4];
-    if (!count(n, 4) || !tensors(args, 4, t)) return nullptr;
+    if (n != 4 || !tensors(args, 4, t)) Py_RETURN_NOTIMPLEMENTED;
     uint64_t ws = 0;
     aclOpExecutor* ex = nullptr;
     aclnnStatus rc;
@@ -182,17 +160,17 @@ PyObject* dynamic_quant(PyObject*, PyObject* const* args, Py_ssize_t n)
 PyObject* block_quant(PyObject*, PyObject* const* args, Py_ssize_t n)
 {
     const aclTensor* t[3];
-    Text mode;
+    const char* mode;
     double min_scale;
     int64_t v[3];
-    if (!count(n, 8) || !tensors(args, 3, t) || !as_double(args[3], &min_scale) || !mode.from(args[4])) return nullptr;
+    if (n != 8 || !tensors(args, 3, t) || !as_double(args[3], &min_scale) || !as_text(args[4], &mode)) Py_RETURN_NOTIMPLEMENTED;
     for (int i = 0; i < 3; i++)
-        if (!as_int64(args[5 + i], &v[i])) return nullptr;
+        if (!as_int64(args[5 + i], &v[i])) Py_RETURN_NOTIMPLEMENTED;
     uint64_t ws = 0;
     aclOpExecutor* ex = nullptr;
     aclnnStatus rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = g_entry.block_quant(t[0], min_scale, const_cast<char*>(mode.c), v[0], v[1], v[2], t[1], t[2], &ws, &ex);
+    rc = g_entry.block_quant(t[0], min_scale, const_cast<char*>(mode), v[0], v[1], v[2], t[1], t[2], &ws, &ex);
     Py_END_ALLOW_THREADS
     return phase1_result(rc, ws, ex);
 }
@@ -200,48 +178,41 @@ PyObject* block_quant(PyObject*, PyObject* const* args, Py_ssize_t n)
 PyObject* mx_quant(PyObject*, PyObject* const* args, Py_ssize_t n)
 {
     const aclTensor* t[3];
-    Text mode;
+    const char* mode;
     int64_t axis, v[3];
-    if (!count(n, 8) || !tensors(args, 3, t) || !as_int64(args[3], &axis) || !mode.from(args[4])) return nullptr;
+    if (n != 8 || !tensors(args, 3, t) || !as_int64(args[3], &axis) || !as_text(args[4], &mode)) Py_RETURN_NOTIMPLEMENTED;
     for (int i = 0; i < 3; i++)
-        if (!as_int64(args[5 + i], &v[i])) return nullptr;
+        if (!as_int64(args[5 + i], &v[i])) Py_RETURN_NOTIMPLEMENTED;
     uint64_t ws = 0;
     aclOpExecutor* ex = nullptr;
     aclnnStatus rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = g_entry.mx_quant(t[0], axis, const_cast<char*>(mode.c), v[0], v[1], v[2], t[1], t[2], &ws, &ex);
+    rc = g_entry.mx_quant(t[0], axis, const_cast<char*>(mode), v[0], v[1], v[2], t[1], t[2], &ws, &ex);
     Py_END_ALLOW_THREADS
     return phase1_result(rc, ws, ex);
 }
 
-// phase2(address, function of ctypes) -> f(workspace, size, executor, stream), the status.  Arguments that only ctypes knows (arrays,
-// byref) go there.
+// phase2(address, function of ctypes) -> f(workspace, size, executor, stream), the status.
 typedef aclnnStatus (*Phase2)(void*, uint64_t, aclOpExecutor*, aclrtStream);
 PyObject* run_phase2(PyObject* self, PyObject* const* args, Py_ssize_t n)
 {
     void *address, *ws, *ex, *stream;
-    uint64_t size = 0;
-    bool ok = n == 4 && as_pointer(PyTuple_GET_ITEM(self, 0), &address) && as_pointer(args[0], &ws) && as_pointer(args[2], &ex) && as_pointer(args[3], &stream);
-    if (ok) {
-        PyObject* v = plain(args[1]);
-        size = v ? PyLong_AsUnsignedLongLongMask(v) : 0;
-        Py_XDECREF(v);
-        ok = !PyErr_Occurred();
-    }
-    if (!ok) {
-        PyErr_Clear();
-        return PyObject_Vectorcall(PyTuple_GET_ITEM(self, 1), args, (size_t)n, nullptr);
-    }
+    int64_t size = 0;
+    if (n != 4 || !as_pointer(PyTuple_GET_ITEM(self, 0), &address) || !as_pointer(args[0], &ws) || !as_int64(args[1], &size) ||
+        !as_pointer(args[2], &ex) || !as_pointer(args[3], &stream)) return PyObject_Vectorcall(PyTuple_GET_ITEM(self, 1), args, (size_t)n, nullptr);
     aclnnStatus rc;
     Py_BEGIN_ALLOW_THREADS
-    rc = ((Phase2)address)(ws, size, (aclOpExecutor*)ex, (aclrtStream)stream);
+    rc = ((Phase2)address)(ws, (uint64_t)size, (aclOpExecutor*)ex, (aclrtStream)stream);
     Py_END_ALLOW_THREADS
     return PyLong_FromLong((long)rc);
 }
 PyMethodDef g_phase2 = {"phase2", (PyCFunction)(void (*)(void))run_phase2, METH_FASTCALL, "(workspace, size, executor, stream) -> status"};
 PyObject* phase2(PyObject*, PyObject* const* args, Py_ssize_t n)
 {
-    if (!count(n, 2)) return nullptr;
+    if (n != 2) {
+        PyErr_SetString(PyExc_TypeError, "an address and a function are wanted");
+        return nullptr;
+    }
     PyObject* self = PyTuple_Pack(2, args[0], args[1]);
     PyObject* f = self ? PyCFunction_New(&g_phase2, self) : nullptr;
     Py_XDECREF(self);
@@ -257,6 +228,5 @@ PyModuleDef g_module = {PyModuleDef_HEAD_INIT, "opsnn_calls", "per-call entry po
 PyMODINIT_FUNC PyInit_opsnn_calls()
 {
     g_handle = PyUnicode_InternFromString("handle");
-    g_value = PyUnicode_InternFromString("value");
-    return g_handle && g_value ? PyModule_Create(&g_module) : nullptr;
+    return g_handle ? PyModule_Create(&g_module) : nullptr;
 }

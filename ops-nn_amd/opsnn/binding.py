@@ -233,7 +233,7 @@ def lib():
 
 
 # What a serving loop calls for every layer goes through a CPython extension instead of ctypes (csrc/python/calls.cpp): the same entry
-# points of the same loaded library.
+# points of the same loaded library.  It takes plain arguments; what else ctypes accepts or refuses goes to ctypes.
 _PHASE1_CALLS = ("aclnnQuantMatmulV5GetWorkspaceSize", "aclnnQuantMatmulWeightNzGetWorkspaceSize", "aclnnWeightQuantBatchMatmulV2GetWorkspaceSize",
                  "aclnnDynamicQuantGetWorkspaceSize", "aclnnDynamicBlockQuantGetWorkspaceSize", "aclnnDynamicMxQuantGetWorkspaceSize")
 _PHASE2_CALLS = ("aclnnQuantMatmulV5", "aclnnQuantMatmulWeightNz", "aclnnWeightQuantBatchMatmulV2", "aclnnDynamicQuant", "aclnnDynamicBlockQuant",
@@ -392,8 +392,16 @@ def quant_matmul_v5_get_workspace(x1, x2, x1_scale, x2_scale, out, *, y_scale=No
                                   ws_ptr=True, ex_ptr=True, weight_nz=False):
     """Phase 1 (of aclnnQuantMatmulWeightNz when weight_nz).  Returns (status, workspace_size, executor)."""
     lib()
-    return _calls.qmm(x1, x2, x1_scale, x2_scale, y_scale, x1_offset, x2_offset, y_offset, bias, out, transpose_x1, transpose_x2, group_size,
+    done = _calls.qmm(x1, x2, x1_scale, x2_scale, y_scale, x1_offset, x2_offset, y_offset, bias, out, transpose_x1, transpose_x2, group_size,
                       ws_ptr, ex_ptr, weight_nz)
+    if done is not NotImplemented:
+        return done
+    ws, ex = C.c_uint64(0), C.c_void_p()
+    fn = lib().aclnnQuantMatmulWeightNzGetWorkspaceSize if weight_nz else lib().aclnnQuantMatmulV5GetWorkspaceSize
+    rc = fn(
+        _h(x1), _h(x2), _h(x1_scale), _h(x2_scale), _h(y_scale), _h(x1_offset), _h(x2_offset), _h(y_offset), _h(bias),
+        transpose_x1, transpose_x2, group_size, _h(out), C.byref(ws) if ws_ptr else None, C.byref(ex) if ex_ptr else None)
+    return rc, ws.value, ex.value
 
 
 # A byte (0 .. 255) to fill every workspace with that the two-phase helpers below allocate, or None.  The parity tests set 0xFF
@@ -436,10 +444,16 @@ def weight_quant_batch_matmul_get_workspace(x, weight, scale, y, *, offset=None,
                                             bias=None, group_size=0, inner_precise=None, weight_nz=False):
     if not weight_nz and inner_precise is None:
         lib()
-        return _calls.wqmm(x, weight, scale, offset, quant_scale, quant_offset, bias, y, group_size)
+        done = _calls.wqmm(x, weight, scale, offset, quant_scale, quant_offset, bias, y, group_size)
+        if done is not NotImplemented:
+            return done
     ws, ex = C.c_uint64(0), C.c_void_p()
     if weight_nz:
         rc = lib().aclnnWeightQuantBatchMatmulNzGetWorkspaceSize(_h(x), _h(weight), _h(scale), _h(offset), _h(quant_scale),
+                                                                 _h(quant_offset), _h(bias), group_size, _h(y),
+                                                                 C.byref(ws), C.byref(ex))
+    elif inner_precise is None:
+        rc = lib().aclnnWeightQuantBatchMatmulV2GetWorkspaceSize(_h(x), _h(weight), _h(scale), _h(offset), _h(quant_scale),
                                                                  _h(quant_offset), _h(bias), group_size, _h(y),
                                                                  C.byref(ws), C.byref(ex))
     else:
@@ -465,9 +479,12 @@ def dynamic_quant_get_workspace(x, y, scale, *, smooth=None, offset=None, group_
                                 is_symmetrical=None, dst_type_max=None):
     """Phase 1 of aclnnDynamicQuant; V2 when v2 / offset / group_index is given; V3 when quant_mode is given; V4 when dst_type_max
     is given too.  Returns (status, workspace, executor)."""
-    if quant_mode is None and not v2 and offset is None and group_index is None:
+    plain = quant_mode is None and not v2 and offset is None and group_index is None
+    if plain:
         lib()
-        return _calls.dynamic_quant(x, smooth, y, scale)
+        done = _calls.dynamic_quant(x, smooth, y, scale)
+        if done is not NotImplemented:
+            return done
     ws, ex = C.c_uint64(0), C.c_void_p()
     if quant_mode is not None:
         sym = (offset is None) if is_symmetrical is None else is_symmetrical
@@ -477,6 +494,8 @@ def dynamic_quant_get_workspace(x, y, scale, *, smooth=None, offset=None, group_
         else:
             rc = lib().aclnnDynamicQuantV4GetWorkspaceSize(_h(x), _h(smooth), _h(group_index), dst_type, sym, quant_mode, dst_type_max, _h(y),
                                                            _h(scale), _h(offset), C.byref(ws), C.byref(ex))
+    elif plain:
+        rc = lib().aclnnDynamicQuantGetWorkspaceSize(_h(x), _h(smooth), _h(y), _h(scale), C.byref(ws), C.byref(ex))
     else:
         rc = lib().aclnnDynamicQuantV2GetWorkspaceSize(_h(x), _h(smooth), _h(group_index), dst_type, _h(y), _h(scale), _h(offset),
                                                        C.byref(ws), C.byref(ex))
@@ -500,13 +519,19 @@ def dynamic_quant(x, y, scale, stream=None, **kw):
 def dynamic_block_quant_get_workspace(x, y, scale, *, dst_type=None, row_block=1, col_block=128, min_scale=0.0, round_mode=b"rint",
                                       dst_type_max=None):
     dst = dst_type if dst_type is not None else (y.dtype if y is not None else 36)
+    if dst_type_max is None:
+        lib()
+        done = _calls.block_quant(x, y, scale, min_scale, round_mode, dst, row_block, col_block)
+        if done is not NotImplemented:
+            return done
+    ws, ex = C.c_uint64(0), C.c_void_p()
     if dst_type_max is not None:   # V2
-        ws, ex = C.c_uint64(0), C.c_void_p()
         rc = lib().aclnnDynamicBlockQuantV2GetWorkspaceSize(_h(x), min_scale, round_mode, dst, row_block, col_block, dst_type_max, _h(y),
                                                             _h(scale), C.byref(ws), C.byref(ex))
         return rc, ws.value, ex.value
-    lib()
-    return _calls.block_quant(x, y, scale, min_scale, round_mode, dst, row_block, col_block)
+    rc = lib().aclnnDynamicBlockQuantGetWorkspaceSize(_h(x), min_scale, round_mode, dst, row_block, col_block, _h(y), _h(scale),
+                                                      C.byref(ws), C.byref(ex))
+    return rc, ws.value, ex.value
 
 
 def dynamic_block_quant(x, y, scale, stream=None, **kw):
@@ -522,14 +547,20 @@ def dynamic_mx_quant_get_workspace(x, y, scale, *, axis=-1, round_mode=b"rint", 
     dst = dst_type if dst_type is not None else (y.dtype if y is not None else 40)
     if dst_type_max is None and max_low_bound is None:
         lib()
-        return _calls.mx_quant(x, y, scale, axis, round_mode, dst, blocksize, scale_alg)
+        done = _calls.mx_quant(x, y, scale, axis, round_mode, dst, blocksize, scale_alg)
+        if done is not NotImplemented:
+            return done
     ws, ex = C.c_uint64(0), C.c_void_p()
     if max_low_bound is not None:
         rc = lib().aclnnDynamicMxQuantV3GetWorkspaceSize(_h(x), axis, round_mode, dst, blocksize, scale_alg, dst_type_max or 0.0, max_low_bound,
                                                          _h(y), _h(scale), C.byref(ws), C.byref(ex))
         return rc, ws.value, ex.value
-    rc = lib().aclnnDynamicMxQuantV2GetWorkspaceSize(_h(x), axis, round_mode, dst, blocksize, scale_alg, dst_type_max, _h(y), _h(scale),
-                                                     C.byref(ws), C.byref(ex))
+    if dst_type_max is not None:
+        rc = lib().aclnnDynamicMxQuantV2GetWorkspaceSize(_h(x), axis, round_mode, dst, blocksize, scale_alg, dst_type_max, _h(y), _h(scale),
+                                                         C.byref(ws), C.byref(ex))
+        return rc, ws.value, ex.value
+    rc = lib().aclnnDynamicMxQuantGetWorkspaceSize(_h(x), axis, round_mode, dst, blocksize, scale_alg, _h(y), _h(scale),
+                                                   C.byref(ws), C.byref(ex))
     return rc, ws.value, ex.value
 
 

@@ -133,3 +133,69 @@ def test_threads_find_the_library_whole(monkeypatch):
     first.join(30)
     second.join(30)
     assert early == [] and len(seen) == 2 and seen[0] is seen[1]
+
+
+# Arguments as ctypes takes them: an int of any size counts by its low bits, a ctypes number only as the parameter's own type.
+PHASE_1_NUMBERS = [0, 128, True, 2 ** 64 + 128, -1, 2 ** 63, C.c_int64(128), C.c_int(128), C.c_float(128.0), C.c_void_p(128), 128.0, "128", None]
+
+
+def _outcome(fn, *args):
+    try:
+        got = fn(*args)
+    except Exception as e:
+        return "refused", isinstance(e, (TypeError, C.ArgumentError))
+    if isinstance(got, tuple):
+        if got[2]:
+            m.check(m.lib().aclDestroyAclOpExecutor(got[2]))
+        got = got[0], got[1], got[2] is None
+    return got
+
+
+@pytest.mark.parametrize("number", PHASE_1_NUMBERS, ids=repr)
+def test_phase_1_takes_the_numbers_that_ctypes_takes(number):
+    K, N = 4096, 1024
+    x, w, y, s = _t((16, K), m.ACL_FLOAT16), _t((K, N), m.ACL_INT4), _t((16, N), m.ACL_FLOAT16), _t((K // 128, N), m.ACL_FLOAT16)
+    assert _outcome(lambda: m.weight_quant_batch_matmul_get_workspace(x, w, s, y, group_size=number)) == _outcome(
+        lambda: _ctypes("aclnnWeightQuantBatchMatmulV2GetWorkspaceSize", x.handle, w.handle, s.handle, None, None, None, None, number, y.handle))
+    x1, x2, s1, s2, out = _t((8, K), m.ACL_INT8), _t((N, K), m.ACL_INT8), _t((8,), m.ACL_FLOAT), _t((N,), m.ACL_FLOAT), _t((8, N), m.ACL_BF16)
+    for group, flag in ((number, True), (0, number)):
+        assert _outcome(lambda: m.quant_matmul_v5_get_workspace(x1, x2, s1, s2, out, group_size=group, transpose_x2=flag)) == _outcome(
+            lambda: _ctypes("aclnnQuantMatmulV5GetWorkspaceSize", x1.handle, x2.handle, s1.handle, s2.handle, None, None, None, None, None, False, flag,
+                            group, out.handle))
+    q, sb, sm = _t((8, K), m.ACL_FLOAT8_E4M3FN), _t((8, K // 128), m.ACL_FLOAT), _t((8, K // 64, 2), m.ACL_FLOAT8_E8M0)
+    xb = _t((8, K), m.ACL_BF16)
+    for low, block in ((0.0, number), (number, 128)):
+        assert _outcome(lambda: m.dynamic_block_quant_get_workspace(xb, q, sb, min_scale=low, col_block=block)) == _outcome(
+            lambda: _ctypes("aclnnDynamicBlockQuantGetWorkspaceSize", xb.handle, low, b"rint", m.ACL_FLOAT8_E4M3FN, 1, block, q.handle, sb.handle))
+    for axis, mode in ((number, b"rint"), (-1, number)):
+        if isinstance(mode, (int, C.c_void_p)):   # (an address of text for ctypes)
+            continue
+        assert _outcome(lambda: m.dynamic_mx_quant_get_workspace(xb, q, sm, axis=axis, round_mode=mode)) == _outcome(
+            lambda: _ctypes("aclnnDynamicMxQuantGetWorkspaceSize", xb.handle, axis, mode, m.ACL_FLOAT8_E4M3FN, 32, 0, q.handle, sm.handle))
+
+
+@pytest.mark.parametrize("name", ["aclnnQuantMatmulV5", "aclnnQuantMatmulWeightNz", "aclnnWeightQuantBatchMatmulV2", "aclnnDynamicQuant",
+                                  "aclnnDynamicBlockQuant", "aclnnDynamicMxQuant"])
+def test_phase_2_takes_the_arguments_that_ctypes_takes(name):
+    class Value:
+        value = 4096
+
+    fn = C.CDLL(m.LIB_PATH)[name]
+    fn.restype, fn.argtypes = m.binding._SIGS[name]
+    some = (C.c_char * 16)()
+    for odd in (C.c_int(4096), C.c_uint64(4096), C.c_void_p(4096), Value(), 4096.0, "4096", b"4096", some, C.byref(some), -1, 2 ** 64 + 4096):
+        for at in range(4):
+            if at == 3 and not isinstance(odd, (C.c_int, C.c_uint64, Value, float)):
+                continue   # (a stream is used as one)
+            args = [None, 0, 4096, None]
+            args[at] = odd
+            assert _outcome(getattr(m.lib(), name), *args) == _outcome(fn, *args), (odd, at)
+
+
+def test_an_object_that_is_no_tensor():
+    x, y, s = _t((8, 2048), m.ACL_BF16), _t((8, 2048), m.ACL_INT8), _t((8,), m.ACL_FLOAT)
+    with pytest.raises(AttributeError):
+        m.dynamic_quant_get_workspace(x, 4096, s)
+    gone = _t((8,), m.ACL_FLOAT)
+    gone.destroy()
+    assert m.dynamic_quant_get_workspace(x, y, gone)[0] != 0
