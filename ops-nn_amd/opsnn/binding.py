@@ -3,6 +3,7 @@ loop calls."""
 import ctypes as C
 import importlib.util
 import os
+import sysconfig
 import threading
 
 import numpy as np
@@ -233,20 +234,28 @@ def lib():
 
 
 # What a serving loop calls for every layer goes through a CPython extension instead of ctypes (csrc/python/calls.cpp): the same entry
-# points of the same loaded library.  It takes plain arguments; what else ctypes accepts or refuses goes to ctypes.
+# points of the same loaded library.  It takes plain arguments; what else ctypes accepts or refuses goes to ctypes, and so does every call
+# where the extension was not built for this interpreter.
 _PHASE1_CALLS = ("aclnnQuantMatmulV5GetWorkspaceSize", "aclnnQuantMatmulWeightNzGetWorkspaceSize", "aclnnWeightQuantBatchMatmulV2GetWorkspaceSize",
                  "aclnnDynamicQuantGetWorkspaceSize", "aclnnDynamicBlockQuantGetWorkspaceSize", "aclnnDynamicMxQuantGetWorkspaceSize")
 _PHASE2_CALLS = ("aclnnQuantMatmulV5", "aclnnQuantMatmulWeightNz", "aclnnWeightQuantBatchMatmulV2", "aclnnDynamicQuant", "aclnnDynamicBlockQuant",
                  "aclnnDynamicMxQuant")
-_calls = None
+CALLS_PATH = os.path.join(os.path.dirname(LIB_PATH), "opsnn_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
+
+
+class _NoCalls:
+    def __getattr__(self, name):
+        return lambda *args: NotImplemented
+
+
+_calls = _NoCalls()
 
 
 def _bind_calls(library):
     global _calls
-    path = os.path.join(os.path.dirname(LIB_PATH), "opsnn_calls.so")
-    if not os.path.exists(path):
-        raise RuntimeError(f"{path} is not built; run `python -c 'import __graft_entry__ as g; g.build()'`")
-    spec = importlib.util.spec_from_file_location("opsnn_calls", path)
+    if not os.path.exists(CALLS_PATH):
+        return
+    spec = importlib.util.spec_from_file_location("opsnn_calls", CALLS_PATH)
     module = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(module)
 

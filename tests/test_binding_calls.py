@@ -1,6 +1,10 @@
 """The binding's extension (csrc/python/calls.cpp) against the same entry points called through ctypes: statuses, workspace sizes and
 whether an executor comes back, for calls that are accepted and for calls that are refused; and views of up to eight dims."""
 import ctypes as C
+import os
+import subprocess
+import sys
+import sysconfig
 import threading
 
 import pytest
@@ -199,3 +203,26 @@ def test_an_object_that_is_no_tensor():
     gone = _t((8,), m.ACL_FLOAT)
     gone.destroy()
     assert m.dynamic_quant_get_workspace(x, y, gone)[0] != 0
+
+
+def test_without_the_extension(monkeypatch, tmp_path):
+    """A tree with the C library alone, or with an extension for another interpreter: the same answers through ctypes."""
+    monkeypatch.setattr(m.binding, "CALLS_PATH", str(tmp_path / "none.so"))
+    monkeypatch.setattr(m.binding, "_lib", None)
+    monkeypatch.setattr(m.binding, "_calls", m.binding._NoCalls())
+    test_quant_matmul_v5(8, 4096, 4096, None)
+    test_quant_matmul_v5(8, 4096, 4096, "scale")
+    test_weight_quant(128, True)
+    test_quantizers(5)
+    test_phase_2_takes_the_arguments_that_ctypes_takes("aclnnQuantMatmulV5")
+
+
+def _make(*args):
+    csrc = os.path.join(os.path.dirname(m.LIB_PATH), "..", "csrc")
+    return subprocess.run(["make", "-n", "-B", "-C", csrc, *args], check=True, capture_output=True, text=True).stdout
+
+
+def test_the_c_library_is_built_without_python():
+    assert "opsnn_calls" + sysconfig.get_config_var("EXT_SUFFIX") in _make(f"PYTHON={sys.executable}")
+    rest = _make("PYTHON=/no/python")
+    assert "opsnn_calls" not in rest and "Python" not in rest and "libopsnn_amd.so" in rest and "examples/" in rest
