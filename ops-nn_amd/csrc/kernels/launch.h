@@ -60,12 +60,22 @@ struct SplitK {
     int splits = 1;
     float* part = nullptr;
 };
-// Whether a weight that a call reads once goes past the last-level cache (256 MB): from 100 MB on.  A step works through three such weights
-// and more, of which none is found there again, and fetched without a line kept there they come faster.  Copies of 128-byte row
-// pieces into LDS, three weights in turn, plain / past the cache: 88 MB 14.2 / 23.4 us, 101 MB 23.5 / 23.6, 117 MB 26.7 / 24.7, 168 MB 34.1 / 30.2, 235 MB 43.3 /
-// 39.2 (one weight again and again, which is the other way round: 117 MB 17.0 / 24.5, 262 MB 38.9 / 40.9).  Not where the pieces are 64
-// bytes, half a line that is then fetched twice: 117 MB 25.0 / 27.5.
-inline bool weight_is_streamed(int64_t bytes) { return bytes > 100000000; }
+// How much of a weight that a call reads once leaves its lines in the last-level cache (256 MB): one in so many of its copies, the others go past it.
+// A step works through three such weights and more, of which none is found there again when all of them pass through; past it they come faster,
+// but then a weight that is used again at once is not found either.  A share of each fits for several weights in turn, and what is found and what
+// comes from memory arrive side by side.  fp8_wide_kernel, us, all kept / none / every second / every fourth copy:
+//                                        one weight again and again      three in turn                   1.4 GB in turn
+//   132 MB, 64 x 18432 x 7168 block      34.9 / 35.9 / 33.6 / 33.9       36.2 / 36.3 / 33.7 / 34.0       36.3 / 36.3 / 35.9 / 35.5
+//   132 MB, 64 x 7168 x 18432 row/column 33.4 / 38.7 / 34.4 / 35.4       37.5 / 39.2 / 34.6 / 35.3       37.5 / 39.2 / 37.1 / 36.8
+//   132 MB, 20 x 18432 x 7168 MX         27.9 / 33.6 / 31.8 / 32.9       35.6 / 34.3 / 32.4 / 32.9       35.6 / 34.5 / 35.4 / 34.7
+//   176 MB, 17 x 8192 x 21504 row/column 30.7 / 37.6 / 32.2 / 33.6       43.0 / 38.9 / 32.7 / 33.7       42.6 / 38.9 / 40.1 / 39.5
+//   235 MB, 64 x 8192 x 28672 block      47.1 / 54.3 / 49.6 / 50.9       56.5 / 53.7 / 55.2 / 50.8       57.8 / 54.3 / 56.7 / 55.3
+//   302 MB, 64 x 16384 x 18432 row/col.  73.3 / 75.7 / 61.0 / 64.7       81.0 / 74.7 / 73.8 / 66.0       80.5 / 74.4 / 73.6 / 71.2
+// So every second one to 150 MB, every fourth one beyond (three such shares are the cache's size), and all of it below 100 MB, where three weights
+// nearly fit as they are (88 MB, copies alone, 14.2 kept and 23.4 past it).  From two weights in turn on nothing is slower than with all of it kept;
+// one weight again and again is, by 0 to 14 % (by 2 to 24 % with none kept).  Not for pieces of 64 bytes, half a line that is then fetched twice:
+// 117 MB 25.0 / 27.5.
+inline int weight_kept_share(int64_t bytes) { return bytes <= 100000000 ? 1 : bytes <= 150000000 ? 2 : 4; }
 // How many ways a call with `tiles` output tiles, `ktiles` K tiles of `tile_us` microseconds each and `out_elems` outputs
 // is split: at most one workgroup per CU, at least four K tiles per workgroup, at most sixteen ways -- and among those the
 // count with the largest estimated gain, if that is at least 3 us: the loop time saved, ktiles * tile_us * (1 - 1/s), less

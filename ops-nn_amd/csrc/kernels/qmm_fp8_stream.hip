@@ -43,7 +43,7 @@ struct Fp8StreamParams {
     int rs_stride, cs_stride;
     const float* bias;
     float* part;                  // [splits][M][N]
-    bool once;                    // x2 is read once and is too large to be found in the last-level cache by the next call
+    int kept;                     // one in so many of x2's copies leaves its lines in the last-level cache
 };
 
 template <int FORM>
@@ -341,9 +341,9 @@ __global__ __launch_bounds__(256, 1) void fp8_stream_kernel(Fp8StreamParams p)
 // (With a ring per wave, x1's share of the LDS is four times as large and too few bytes of x2 are in flight: 64 x 18432 x 7168 stays at
 // 2.7 TB/s.)  Rows of 128 bytes, 16-byte chunk c of row r at c ^ (r / 2 % 8).
 template <int MB, int NB, int FORM> constexpr int fw_tile = MB * 2048 + NB * 8192 + (FORM == FP8X_BLOCK ? 1024 : FORM == FP8X_MX ? 1024 + 1024 : 0);
-// ONCE: x2 comes past the last-level cache (weight_is_streamed; a flag tested in the loop took half of the gain: 64 x 18432 x 7168
-// block scales with their quantizer 44.2 us without, 42.4 with the flag, 40.9 so).
-template <int MB, int NB, int FORM, int S, bool ONCE>
+// KEPT: all of x2 by way of the last-level cache (1), or one in so many of a wave's copies of a tile and the others past it (weight_kept_share; a
+// flag tested in the loop took half of the gain).
+template <int MB, int NB, int FORM, int S, int KEPT>
 __global__ __launch_bounds__(256, 2) void fp8_wide_kernel(Fp8StreamParams p)
 {
     constexpr int TILE = fw_tile<MB, NB, FORM>;
@@ -390,7 +390,7 @@ __global__ __launch_bounds__(256, 2) void fp8_wide_kernel(Fp8StreamParams p)
         for (int i = 0; i < XC; i++) copy16_sbase(p.a + k, xo[i], at + ((wave * XC + i) * 1024) % (MB * 2048));
 #pragma unroll
         for (int i = 0; i < 2 * NB; i++) {
-            if constexpr (ONCE) copy16_sbase_once(wbase + k, wo[i], at + MB * 2048 + (wave * 2 * NB + i) * 1024);
+            if (i % KEPT != 0) copy16_sbase_once(wbase + k, wo[i], at + MB * 2048 + (wave * 2 * NB + i) * 1024);
             else copy16_sbase(wbase + k, wo[i], at + MB * 2048 + (wave * 2 * NB + i) * 1024);
         }
         const uint32_t sc = at + MB * 2048 + NB * 8192 + wave * 256;
@@ -553,14 +553,14 @@ int launch_one(const Fp8StreamParams& p, hipStream_t st)
 }
 // stages of the wide kernel: two workgroups a CU
 template <int MB, int NB, int FORM> constexpr int fw_stages = at_most_8((81920 - fs_table<FORM>) / fw_tile<MB, NB, FORM>);
-template <int MB, int NB, int FORM, bool ONCE>
+template <int MB, int NB, int FORM, int KEPT>
 int launch_wide_one(const Fp8StreamParams& p, hipStream_t st)
 {
     constexpr int S = fw_stages<MB, NB, FORM>;
     constexpr size_t lds = (size_t)S * fw_tile<MB, NB, FORM> + fs_table<FORM>;
     static_assert(S >= 2, "the ring");
     const dim3 grid((unsigned)((p.N + 64 * NB - 1) / (64 * NB)), (unsigned)p.splits, (unsigned)((p.M + 16 * MB - 1) / (16 * MB)));
-    auto k = fp8_wide_kernel<MB, NB, FORM, S, ONCE>;
+    auto k = fp8_wide_kernel<MB, NB, FORM, S, KEPT>;
     static std::atomic<uint64_t> attr_set{0};   // one bit per device: the attribute belongs to the (kernel, device) pair
     if (!device_flag_test(attr_set)) {
         hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -575,7 +575,7 @@ int launch_wide_one(const Fp8StreamParams& p, hipStream_t st)
 template <int FORM>
 int launch_form(const Fp8StreamParams& p, const Fp8StreamPlan& pl, hipStream_t st)
 {
-#define ONE(MB, NB) if (pl.mb == MB && pl.nb == NB) return !pl.wide ? launch_one<MB, NB, FORM>(p, st) : p.once ? launch_wide_one<MB, NB, FORM, true>(p, st) : launch_wide_one<MB, NB, FORM, false>(p, st);
+#define ONE(MB, NB) if (pl.mb == MB && pl.nb == NB) return !pl.wide ? launch_one<MB, NB, FORM>(p, st) : p.kept == 1 ? launch_wide_one<MB, NB, FORM, 1>(p, st) : NB == 1 || p.kept == 2 ? launch_wide_one<MB, NB, FORM, 2>(p, st) : launch_wide_one<MB, NB, FORM, 2 * NB>(p, st);
     ONE(1, 1) ONE(1, 2) ONE(2, 1) ONE(2, 2) ONE(4, 1) ONE(4, 2)
 #undef ONE
     if constexpr (FORM != FP8X_BLOCK) {   // (K % 128 == 64 only)
@@ -744,7 +744,7 @@ int launch_fp8_stream(const OpsnnQmmArgs& a, Fp8xForm form, SplitK sk, hipStream
     if (((uintptr_t)p.a | (uintptr_t)p.b | (uint64_t)p.lda | (uint64_t)p.ldb) % 16) return OPSNN_NOT_TAKEN;
     p.out = a.out; p.out_dt = a.out_dtype; p.M = (int)a.M; p.N = (int)a.N; p.tiles = (int)(a.K / 64); p.splits = splits;
     p.part = sk.part; p.bias = (const float*)a.bias;
-    p.once = a.M <= 64 && weight_is_streamed(a.N * a.K);
+    p.kept = a.M <= 64 ? weight_kept_share(a.N * a.K) : 1;
     if (form == FP8X_BLOCK) {
         p.s1 = (const float*)a.x1_scale_mat.ptr; p.s1_rs = a.x1_scale_mat.row_stride; p.s1_cs = a.x1_scale_mat.col_stride;
         p.s2 = (const float*)a.x2_scale_mat.ptr; p.s2_rs = a.x2_scale_mat.row_stride; p.s2_cs = a.x2_scale_mat.col_stride;

@@ -94,8 +94,10 @@ def test_row_column_and_mx_scales(gpu, form, M, K, N):
     del keep
 
 
-# a weight from 100 MB on: the wide kernel's copies go past the last-level cache, a last strip of one column, segments
-@pytest.mark.parametrize("form,M,K,N", [("block", 17, 12288, 8193), ("rowcol", 33, 13568, 7400), ("mx", 20, 18432, 5440)])
+# a weight from 100 MB on: every second of the wide kernel's copies goes past the last-level cache, from 150 MB on three of four; a last strip of
+# one column, segments
+@pytest.mark.parametrize("form,M,K,N", [("block", 17, 12288, 8193), ("rowcol", 33, 13568, 7400), ("mx", 20, 18432, 5440),
+                                        ("block", 18, 16384, 9217), ("rowcol", 20, 18432, 8200), ("mx", 33, 12800, 11800)])
 def test_weights_from_100_mb_on(gpu, form, M, K, N):
     assert N * K > 100_000_000
     if form == "block":
