@@ -640,11 +640,12 @@ float decode_typical_us(const QmmDecodePlan& pl, bool mx, int64_t M, int64_t N, 
            (pl.splits > 1 ? (mx ? 2.06f : 2.17f) + (mx ? 1.53f : 1.76f) * (float)pl.splits * out_m : 0.0f);
 }
 // The exact tiles of qmm_fp8_exact.hip on the same terms: their plan's estimate with what it leaves out, and corrected where it is off
-// (524 calls of 65 .. 512 rows, median error 2 %).  K is cut there from 129 rows, MX from 65.
+// (1066 calls of 65 .. 512 rows, half of them for the fit; median error of the others 2 %; block scales a little high, as the stream kernel's estimate is
+// there).  K is cut there from 129 rows, MX from 65.
 float tiles_typical_us(int64_t M, int64_t N, int64_t K, Fp8xForm form, bool may_split)
 {
     static const struct { float scale, start, out, split; } cost[3] = {   // by Fp8xForm
-        {0.978f, 1.85f, 0.38f, -0.96f}, {0.898f, 6.49f, 0.431f, -4.33f}, {1.03f, -0.78f, 0.434f, -1.2f}};
+        {1.05f, 0.2f, 0.21f, 0.7f}, {1.005f, 3.1f, 0.42f, -1.9f}, {1.03f, -2.05f, 0.7f, 1.3f}};
     const auto& c = cost[form];
     const Fp8xPlan pl = fp8x_plan(M, N, K, 1, form, may_split && (M > 128 || form == FP8X_MX));
     const float out_m = (float)M * (float)N * 1e-6f;
@@ -670,7 +671,9 @@ constexpr int narrow_per_cu(int mb, int nb)
 // From 65 to 512 rows, in slabs of 64: products that leave most of the exact tiles without a CU's worth of work, by the estimates
 // (typical times there and here, MX 65 x 2048 x 2304 13.4 and 10.1 us, 128 x 1664 x 1472 15.2 and 8.9, 128 x 13568 x 8960 52 and 67,
 // 96 x 7424 x 18816 55 and 77; row / column scales 181 x 2560 x 2368 16.4 and 11.1, 114 x 11520 x 22208 89 and 108; block scales
-// 405 x 1664 x 3848 24.2 and 18.9).  A last half K tile runs on padded copies there: here up to so many multiplications above 128 rows (row /
+// 405 x 1664 x 3848 24.2 and 18.9; of 1066 calls 6 run 5 % longer than on the other side, the worst 1.13 times.  With the corrections of the tiles'
+// former plan 31 did, the worst 1.29 times: row / column scales 109 x 16640 x 15253 91 here and 106 there, MX 114 x 2944 x 4757 18.2 and
+// 19.5, block scales 194 x 6144 x 1472 16.9 and 18.8).  A last half K tile runs on padded copies there: here up to so many multiplications above 128 rows (row /
 // column scales 246 x 12224 x 2560 76 and 49).
 constexpr int64_t FS_MANY_ROWS_TAIL = 3200000000, FS_MANY_ROWS_TAIL_PLAIN = 12000000000;
 bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8StreamPlan& pl)
@@ -706,7 +709,8 @@ bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8St
         const int64_t per_wave = wide ? seg : (seg + 3) / 4;
         if (splits > 1 && (!may_split || units < 4 * splits)) return;
         if (form == FP8X_BLOCK && per_wave > FS_MOST_BLOCKS) return;
-        // (partial sums of a row that is no whole number of quads: stored piece by piece, added one column per thread)
+        // (partial sums of a row that is no whole number of quads count twice: their stores straddle lines, and where they did not count so,
+        // 19 of 200 such calls of up to 64 rows were cut otherwise and took 1.026 times as long, fp8 and weight-only together)
         const float us = stream_us(wide ? wide_cost[form] : narrow_cost[form], mb, nb, strips * splits * slabs, wide ? seg : 2 * per_wave, slabs, splits, per_cu, x2_mb, a.N % 4 ? 2.0f * out_m : out_m);
         if (us < best) { best = us; pl.wide = wide; pl.nb = nb; pl.splits = splits; wgs = strips * splits * slabs; k_tiles = wide ? seg : 2 * per_wave; cu_wgs = per_cu; }
     };
@@ -720,7 +724,7 @@ bool fp8_stream_plan(const OpsnnQmmArgs& a, Fp8xForm form, bool may_split, Fp8St
     for (int i = 0; !whole && i < 6; i++) consider(false, 4, steps[i], 1);
     if (best >= 1e30f) return false;
     if (whole && (a.M > 64 || (a.M <= 16 && form != FP8X_PLAIN))) {
-        const float out = a.N % 4 ? 2.0f * out_m : out_m, here = stream_typical_us((pl.wide ? wide_time : narrow_time)[form], pl, wgs, k_tiles, slabs, cu_wgs, x2_mb, out);
+        const float out = a.N % 4 && a.M <= 64 ? 2.0f * out_m : out_m, here = stream_typical_us((pl.wide ? wide_time : narrow_time)[form], pl, wgs, k_tiles, slabs, cu_wgs, x2_mb, out);
         if (a.M > 64) return here <= tiles_typical_us(a.M, a.N, a.K, form, may_split);
         // (1.04: this kernel's estimate is 2 to 10 % high up to 16 rows.  Of 700 calls drawn after the fit 33 are 5 % slower or more than on the other
         // kernel, of 900 without x1's load and this factor 78.)

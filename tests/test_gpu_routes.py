@@ -100,6 +100,32 @@ def test_from_65_rows_of_fp8(gpu, mode, M, K, N, want):
     assert got[0] in want.split(), got
 
 
+def rowcol_route(m, M, K, N):
+    d1, d2, ds = (m.DeviceBuffer(host=np.zeros(n, t)) for n, t in ((M * K, np.uint8), (N * K, np.uint8), (max(M, N), np.float32)))
+    out = m.DeviceBuffer(M * N * 2)
+    fp8 = m.ACL_FLOAT8_E4M3FN
+    t = [m.Tensor((M, K), fp8, d1), m.Tensor((N, K), fp8, d2), m.Tensor((M,), m.ACL_FLOAT, ds), m.Tensor((N,), m.ACL_FLOAT, ds), m.Tensor((M, N), m.ACL_BF16, out)]
+    workspace = m.quant_matmul_v5(*t, transpose_x2=True)
+    m.check(m.lib().aclrtSynchronizeDevice(), "sync")
+    del workspace
+    return route(m)
+
+
+# calls that the corrections of the tiles' former plan sent to the tiles: us here and there
+@pytest.mark.parametrize("mode,M,K,N", [
+    ("rowcol", 109, 16640, 15253),   # 91 and 106
+    ("rowcol", 204, 2688, 5018),     # 18.5 and 21.1
+    ("rowcol", 171, 8704, 2388),     # 19.8 and 21.1
+    ("block", 194, 6144, 1472),      # 16.9 and 18.8
+    ("block", 184, 10240, 1399),     # 19.1 and 20.1
+    ("block", 147, 12416, 1792),     # 20.8 and 22.0
+    ("mx", 114, 2944, 4757),         # 18.2 and 19.5
+    ("mx", 160, 3840, 1450)])        # 14.1 and 15.6
+def test_from_65_rows_of_fp8_on_the_stream_kernel(gpu, mode, M, K, N):
+    got = rowcol_route(gpu, M, K, N) if mode == "rowcol" else mx_route(gpu, M, K, N, False) if mode == "mx" else block_route(gpu, M, K, N)
+    assert got[0] in ("fp8_wide", "fp8_stream"), got
+
+
 # with the 8-bit instruction asked for, MXFP8 with few rows keeps its kernels, also below 64 x 64 outputs
 @pytest.mark.parametrize("M,K,N", [(1, 2176, 256), (1, 3968, 3968), (1, 10624, 3968), (2, 2112, 1088), (16, 3200, 1920), (24, 1536, 512), (100, 1664, 1472)])
 def test_mxfp8_few_rows_with_the_8_bit_instruction(gpu, M, K, N):
