@@ -130,8 +130,7 @@ constexpr int ww_stages(int wbits, int mb)
     return wbits == 4 ? (mb <= 2 ? 6 : mb <= 4 ? 4 : 3) : (mb <= 4 ? 4 : 3);
 }
 constexpr int ww_ring(int wbits, int mb) { const int a = ww_tile(wbits, mb) * ww_stages(wbits, mb); return a > 65536 ? a : 65536; }
-constexpr int WW_FLAGS = 32;   // bytes behind the table, a word a wave
-constexpr int ww_groups(int wbits, int mb) { return (163840 - WW_FLAGS - ww_ring(wbits, mb)) / (WW_COLS * 4); }
+constexpr int ww_groups(int wbits, int mb) { return (163840 - ww_ring(wbits, mb)) / (WW_COLS * 4); }
 
 // [N, K] storage; [K, N] storage with rows of whole 16-byte pieces; of whole dwords
 enum WwStorage { WW_NK, WW_KN, WW_KN4 };
@@ -298,6 +297,10 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
             }
         }
     };
+    // Without offsets the upper halves of the table's words are free.  Those of the first eight hold a flag of each wave: the table can be as large as
+    // the LDS has room for (212 x 10112 x 12096 in groups of 128 fills it; with the flags behind it K had to be cut in four: bf16 in [K, N] storage 97.8 us so, 102.5 cut).
+    typedef uint16_t __attribute__((may_alias)) Half;
+    Half* const halves = (Half*)tab;
     bool large = false;   // a scale from 2^125 on, an infinity or NaN
     auto store8 = [&](const Eight& v, int i) {
         const int g = t_g + 32 * i - g_lo;
@@ -305,7 +308,9 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
         for (int e = 0; e < 8; e++) {
             if constexpr (MAY_E4M3) large = large || (v.s[e] & 0x7f80) >= 0x7e00;
             const int ge = g + (by_group ? e : 0), ne = t_col + (by_group ? 0 : e);
-            if (ge >= 0 && ge < gmax) tab[ge * WW_COLS + ne] = HAS_OFF ? v.s[e] | (uint32_t)v.o[e] << 16 : v.s[e];
+            if (ge < 0 || ge >= gmax) continue;
+            if constexpr (MAY_E4M3) halves[2 * (ge * WW_COLS + ne)] = v.s[e];
+            else tab[ge * WW_COLS + ne] = HAS_OFF ? v.s[e] | (uint32_t)v.o[e] << 16 : v.s[e];
         }
     };
     {
@@ -319,10 +324,9 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
         store8(v0, 0);
         if (32 < gmax + 7) store8(v1, 1);
     }
-    uint32_t* const flags = tab + gmax * WW_COLS;
     if constexpr (MAY_E4M3) {
         const uint64_t any = __ballot(large);
-        if (lane == 0) flags[wave] = any != 0;
+        if (lane == 0) halves[2 * wave + 1] = any != 0;
     }
     wait_copies<(S - 1) * CPT>();
     __syncthreads();
@@ -371,7 +375,7 @@ __global__ __launch_bounds__(512, 1) void wq_wide_kernel(WqParams p, int tiles, 
     if constexpr (MAY_E4M3) {
         uint32_t any = 0;
 #pragma unroll
-        for (int i = 0; i < WW_FLAGS / 4; i++) any |= flags[i];
+        for (int i = 0; i < 8; i++) any |= halves[2 * i + 1];
         if (__builtin_amdgcn_readfirstlane(any)) walk(std::false_type{});
         else walk(std::true_type{});
     } else walk(std::false_type{});
@@ -457,7 +461,7 @@ int launch_one(const WqParams& p, const WqWidePlan& pl, hipStream_t st)
     const int tiles = (int)((p.K + WW_KT - 1) / WW_KT);
     const dim3 grid((unsigned)((p.N + WW_COLS - 1) / WW_COLS), (unsigned)pl.splits, (unsigned)((p.M + 16 * MB - 1) / (16 * MB)));
     note_route("wq_wide", pl.splits);
-    hipLaunchKernelGGL(k, grid, dim3(512), ww_ring(WBITS, MB) + pl.groups * WW_COLS * 4 + WW_FLAGS, st, p, tiles, pl.splits, pl.groups);
+    hipLaunchKernelGGL(k, grid, dim3(512), ww_ring(WBITS, MB) + pl.groups * WW_COLS * 4, st, p, tiles, pl.splits, pl.groups);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || pl.splits == 1) return (int)e;
     launch_wq_splitk_reduce(p, pl.splits, XDT, st);
     return (int)hipGetLastError();

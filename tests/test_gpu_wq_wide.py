@@ -154,3 +154,17 @@ def test_scales_at_the_end_of_the_range(gpu, M, K, N, group, nk):
     rest[N - 2] = False
     _b16_bar(np.ascontiguousarray(got[:, rest]), np.ascontiguousarray(want[:, rest]), orc.BF16, "wide, other columns", K)
     assert np.abs(g[:, N - 2] / w[:, N - 2] - 1).max() <= 2.0 ** -7
+
+
+@pytest.mark.parametrize("x_dt,off", [("bf16", False), ("f16", True)])
+def test_table_of_scales_as_large_as_the_lds_has_room_for(gpu, x_dt, off):
+    """79 groups of 128 and one that a segment could begin in: the table of 80 fills the LDS beside the ring, K in one piece."""
+    m = gpu
+    M, K, N = 212, 10112, 12096
+    xd = m.ACL_FLOAT16 if x_dt == "f16" else m.ACL_BF16
+    inp = cases.make_wq_inputs(m, M, K, N, 7, xd, m.ACL_INT4, 128, False, off, None)
+    print(f"case wide, full table M={M} K={K} N={N} {x_dt} off={off}", flush=True)
+    got = cases.run_wq_aclnn(m, inp, M, K, N)
+    assert route(m) == ("wq_wide", 1), route(m)
+    rows = np.array([0, 63, 64, 127, 128, 211])
+    _b16_bar(np.ascontiguousarray(got[rows]), cases.oracle_wq(m, inp, M, K, N, rows=rows), orc.F16 if x_dt == "f16" else orc.BF16, "full table", K)
