@@ -492,16 +492,14 @@ int launch_mx_mfma(const OpsnnQmmArgs& a0, hipStream_t st, SplitK sk)
         // chosen below, whole ones
         const bool split = fp4_cut;
         if (split) { g.splits = sk.splits; g.part = (int32_t*)sk.part; }
-        note_route(fp4_small ? "mxfp4_tiles_128" : "mxfp4_tiles_256", split ? sk.splits : 1);
+        // Small tiles: eight waves of 64 x 32 where a CU has at most two workgroups of at most 18 K tiles of 128 each, in one piece, which are a matter of
+        // latency (235 x 1536 x 7335 9.5 -> 8.1 us, 8 x 93 x 1152 x 1208 8.7 -> 7.2; 33 drawn calls 0.88 of the time); four of 64 x 64, with fewer reads,
+        // where there is more (8 x 36 x 3840 x 10048 50.5 so, 55.5 on eight) and in segments, which end in stores of partial sums (45 drawn calls
+        // of such a size 1.017 times as long on eight: 107 x 16896 x 1536 in twelve 16.7 and 17.6, 74 x 9216 x 3840 in six 16.0 and 17.0).
+        const bool eight = fp4_small && !split && a.K <= 18 * 128 && (a.M + 127) / 128 * ((a.N + 127) / 128) * a.batch <= 512;
+        note_route(eight ? "mxfp4_tiles_128_w8" : fp4_small ? "mxfp4_tiles_128" : "mxfp4_tiles_256", split ? sk.splits : 1);
         if (fp4_small) {
-            // Eight waves of 64 x 32 where a CU has at most two workgroups of at most 18 K tiles of 128 each, which are a matter of latency (235 x 1536 x
-            // 7335 9.5 -> 8.1 us, 8 x 93 x 1152 x 1208 8.7 -> 7.2, 71 x 5120 x 5688 in four segments 14.6 -> 13.8); four of 64 x 64, with fewer reads,
-            // where there is more (486 x 5760 x 3584 in two 28.1 so, 29.2 on eight; 8 x 36 x 3840 x 10048 50.5 and 55.5).
-            const int64_t cut = split ? sk.splits : 1, wgs = (a.M + 127) / 128 * ((a.N + 127) / 128) * a.batch * cut;
-            if (wgs <= 512 && a.K <= 18 * 128 * cut) {
-                if (split) return qgemm_launch_split_mx<MODE_MXFP4, 128, 128, 64, 2, 4, 4, 1>(g, a.batch, a.out_dtype, st);
-                return qgemm_launch<MODE_MXFP4, 128, 128, 64, 2, 4, 4, 1>(g, a.batch, a.out_dtype, st);
-            }
+            if (eight) return qgemm_launch<MODE_MXFP4, 128, 128, 64, 2, 4, 4, 1>(g, a.batch, a.out_dtype, st);
             if (split) return qgemm_launch_split_mx<MODE_MXFP4, 128, 128, 64, 2, 2, 4, 1>(g, a.batch, a.out_dtype, st);
             return qgemm_launch<MODE_MXFP4, 128, 128, 64, 2, 2, 4, 1>(g, a.batch, a.out_dtype, st);
         }

@@ -73,7 +73,7 @@ def test_scale_rows_of_both_operands_beyond_the_grids_second_axis(gpu, M, K, N, 
                 "mxfp4 tail, many scale rows")
 
 
-@pytest.mark.parametrize("M,K,N", [(40, 256, 65408), (97, 384, 65500)])
+@pytest.mark.parametrize("M,K,N", [(40, 256, 65536), (97, 384, 65500)])
 def test_eight_waves_and_four_give_the_same_bits(gpu, M, K, N):
     """128 x 128 tiles on either side of the line between eight and four waves, 512 workgroups: the same columns by themselves and with 128 more."""
     m = gpu
@@ -82,9 +82,20 @@ def test_eight_waves_and_four_give_the_same_bits(gpu, M, K, N):
     few["x2"], few["s2"] = (np.ascontiguousarray(inp[k][:, :N]) for k in ("x2", "s2"))
     print(f"case mxfp4 eight and four waves M={M} K={K} N={N}", flush=True)
     got = []
-    for i, n in ((few, N), (inp, N + 128)):
+    for i, n, want in ((few, N, "mxfp4_tiles_128_w8"), (inp, N + 128, "mxfp4_tiles_128")):
         got.append(cases.run_mx_aclnn(m, i, M, K, n, True, m.ACL_BF16, None).reshape(M, n)[:, :N])
-        assert route(m) == ("mxfp4_tiles_128", 1), route(m)
+        assert route(m) == (want, 1), route(m)
     assert np.array_equal(got[0], got[1])
     rows = [0, 31, 32, M - 1]
     check_close(np.ascontiguousarray(got[0][rows]).reshape(1, 4, N), cases.oracle_mx(m, few, M, K, N, True, m.ACL_BF16, rows=rows), orc.BF16, "mxfp4 eight waves")
+
+
+@pytest.mark.parametrize("M,K,N", [(107, 16896, 1536), (74, 9216, 3840)])
+def test_segments_of_small_tiles_are_four_waves(gpu, M, K, N):
+    m = gpu
+    print(f"case mxfp4 segments of small tiles M={M} K={K} N={N}", flush=True)
+    inp = cases.make_mx_inputs(m, M, K, N, M, True, True)
+    got = cases.run_mx_aclnn(m, inp, M, K, N, True, m.ACL_BF16, None)
+    name, segments = route(m)
+    assert name == "mxfp4_tiles_128" and segments > 1 and K <= 18 * 128 * segments, (name, segments)
+    check_close(got, cases.oracle_mx(m, inp, M, K, N, True, m.ACL_BF16, None), orc.BF16, "mxfp4 segments of small tiles")
