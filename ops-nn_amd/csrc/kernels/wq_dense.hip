@@ -274,7 +274,8 @@ int launch_wq_dense(const OpsnnWqmmArgs& a, hipStream_t st)
             if (rc != OPSNN_NOT_TAKEN) return rc;
         }
     }
-    note_route("wq_dense");
+    const bool two = pl.last.rows || pl.last.cols;   // (the product of the last strip, of all columns where there is one)
+    note_route(two ? "wq_dense_two" : "wq_dense", two ? pl.last.rest_splits : pl.last.splits);
     uint16_t* w16 = (uint16_t*)a.workspace;
     WqParams p{};
     p.ldw = (kn ? a.w.row_stride : a.w.col_stride) * wbits / 8;
