@@ -168,7 +168,7 @@ static double tile_kernel_us(const OpsnnWqmmArgs& a, const WqForm& f)
 // codes: the many-rows kernel where its shape conditions hold (with groups in [K, N] storage its scale table, and so its
 // 192- and 256-row instances, do not apply); else, from 129 rows, the tile kernel and up to 128 rows the streaming kernel.
 // With groups that are not whole chunks the general kernel is left, which counts where wq_general_counts says so.
-// (Of 368 measured calls 362 go to the faster side or one within 3 % of it (profiles/weight_only_routes.txt): 1999 x 4096 x 11008
+// (The rule from 1025 rows on.  Of 368 calls of 65 .. 2100 rows, measured with the product's former plan, 362 go to the faster side or one within 3 % of it (profiles/weight_only_routes.txt): 1999 x 4096 x 11008
 // bf16 x int4 228 -> 164 us, [K, N] storage 613 -> 162; 1000 x 8192 x 28672 fp16 x int4 stays on the many-rows kernel, 477 against 526; 65 x 4096 x 22896 on the streaming kernel, 54 against 93; 192 x 8192 x 22896 on the tile kernel, 127
 // against 230; 128 x 11008 x 4096 in [K, N] storage with the re-layout, 61 against 75.)
 struct DenseEstimate { double here, other; };
@@ -194,34 +194,65 @@ static DenseEstimate dense_estimate(const OpsnnWqmmArgs& a, double product_us)
     if (!f.nk) other += 2.0 + codes * f.wbits / 8.0 / (four ? 0.62e6 : 0.73e6);
     return {here, other};
 }
+// The kernels of 33 rows and more on the terms of wq_cost.h.  The many-rows kernel up to 64 rows: its estimate as corrected by 396 calls (median error
+// 4 %).
+static double rows_typical_us(const OpsnnWqmmArgs& a, const WqForm& f)
+{
+    static const double rate[2][2] = {{1.19, 1.02}, {1.1, 1.1}}, offs[2][2] = {{0.03, 0.28}, {0.12, 0.11}};   // [8 bits][bf16]
+    const int w8 = f.wbits == 8, bf = a.x_dtype == DT_BF16;
+    return rows_kernel_us(a, f.wbits, f.group) * rate[w8][bf] * (a.offset ? 1.0 + offs[w8][bf] : 1.0) - 3.88 + 1.49e-6 * (double)a.M * (double)a.N;
+}
+// From 65 rows, to 1024: a workgroup of 128 columns and R rows as in rows_kernel_us, fitted to 340 calls (half of them for the fit, median error of the
+// others 4 %).  Where the instance of 192 or 256 rows has no room for its table of scales beside x, or K is no multiple of 512, the call runs on the
+// tile kernel: 682 x 12288 x 9856 int4 in groups of 128 takes 575 us there, 230 on the wide kernel.
+static double many_rows_typical_us(const OpsnnWqmmArgs& a, const WqForm& f)
+{
+    static const double dq[2][2] = {{7.12, 10.9}, {11.6, 19.6}}, dq_off[2][2] = {{1.9, 9.4}, {4.9, 4.3}};          // [8 bits][bf16]
+    static const double more[2][2][2] = {{{0.95, 1.04}, {0.85, 0.85}}, {{0.915, 0.937}, {1.03, 1.43}}};             // [more than 192 rows]: of R
+    const int w8 = f.wbits == 8, bf = a.x_dtype == DT_BF16;
+    const int64_t wgs = (a.N + 127) / 128, kc = 4 * (128 / f.wbits), slab = wq_narrow_slab_rows(a.M, a.N, true);
+    const int64_t ks = wq_rows_ksplit(f.wbits, a.M, a.N, a.K, f.group, true), most = slab ? slab : a.M < 256 ? a.M : 256;
+    if (most > 128) {
+        int64_t pitch = 1;
+        while (pitch * f.group < a.K) pitch *= 2;
+        if (a.K % 512 != 0 || (most > 192 ? 131072 : 98304) + 512 * pitch > 163840) return tile_kernel_us(a, f);
+    }
+    const double cols = dq[w8][bf] + (a.offset ? dq_off[w8][bf] : 0.0), out_m = (double)a.M * (double)a.N * 1e-6;
+    auto launch_us = [&](int64_t rows, int64_t slabs) {
+        const int64_t r = (rows + 63) / 64 * 64, n = wgs * slabs * ks;
+        const bool cols64 = r <= 64 && ks == 1 && wgs * slabs <= 128 && a.K % (4 * kc) == 0;
+        const double rounds = cols64 ? 0.597 : (double)((n + 255) / 256);
+        return 4.39 + rounds * (double)a.K / (4096.0 * (double)ks) * (cols + 0.173 * (double)r) * (r > 128 ? more[r > 192][w8][bf] : 1.0);
+    };
+    const double rest = 1.486 * out_m + (ks > 1 ? 2.0 + 3.41 * (double)ks * out_m : 0.0);
+    if (slab) return launch_us(slab, (a.M + slab - 1) / slab) + rest;
+    return (double)(a.M / 256) * launch_us(256, 1) + (a.M % 256 ? launch_us(a.M % 256, 1) : 0.0) + rest;
+}
+// The pass with its product, from 65 rows to 1024 (937 calls, half of them for the fit, 4 %).
+static double dense_typical_us(const OpsnnWqmmArgs& a, const WqForm& f, double product_us)
+{
+    static const double pass[2][2] = {{0.3925, 0.4075}, {0.31, 0.336}};   // [K-contiguous][8 bits]: us per 10^6 codes
+    const double codes = (double)a.N * (double)a.K * 1e-6;
+    return 7.71 + codes * pass[f.nk][f.wbits == 8] * (1.0 + 0.578 * (codes < 200.0 ? codes / 100.0 : 2.0)) + 0.769 * product_us +
+           0.704e-6 * (double)a.M * (double)a.N;
+}
+// Up to 1024 rows the typical times decide, as they do between this route and the wide kernel; beyond, the estimates above.  (With those for all
+// of them, fitted to the product's former estimate, 558 x 1728 x 27136 bf16 x int8 went to the tile kernel, 85 -> 111 us.)
 static bool dense_is_faster(const OpsnnWqmmArgs& a, double product_us)
 {
     const DenseEstimate e = dense_estimate(a, product_us);
-    return e.here < 0.97 * e.other;   // (in doubt without the pass)
+    if (a.M > 1024) return e.here < 0.97 * e.other;   // (in doubt without the pass)
+    const WqForm f = wq_form(a);
+    return dense_typical_us(a, f, product_us) < (f.rows && f.nk ? many_rows_typical_us(a, f) : e.other);
 }
-// What a call of 33 rows and more typically takes without the wide kernel (wq_wide.hip), for its rule: the many-rows kernel's estimate as
-// corrected by 396 calls (median error 3 to 4 %), the pass by 944 (5 %).
-static double rows_typical_us(const OpsnnWqmmArgs& a, const WqForm& f)
-{
-    static const double rate[2][2][2] = {{{1.19, 1.02}, {1.1, 1.1}}, {{1.025, 0.977}, {1.0, 1.035}}};               // [from 65 rows][8 bits][bf16]
-    static const double offs[2][2][2] = {{{0.03, 0.28}, {0.12, 0.11}}, {{0.02, 0.27}, {0.07, 0.1}}};
-    const int many = a.M > 64, w8 = f.wbits == 8, bf = a.x_dtype == DT_BF16;
-    return rows_kernel_us(a, f.wbits, f.group) * rate[many][w8][bf] * (a.offset ? 1.0 + offs[many][w8][bf] : 1.0) - (many ? 1.36 : 3.88) +
-           (many ? 0.18e-6 : 1.49e-6) * (double)a.M * (double)a.N;
-}
+// What a call of 33 to 1024 rows typically takes without the wide kernel (wq_wide.hip), for its rule.
 double wq_many_rows_typical_us(const OpsnnWqmmArgs& a)
 {
     const WqForm f = wq_form(a);
     if (a.M <= 64) return f.rows && f.nk ? rows_typical_us(a, f) : 1e30;
     const double product_us = dense_plan(a.M, a.N, a.K).us;
-    const DenseEstimate e = dense_estimate(a, product_us);
-    if (a.K % 64 == 0 && a.N >= 128 && e.here < 0.97 * e.other) {
-        static const double pass[2][2] = {{0.467, 0.49}, {0.427, 0.421}};   // [K-contiguous][8 bits]: us per 10^6 codes
-        const double codes = (double)a.N * (double)a.K * 1e-6;
-        return 7.85 + codes * pass[f.nk][f.wbits == 8] * (1.0 + 0.299 * (codes < 200.0 ? codes / 100.0 : 2.0)) + 0.766 * product_us +
-               0.682e-6 * (double)a.M * (double)a.N;
-    }
-    return f.rows && f.nk ? rows_typical_us(a, f) : e.other;
+    if (a.K % 64 == 0 && a.N >= 128 && dense_is_faster(a, product_us)) return dense_typical_us(a, f, product_us);
+    return f.rows && f.nk ? many_rows_typical_us(a, f) : dense_estimate(a, product_us).other;
 }
 
 // Can the call run here?

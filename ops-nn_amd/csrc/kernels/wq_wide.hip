@@ -519,14 +519,26 @@ bool wide_plan(const OpsnnWqmmArgs& a, const WqForm& f, WqWidePlan& pl)
     return pl.us < 1e30f;
 }
 
-// Whether a call runs here at all: what the chosen layout typically takes (median error 3 %; see wq_cost.h).
+// Whether a call runs here at all: what the chosen layout typically takes (see wq_cost.h).  From 65 rows fitted to 937 calls of 65 .. 1024 (half of
+// them for the fit, median error of the others 3 %); up to 64 rows to the kernel before its 32 x 32 x 16 products, whose times some calls are
+// now a few percent below.
 double wide_typical_us(const OpsnnWqmmArgs& a, int wbits, const WqWidePlan& pl)
 {
-    static const double tile[2][2][2] = {{{0.343, 0.444}, {0.486, 0.82}}, {{0.407, 0.502}, {0.449, 0.802}}};   // [8 bits][bf16][offset]
+    const int w8 = wbits == 8, bf = a.x_dtype == DT_BF16;
+    const bool off = a.offset != nullptr;
     const int64_t strips = (a.N + WW_COLS - 1) / WW_COLS, tiles = (a.K + WW_KT - 1) / WW_KT, slabs = (a.M + 16 * pl.mb - 1) / (16 * pl.mb);
-    const double t = tile[wbits == 8][a.x_dtype == DT_BF16][a.offset != nullptr] + 0.066 * pl.mb + (pl.kn ? 0.056 : 0.0) + (pl.dwords ? 0.0125 * wbits : 0.0), out_m = (double)a.M * (double)a.N * 1e-6;
-    const double cu = (double)((strips * slabs * pl.splits + 255) / 256) * ((double)((tiles + pl.splits - 1) / pl.splits) * t + 1.91 + 0.355 * pl.mb + 0.0143 * pl.groups);
-    return 2.39 + 1.33 * out_m + wq_typical_both(cu, wq_typical_mb(wbits, a.N, a.K) / 6.56) + (pl.splits > 1 ? 2.9 + 2.09 * pl.splits * out_m * (a.N % 4 ? 2.0 : 1.0) : 0.0);
+    const double out_m = (double)a.M * (double)a.N * 1e-6, mb = (double)pl.mb, mbytes = wq_typical_mb(wbits, a.N, a.K);
+    const double rounds = (double)((strips * slabs * pl.splits + 255) / 256), steps = (double)((tiles + pl.splits - 1) / pl.splits);
+    if (a.M > 64) {
+        static const double tile[2][2] = {{0.175, 0.230}, {0.247, 0.282}}, offs[2] = {0.071, 0.241};   // [8 bits][bf16]
+        const double t = tile[w8][bf] + (off ? offs[bf] : 0.0) + 0.0924 * mb + (pl.kn ? 0.0386 : 0.0) + (pl.dwords ? 0.0233 * wbits : 0.0);
+        return 2.22 + 1.206 * out_m + wq_typical_both(rounds * (steps * t + 2.73 + 0.045 * mb + 0.0324 * pl.groups), mbytes / 6.86) +
+               (pl.splits > 1 ? 3.82 + 1.247 * pl.splits * out_m : 0.0);
+    }
+    static const double tile[2][2][2] = {{{0.343, 0.444}, {0.486, 0.82}}, {{0.407, 0.502}, {0.449, 0.802}}};   // [8 bits][bf16][offset]
+    const double t = tile[w8][bf][off] + 0.066 * mb + (pl.kn ? 0.056 : 0.0) + (pl.dwords ? 0.0125 * wbits : 0.0);
+    return 2.39 + 1.33 * out_m + wq_typical_both(rounds * (steps * t + 1.91 + 0.355 * mb + 0.0143 * pl.groups), mbytes / 6.56) +
+           (pl.splits > 1 ? 2.9 + 2.09 * pl.splits * out_m * (a.N % 4 ? 2.0 : 1.0) : 0.0);
 }
 // What the call typically takes on the kernel that it runs on otherwise.
 double others_typical_us(const OpsnnWqmmArgs& a, const WqForm& f)
@@ -548,19 +560,15 @@ double others_typical_us(const OpsnnWqmmArgs& a, const WqForm& f)
 
 // Does the call run here?  Looks at what both phases know: not at the weight's address (launch_wq_wide declines an unaligned one).
 //
-// Where the two estimates above say so.  (Of 2989 calls, 1797 of them drawn after the fit, timed on either side with the weight from memory and in
-// the last-level cache, 1983 run here, 46 of them 5 % slower or more than there, 14 by 10 %, the worst 1.28 times; among other fitted ones the
-// worst is 1.4, 339 x 15872 x 12160 bf16 x int8 226 us, 162 on the many-rows kernel.  Before there were estimates for [K, N] storage and up to 16
-// rows, and with the other estimates fitted to the weight from memory, 153 were, 82 by 10 %: 491 x 8448 x 2112 [K, N] int8 48 us with the pass
-// and 75 here, 27 x 17920 x 25376 [K, N] bf16 124 and 156, 3 x 1536 x 13184 bf16 10.7 and 13.6, 18 x 3328 x 1152 bf16 x int8 9.8 and 11.1.)
+// Where the two estimates above say so, the weight from memory and in the last-level cache.  From 65 rows, of 1151 calls timed here, on the pass and
+// on the other kernels 28 take 5 % longer than on the fastest, 6 by 10 %, the worst 1.19 times; with all estimates fitted to these kernels' former
+// times 95 did, 52 by 10 %: 576 x 14336 x 14144 int8 280 us on the many-rows kernel, 328 here.  Up to 64 rows: profiles/weight_only_wide_rule.txt.
 //
 // Below 2^20 codes nothing was timed; from 65 rows the pass is ahead below 2^21 (189 x 1152 x 1088 12.1 there, 13.7 here).  Up to 16 rows:
 // [K, N] storage not where the weight is large and wide, of 68 such calls 56 faster there (16 x 8192 x 28672 40.7 us, 47.9 here; 5 x 12288 x 27072 61
 // and 86); [N, K] storage from 8 MB, and not where K is one whole shape of the x-in-registers kernel (16 x 8192 x 28672 36 there, 44 here;
-// 4 x 3072 x 3128 7.3 and 10.5).  To 1024 rows: of 70 drawn calls of 513 .. 1024 the estimates
-// send 26 here, 1.15 times as fast as on the pass and the many-rows kernel, one slower by more than 2 % (762 x 10624 x 24704 472 us there, 500
-// here): 630 x 9472 x 18624 int4 fp16 326 -> 268, 707 x 9024 x 4160 int8 99 -> 77, 580 x 1408 x 5231 27.5 -> 21.6; of seven beyond one gained (1.07)
-// and one lost (1534 x 1728 x 2184 21 -> 26).
+// 4 x 3072 x 3128 7.3 and 10.5).  To 1024 rows (630 x 9472 x 18624 int4 fp16 326 -> 268,
+// 707 x 9024 x 4160 int8 99 -> 77); of seven calls beyond one gained (1.07) and one lost (1534 x 1728 x 2184 21 -> 26).
 //
 // Rows in dwords: of 126 drawn calls of that kind 68 come here, 1.22 times as fast as on the pass and the [K, N] decode kernel: 156 x 7168 x 21520 int4 bf16 208 -> 100 us, 85 x 11008 x 2456 37 -> 21, 53 x 1408 x 22192 28 -> 15.
 // Not where the estimates were wrong about them: from 257 rows with few k (510 x 1152 x 5744 21 there, 24 here), int8 up to 16 rows

@@ -164,3 +164,13 @@ def test_weight_only(gpu, M, K, N, group, w, x, nk, off, want):
     xd = m.ACL_FLOAT16 if x == "f16" else m.ACL_BF16
     cases.run_wq_aclnn(m, cases.make_wq_inputs(m, M, K, N, 1, xd, m.ACL_INT4 if w == "i4" else m.ACL_INT8, group, nk, off, None), M, K, N)
     assert route(m)[0] == want, route(m)
+
+
+# the same from 65 rows: pass, wide kernel or many-rows kernel.  us on the one taken and on the next
+@pytest.mark.parametrize("M,K,N,group,w,x,nk,off,want", [
+    (558, 1728, 27136, 0, "i8", "bf16", True, False, "wq_dense"),     # 84, tile kernel 111
+    (827, 12288, 6976, 128, "i4", "bf16", True, False, "wq_dense"),   # 187, tile kernel 700: the many-rows kernel's table does not fit
+    (257, 8192, 13312, 0, "i8", "f16", True, False, "wq_rows"),       # 84, wide kernel 118
+    (257, 7040, 1090, 128, "i4", "bf16", True, True, "wq_wide")])     # 23.3, pass 25.9
+def test_weight_only_from_65_rows(gpu, M, K, N, group, w, x, nk, off, want):
+    test_weight_only(gpu, M, K, N, group, w, x, nk, off, want)

@@ -20,7 +20,6 @@ ELSEWHERE.update({(1, 1056, 16416) + k: "wq_kn" for k in KINDS if k[1:] == ("bf1
 ELSEWHERE.update({(1, 1056, 1024) + k: "wq_general" for k in KINDS if k[0] == "i8"})
 ELSEWHERE.update({shape + k: "wq_general" for shape in [(1, 4128, 1064), (16, 4128, 1080)] for k in KINDS if k[0] == "i8"})
 ELSEWHERE[(33, 8192, 1048, "i4", "bf16", False)] = "wq_kn"
-ELSEWHERE.update({(257, 7040, 1090) + k: "wq_dense" for k in KINDS if k[1:] == ("bf16", True)})
 
 
 def _check(m, M, K, N, group, nk, w_dt, x_dt, off):
