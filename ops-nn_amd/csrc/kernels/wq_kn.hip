@@ -278,7 +278,7 @@ static int launch_kn_one(const WqParams& p, int splits, hipStream_t st)
         if (e != hipSuccess) return (int)e;
         device_flag_set(attr_set);
     }
-    note_route(TABLE ? "wq_kn_table" : "wq_kn", splits);
+    note_route(NW == 8 ? "wq_kn_table_w8" : TABLE ? "wq_kn_table" : "wq_kn", splits);
     hipLaunchKernelGGL(k, grid, dim3(64 * NW), lds, st, p, splits, window);
     if (hipError_t e = hipGetLastError(); e != hipSuccess || splits == 1) return (int)e;
     launch_wq_splitk_reduce(p, splits, XDT, st);

@@ -158,7 +158,7 @@ def test_fp32_outputs_with_the_8_bit_instruction(gpu, M, K, N):
     (110, 11008, 4096, 128, "i4", "f16", False, True, "wq_wide"), (9, 17280, 1888, 64, "i4", "f16", False, True, "wq_wide"),
     (3, 1536, 13184, 0, "i4", "bf16", True, True, "wq_resx"), (9, 1536, 6144, 0, "i8", "f16", True, False, "wq_resx"),
     (18, 3328, 1152, 0, "i8", "bf16", True, True, "wq_nk"), (57, 9856, 4352, 128, "i4", "f16", True, True, "wq_wide"),
-    (16, 8192, 28672, 128, "i4", "f16", False, True, "wq_kn_table"), (55, 2432, 1024, 128, "i4", "f16", True, False, "wq_nk"), (4, 3072, 3136, 128, "i4", "f16", True, False, "wq_resx")])
+    (16, 8192, 28672, 128, "i4", "f16", False, True, "wq_kn_table_w8"), (55, 2432, 1024, 128, "i4", "f16", True, False, "wq_nk"), (4, 3072, 3136, 128, "i4", "f16", True, False, "wq_resx")])
 def test_weight_only(gpu, M, K, N, group, w, x, nk, off, want):
     m = gpu
     xd = m.ACL_FLOAT16 if x == "f16" else m.ACL_BF16

@@ -55,7 +55,7 @@ def test_table_of_scales_in_several_windows(gpu, w_dt, x_dt, off):
     inp = cases.make_wq_inputs(m, M, K, N, 11, xd, m.ACL_INT4, 32, False, off, None)
     print(f"case kn windows M={M} K={K} N={N} {x_dt}", flush=True)
     got = cases.run_wq_aclnn(m, inp, M, K, N)
-    assert m.lib().opsnnDebugLastRoute(None) == b"wq_kn_table"
+    assert m.lib().opsnnDebugLastRoute(None) == b"wq_kn_table_w8"
     _b16_bar(got, cases.oracle_wq(m, inp, M, K, N), orc.F16 if x_dt == "f16" else orc.BF16, "kn windows", K)
 
 
@@ -70,5 +70,21 @@ def test_eight_waves(gpu, M, K, N, group, w_dt, x_dt, off):
     inp = cases.make_wq_inputs(m, M, K, N, M + K, xd, m.ACL_INT4 if w_dt == "i4" else m.ACL_INT8, group, False, off, xd if M % 2 else None)
     print(f"case kn eight waves M={M} K={K} N={N} g={group} {w_dt} {x_dt}", flush=True)
     got = cases.run_wq_aclnn(m, inp, M, K, N)
-    assert route(m) == ("wq_kn_table", 2), route(m)
+    assert route(m) == ("wq_kn_table_w8", 2), route(m)
     _b16_bar(got, cases.oracle_wq(m, inp, M, K, N), orc.F16 if x_dt == "f16" else orc.BF16, "kn eight waves", K)
+
+
+@pytest.mark.parametrize("M,x_dt,off,bias", [(16, "f16", True, True), (5, "bf16", False, True), (9, "bf16", True, False)])
+def test_eight_waves_in_one_segment(gpu, M, x_dt, off, bias):
+    """A plan of two segments is one workgroup of eight waves, which rounds and adds the bias itself; a ragged last strip of columns."""
+    import numpy as np
+    from test_gpu_routes import route
+    m = gpu
+    K, N = 3072, 44680
+    xd = m.ACL_FLOAT16 if x_dt == "f16" else m.ACL_BF16
+    inp = cases.make_wq_inputs(m, M, K, N, M, xd, m.ACL_INT4, 128, False, off, xd if bias else None)
+    print(f"case kn eight waves, one segment M={M} K={K} N={N} {x_dt}", flush=True)
+    got = cases.run_wq_aclnn(m, inp, M, K, N)
+    assert route(m) == ("wq_kn_table_w8", 1), route(m)
+    rows = np.array([0, M // 2, M - 1])
+    _b16_bar(np.ascontiguousarray(got[rows]), cases.oracle_wq(m, inp, M, K, N, rows=rows), orc.F16 if x_dt == "f16" else orc.BF16, "kn eight waves, one segment", K)
