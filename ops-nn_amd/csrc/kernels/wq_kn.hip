@@ -33,8 +33,9 @@ constexpr int kn_pf(int wbits, int mb) { return (mb == 2 || (mb == 1 && wbits ==
 constexpr int kn_cpl(int mb) { return mb == 1 ? 16 : 8; }   // codes per lane: with 16 and two row blocks the loop spills
 
 // Segments of K: as many workgroups as two per CU, less what a slice of partial sums costs.  (A step is 4 KB (int8: 8 KB) per
-// wave; at 5 TB/s the eight waves of a CU take 1.7 us for one each.  3 us: the second kernel.  Of 40 calls 33 run within 3 % of the
-// fastest count, the worst 13 % behind: 16 x 2048 x 16384 15.5 us, 13.7 with four segments; profiles/tile_plans.txt.  512: two
+// wave; at 5 TB/s the eight waves of a CU take 1.7 us for one each.  3 us: the second kernel.  Segments that run in pairs on eight waves
+// (launch_kn_mb) are priced one by one, which charges them for partial sums that they don't write.  Of 40 calls 35 run within 3 % of the
+// fastest count, the worst 5.5 % behind: 64 x 2048 x 16384 24.2 us, 22.9 with two segments; profiles/tile_plans.txt.  512: two
 // workgroups on each of the chip's 256 CUs, a constant, since phase 1 plans too and makes no HIP call.)
 static WqKnPlan kn_plan(int wbits, int64_t M, int64_t N, int64_t K)
 {

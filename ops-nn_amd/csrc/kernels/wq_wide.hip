@@ -565,8 +565,8 @@ double others_typical_us(const OpsnnWqmmArgs& a, const WqForm& f)
 // times 95 did, 52 by 10 %: 576 x 14336 x 14144 int8 280 us on the many-rows kernel, 328 here.  Up to 64 rows: profiles/weight_only_wide_rule.txt.
 //
 // Below 2^20 codes nothing was timed; from 65 rows the pass is ahead below 2^21 (189 x 1152 x 1088 12.1 there, 13.7 here).  Up to 16 rows:
-// [K, N] storage not where the weight is large and wide, of 68 such calls 56 faster there (16 x 8192 x 28672 40.7 us, 47.9 here; 5 x 12288 x 27072 61
-// and 86); [N, K] storage from 8 MB, and not where K is one whole shape of the x-in-registers kernel (16 x 8192 x 28672 36 there, 44 here;
+// [K, N] storage not where the weight is large and wide, of 13 such calls seven 8 to 36 % faster there, one 12 % faster here (5 x 16256 x 25792 60 us there, 77
+// here; 4 x 2560 x 27968 26.6 and 23.4), of 47 others none slower by the estimates than there, six that stay there 5 to 18 % faster here; [N, K] storage from 8 MB, and not where K is one whole shape of the x-in-registers kernel (16 x 8192 x 28672 36 there, 44 here;
 // 4 x 3072 x 3128 7.3 and 10.5).  To 1024 rows (630 x 9472 x 18624 int4 fp16 326 -> 268,
 // 707 x 9024 x 4160 int8 99 -> 77); of seven calls beyond one gained (1.07) and one lost (1534 x 1728 x 2184 21 -> 26).
 //
